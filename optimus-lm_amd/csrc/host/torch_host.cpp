@@ -1,0 +1,1130 @@
+// The host side of the MoE block in C++: allocations, launches of the C-ABI entry points and the
+// autograd nodes around them, as the Python module `optimus_torch_host`.
+//
+// What bounded the small calls was the interpreter: a training step of the tiny layer is 22 launches of
+// 2-14 us each, and enqueueing them through ctypes and Python autograd functions took 510 us.  Here a
+// layer is two autograd nodes (router, experts) whose forward and backward run without the interpreter:
+// each reads the three run-time switches of the Python modules once (launch log, profiler, in-place
+// weight gradients) and then only allocates and launches.
+//
+// The nodes are plain torch::autograd::Node objects: outputs nobody differentiates arrive as undefined
+// tensors (nothing is filled or added for them), and a weight whose gradient already lives in a flat
+// buffer gets it added there by the GEMM and an undefined gradient returned.
+#include <torch/extension.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <c10/hip/HIPStream.h>
+
+#include "../../../include/optimus_mi355x.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+namespace {
+
+struct NativeError : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+// ---- the Python modules' run-time switches --------------------------------------------------------
+
+PyObject *module_attr(const char *module, const char *name) {   // new reference; GIL held
+    PyObject *m = PyImport_ImportModule(module);
+    if (!m) throw py::error_already_set();
+    PyObject *v = PyObject_GetAttrString(m, name);
+    Py_DECREF(m);
+    if (!v) throw py::error_already_set();
+    return v;
+}
+bool attr_is(const char *module, const char *name, PyObject *what) {
+    PyObject *v = module_attr(module, name);
+    const bool same = v == what;
+    Py_DECREF(v);
+    return same;
+}
+
+struct Call {
+    bool log = false;        // optimus._native.launch_log is a list: time every launch
+    bool profile = false;    // optimus.globals.profiler is set
+    bool in_place = true;    // moe.accumulate_weight_grads_in_place
+    void *stream = nullptr;
+};
+
+Call begin_call() {
+    Call c;
+    {
+        py::gil_scoped_acquire gil;
+        c.log = !attr_is("optimus._native", "launch_log", Py_None);
+        c.profile = !attr_is("optimus.globals", "profiler", Py_None);
+        c.in_place = attr_is("optimus.models.common.moe", "accumulate_weight_grads_in_place", Py_True);
+    }
+    c.stream = c10::hip::getCurrentHIPStream().stream();
+    return c;
+}
+
+void check(int code, const char *what) {
+    if (code != 0)
+        throw NativeError(std::string(what) + " failed with code " + std::to_string(code) + ": " + om_strerror(code));
+}
+
+template <typename F> void launch(const Call &c, const char *name, F &&fn) {
+    if (!c.log) {
+        check(fn(), name);
+        return;
+    }
+    py::object start;
+    {
+        py::gil_scoped_acquire gil;
+        start = py::module_::import("optimus._native").attr("timed_begin")(name);
+    }
+    const int code = fn();
+    {
+        py::gil_scoped_acquire gil;
+        py::module_::import("optimus._native").attr("timed_end")(name, start);
+        start = py::object();
+    }
+    check(code, name);
+}
+#define OM(c, fn, ...) launch(c, #fn, [&] { return fn(__VA_ARGS__); })
+
+// optimus.profilers.record_pcl_function(name) around a scope, when a profiler is set
+struct ProfiledScope {
+    py::object context;
+    ProfiledScope(const Call &c, const char *name) {
+        if (!c.profile) return;
+        py::gil_scoped_acquire gil;
+        context = py::module_::import("optimus.profilers").attr("record_pcl_function")(name);
+        context.attr("__enter__")();
+    }
+    ~ProfiledScope() {
+        if (!context) return;
+        py::gil_scoped_acquire gil;
+        context.attr("__exit__")(py::none(), py::none(), py::none());
+        context = py::object();
+    }
+};
+
+// ---- tensor helpers -------------------------------------------------------------------------------
+
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+const int32_t *iptr(const Tensor &t) { return t.defined() ? t.data_ptr<int32_t>() : nullptr; }
+int dtype_code(const Tensor &t) {
+    if (t.scalar_type() == at::kFloat) return OM_F32;
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16, "unsupported dtype ", t.scalar_type(),
+                     ": the HIP kernels take float32 or bfloat16");
+    return OM_BF16;
+}
+int index_code(const Tensor &t) {
+    if (t.scalar_type() == at::kLong) return OM_I64;
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kInt, "expert indices must be int64 or int32, got ", t.scalar_type());
+    return OM_I32;
+}
+void require_device(const Tensor &t) {
+    if (!t.defined()) return;
+    if (!t.is_cuda())
+        throw NativeError("the HIP kernels need device tensors (got a CPU tensor); there is no CPU fallback");
+    if (!t.is_contiguous()) throw NativeError("the HIP kernels need contiguous row-major tensors");
+}
+void require_bf16(const Tensor &t) {
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16, "the fused expert kernels run in bfloat16 (got ",
+                     t.scalar_type(), "); cast the module with .to(torch.bfloat16)");
+}
+Tensor make(at::IntArrayRef size, const Tensor &like) { return at::empty(size, like.options()); }
+Tensor make(at::IntArrayRef size, const Tensor &like, at::ScalarType dt) { return at::empty(size, like.options().dtype(dt)); }
+
+// Elements between consecutive experts of a [G, out, in] weight whose inner two dims are dense; 0 for
+// the packed layout.
+int64_t expert_stride(const Tensor &w) {
+    const int64_t o = w.size(1), i = w.size(2);
+    if (w.stride(2) != 1 || w.stride(1) != i) throw NativeError("expert weights must be dense [out, in] matrices");
+    const int64_t s = w.size(0) > 1 ? w.stride(0) : o * i;
+    return s == o * i ? 0 : s;
+}
+
+// [G, out, in] over per-expert matrices that lie at a constant pitch in one storage; undefined when
+// they do not.
+Tensor strided_view_or_undefined(const Tensor *w, size_t step, int64_t G) {
+    const Tensor &w0 = w[0];
+    if (w0.dim() != 2) return Tensor();
+    const int64_t o = w0.size(0), i = w0.size(1);
+    if (G == 1) return w0.unsqueeze(0);
+    const int64_t esz = w0.element_size();
+    const char *p0 = static_cast<const char *>(w0.data_ptr());
+    const int64_t pitch = static_cast<const char *>(w[step].data_ptr()) - p0;
+    if (pitch <= 0 || pitch % esz != 0 || pitch < o * i * esz) return Tensor();
+    for (int64_t n = 0; n < G; n++) {
+        const Tensor &t = w[n * step];
+        if (!t.is_contiguous() || t.dim() != 2 || t.size(0) != o || t.size(1) != i ||
+            t.scalar_type() != w0.scalar_type() || static_cast<const char *>(t.data_ptr()) != p0 + n * pitch ||
+            !t.storage().is_alias_of(w0.storage()))
+            return Tensor();
+    }
+    return w0.as_strided({G, o, i}, {pitch / esz, i, 1});
+}
+Tensor strided_view(const Tensor *w, size_t step, int64_t G) {
+    Tensor v = strided_view_or_undefined(w, step, G);
+    if (!v.defined())
+        throw NativeError("per-expert weights must lie at a constant pitch inside one buffer (merge them with "
+                          "pack_expert_weights, or build the optimizer first so they alias flat_param)");
+    return v;
+}
+
+// ---- weight gradients that live in a flat buffer ----------------------------------------------------
+
+// param.grad if the weight-gradient kernels may add into it in place: a leaf parameter whose gradient
+// already exists as a dense view of a larger buffer, same dtype and shape, with no hooks that would
+// have to see the incoming gradient; else undefined.
+Tensor live_grad(const Tensor &param) {
+    if (!param.defined() || !param.is_leaf() || !param.requires_grad()) return Tensor();
+    const Tensor &grad = param.grad();
+    if (!grad.defined() || !grad.is_view() || grad.scalar_type() != param.scalar_type() ||
+        grad.sizes() != param.sizes() || !grad.is_cuda() || !grad.is_contiguous() || grad.requires_grad())
+        return Tensor();
+    if (!torch::autograd::impl::hooks(param).empty() || torch::autograd::impl::post_acc_grad_hooks(param) != nullptr)
+        return Tensor();
+    return grad;
+}
+
+// One projection's gradient: where the GEMM writes it.
+struct Sink {
+    Tensor grad;          // [G, out, in]: the live buffer, or a fresh tensor
+    int64_t pitch = 0;
+    bool accumulate = false;
+};
+// `leaves`: the parameter itself, or the G per-expert parameters `step` apart
+Sink grad_sink(const Call &c, const Tensor *leaves, size_t step, int64_t n_leaves, const Tensor &view) {
+    Sink s;
+    if (c.in_place && !at::GradMode::is_enabled()) {
+        if (n_leaves == 1) {
+            s.grad = live_grad(leaves[0]);
+            if (s.grad.defined() && s.grad.dim() == 2) s.grad = s.grad.unsqueeze(0);
+        } else {
+            std::vector<Tensor> grads;
+            grads.reserve(n_leaves);
+            for (int64_t n = 0; n < n_leaves; n++) {
+                grads.push_back(live_grad(leaves[n * step]));
+                if (!grads.back().defined()) break;
+            }
+            if (grads.back().defined()) s.grad = strided_view_or_undefined(grads.data(), 1, n_leaves);
+        }
+    }
+    if (s.grad.defined()) {
+        s.pitch = expert_stride(s.grad);
+        s.accumulate = true;
+    } else {
+        s.grad = make(view.sizes(), view);
+    }
+    return s;
+}
+
+// ---- index construction ---------------------------------------------------------------------------
+
+// The arrays of om_moe_sort and the tensors that own them.
+struct Index {
+    std::vector<Tensor> owners;     // one buffer that holds them all, or five tensors (cum, cum_ep, in, out, sel)
+    int64_t NR = 0, T = 0, TK = 0;  // the one buffer's parts
+    void resolve() {
+        if (owners.size() == 1) {
+            int32_t *p = owners[0].data_ptr<int32_t>();
+            cum = p; cum_ep = p + NR + 1; in = cum_ep + T + 1; out = in + TK; sel = out + TK;
+        } else {
+            cum = iptr(owners[0]); cum_ep = iptr(owners[1]); in = iptr(owners[2]); out = iptr(owners[3]); sel = iptr(owners[4]);
+        }
+    }
+    const int32_t *cum = nullptr, *cum_ep = nullptr, *in = nullptr, *out = nullptr, *sel = nullptr;
+    int64_t rows = 0;               // entries of the three last: the routed rows, or an upper bound of them
+    bool bound = false;
+};
+
+std::vector<Tensor> sort_tensors(const Call &c, const Tensor &experts, int64_t start, int64_t end) {
+    require_device(experts);
+    const int64_t T = experts.size(0), K = experts.size(1), NR = end - start;
+    const auto opt = experts.options().dtype(at::kInt);
+    std::vector<Tensor> r = {at::empty({NR + 1}, opt), at::empty({T + 1}, opt), at::empty({T * K}, opt),
+                             at::empty({T * K}, opt), at::empty({T * K}, opt)};
+    const int64_t ws_bytes = om_moe_sort_workspace_bytes(T, K, NR);
+    Tensor ws = at::empty({std::max<int64_t>(ws_bytes / 4, 1)}, opt);
+    OM(c, om_moe_sort, ptr(experts), index_code(experts), T, K, start, end, r[0].data_ptr<int32_t>(),
+       r[1].data_ptr<int32_t>(), r[2].data_ptr<int32_t>(), r[3].data_ptr<int32_t>(), r[4].data_ptr<int32_t>(),
+       ptr(ws), ws_bytes, c.stream);
+    return r;
+}
+
+Index sort_index(const Call &c, const Tensor &experts, int64_t start, int64_t end) {
+    require_device(experts);
+    const int64_t T = experts.size(0), K = experts.size(1), NR = end - start, TK = T * K;
+    const int64_t ws_bytes = om_moe_sort_workspace_bytes(T, K, NR);
+    const int64_t ws_at = (NR + 1 + T + 1 + 3 * TK + 3) & ~int64_t(3);
+    Tensor buf = at::empty({ws_at + std::max<int64_t>(ws_bytes / 4, 1)}, experts.options().dtype(at::kInt));
+    int32_t *p = buf.data_ptr<int32_t>();
+    int32_t *cum = p, *cum_ep = cum + NR + 1, *in = cum_ep + T + 1, *out = in + TK, *sel = out + TK;
+    OM(c, om_moe_sort, ptr(experts), index_code(experts), T, K, start, end, cum, cum_ep, in, out, sel, p + ws_at,
+       ws_bytes, c.stream);
+    Index ix;
+    ix.owners = {buf};
+    ix.NR = NR; ix.T = T; ix.TK = TK;
+    ix.resolve();
+    ix.rows = TK;
+    return ix;
+}
+
+// ---- the expert MLP ---------------------------------------------------------------------------------
+
+struct MlpWeights {
+    Tensor gate, up, down;   // [G, I, H], [G, I, H], [G, H, I]
+    int64_t G() const { return gate.size(0); }
+    int64_t I() const { return gate.size(1); }
+    int64_t H() const { return gate.size(2); }
+};
+struct MlpState {
+    Tensor cum, g, u, h;     // cum undefined: the caller's index holds the offsets
+};
+
+int64_t shared_pitch(const MlpWeights &w) {
+    const int64_t s = expert_stride(w.gate);
+    if (expert_stride(w.up) != s) throw NativeError("gate and up expert weights must share one expert pitch");
+    return s;
+}
+
+void gemm_dtype(const Tensor &a, const Tensor &b, const Tensor &c) {
+    const auto dt = a.scalar_type();
+    TORCH_CHECK_TYPE((dt == at::kBFloat16 || dt == at::kFloat) && b.scalar_type() == dt && c.scalar_type() == dt,
+                     "the grouped expert GEMMs take operands that are all bfloat16 or all float32 (got ", dt, ", ",
+                     b.scalar_type(), ", ", c.scalar_type(), ")");
+}
+
+const float *fp(const Tensor &t) { return static_cast<const float *>(ptr(t)); }
+float *fpm(const Tensor &t) { return static_cast<float *>(ptr(t)); }
+
+Tensor gathered_rows(const Call &c, const Tensor &x, const int32_t *x_rows, int64_t rows) {
+    if (!x_rows) return x;
+    Tensor out = make({rows, x.size(1)}, x);
+    OM(c, om_index_gather, ptr(x), x_rows, ptr(out), rows, x.size(1), dtype_code(x), c.stream);
+    return out;
+}
+
+// y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment; with x_rows the MLP input is x[x_rows]
+Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const int32_t *cum, const int32_t *x_rows,
+                      int64_t rows, MlpState &s) {
+    require_device(x);
+    gemm_dtype(x, w.gate, w.up);
+    gemm_dtype(x, w.gate, w.down);
+    const int64_t G = w.G(), I = w.I(), H = w.H();
+    s.g = make({rows, I}, x);
+    s.u = make({rows, I}, x);
+    s.h = make({rows, I}, x);
+    Tensor y = make({rows, H}, x);
+    ProfiledScope scope(c, "1moeblock--7gmlp_fwd");
+    if (x.scalar_type() == at::kFloat) {
+        // float32 modules: three grouped GEMMs and the SwiGLU glue kernel
+        const Tensor xs = gathered_rows(c, x, x_rows, rows);
+        OM(c, om_grouped_gemm_fwd_f32, fp(xs), fp(w.gate), fpm(s.g), cum, rows, G, I, H, expert_stride(w.gate), c.stream);
+        OM(c, om_grouped_gemm_fwd_f32, fp(xs), fp(w.up), fpm(s.u), cum, rows, G, I, H, expert_stride(w.up), c.stream);
+        if (rows) OM(c, om_swiglu_fwd, ptr(s.g), ptr(s.u), ptr(s.h), rows * I, OM_F32, c.stream);
+        OM(c, om_grouped_gemm_fwd_f32, fp(s.h), fp(w.down), fpm(y), cum, rows, G, H, I, expert_stride(w.down), c.stream);
+        return y;
+    }
+    const int64_t pitch = shared_pitch(w);
+    if (x_rows && rows > 0)
+        OM(c, om_merged_mlp_gate_up_fwd_gathered, ptr(x), x_rows, x.size(0), ptr(w.gate), ptr(w.up), ptr(s.g), ptr(s.u),
+           ptr(s.h), cum, rows, G, I, H, pitch, c.stream);
+    else
+        OM(c, om_merged_mlp_gate_up_fwd, ptr(x), ptr(w.gate), ptr(w.up), ptr(s.g), ptr(s.u), ptr(s.h), cum, rows, G, I, H,
+           pitch, c.stream);
+    OM(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), cum, rows, G, H, I, expert_stride(w.down), c.stream);
+    return y;
+}
+
+enum class WgradRows { PLAIN, INPUT, OUTPUT_GRAD };
+
+// One of the bf16 weight-gradient entry points: plain, or with the rows of `input` or of
+// `output_grad` taken through an index, writing or (accumulate) adding into the sink.
+void wgrad(const Call &c, const Tensor &output_grad, const Tensor &input, const Sink &s, const int32_t *cum,
+           int64_t rows, int64_t G, int64_t N, int64_t K, WgradRows kind = WgradRows::PLAIN,
+           const int32_t *index = nullptr, int64_t src_rows = 0) {
+    void *out = ptr(s.grad);
+#define OM_W(fn, ...)                                                                    \
+    do {                                                                                 \
+        if (s.accumulate) OM(c, fn##_accumulate, __VA_ARGS__);                           \
+        else OM(c, fn, __VA_ARGS__);                                                     \
+    } while (0)
+    if (kind == WgradRows::INPUT)
+        OM_W(om_grouped_gemm_wgrad_gathered, ptr(output_grad), ptr(input), index, src_rows, out, cum, rows, G, N, K,
+             s.pitch, c.stream);
+    else if (kind == WgradRows::OUTPUT_GRAD)
+        OM_W(om_grouped_gemm_wgrad_gathered_out, ptr(output_grad), index, src_rows, ptr(input), out, cum, rows, G, N, K,
+             s.pitch, c.stream);
+    else
+        OM_W(om_grouped_gemm_wgrad, ptr(output_grad), ptr(input), out, cum, rows, G, N, K, s.pitch, c.stream);
+#undef OM_W
+}
+void wgrad_f32(const Call &c, const Tensor &output_grad, const Tensor &input, const Sink &s, const int32_t *cum,
+               int64_t rows, int64_t G, int64_t N, int64_t K) {
+    if (s.accumulate)
+        OM(c, om_grouped_gemm_wgrad_f32_accumulate, fp(output_grad), fp(input), fpm(s.grad), cum, rows, G, N, K, s.pitch, c.stream);
+    else
+        OM(c, om_grouped_gemm_wgrad_f32, fp(output_grad), fp(input), fpm(s.grad), cum, rows, G, N, K, s.pitch, c.stream);
+}
+
+struct Sinks {
+    Sink gate, up, down;
+    static Tensor fresh(const Sink &s) { return s.accumulate ? Tensor() : s.grad; }
+};
+
+// Backward of merged_forward: returns dx (of the gathered matrix when x_rows is set); the weight
+// gradients go into the sinks.
+Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeights &w, const int32_t *cum,
+                       const MlpState &s, const int32_t *x_rows, const Sinks &k) {
+    dy = dy.contiguous();
+    const int64_t rows = dy.size(0), H = dy.size(1), G = w.G(), I = w.I();
+    Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx = make({rows, H}, x);
+    ProfiledScope scope(c, "1moeblock--7gmlp_bwd");
+    if (x.scalar_type() == at::kFloat) {
+        const Tensor xs = gathered_rows(c, x, x_rows, rows);
+        Tensor dh = make({rows, I}, x), dx2 = make({rows, H}, x);
+        wgrad_f32(c, dy, s.h, k.down, cum, rows, G, H, I);
+        OM(c, om_grouped_gemm_dgrad_f32, fp(dy), fp(w.down), fpm(dh), cum, rows, G, H, I, expert_stride(w.down), c.stream);
+        if (rows) OM(c, om_swiglu_bwd, ptr(dh), ptr(s.g), ptr(s.u), ptr(dg), ptr(du), rows * I, OM_F32, c.stream);
+        wgrad_f32(c, dg, xs, k.gate, cum, rows, G, I, H);
+        wgrad_f32(c, du, xs, k.up, cum, rows, G, I, H);
+        OM(c, om_grouped_gemm_dgrad_f32, fp(dg), fp(w.gate), fpm(dx), cum, rows, G, I, H, expert_stride(w.gate), c.stream);
+        OM(c, om_grouped_gemm_dgrad_f32, fp(du), fp(w.up), fpm(dx2), cum, rows, G, I, H, expert_stride(w.up), c.stream);
+        dx.add_(dx2);
+        return dx;
+    }
+    wgrad(c, dy, s.h, k.down, cum, rows, G, H, I);
+    OM(c, om_merged_mlp_down_dgrad, ptr(dy), ptr(w.down), ptr(s.g), ptr(s.u), ptr(dg), ptr(du), cum, rows, G, I, H,
+       expert_stride(w.down), c.stream);
+    const WgradRows kind = x_rows && rows > 0 ? WgradRows::INPUT : WgradRows::PLAIN;
+    wgrad(c, dg, x, k.gate, cum, rows, G, I, H, kind, x_rows, x.size(0));
+    wgrad(c, du, x, k.up, cum, rows, G, I, H, kind, x_rows, x.size(0));
+    OM(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx), cum, rows, G, I, H,
+       expert_stride(w.gate), c.stream);
+    return dx;
+}
+
+// The routed half of a bf16 block: gather, weighted SwiGLU MLP, unweighted sum of a token's rows.
+Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const Index &ix, const MlpWeights &w,
+                      const Tensor &residual, MlpState &s, Tensor &row_weights) {
+    require_device(x);
+    require_device(rw);
+    require_device(residual);
+    require_bf16(x);
+    require_bf16(w.gate);
+    require_bf16(w.up);
+    require_bf16(w.down);
+    const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
+    const int64_t pitch = shared_pitch(w);
+    row_weights = make({rows}, x, at::kFloat);
+    s.g = make({rows, I}, x);
+    s.u = make({rows, I}, x);
+    s.h = make({rows, I}, x);
+    Tensor y = make({rows, H}, x), final = make({T, H}, x);
+    {
+        ProfiledScope scope(c, "1moeblock--7gmlp_fwd");
+        OM(c, om_moe_row_weights, ptr(rw), ix.sel, ix.in, ix.out, fpm(row_weights), rows, K, dtype_code(rw), c.stream);
+        OM(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), fp(row_weights), ptr(s.g),
+           ptr(s.u), ptr(s.h), ix.cum, rows, G, I, H, pitch, c.stream);
+        OM(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, G, H, I, expert_stride(w.down), c.stream);
+    }
+    ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_fwd");
+    OM(c, om_sum_ggemm_output, ptr(y), ix.cum_ep, ix.out, ptr(residual), ptr(final), T, H, OM_BF16, c.stream);
+    return final;
+}
+
+// -> (dx, d routing_weights); `base` [T,H]: another gradient of the same hidden states, added to dx
+// inside the per-token sum.
+std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, const Tensor &x, const Tensor &rw,
+                                          const Index &ix, const MlpWeights &w, const MlpState &s,
+                                          const Tensor &row_weights, const Sinks &k, const Tensor &base) {
+    const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
+    Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx_rows = make({rows, H}, x);
+    // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window stay zero
+    Tensor drw = rows == rw.numel() && !ix.bound ? make(rw.sizes(), rw) : at::zeros(rw.sizes(), rw.options());
+    Tensor dx = make(x.sizes(), x);
+    {
+        ProfiledScope scope(c, "1moeblock--7gmlp_bwd");
+        if (rows > 0) {
+            const int parts = om_merged_mlp_row_dot_parts(I);
+            if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
+            Tensor row_dot = make({parts, rows}, x, at::kFloat);
+            wgrad(c, dfinal, s.h, k.down, ix.cum, rows, G, H, I, WgradRows::OUTPUT_GRAD, ix.in, T);
+            OM(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
+               fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows, G, I, H, expert_stride(w.down), c.stream);
+            OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
+               c.stream);
+            wgrad(c, dg, x, k.gate, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
+            wgrad(c, du, x, k.up, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
+            OM(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows, G, I,
+               H, expert_stride(w.gate), c.stream);
+        } else {   // nothing routed to these experts: fresh weight gradients are zero, live ones stay as they are
+            for (const Sink *sk : {&k.down, &k.gate, &k.up})
+                if (!sk->accumulate) {
+                    const int64_t n = sk->grad.size(1), kk = sk->grad.size(2);
+                    OM(c, om_grouped_gemm_wgrad, nullptr, nullptr, ptr(sk->grad), ix.cum, 0, G, n, kk, 0, c.stream);
+                }
+        }
+    }
+    ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
+    require_device(base);
+    OM(c, om_sum_ggemm_output, ptr(dx_rows), ix.cum_ep, ix.out, ptr(base), ptr(dx), T, H, OM_BF16, c.stream);
+    return {dx, drw};
+}
+
+// ---- autograd plumbing --------------------------------------------------------------------------------
+
+bool any_requires_grad(at::ArrayRef<Tensor> ts) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor &t : ts)
+        if (t.defined() && t.requires_grad()) return true;
+    return false;
+}
+
+template <typename N> std::shared_ptr<N> make_node(const variable_list &inputs) {
+    std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(inputs));
+    return node;
+}
+
+// A node's backward: kernel errors become the package's own exception type in the thread that called
+// backward().
+struct HostNode : Node {
+    virtual variable_list run(variable_list &&grads) = 0;
+    variable_list apply(variable_list &&grads) override {
+        try {
+            at::AutoDispatchBelowADInplaceOrView below;
+            return run(std::move(grads));
+        } catch (const NativeError &e) {
+            py::gil_scoped_acquire gil;
+            PyObject *cls = module_attr("optimus._native", "NativeLibraryError");
+            PyErr_SetString(cls, e.what());
+            Py_DECREF(cls);
+            python_error err;
+            err.persist();
+            throw std::move(err);
+        }
+    }
+    // Everything the backward needs is saved through SavedVariable, so that saved-tensor hooks (activation
+    // checkpointing, offloading) see all of it and a second backward is refused.
+    std::vector<SavedVariable> vars;
+    void save(const Tensor &t) { vars.emplace_back(t, false); }
+    std::vector<Tensor> saved() {
+        std::vector<Tensor> out;
+        out.reserve(vars.size());
+        for (auto &v : vars) out.push_back(v.unpack(shared_from_this()));
+        return out;
+    }
+    void release_variables() override {
+        for (auto &v : vars) v.reset_data();
+    }
+};
+
+MlpWeights weights_of(const std::vector<Tensor> &leaves, bool merged, size_t first, int64_t n_groups) {
+    MlpWeights w;
+    if (merged) {
+        w = {leaves[first], leaves[first + 1], leaves[first + 2]};
+        if (w.gate.dim() == 2) w = {w.gate.unsqueeze(0), w.up.unsqueeze(0), w.down.unsqueeze(0)};
+    } else {
+        w = {strided_view(&leaves[first], 3, n_groups), strided_view(&leaves[first + 1], 3, n_groups),
+             strided_view(&leaves[first + 2], 3, n_groups)};
+    }
+    return w;
+}
+Sinks sinks_of(const Call &c, const std::vector<Tensor> &leaves, bool merged, size_t first, int64_t n_groups,
+               const MlpWeights &w) {
+    const int64_t n = merged ? 1 : n_groups;
+    return {grad_sink(c, &leaves[first], 3, n, w.gate), grad_sink(c, &leaves[first + 1], 3, n, w.up),
+            grad_sink(c, &leaves[first + 2], 3, n, w.down)};
+}
+// gradients in the order of the leaves; undefined for a projection whose gradient went into its live buffer
+void push_grads(variable_list &out, const Sinks &k, bool merged, int64_t n_groups, bool single) {
+    const Tensor g[3] = {Sinks::fresh(k.gate), Sinks::fresh(k.up), Sinks::fresh(k.down)};
+    if (merged) {
+        for (const Tensor &t : g) out.push_back(single && t.defined() ? t.select(0, 0) : t);
+        return;
+    }
+    for (int64_t n = 0; n < n_groups; n++)
+        for (const Tensor &t : g) out.push_back(t.defined() ? t.select(0, n) : t);
+}
+
+// ---- router nodes -------------------------------------------------------------------------------------
+
+void require_gate_shape(const Tensor &weight, const char *what) {
+    const int64_t N = weight.size(0), H = weight.size(1);
+    if (N > 256 || H % 8 != 0)
+        throw NativeError(std::string(what) + ": the gate kernels take at most 256 experts and hidden sizes that are "
+                          "multiples of 8 (got " + std::to_string(N) + " experts, hidden " + std::to_string(H) +
+                          "); there is no library fallback");
+}
+
+Tensor gate_weight_grad(const Call &c, const Tensor &x, const Tensor &weight, Tensor dlogits) {
+    require_gate_shape(weight, "gate weight gradient");
+    const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+    const int64_t ws_bytes = om_router_gate_wgrad_workspace_bytes(T, H, N);
+    if (ws_bytes < 0) check(static_cast<int>(ws_bytes), "om_router_gate_wgrad_workspace_bytes");
+    Tensor ws = make({std::max<int64_t>(ws_bytes, 16)}, x, at::kByte), dw = make(weight.sizes(), weight);
+    dlogits = dlogits.contiguous();
+    OM(c, om_router_gate_wgrad, ptr(x), fp(dlogits), T, H, N, ptr(dw), dtype_code(dw), ptr(ws), ws_bytes, c.stream);
+    return dw;
+}
+
+// dx = bf16(dlogits) @ weight (+ other_grad, the gradient that reached the same hidden states through
+// the experts, with autograd's two roundings)
+Tensor gate_input_grad(const Call &c, const Tensor &weight, Tensor dlogits, Tensor other_grad) {
+    require_gate_shape(weight, "gate input gradient");
+    const int64_t T = dlogits.size(0), N = weight.size(0), H = weight.size(1);
+    dlogits = dlogits.contiguous();
+    if (other_grad.defined()) {
+        other_grad = other_grad.contiguous();
+        require_bf16(other_grad);
+    }
+    Tensor dx = make({T, H}, dlogits, at::kBFloat16);
+    OM(c, om_router_gate_dgrad, fp(dlogits), ptr(weight), ptr(other_grad), ptr(dx), T, H, N, c.stream);
+    return dx;
+}
+
+// (dx, dweight) of logits = x @ weight.T from the gradient of the logits; float32 modules run the plain
+// float32 gate kernels.
+std::pair<Tensor, Tensor> gate_backward(const Call &c, const Tensor &x, const Tensor &weight, Tensor dlogits, bool need_x,
+                                        bool need_w, const Tensor &other_grad) {
+    dlogits = dlogits.to(at::kFloat).contiguous();
+    Tensor dx, dw;
+    if (x.scalar_type() == at::kFloat) {
+        const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+        if (need_x) {
+            dx = make(x.sizes(), x);
+            OM(c, om_router_gate_dgrad_f32, fp(dlogits), fp(weight), T, H, N, fpm(dx), c.stream);
+            if (other_grad.defined()) dx.add_(other_grad);
+        }
+        if (need_w) {
+            dw = make(weight.sizes(), weight);
+            OM(c, om_router_gate_wgrad_f32, fp(x), fp(dlogits), T, H, N, fpm(dw), c.stream);
+        }
+        return {dx, dw};
+    }
+    require_bf16(x);
+    require_bf16(weight);
+    if (need_x) dx = gate_input_grad(c, weight, dlogits, other_grad);
+    if (need_w) dw = gate_weight_grad(c, x, weight, dlogits);
+    return {dx, dw};
+}
+
+Tensor gate_logits_forward(const Call &c, const Tensor &x, const Tensor &weight) {
+    require_device(x);
+    require_device(weight);
+    const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+    Tensor logits = make({T, N}, x, at::kFloat);
+    if (x.scalar_type() == at::kFloat) {
+        OM(c, om_router_gate_logits_f32, fp(x), fp(weight), T, H, N, fpm(logits), c.stream);
+        return logits;
+    }
+    require_gate_shape(weight, "gate projection");
+    if (N > 64 || H % 512 != 0) {
+        // many experts: the weight no longer fits a block's re-reads; split over H instead (also the
+        // form for hidden sizes the one-pass kernel does not take)
+        const int64_t ws_bytes = om_router_gate_logits_split_workspace_bytes(T, H, N);
+        if (ws_bytes < 0) check(static_cast<int>(ws_bytes), "om_router_gate_logits_split_workspace_bytes");
+        Tensor ws = make({std::max<int64_t>(ws_bytes, 16)}, x, at::kByte);
+        OM(c, om_router_gate_logits_split, ptr(x), ptr(weight), T, H, N, fpm(logits), ptr(ws), ws_bytes, c.stream);
+    } else {
+        OM(c, om_router_gate_logits, ptr(x), ptr(weight), T, H, N, fpm(logits), c.stream);
+    }
+    return logits;
+}
+
+// Gate projection and routing.  Outputs: the logits and the selection that follows from them, and x
+// itself: experts fed from that output make their input gradient arrive here, where the gate's own is
+// added to it inside its kernel.
+struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits as the selection saw them, experts
+    bool renorm = false, sigmoid = false;
+    double scale = 1.0;
+    int out_logits = -1, out_weights = -1, out_x = -1;   // positions of the differentiable outputs
+    std::string name() const override { return "OptimusRouterBackward"; }
+    variable_list run(variable_list &&grads) override {
+        auto grad = [&](int at) { return at >= 0 && at < static_cast<int>(grads.size()) ? grads[at] : Tensor(); };
+        Tensor logits_grad = grad(out_logits), weights_grad = grad(out_weights), x_grad = grad(out_x);
+        if (!logits_grad.defined() && !weights_grad.defined()) return {x_grad, Tensor()};
+        const Call c = begin_call();
+        const std::vector<Tensor> kept = saved();
+        const Tensor &xs = kept[0], &ws = kept[1];
+        Tensor dlogits = logits_grad;
+        if (weights_grad.defined()) {
+            const Tensor &logits = kept[2], &experts = kept[3];
+            const int64_t T = logits.size(0), N = logits.size(1), K = experts.size(1);
+            dlogits = make(logits.sizes(), logits);
+            if (sigmoid) {
+                weights_grad = weights_grad.contiguous().to(at::kFloat);
+                OM(c, om_route_sigmoid_topk_bwd, fp(logits), experts.data_ptr<int64_t>(), fp(weights_grad), T, N, K, renorm,
+                   scale, fpm(dlogits), c.stream);
+            } else {
+                weights_grad = weights_grad.contiguous();
+                OM(c, om_route_softmax_topk_bwd, ptr(logits), dtype_code(logits), experts.data_ptr<int64_t>(),
+                   ptr(weights_grad), dtype_code(weights_grad), T, N, K, renorm, ptr(dlogits), c.stream);
+            }
+            if (logits_grad.defined()) dlogits = dlogits.add(logits_grad);
+        }
+        auto d = gate_backward(c, xs, ws, dlogits, task_should_compute_output(0), task_should_compute_output(1), x_grad);
+        return {d.first, d.second};
+    }
+};
+
+void set_outputs(const std::shared_ptr<RouterNode> &node, Tensor *logits, Tensor *weights, Tensor *x) {
+    int at = 0;
+    if (weights) { node->out_weights = at++; torch::autograd::set_history(*weights, node); }
+    if (logits) { node->out_logits = at++; torch::autograd::set_history(*logits, node); }
+    if (x) { node->out_x = at++; torch::autograd::set_history(*x, node); }
+}
+
+std::shared_ptr<RouterNode> router_node(const Tensor &x, const Tensor &weight) {
+    auto node = make_node<RouterNode>({x, weight});
+    node->save(x);
+    node->save(weight);
+    return node;
+}
+
+// (logits float32, x)
+std::tuple<Tensor, Tensor> gate_logits(const Tensor &x, const Tensor &weight) {
+    Tensor logits, x_out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        logits = gate_logits_forward(begin_call(), x, weight);
+        x_out = x.alias();
+    }
+    if (any_requires_grad({x, weight})) {
+        auto node = router_node(x, weight);
+        set_outputs(node, &logits, nullptr, &x_out);
+    }
+    return {logits, x_out};
+}
+
+// softmax top-K router -> (routing_weights, selected_experts int64, logits, x).  `fused`: one launch for
+// projection and routing (shapes of om_router_gate_softmax_topk).  `bf16_logits`: the logits are rounded
+// to bf16 before the softmax, as a bf16 linear layer returns them.
+std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
+                                                         at::ScalarType out_dtype, bool fused, bool bf16_logits) {
+    const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+    Tensor logits, weights, experts, x_out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
+        require_device(x);
+        require_device(weight);
+        weights = make({T, top_k}, x, out_dtype);
+        experts = make({T, top_k}, x, at::kLong);
+        if (fused) {
+            logits = make({T, N}, x, at::kFloat);
+            OM(c, om_router_gate_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, fpm(logits), ptr(weights),
+               dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
+        } else {
+            logits = gate_logits_forward(c, x, weight);
+            if (bf16_logits) logits = logits.to(at::kBFloat16);
+            OM(c, om_route_softmax_topk, ptr(logits), dtype_code(logits), T, N, top_k, renorm, ptr(weights),
+               dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
+        }
+        x_out = x.alias();
+    }
+    if (any_requires_grad({x, weight})) {
+        auto node = router_node(x, weight);
+        // (a detached alias: saving an output itself would tie the node to itself)
+        node->save(logits.detach());
+        node->save(experts);
+        node->renorm = renorm;
+        set_outputs(node, &logits, &weights, &x_out);
+    }
+    return {weights, experts, logits, x_out};
+}
+
+// sigmoid / group-limited router -> (selected_experts int64, routing_weights float32, x)
+std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &weight, const Tensor &bias, int64_t n_group,
+                                                 int64_t topk_group, int64_t top_k, bool renorm, double scale) {
+    const int64_t T = x.size(0), N = weight.size(0);
+    Tensor logits, weights, experts, x_out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
+        require_device(bias);
+        logits = gate_logits_forward(c, x, weight);
+        weights = make({T, top_k}, x, at::kFloat);
+        experts = make({T, top_k}, x, at::kLong);
+        OM(c, om_route_sigmoid_group_topk, fp(logits), fp(bias), T, N, n_group, topk_group, top_k, renorm, scale,
+           experts.data_ptr<int64_t>(), fpm(weights), c.stream);
+        x_out = x.alias();
+    }
+    if (any_requires_grad({x, weight})) {
+        auto node = router_node(x, weight);
+        node->save(logits);
+        node->save(experts);
+        node->renorm = renorm;
+        node->sigmoid = true;
+        node->scale = scale;
+        set_outputs(node, nullptr, &weights, &x_out);
+    }
+    return {experts, weights, x_out};
+}
+
+// ---- expert nodes -------------------------------------------------------------------------------------
+
+// The expert half of a bf16 block (see routed_forward), with an optional residual or shared expert.
+// Inputs in order: hidden_states, routing_weights, residual, routed leaves, shared leaves.
+struct RoutedNode : HostNode {
+    Index ix;                        // (without its owners)
+    std::vector<Tensor> leaves;      // the routed weights as the caller holds them, then the shared expert's three
+    MlpWeights w, ws;
+    bool merged = false, has_residual = false, has_shared = false;
+    int64_t G = 0;
+    std::string name() const override { return "OptimusRoutedExpertsBackward"; }
+    variable_list run(variable_list &&grads) override {
+        const size_t n_in = 3 + leaves.size();
+        if (!grads[0].defined()) return variable_list(n_in);
+        const Call c = begin_call();
+        const Tensor dfinal = grads[0].contiguous();
+        // x, rw, row_weights, g, u, h [, shared g, u, h, cum], the index arrays' owners, the weights
+        const std::vector<Tensor> kept = saved();
+        const MlpState s{Tensor(), kept[3], kept[4], kept[5]};
+        size_t at = 6;
+        MlpState ss;
+        if (has_shared) {
+            ss = {kept[9], kept[6], kept[7], kept[8]};
+            at = 10;
+        }
+        Index index = ix;
+        index.owners.assign(kept.begin() + at, kept.begin() + kept.size() - leaves.size());
+        index.resolve();
+        const size_t n_routed = leaves.size() - (has_shared ? 3 : 0);
+        Tensor base;
+        Sinks ks;
+        if (has_shared) {   // first: its input gradient is the base of the routed experts' per-token sum
+            ks = sinks_of(c, leaves, true, n_routed, 1, ws);
+            base = merged_backward(c, dfinal, kept[0], ws, iptr(ss.cum), ss, nullptr, ks);
+        }
+        const Sinks k = sinks_of(c, leaves, merged, 0, G, w);
+        auto d = routed_backward(c, dfinal, kept[0], kept[1], index, w, s, kept[2], k, base);
+        variable_list out = {d.first, d.second, has_residual ? grads[0] : Tensor()};
+        out.reserve(n_in);
+        push_grads(out, k, merged, G, false);
+        if (has_shared) push_grads(out, ks, true, 1, true);
+        return out;
+    }
+};
+
+Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor &residual_in, bool merged,
+                      const std::vector<Tensor> &leaves, bool has_shared, const Tensor &one,
+                      const std::function<void(Index &)> &after_shared = nullptr) {
+    variable_list inputs = {x, rw, residual_in};
+    inputs.insert(inputs.end(), leaves.begin(), leaves.end());
+    const size_t n_routed = leaves.size() - (has_shared ? 3 : 0);
+    const int64_t G = merged ? leaves[0].size(0) : static_cast<int64_t>(n_routed / 3);
+    MlpWeights w, ws;
+    MlpState s, ss;
+    Tensor row_weights, final, xc, rwc;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        w = weights_of(leaves, merged, 0, G);
+        xc = x.contiguous();
+        rwc = rw.contiguous();
+        Tensor residual = residual_in.defined() ? residual_in.contiguous() : Tensor();
+        if (has_shared) {
+            ws = weights_of(leaves, true, n_routed, 1);
+            residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
+        }
+        if (after_shared) after_shared(ix);
+        final = routed_forward(c, xc, rwc, ix, w, residual, s, row_weights);
+    }
+    if (any_requires_grad(inputs)) {
+        auto node = make_node<RoutedNode>(inputs);
+        node->vars.reserve(16 + leaves.size());
+        node->save(xc.is_same(x) ? x : xc);
+        node->save(rwc.is_same(rw) ? rw : rwc);
+        for (const Tensor &t : {row_weights, s.g, s.u, s.h}) node->save(t);
+        if (has_shared)
+            for (const Tensor &t : {ss.g, ss.u, ss.h, one}) node->save(t);
+        for (const Tensor &t : ix.owners) node->save(t);
+        for (const Tensor &t : leaves) node->save(t);
+        ix.owners.clear();
+        node->ix = ix;
+        node->leaves = leaves;
+        node->w = w;
+        node->ws = ws;
+        node->merged = merged;
+        node->has_residual = residual_in.defined();
+        node->has_shared = has_shared;
+        node->G = G;
+        torch::autograd::set_history(final, node);
+    }
+    return final;
+}
+
+// RoutedMLPFunction / RoutedAndSharedMLPFunction over index arrays the caller has built
+Tensor routed_mlp(const Tensor &x, const Tensor &rw, const Tensor &in, const Tensor &cum_ep, const Tensor &out,
+                  const Tensor &sel, Tensor cum, const std::optional<Tensor> &residual, bool bound, bool merged,
+                  const std::vector<Tensor> &leaves, bool has_shared, const std::optional<Tensor> &one) {
+    const Call c = begin_call();
+    for (const Tensor *t : {&in, &cum_ep, &out, &sel}) require_device(*t);
+    if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
+    cum = cum.to(at::kInt).contiguous();
+    Index ix;
+    ix.owners = {cum, cum_ep, in, out, sel};
+    ix.resolve();
+    ix.rows = in.size(0);
+    ix.bound = bound;
+    return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, one.value_or(Tensor()));
+}
+
+// Activations of the expert MLP sized by the upper bound T*K instead of the routed rows of an expert
+// window cost expert_parallelism times their memory, and save the host the wait for the count.  Up to
+// this many bytes of them the wait costs more than the memory (a decode batch's are a few MB; 64 MB is
+// 0.02 % of the card).
+constexpr int64_t BOUND_ROWS_BYTES = 64 << 20;
+
+// One device integer on its way to the host.
+struct CountReadback {
+    Tensor value = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    hipEvent_t copied = nullptr;
+    CountReadback(const int32_t *device, void *stream) {
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        if (hipEventCreateWithFlags(&copied, hipEventDisableTiming) != hipSuccess ||
+            hipMemcpyAsync(value.data_ptr(), device, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
+            hipEventRecord(copied, st) != hipSuccess)
+            throw NativeError("reading the routed row count back failed");
+    }
+    CountReadback(const CountReadback &) = delete;
+    int64_t wait() {
+        py::gil_scoped_release nogil;
+        if (hipEventSynchronize(copied) != hipSuccess) throw NativeError("reading the routed row count back failed");
+        return value.data_ptr<int32_t>()[0];
+    }
+    ~CountReadback() {
+        if (copied) {
+            (void)hipEventSynchronize(copied);   // the pinned word may be handed out again
+            (void)hipEventDestroy(copied);
+        }
+    }
+};
+
+// Sort and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
+// sync_free: never read the routed-row count of an expert window back.
+Tensor moe_experts(const Tensor &x, const Tensor &rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
+                   bool sync_free, const std::optional<Tensor> &residual, bool merged, const std::vector<Tensor> &leaves,
+                   bool has_shared, const std::optional<Tensor> &one) {
+    const Call c = begin_call();
+    Index ix;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        ProfiledScope scope(c, "1moeblock--3index_calculation");
+        ix = sort_index(c, experts, start, end);
+    }
+    const bool windowed = !(start == 0 && end == n_total);
+    if (windowed) {
+        const int64_t I = leaves[0].size(-2), H = x.size(1);
+        if (sync_free || ix.rows * (3 * I + H) * 2 <= BOUND_ROWS_BYTES) {
+            ix.bound = true;
+        } else {
+            // read the count back (as the reference does), behind the shared expert's kernels: they do not
+            // need it, and while the GPU runs them the host waits for a copy that was enqueued before them
+            auto count = std::make_shared<CountReadback>(ix.cum + (end - start), c.stream);
+            return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared,
+                                  one.value_or(Tensor()), [count](Index &index) { index.rows = count->wait(); });
+        }
+    }
+    return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, one.value_or(Tensor()));
+}
+
+// The expert MLPs without routing weights (MergedMLPFunction, GroupMLPFunction and their gathered
+// forms).  Inputs in order: x, leaves.
+struct MergedNode : HostNode {
+    std::vector<Tensor> leaves;
+    MlpWeights w;
+    bool merged = false, single = false;
+    int64_t G = 0;
+    std::string name() const override { return "OptimusExpertMlpBackward"; }
+    variable_list run(variable_list &&grads) override {
+        if (!grads[0].defined()) return variable_list(1 + leaves.size());
+        const Call c = begin_call();
+        // x, cum, g, u, h, the gathered forms' index arrays (x_rows, cum_ep, out_rows), the weights
+        const std::vector<Tensor> kept = saved();
+        const Tensor &xs = kept[0];
+        const MlpState s{kept[1], kept[2], kept[3], kept[4]};
+        const Sinks k = sinks_of(c, leaves, merged, 0, G, w);
+        Tensor dx = merged_backward(c, grads[0], xs, w, iptr(s.cum), s, iptr(kept[5]), k);
+        if (kept[5].defined()) {
+            ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
+            Tensor sum = make(xs.sizes(), xs);
+            OM(c, om_shuffle_sub_matrix_reduce, ptr(dx), iptr(kept[6]), iptr(kept[7]), ptr(sum), xs.size(0), xs.size(1),
+               dtype_code(xs), c.stream);
+            dx = sum;
+        }
+        variable_list out = {dx};
+        out.reserve(1 + leaves.size());
+        push_grads(out, k, merged, G, single);
+        return out;
+    }
+};
+
+Tensor merged_mlp(const Tensor &x, Tensor cum, bool merged, const std::vector<Tensor> &leaves,
+                  const std::optional<Tensor> &x_rows, const std::optional<Tensor> &cum_ep,
+                  const std::optional<Tensor> &out_rows) {
+    variable_list inputs = {x};
+    inputs.insert(inputs.end(), leaves.begin(), leaves.end());
+    const int64_t G = merged ? 1 : static_cast<int64_t>(leaves.size() / 3);
+    MlpWeights w;
+    MlpState s;
+    Tensor y, xc = x;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
+        if (x_rows) xc = x.contiguous();
+        require_device(xc);
+        for (const auto *t : {&x_rows, &cum_ep, &out_rows}) require_device(t->value_or(Tensor()));
+        if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
+        s.cum = cum.to(at::kInt).contiguous();
+        w = weights_of(leaves, merged, 0, G);
+        y = merged_forward(c, xc, w, iptr(s.cum), x_rows ? iptr(*x_rows) : nullptr, x_rows ? x_rows->size(0) : xc.size(0), s);
+    }
+    if (any_requires_grad(inputs)) {
+        auto node = make_node<MergedNode>(inputs);
+        node->vars.reserve(8 + leaves.size());
+        node->save(xc.is_same(x) ? x : xc);
+        for (const Tensor &t : {s.cum, s.g, s.u, s.h}) node->save(t);
+        for (const auto *t : {&x_rows, &cum_ep, &out_rows}) node->save(t->value_or(Tensor()));
+        for (const Tensor &t : leaves) node->save(t);
+        node->leaves = leaves;
+        node->w = w;
+        node->merged = merged;
+        node->single = merged && leaves[0].dim() == 2;
+        node->G = G;
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
+// K6 (GroupGemmOutputReduction[Residual]Function): final[t] = (residual[t] +) sum_k w[t,k] y[pos(t,k)].
+struct CombineNode : HostNode {      // saves y, rw, sel, in, out
+    bool has_residual = false;
+    std::string name() const override { return "OptimusCombineBackward"; }
+    variable_list run(variable_list &&grads) override {
+        if (!grads[0].defined()) return variable_list(3);
+        const Call c = begin_call();
+        const std::vector<Tensor> kept = saved();
+        const Tensor dfinal = grads[0].contiguous();
+        const Tensor &ys = kept[0], &rws = kept[1], &sel = kept[2], &in = kept[3], &out = kept[4];
+        Tensor dy = make(ys.sizes(), ys);
+        // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window
+        // stay zero (the reference pre-zeroes the whole tensor, moe.py:336)
+        Tensor drw = out.size(0) == rws.numel() ? make(rws.sizes(), rws) : at::zeros(rws.sizes(), rws.options());
+        ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_bwd");
+        OM(c, om_reduce_ggemm_output_backward, ptr(dfinal), ptr(ys), ptr(rws), iptr(sel), iptr(in), iptr(out), ptr(dy),
+           ptr(drw), out.size(0), rws.size(1), dfinal.size(1), dtype_code(ys), dtype_code(rws), c.stream);
+        return {dy, drw, has_residual ? grads[0] : Tensor()};
+    }
+};
+
+Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const Tensor &sel, const Tensor &in,
+               const Tensor &out, const std::optional<Tensor> &residual) {
+    Tensor final, rw = rw_in;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
+        rw = rw_in.contiguous();
+        for (const Tensor *t : std::initializer_list<const Tensor *>{&y, &rw, &cum_ep, &sel, &in, &out}) require_device(*t);
+        const int64_t T = rw.size(0), K = rw.size(1), H = y.size(1);
+        ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_fwd");
+        final = make({T, H}, y);
+        if (residual) {
+            const Tensor res = residual->contiguous();
+            require_device(res);
+            OM(c, om_reduce_ggemm_output_residual, ptr(y), ptr(rw), iptr(cum_ep), iptr(sel), iptr(out), ptr(res), ptr(final),
+               T, K, H, dtype_code(y), dtype_code(rw), c.stream);
+        } else {
+            OM(c, om_reduce_ggemm_output, ptr(y), ptr(rw), iptr(cum_ep), iptr(sel), iptr(out), ptr(final), T, K, H,
+               dtype_code(y), dtype_code(rw), 0, c.stream);
+        }
+    }
+    if (any_requires_grad({y, rw_in, residual.value_or(Tensor())})) {
+        auto node = make_node<CombineNode>({y, rw_in, residual.value_or(Tensor())});
+        node->save(y);
+        node->save(rw.is_same(rw_in) ? rw_in : rw);
+        for (const Tensor &t : {sel, in, out}) node->save(t);
+        node->has_residual = residual.has_value();
+        torch::autograd::set_history(final, node);
+    }
+    return final;
+}
+
+// ---- Python module ----------------------------------------------------------------------------------
+
+// The (gate, up, down) weights of a ModuleList of expert MLPs in GroupMLPFunction's order.  Walks the
+// modules' dictionaries: nn.Module attribute access costs about a microsecond each, and a DeepSeek-V3
+// share has 96 of these.
+std::vector<Tensor> expert_parameters(py::handle experts) {
+    static PyObject *s_modules = PyUnicode_InternFromString("_modules"), *s_parameters = PyUnicode_InternFromString("_parameters"),
+                    *s_weight = PyUnicode_InternFromString("weight");
+    static PyObject *names[3] = {PyUnicode_InternFromString("gate_proj"), PyUnicode_InternFromString("up_proj"),
+                                 PyUnicode_InternFromString("down_proj")};
+    auto in_dict = [](py::handle owner, PyObject *dict_name, PyObject *key) -> py::object {   // null when absent
+        py::object d = py::reinterpret_steal<py::object>(PyObject_GetAttr(owner.ptr(), dict_name));
+        if (!d) throw py::error_already_set();
+        if (!PyDict_Check(d.ptr())) return py::object();
+        return py::reinterpret_borrow<py::object>(PyDict_GetItemWithError(d.ptr(), key));
+    };
+    std::vector<Tensor> out;
+    py::object children = experts.attr("_modules");
+    for (auto item : py::cast<py::dict>(children))
+        for (PyObject *name : names) {
+            py::object lin = in_dict(item.second, s_modules, name);
+            if (!lin) lin = py::getattr(item.second, name);
+            py::object weight = in_dict(lin, s_parameters, s_weight);
+            if (!weight) weight = lin.attr("weight");
+            out.push_back(weight.cast<Tensor>());
+        }
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    py::register_local_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (const NativeError &e) {
+            PyObject *cls = module_attr("optimus._native", "NativeLibraryError");
+            PyErr_SetString(cls, e.what());
+            Py_DECREF(cls);
+        }
+    });
+    m.def("build_token_permutation", [](const Tensor &experts, int64_t start, int64_t end) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto r = sort_tensors(begin_call(), experts, start, end);
+        return std::make_tuple(r[0], r[1], r[2], r[3], r[4]);
+    });
+    m.def("gate_logits", &gate_logits);
+    m.def("gate_weight_grad", [](const Tensor &x, const Tensor &w, const Tensor &dlogits) {
+        return gate_weight_grad(begin_call(), x, w, dlogits);
+    });
+    m.def("gate_input_grad", [](const Tensor &w, const Tensor &dlogits, const std::optional<Tensor> &other) {
+        return gate_input_grad(begin_call(), w, dlogits, other.value_or(Tensor()));
+    });
+    m.def("gate_backward", [](const Tensor &x, const Tensor &w, const Tensor &dlogits, bool need_x, bool need_w,
+                              const std::optional<Tensor> &other) {
+        return gate_backward(begin_call(), x, w, dlogits, need_x, need_w, other.value_or(Tensor()));
+    });
+    m.def("route_softmax", [](const Tensor &x, const Tensor &w, int64_t top_k, bool renorm, py::object dtype, bool fused,
+                              bool bf16_logits) {
+        return route_softmax(x, w, top_k, renorm, torch::python::detail::py_object_to_dtype(dtype), fused, bf16_logits);
+    });
+    m.def("route_sigmoid", &route_sigmoid);
+    m.def("routed_mlp", &routed_mlp);
+    m.def("moe_experts", &moe_experts);
+    m.def("merged_mlp", &merged_mlp);
+    m.def("combine", &combine);
+    m.def("expert_parameters", &expert_parameters);
+    m.def("constant_pitch", [](const std::vector<Tensor> &weights) {
+        at::NoGradGuard no_grad;
+        return weights.empty() || strided_view_or_undefined(weights.data(), 1, static_cast<int64_t>(weights.size())).defined();
+    });
+}

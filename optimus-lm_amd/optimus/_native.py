@@ -5,12 +5,14 @@ This is the only place that touches the library.  Tensors are passed as raw devi
 the library is missing or a call returns an error code, an exception is raised.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG_ROOT, "lib", "liboptimus_mi355x.so")
+HOST_PATH = os.path.join(_PKG_ROOT, "lib", "optimus_torch_host.so")
 
 OM_F32, OM_BF16 = 0, 1
 OM_I32, OM_I64 = 0, 1
@@ -145,6 +147,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 # Optional per-launch timing: when set to a list, every call of a kernel-launching entry point
 # appends (name, start_event, end_event) recorded on the current stream.  Used by bench.py to get
@@ -175,16 +178,29 @@ class _Library:
     @staticmethod
     def _maybe_timed(name, fn):
         def call(*args):
-            if launch_log is None or (launch_filter is not None and name not in launch_filter):
+            if launch_log is None:
                 return fn(*args)
-            a = torch.cuda.Event(enable_timing=True)
-            b = torch.cuda.Event(enable_timing=True)
-            a.record()
+            start = timed_begin(name)
             rc = fn(*args)
-            b.record()
-            launch_log.append((name, a, b))
+            timed_end(name, start)
             return rc
         return call
+
+
+def timed_begin(name):
+    """The start event of a launch of entry point `name`, or None when it is not timed."""
+    if launch_log is None or (launch_filter is not None and name not in launch_filter):
+        return None
+    start = torch.cuda.Event(enable_timing=True)
+    start.record()
+    return start
+
+
+def timed_end(name, start):
+    if start is not None:
+        end = torch.cuda.Event(enable_timing=True)
+        end.record()
+        launch_log.append((name, start, end))
 
 
 def lib():
@@ -197,6 +213,23 @@ def lib():
                 "(there is no non-HIP fallback)")
         _lib = _Library(ctypes.CDLL(LIB_PATH))
     return _lib
+
+
+def host():
+    """The C++ host module (csrc/host/torch_host.cpp): the blocks' allocations, launches and autograd
+    nodes.  Loaded once; raises if it has not been built."""
+    global _host
+    if _host is None:
+        if not os.path.exists(HOST_PATH):
+            raise NativeLibraryError(
+                f"{HOST_PATH} not found: build it with `python optimus-lm_amd/build.py` "
+                "(there is no non-native fallback)")
+        lib()      # (the module links against it)
+        spec = importlib.util.spec_from_file_location("optimus_torch_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def check(code, what):

@@ -143,35 +143,14 @@ def _gate_weight_grad(x, weight, dlogits):
     """dweight[n,h] = sum_t dlogits[t,n] x[t,h]: a long contraction with a tiny output, split
     over token ranges on the device (om_router_gate_wgrad) instead of a library GEMM that would
     run on a few CUs."""
-    _require_gate_shape(weight, 8, "gate weight gradient")
-    T, (N, H) = x.shape[0], weight.shape
-    lib = _n.lib()
-    ws_bytes = lib.om_router_gate_wgrad_workspace_bytes(T, H, N)
-    if ws_bytes < 0:
-        _n.check(int(ws_bytes), "om_router_gate_wgrad_workspace_bytes")
-    workspace = torch.empty(max(int(ws_bytes), 16), dtype=torch.uint8, device=x.device)
-    dw = torch.empty_like(weight)
-    dlogits = dlogits.contiguous()
-    _n.check(lib.om_router_gate_wgrad(_n.ptr(x), _n.ptr(dlogits), T, H, N, _n.ptr(dw), _n.dtype_code(dw),
-                                      _n.ptr(workspace), int(ws_bytes), _n.stream()),
-             "om_router_gate_wgrad")
-    return dw
+    return _n.host().gate_weight_grad(x, weight, dlogits)
 
 
 def _gate_input_grad(weight, dlogits, other_grad=None):
     """dx = bf16(dlogits) @ weight (om_router_gate_dgrad).  With `other_grad` [T,H] (the gradient
     that reached the same hidden states through the experts) the sum of the two is returned, formed
     inside the kernel with autograd's two roundings, so no separate accumulation pass runs."""
-    _require_gate_shape(weight, 8, "gate input gradient")
-    T, (N, H) = dlogits.shape[0], weight.shape
-    dlogits = dlogits.contiguous()
-    if other_grad is not None:
-        other_grad = other_grad.contiguous()
-        _require_bf16(other_grad)
-    dx = torch.empty((T, H), dtype=torch.bfloat16, device=dlogits.device)
-    _n.check(_n.lib().om_router_gate_dgrad(_n.ptr(dlogits), _n.ptr(weight), _n.ptr(other_grad), _n.ptr(dx),
-                                           T, H, N, _n.stream()), "om_router_gate_dgrad")
-    return dx
+    return _n.host().gate_input_grad(weight, dlogits, other_grad)
 
 
 def _gate_backward(x, weight, dlogits, needs, other_grad=None):
@@ -180,96 +159,22 @@ def _gate_backward(x, weight, dlogits, needs, other_grad=None):
     bf16 MFMA with fp32 accumulation: om_router_gate_dgrad and om_router_gate_wgrad.  `other_grad`
     is added to dx inside the kernel (see _gate_input_grad)."""
     _require_bf16(x, weight)
-    dlogits = dlogits.to(torch.float32)
-    dx = dw = None
-    if needs[0]:
-        dx = _gate_input_grad(weight, dlogits, other_grad)
-    if needs[1]:
-        dw = _gate_weight_grad(x, weight, dlogits)
-    return dx, dw
-
-
-class GateLogitsFunction(torch.autograd.Function):
-    """fp32 logits of a bf16 gate through om_router_gate_logits (one pass over x).  Returns
-    (logits, x): the second output is the input itself; a caller that feeds the rest of the layer
-    from it makes that part's input gradient arrive here, where the gate's own input gradient is
-    added to it inside om_router_gate_dgrad instead of by a separate accumulation pass."""
-
-    @staticmethod
-    def forward(ctx, x, weight):
-        T, (N, H) = x.shape[0], weight.shape
-        logits = torch.empty((T, N), dtype=torch.float32, device=x.device)
-        lib = _n.lib()
-        if N > 64 or H % 512 != 0:
-            # many experts: the weight no longer fits a block's re-reads; split over H instead
-            # (also the form for hidden sizes the one-pass kernel does not take)
-            ws_bytes = lib.om_router_gate_logits_split_workspace_bytes(T, H, N)
-            if ws_bytes < 0:
-                _n.check(int(ws_bytes), "om_router_gate_logits_split_workspace_bytes")
-            workspace = torch.empty(max(int(ws_bytes), 16), dtype=torch.uint8, device=x.device)
-            _n.check(lib.om_router_gate_logits_split(_n.ptr(x), _n.ptr(weight), T, H, N, _n.ptr(logits),
-                                                     _n.ptr(workspace), int(ws_bytes), _n.stream()),
-                     "om_router_gate_logits_split")
-        else:
-            _n.check(lib.om_router_gate_logits(_n.ptr(x), _n.ptr(weight), T, H, N, _n.ptr(logits),
-                                               _n.stream()), "om_router_gate_logits")
-        ctx.save_for_backward(x, weight)
-        ctx.set_materialize_grads(False)
-        return logits, x.view_as(x)
-
-    @staticmethod
-    def backward(ctx, dlogits, x_grad):
-        x, weight = ctx.saved_tensors
-        if dlogits is None:
-            return x_grad, None
-        return _gate_backward(x, weight, dlogits, ctx.needs_input_grad, other_grad=x_grad)
-
-
-class GateLogitsF32Function(torch.autograd.Function):
-    """logits = x @ weight.T for a float32 gate (om_router_gate_logits_f32) with both backward
-    products (om_router_gate_dgrad_f32, om_router_gate_wgrad_f32): the float32 module's gate without
-    a library GEMM."""
-
-    @staticmethod
-    def forward(ctx, x, weight):
-        _n.require_cuda_contiguous(x, weight)
-        T, (N, H) = x.shape[0], weight.shape
-        logits = torch.empty((T, N), dtype=torch.float32, device=x.device)
-        _n.check(_n.lib().om_router_gate_logits_f32(_n.ptr(x), _n.ptr(weight), T, H, N, _n.ptr(logits),
-                                                    _n.stream()), "om_router_gate_logits_f32")
-        ctx.save_for_backward(x, weight)
-        return logits
-
-    @staticmethod
-    def backward(ctx, dlogits):
-        x, weight = ctx.saved_tensors
-        T, (N, H) = x.shape[0], weight.shape
-        dlogits = dlogits.to(torch.float32).contiguous()
-        dx = dw = None
-        if ctx.needs_input_grad[0]:
-            dx = torch.empty_like(x)
-            _n.check(_n.lib().om_router_gate_dgrad_f32(_n.ptr(dlogits), _n.ptr(weight), T, H, N, _n.ptr(dx),
-                                                       _n.stream()), "om_router_gate_dgrad_f32")
-        if ctx.needs_input_grad[1]:
-            dw = torch.empty_like(weight)
-            _n.check(_n.lib().om_router_gate_wgrad_f32(_n.ptr(x), _n.ptr(dlogits), T, H, N, _n.ptr(dw),
-                                                       _n.stream()), "om_router_gate_wgrad_f32")
-        return dx, dw
+    return _n.host().gate_backward(x, weight, dlogits, needs[0], needs[1], other_grad)
 
 
 def fp32_logits_with_passthrough(x, weight):
     """(router logits in float32, x) from 2-D x [T,H] and weight [N,H] (the gate's nn.Linear weight).
     bf16 operands go through the gate kernels (at most 256 experts, H a multiple of 8; anything
-    else raises), and the returned x is GateLogitsFunction's pass-through; a float32 module's gate
-    runs on the plain float32 gate kernels (GateLogitsF32Function) and x comes back as it is."""
+    else raises), a float32 module's on the plain float32 gate kernels.  The second result is the input
+    itself; a caller that feeds the rest of the layer from it makes that part's input gradient arrive at
+    the gate, where the gate's own is added to it."""
     if x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16:
-        _n.require_cuda_contiguous(x.contiguous(), weight.contiguous())
         # (the forward and the two backward kernels take the same shapes, so a shape that passes here
         # passes in backward)
         _require_gate_shape(weight, 8, "gate projection")
-        return GateLogitsFunction.apply(x.contiguous(), weight.contiguous())
+        return _n.host().gate_logits(x.contiguous(), weight.contiguous())
     if x.dtype == torch.float32 and weight.dtype == torch.float32:
-        return GateLogitsF32Function.apply(x.contiguous(), weight.contiguous()), x
+        return _n.host().gate_logits(x.contiguous(), weight.contiguous())
     raise TypeError(f"router gate: activations and weight must both be bfloat16 or both float32 "
                     f"(got {x.dtype}, {weight.dtype})")
 
@@ -294,14 +199,32 @@ def gate_logits_with_passthrough(x, gate):
         logits, x = fp32_logits_with_passthrough(x, gate.weight)
         return logits.to(torch.bfloat16), x
     if x.dtype == torch.float32 and gate.weight.dtype == torch.float32 and x.is_cuda and gate.bias is None:
-        return fp32_logits(x, gate.weight), x
+        return fp32_logits_with_passthrough(x, gate.weight)
     return gate(x), x
 
 
-class GateSoftmaxTopkFunction(torch.autograd.Function):
+class GateLogitsFunction:
+    """apply(x, weight) -> (fp32 logits of a bf16 gate, x); see fp32_logits_with_passthrough."""
+
+    @staticmethod
+    def apply(x, weight):
+        return _n.host().gate_logits(x, weight)
+
+
+class GateLogitsF32Function:
+    """apply(x, weight) -> logits = x @ weight.T for a float32 gate (om_router_gate_logits_f32, with both
+    backward products on the float32 gate kernels)."""
+
+    @staticmethod
+    def apply(x, weight):
+        return _n.host().gate_logits(x, weight)[0]
+
+
+class GateSoftmaxTopkFunction:
     """The OLMoE router in one launch (om_router_gate_softmax_topk): gate projection with fp32
-    logits, softmax, top-K, optional renormalisation.  Returns (routing_weights, selected_experts,
-    router_logits fp32, hidden_states); reference moe.py:456 and :467-471.
+    logits, softmax, top-K, optional renormalisation.  apply(x, weight, top_k, norm_topk_prob, out_dtype)
+    returns (routing_weights, selected_experts, router_logits fp32, hidden_states); reference
+    moe.py:456 and :467-471.
 
     The fourth output is the input itself.  A caller that feeds the experts from it (instead of from
     the tensor it passed in) makes the experts' input gradient arrive here, where the gate's own
@@ -309,44 +232,8 @@ class GateSoftmaxTopkFunction(torch.autograd.Function):
     matmul output plus autograd's accumulation kernel."""
 
     @staticmethod
-    def forward(ctx, x, weight, top_k, norm_topk_prob, out_dtype):
-        T, (N, H) = x.shape[0], weight.shape
-        dev = x.device
-        logits = torch.empty((T, N), dtype=torch.float32, device=dev)
-        weights = torch.empty((T, top_k), dtype=out_dtype, device=dev)
-        experts = torch.empty((T, top_k), dtype=torch.int64, device=dev)
-        _n.check(_n.lib().om_router_gate_softmax_topk(
-            _n.ptr(x), _n.ptr(weight), T, H, N, top_k, int(bool(norm_topk_prob)), _n.ptr(logits),
-            _n.ptr(weights), _n.dtype_code(weights), _n.ptr(experts), _n.stream()),
-            "om_router_gate_softmax_topk")
-        ctx.save_for_backward(x, weight, logits, experts)
-        ctx.norm_topk_prob = bool(norm_topk_prob)
-        ctx.mark_non_differentiable(experts)
-        # an output nobody differentiates (the logits without an auxiliary loss) arrives as None in
-        # backward instead of a tensor of zeros that would have to be filled and added
-        ctx.set_materialize_grads(False)
-        return weights, experts, logits, x.view_as(x)
-
-    @staticmethod
-    def backward(ctx, weights_grad, _experts_grad, logits_grad, x_grad):
-        x, weight, logits, experts = ctx.saved_tensors
-        T, N = logits.shape
-        K = experts.shape[1]
-        if weights_grad is None and logits_grad is None:
-            return x_grad, None, None, None, None
-        if weights_grad is None:
-            dlogits = logits_grad.to(torch.float32).contiguous()
-        else:
-            weights_grad = weights_grad.contiguous()
-            dlogits = torch.empty_like(logits)
-            _n.check(_n.lib().om_route_softmax_topk_bwd(
-                _n.ptr(logits), _n.OM_F32, _n.ptr(experts), _n.ptr(weights_grad),
-                _n.dtype_code(weights_grad), T, N, K, int(ctx.norm_topk_prob), _n.ptr(dlogits),
-                _n.stream()), "om_route_softmax_topk_bwd")
-            if logits_grad is not None:
-                dlogits = dlogits + logits_grad
-        dx, dw = _gate_backward(x, weight, dlogits, ctx.needs_input_grad, other_grad=x_grad)
-        return dx, dw, None, None, None
+    def apply(x, weight, top_k, norm_topk_prob, out_dtype):
+        return _n.host().route_softmax(x, weight, top_k, bool(norm_topk_prob), out_dtype, True, False)
 
 
 class SoftmaxTopkRouterFunction(torch.autograd.Function):
@@ -393,24 +280,7 @@ def build_token_permutation(selected_experts, expert_start_idx, expert_end_idx):
     input_indices, output_indices, selected_experts_indices) — the last three sized T*K; only
     the first cum_token_counts[-1] entries are meaningful.  Same values as the reference's
     K1 -> cumsum -> K3 sequence (moe.py:499-554).  Nothing is copied to the host."""
-    _n.require_cuda_contiguous(selected_experts)
-    T, K = selected_experts.shape
-    NR = expert_end_idx - expert_start_idx
-    dev = selected_experts.device
-    i32 = dict(dtype=torch.int32, device=dev)
-    cum_token_counts = torch.empty(NR + 1, **i32)
-    cum_expert_counts_ep = torch.empty(T + 1, **i32)
-    input_indices = torch.empty(T * K, **i32)
-    output_indices = torch.empty(T * K, **i32)
-    selected_experts_indices = torch.empty(T * K, **i32)
-    ws_bytes = _n.lib().om_moe_sort_workspace_bytes(T, K, NR)
-    workspace = torch.empty(max(ws_bytes // 4, 1), **i32)
-    _n.check(_n.lib().om_moe_sort(
-        _n.ptr(selected_experts), _n.index_code(selected_experts), T, K, int(expert_start_idx),
-        int(expert_end_idx), _n.ptr(cum_token_counts), _n.ptr(cum_expert_counts_ep),
-        _n.ptr(input_indices), _n.ptr(output_indices), _n.ptr(selected_experts_indices),
-        _n.ptr(workspace), ws_bytes, _n.stream()), "om_moe_sort")
-    return cum_token_counts, cum_expert_counts_ep, input_indices, output_indices, selected_experts_indices
+    return _n.host().build_token_permutation(selected_experts, int(expert_start_idx), int(expert_end_idx))
 
 
 # ----------------------------------------------------------------------------------------------
@@ -440,32 +310,6 @@ def _live_grad(param):
     if param._backward_hooks or getattr(param, "_post_accumulate_grad_hooks", None):
         return None
     return grad
-
-
-def _grad_sink(leaves):
-    """[G, out, in] tensor over the live gradient buffer(s) of an expert weight, or None.  `leaves`
-    is the parameter itself ([G, out, in], or [out, in] for a single MLP) or the list of the G
-    per-expert [out, in] parameters, whose gradients must then lie at one constant pitch inside one
-    buffer (true when they are views of a flat gradient buffer in parameter order)."""
-    if isinstance(leaves, (list, tuple)):
-        grads = [_live_grad(w) for w in leaves]
-        if any(g is None for g in grads):
-            return None
-        try:
-            return _strided_expert_view(grads)
-        except _n.NativeLibraryError:
-            return None
-    grad = _live_grad(leaves)
-    if grad is not None and grad.dim() == 2:
-        grad = grad.unsqueeze(0)
-    return grad
-
-
-def _weight_grad_out(sink, shape, like):
-    """-> (tensor the weight-gradient GEMM writes, its expert pitch argument, accumulate flag)."""
-    if sink is not None:
-        return sink, _expert_stride(sink), True
-    return torch.empty(shape, dtype=like.dtype, device=like.device), 0, False
 
 
 # ----------------------------------------------------------------------------------------------
@@ -498,8 +342,11 @@ class GroupedGemmFunction(torch.autograd.Function):
         num_experts, ofm, ifm = merged_weight.shape
         rows = input.shape[0]
         input_grad = torch.empty_like(input)
-        weight_grad, pitch, acc = _weight_grad_out(_grad_sink(merged_weight), (num_experts, ofm, ifm),
-                                                   merged_weight)
+        weight_grad = _live_grad(merged_weight)
+        acc = weight_grad is not None
+        if not acc:
+            weight_grad = torch.empty((num_experts, ofm, ifm), dtype=merged_weight.dtype, device=merged_weight.device)
+        pitch = _expert_stride(weight_grad)
         _grouped_gemm("dgrad", output_grad, merged_weight, input_grad, cum, rows, num_experts, ofm, ifm,
                       _expert_stride(merged_weight))
         _grouped_gemm("wgrad", output_grad, input, weight_grad, cum, rows, num_experts, ofm, ifm, pitch,
@@ -507,180 +354,23 @@ class GroupedGemmFunction(torch.autograd.Function):
         return input_grad, (None if acc else weight_grad), None, None, None
 
 
-def _merged_mlp_forward(x, w_gate, w_up, w_down, cum_token_counts, x_rows=None):
-    """-> (y, cum, g, u, h).  Fused gate+up+SwiGLU launch, then the down projection.  With
-    `x_rows` (int32 [rows]) the MLP input is x[x_rows] without that matrix being built."""
-    if _gemm_dtype(x, w_gate, w_up, w_down) == torch.float32:
-        return _merged_mlp_forward_f32(x, w_gate, w_up, w_down, cum_token_counts, x_rows)
-    _n.require_cuda_contiguous(x, x_rows)
-    rows, H = x.shape
-    if x_rows is not None:
-        rows = x_rows.shape[0]
-    G, I, _ = w_gate.shape
-    cum = _device_counts(cum_token_counts, x.device)
-    g = torch.empty((rows, I), dtype=x.dtype, device=x.device)
-    u = torch.empty_like(g)
-    h = torch.empty_like(g)
-    y = torch.empty((rows, H), dtype=x.dtype, device=x.device)
-    lib = _n.lib()
-    sgu = _expert_stride(w_gate)
-    if _expert_stride(w_up) != sgu:
-        raise _n.NativeLibraryError("gate and up expert weights must share one expert pitch")
-    with record_pcl_function("1moeblock--7gmlp_fwd"):
-        if x_rows is not None and rows > 0:
-            _n.check(lib.om_merged_mlp_gate_up_fwd_gathered(
-                _n.ptr(x), _n.ptr(x_rows), x.shape[0], _n.ptr(w_gate), _n.ptr(w_up), _n.ptr(g),
-                _n.ptr(u), _n.ptr(h), _n.ptr(cum), rows, G, I, H, sgu, _n.stream()),
-                "om_merged_mlp_gate_up_fwd_gathered")
-        else:
-            _n.check(lib.om_merged_mlp_gate_up_fwd(
-                _n.ptr(x), _n.ptr(w_gate), _n.ptr(w_up), _n.ptr(g), _n.ptr(u), _n.ptr(h), _n.ptr(cum),
-                rows, G, I, H, sgu, _n.stream()), "om_merged_mlp_gate_up_fwd")
-        _n.check(lib.om_grouped_gemm_fwd(
-            _n.ptr(h), _n.ptr(w_down), _n.ptr(y), _n.ptr(cum), rows, G, H, I,
-            _expert_stride(w_down), _n.stream()), "om_grouped_gemm_fwd")
-    return y, cum, g, u, h
-
-
-def _gathered_rows(x, x_rows):
-    if x_rows is None:
-        return x
-    out = torch.empty((x_rows.shape[0], x.shape[1]), dtype=x.dtype, device=x.device)
-    pcl_xpu_customops.index_gather(x, x_rows, out)
-    return out
-
-
-def _merged_mlp_forward_f32(x, w_gate, w_up, w_down, cum_token_counts, x_rows=None):
-    """float32 modules: the reference's own sequence (moe.py:396-405), three grouped GEMMs and the
-    SwiGLU glue kernel, on the plain fp32 kernels; nothing is fused."""
-    _n.require_cuda_contiguous(x, x_rows)
-    xs = _gathered_rows(x, x_rows)
-    rows, H = xs.shape
-    G, I, _ = w_gate.shape
-    cum = _device_counts(cum_token_counts, x.device)
-    g = torch.empty((rows, I), dtype=x.dtype, device=x.device)
-    u = torch.empty_like(g)
-    h = torch.empty_like(g)
-    y = torch.empty((rows, H), dtype=x.dtype, device=x.device)
-    with record_pcl_function("1moeblock--7gmlp_fwd"):
-        _grouped_gemm("fwd", xs, w_gate, g, cum, rows, G, I, H, _expert_stride(w_gate))
-        _grouped_gemm("fwd", xs, w_up, u, cum, rows, G, I, H, _expert_stride(w_up))
-        if rows:
-            _n.check(_n.lib().om_swiglu_fwd(_n.ptr(g), _n.ptr(u), _n.ptr(h), rows * I, _n.OM_F32, _n.stream()),
-                     "om_swiglu_fwd")
-        _grouped_gemm("fwd", h, w_down, y, cum, rows, G, H, I, _expert_stride(w_down))
-    return y, cum, g, u, h
-
-
-def _merged_mlp_backward_f32(dy, x, w_gate, w_up, w_down, cum, g, u, h, x_rows=None,
-                             sinks=(None, None, None)):
-    dy = dy.contiguous()
-    xs = _gathered_rows(x, x_rows)
-    rows, H = dy.shape
-    G, I, _ = w_gate.shape
-    new = lambda *shape: torch.empty(shape, dtype=x.dtype, device=x.device)
-    dh, dg, du, dx, dx2 = new(rows, I), new(rows, I), new(rows, I), new(rows, H), new(rows, H)
-    (dw_gate, sg, ag), (dw_up, su, au), (dw_down, sd, ad) = (
-        _weight_grad_out(sinks[0], (G, I, H), x), _weight_grad_out(sinks[1], (G, I, H), x),
-        _weight_grad_out(sinks[2], (G, H, I), x))
-    with record_pcl_function("1moeblock--7gmlp_bwd"):
-        _grouped_gemm("wgrad", dy, h, dw_down, cum, rows, G, H, I, sd, accumulate=ad)
-        _grouped_gemm("dgrad", dy, w_down, dh, cum, rows, G, H, I, _expert_stride(w_down))
-        if rows:
-            _n.check(_n.lib().om_swiglu_bwd(_n.ptr(dh), _n.ptr(g), _n.ptr(u), _n.ptr(dg), _n.ptr(du), rows * I,
-                                            _n.OM_F32, _n.stream()), "om_swiglu_bwd")
-        _grouped_gemm("wgrad", dg, xs, dw_gate, cum, rows, G, I, H, sg, accumulate=ag)
-        _grouped_gemm("wgrad", du, xs, dw_up, cum, rows, G, I, H, su, accumulate=au)
-        _grouped_gemm("dgrad", dg, w_gate, dx, cum, rows, G, I, H, _expert_stride(w_gate))
-        _grouped_gemm("dgrad", du, w_up, dx2, cum, rows, G, I, H, _expert_stride(w_up))
-        dx += dx2
-    return dx, (None if ag else dw_gate), (None if au else dw_up), (None if ad else dw_down)
-
-
-def _wgrad(output_grad, input, weight_grad, cum, rows, G, N, K, pitch, accumulate, what,
-           input_rows=None, output_grad_rows=None, src_rows=0):
-    """One of the bf16 weight-gradient entry points: plain, with the rows of `input` or of
-    `output_grad` taken through an index, each writing or (accumulate) adding into weight_grad."""
-    lib, st = _n.lib(), _n.stream()
-    tail = "_accumulate" if accumulate else ""
-    if input_rows is not None:
-        name = "om_grouped_gemm_wgrad_gathered" + tail
-        rc = getattr(lib, name)(_n.ptr(output_grad), _n.ptr(input), _n.ptr(input_rows), src_rows,
-                                _n.ptr(weight_grad), _n.ptr(cum), rows, G, N, K, pitch, st)
-    elif output_grad_rows is not None:
-        name = "om_grouped_gemm_wgrad_gathered_out" + tail
-        rc = getattr(lib, name)(_n.ptr(output_grad), _n.ptr(output_grad_rows), src_rows, _n.ptr(input),
-                                _n.ptr(weight_grad), _n.ptr(cum), rows, G, N, K, pitch, st)
-    else:
-        name = "om_grouped_gemm_wgrad" + tail
-        rc = getattr(lib, name)(_n.ptr(output_grad), _n.ptr(input), _n.ptr(weight_grad), _n.ptr(cum), rows,
-                                G, N, K, pitch, st)
-    _n.check(rc, f"{name}({what})")
-
-
-def _merged_mlp_backward(dy, x, w_gate, w_up, w_down, cum, g, u, h, x_rows=None, sinks=(None, None, None)):
-    """-> (dx, dw_gate [G,I,H], dw_up [G,I,H], dw_down [G,H,I]).  With `x_rows` the MLP input was
-    x[x_rows]; dx is then the gradient of that gathered matrix.  `sinks` (gate, up, down): a weight
-    whose entry is a tensor gets its gradient added into that tensor by the GEMM and None returned;
-    the others get a freshly allocated gradient."""
-    if x.dtype == torch.float32:
-        return _merged_mlp_backward_f32(dy, x, w_gate, w_up, w_down, cum, g, u, h, x_rows, sinks)
-    dy = dy.contiguous()
-    rows, H = dy.shape
-    G, I, _ = w_gate.shape
-    lib = _n.lib()
-    st = _n.stream()
-    dg = torch.empty_like(g)
-    du = torch.empty_like(u)
-    dx = torch.empty((rows, H), dtype=x.dtype, device=x.device)
-    (dw_gate, sg, ag), (dw_up, su, au), (dw_down, sd, ad) = (
-        _weight_grad_out(sinks[0], (G, I, H), x), _weight_grad_out(sinks[1], (G, I, H), x),
-        _weight_grad_out(sinks[2], (G, H, I), x))
-    with record_pcl_function("1moeblock--7gmlp_bwd"):
-        _wgrad(dy, h, dw_down, cum, rows, G, H, I, sd, ad, "down")
-        _n.check(lib.om_merged_mlp_down_dgrad(_n.ptr(dy), _n.ptr(w_down), _n.ptr(g), _n.ptr(u),
-                                              _n.ptr(dg), _n.ptr(du), _n.ptr(cum), rows, G, I, H,
-                                              _expert_stride(w_down), st), "om_merged_mlp_down_dgrad")
-        gathered = dict(input_rows=x_rows, src_rows=x.shape[0]) if (x_rows is not None and rows > 0) else {}
-        _wgrad(dg, x, dw_gate, cum, rows, G, I, H, sg, ag, "gate", **gathered)
-        _wgrad(du, x, dw_up, cum, rows, G, I, H, su, au, "up", **gathered)
-        _n.check(lib.om_merged_mlp_gate_up_dgrad(_n.ptr(dg), _n.ptr(du), _n.ptr(w_gate),
-                                                 _n.ptr(w_up), _n.ptr(dx), _n.ptr(cum), rows, G,
-                                                 I, H, _expert_stride(w_gate), st),
-                 "om_merged_mlp_gate_up_dgrad")
-    return dx, (None if ag else dw_gate), (None if au else dw_up), (None if ad else dw_down)
-
-
-class MergedMLPFunction(torch.autograd.Function):
+class MergedMLPFunction:
     """y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment, with the fused kernels:
     gate+up+SwiGLU in one launch forward; backward = down dgrad fused with the SwiGLU backward,
     one dual-operand dgrad for dx, and three weight-gradient GEMMs.
 
     Same mathematics as the three GroupedGemmFunction calls and two elementwise ops of the
     reference's MergedMLP.forward (moe.py:396-405) under autograd; g and u are kept in bf16 for
-    the backward like the reference keeps output_gproj / output_uproj."""
+    the backward like the reference keeps output_gproj / output_uproj.  float32 modules run the
+    reference's own sequence on the plain fp32 kernels."""
 
     @staticmethod
-    def forward(ctx, x, w_gate, w_up, w_down, cum_token_counts):
+    def apply(x, w_gate, w_up, w_down, cum_token_counts):
         # a single MLP may hand its three [out, in] weights over as they are
-        ctx.leaves = (w_gate, w_up, w_down)
-        ctx.single = w_gate.dim() == 2
-        if ctx.single:
-            w_gate, w_up, w_down = w_gate.unsqueeze(0), w_up.unsqueeze(0), w_down.unsqueeze(0)
-        y, cum, g, u, h = _merged_mlp_forward(x, w_gate, w_up, w_down, cum_token_counts)
-        ctx.save_for_backward(x, w_gate, w_up, w_down, cum, g, u, h)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        sinks = tuple(_grad_sink(w) for w in ctx.leaves)
-        dx, *dws = _merged_mlp_backward(dy, *ctx.saved_tensors, sinks=sinks)
-        if ctx.single:
-            dws = [None if dw is None else dw[0] for dw in dws]
-        return (dx, *dws, None)
+        return _n.host().merged_mlp(x, cum_token_counts, True, [w_gate, w_up, w_down], None, None, None)
 
 
-class GatheredMergedMLPFunction(torch.autograd.Function):
+class GatheredMergedMLPFunction:
     """PrepareInputForGroupGemmFunction followed by MergedMLPFunction (reference moe.py:217-282 and
     :396-405) without the gathered copy of the activations: the gate/up forward GEMM and the two
     gate/up weight-gradient GEMMs read hidden_states through input_indices.  Bit-identical to the
@@ -688,102 +378,38 @@ class GatheredMergedMLPFunction(torch.autograd.Function):
     gradients (shuffle_sub_matrix_reduce)."""
 
     @staticmethod
-    def forward(ctx, hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate, w_up,
-                w_down, cum_token_counts):
-        hidden_states = hidden_states.contiguous()
-        y, cum, g, u, h = _merged_mlp_forward(hidden_states, w_gate, w_up, w_down, cum_token_counts,
-                                              x_rows=input_indices)
-        ctx.save_for_backward(hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate,
-                              w_up, w_down, cum, g, u, h)
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        (hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate, w_up, w_down, cum,
-         g, u, h) = ctx.saved_tensors
-        sinks = tuple(_grad_sink(w) for w in (w_gate, w_up, w_down))
-        dx_rows, dw_gate, dw_up, dw_down = _merged_mlp_backward(dy, hidden_states, w_gate, w_up, w_down,
-                                                                cum, g, u, h, x_rows=input_indices,
-                                                                sinks=sinks)
-        with record_pcl_function("1moeblock--6gmlp_input_prep_bwd"):
-            hidden_states_grad = torch.empty_like(hidden_states)
-            pcl_xpu_customops.shuffle_sub_matrix_reduce(dx_rows, cum_expert_counts_ep, output_indices,
-                                                        hidden_states_grad)
-        return hidden_states_grad, None, None, None, dw_gate, dw_up, dw_down, None
+    def apply(hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate, w_up, w_down,
+              cum_token_counts):
+        return _n.host().merged_mlp(hidden_states, cum_token_counts, True, [w_gate, w_up, w_down],
+                                    input_indices, cum_expert_counts_ep, output_indices)
 
 
-def _per_expert_leaves(weight_tuple):
-    """(gate, up, down) lists of the per-expert parameters of a (gate_0, up_0, down_0, gate_1, ...)
-    tuple."""
-    N = len(weight_tuple) // 3
-    return tuple([weight_tuple[3 * n + j] for n in range(N)] for j in range(3))
-
-
-def _per_expert_grads(dwg, dwu, dwd, G):
-    """Gradients in the (gate_0, up_0, down_0, gate_1, ...) order of the inputs; None for a
-    projection whose gradient went into its live buffer."""
-    flat = []
-    for n in range(G):
-        flat += [None if dw is None else dw[n] for dw in (dwg, dwu, dwd)]
-    return flat
-
-
-class GroupMLPFunction(torch.autograd.Function):
+class GroupMLPFunction:
     """Un-merged layout of the reference (moe.py:43-161): weights arrive as 3*N separate
     [out, in] tensors (gate_0, up_0, down_0, gate_1, ...).  They must sit at one constant pitch
     inside a single buffer (true for parameters re-pointed into MixedPrecisionAdamW.flat_param and
     after pack_expert_weights); the same fused kernels then run on strided views, no copies."""
 
     @staticmethod
-    def forward(ctx, input, cum_token_counts, use_triton_path, *weight_tuple):
-        ctx.leaves = _per_expert_leaves(weight_tuple)
-        wg, wu, wd = [_strided_expert_view(ws) for ws in ctx.leaves]
-        y, cum, g, u, h = _merged_mlp_forward(input, wg, wu, wd, cum_token_counts)
-        ctx.save_for_backward(input, wg, wu, wd, cum, g, u, h)
-        return y
-
-    @staticmethod
-    def backward(ctx, output_grad):
-        sinks = tuple(_grad_sink(ws) for ws in ctx.leaves)
-        dx, dwg, dwu, dwd = _merged_mlp_backward(output_grad, *ctx.saved_tensors, sinks=sinks)
-        return (dx, None, None, *_per_expert_grads(dwg, dwu, dwd, len(ctx.leaves[0])))
+    def apply(input, cum_token_counts, use_triton_path, *weight_tuple):
+        return _n.host().merged_mlp(input, cum_token_counts, False, list(weight_tuple), None, None, None)
 
 
-class GatheredGroupMLPFunction(torch.autograd.Function):
+class GatheredGroupMLPFunction:
     """GroupMLPFunction on hidden_states[input_indices] without the gathered copy (see
     GatheredMergedMLPFunction); weights as in GroupMLPFunction."""
 
     @staticmethod
-    def forward(ctx, hidden_states, input_indices, cum_expert_counts_ep, output_indices, cum_token_counts,
-                *weight_tuple):
-        ctx.leaves = _per_expert_leaves(weight_tuple)
-        wg, wu, wd = [_strided_expert_view(ws) for ws in ctx.leaves]
-        hidden_states = hidden_states.contiguous()
-        y, cum, g, u, h = _merged_mlp_forward(hidden_states, wg, wu, wd, cum_token_counts,
-                                              x_rows=input_indices)
-        ctx.save_for_backward(hidden_states, input_indices, cum_expert_counts_ep, output_indices, wg, wu,
-                              wd, cum, g, u, h)
-        return y
-
-    @staticmethod
-    def backward(ctx, output_grad):
-        (hidden_states, input_indices, cum_expert_counts_ep, output_indices, wg, wu, wd, cum, g, u,
-         h) = ctx.saved_tensors
-        sinks = tuple(_grad_sink(ws) for ws in ctx.leaves)
-        dx_rows, dwg, dwu, dwd = _merged_mlp_backward(output_grad, hidden_states, wg, wu, wd, cum, g, u, h,
-                                                      x_rows=input_indices, sinks=sinks)
-        with record_pcl_function("1moeblock--6gmlp_input_prep_bwd"):
-            hidden_states_grad = torch.empty_like(hidden_states)
-            pcl_xpu_customops.shuffle_sub_matrix_reduce(dx_rows, cum_expert_counts_ep, output_indices,
-                                                        hidden_states_grad)
-        return (hidden_states_grad, None, None, None, None,
-                *_per_expert_grads(dwg, dwu, dwd, len(ctx.leaves[0])))
+    def apply(hidden_states, input_indices, cum_expert_counts_ep, output_indices, cum_token_counts,
+              *weight_tuple):
+        return _n.host().merged_mlp(hidden_states, cum_token_counts, False, list(weight_tuple),
+                                    input_indices, cum_expert_counts_ep, output_indices)
 
 
 def routed_mlp_unfit_reason(hidden_states, routing_weights, w_gate, w_down):
     """None when RoutedMLPFunction's kernels take these operands (bf16 activations and expert
     weights on the GPU, fp32 or bf16 routing weights, H and I multiples of 8), else why not."""
-    G, I, H = w_gate.shape
+    I, H = w_gate.shape[-2:]
     if not (hidden_states.is_cuda and hidden_states.dim() == 2):
         return "the hidden states are not a 2-D device tensor"
     if not (hidden_states.dtype == torch.bfloat16 and w_gate.dtype == torch.bfloat16
@@ -801,117 +427,7 @@ def routed_mlp_kernel_fits(hidden_states, routing_weights, w_gate, w_down):
     return routed_mlp_unfit_reason(hidden_states, routing_weights, w_gate, w_down) is None
 
 
-def _routed_mlp_forward(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                        output_indices, selected_experts_indices, w_gate, w_up, w_down,
-                        cum_token_counts, residual):
-    """-> (final [T,H], cum, g, u, h, row_weights): gather, weighted SwiGLU MLP, unweighted sum."""
-    _n.require_cuda_contiguous(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                               output_indices, selected_experts_indices, residual)
-    _require_bf16(hidden_states, w_gate, w_up, w_down)
-    T, H = hidden_states.shape
-    K = routing_weights.shape[1]
-    rows = input_indices.shape[0]
-    G, I, _ = w_gate.shape
-    dev, dt = hidden_states.device, hidden_states.dtype
-    cum = _device_counts(cum_token_counts, dev)
-    lib, st = _n.lib(), _n.stream()
-    sgu = _expert_stride(w_gate)
-    if _expert_stride(w_up) != sgu:
-        raise _n.NativeLibraryError("gate and up expert weights must share one expert pitch")
-    row_weights = torch.empty((rows,), dtype=torch.float32, device=dev)
-    g = torch.empty((rows, I), dtype=dt, device=dev)
-    u = torch.empty_like(g)
-    h = torch.empty_like(g)
-    y = torch.empty((rows, H), dtype=dt, device=dev)
-    final = torch.empty((T, H), dtype=dt, device=dev)
-    with record_pcl_function("1moeblock--7gmlp_fwd"):
-        _n.check(lib.om_moe_row_weights(
-            _n.ptr(routing_weights), _n.ptr(selected_experts_indices), _n.ptr(input_indices),
-            _n.ptr(output_indices), _n.ptr(row_weights), rows, K, _n.dtype_code(routing_weights), st),
-            "om_moe_row_weights")
-        _n.check(lib.om_merged_mlp_gate_up_fwd_weighted(
-            _n.ptr(hidden_states), _n.ptr(input_indices), T, _n.ptr(w_gate), _n.ptr(w_up),
-            _n.ptr(row_weights), _n.ptr(g), _n.ptr(u), _n.ptr(h), _n.ptr(cum), rows, G, I, H, sgu, st),
-            "om_merged_mlp_gate_up_fwd_weighted")
-        _n.check(lib.om_grouped_gemm_fwd(
-            _n.ptr(h), _n.ptr(w_down), _n.ptr(y), _n.ptr(cum), rows, G, H, I, _expert_stride(w_down), st),
-            "om_grouped_gemm_fwd")
-    with record_pcl_function("1moeblock--8gmlp_output_reduction_fwd"):
-        _n.check(lib.om_sum_ggemm_output(
-            _n.ptr(y), _n.ptr(cum_expert_counts_ep), _n.ptr(output_indices), _n.ptr(residual),
-            _n.ptr(final), T, H, _n.dtype_code(final), st), "om_sum_ggemm_output")
-    return final, cum, g, u, h, row_weights
-
-
-def _routed_mlp_backward(dfinal, hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                         output_indices, selected_experts_indices, w_gate, w_up, w_down, cum, g, u, h,
-                         row_weights, sinks=(None, None, None), base=None, rows_is_bound=False):
-    """-> (hidden_states_grad, routing_weights_grad, dw_gate, dw_up, dw_down); `sinks` as in
-    _merged_mlp_backward.  `base` [T,H]: another gradient of the same hidden states, added to the
-    result inside the per-token sum (base + cast(sum of the token's rows): autograd's bits).
-    `rows_is_bound`: the index arrays are sized by an upper bound of the routed rows."""
-    dfinal = dfinal.contiguous()
-    T, H = hidden_states.shape
-    K = routing_weights.shape[1]
-    rows = input_indices.shape[0]
-    G, I, _ = w_gate.shape
-    dev, dt = hidden_states.device, hidden_states.dtype
-    lib, st = _n.lib(), _n.stream()
-    dg = torch.empty_like(g)
-    du = torch.empty_like(u)
-    dx_rows = torch.empty((rows, H), dtype=dt, device=dev)
-    (dw_gate, sg, ag), (dw_up, su, au), (dw_down, sd, ad) = (
-        _weight_grad_out(sinks[0], (G, I, H), hidden_states), _weight_grad_out(sinks[1], (G, I, H), hidden_states),
-        _weight_grad_out(sinks[2], (G, H, I), hidden_states))
-    # the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window
-    # stay zero
-    if rows == routing_weights.numel() and not rows_is_bound:
-        routing_weights_grad = torch.empty_like(routing_weights)
-    else:
-        routing_weights_grad = torch.zeros_like(routing_weights)
-    hidden_states_grad = torch.empty_like(hidden_states)
-    with record_pcl_function("1moeblock--7gmlp_bwd"):
-        if rows > 0:
-            parts = lib.om_merged_mlp_row_dot_parts(I)
-            if parts < 1:
-                _n.check(parts, "om_merged_mlp_row_dot_parts")
-            row_dot = torch.empty((parts, rows), dtype=torch.float32, device=dev)
-            _wgrad(dfinal, h, dw_down, cum, rows, G, H, I, sd, ad, "down", output_grad_rows=input_indices,
-                   src_rows=T)
-            _n.check(lib.om_merged_mlp_down_dgrad_weighted(
-                _n.ptr(dfinal), _n.ptr(input_indices), T, _n.ptr(w_down), _n.ptr(g), _n.ptr(u),
-                _n.ptr(row_weights), _n.ptr(dg), _n.ptr(du), _n.ptr(row_dot), _n.ptr(cum), rows, G, I, H,
-                _expert_stride(w_down), st), "om_merged_mlp_down_dgrad_weighted")
-            _n.check(lib.om_moe_row_weights_grad(
-                _n.ptr(row_dot), parts, _n.ptr(selected_experts_indices), _n.ptr(input_indices),
-                _n.ptr(output_indices), _n.ptr(routing_weights_grad), rows, K,
-                _n.dtype_code(routing_weights_grad), st), "om_moe_row_weights_grad")
-            _wgrad(dg, hidden_states, dw_gate, cum, rows, G, I, H, sg, ag, "gate", input_rows=input_indices,
-                   src_rows=T)
-            _wgrad(du, hidden_states, dw_up, cum, rows, G, I, H, su, au, "up", input_rows=input_indices,
-                   src_rows=T)
-            _n.check(lib.om_merged_mlp_gate_up_dgrad(
-                _n.ptr(dg), _n.ptr(du), _n.ptr(w_gate), _n.ptr(w_up), _n.ptr(dx_rows), _n.ptr(cum), rows,
-                G, I, H, _expert_stride(w_gate), st), "om_merged_mlp_gate_up_dgrad")
-        else:   # nothing routed to these experts: the weight gradients are zero
-            for dw, n_, k_, acc in ((dw_down, H, I, ad), (dw_gate, I, H, ag), (dw_up, I, H, au)):
-                if not acc:     # (a live gradient buffer stays as it is)
-                    _n.check(lib.om_grouped_gemm_wgrad(None, None, _n.ptr(dw), _n.ptr(cum), 0, G, n_, k_, 0, st),
-                             "om_grouped_gemm_wgrad(empty)")
-    with record_pcl_function("1moeblock--6gmlp_input_prep_bwd"):
-        if base is None:
-            pcl_xpu_customops.shuffle_sub_matrix_reduce(dx_rows, cum_expert_counts_ep, output_indices,
-                                                        hidden_states_grad)
-        else:
-            _n.require_cuda_contiguous(base)
-            _n.check(lib.om_sum_ggemm_output(
-                _n.ptr(dx_rows), _n.ptr(cum_expert_counts_ep), _n.ptr(output_indices), _n.ptr(base),
-                _n.ptr(hidden_states_grad), T, H, _n.dtype_code(hidden_states_grad), st), "om_sum_ggemm_output")
-    return (hidden_states_grad, routing_weights_grad, None if ag else dw_gate, None if au else dw_up,
-            None if ad else dw_down)
-
-
-class RoutedMLPFunction(torch.autograd.Function):
+class RoutedMLPFunction:
     """The expert half of the block in one function: PrepareInputForGroupGemmFunction, the SwiGLU
     MLP of every expert and GroupGemmOutputReductionFunction (reference moe.py:217-405), with both
     row permutations and the routing weight folded into the GEMMs:
@@ -931,45 +447,17 @@ class RoutedMLPFunction(torch.autograd.Function):
     3*G per-expert matrices of GroupMLPFunction."""
 
     @staticmethod
-    def forward(ctx, hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-                selected_experts_indices, cum_token_counts, residual, n_merged, *weights):
+    def apply(hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
+              selected_experts_indices, cum_token_counts, residual, n_merged, *weights):
         # n_merged: True = merged weights; False = per-expert weights; "bound" forms of both say that
         # the index arrays are sized by an upper bound of the routed rows (expert_computation)
-        ctx.rows_is_bound = n_merged in ("merged_bound", "per_expert_bound")
-        n_merged = n_merged in (True, "merged_bound")
-        if n_merged:
-            wg, wu, wd = ctx.leaves = weights
-        else:
-            ctx.leaves = _per_expert_leaves(weights)
-            wg, wu, wd = [_strided_expert_view(ws) for ws in ctx.leaves]
-        hidden_states = hidden_states.contiguous()
-        routing_weights = routing_weights.contiguous()
-        if residual is not None:
-            residual = residual.contiguous()
-        final, cum, g, u, h, row_weights = _routed_mlp_forward(
-            hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-            selected_experts_indices, wg, wu, wd, cum_token_counts, residual)
-        ctx.save_for_backward(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                              output_indices, selected_experts_indices, wg, wu, wd, cum, g, u, h,
-                              row_weights)
-        ctx.n_merged = bool(n_merged)
-        ctx.has_residual = residual is not None
-        return final
-
-    @staticmethod
-    def backward(ctx, dfinal):
-        sinks = tuple(_grad_sink(w) for w in ctx.leaves)
-        dx, drw, dwg, dwu, dwd = _routed_mlp_backward(dfinal, *ctx.saved_tensors, sinks=sinks,
-                                                      rows_is_bound=ctx.rows_is_bound)
-        if ctx.n_merged:
-            wgrads = (dwg, dwu, dwd)
-        else:
-            wgrads = _per_expert_grads(dwg, dwu, dwd, len(ctx.leaves[0]))
-        return (dx, drw, None, None, None, None, None, dfinal if ctx.has_residual else None, None,
-                *wgrads)
+        return _n.host().routed_mlp(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
+                                    output_indices, selected_experts_indices, cum_token_counts, residual,
+                                    n_merged in ("merged_bound", "per_expert_bound"),
+                                    n_merged in (True, "merged_bound"), list(weights), False, None)
 
 
-class RoutedAndSharedMLPFunction(torch.autograd.Function):
+class RoutedAndSharedMLPFunction:
     """shared_mlp(x) + the routed experts' weighted sum (reference modeling_deepseek_v3.py:265,
     `self.moe(...) + self.shared_experts(residuals)`) as one function: RoutedMLPFunction over the
     per-expert weights with the shared MLP's output as its residual.  Same kernels and bits forward
@@ -982,71 +470,17 @@ class RoutedAndSharedMLPFunction(torch.autograd.Function):
     down [out, in] matrices."""
 
     @staticmethod
-    def forward(ctx, hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-                selected_experts_indices, cum_token_counts, rows_is_bound, *weights):
-        routed, shared = weights[:-3], weights[-3:]
-        ctx.leaves = _per_expert_leaves(routed)
-        ctx.shared_leaves = shared
-        ctx.rows_is_bound = bool(rows_is_bound)
-        wg, wu, wd = [_strided_expert_view(ws) for ws in ctx.leaves]
-        sg, su, sd = [w.unsqueeze(0) for w in shared]
-        hidden_states = hidden_states.contiguous()
-        routing_weights = routing_weights.contiguous()
+    def apply(hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
+              selected_experts_indices, cum_token_counts, rows_is_bound, *weights):
         one = single_segment_counts(hidden_states.shape[0], hidden_states.device)
-        y_shared, one, gs, us, hs = _merged_mlp_forward(hidden_states, sg, su, sd, one)
-        final, cum, g, u, h, row_weights = _routed_mlp_forward(
-            hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-            selected_experts_indices, wg, wu, wd, cum_token_counts, y_shared)
-        ctx.save_for_backward(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                              output_indices, selected_experts_indices, wg, wu, wd, cum, g, u, h,
-                              row_weights, sg, su, sd, one, gs, us, hs)
-        return final
-
-    @staticmethod
-    def backward(ctx, dfinal):
-        saved = ctx.saved_tensors
-        routed_saved, (sg, su, sd, one, gs, us, hs) = saved[:14], saved[14:]
-        hidden_states = saved[0]
-        dfinal = dfinal.contiguous()
-        dx_shared, *dws_shared = _merged_mlp_backward(
-            dfinal, hidden_states, sg, su, sd, one, gs, us, hs,
-            sinks=tuple(_grad_sink(w) for w in ctx.shared_leaves))
-        dx, drw, dwg, dwu, dwd = _routed_mlp_backward(
-            dfinal, *routed_saved, sinks=tuple(_grad_sink(w) for w in ctx.leaves), base=dx_shared,
-            rows_is_bound=ctx.rows_is_bound)
-        dws_shared = [None if dw is None else dw[0] for dw in dws_shared]
-        return (dx, drw, None, None, None, None, None, None,
-                *_per_expert_grads(dwg, dwu, dwd, len(ctx.leaves[0])), *dws_shared)
-
-
-def _strided_expert_view(weights):
-    """[G, out, in] view over per-expert matrices that lie at a constant pitch in one storage."""
-    w0 = weights[0]
-    o, i = w0.shape
-    G = len(weights)
-    if G == 1:
-        return w0.unsqueeze(0)
-    esz = w0.element_size()
-    pitch_bytes = weights[1].data_ptr() - w0.data_ptr()
-    ok = pitch_bytes > 0 and pitch_bytes % esz == 0 and pitch_bytes >= o * i * esz
-    for n, w in enumerate(weights):
-        ok = ok and w.is_contiguous() and w.shape == w0.shape and w.dtype == w0.dtype \
-            and w.data_ptr() == w0.data_ptr() + n * pitch_bytes \
-            and w.untyped_storage().data_ptr() == w0.untyped_storage().data_ptr()
-    if not ok:
-        raise _n.NativeLibraryError(
-            "per-expert weights must lie at a constant pitch inside one buffer (merge them with "
-            "pack_expert_weights, or build the optimizer first so they alias flat_param)")
-    pitch = pitch_bytes // esz
-    return torch.as_strided(w0, (G, o, i), (pitch, i, 1))
+        return _n.host().routed_mlp(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
+                                    output_indices, selected_experts_indices, cum_token_counts, None,
+                                    bool(rows_is_bound), False, list(weights), True, one)
 
 
 def has_constant_pitch(weights):
-    try:
-        _strided_expert_view(weights)
-        return True
-    except _n.NativeLibraryError:
-        return False
+    """True when the matrices lie at one constant pitch inside one buffer."""
+    return _n.host().constant_pitch(list(weights))
 
 
 def pack_expert_weights(experts, names=("gate_proj", "up_proj", "down_proj")):
@@ -1061,6 +495,16 @@ def pack_expert_weights(experts, names=("gate_proj", "up_proj", "down_proj")):
         buf = torch.stack([w.data for w in ws]).contiguous()
         for n, w in enumerate(ws):
             w.data = buf[n]
+
+
+def packed_expert_parameters(experts):
+    """The (gate, up, down) weights of every expert in GroupMLPFunction's order, packed (see
+    pack_expert_weights)."""
+    params = _n.host().expert_parameters(experts)
+    if not all(_n.host().constant_pitch(params[j::3]) for j in range(3)):
+        pack_expert_weights(experts)
+        params = _n.host().expert_parameters(experts)
+    return params
 
 
 class PrepareInputForGroupGemmFunction(torch.autograd.Function):
@@ -1095,50 +539,21 @@ class PrepareInputForGroupGemmFunction(torch.autograd.Function):
         return hidden_states_grad, None, None, None, None, None, None, None
 
 
-class GroupGemmOutputReductionFunction(torch.autograd.Function):
+class GroupGemmOutputReductionFunction:
     """K6: final[t] = sum_k w[t,k] * ggemm_output[pos(t,k)] in fp32, one rounding; backward gives
     ggemm_output_grad and routing_weights_grad (reference moe.py:284-377).  The four trailing
     flags are accepted and ignored.  routing_weights may be fp32 while activations are bf16."""
 
     @staticmethod
-    def forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-                input_indices, output_indices,
-                use_ref_path_fwd=False, use_ref_path_bwd=False,
-                use_triton_path_fwd=False, use_triton_path_bwd=False):
-        routing_weights = routing_weights.contiguous()
-        ctx.save_for_backward(ggemm_output, routing_weights, cum_expert_counts_ep,
-                              selected_experts_indices, input_indices, output_indices)
-        num_tokens, _ = routing_weights.shape
-        hidden_dim = ggemm_output.shape[1]
-        with record_pcl_function("1moeblock--8gmlp_output_reduction_fwd"):
-            final_hidden_states = torch.empty((num_tokens, hidden_dim), dtype=ggemm_output.dtype,
-                                              device=ggemm_output.device)
-            pcl_xpu_customops.reduce_ggemm_output(ggemm_output, routing_weights, cum_expert_counts_ep,
-                                                  selected_experts_indices, output_indices,
-                                                  final_hidden_states, False)
-        return final_hidden_states
-
-    @staticmethod
-    def backward(ctx, final_hidden_states_grad):
-        (ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices, input_indices,
-         output_indices) = ctx.saved_tensors
-        final_hidden_states_grad = final_hidden_states_grad.contiguous()
-        ggemm_output_grad = torch.empty_like(ggemm_output)
-        # the kernel writes the entry of every routed (token, k) pair; pairs outside the expert
-        # window stay zero (the reference pre-zeroes the whole tensor, moe.py:336)
-        if output_indices.shape[0] == routing_weights.numel():
-            routing_weights_grad = torch.empty_like(routing_weights)
-        else:
-            routing_weights_grad = torch.zeros_like(routing_weights)
-        with record_pcl_function("1moeblock--8gmlp_output_reduction_bwd"):
-            pcl_xpu_customops.reduce_ggemm_output_backward(
-                final_hidden_states_grad, ggemm_output, routing_weights, cum_expert_counts_ep,
-                selected_experts_indices, input_indices, output_indices, ggemm_output_grad,
-                routing_weights_grad)
-        return ggemm_output_grad, routing_weights_grad, None, None, None, None, None, None, None, None
+    def apply(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+              input_indices, output_indices,
+              use_ref_path_fwd=False, use_ref_path_bwd=False,
+              use_triton_path_fwd=False, use_triton_path_bwd=False):
+        return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                                 input_indices, output_indices, None)
 
 
-class GroupGemmOutputReductionResidualFunction(torch.autograd.Function):
+class GroupGemmOutputReductionResidualFunction:
     """residual + GroupGemmOutputReductionFunction(...) in one pass: the combined sum is rounded to
     the activation dtype and then added to `residual` (both roundings of the two-step form).  Used
     for the decoder layer's residual connection (modeling_olmoe.py:415) and for the DeepSeek-V3
@@ -1146,23 +561,10 @@ class GroupGemmOutputReductionResidualFunction(torch.autograd.Function):
     `residual` unchanged and into the combine's backward."""
 
     @staticmethod
-    def forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-                input_indices, output_indices, residual):
-        routing_weights = routing_weights.contiguous()
-        residual = residual.contiguous()
-        ctx.save_for_backward(ggemm_output, routing_weights, cum_expert_counts_ep,
-                              selected_experts_indices, input_indices, output_indices)
-        with record_pcl_function("1moeblock--8gmlp_output_reduction_fwd"):
-            final_hidden_states = torch.empty_like(residual)
-            pcl_xpu_customops.reduce_ggemm_output_residual(
-                ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-                output_indices, residual, final_hidden_states)
-        return final_hidden_states
-
-    @staticmethod
-    def backward(ctx, final_hidden_states_grad):
-        grads = GroupGemmOutputReductionFunction.backward(ctx, final_hidden_states_grad)
-        return grads[0], grads[1], None, None, None, None, final_hidden_states_grad
+    def apply(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+              input_indices, output_indices, residual):
+        return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                                 input_indices, output_indices, residual)
 
 
 # ----------------------------------------------------------------------------------------------
@@ -1198,7 +600,7 @@ class MergedMLP(nn.Module):
 
 def expert_computation(hidden_states, routing_weights, selected_experts, expert_start_idx,
                        expert_end_idx, experts_fn, num_total_experts, gathered_experts_fn=None,
-                       residual=None, routed_experts_fn=None, sync_free_window=False):
+                       residual=None, routed_experts_fn=None, sync_free_window=False, fused_experts_fn=None):
     """K1..K6 for 2-D hidden_states [T,H]: permute, run `experts_fn(ggemm_input, cum_token_counts)`,
     combine.  Shared by the OLMoE and DeepSeek-V3 blocks.  With `gathered_experts_fn(hidden_states,
     input_indices, cum_expert_counts_ep, output_indices, cum_token_counts)` the experts read the
@@ -1207,6 +609,8 @@ def expert_computation(hidden_states, routing_weights, selected_experts, expert_
     routing_weights, input_indices, cum_expert_counts_ep, output_indices, selected_experts_indices,
     cum_token_counts, residual)` may do gather, experts and combine in one function
     (RoutedMLPFunction); it returns None when its kernels do not take the operands.
+    `fused_experts_fn(hidden_states, routing_weights, selected_experts, residual)` does the same
+    including the permutation, whose arrays then never become Python objects.
 
     Under an expert window the number of routed rows is only known on the device.  By default it is
     read back once, like the reference does (moe.py:520).  With `sync_free_window` and a
@@ -1215,6 +619,10 @@ def expert_computation(hidden_states, routing_weights, selected_experts, expert_
     only the routed ones are computed, and the function is called with `rows_is_bound=True`.  That
     makes the step capturable in a HIP graph at the price of expert_parallelism times the
     activation memory."""
+    if fused_experts_fn is not None:
+        final = fused_experts_fn(hidden_states, routing_weights, selected_experts, residual)
+        if final is not None:
+            return final
     T, K = selected_experts.shape
     with record_pcl_function("1moeblock--3index_calculation"):
         (cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
@@ -1304,52 +712,35 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
     def _experts_fn(self, ggemm_input, cum_token_counts):
         if isinstance(self.experts, MergedMLP):
             return self.experts(ggemm_input, cum_token_counts)
-        pack_expert_weights(self.experts)   # no-op once the weights share a buffer
-        mlp_params = []
-        for expert in self.experts:
-            mlp_params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
-        return GroupMLPFunction.apply(ggemm_input, cum_token_counts, False, *mlp_params)
+        return GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
+                                      *packed_expert_parameters(self.experts))
 
     def _gathered_experts_fn(self, hidden_states, input_indices, cum_expert_counts_ep, output_indices,
                              cum_token_counts):
         if isinstance(self.experts, MergedMLP):
             return self.experts.forward_gathered(hidden_states, input_indices, cum_expert_counts_ep,
                                                  output_indices, cum_token_counts)
-        pack_expert_weights(self.experts)
-        mlp_params = []
-        for expert in self.experts:
-            mlp_params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
         return GatheredGroupMLPFunction.apply(hidden_states, input_indices, cum_expert_counts_ep,
-                                              output_indices, cum_token_counts, *mlp_params)
+                                              output_indices, cum_token_counts,
+                                              *packed_expert_parameters(self.experts))
 
-    def _routed_experts_fn(self, hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                           output_indices, selected_experts_indices, cum_token_counts, residual,
-                           rows_is_bound=False):
-        if isinstance(self.experts, MergedMLP):
-            weights = (self.experts.gate_proj_merged_weight, self.experts.up_proj_merged_weight,
-                       self.experts.down_proj_merged_weight)
+    def _fused_experts_fn(self, hidden_states, routing_weights, selected_experts, residual):
+        """Permutation and RoutedMLPFunction in one call; None when the kernels do not take the operands."""
+        merged = isinstance(self.experts, MergedMLP)
+        if merged:
+            ex = self.experts._parameters
+            weights = [ex["gate_proj_merged_weight"], ex["up_proj_merged_weight"], ex["down_proj_merged_weight"]]
             why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
-            if why is not None:
-                if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
-                    note_unfused_path("routing weight inside the expert MLP", why)
-                return None
-            return RoutedMLPFunction.apply(hidden_states, routing_weights, input_indices,
-                                           cum_expert_counts_ep, output_indices, selected_experts_indices,
-                                           cum_token_counts, residual,
-                                           "merged_bound" if rows_is_bound else True, *weights)
-        pack_expert_weights(self.experts)
-        w0, d0 = self.experts[0].gate_proj.weight, self.experts[0].down_proj.weight
-        why = routed_mlp_unfit_reason(hidden_states, routing_weights, w0.unsqueeze(0), d0.unsqueeze(0))
+        else:
+            weights = packed_expert_parameters(self.experts)
+            why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
         if why is not None:
             if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
                 note_unfused_path("routing weight inside the expert MLP", why)
             return None
-        mlp_params = []
-        for expert in self.experts:
-            mlp_params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
-        return RoutedMLPFunction.apply(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                                       output_indices, selected_experts_indices, cum_token_counts,
-                                       residual, "per_expert_bound" if rows_is_bound else False, *mlp_params)
+        return _n.host().moe_experts(hidden_states, routing_weights, selected_experts, self.expert_start_idx,
+                                     self.expert_end_idx, self.num_experts, self.sync_free_expert_window,
+                                     residual, merged, weights, False, None)
 
     def forward_with_residual(self, hidden_states, residual):
         """(residual + forward(hidden_states)[0], router_logits): the decoder layer's
@@ -1364,35 +755,33 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         if self.router_logits_fp32 and gate_unfit is not None and flat.dtype == torch.bfloat16:
             note_unfused_path("gate projection fused with the routing", gate_unfit,
                               instead="running the projection and the routing as separate kernels (same fp32 logits)")
-        if self.router_logits_fp32 and gate_unfit is None:
-            # the experts read the router function's pass-through of the hidden states, so that their
-            # input gradient and the gate's are added in one kernel (GateSoftmaxTopkFunction)
-            routing_weights, selected_experts, router_logits, flat = GateSoftmaxTopkFunction.apply(
-                flat.contiguous(), self.gate.weight, self.num_experts_per_tok, self.norm_topk_prob,
-                hidden_states.dtype)
-            hidden_states = flat.view(batch_size, sequence_length, hidden_dim)
+        # (the experts are fed from the router's pass-through of the hidden states, so that their input
+        # gradient and the gate's are added in one kernel)
+        weight = self.gate.weight
+        if flat.is_cuda and flat.dtype == weight.dtype and flat.dtype in (torch.bfloat16, torch.float32) \
+                and self.gate.bias is None:
+            bf16 = flat.dtype == torch.bfloat16
+            routing_weights, selected_experts, router_logits, flat = _n.host().route_softmax(
+                flat.contiguous(), weight, self.num_experts_per_tok, bool(self.norm_topk_prob), flat.dtype,
+                self.router_logits_fp32 and gate_unfit is None, bf16 and not self.router_logits_fp32)
         else:
-            # (the experts are fed from the gate projection's pass-through here too: their input
-            # gradient is then added to the gate's inside om_router_gate_dgrad)
             if self.router_logits_fp32:
-                router_logits, flat = fp32_logits_with_passthrough(flat, self.gate.weight)
+                router_logits, flat = fp32_logits_with_passthrough(flat, weight)
             else:
                 router_logits, flat = gate_logits_with_passthrough(flat, self.gate)
-            hidden_states = flat.view(batch_size, sequence_length, hidden_dim)
             routing_weights, selected_experts = SoftmaxTopkRouterFunction.apply(
-                router_logits.contiguous(), self.num_experts_per_tok, self.norm_topk_prob,
-                hidden_states.dtype)
+                router_logits.contiguous(), self.num_experts_per_tok, self.norm_topk_prob, flat.dtype)
+        hidden_states = flat.view(batch_size, sequence_length, hidden_dim)
 
         def expert_computation_block(hidden_states, selected_experts, routing_weights, residual=None):
             b, s, h = hidden_states.shape
             gathered = self._gathered_experts_fn if self.fuse_input_gather else None
-            routed = self._routed_experts_fn if (self.fuse_input_gather and self.fuse_routing_weights) else None
+            fused = self._fused_experts_fn if (self.fuse_input_gather and self.fuse_routing_weights) else None
             out = expert_computation(hidden_states.reshape(-1, h), routing_weights, selected_experts,
                                      self.expert_start_idx, self.expert_end_idx, self._experts_fn,
                                      self.num_experts, gathered_experts_fn=gathered,
                                      residual=None if residual is None else residual.reshape(-1, h),
-                                     routed_experts_fn=routed,
-                                     sync_free_window=self.sync_free_expert_window)
+                                     fused_experts_fn=fused)
             return out.reshape(b, s, h)
 
         args = [hidden_states, selected_experts, routing_weights]

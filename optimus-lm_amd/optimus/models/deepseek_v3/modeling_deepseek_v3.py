@@ -110,12 +110,12 @@ class DeepseekV3ParallelTopkRouter(nn.Module):
         projection's pass-through of its input; experts fed from it get their input gradient added
         to the gate's inside the gate's input-gradient kernel (GateLogitsFunction)."""
         hidden_states = hidden_states.reshape(-1, self.config.hidden_size)
-        router_logits, hidden_states = _moe.fp32_logits_with_passthrough(hidden_states, self.weight)
-        topk_indices, topk_weights = SigmoidGroupTopkRouterFunction.apply(
-            router_logits.contiguous(), self.e_score_correction_bias.float().contiguous(),
-            self.n_group, self.topk_group, self.top_k, self.norm_topk_prob,
-            self.routed_scaling_factor)
-        return topk_indices, topk_weights, hidden_states
+        if hidden_states.dtype != self.weight.dtype or hidden_states.dtype not in (torch.bfloat16, torch.float32):
+            raise TypeError(f"router gate: activations and weight must both be bfloat16 or both float32 "
+                            f"(got {hidden_states.dtype}, {self.weight.dtype})")
+        return _n.host().route_sigmoid(
+            hidden_states.contiguous(), self.weight.contiguous(), self.e_score_correction_bias.float().contiguous(),
+            self.n_group, self.topk_group, self.top_k, bool(self.norm_topk_prob), float(self.routed_scaling_factor))
 
 
 class DeepseekV3ParallelMoE(nn.Module):
@@ -139,48 +139,37 @@ class DeepseekV3ParallelMoE(nn.Module):
             self.use_activation_checkpointing_for_moe = config.activation_checkpointing_level & (1 << 0)
 
     def _experts_fn(self, ggemm_input, cum_token_counts):
-        _moe.pack_expert_weights(self.experts)   # no-op once the weights share a buffer
-        params = []
-        for expert in self.experts:
-            params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
-        return _moe.GroupMLPFunction.apply(ggemm_input, cum_token_counts, False, *params)
+        return _moe.GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
+                                           *_moe.packed_expert_parameters(self.experts))
 
     def _gathered_experts_fn(self, hidden_states, input_indices, cum_expert_counts_ep, output_indices,
                              cum_token_counts):
-        _moe.pack_expert_weights(self.experts)
-        params = []
-        for expert in self.experts:
-            params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
         return _moe.GatheredGroupMLPFunction.apply(hidden_states, input_indices, cum_expert_counts_ep,
-                                                   output_indices, cum_token_counts, *params)
+                                                   output_indices, cum_token_counts,
+                                                   *_moe.packed_expert_parameters(self.experts))
 
     def _routed_kernels_fit(self, hidden_states, routing_weights):
         w0, d0 = self.experts[0].gate_proj.weight, self.experts[0].down_proj.weight
-        return _moe.routed_mlp_kernel_fits(hidden_states, routing_weights, w0.unsqueeze(0), d0.unsqueeze(0))
+        return _moe.routed_mlp_kernel_fits(hidden_states, routing_weights, w0, d0)
 
-    def _routed_experts_fn(self, hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                           output_indices, selected_experts_indices, cum_token_counts, residual,
-                           rows_is_bound=False, with_shared=False):
-        _moe.pack_expert_weights(self.experts)
-        w0, d0 = self.experts[0].gate_proj.weight, self.experts[0].down_proj.weight
-        why = _moe.routed_mlp_unfit_reason(hidden_states, routing_weights, w0.unsqueeze(0), d0.unsqueeze(0))
+    def _fused_experts_fn(self, hidden_states, routing_weights, selected_experts, residual, with_shared=False):
+        """Permutation, RoutedMLPFunction and (with_shared) the shared experts in one call; None when the
+        kernels do not take the operands."""
+        params = _moe.packed_expert_parameters(self.experts)
+        why = _moe.routed_mlp_unfit_reason(hidden_states, routing_weights, params[0], params[2])
         if why is not None:
             if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
                 _moe.note_unfused_path("routing weight inside the expert MLP", why)
             return None
-        params = []
-        for expert in self.experts:
-            params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
+        one = None
         if with_shared:
             sh = self.shared_experts
-            return _moe.RoutedAndSharedMLPFunction.apply(
-                hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-                selected_experts_indices, cum_token_counts, rows_is_bound, *params, sh.gate_proj.weight,
-                sh.up_proj.weight, sh.down_proj.weight)
-        return _moe.RoutedMLPFunction.apply(hidden_states, routing_weights, input_indices,
-                                            cum_expert_counts_ep, output_indices, selected_experts_indices,
-                                            cum_token_counts, residual,
-                                            "per_expert_bound" if rows_is_bound else False, *params)
+            params += [sh.gate_proj.weight, sh.up_proj.weight, sh.down_proj.weight]
+            one = _moe.single_segment_counts(hidden_states.shape[0], hidden_states.device)
+        return _n.host().moe_experts(hidden_states, routing_weights, selected_experts, self.expert_start_idx,
+                                     self.expert_end_idx, self.config.n_routed_experts,
+                                     bool(getattr(self.config, "sync_free_expert_window", False)), residual,
+                                     False, params, with_shared, one)
 
     def _fuses_routing_weights(self):
         return getattr(self.config, "fuse_input_gather", True) and \
@@ -195,18 +184,17 @@ class DeepseekV3ParallelMoE(nn.Module):
         (needs the fused path): the shared experts run inside the same function and their output
         is that residual (RoutedAndSharedMLPFunction)."""
         gathered = self._gathered_experts_fn if getattr(self.config, "fuse_input_gather", True) else None
-        routed = None
+        fused = None
         if self._fuses_routing_weights():
-            routed = self._routed_experts_fn
+            fused = self._fused_experts_fn
             if with_shared:
-                routed = lambda *a, **kw: self._routed_experts_fn(*a, with_shared=True, **kw)
+                fused = lambda *a: self._fused_experts_fn(*a, with_shared=True)
         elif with_shared:
             raise ValueError("with_shared needs the fused routing-weight path")
         return _moe.expert_computation(hidden_states, topk_weights, topk_indices,
                                        self.expert_start_idx, self.expert_end_idx, self._experts_fn,
                                        self.config.n_routed_experts, gathered_experts_fn=gathered,
-                                       residual=residual, routed_experts_fn=routed,
-                                       sync_free_window=getattr(self.config, "sync_free_expert_window", False))
+                                       residual=residual, fused_experts_fn=fused)
 
     def forward(self, hidden_states):
         # the experts are fed from the gate projection's pass-through of the hidden states, so that

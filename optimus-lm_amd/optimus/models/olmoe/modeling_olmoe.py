@@ -67,16 +67,9 @@ class OlmoeParallelSparseMoeBlock(nn.Module):
         if getattr(config, "force_uniform_routing", False):
             raise NotImplementedError("force_uniform_routing is not part of this build")
 
-    def _expert_weights(self):
-        params = []
-        for expert in self.experts:
-            params += [expert.gate_proj.weight, expert.up_proj.weight, expert.down_proj.weight]
-        return params
-
     def _experts_fn(self, ggemm_input, cum_token_counts):
-        _moe.pack_expert_weights(self.experts)   # no-op once the weights share a buffer
         return _moe.GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
-                                           *self._expert_weights())
+                                           *_moe.packed_expert_parameters(self.experts))
 
     def forward(self, hidden_states):
         batch_size, sequence_length, hidden_dim = hidden_states.shape
