@@ -190,14 +190,17 @@ int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t T, int H, 
  * `router_logits = self.gate(hidden_states)` (optimus/models/common/moe.py:456) where the block is
  * kept in float32 (the reference's small CPU-runnable configuration): plain float32 products,
  * sums in a fixed order (the weight gradient's sum over the tokens is kept in double and rounded
- * once).  Any T, H, N <= 65535.  Parity path, not tuned.
+ * once).  Any T, H, N <= 65535.
  *   om_router_gate_logits_f32 : logits[t,n]  = sum_h x[t,h] * gate_weight[n,h]
  *   om_router_gate_dgrad_f32  : dx[t,h]      = sum_n dlogits[t,n] * gate_weight[n,h]
+ *   om_router_gate_dgrad_f32_add : the same plus base[t,h] (another gradient of x, may be null)
  *   om_router_gate_wgrad_f32  : dweight[n,h] = sum_t dlogits[t,n] * x[t,h]                       */
 int om_router_gate_logits_f32(const float *x, const float *gate_weight, int64_t T, int H, int N,
                               float *logits_out, void *stream);
 int om_router_gate_dgrad_f32(const float *dlogits, const float *gate_weight, int64_t T, int H, int N,
                              float *dx, void *stream);
+int om_router_gate_dgrad_f32_add(const float *dlogits, const float *gate_weight, const float *base, int64_t T,
+                                 int H, int N, float *dx, void *stream);
 int om_router_gate_wgrad_f32(const float *x, const float *dlogits, int64_t T, int H, int N,
                              float *dweight, void *stream);
 
@@ -556,6 +559,26 @@ int om_grouped_gemm_wgrad_gathered_out_accumulate(const void *output_grad, const
 int om_grouped_gemm_wgrad_f32_accumulate(const float *output_grad, const float *input, float *weight_grad,
                                          const int32_t *cum_token_counts, int64_t rows, int G, int N,
                                          int K, int64_t w_stride, void *stream);
+
+/* The merged MLP of a float32 module (moe.py:396-405 and its autograd), the forms of the bf16 entry points
+ * above: gate and up in one launch with h = silu(g) * u formed in the epilogue, the SwiGLU backward in the
+ * epilogue of dh = dy W_down, dx as one accumulation over both products, and both weight gradients in one
+ * launch (`accumulate` bit 0: add into dw_gate, bit 1: into dw_up).  x_rows (may be null): row r of x is row
+ * x_rows[r] of a [src_rows, H] matrix.  I and H multiples of 8.                                             */
+int om_merged_mlp_gate_up_fwd_f32(const float *x, const int32_t *x_rows, int64_t src_rows, const float *w_gate,
+                                  const float *w_up, float *g, float *u, float *h, const int32_t *cum_token_counts,
+                                  int64_t rows, int G, int I, int H, int64_t gate_stride, int64_t up_stride,
+                                  void *stream);
+int om_merged_mlp_down_dgrad_f32(const float *dy, const float *w_down, const float *g, const float *u, float *dg,
+                                 float *du, const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                                 int64_t w_stride, void *stream);
+int om_merged_mlp_gate_up_dgrad_f32(const float *dg, const float *du, const float *w_gate, const float *w_up, float *dx,
+                                    const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                                    int64_t gate_stride, int64_t up_stride, void *stream);
+int om_merged_mlp_gate_up_wgrad_f32(const float *dg, const float *du, const float *x, const int32_t *x_rows,
+                                    int64_t src_rows, float *dw_gate, float *dw_up, const int32_t *cum_token_counts,
+                                    int64_t rows, int G, int I, int H, int64_t gate_stride, int64_t up_stride,
+                                    int accumulate, void *stream);
 
 /* Stand-alone SwiGLU glue (moe.py:401-402 forward; moe.py:37-41 and :133-147 backward),
  * for callers that keep the three GEMMs separate.  n elements, dtype OM_F32 or OM_BF16.   */

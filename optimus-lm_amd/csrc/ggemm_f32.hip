@@ -1,134 +1,262 @@
 // Grouped expert GEMMs in float32 (v_mfma_f32_32x32x2_f32, fp32 operands and accumulation), for
 // modules kept in float32 like the reference's small CPU-runnable configuration
 // (GroupedGemmFunction, optimus/models/common/moe.py:163-215, runs torch.matmul per expert in
-// whatever dtype the module has).  Same three products and the same variable-rows-per-expert
-// contract as the bf16 kernels; this path is for parity at fp32 accuracy, not for speed: one
-// 64x64 output tile per 256-thread block, contraction steps of 16 staged through LDS from
-// registers, one stage.
+// whatever dtype the module has).  Same products and the same variable-rows-per-expert contract as
+// the bf16 kernels: forward, input gradient, weight gradient, and the merged MLP's forms of them (gate
+// and up in one launch with the SwiGLU or its backward in the epilogue, the token gather in the loads).
 //
-// An operand tile is always kept in LDS as [row][c] (c = contraction index, 17-float row pitch).
-// CONTIG operands ([row][c] in memory) are copied as float4 along c; STRIDED operands ([c][row] in
-// memory: the weight in dgrad, both operands in wgrad) are read as float4 along the rows (coalesced)
-// and written to LDS transposed.
+// One 64x64 output tile per 256-thread block, contraction steps of 32, two LDS stages: the global
+// loads of step s+1 are in registers' flight while step s is multiplied, and are written to the other
+// stage behind one barrier per step.  These launches are small (the tiny layer: 1.07 GFLOP a product,
+// 7 us of matrix-core time per tile), so what bounds them is the latency of a step's loads and the
+// number of launches.  Tiny layer (2048 tokens, hidden 256, ffn 512, 8 experts, top-2) per step: 15
+// launches of 24-37 us with one stage of 16 and a barrier on each side of the loads, 6 of 9-18 us now.
+//
+// CONTIG operands ([row][c] in memory, c = contraction index) lie in LDS as [row][c] with a 36-float
+// pitch: 16-byte writes and reads, 16 consecutive rows in 16 different 16-byte bank groups.  STRIDED
+// operands ([c][row] in memory: the weight in dgrad, both operands in wgrad) lie as [c][row] with a
+// 68-float pitch, read 4 bytes at a time (one read per 64-cycle MFMA: not what bounds).
 #include "common.h"
 
 namespace {
 
 constexpr int TB = 64;      // tile rows and columns
-constexpr int KS = 16;      // contraction step
-constexpr int PITCH = KS + 1;
+constexpr int KS = 32;      // contraction step
+constexpr int PITCH_C = KS + 4, PITCH_S = TB + 4;
+constexpr int STAGE = TB * PITCH_C > KS * PITCH_S ? TB * PITCH_C : KS * PITCH_S;   // floats per operand tile
 typedef __attribute__((ext_vector_type(4))) float f4;
 
 enum { F_CONTIG = 0, F_STRIDED = 1 };
+enum { E_STORE = 0, E_SWIGLU = 1, E_SWIGLU_BWD = 2 };
 
 struct F32Params {
-    const float *A, *B;
-    float *C;
+    const float *A[2], *B[2];   // second pair: up matrix (E_SWIGLU), second phase, or second weight gradient
+    float *C[3];                // output; E_SWIGLU: g, u, h; E_SWIGLU_BWD: dg, du; two weight gradients
+    const float *G, *U;         // E_SWIGLU_BWD: saved g, u
     const int32_t *cum;
-    int64_t lda, ldb, ldc, strideB, strideC;
-    int n_experts, n_cols, kc;
-    int accumulate;   // wgrad: C += product instead of C = product
+    const int32_t *row_index;   // row r of A (rows products) or contraction row r of B (wgrad) is row row_index[r]
+    int64_t lda, ldb, ldc, strideB[2], strideC[2];
+    int n_experts, n_cols, kc, phases;
+    int accumulate;             // wgrad, bit w: C[w] += product instead of C[w] = product
 };
 
-// Fill tile[row][c] (64 x 16) from an operand.  CONTIG: element (row, c) at base[(r0+row)*ld + c0+c];
-// STRIDED: element (row, c) at base[(c0+c)*ld + r0+row].  Rows >= r_end and contraction indices
-// >= c_end read as zero (extents are multiples of 4, so a float4 is inside or outside as a whole).
-template <int KIND>
-__device__ __forceinline__ void load_tile(float (*tile)[PITCH], const float *base, int64_t ld, int64_t r0,
-                                          int64_t r_end, int64_t c0, int64_t c_end, int tid) {
-    if (KIND == F_CONTIG) {
-        const int row = tid >> 2, c4 = (tid & 3) * 4;
-        f4 v = {0.f, 0.f, 0.f, 0.f};
-        if (r0 + row < r_end && c0 + c4 < c_end) v = *reinterpret_cast<const f4 *>(base + (r0 + row) * ld + c0 + c4);
-        tile[row][c4] = v[0]; tile[row][c4 + 1] = v[1]; tile[row][c4 + 2] = v[2]; tile[row][c4 + 3] = v[3];
-    } else {
-        const int c = tid >> 4, row4 = (tid & 15) * 4;
-        f4 v = {0.f, 0.f, 0.f, 0.f};
-        if (c0 + c < c_end && r0 + row4 < r_end) v = *reinterpret_cast<const f4 *>(base + (c0 + c) * ld + r0 + row4);
-        tile[row4][c] = v[0]; tile[row4 + 1][c] = v[1]; tile[row4 + 2][c] = v[2]; tile[row4 + 3][c] = v[3];
-    }
+// One thread's part of a tile and step: 8 floats along c (CONTIG) or along the rows (STRIDED).
+struct Fetched { f4 v[2]; };
+template <int KIND> __device__ __forceinline__ int slot_row(int tid) { return KIND == F_CONTIG ? tid >> 2 : (tid & 7) * 8; }
+template <int KIND> __device__ __forceinline__ int slot_c(int tid) { return KIND == F_CONTIG ? (tid & 3) * 8 : tid >> 3; }
+template <int KIND> __device__ __forceinline__ void stash(float *tile, const Fetched &q, int tid) {
+    float *p = KIND == F_CONTIG ? tile + slot_row<KIND>(tid) * PITCH_C + slot_c<KIND>(tid)
+                                : tile + slot_c<KIND>(tid) * PITCH_S + slot_row<KIND>(tid);
+    reinterpret_cast<f4 *>(p)[0] = q.v[0];
+    reinterpret_cast<f4 *>(p)[1] = q.v[1];
+}
+// 8 floats at p, the two halves masked
+__device__ __forceinline__ Fetched fetch8(const float *p, bool lo, bool hi) {
+    Fetched q;
+    q.v[0] = lo ? reinterpret_cast<const f4 *>(p)[0] : f4{0.f, 0.f, 0.f, 0.f};
+    q.v[1] = hi ? reinterpret_cast<const f4 *>(p)[1] : f4{0.f, 0.f, 0.f, 0.f};
+    return q;
+}
+// Fragment of contraction indices 8s + 4*(lane/32) .. +3 of operand row `row`; element j goes to MFMA j.
+template <int KIND> __device__ __forceinline__ f4 fragment(const float *tile, int row, int s, int half) {
+    if (KIND == F_CONTIG) return *reinterpret_cast<const f4 *>(tile + row * PITCH_C + s * 8 + half * 4);
+    f4 v;
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = tile[(s * 8 + half * 4 + j) * PITCH_S + row];
+    return v;
 }
 
-// One 64x64 tile: C[m0.., n0..] = sum over c in [c0, c1) of A(m, c) * B(n, c); rows >= m_end and
-// columns >= n_end are not stored.
-template <int AKIND, int BKIND>
-__device__ __forceinline__ void tile_product(const float *A, int64_t lda, int64_t a_r0, int64_t a_rend,
-                                             const float *B, int64_t ldb, int64_t b_r0, int64_t b_rend,
-                                             int64_t c0, int64_t c1, float *C, int64_t ldc, int64_t m0,
-                                             int64_t m_end, int64_t n0, int64_t n_end, bool accumulate = false) {
-    __shared__ float ta[TB][PITCH], tb[TB][PITCH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    f32x16 acc;
+// The main loop: `fetch_a(step)` / `fetch_b(step)` deliver this thread's part of a step.
+template <int AKIND, int BKIND, typename FA, typename FB>
+__device__ __forceinline__ void multiply(float *lds, int n_steps, int wm, int wn, FA &&fetch_a, FB &&fetch_b, f32x16 &acc) {
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-    for (int64_t c = c0; c < c1; c += KS) {
-        __syncthreads();
-        load_tile<AKIND>(ta, A, lda, a_r0, a_rend, c, c1, tid);
-        load_tile<BKIND>(tb, B, ldb, b_r0, b_rend, c, c1, tid);
-        __syncthreads();
+    if (n_steps <= 0) return;
+    Fetched a = fetch_a(0), b = fetch_b(0);
+    for (int s = 0; s < n_steps; s++) {
+        float *ta = lds + (s & 1) * 2 * STAGE, *tb = ta + STAGE;
+        stash<AKIND>(ta, a, tid);
+        stash<BKIND>(tb, b, tid);
+        __syncthreads();   // (a stage is rewritten two steps later, behind the barrier of the step between)
+        if (s + 1 < n_steps) { a = fetch_a(s + 1); b = fetch_b(s + 1); }
 #pragma unroll
-        for (int k = 0; k < KS; k += 2) {
-            const float a = ta[wm + (lane & 31)][k + (lane >> 5)];
-            const float b = tb[wn + (lane & 31)][k + (lane >> 5)];
-            // operands swapped: lane l then holds output row wm + l%32 and columns
-            // wn + 8*(r/4) + 4*(l/32) + r%4
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b, a, acc, 0, 0, 0);
+        for (int g = 0; g < KS / 8; g++) {
+            const f4 fa = fragment<AKIND>(ta, wm + (lane & 31), g, half);
+            const f4 fb = fragment<BKIND>(tb, wn + (lane & 31), g, half);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                // operands swapped: lane l then holds output row wm + l%32 and columns
+                // wn + 8*(r/4) + 4*(l/32) + r%4
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[j], acc, 0, 0, 0);
         }
     }
-    const int64_t m = m0 + wm + (lane & 31);
-    if (m < m_end) {
+}
+
+// Which expert owns row tile `tile`: every wavefront scans the counts 64 experts at a time.
+__device__ __forceinline__ bool find_row_tile(const int32_t *cum, int n_experts, int tile, int &expert, int &begin, int &end) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int e0 = 0; e0 < n_experts; e0 += 64) {
+        const int e = e0 + lane;
+        int s = 0, cnt = 0;
+        if (e < n_experts) { s = cum[e]; cnt = cum[e + 1] - s; }
+        const int tiles = (cnt + TB - 1) / TB;
+        int incl = tiles;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
+        }
+        const unsigned long long mine = __ballot(tile >= base + incl - tiles && tile < base + incl);
+        if (mine) {
+            const int src = __ffsll(static_cast<long long>(mine)) - 1;
+            expert = e0 + src;
+            begin = __shfl(s + (tile - base - (incl - tiles)) * TB, src, 64);
+            end = __shfl(s + cnt, src, 64);
+            return true;
+        }
+        base += __shfl(incl, 63, 64);
+    }
+    return false;
+}
+
+#pragma clang fp contract(off)
+
+// blockIdx.x = row tile (cut per expert), blockIdx.y = column tile (E_SWIGLU: 32 columns of gate and the
+// same 32 of up, side by side in the tile)
+template <int BKIND, int EPI, bool GATHER>
+__global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) {
+    __shared__ __attribute__((aligned(16))) float lds[4 * STAGE];
+    int expert, m0, m_end;
+    if (!find_row_tile(p.cum, p.n_experts, blockIdx.x, expert, m0, m_end)) return;   // (the whole block: blockIdx only)
+    constexpr int COLS = EPI == E_SWIGLU ? TB / 2 : TB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int n0 = blockIdx.y * COLS;
+    const int steps = (p.kc + KS - 1) / KS;
+    // A: [row][c]
+    const int arow = m0 + slot_row<F_CONTIG>(tid), ac = slot_c<F_CONTIG>(tid);
+    const bool a_in = arow < m_end;
+    const int64_t a_src = !a_in ? 0 : GATHER ? p.row_index[arow] : arow;
+    auto fetch_a = [&](int s) {
+        const int ph = s >= steps ? 1 : 0, c = (s - ph * steps) * KS + ac;
+        return fetch8(p.A[ph] + a_src * p.lda + c, a_in && c < p.kc, a_in && c + 4 < p.kc);
+    };
+    // B: W[g] as [n][k] (forward) or [c][col] with c the contraction index (input gradient)
+    const int brow = slot_row<BKIND>(tid), bc = slot_c<BKIND>(tid);
+    const int64_t b0[2] = {expert * p.strideB[0], expert * p.strideB[1]};
+    auto fetch_b = [&](int s) {
+        const int ph = s >= steps ? 1 : 0, c = (s - ph * steps) * KS + bc;
+        if (BKIND == F_CONTIG) {
+            const int which = EPI == E_SWIGLU ? brow >> 5 : ph;
+            const int n = n0 + (EPI == E_SWIGLU ? brow & 31 : brow);
+            const bool in = n < p.n_cols;
+            return fetch8(p.B[which] + b0[which] + static_cast<int64_t>(n) * p.ldb + c, in && c < p.kc, in && c + 4 < p.kc);
+        }
+        const int n = n0 + brow;
+        return fetch8(p.B[ph] + b0[ph] + static_cast<int64_t>(c) * p.ldb + n, c < p.kc && n < p.n_cols, c < p.kc && n + 4 < p.n_cols);
+    };
+    f32x16 acc;
+    multiply<F_CONTIG, BKIND>(lds, steps * p.phases, wm, wn, fetch_a, fetch_b, acc);
+    const int m = m0 + wm + (lane & 31);
+    if (EPI == E_SWIGLU) {
+        // the up half goes to the wavefront that holds the gate half of the same rows and columns
+        __syncthreads();
+        float *ex = lds + (wave >> 1) * 16 * 64;
+        if (wn) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) ex[r * 64 + lane] = acc[r];
+        }
+        __syncthreads();
+        if (m >= m_end) return;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
+            const int n = n0 + q * 8 + (lane >> 5) * 4;
+            if (n >= p.n_cols) continue;
+            const int64_t o = static_cast<int64_t>(m) * p.ldc + n;
             f4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
-            const int64_t n = n0 + wn + q * 8 + (lane >> 5) * 4;
-            if (n >= n_end) continue;
-            f4 *dst = reinterpret_cast<f4 *>(C + m * ldc + n);
-            if (accumulate) v += *dst;
-            *dst = v;
+            *reinterpret_cast<f4 *>(p.C[wn ? 1 : 0] + o) = v;
+            if (wn) continue;
+            f4 h;
+#pragma unroll
+            for (int j = 0; j < 4; j++) h[j] = (v[j] / (1.0f + expf(-v[j]))) * ex[(q * 4 + j) * 64 + lane];
+            *reinterpret_cast<f4 *>(p.C[2] + o) = h;
+        }
+        return;
+    }
+    if (m >= m_end) return;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int n = n0 + wn + q * 8 + (lane >> 5) * 4;
+        if (n >= p.n_cols) continue;
+        const int64_t o = static_cast<int64_t>(m) * p.ldc + n;
+        f4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
+        if (EPI == E_SWIGLU_BWD) {
+            const f4 a = *reinterpret_cast<const f4 *>(p.G + o), b = *reinterpret_cast<const f4 *>(p.U + o);
+            f4 og, ou;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float sg = 1.0f / (1.0f + expf(-a[j]));
+                ou[j] = v[j] * (a[j] / (1.0f + expf(-a[j])));
+                og[j] = (v[j] * b[j]) * (sg * (1.0f + a[j] * (1.0f - sg)));
+            }
+            *reinterpret_cast<f4 *>(p.C[0] + o) = og;
+            *reinterpret_cast<f4 *>(p.C[1] + o) = ou;
+        } else {
+            *reinterpret_cast<f4 *>(p.C[0] + o) = v;
         }
     }
 }
 
-// blockIdx.x = row tile (cut per expert, located by a scan of cum), blockIdx.y = column tile
-template <int BKIND>
-__global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) {
-    __shared__ int s_expert, s_begin, s_end;
-    if (threadIdx.x == 0) {
-        int tile = blockIdx.x, found = -1, begin = 0, end = 0;
-        for (int e = 0; e < p.n_experts; e++) {
-            const int s = p.cum[e], cnt = p.cum[e + 1] - s;
-            const int tiles = (cnt + TB - 1) / TB;
-            if (tile < tiles) { found = e; begin = s + tile * TB; end = s + cnt; break; }
-            tile -= tiles;
-        }
-        s_expert = found; s_begin = begin; s_end = end;
-    }
-    __syncthreads();
-    const int expert = s_expert;
-    if (expert < 0) return;
-    const int64_t m0 = s_begin, m_end = s_end, n0 = static_cast<int64_t>(blockIdx.y) * TB;
-    const float *B = p.B + expert * p.strideB;
-    // fwd:   B = W[g] [n][k], operand rows n0.., contraction k
-    // dgrad: B = W[g] [c][col] with c the contraction index, operand rows n0..
-    tile_product<F_CONTIG, BKIND>(p.A, p.lda, m0, m_end, B, p.ldb, n0, p.n_cols, 0, p.kc, p.C, p.ldc, m0,
-                                  m_end, n0, p.n_cols);
-}
-
-// blockIdx = (column tile of dW, row tile of dW, expert): dW[g][n][k] = sum_r dout[r][n] * in[r][k]
+// blockIdx = (column tile of dW, row tile of dW, expert and which of up to two weight gradients):
+// dW[g][n][k] = sum_r dout[r][n] * in[r][k]
+template <bool GATHER>
 __global__ __launch_bounds__(256) void ggemm_f32_wgrad_kernel(const F32Params p) {
-    const int expert = blockIdx.z;
-    const int64_t r0 = p.cum[expert], r1 = p.cum[expert + 1];
-    const int64_t n0 = static_cast<int64_t>(blockIdx.y) * TB, k0 = static_cast<int64_t>(blockIdx.x) * TB;
-    float *C = p.C + expert * p.strideC;
-    const int64_t n_end = p.kc < n0 + TB ? p.kc : n0 + TB;   // rows of dW: the N extent
-    tile_product<F_STRIDED, F_STRIDED>(p.A, p.lda, n0, p.kc, p.B, p.ldb, k0, p.n_cols, r0, r1, C, p.ldc,
-                                       n0, n_end, k0, p.n_cols, p.accumulate != 0);
+    __shared__ __attribute__((aligned(16))) float lds[4 * STAGE];
+    const int expert = blockIdx.z % p.n_experts, which = blockIdx.z / p.n_experts;
+    const int r0 = p.cum[expert], r1 = p.cum[expert + 1];
+    const int n0 = blockIdx.y * TB, k0 = blockIdx.x * TB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int row = slot_row<F_STRIDED>(tid), c = slot_c<F_STRIDED>(tid);
+    auto fetch_a = [&](int s) {
+        const int r = r0 + s * KS + c;
+        return fetch8(p.A[which] + static_cast<int64_t>(r) * p.lda + n0 + row, r < r1 && n0 + row < p.kc, r < r1 && n0 + row + 4 < p.kc);
+    };
+    auto fetch_b = [&](int s) {
+        const int r = r0 + s * KS + c;
+        const int64_t src = r >= r1 ? 0 : GATHER ? p.row_index[r] : r;
+        return fetch8(p.B[0] + src * p.ldb + k0 + row, r < r1 && k0 + row < p.n_cols, r < r1 && k0 + row + 4 < p.n_cols);
+    };
+    f32x16 acc;
+    multiply<F_STRIDED, F_STRIDED>(lds, (r1 - r0 + KS - 1) / KS, wm, wn, fetch_a, fetch_b, acc);
+    float *C = p.C[which] + expert * p.strideC[which];
+    const int n = n0 + wm + (lane & 31);
+    if (n >= p.kc) return;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = k0 + wn + q * 8 + (lane >> 5) * 4;
+        if (k >= p.n_cols) continue;
+        f4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
+        f4 *dst = reinterpret_cast<f4 *>(C + static_cast<int64_t>(n) * p.ldc + k);
+        if ((p.accumulate >> which) & 1) v += *dst;
+        *dst = v;
+    }
 }
 
 inline bool mult8(int64_t v) { return v > 0 && v % 8 == 0; }
-inline unsigned tiles_of(int v) { return static_cast<unsigned>((v + TB - 1) / TB); }
+inline unsigned tiles_of(int v, int tile = TB) { return static_cast<unsigned>((v + tile - 1) / tile); }
 inline bool fits31(int64_t v) { return v >= 0 && v < (1LL << 31); }
+
+template <int BKIND, int EPI> int rows_launch(const F32Params &p, int64_t rows, void *stream) {
+    const int64_t m_tiles = (rows + TB - 1) / TB + p.n_experts;
+    const unsigned n_tiles = tiles_of(p.n_cols, EPI == E_SWIGLU ? TB / 2 : TB);
+    if (m_tiles > 0x7fffffffLL || n_tiles > 65535) return OM_ERR_SHAPE;
+    const dim3 grid(static_cast<unsigned>(m_tiles), n_tiles);
+    if (p.row_index) ggemm_f32_rows_kernel<BKIND, EPI, true><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
+    else ggemm_f32_rows_kernel<BKIND, EPI, false><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
+    return om_launch_status();
+}
 
 }  // namespace
 
@@ -140,16 +268,13 @@ extern "C" int om_grouped_gemm_fwd_f32(const float *input, const float *weight, 
     if (!input || !weight || !output || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(input) || !om_aligned16(weight) || !om_aligned16(output)) return OM_ERR_ALIGN;
     F32Params p = {};
-    p.A = input; p.B = weight; p.C = output; p.cum = cum_token_counts;
+    p.A[0] = input; p.B[0] = weight; p.C[0] = output; p.cum = cum_token_counts;
     p.lda = K; p.ldb = K; p.ldc = N;
-    p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
-    if (p.strideB % 4 != 0) return OM_ERR_ALIGN;
-    if (!fits31(rows * K) || !fits31(rows * N) || !fits31(p.strideB * G)) return OM_ERR_SHAPE;
-    p.n_experts = G; p.n_cols = N; p.kc = K;
-    const int64_t m_tiles = (rows + TB - 1) / TB + G;
-    if (m_tiles > 0x7fffffffLL || tiles_of(N) > 65535) return OM_ERR_SHAPE;
-    ggemm_f32_rows_kernel<F_CONTIG><<<dim3(static_cast<unsigned>(m_tiles), tiles_of(N)), dim3(256), 0, om_stream(stream)>>>(p);
-    return om_launch_status();
+    p.strideB[0] = w_stride ? w_stride : static_cast<int64_t>(N) * K;
+    if (p.strideB[0] % 4 != 0) return OM_ERR_ALIGN;
+    if (!fits31(rows * K) || !fits31(rows * N) || !fits31(p.strideB[0] * G)) return OM_ERR_SHAPE;
+    p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
+    return rows_launch<F_CONTIG, E_STORE>(p, rows, stream);
 }
 
 extern "C" int om_grouped_gemm_dgrad_f32(const float *output_grad, const float *weight, float *input_grad,
@@ -160,34 +285,106 @@ extern "C" int om_grouped_gemm_dgrad_f32(const float *output_grad, const float *
     if (!output_grad || !weight || !input_grad || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(output_grad) || !om_aligned16(weight) || !om_aligned16(input_grad)) return OM_ERR_ALIGN;
     F32Params p = {};
-    p.A = output_grad; p.B = weight; p.C = input_grad; p.cum = cum_token_counts;
+    p.A[0] = output_grad; p.B[0] = weight; p.C[0] = input_grad; p.cum = cum_token_counts;
     p.lda = N; p.ldb = K; p.ldc = K;   // din[r][k] = sum_n dout[r][n] * W[n][k]: B is [c = n][row = k]
-    p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
-    if (p.strideB % 4 != 0) return OM_ERR_ALIGN;
-    if (!fits31(rows * K) || !fits31(rows * N) || !fits31(p.strideB * G)) return OM_ERR_SHAPE;
-    p.n_experts = G; p.n_cols = K; p.kc = N;
-    const int64_t m_tiles = (rows + TB - 1) / TB + G;
-    if (m_tiles > 0x7fffffffLL || tiles_of(K) > 65535) return OM_ERR_SHAPE;
-    ggemm_f32_rows_kernel<F_STRIDED><<<dim3(static_cast<unsigned>(m_tiles), tiles_of(K)), dim3(256), 0, om_stream(stream)>>>(p);
-    return om_launch_status();
+    p.strideB[0] = w_stride ? w_stride : static_cast<int64_t>(N) * K;
+    if (p.strideB[0] % 4 != 0) return OM_ERR_ALIGN;
+    if (!fits31(rows * K) || !fits31(rows * N) || !fits31(p.strideB[0] * G)) return OM_ERR_SHAPE;
+    p.n_experts = G; p.n_cols = K; p.kc = N; p.phases = 1;
+    return rows_launch<F_STRIDED, E_STORE>(p, rows, stream);
+}
+
+// g = x Wg^T, u = x Wu^T, h = silu(g) * u in one launch; `x_rows` != null: row r of x is row x_rows[r] of
+// a [src_rows, H] matrix
+extern "C" int om_merged_mlp_gate_up_fwd_f32(const float *x, const int32_t *x_rows, int64_t src_rows, const float *w_gate,
+                                             const float *w_up, float *g, float *u, float *h,
+                                             const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                                             int64_t gate_stride, int64_t up_stride, void *stream) {
+    if (rows < 0 || G < 1 || !mult8(I) || !mult8(H)) return OM_ERR_SHAPE;
+    if (rows == 0) return OM_OK;
+    if (!x || !w_gate || !w_up || !g || !u || !h || !cum_token_counts) return OM_ERR_NULL;
+    if (!om_aligned16(x) || !om_aligned16(w_gate) || !om_aligned16(w_up) || !om_aligned16(g) || !om_aligned16(u) ||
+        !om_aligned16(h))
+        return OM_ERR_ALIGN;
+    if (x_rows && src_rows < 1) return OM_ERR_SHAPE;
+    F32Params p = {};
+    p.A[0] = x; p.B[0] = w_gate; p.B[1] = w_up; p.C[0] = g; p.C[1] = u; p.C[2] = h;
+    p.cum = cum_token_counts; p.row_index = x_rows;
+    p.lda = H; p.ldb = H; p.ldc = I;
+    p.strideB[0] = gate_stride ? gate_stride : static_cast<int64_t>(I) * H;
+    p.strideB[1] = up_stride ? up_stride : static_cast<int64_t>(I) * H;
+    if (p.strideB[0] % 4 != 0 || p.strideB[1] % 4 != 0) return OM_ERR_ALIGN;
+    if (!fits31((x_rows ? src_rows : rows) * H) || !fits31(rows * I) || !fits31(p.strideB[0] * G) || !fits31(p.strideB[1] * G)) return OM_ERR_SHAPE;
+    p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
+    return rows_launch<F_CONTIG, E_SWIGLU>(p, rows, stream);
+}
+
+// dg, du = SwiGLU backward of dh = dy W_down, in one launch
+extern "C" int om_merged_mlp_down_dgrad_f32(const float *dy, const float *w_down, const float *g, const float *u, float *dg,
+                                            float *du, const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                                            int64_t w_stride, void *stream) {
+    if (rows < 0 || G < 1 || !mult8(I) || !mult8(H)) return OM_ERR_SHAPE;
+    if (rows == 0) return OM_OK;
+    if (!dy || !w_down || !g || !u || !dg || !du || !cum_token_counts) return OM_ERR_NULL;
+    if (!om_aligned16(dy) || !om_aligned16(w_down) || !om_aligned16(g) || !om_aligned16(u) || !om_aligned16(dg) ||
+        !om_aligned16(du))
+        return OM_ERR_ALIGN;
+    F32Params p = {};
+    p.A[0] = dy; p.B[0] = w_down; p.C[0] = dg; p.C[1] = du; p.G = g; p.U = u; p.cum = cum_token_counts;
+    p.lda = H; p.ldb = I; p.ldc = I;   // B = W_down[g] [c = h][row = i]
+    p.strideB[0] = w_stride ? w_stride : static_cast<int64_t>(H) * I;
+    if (p.strideB[0] % 4 != 0) return OM_ERR_ALIGN;
+    if (!fits31(rows * H) || !fits31(rows * I) || !fits31(p.strideB[0] * G)) return OM_ERR_SHAPE;
+    p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
+    return rows_launch<F_STRIDED, E_SWIGLU_BWD>(p, rows, stream);
+}
+
+// dx = dg W_gate + du W_up, one accumulation over both
+extern "C" int om_merged_mlp_gate_up_dgrad_f32(const float *dg, const float *du, const float *w_gate, const float *w_up,
+                                               float *dx, const int32_t *cum_token_counts, int64_t rows, int G, int I,
+                                               int H, int64_t gate_stride, int64_t up_stride, void *stream) {
+    if (rows < 0 || G < 1 || !mult8(I) || !mult8(H)) return OM_ERR_SHAPE;
+    if (rows == 0) return OM_OK;
+    if (!dg || !du || !w_gate || !w_up || !dx || !cum_token_counts) return OM_ERR_NULL;
+    if (!om_aligned16(dg) || !om_aligned16(du) || !om_aligned16(w_gate) || !om_aligned16(w_up) || !om_aligned16(dx))
+        return OM_ERR_ALIGN;
+    F32Params p = {};
+    p.A[0] = dg; p.A[1] = du; p.B[0] = w_gate; p.B[1] = w_up; p.C[0] = dx; p.cum = cum_token_counts;
+    p.lda = I; p.ldb = H; p.ldc = H;
+    p.strideB[0] = gate_stride ? gate_stride : static_cast<int64_t>(I) * H;
+    p.strideB[1] = up_stride ? up_stride : static_cast<int64_t>(I) * H;
+    if (p.strideB[0] % 4 != 0 || p.strideB[1] % 4 != 0) return OM_ERR_ALIGN;
+    if (!fits31(rows * H) || !fits31(rows * I) || !fits31(p.strideB[0] * G) || !fits31(p.strideB[1] * G)) return OM_ERR_SHAPE;
+    p.n_experts = G; p.n_cols = H; p.kc = I; p.phases = 2;
+    return rows_launch<F_STRIDED, E_STORE>(p, rows, stream);
 }
 
 namespace {
-int wgrad_f32_launch(const float *output_grad, const float *input, float *weight_grad,
-                     const int32_t *cum_token_counts, int64_t rows, int G, int N, int K, int64_t w_stride,
-                     void *stream, bool accumulate) {
-    if (rows < 0 || G < 1 || G > 65535 || !mult8(N) || !mult8(K)) return OM_ERR_SHAPE;
-    if (!weight_grad || !cum_token_counts || (rows > 0 && (!output_grad || !input))) return OM_ERR_NULL;
-    if (!om_aligned16(output_grad) || !om_aligned16(input) || !om_aligned16(weight_grad)) return OM_ERR_ALIGN;
+// n_sets 1 or 2: dW[s] (+)= dout[s]^T in, over the same rows of `input` (through input_rows when given)
+int wgrad_f32_launch(int n_sets, const float *const *output_grad, const float *input, const int32_t *input_rows,
+                     int64_t src_rows, float *const *weight_grad, const int32_t *cum_token_counts, int64_t rows, int G,
+                     int N, int K, const int64_t *w_stride, void *stream, int accumulate) {
+    if (rows < 0 || G < 1 || n_sets * static_cast<int64_t>(G) > 65535 || !mult8(N) || !mult8(K)) return OM_ERR_SHAPE;
+    if (!cum_token_counts || (rows > 0 && !input)) return OM_ERR_NULL;
+    if (!om_aligned16(input)) return OM_ERR_ALIGN;
     F32Params p = {};
-    p.A = output_grad; p.B = input; p.C = weight_grad; p.cum = cum_token_counts;
+    for (int s = 0; s < n_sets; s++) {
+        if (!weight_grad[s] || (rows > 0 && !output_grad[s])) return OM_ERR_NULL;
+        if (!om_aligned16(output_grad[s]) || !om_aligned16(weight_grad[s])) return OM_ERR_ALIGN;
+        p.A[s] = output_grad[s];
+        p.C[s] = weight_grad[s];
+        p.strideC[s] = w_stride[s] ? w_stride[s] : static_cast<int64_t>(N) * K;
+        if (p.strideC[s] % 4 != 0) return OM_ERR_ALIGN;
+        if (!fits31(p.strideC[s] * G)) return OM_ERR_SHAPE;
+    }
+    p.B[0] = input; p.cum = cum_token_counts; p.row_index = input_rows;
     p.lda = N; p.ldb = K; p.ldc = K;
-    p.strideC = w_stride ? w_stride : static_cast<int64_t>(N) * K;
-    if (p.strideC % 4 != 0) return OM_ERR_ALIGN;
-    if (!fits31(rows * K) || !fits31(rows * N) || !fits31(p.strideC * G) || tiles_of(N) > 65535) return OM_ERR_SHAPE;
+    if (!fits31((input_rows ? src_rows : rows) * K) || !fits31(rows * N) || tiles_of(N) > 65535) return OM_ERR_SHAPE;
     p.n_experts = G; p.n_cols = K; p.kc = N;
-    p.accumulate = accumulate ? 1 : 0;
-    ggemm_f32_wgrad_kernel<<<dim3(tiles_of(K), tiles_of(N), G), dim3(256), 0, om_stream(stream)>>>(p);
+    p.accumulate = accumulate;
+    const dim3 grid(tiles_of(K), tiles_of(N), n_sets * G);
+    if (input_rows) ggemm_f32_wgrad_kernel<true><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
+    else ggemm_f32_wgrad_kernel<false><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
     return om_launch_status();
 }
 }  // namespace
@@ -195,14 +392,28 @@ int wgrad_f32_launch(const float *output_grad, const float *input, float *weight
 extern "C" int om_grouped_gemm_wgrad_f32(const float *output_grad, const float *input, float *weight_grad,
                                          const int32_t *cum_token_counts, int64_t rows, int G, int N, int K,
                                          int64_t w_stride, void *stream) {
-    return wgrad_f32_launch(output_grad, input, weight_grad, cum_token_counts, rows, G, N, K, w_stride, stream,
-                            false);
+    return wgrad_f32_launch(1, &output_grad, input, nullptr, 0, &weight_grad, cum_token_counts, rows, G, N, K, &w_stride,
+                            stream, 0);
 }
 
 extern "C" int om_grouped_gemm_wgrad_f32_accumulate(const float *output_grad, const float *input,
                                                     float *weight_grad, const int32_t *cum_token_counts,
                                                     int64_t rows, int G, int N, int K, int64_t w_stride,
                                                     void *stream) {
-    return wgrad_f32_launch(output_grad, input, weight_grad, cum_token_counts, rows, G, N, K, w_stride, stream,
-                            true);
+    return wgrad_f32_launch(1, &output_grad, input, nullptr, 0, &weight_grad, cum_token_counts, rows, G, N, K, &w_stride,
+                            stream, 1);
+}
+
+// dW_gate (+)= dg^T x (bit 0 of accumulate) and dW_up (+)= du^T x (bit 1) in one launch, the rows of x
+// through x_rows when given
+extern "C" int om_merged_mlp_gate_up_wgrad_f32(const float *dg, const float *du, const float *x, const int32_t *x_rows,
+                                               int64_t src_rows, float *dw_gate, float *dw_up,
+                                               const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                                               int64_t gate_stride, int64_t up_stride, int accumulate, void *stream) {
+    if (x_rows && rows > 0 && src_rows < 1) return OM_ERR_SHAPE;
+    const float *dout[2] = {dg, du};
+    float *dw[2] = {dw_gate, dw_up};
+    const int64_t strides[2] = {gate_stride, up_stride};
+    return wgrad_f32_launch(2, dout, x, x_rows, src_rows, dw, cum_token_counts, rows, G, I, H, strides, stream,
+                            accumulate);
 }

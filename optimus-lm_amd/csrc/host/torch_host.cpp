@@ -302,13 +302,6 @@ void gemm_dtype(const Tensor &a, const Tensor &b, const Tensor &c) {
 const float *fp(const Tensor &t) { return static_cast<const float *>(ptr(t)); }
 float *fpm(const Tensor &t) { return static_cast<float *>(ptr(t)); }
 
-Tensor gathered_rows(const Call &c, const Tensor &x, const int32_t *x_rows, int64_t rows) {
-    if (!x_rows) return x;
-    Tensor out = make({rows, x.size(1)}, x);
-    OM(c, om_index_gather, ptr(x), x_rows, ptr(out), rows, x.size(1), dtype_code(x), c.stream);
-    return out;
-}
-
 // y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment; with x_rows the MLP input is x[x_rows]
 Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const int32_t *cum, const int32_t *x_rows,
                       int64_t rows, MlpState &s) {
@@ -322,11 +315,8 @@ Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const
     Tensor y = make({rows, H}, x);
     ProfiledScope scope(c, "1moeblock--7gmlp_fwd");
     if (x.scalar_type() == at::kFloat) {
-        // float32 modules: three grouped GEMMs and the SwiGLU glue kernel
-        const Tensor xs = gathered_rows(c, x, x_rows, rows);
-        OM(c, om_grouped_gemm_fwd_f32, fp(xs), fp(w.gate), fpm(s.g), cum, rows, G, I, H, expert_stride(w.gate), c.stream);
-        OM(c, om_grouped_gemm_fwd_f32, fp(xs), fp(w.up), fpm(s.u), cum, rows, G, I, H, expert_stride(w.up), c.stream);
-        if (rows) OM(c, om_swiglu_fwd, ptr(s.g), ptr(s.u), ptr(s.h), rows * I, OM_F32, c.stream);
+        OM(c, om_merged_mlp_gate_up_fwd_f32, fp(x), rows ? x_rows : nullptr, x.size(0), fp(w.gate), fp(w.up), fpm(s.g),
+           fpm(s.u), fpm(s.h), cum, rows, G, I, H, expert_stride(w.gate), expert_stride(w.up), c.stream);
         OM(c, om_grouped_gemm_fwd_f32, fp(s.h), fp(w.down), fpm(y), cum, rows, G, H, I, expert_stride(w.down), c.stream);
         return y;
     }
@@ -386,16 +376,13 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
     Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx = make({rows, H}, x);
     ProfiledScope scope(c, "1moeblock--7gmlp_bwd");
     if (x.scalar_type() == at::kFloat) {
-        const Tensor xs = gathered_rows(c, x, x_rows, rows);
-        Tensor dh = make({rows, I}, x), dx2 = make({rows, H}, x);
         wgrad_f32(c, dy, s.h, k.down, cum, rows, G, H, I);
-        OM(c, om_grouped_gemm_dgrad_f32, fp(dy), fp(w.down), fpm(dh), cum, rows, G, H, I, expert_stride(w.down), c.stream);
-        if (rows) OM(c, om_swiglu_bwd, ptr(dh), ptr(s.g), ptr(s.u), ptr(dg), ptr(du), rows * I, OM_F32, c.stream);
-        wgrad_f32(c, dg, xs, k.gate, cum, rows, G, I, H);
-        wgrad_f32(c, du, xs, k.up, cum, rows, G, I, H);
-        OM(c, om_grouped_gemm_dgrad_f32, fp(dg), fp(w.gate), fpm(dx), cum, rows, G, I, H, expert_stride(w.gate), c.stream);
-        OM(c, om_grouped_gemm_dgrad_f32, fp(du), fp(w.up), fpm(dx2), cum, rows, G, I, H, expert_stride(w.up), c.stream);
-        dx.add_(dx2);
+        OM(c, om_merged_mlp_down_dgrad_f32, fp(dy), fp(w.down), fp(s.g), fp(s.u), fpm(dg), fpm(du), cum, rows, G, I, H,
+           expert_stride(w.down), c.stream);
+        OM(c, om_merged_mlp_gate_up_wgrad_f32, fp(dg), fp(du), fp(x), rows ? x_rows : nullptr, x.size(0), fpm(k.gate.grad),
+           fpm(k.up.grad), cum, rows, G, I, H, k.gate.pitch, k.up.pitch, k.gate.accumulate | k.up.accumulate << 1, c.stream);
+        OM(c, om_merged_mlp_gate_up_dgrad_f32, fp(dg), fp(du), fp(w.gate), fp(w.up), fpm(dx), cum, rows, G, I, H,
+           expert_stride(w.gate), expert_stride(w.up), c.stream);
         return dx;
     }
     wgrad(c, dy, s.h, k.down, cum, rows, G, H, I);
@@ -599,8 +586,8 @@ std::pair<Tensor, Tensor> gate_backward(const Call &c, const Tensor &x, const Te
         const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
         if (need_x) {
             dx = make(x.sizes(), x);
-            OM(c, om_router_gate_dgrad_f32, fp(dlogits), fp(weight), T, H, N, fpm(dx), c.stream);
-            if (other_grad.defined()) dx.add_(other_grad);
+            const Tensor base = other_grad.defined() ? other_grad.contiguous() : Tensor();
+            OM(c, om_router_gate_dgrad_f32_add, fp(dlogits), fp(weight), fp(base), T, H, N, fpm(dx), c.stream);
         }
         if (need_w) {
             dw = make(weight.sizes(), weight);

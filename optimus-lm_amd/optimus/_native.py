@@ -54,6 +54,7 @@ SIGNATURES = {
     "om_router_gate_dgrad": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p]),
     "om_router_gate_logits_f32": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_void_p]),
     "om_router_gate_dgrad_f32": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_void_p]),
+    "om_router_gate_dgrad_f32_add": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_void_p]),
     "om_router_gate_wgrad_f32": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_void_p]),
     "om_router_balance_workspace_bytes": (c_i64, [c_i64, c_int]),
     "om_router_balance_stats": (c_int, [c_void_p, c_int, c_i64, c_int, c_int, c_void_p, c_void_p,
@@ -141,6 +142,12 @@ SIGNATURES = {
                                          c_void_p, c_i64, c_int, c_int, c_int, c_i64, c_void_p]),
     "om_merged_mlp_gate_up_dgrad": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                             c_void_p, c_i64, c_int, c_int, c_int, c_i64, c_void_p]),
+    "om_merged_mlp_gate_up_fwd_f32": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 6 +
+                                      [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_void_p]),
+    "om_merged_mlp_down_dgrad_f32": (c_int, [c_void_p] * 7 + [c_i64, c_int, c_int, c_int, c_i64, c_void_p]),
+    "om_merged_mlp_gate_up_dgrad_f32": (c_int, [c_void_p] * 6 + [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_void_p]),
+    "om_merged_mlp_gate_up_wgrad_f32": (c_int, [c_void_p] * 4 + [c_i64] + [c_void_p] * 3 +
+                                        [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_int, c_void_p]),
     "om_swiglu_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_void_p]),
     "om_swiglu_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int,
                               c_void_p]),

@@ -435,3 +435,47 @@ def test_few_rows_kernels_give_the_bits_of_the_direct_load_kernels(cuda, N, K):
     assert float(res[0][0].float().abs().max()) > 0
     assert (bits(res[0][0]) == bits(res[1][0])).all()
     assert (bits(res[0][1]) == bits(res[1][1])).all()
+
+
+@pytest.mark.parametrize("T,K,N,start,end,I,H", [
+    (1, 1, 1, 0, 1, 8, 8),              # one row, one 8-wide step
+    (65, 2, 4, 0, 4, 72, 40),           # one row past a 64-row tile; extents between 32 and 64 and above
+    (300, 3, 12, 2, 9, 264, 136),       # an expert window; remainders along every extent
+    (40, 4, 80, 0, 80, 32, 64),         # more experts than a wavefront has lanes, some empty
+])
+@pytest.mark.parametrize("live", [False, True])
+def test_merged_mlp_float32_gathered(cuda, T, K, N, start, end, I, H, live):
+    """The float32 merged MLP through the token gather (om_merged_mlp_*_f32), forward and backward, against
+    float64.  Bound: a float32 dot product of n terms is off by about sqrt(n) 2^-24 of its norm (n <= 300:
+    1e-6), three products and the sigmoid in a chain: 1e-5 of the 2-norm.  `live`: the gate weight's
+    gradient is a view of a larger buffer and gets added into it, the others are fresh."""
+    from optimus.models.common.moe import GatheredMergedMLPFunction, build_token_permutation
+    g = torch.Generator().manual_seed(T + I)
+    G = end - start
+    se = torch.stack([torch.randperm(N, generator=g)[:K] for _ in range(T)])
+    cum, cum_ep, ii, oi, _ = build_token_permutation(se.to(cuda), start, end)
+    rows = int(cum[-1].item())
+    x = torch.randn(T, H, generator=g)
+    ws = [torch.randn(s, generator=g) * 0.2 for s in ((G, I, H), (G, I, H), (G, H, I))]
+    xd = x.to(cuda).requires_grad_(True)
+    wd = [w.to(cuda).requires_grad_(True) for w in ws]
+    before = torch.randn(G, I, H, generator=g)
+    if live:
+        wd[0].grad = torch.cat([before.flatten(), torch.zeros(8)]).to(cuda)[:-8].view(G, I, H)
+    y = GatheredMergedMLPFunction.apply(xd, ii[:rows], cum_ep, oi[:rows], *wd, cum)
+    dy = torch.randn(rows, H, generator=g)
+    y.backward(dy.to(cuda))
+    x64 = x.double().requires_grad_(True)
+    w64 = [w.double().requires_grad_(True) for w in ws]
+    c, idx = cum.cpu().tolist(), ii[:rows].cpu().long()
+    parts = []
+    for e in range(G):
+        xe = x64[idx[c[e]:c[e + 1]]]
+        parts.append((torch.nn.functional.silu(xe @ w64[0][e].t()) * (xe @ w64[1][e].t())) @ w64[2][e].t())
+    ref = torch.cat(parts)
+    ref.backward(dy.double())
+    want_gate = w64[0].grad + (before.double() if live else 0)
+    for got, want in ((y, ref), (xd.grad, x64.grad), (wd[0].grad, want_gate), (wd[1].grad, w64[1].grad),
+                      (wd[2].grad, w64[2].grad)):
+        err = (got.detach().double().cpu() - want.detach()).norm()
+        assert float(err) <= 1e-5 * float(want.detach().norm()) + 1e-12
