@@ -171,6 +171,22 @@ int om_router_gate_logits_split(const void *x, const void *gate_weight, int64_t 
                                 float *logits_out, void *workspace, int64_t workspace_bytes,
                                 void *stream);
 
+/* The whole router for a bf16 gate of any shape (N <= 256, H a multiple of 8): the projection split over
+ * slices of H, then one launch that adds the slices in order, writes the logits and routes.
+ *   om_router_gate_split_softmax_topk       : the softmax router above; logits_out in logits_dtype (OM_BF16:
+ *       rounded to bf16 before the softmax, the logits of a bf16 linear layer)
+ *   om_router_gate_split_sigmoid_group_topk : the DeepSeek-V3 router (om_route_sigmoid_group_topk below)
+ * workspace: om_router_gate_route_workspace_bytes(T,H,N) bytes, 16-byte aligned (negative = error code). */
+int64_t om_router_gate_route_workspace_bytes(int64_t T, int H, int N);
+int om_router_gate_split_softmax_topk(const void *x, const void *gate_weight, int64_t T, int H, int N, int K,
+                                      int norm_topk_prob, void *logits_out, int logits_dtype, void *weights_out,
+                                      int weights_dtype, int64_t *experts_out, void *workspace,
+                                      int64_t workspace_bytes, void *stream);
+int om_router_gate_split_sigmoid_group_topk(const void *x, const void *gate_weight, const float *bias, int64_t T, int H,
+                                            int N, int n_group, int topk_group, int K, int norm_topk_prob,
+                                            double routed_scaling_factor, float *logits_out, int64_t *experts_out,
+                                            float *weights_out, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* om_router_gate_wgrad: gradient of the gate's weight,
  *   dweight[n,h] = sum_t dlogits[t,n] * x[t,h]
  * i.e. what autograd computes for the nn.Linear behind `router_logits = self.gate(hidden_states)`
@@ -280,8 +296,16 @@ int om_route_sigmoid_topk_bwd(const float *logits, const int64_t *experts, const
  *   om_moe_row_weights_grad skip them, the expert GEMMs and the per-token sums only ever read
  *   entries below TR).
  * All outputs stay on the device; nothing is read back.
+ * om_moe_sort_weighted: the same, and when row_weights is not null row_weights[pos] (fp32, T*K entries) =
+ *   routing_weights[t,k] of the pair at sorted row pos (weights_dtype), what om_moe_row_weights makes of
+ *   the arrays.
  * workspace: om_moe_sort_workspace_bytes(T, K, NR) bytes, 4-byte aligned, no pre-zeroing. */
 int64_t om_moe_sort_workspace_bytes(int64_t T, int K, int NR);
+int om_moe_sort_weighted(const void *selected_experts, int index_dtype, int64_t T, int K, int expert_start_idx,
+                         int expert_end_idx, int32_t *cum_token_counts, int32_t *cum_expert_counts_ep,
+                         int32_t *input_indices, int32_t *output_indices, int32_t *selected_experts_indices,
+                         const void *routing_weights, int weights_dtype, float *row_weights, void *workspace,
+                         int64_t workspace_bytes, void *stream);
 int om_moe_sort(const void *selected_experts, int index_dtype, int64_t T, int K,
                 int expert_start_idx, int expert_end_idx, int32_t *cum_token_counts,
                 int32_t *cum_expert_counts_ep, int32_t *input_indices, int32_t *output_indices,

@@ -81,3 +81,9 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
 }
+
+// The split gate projection (gate_fwd.hip) as the routing kernels' producer (route.hip): slices of H, and
+// the launch that leaves partial[splits][T][N].  Arguments are checked by the caller.
+int om_gate_route_splits(int64_t T, int H, int N);
+void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, int splits, float *partial,
+                             hipStream_t stream);

@@ -166,6 +166,28 @@ inline int gate_split_count(int64_t T, int H) {
 
 }  // namespace
 
+// Behind a routing kernel that adds the slices itself: eight of them where the steps divide (the order of
+// the sums is then that of om_router_gate_softmax_topk, bit for bit), else as above.
+int om_gate_route_splits(int64_t T, int H, int N) {
+    const int steps = (H + GK - 1) / GK;
+    return N <= 64 && H % 512 == 0 && steps % 8 == 0 ? 8 : gate_split_count(T, H);
+}
+
+void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, int splits, float *ws,
+                             hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>((T + GT - 1) / GT), splits);
+    const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(gate_weight);
+    const int hps = (H + GK - 1) / GK / splits * GK;   // a whole number of steps; the last slice may end early
+    if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    else if (N <= 128) gate_logits_split_kernel<4><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    else gate_logits_split_kernel<8><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+}
+
+extern "C" int64_t om_router_gate_route_workspace_bytes(int64_t T, int H, int N) {
+    if (!gate_split_shape_ok(T, H, N)) return OM_ERR_SHAPE;
+    return static_cast<int64_t>(om_gate_route_splits(T, H, N)) * T * N * 4;
+}
+
 extern "C" int64_t om_router_gate_logits_split_workspace_bytes(int64_t T, int H, int N) {
     if (!gate_split_shape_ok(T, H, N)) return OM_ERR_SHAPE;
     return static_cast<int64_t>(gate_split_count(T, H)) * T * N * 4;
@@ -182,13 +204,8 @@ extern "C" int om_router_gate_logits_split(const void *x, const void *gate_weigh
     const int64_t tn = T * N;
     if (workspace_bytes < splits * tn * 4) return OM_ERR_WORKSPACE;
     hipStream_t st = om_stream(stream);
-    const dim3 grid(static_cast<unsigned>((T + GT - 1) / GT), splits);
-    const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(gate_weight);
     float *ws = static_cast<float *>(workspace);
-    const int hps = (H + GK - 1) / GK / splits * GK;   // a whole number of steps; the last slice may end early
-    if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
-    else if (N <= 128) gate_logits_split_kernel<4><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
-    else gate_logits_split_kernel<8><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    om_launch_gate_partials(x, gate_weight, T, H, N, splits, ws, st);
     gate_logits_reduce_kernel<<<dim3(static_cast<unsigned>((tn + 255) / 256)), dim3(256), 0, st>>>(ws, splits, tn, logits_out);
     return om_launch_status();
 }

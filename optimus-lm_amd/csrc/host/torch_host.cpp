@@ -233,11 +233,13 @@ struct Index {
         if (owners.size() == 1) {
             int32_t *p = owners[0].data_ptr<int32_t>();
             cum = p; cum_ep = p + NR + 1; in = cum_ep + T + 1; out = in + TK; sel = out + TK;
+            row_weights = reinterpret_cast<const float *>(sel + TK);
         } else {
             cum = iptr(owners[0]); cum_ep = iptr(owners[1]); in = iptr(owners[2]); out = iptr(owners[3]); sel = iptr(owners[4]);
         }
     }
     const int32_t *cum = nullptr, *cum_ep = nullptr, *in = nullptr, *out = nullptr, *sel = nullptr;
+    const float *row_weights = nullptr;   // the routing weight of every sorted row (one-buffer form only)
     int64_t rows = 0;               // entries of the three last: the routed rows, or an upper bound of them
     bool bound = false;
 };
@@ -256,21 +258,22 @@ std::vector<Tensor> sort_tensors(const Call &c, const Tensor &experts, int64_t s
     return r;
 }
 
-Index sort_index(const Call &c, const Tensor &experts, int64_t start, int64_t end) {
+Index sort_index(const Call &c, const Tensor &experts, int64_t start, int64_t end, const Tensor &rw) {
     require_device(experts);
-    const int64_t T = experts.size(0), K = experts.size(1), NR = end - start, TK = T * K;
-    const int64_t ws_bytes = om_moe_sort_workspace_bytes(T, K, NR);
-    const int64_t ws_at = (NR + 1 + T + 1 + 3 * TK + 3) & ~int64_t(3);
-    Tensor buf = at::empty({ws_at + std::max<int64_t>(ws_bytes / 4, 1)}, experts.options().dtype(at::kInt));
-    int32_t *p = buf.data_ptr<int32_t>();
-    int32_t *cum = p, *cum_ep = cum + NR + 1, *in = cum_ep + T + 1, *out = in + TK, *sel = out + TK;
-    OM(c, om_moe_sort, ptr(experts), index_code(experts), T, K, start, end, cum, cum_ep, in, out, sel, p + ws_at,
-       ws_bytes, c.stream);
+    require_device(rw);
     Index ix;
-    ix.owners = {buf};
-    ix.NR = NR; ix.T = T; ix.TK = TK;
+    const int64_t K = experts.size(1);
+    ix.T = experts.size(0);
+    ix.NR = end - start;
+    ix.TK = ix.rows = ix.T * K;
+    const int64_t ws_bytes = om_moe_sort_workspace_bytes(ix.T, K, ix.NR);
+    const int64_t ws_at = ix.NR + 1 + ix.T + 1 + 4 * ix.TK;
+    ix.owners = {at::empty({ws_at + std::max<int64_t>(ws_bytes / 4, 1)}, experts.options().dtype(at::kInt))};
     ix.resolve();
-    ix.rows = TK;
+    int32_t *p = ix.owners[0].data_ptr<int32_t>();
+    auto rwp = [](const auto *q) { return const_cast<std::remove_const_t<std::remove_pointer_t<decltype(q)>> *>(q); };
+    OM(c, om_moe_sort_weighted, ptr(experts), index_code(experts), ix.T, K, start, end, rwp(ix.cum), rwp(ix.cum_ep),
+       rwp(ix.in), rwp(ix.out), rwp(ix.sel), ptr(rw), dtype_code(rw), rwp(ix.row_weights), p + ws_at, ws_bytes, c.stream);
     return ix;
 }
 
@@ -408,15 +411,19 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
     require_bf16(w.down);
     const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
     const int64_t pitch = shared_pitch(w);
-    row_weights = make({rows}, x, at::kFloat);
     s.g = make({rows, I}, x);
     s.u = make({rows, I}, x);
     s.h = make({rows, I}, x);
     Tensor y = make({rows, H}, x), final = make({T, H}, x);
     {
         ProfiledScope scope(c, "1moeblock--7gmlp_fwd");
-        OM(c, om_moe_row_weights, ptr(rw), ix.sel, ix.in, ix.out, fpm(row_weights), rows, K, dtype_code(rw), c.stream);
-        OM(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), fp(row_weights), ptr(s.g),
+        const float *weights = ix.row_weights;
+        if (!weights) {
+            row_weights = make({rows}, x, at::kFloat);
+            weights = fp(row_weights);
+            OM(c, om_moe_row_weights, ptr(rw), ix.sel, ix.in, ix.out, fpm(row_weights), rows, K, dtype_code(rw), c.stream);
+        }
+        OM(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
            ptr(s.u), ptr(s.h), ix.cum, rows, G, I, H, pitch, c.stream);
         OM(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, G, H, I, expert_stride(w.down), c.stream);
     }
@@ -443,7 +450,7 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
             Tensor row_dot = make({parts, rows}, x, at::kFloat);
             wgrad(c, dfinal, s.h, k.down, ix.cum, rows, G, H, I, WgradRows::OUTPUT_GRAD, ix.in, T);
             OM(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
-               fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows, G, I, H, expert_stride(w.down), c.stream);
+               ix.row_weights ? ix.row_weights : fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows, G, I, H, expert_stride(w.down), c.stream);
             OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
                c.stream);
             wgrad(c, dg, x, k.gate, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
@@ -690,11 +697,17 @@ std::tuple<Tensor, Tensor> gate_logits(const Tensor &x, const Tensor &weight) {
     return {logits, x_out};
 }
 
-// softmax top-K router -> (routing_weights, selected_experts int64, logits, x).  `fused`: one launch for
+Tensor route_workspace(const Tensor &x, int64_t T, int64_t H, int64_t N) {
+    const int64_t bytes = om_router_gate_route_workspace_bytes(T, H, N);
+    if (bytes < 0) check(static_cast<int>(bytes), "om_router_gate_route_workspace_bytes");
+    return make({std::max<int64_t>(bytes, 16)}, x, at::kByte);
+}
+
+// softmax top-K router -> (routing_weights, selected_experts int64, logits, x).  `one_pass`: one launch for
 // projection and routing (shapes of om_router_gate_softmax_topk).  `bf16_logits`: the logits are rounded
 // to bf16 before the softmax, as a bf16 linear layer returns them.
 std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
-                                                         at::ScalarType out_dtype, bool fused, bool bf16_logits) {
+                                                         at::ScalarType out_dtype, bool one_pass, bool bf16_logits) {
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
     Tensor logits, weights, experts, x_out;
     {
@@ -704,15 +717,20 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
         require_device(weight);
         weights = make({T, top_k}, x, out_dtype);
         experts = make({T, top_k}, x, at::kLong);
-        if (fused) {
+        if (x.scalar_type() == at::kFloat) {
+            logits = gate_logits_forward(c, x, weight);
+            OM(c, om_route_softmax_topk, ptr(logits), dtype_code(logits), T, N, top_k, renorm, ptr(weights),
+               dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
+        } else if (one_pass) {
             logits = make({T, N}, x, at::kFloat);
             OM(c, om_router_gate_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, fpm(logits), ptr(weights),
                dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
         } else {
-            logits = gate_logits_forward(c, x, weight);
-            if (bf16_logits) logits = logits.to(at::kBFloat16);
-            OM(c, om_route_softmax_topk, ptr(logits), dtype_code(logits), T, N, top_k, renorm, ptr(weights),
-               dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
+            require_gate_shape(weight, "gate projection");
+            logits = make({T, N}, x, bf16_logits ? at::kBFloat16 : at::kFloat);
+            const Tensor ws = route_workspace(x, T, H, N);
+            OM(c, om_router_gate_split_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, ptr(logits),
+               dtype_code(logits), ptr(weights), dtype_code(weights), experts.data_ptr<int64_t>(), ptr(ws), ws.numel(), c.stream);
         }
         x_out = x.alias();
     }
@@ -736,11 +754,21 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
         at::AutoDispatchBelowADInplaceOrView below;
         const Call c = begin_call();
         require_device(bias);
-        logits = gate_logits_forward(c, x, weight);
+        require_device(x);
+        require_device(weight);
         weights = make({T, top_k}, x, at::kFloat);
         experts = make({T, top_k}, x, at::kLong);
-        OM(c, om_route_sigmoid_group_topk, fp(logits), fp(bias), T, N, n_group, topk_group, top_k, renorm, scale,
-           experts.data_ptr<int64_t>(), fpm(weights), c.stream);
+        if (x.scalar_type() == at::kFloat) {
+            logits = gate_logits_forward(c, x, weight);
+            OM(c, om_route_sigmoid_group_topk, fp(logits), fp(bias), T, N, n_group, topk_group, top_k, renorm, scale,
+               experts.data_ptr<int64_t>(), fpm(weights), c.stream);
+        } else {
+            require_gate_shape(weight, "gate projection");
+            logits = make({T, N}, x, at::kFloat);
+            const Tensor ws = route_workspace(x, T, x.size(1), N);
+            OM(c, om_router_gate_split_sigmoid_group_topk, ptr(x), ptr(weight), fp(bias), T, x.size(1), N, n_group, topk_group,
+               top_k, renorm, scale, fpm(logits), experts.data_ptr<int64_t>(), fpm(weights), ptr(ws), ws.numel(), c.stream);
+        }
         x_out = x.alias();
     }
     if (any_requires_grad({x, weight})) {
@@ -894,17 +922,18 @@ struct CountReadback {
     }
 };
 
-// Sort and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
+// Sort (with the routing weights laid out per sorted row) and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
 // sync_free: never read the routed-row count of an expert window back.
-Tensor moe_experts(const Tensor &x, const Tensor &rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
+Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
                    bool sync_free, const std::optional<Tensor> &residual, bool merged, const std::vector<Tensor> &leaves,
                    bool has_shared, const std::optional<Tensor> &one) {
     const Call c = begin_call();
     Index ix;
+    rw = rw.contiguous();
     {
         at::AutoDispatchBelowADInplaceOrView below;
         ProfiledScope scope(c, "1moeblock--3index_calculation");
-        ix = sort_index(c, experts, start, end);
+        ix = sort_index(c, experts, start, end, rw);
     }
     const bool windowed = !(start == 0 && end == n_total);
     if (windowed) {

@@ -72,16 +72,33 @@ __device__ __forceinline__ float fetch_expert_value(const float (&x)[PER], int e
     return out;
 }
 
-// softmax probabilities of this token's row into p[PER]; returns nothing else.
-template <int PER, typename T>
-__device__ __forceinline__ void row_softmax(const T *row, int N, int lane, float (&p)[PER]) {
-    float mx = -INFINITY;
+// The logits of token t of a gate projection that was split over H: the slices' partial sums
+// [splits][Tn][N] added in slice order; lanes past N get -inf.
+template <int PER>
+__device__ __forceinline__ void partial_logits(const float *partial, int splits, int64_t Tn, int64_t t, int N, int lane,
+                                               float (&x)[PER]) {
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int i = lane + 64 * j;
-        p[j] = (i < N) ? load_logit<T>(row + i) : -INFINITY;
-        mx = fmaxf(mx, p[j]);
+        x[j] = -INFINITY;
+        if (i >= N) continue;
+        float s = 0.0f;
+        for (int k0 = 0; k0 < splits; k0 += 8) {   // eight loads in flight
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = (k0 + u < splits) ? partial[((k0 + u) * Tn + t) * N + i] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; u++) s += v[u];
+        }
+        x[j] = s;
     }
+}
+
+// logits (lanes past N: -inf) -> softmax probabilities, in place
+template <int PER> __device__ __forceinline__ void softmax_in_place(int N, int lane, float (&p)[PER]) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < PER; j++) mx = fmaxf(mx, p[j]);
     mx = wave_max_dpp(mx);
     float sum = 0.0f;
 #pragma unroll
@@ -93,6 +110,17 @@ __device__ __forceinline__ void row_softmax(const T *row, int N, int lane, float
     sum = wave_sum(sum);
 #pragma unroll
     for (int j = 0; j < PER; j++) p[j] = p[j] / sum;
+}
+
+// softmax probabilities of this token's row into p[PER]; returns nothing else.
+template <int PER, typename T>
+__device__ __forceinline__ void row_softmax(const T *row, int N, int lane, float (&p)[PER]) {
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int i = lane + 64 * j;
+        p[j] = (i < N) ? load_logit<T>(row + i) : -INFINITY;
+    }
+    softmax_in_place<PER>(N, lane, p);
 }
 
 // K rounds of wave arg-max over s[PER] (entries with index >= N must be < every real score).
@@ -128,6 +156,39 @@ __global__ __launch_bounds__(256) void softmax_topk_kernel(const T *__restrict__
     if (t >= Tn) return;
     float p[PER];
     row_softmax<PER, T>(logits + t * N, N, lane, p);
+    float w; int e;
+    select_topk<PER>(p, N, K, lane, w, e);
+    if (renorm) {
+        const float s = wave_sum(lane < K ? w : 0.0f);
+        w = w / s;
+    }
+    if (lane < K) {
+        Elem<TW>::store(weights_out + t * K + lane, w);
+        experts_out[t * K + lane] = e;
+    }
+}
+
+// The same behind a gate projection that was split over H: adds the slices, writes the logits (rounded to
+// TL first, which is what the softmax then sees) and routes.  One launch instead of a reduction, a
+// conversion and a routing launch, each of which is a few microseconds of latency for a small batch.
+template <int PER, typename TL, typename TW>
+__global__ __launch_bounds__(256) void partial_softmax_topk_kernel(const float *__restrict__ partial, int splits, int64_t Tn,
+                                                                   int N, int K, int renorm, TL *__restrict__ logits_out,
+                                                                   TW *__restrict__ weights_out,
+                                                                   int64_t *__restrict__ experts_out) {
+    const int lane = threadIdx.x & 63;
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * TOKENS_PER_BLOCK + (threadIdx.x >> 6);
+    if (t >= Tn) return;
+    float p[PER];
+    partial_logits<PER>(partial, splits, Tn, t, N, lane, p);
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int i = lane + 64 * j;
+        if (i >= N) continue;
+        Elem<TL>::store(logits_out + t * N + i, p[j]);
+        if (sizeof(TL) == 2) p[j] = bf16_bits_to_f32(f32_to_bf16_bits(p[j]));
+    }
+    softmax_in_place<PER>(N, lane, p);
     float w; int e;
     select_topk<PER>(p, N, K, lane, w, e);
     if (renorm) {
@@ -183,9 +244,10 @@ __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(const T *__restri
 
 // DeepSeek-V3 group-limited routing.  LDS holds the choice scores of the 4 tokens of the block
 // so a lane can scan "its" group; everything else stays in registers.
-template <int PER>
+// PARTIAL: the logits are the sum of a split gate projection's slices and are written out.
+template <int PER, bool PARTIAL>
 __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
-    const float *__restrict__ logits, const float *__restrict__ bias, int64_t Tn, int N, int n_group,
+    const float *__restrict__ logits, int splits, float *__restrict__ logits_out, const float *__restrict__ bias, int64_t Tn, int N, int n_group,
     int topk_group, int K, int renorm, float scale, int64_t *__restrict__ experts_out,
     float *__restrict__ weights_out) {
     __shared__ float choice_lds[TOKENS_PER_BLOCK][PER * 64];
@@ -193,12 +255,14 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
     const int wv = threadIdx.x >> 6;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * TOKENS_PER_BLOCK + wv;
     if (t >= Tn) return;  // whole wavefront leaves together; no block-wide barrier below
-    float score[PER], choice[PER];
+    float score[PER], choice[PER], row[PER];
+    if (PARTIAL) partial_logits<PER>(logits, splits, Tn, t, N, lane, row);
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int i = lane + 64 * j;
         if (i < N) {
-            const float x = logits[t * N + i];
+            const float x = PARTIAL ? row[j] : logits[t * N + i];
+            if (PARTIAL) logits_out[t * N + i] = x;
             score[j] = 1.0f / (1.0f + expf(-x));
             choice[j] = score[j] + bias[i];
             choice_lds[wv][i] = choice[j];
@@ -558,8 +622,8 @@ extern "C" int om_route_sigmoid_group_topk(const float *logits, const float *bia
     hipStream_t st = om_stream(stream);
     const unsigned nb = token_blocks(T);
     const float scale = static_cast<float>(routed_scaling_factor);
-    OM_DISPATCH_PER(N, (sigmoid_group_topk_kernel<PER><<<nb, 256, 0, st>>>(
-                           logits, bias, T, N, n_group, topk_group, K, norm_topk_prob, scale,
+    OM_DISPATCH_PER(N, (sigmoid_group_topk_kernel<PER, false><<<nb, 256, 0, st>>>(
+                           logits, 0, nullptr, bias, T, N, n_group, topk_group, K, norm_topk_prob, scale,
                            experts_out, weights_out)));
     return om_launch_status();
 }
@@ -596,6 +660,70 @@ extern "C" int om_router_gate_softmax_topk(const void *x, const void *gate_weigh
                                         weights_out, experts_out, st);
     return launch_gate<true, uint16_t>(x, gate_weight, T, H, N, K, norm_topk_prob, logits_out,
                                        weights_out, experts_out, st);
+}
+
+namespace {
+// What the two entry points below have in common: the projection's slices into the workspace.
+int gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, void *workspace, int64_t workspace_bytes,
+                  void *stream, int &splits) {
+    const int64_t need = om_router_gate_route_workspace_bytes(T, H, N);
+    if (need < 0) return static_cast<int>(need);
+    if (!x || !gate_weight || !workspace) return OM_ERR_NULL;
+    if (!om_aligned16(x) || !om_aligned16(gate_weight) || !om_aligned16(workspace)) return OM_ERR_ALIGN;
+    if (workspace_bytes < need) return OM_ERR_WORKSPACE;
+    splits = om_gate_route_splits(T, H, N);
+    om_launch_gate_partials(x, gate_weight, T, H, N, splits, static_cast<float *>(workspace), om_stream(stream));
+    return OM_OK;
+}
+}  // namespace
+
+extern "C" int om_router_gate_split_softmax_topk(const void *x, const void *gate_weight, int64_t T, int H, int N, int K,
+                                                 int norm_topk_prob, void *logits_out, int logits_dtype,
+                                                 void *weights_out, int weights_dtype, int64_t *experts_out,
+                                                 void *workspace, int64_t workspace_bytes, void *stream) {
+    if ((weights_dtype != OM_F32 && weights_dtype != OM_BF16) || (logits_dtype != OM_F32 && logits_dtype != OM_BF16))
+        return OM_ERR_DTYPE;
+    if (T < 0 || N < 1 || K < 1 || K > N || K > 64) return OM_ERR_SHAPE;
+    if (T == 0) return OM_OK;
+    if (!logits_out || !weights_out || !experts_out) return OM_ERR_NULL;
+    int splits = 0;
+    const int rc = gate_partials(x, gate_weight, T, H, N, workspace, workspace_bytes, stream, splits);
+    if (rc != OM_OK) return rc;
+    hipStream_t st = om_stream(stream);
+    const unsigned nb = token_blocks(T);
+    const float *part = static_cast<const float *>(workspace);
+#define OM_PR(TL, TW)                                                                                     \
+    OM_DISPATCH_PER(N, (partial_softmax_topk_kernel<PER, TL, TW><<<nb, 256, 0, st>>>(                     \
+                           part, splits, T, N, K, norm_topk_prob, static_cast<TL *>(logits_out),          \
+                           static_cast<TW *>(weights_out), experts_out)))
+    if (logits_dtype == OM_F32 && weights_dtype == OM_F32) { OM_PR(float, float); }
+    else if (logits_dtype == OM_F32) { OM_PR(float, uint16_t); }
+    else if (weights_dtype == OM_F32) { OM_PR(uint16_t, float); }
+    else { OM_PR(uint16_t, uint16_t); }
+#undef OM_PR
+    return om_launch_status();
+}
+
+extern "C" int om_router_gate_split_sigmoid_group_topk(const void *x, const void *gate_weight, const float *bias, int64_t T,
+                                                       int H, int N, int n_group, int topk_group, int K,
+                                                       int norm_topk_prob, double routed_scaling_factor,
+                                                       float *logits_out, int64_t *experts_out, float *weights_out,
+                                                       void *workspace, int64_t workspace_bytes, void *stream) {
+    if (T < 0 || N < 1 || K < 1 || K > N || K > 64 || n_group < 1 || n_group > 64 || N % n_group != 0 ||
+        topk_group < 1 || topk_group > n_group)
+        return OM_ERR_SHAPE;
+    if (T == 0) return OM_OK;
+    if (!bias || !logits_out || !experts_out || !weights_out) return OM_ERR_NULL;
+    int splits = 0;
+    const int rc = gate_partials(x, gate_weight, T, H, N, workspace, workspace_bytes, stream, splits);
+    if (rc != OM_OK) return rc;
+    hipStream_t st = om_stream(stream);
+    const unsigned nb = token_blocks(T);
+    const float scale = static_cast<float>(routed_scaling_factor);
+    OM_DISPATCH_PER(N, (sigmoid_group_topk_kernel<PER, true><<<nb, 256, 0, st>>>(
+                           static_cast<const float *>(workspace), splits, logits_out, bias, T, N, n_group, topk_group, K,
+                           norm_topk_prob, scale, experts_out, weights_out)));
+    return om_launch_status();
 }
 
 extern "C" int om_router_gate_logits(const void *x, const void *gate_weight, int64_t T, int H, int N,

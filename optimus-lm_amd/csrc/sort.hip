@@ -1,6 +1,6 @@
 // Token permutation for the fast MoE block: a stable counting sort of the (token, k) pairs by
 // local expert, producing exactly the arrays the reference builds with its two index kernels and
-// two cumsums.  Three small launches:
+// two cumsums.  Up to 8192 pairs are one launch of one block (sort_small_kernel); more are three:
 //   count   — every block histograms its chunk of pairs per expert (wave ballots -> LDS);
 //   scan    — one block (16 wavefront-wide scans at a time) turns the [block][expert] table into exclusive offsets in
 //             (expert-major, block-minor) order = the stable order, and writes cum_token_counts;
@@ -20,6 +20,19 @@ constexpr int SORT_WAVES = SORT_THREADS / 64;
 constexpr int SORT_ITERS = 8;                                    // 64-pair steps per wavefront
 constexpr int SORT_CHUNK = SORT_THREADS * SORT_ITERS;            // pairs per block
 constexpr int SORT_MAX_NR = 1024;                                // local experts supported
+
+// The routing weight of every sorted row, for expert kernels that apply it themselves: row_weights[pos] =
+// routing_weights[pair], float32 or bf16 -> float32.  Absent (row_weights null) where nobody asks for it.
+struct RowWeights {
+    const void *routing_weights = nullptr;
+    float *row_weights = nullptr;
+    int bf16 = 0;
+    __device__ __forceinline__ void put(int pos, int64_t pair) const {
+        if (!row_weights) return;
+        row_weights[pos] = bf16 ? bf16_bits_to_f32(static_cast<const uint16_t *>(routing_weights)[pair])
+                                : static_cast<const float *>(routing_weights)[pair];
+    }
+};
 
 template <typename TI>
 __device__ __forceinline__ int local_key(const TI *selected_experts, int64_t j, int64_t n_pairs,
@@ -152,7 +165,7 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
     const TI *__restrict__ selected_experts, int64_t n_pairs, int K, int start, int end, int NR,
     int nbits, const int32_t *__restrict__ block_offsets, const int32_t *__restrict__ hits_base,
     int32_t *__restrict__ cum_expert_counts_ep, int32_t *__restrict__ input_indices,
-    int32_t *__restrict__ output_indices, int32_t *__restrict__ selected_experts_indices) {
+    int32_t *__restrict__ output_indices, int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
     extern __shared__ int lds[];  // [SORT_WAVES][NR] then [SORT_WAVES] wave hit counts
     int *wave_hits = lds + SORT_WAVES * NR;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -203,8 +216,101 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
             input_indices[pos] = static_cast<int32_t>(t);
             output_indices[oi] = pos;
             selected_experts_indices[oi] = k;
+            rw.put(pos, j);
         } else {
             __builtin_amdgcn_wave_barrier();
+        }
+        oi_base += __popcll(kept);
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (up to 8 x 64)
+// pairs' keys and ranks in registers between the passes.  A decode batch or a small training batch spends
+// nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced),
+// one of 6 now.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront)
+// reaches what the three launches take.
+constexpr int SMALL_WAVES = 16;
+constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SORT_ITERS;
+constexpr int SMALL_MAX_NR = 256;
+template <typename TI>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
+    const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits, int iters,
+    int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
+    int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
+    int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
+    __shared__ int off[SMALL_WAVES][SMALL_MAX_NR];   // counts, then running offsets
+    __shared__ int wave_hits[SMALL_WAVES], chunk_total[SMALL_MAX_NR / 64], kept_total;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    for (int i = tid; i < SMALL_WAVES * NR; i += SMALL_WAVES * 64) off[i / NR][i % NR] = 0;
+    const int base = wv * iters * 64;
+    int key[SORT_ITERS];
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++)
+        key[it] = it < iters ? local_key(selected_experts, base + it * 64 + lane, n_pairs, start, end, NR) : NR;
+    __syncthreads();
+    volatile int *mine = off[wv];
+    int hits = 0;
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++) {
+        if (it >= iters) break;
+        const unsigned long long m = match_key(key[it], nbits);
+        if (key[it] < NR && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] += __popcll(m);
+        hits += __popcll(__ballot(key[it] < NR));
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (lane == 0) wave_hits[wv] = hits;
+    __syncthreads();
+    // thread e: expert e's total over the wavefronts, exclusive positions of the wavefronts within it
+    int total = 0;
+    if (tid < NR)
+        for (int w = 0; w < SMALL_WAVES; w++) {
+            const int c = off[w][tid];
+            off[w][tid] = total;
+            total += c;
+        }
+    const int incl = wave_incl_scan(total, lane);
+    if (tid < SMALL_MAX_NR && lane == 63) chunk_total[wv] = incl;
+    __syncthreads();
+    int before = incl - total;   // rows of the experts before this one
+    for (int w = 0; w < wv && w < SMALL_MAX_NR / 64; w++) before += chunk_total[w];
+    if (tid < NR) {
+        for (int w = 0; w < SMALL_WAVES; w++) off[w][tid] += before;
+        cum_token_counts[tid] = before;
+        if (tid == NR - 1) {
+            cum_token_counts[NR] = before + total;
+            cum_expert_counts_ep[n_pairs / K] = before + total;
+            kept_total = before + total;
+        }
+    }
+    __syncthreads();
+    int oi_base = 0;
+    for (int w = 0; w < wv; w++) oi_base += wave_hits[w];
+    const int kept_all = kept_total;
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++) {
+        if (it >= iters) break;
+        const int j = base + it * 64 + lane;
+        if (j < n_pairs && j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
+            output_indices[j] = -1;
+            input_indices[j] = 0;
+            selected_experts_indices[j] = 0;
+        }
+        const unsigned long long m = match_key(key[it], nbits);
+        const unsigned long long kept = __ballot(key[it] < NR);
+        const int oi = oi_base + __popcll(kept & lanemask_lt(lane));
+        const bool valid = j < n_pairs;
+        const int t = valid ? j / K : 0, k = valid ? j - t * K : 0;
+        if (valid && k == 0) cum_expert_counts_ep[t] = oi;
+        int pos = 0;
+        if (key[it] < NR) pos = mine[key[it]] + __popcll(m & lanemask_lt(lane));
+        __builtin_amdgcn_wave_barrier();
+        if (key[it] < NR) {
+            if ((__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] += __popcll(m);
+            input_indices[pos] = t;
+            output_indices[oi] = pos;
+            selected_experts_indices[oi] = k;
+            rw.put(pos, j);
         }
         oi_base += __popcll(kept);
         __builtin_amdgcn_wave_barrier();
@@ -334,9 +440,24 @@ namespace {
 int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, int K,
                     int expert_start_idx, int expert_end_idx, int32_t *cum_token_counts,
                     int32_t *cum_expert_counts_ep, int32_t *input_indices, int32_t *output_indices,
-                    int32_t *selected_experts_indices, int32_t *workspace, hipStream_t st) {
+                    int32_t *selected_experts_indices, int32_t *workspace, hipStream_t st,
+                    const RowWeights &rw = RowWeights()) {
     const int NR = expert_end_idx - expert_start_idx;
     const int64_t n_pairs = T * K;
+    if (n_pairs > 0 && n_pairs <= SMALL_PAIRS && NR <= SMALL_MAX_NR) {
+        const int iters = static_cast<int>((n_pairs + SMALL_WAVES * 64 - 1) / (SMALL_WAVES * 64));
+        if (index_dtype == OM_I64)
+            sort_small_kernel<int64_t><<<1, SMALL_WAVES * 64, 0, st>>>(
+                static_cast<const int64_t *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx,
+                expert_end_idx, NR, key_bits(NR), iters, cum_token_counts, cum_expert_counts_ep, input_indices,
+                output_indices, selected_experts_indices, rw);
+        else
+            sort_small_kernel<int32_t><<<1, SMALL_WAVES * 64, 0, st>>>(
+                static_cast<const int32_t *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx,
+                expert_end_idx, NR, key_bits(NR), iters, cum_token_counts, cum_expert_counts_ep, input_indices,
+                output_indices, selected_experts_indices, rw);
+        return om_launch_status();
+    }
     const int64_t NB = (n_pairs + SORT_CHUNK - 1) / SORT_CHUNK;
     int32_t *block_hist = workspace;
     int32_t *hits_base = block_hist + NB * NR;
@@ -360,12 +481,12 @@ int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, in
             sort_scatter_kernel<int64_t><<<static_cast<unsigned>(NB), SORT_THREADS, lds_scatter, st>>>(
                 static_cast<const int64_t *>(selected_experts), n_pairs, K, expert_start_idx,
                 expert_end_idx, NR, nbits, block_hist, hits_base, cum_expert_counts_ep, input_indices,
-                output_indices, selected_experts_indices);
+                output_indices, selected_experts_indices, rw);
         else
             sort_scatter_kernel<int32_t><<<static_cast<unsigned>(NB), SORT_THREADS, lds_scatter, st>>>(
                 static_cast<const int32_t *>(selected_experts), n_pairs, K, expert_start_idx,
                 expert_end_idx, NR, nbits, block_hist, hits_base, cum_expert_counts_ep, input_indices,
-                output_indices, selected_experts_indices);
+                output_indices, selected_experts_indices, rw);
     }
     return om_launch_status();
 }
@@ -386,21 +507,40 @@ int moe_sort_check(const void *selected_experts, int index_dtype, int64_t T, int
 
 }  // namespace
 
+extern "C" int om_moe_sort_weighted(const void *selected_experts, int index_dtype, int64_t T, int K,
+                                    int expert_start_idx, int expert_end_idx, int32_t *cum_token_counts,
+                                    int32_t *cum_expert_counts_ep, int32_t *input_indices,
+                                    int32_t *output_indices, int32_t *selected_experts_indices,
+                                    const void *routing_weights, int weights_dtype, float *row_weights,
+                                    void *workspace, int64_t workspace_bytes, void *stream) {
+    const int rc = moe_sort_check(selected_experts, index_dtype, T, K, expert_start_idx, expert_end_idx,
+                                  cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
+                                  selected_experts_indices);
+    if (rc != OM_OK) return rc;
+    if (row_weights) {
+        if (weights_dtype != OM_F32 && weights_dtype != OM_BF16) return OM_ERR_DTYPE;
+        if (T > 0 && !routing_weights) return OM_ERR_NULL;
+    }
+    if (workspace_bytes < om_moe_sort_workspace_bytes(T, K, expert_end_idx - expert_start_idx))
+        return OM_ERR_WORKSPACE;
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 3u)) return OM_ERR_ALIGN;
+    RowWeights rw;
+    rw.routing_weights = routing_weights;
+    rw.row_weights = row_weights;
+    rw.bf16 = weights_dtype == OM_BF16;
+    return moe_sort_launch(selected_experts, index_dtype, T, K, expert_start_idx, expert_end_idx,
+                           cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
+                           selected_experts_indices, static_cast<int32_t *>(workspace), om_stream(stream), rw);
+}
+
 extern "C" int om_moe_sort(const void *selected_experts, int index_dtype, int64_t T, int K,
                            int expert_start_idx, int expert_end_idx, int32_t *cum_token_counts,
                            int32_t *cum_expert_counts_ep, int32_t *input_indices,
                            int32_t *output_indices, int32_t *selected_experts_indices,
                            void *workspace, int64_t workspace_bytes, void *stream) {
-    const int rc = moe_sort_check(selected_experts, index_dtype, T, K, expert_start_idx, expert_end_idx,
-                                  cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
-                                  selected_experts_indices);
-    if (rc != OM_OK) return rc;
-    if (workspace_bytes < om_moe_sort_workspace_bytes(T, K, expert_end_idx - expert_start_idx))
-        return OM_ERR_WORKSPACE;
-    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 3u)) return OM_ERR_ALIGN;
-    return moe_sort_launch(selected_experts, index_dtype, T, K, expert_start_idx, expert_end_idx,
-                           cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
-                           selected_experts_indices, static_cast<int32_t *>(workspace), om_stream(stream));
+    return om_moe_sort_weighted(selected_experts, index_dtype, T, K, expert_start_idx, expert_end_idx, cum_token_counts,
+                                cum_expert_counts_ep, input_indices, output_indices, selected_experts_indices, nullptr,
+                                OM_F32, nullptr, workspace, workspace_bytes, stream);
 }
 
 // ---- om_moe_sort for callers that cannot allocate ----------------------------------------------

@@ -48,6 +48,12 @@ SIGNATURES = {
     "om_router_gate_logits_split_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
     "om_router_gate_logits_split": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_void_p,
                                             c_i64, c_void_p]),
+    "om_router_gate_route_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
+    "om_router_gate_split_softmax_topk": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int, c_void_p, c_int,
+                                                  c_void_p, c_int, c_void_p, c_void_p, c_i64, c_void_p]),
+    "om_router_gate_split_sigmoid_group_topk": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int,
+                                                        c_int, c_int, c_double, c_void_p, c_void_p, c_void_p, c_void_p,
+                                                        c_i64, c_void_p]),
     "om_router_gate_wgrad_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
     "om_router_gate_wgrad": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_void_p, c_int, c_void_p,
                                      c_i64, c_void_p]),
@@ -75,6 +81,8 @@ SIGNATURES = {
     "om_moe_sort_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
     "om_moe_sort": (c_int, [c_void_p, c_int, c_i64, c_int, c_int, c_int, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_void_p]),
+    "om_moe_sort_weighted": (c_int, [c_void_p, c_int, c_i64, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
+                                     c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_i64, c_void_p]),
     "om_moe_sort_static_capacity_bytes": (c_i64, []),
     "om_moe_sort_static": (c_int, [c_void_p, c_int, c_i64, c_int, c_int, c_int, c_void_p, c_void_p,
                                    c_void_p, c_void_p, c_void_p, c_void_p]),
@@ -164,7 +172,7 @@ launch_filter = None   # optional set of entry-point names: only these are timed
 _UNTIMED = {"om_version", "om_arch", "om_strerror", "om_moe_sort_workspace_bytes",
             "om_moe_sort_static_capacity_bytes",
             "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes",
-            "om_router_gate_wgrad_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
+            "om_router_gate_wgrad_workspace_bytes", "om_router_gate_route_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
             "om_merged_mlp_row_dot_parts"}
 
 

@@ -442,3 +442,25 @@ def test_float32_gate_kernels_match_float64_products(cuda, T, H, N):
         err = (got.detach().double().cpu() - ref).abs()
         bound = k * eps * absum + 1e-30
         assert bool((err <= bound).all()), (name, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 2048, 64, 8), (129, 512, 32, 4), (33, 1000, 12, 3), (5, 8, 3, 3), (300, 7168, 256, 8),
+                                     (64, 64, 100, 1)])
+@pytest.mark.parametrize("bf16_logits", [False, True])
+def test_split_gate_router_equals_its_steps(cuda, T, H, N, K, bf16_logits):
+    """om_router_gate_split_softmax_topk against the projection (to the fp32 order of the sum) and, bit for
+    bit, against the router on its own logits; the logits are rounded to bf16 where asked for."""
+    from optimus import _native as n
+    from optimus.models.common.moe import SoftmaxTopkRouterFunction, fp32_logits
+    x, w = _gate_inputs(T, H, N, seed=T + H)
+    x, w = x.to(cuda), w.to(cuda)
+    we, e, logits, x_out = n.host().route_softmax(x, w, K, True, torch.bfloat16, False, bf16_logits)
+    assert logits.dtype == (torch.bfloat16 if bf16_logits else torch.float32) and x_out.data_ptr() == x.data_ptr()
+    w2, e2 = SoftmaxTopkRouterFunction.apply(logits, K, True, torch.bfloat16)
+    assert torch.equal(e, e2) and torch.equal(we.view(torch.int16), w2.view(torch.int16))
+    ref = x.double() @ w.double().t()
+    # fp32 sum of H exact products in another order, then (bf16) one rounding of 2^-9
+    bound = 8 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + (2.0 ** -8 * ref.abs() if bf16_logits else 0)
+    assert bool(((logits.double() - ref).abs() <= bound + 1e-30).all())
+    if not bf16_logits and N <= 64 and H % 512 == 0:
+        assert torch.equal(logits, fp32_logits(x, w))       # eight slices in order: the one-pass kernel's bits

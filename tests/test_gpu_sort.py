@@ -126,3 +126,41 @@ def test_moe_sort_random_shapes(cuda, oracle_lib, seed):
     assert np.array_equal(ii[:TR], ref["input_indices"]), tag
     assert np.array_equal(oi[:TR], ref["output_indices"]), tag
     assert np.array_equal(si[:TR], ref["selected_experts_indices"]), tag
+
+
+@pytest.mark.parametrize("T,N,K,start,end", [
+    (1, 8, 2, 0, 8), (1, 64, 8, 0, 64),
+    (1024, 64, 8, 0, 64), (8192, 40, 1, 3, 37),           # 8192 pairs: the most the one-block sort takes
+    (2731, 64, 3, 0, 64),                                 # 8193: the three-launch sort
+    (700, 300, 8, 10, 266), (700, 300, 8, 10, 267),       # 256 and 257 local experts
+])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_weighted_sort_on_both_sides_of_the_one_block_line(cuda, oracle_lib, T, N, K, start, end, dt):
+    """om_moe_sort_weighted: the arrays bit for bit against the restatement, the unused tail marked, and
+    every sorted row's routing weight exact."""
+    from optimus import _native as n
+    se = routed_experts(T, N, K, seed=T + N, skew=0.7)
+    ref = oracle_lib.index_construction(se.numpy(), end - start, start, end, tokens_per_thread=1)
+    w = torch.rand(T, K, generator=torch.Generator().manual_seed(T)).to(dt)
+    NR, P = end - start, T * K
+    i32 = dict(dtype=torch.int32, device=cuda)
+    cum, cum_ep = torch.full((NR + 1,), -7, **i32), torch.full((T + 1,), -7, **i32)
+    ii, oi, si = (torch.full((P,), -7, **i32) for _ in range(3))
+    rows = torch.full((P,), -7.0, device=cuda)
+    sed, wd = se.to(cuda), w.to(cuda)
+    ws_bytes = int(n.lib().om_moe_sort_workspace_bytes(T, K, NR))
+    ws = torch.empty(max(ws_bytes // 4, 1), **i32)
+    n.check(n.lib().om_moe_sort_weighted(n.ptr(sed), n.OM_I64, T, K, start, end, n.ptr(cum), n.ptr(cum_ep), n.ptr(ii),
+                                         n.ptr(oi), n.ptr(si), n.ptr(wd), n.dtype_code(wd), n.ptr(rows), n.ptr(ws),
+                                         ws_bytes, n.stream()), "om_moe_sort_weighted")
+    torch.cuda.synchronize()
+    TR = ref["num_routed_tokens"]
+    for got, name in ((cum, "cum_token_counts"), (cum_ep, "cum_expert_counts_ep"), (ii[:TR], "input_indices"),
+                      (oi[:TR], "output_indices"), (si[:TR], "selected_experts_indices")):
+        assert np.array_equal(got.cpu().numpy(), ref[name]), name
+    assert bool((oi[TR:] == -1).all()) and bool((ii[TR:] == 0).all()) and bool((si[TR:] == 0).all())
+    t = ii[:TR].long()
+    pos = oi[:TR].long()
+    want = torch.empty(TR, device=cuda)
+    want[pos] = wd[t[pos], si[:TR].long()].float()
+    assert torch.equal(rows[:TR], want)
