@@ -599,7 +599,7 @@ def bench_adamw(args, device):
         lg, _native.launch_log = _native.launch_log, None
         return sum(a.elapsed_time(b) for nm, a, b in lg if nm in names) / reps * 1e-3
 
-    t_norm = timed(lambda: plan.run(st["grad"]), ("om_grad_sumsq", "om_grad_norm_clip_coef"))
+    t_norm = timed(lambda: plan.run(st["grad"]), ("om_grad_sumsq", "om_grad_norm_clip_coef", "om_grad_norm"))
     t_clip = {}
     for store in (True, False):
         t_clip[store] = timed(lambda: adamw_step_(
@@ -636,7 +636,7 @@ def bench_adamw(args, device):
         adamw_step_(sh["param"], sh["grad"], sh["master"], sh["exp_avg"], sh["exp_avg_sq"], hp["step_id"] + 1,
                     hp["lr"], hp["betas"][0], hp["betas"][1], hp["eps"], hp["weight_decay"],
                     grad_scale=clip_buf[1:2], store_scaled_grad=True)
-    t_shard = timed(shard_step, ("om_grad_sumsq", "om_grad_norm_clip_coef", "om_shard_clip_multiplier",
+    t_shard = timed(shard_step, ("om_grad_sumsq", "om_grad_norm_clip_coef", "om_grad_norm", "om_shard_clip_multiplier",
                                  "om_adamw_step_clipped"))
     sharded = {"what": "one rank's shard of C2 under 8-way sharding: shard norm, device-side clip decision, "
                        "clipped update storing the scaled gradient (4 launches, 32 B/param)",

@@ -96,6 +96,14 @@ int om_grad_norm_clip_coef(const float *partials, const int64_t *seg_first_chunk
                            int64_t n_segs, int grad_dtype, double max_norm, float *seg_norms,
                            float *total_norm, float *clip_coef, void *stream);
 
+/* om_grad_norm: both of the above in one launch for small buffers (om_grad_norm_fits(n_chunks, n_segs) != 0):
+ * the block that finishes last takes the norms.  total_cast (may be null): the total norm in the gradient
+ * dtype.  blocks_done: one device word, zero before the first call, left zero by every call.          */
+int om_grad_norm_fits(int64_t n_chunks, int64_t n_segs);
+int om_grad_norm(const void *grad, int grad_dtype, const int64_t *chunk_offsets, int64_t n_chunks,
+                 const int64_t *seg_first_chunk, int64_t n_segs, double max_norm, float *partials, float *seg_norms,
+                 float *total_norm, float *clip_coef, void *total_cast, unsigned *blocks_done, void *stream);
+
 /* om_grad_scale: grad = cast(float(grad) * *coef) in place over n elements, coef a device fp32
  * scalar (the clip_coef above): the in-place multiply of clip_grads_with_norm_
  * (optimizers.py:145/150/154) for gradient tensors that no update kernel reads (parameters of the

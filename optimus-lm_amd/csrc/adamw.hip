@@ -3,6 +3,7 @@
 // v 4 + param 2 = 28 bytes (bf16 mode).  Each fp32 operation is rounded on its own (no FMA
 // contraction) so the result is reproducible bit for bit by a scalar CPU loop.
 #include "common.h"
+#include <type_traits>
 
 namespace {
 
@@ -48,6 +49,38 @@ template <typename T> __device__ __forceinline__ void stream_store(T *p, T v) { 
 // (the traffic probe writes back what it read and must keep its stores).
 __device__ __forceinline__ void opaque(f32x4 &v) { asm volatile("" : "+v"(v)); }
 
+// Elements past the last full vector of 4 (at most 3), taken by the lane that would own that vector.
+__device__ __forceinline__ void adam_tail(uint16_t *param, const uint16_t *grad, uint16_t *grad_store, float coef, bool clip,
+                                          float *master, float *exp_avg, float *exp_avg_sq, int64_t start, int64_t n,
+                                          const AdamScalars &s) {
+    for (int64_t i = start; i < n; i++) {
+        float m = exp_avg[i], v = exp_avg_sq[i], w = master[i];
+        float g = bf16_bits_to_f32(grad[i]);
+        if (clip) {
+            const uint16_t gb = f32_to_bf16_bits(g * coef);
+            g = bf16_bits_to_f32(gb);
+            if (grad_store) grad_store[i] = gb;
+        }
+        adam_update(g, m, v, w, s);
+        exp_avg[i] = m; exp_avg_sq[i] = v; master[i] = w;
+        param[i] = f32_to_bf16_bits(w);
+    }
+}
+__device__ __forceinline__ void adam_tail(float *master, const float *grad, float *grad_store, float coef, bool clip,
+                                          float *exp_avg, float *exp_avg_sq, int64_t start, int64_t n,
+                                          const AdamScalars &s) {
+    for (int64_t i = start; i < n; i++) {
+        float m = exp_avg[i], v = exp_avg_sq[i], w = master[i];
+        float g = grad[i];
+        if (clip) {
+            g = g * coef;
+            if (grad_store) grad_store[i] = g;
+        }
+        adam_update(g, m, v, w, s);
+        exp_avg[i] = m; exp_avg_sq[i] = v; master[i] = w;
+    }
+}
+
 // CLIP selects what happens to the gradient before the update (reference optimizers.py:136-152,
 // torch.nn.utils.clip_grads_with_norm_): 0 = used as is; 1 = multiplied by *grad_scale and rounded
 // back to the gradient dtype, as the in-place multiply of the bf16 gradient views does; 2 = the
@@ -55,7 +88,9 @@ __device__ __forceinline__ void opaque(f32x4 &v) { asm volatile("" : "+v"(v)); }
 // source and the destination).
 // MATH = false is the traffic probe: the same loads and stores with the arithmetic left out (the
 // fp32 states are written back as read, param = bf16(master)).
-template <int CLIP, bool MATH>
+// TAIL: the lane after the last full vector takes the elements behind it (a branch that the large launches
+// do without: it costs them 1-2 %).
+template <int CLIP, bool MATH, bool TAIL>
 __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__restrict__ param,
                                                                       const uint16_t *__restrict__ grad,
                                                                       uint16_t *grad_rw,
@@ -63,12 +98,16 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__r
                                                                       float *__restrict__ master,
                                                                       float *__restrict__ exp_avg,
                                                                       float *__restrict__ exp_avg_sq,
-                                                                      int64_t n_vec4, AdamScalars s) {
+                                                                      int64_t n_vec4, int64_t n, AdamScalars s) {
     const int64_t c = static_cast<int64_t>(blockIdx.x) * ADAMW_THREADS + threadIdx.x;
-    if (c >= n_vec4) return;
     const uint16_t *gsrc = CLIP == 2 ? grad_rw : grad;
     float coef = 1.0f;
     if (CLIP) coef = *grad_scale;
+    if (c >= n_vec4) {
+        if (TAIL && c == n_vec4)
+            adam_tail(param, gsrc, CLIP == 2 ? grad_rw : nullptr, coef, CLIP != 0, master, exp_avg, exp_avg_sq, c * 4, n, s);
+        return;
+    }
     const u32x2 gq = stream_load(reinterpret_cast<const u32x2 *>(gsrc) + c);
     f32x4 m0 = stream_load(reinterpret_cast<const f32x4 *>(exp_avg) + c);
     f32x4 v0 = stream_load(reinterpret_cast<const f32x4 *>(exp_avg_sq) + c);
@@ -112,39 +151,24 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__r
     stream_store(reinterpret_cast<u32x2 *>(param) + c, pk);
 }
 
-// Elements past the last full vector of 4 (at most 3).
-__global__ void adamw_bf16_tail_kernel(uint16_t *param, uint16_t *grad, const float *grad_scale,
-                                       int store_grad, float *master, float *exp_avg,
-                                       float *exp_avg_sq, int64_t start, int64_t n, AdamScalars s) {
-    const int64_t i = start + threadIdx.x;
-    if (i < n) {
-        float m = exp_avg[i], v = exp_avg_sq[i], w = master[i];
-        float g = bf16_bits_to_f32(grad[i]);
-        if (grad_scale) {
-            const uint16_t gb = f32_to_bf16_bits(g * *grad_scale);
-            g = bf16_bits_to_f32(gb);
-            if (store_grad) grad[i] = gb;
-        }
-        adam_update(g, m, v, w, s);
-        exp_avg[i] = m; exp_avg_sq[i] = v; master[i] = w;
-        param[i] = f32_to_bf16_bits(w);
-    }
-}
-
 // fp32 mode: the parameter buffer is the master buffer (16 B read, 12 B written per element).
-template <int CLIP>
+template <int CLIP, bool TAIL>
 __global__ __launch_bounds__(ADAMW_THREADS) void adamw_f32_kernel(float *__restrict__ master,
                                                                   const float *__restrict__ grad,
                                                                   float *grad_rw,
                                                                   const float *__restrict__ grad_scale,
                                                                   float *__restrict__ exp_avg,
                                                                   float *__restrict__ exp_avg_sq,
-                                                                  int64_t n_vec4, AdamScalars s) {
+                                                                  int64_t n_vec4, int64_t n, AdamScalars s) {
     const int64_t c = static_cast<int64_t>(blockIdx.x) * ADAMW_THREADS + threadIdx.x;
-    if (c >= n_vec4) return;
     const float *gsrc = CLIP == 2 ? grad_rw : grad;
     float coef = 1.0f;
     if (CLIP) coef = *grad_scale;
+    if (c >= n_vec4) {
+        if (TAIL && c == n_vec4)
+            adam_tail(master, gsrc, CLIP == 2 ? grad_rw : nullptr, coef, CLIP != 0, exp_avg, exp_avg_sq, c * 4, n, s);
+        return;
+    }
     f32x4 g = stream_load(reinterpret_cast<const f32x4 *>(gsrc) + c);
     f32x4 m = stream_load(reinterpret_cast<const f32x4 *>(exp_avg) + c);
     f32x4 v = stream_load(reinterpret_cast<const f32x4 *>(exp_avg_sq) + c);
@@ -163,21 +187,6 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_f32_kernel(float *__restr
     stream_store(reinterpret_cast<f32x4 *>(exp_avg) + c, m);
     stream_store(reinterpret_cast<f32x4 *>(exp_avg_sq) + c, v);
     stream_store(reinterpret_cast<f32x4 *>(master) + c, w);
-}
-__global__ void adamw_f32_tail_kernel(float *master, float *grad, const float *grad_scale,
-                                      int store_grad, float *exp_avg, float *exp_avg_sq,
-                                      int64_t start, int64_t n, AdamScalars s) {
-    const int64_t i = start + threadIdx.x;
-    if (i < n) {
-        float m = exp_avg[i], v = exp_avg_sq[i], w = master[i];
-        float g = grad[i];
-        if (grad_scale) {
-            g = g * *grad_scale;
-            if (store_grad) grad[i] = g;
-        }
-        adam_update(g, m, v, w, s);
-        exp_avg[i] = m; exp_avg_sq[i] = v; master[i] = w;
-    }
 }
 
 }  // namespace
@@ -231,45 +240,41 @@ static int adamw_launch(void *param, void *grad, float *master, float *exp_avg, 
 
     hipStream_t st = om_stream(stream);
     const int64_t n_vec = n / 4;
-    const int64_t blocks = (n_vec + ADAMW_THREADS - 1) / ADAMW_THREADS;
+    // A launch that fits the chip at full occupancy (32 wavefronts on each of 256 CUs) is over in one wave of
+    // blocks and bound by latency, not by the queues that the residency bound keeps short, and takes its tail
+    // along: 1.3e6 float32 elements 9.5 + 3 us as two bounded launches, 7 as one.  A larger one leaves the
+    // tail to a second launch over the last few elements.
+    constexpr int64_t SMALL_BLOCKS = 256 * 32;
+    const int64_t tail = n - n_vec * 4;
+    const bool small = (n_vec + ADAMW_THREADS) / ADAMW_THREADS <= SMALL_BLOCKS;
+    const bool with_tail = small && tail > 0;
+    const int64_t lanes = n_vec + (with_tail ? 1 : 0), blocks = (lanes + ADAMW_THREADS - 1) / ADAMW_THREADS;
     if (blocks * ADAMW_THREADS >= (1LL << 32)) return OM_ERR_SHAPE;   // (not reached: see MAX_PER_LAUNCH)
-    const dim3 grid(static_cast<unsigned>(blocks)), block(ADAMW_THREADS);
-    if (param_dtype == OM_BF16) {
-        uint16_t *p = static_cast<uint16_t *>(param), *g = static_cast<uint16_t *>(grad);
-        if (n_vec > 0) {
-            if (clip == ADAMW_PROBE)
-                adamw_bf16_kernel<0, false><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(p, g, nullptr, nullptr, master, exp_avg,
-                                                                    exp_avg_sq, n_vec, s);
-            else if (clip == 0)
-                adamw_bf16_kernel<0, true><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(p, g, nullptr, nullptr, master, exp_avg,
-                                                                   exp_avg_sq, n_vec, s);
-            else if (clip == 1)
-                adamw_bf16_kernel<1, true><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(p, g, nullptr, grad_scale, master, exp_avg,
-                                                                   exp_avg_sq, n_vec, s);
-            else
-                adamw_bf16_kernel<2, true><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(p, nullptr, g, grad_scale, master, exp_avg,
-                                                                   exp_avg_sq, n_vec, s);
+    const size_t lds = small ? 0 : ADAMW_OCCUPANCY_LDS;
+    const dim3 block(ADAMW_THREADS);
+    // `lo`: first element, `vecs` full vectors and (TAIL) the elements up to `count`
+    auto go = [&](auto tail_tag, unsigned grid, int64_t lo, int64_t vecs, int64_t count) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        float *w = master + lo, *m = exp_avg + lo, *v = exp_avg_sq + lo;
+        if (param_dtype == OM_BF16) {
+            uint16_t *p = static_cast<uint16_t *>(param) + lo, *g = static_cast<uint16_t *>(grad) + lo;
+            if (clip == ADAMW_PROBE) adamw_bf16_kernel<0, false, false><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
+            else if (clip == 0) adamw_bf16_kernel<0, true, TAIL><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
+            else if (clip == 1) adamw_bf16_kernel<1, true, TAIL><<<grid, block, lds, st>>>(p, g, nullptr, grad_scale, w, m, v, vecs, count, s);
+            else adamw_bf16_kernel<2, true, TAIL><<<grid, block, lds, st>>>(p, nullptr, g, grad_scale, w, m, v, vecs, count, s);
+        } else {
+            float *g = static_cast<float *>(grad) + lo;
+            if (clip == 0) adamw_f32_kernel<0, TAIL><<<grid, block, lds, st>>>(w, g, nullptr, nullptr, m, v, vecs, count, s);
+            else if (clip == 1) adamw_f32_kernel<1, TAIL><<<grid, block, lds, st>>>(w, g, nullptr, grad_scale, m, v, vecs, count, s);
+            else adamw_f32_kernel<2, TAIL><<<grid, block, lds, st>>>(w, nullptr, g, grad_scale, m, v, vecs, count, s);
         }
-        if (n_vec * 4 < n && clip != ADAMW_PROBE)
-            adamw_bf16_tail_kernel<<<1, 64, 0, st>>>(p, g, clip ? grad_scale : nullptr, clip == 2,
-                                                     master, exp_avg, exp_avg_sq, n_vec * 4, n, s);
+    };
+    if (param_dtype == OM_F32 && clip == ADAMW_PROBE) return OM_ERR_DTYPE;
+    if (with_tail) {
+        go(std::true_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
     } else {
-        if (clip == ADAMW_PROBE) return OM_ERR_DTYPE;
-        float *g = static_cast<float *>(grad);
-        if (n_vec > 0) {
-            if (clip == 0)
-                adamw_f32_kernel<0><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(master, g, nullptr, nullptr, exp_avg, exp_avg_sq,
-                                                            n_vec, s);
-            else if (clip == 1)
-                adamw_f32_kernel<1><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(master, g, nullptr, grad_scale, exp_avg,
-                                                            exp_avg_sq, n_vec, s);
-            else
-                adamw_f32_kernel<2><<<grid, block, ADAMW_OCCUPANCY_LDS, st>>>(master, nullptr, g, grad_scale, exp_avg,
-                                                            exp_avg_sq, n_vec, s);
-        }
-        if (n_vec * 4 < n)
-            adamw_f32_tail_kernel<<<1, 64, 0, st>>>(master, g, clip ? grad_scale : nullptr, clip == 2,
-                                                    exp_avg, exp_avg_sq, n_vec * 4, n, s);
+        if (n_vec > 0) go(std::false_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
+        if (tail > 0 && clip != ADAMW_PROBE) go(std::true_type(), 1u, n_vec * 4, 0, tail);
     }
     return om_launch_status();
 }

@@ -33,6 +33,8 @@ SIGNATURES = {
     "om_grad_sumsq": (c_int, [c_void_p, c_int, c_void_p, c_i64, c_void_p, c_void_p]),
     "om_grad_norm_clip_coef": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_double, c_void_p, c_void_p,
                                        c_void_p, c_void_p]),
+    "om_grad_norm_fits": (c_int, [c_i64, c_i64]),
+    "om_grad_norm": (c_int, [c_void_p, c_int, c_void_p, c_i64, c_void_p, c_i64, c_double] + [c_void_p] * 7),
     "om_grad_scale": (c_int, [c_void_p, c_i64, c_int, c_void_p, c_void_p]),
     "om_shard_clip_multiplier": (c_int, [c_void_p, c_int, c_int, c_double, c_void_p, c_void_p, c_void_p]),
     "om_adamw_step_clipped": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64,
@@ -173,7 +175,7 @@ _UNTIMED = {"om_version", "om_arch", "om_strerror", "om_moe_sort_workspace_bytes
             "om_moe_sort_static_capacity_bytes",
             "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes",
             "om_router_gate_wgrad_workspace_bytes", "om_router_gate_route_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
-            "om_merged_mlp_row_dot_parts"}
+            "om_merged_mlp_row_dot_parts", "om_grad_norm_fits"}
 
 
 class NativeLibraryError(RuntimeError):

@@ -133,6 +133,7 @@ class MixedPrecisionAdamW(Optimizer):
         self._norm_plan = GradNormPlan(self.param_start_inds, self.param_sizes, device) \
             if self.flat_param_size > 0 else None
         self._foreign_plans = {}
+        self._owned = {id(p) for p in self.param_list}
 
     def zero_grad(self):
         self.flat_grad.zero_()
@@ -142,8 +143,7 @@ class MixedPrecisionAdamW(Optimizer):
         reference takes the norm, and clips, over model.parameters(), optimizers.py:143-158)."""
         if self.model is None:
             return []
-        owned = {id(p) for p in self.param_list}
-        return [p.grad for p in self.model.parameters() if id(p) not in owned and p.grad is not None]
+        return _n.host().foreign_grads(self.model, self._owned)
 
     def _grad_norm_and_clip(self):
         """Gradient norm (always) and the clip to 1.0 (after warm-up), reference
@@ -158,12 +158,13 @@ class MixedPrecisionAdamW(Optimizer):
         if self._norm_plan is None and not foreign:
             zero = torch.zeros((), dtype=self.flat_grad.dtype, device=self.device)
             return zero, None
+        norm = torch.empty((), dtype=self.flat_grad.dtype, device=self.flat_grad.device)
         total, coef = run_grad_norm(self._norm_plan, self.flat_grad, foreign, self._foreign_plans,
-                                    max_norm=1.0)
+                                    max_norm=1.0, norm_out=norm)
         if clip_now:
             for g in foreign:
                 scale_grad_(g, coef)
-        return total.to(self.flat_grad.dtype, copy=True), (coef if clip_now else None)
+        return norm, (coef if clip_now else None)
 
     def step(self, closure=None):
         with record_pcl_function("3dp-comms-1grad_acc-block"):
@@ -457,7 +458,10 @@ class GradNormPlan:
     CHUNK = 1 << 16
 
     def __init__(self, starts, sizes, device, chunk=None):
-        chunk = int(chunk or self.CHUNK)
+        # two blocks per CU for a small buffer (a chunk is one block's work), 64 K elements each for a large one
+        if chunk is None:
+            chunk = min(self.CHUNK, max(4096, 1 << (sum(int(sz) for sz in sizes) // 512).bit_length()))
+        chunk = int(chunk)
         if len(sizes) == 0 or len(starts) != len(sizes):
             raise ValueError("GradNormPlan needs one (start, size) pair per parameter")
         begins, first, pos = [], [0], int(starts[0])
@@ -474,23 +478,36 @@ class GradNormPlan:
         self.n_segs = len(sizes)
         self.chunk_offsets = table.to(device)
         self.seg_first_chunk = torch.tensor(first, dtype=torch.int64).to(device)
+        self.one_launch = bool(_n.lib().om_grad_norm_fits(self.n_chunks, self.n_segs))
+        # one buffer: total norm, clip coefficient, the one-launch kernel's block count (starts at zero)
+        self._words = torch.zeros(3, dtype=torch.float32, device=device)
+        self.total, self.coef = self._words[0], self._words[1:2]
         self.partials = torch.empty(max(self.n_chunks, 1), dtype=torch.float32, device=device)
         self.seg_norms = torch.empty(self.n_segs, dtype=torch.float32, device=device)
-        self.out = torch.empty(2, dtype=torch.float32, device=device)   # total norm, clip coef
 
-    def run(self, flat_grad, max_norm=1.0):
+    def run(self, flat_grad, max_norm=1.0, norm_out=None):
         """Returns (total_norm, clip_coef) as 0-dim float32 device tensors (views of one buffer
-        that the next call overwrites)."""
+        that the next call overwrites).  `norm_out`: a 0-dim tensor of the gradient dtype that receives
+        the total norm too."""
         _n.require_cuda_contiguous(flat_grad)
+        if self.one_launch:
+            _n.check(_n.lib().om_grad_norm(
+                _n.ptr(flat_grad), _n.dtype_code(flat_grad), _n.ptr(self.chunk_offsets), self.n_chunks,
+                _n.ptr(self.seg_first_chunk), self.n_segs, float(max_norm), _n.ptr(self.partials),
+                _n.ptr(self.seg_norms), _n.ptr(self._words), _n.ptr(self._words) + 4, _n.ptr(norm_out),
+                _n.ptr(self._words) + 8, _n.stream()), "om_grad_norm")
+            return self.total, self.coef
         code = _n.dtype_code(flat_grad)
         lib = _n.lib()
         _n.check(lib.om_grad_sumsq(_n.ptr(flat_grad), code, _n.ptr(self.chunk_offsets), self.n_chunks,
                                    _n.ptr(self.partials), _n.stream()), "om_grad_sumsq")
         _n.check(lib.om_grad_norm_clip_coef(_n.ptr(self.partials), _n.ptr(self.seg_first_chunk),
                                             self.n_segs, code, float(max_norm), _n.ptr(self.seg_norms),
-                                            _n.ptr(self.out), _n.ptr(self.out) + 4, _n.stream()),
+                                            _n.ptr(self._words), _n.ptr(self._words) + 4, _n.stream()),
                  "om_grad_norm_clip_coef")
-        return self.out[0], self.out[1:2]
+        if norm_out is not None:
+            norm_out.copy_(self.total)
+        return self.total, self.coef
 
 
 def scale_grad_(grad, coef):
@@ -503,12 +520,12 @@ def scale_grad_(grad, coef):
                                     _n.stream()), "om_grad_scale")
 
 
-def run_grad_norm(plan, flat_grad, foreign, cache, max_norm=1.0):
+def run_grad_norm(plan, flat_grad, foreign, cache, max_norm=1.0, norm_out=None):
     """Total gradient norm and clip coefficient over flat_grad's parameters (through `plan`, may be
     None) followed by the tensors in `foreign`, each counted as one more parameter.  `cache` keeps
     the foreign tensors' chunk tables between steps."""
     if not foreign:
-        return plan.run(flat_grad, max_norm)
+        return plan.run(flat_grad, max_norm, norm_out)
     dtype = flat_grad.dtype
     for g in foreign:
         if g.dtype != dtype:
@@ -518,7 +535,10 @@ def run_grad_norm(plan, flat_grad, foreign, cache, max_norm=1.0):
     if joint is None:
         cache.clear()
         joint = cache[key] = JointGradNormPlan(plan, [g.numel() for g in foreign], flat_grad.device)
-    return joint.run(flat_grad, foreign, max_norm)
+    total, coef = joint.run(flat_grad, foreign, max_norm)
+    if norm_out is not None:
+        norm_out.copy_(total)
+    return total, coef
 
 
 class JointGradNormPlan:
