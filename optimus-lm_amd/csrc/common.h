@@ -82,6 +82,22 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
+// 1 / (1 + e^-x) with the hardware exponential and reciprocal (about 1 ulp each, far inside one
+// bf16 rounding of the results it feeds).  An IEEE division here costs ten instructions per
+// element, and the SwiGLU epilogues are bound by vector-ALU issue.
+__device__ __forceinline__ float fast_sigmoid(float x) {
+    return __builtin_amdgcn_rcpf(1.0f + __expf(-x));
+}
+
+// The grouped products of few rows per expert (ggemm_stream.hip): the rule, and the launches that the entry
+// points of ggemm.hip make under it.  Arguments are checked by the caller.
+bool om_ggemm_streams(int64_t rows, int n_experts, int cols);   // cols: weight rows per expert (gate and up: both)
+int om_ggemm_stream_gate_up(const void *x, const int32_t *x_rows, const void *w_gate, const void *w_up,
+                            const float *row_weights, void *g, void *u, void *h, const int32_t *cum, int64_t rows, int G,
+                            int I, int H, int64_t w_stride, hipStream_t st);
+int om_ggemm_stream_fwd(const void *x, const void *w, void *out, const int32_t *cum, int64_t rows, int G, int N, int K,
+                        int64_t w_stride, hipStream_t st);
+
 // The split gate projection (gate_fwd.hip) as the routing kernels' producer (route.hip): slices of H, and
 // the launch that leaves partial[splits][T][N].  Arguments are checked by the caller.
 int om_gate_route_splits(int64_t T, int H, int N);

@@ -156,13 +156,6 @@ __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
-// 1 / (1 + e^-x) with the hardware exponential and reciprocal (about 1 ulp each, far inside one
-// bf16 rounding of the results it feeds).  An IEEE division here costs ten instructions per
-// element, and the SwiGLU epilogues are bound by vector-ALU issue.
-__device__ __forceinline__ float fast_sigmoid(float x) {
-    return __builtin_amdgcn_rcpf(1.0f + __expf(-x));
-}
-
 // Sum over aligned groups of N neighbouring lanes (N = 4, 8 or 16); every lane of the group gets
 // it.  DPP: swap within pairs, swap pairs within quads, mirror within 8, mirror within 16.
 template <int CTRL> __device__ __forceinline__ float dpp_move(float x) {
@@ -1177,6 +1170,8 @@ extern "C" int om_grouped_gemm_fwd(const void *input, const void *weight, void *
     p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
+    if (G <= MAX_EXPERTS && om_ggemm_streams(rows, G, N))
+        return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, G, N, K, p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
     return launch_rows_auto<CONTIG, CONTIG, EPI_STORE>(p, rows, om_stream(stream));
 }
@@ -1348,6 +1343,9 @@ int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, c
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
+    if (G <= MAX_EXPERTS && om_ggemm_streams(rows, G, 2 * I))
+        return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, G, I, H,
+                                       p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
     if (row_weights) return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A, true>(p, rows, om_stream(stream));
     if (x_rows) return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A>(p, rows, om_stream(stream));

@@ -479,3 +479,53 @@ def test_merged_mlp_float32_gathered(cuda, T, K, N, start, end, I, H, live):
                       (wd[2].grad, w64[2].grad)):
         err = (got.detach().double().cpu() - want.detach()).norm()
         assert float(err) <= 1e-5 * float(want.detach().norm()) + 1e-12
+
+
+STREAM_COUNTS = [[1], [16], [64], [0, 1, 0, 15, 16, 17, 0, 3], [0] * 170 + [32, 33, 1] + [0] * 30 + [64, 65, 130], [0, 0, 72]]
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("N,K", [(8, 8), (40, 72), (200, 512), (328, 1000), (256, 1088)])
+@pytest.mark.parametrize("counts", STREAM_COUNTS, ids=lambda c: f"{len(c)}x{max(c)}")
+def test_few_row_products_stream_the_weights(cuda, counts, N, K, weighted):
+    """The kernels for a handful of rows per expert (at most 64 + 16 per expert in all): row tiles of 64 in
+    fragments of 16, a contraction shared by eight wavefronts in pieces of 64, column tiles of 16 + 16.
+    Counts on both sides of each edge, experts beyond one scan of 64, a pitch between the experts'
+    weights, rows through an index, extents that no tile divides.  Each product is one rounding of a
+    float32 sum; h adds the rounding-free weight."""
+    from optimus import _native as n
+    G, rows = len(counts), sum(counts)
+    # (the rule: otherwise the tiled kernels run)
+    assert rows <= 64 + 16 * G and (rows <= 2 * G or (min(rows, G) + rows // 128) * ((2 * N + 127) // 128) <= 256)
+    g = torch.Generator().manual_seed(rows + N + K)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    T, pitch = 37, N * K + 64
+    x = torch.randn(T, K, generator=g).to(torch.bfloat16)
+    index = torch.randint(0, T, (rows,), generator=g).int()
+    scale = torch.rand(rows, generator=g)
+    store = [(torch.randn(G * pitch, generator=g) * 0.05).to(torch.bfloat16) for _ in range(2)]
+    w = [s.view(G, pitch)[:, :N * K].view(G, N, K).float() for s in store]
+    d = dict(x=x, index=index, scale=scale, cum=cum, wg=store[0], wu=store[1])
+    d = {k: v.to(cuda) for k, v in d.items()}
+    P = n.ptr
+    guard = 3
+    out = [torch.full((rows + guard, N), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(4)]
+    xr = x[index.long()]
+    d["xr"] = xr.to(cuda)
+    if weighted:
+        n.check(n.lib().om_merged_mlp_gate_up_fwd_weighted(P(d["x"]), P(d["index"]), T, P(d["wg"]), P(d["wu"]), P(d["scale"]),
+                                                          P(out[0]), P(out[1]), P(out[2]), P(d["cum"]), rows, G, N, K, pitch,
+                                                          n.stream()), "gate_up")
+    else:
+        n.check(n.lib().om_merged_mlp_gate_up_fwd(P(d["xr"]), P(d["wg"]), P(d["wu"]), P(out[0]), P(out[1]), P(out[2]),
+                                                 P(d["cum"]), rows, G, N, K, pitch, n.stream()), "gate_up")
+    n.check(n.lib().om_grouped_gemm_fwd(P(d["xr"]), P(d["wg"]), P(out[3]), P(d["cum"]), rows, G, N, K, pitch, n.stream()), "fwd")
+    torch.cuda.synchronize()
+    ref = [_ref_fwd(xr, m, cum) for m in w]
+    h = torch.nn.functional.silu(ref[0]) * ref[1] * (scale[:, None] if weighted else 1.0)
+    for name, got, want in zip(("g", "u", "h", "y"), out, (ref[0], ref[1], h, ref[0])):
+        assert (got[rows:] == 7.0).all(), name
+        # one bf16 rounding (2^-9 of the value), and sums of K products in another order; h from unrounded g, u
+        err = (got[:rows].float().cpu() - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + 1e-6 * K ** 0.5).all(), (name, float(err.max()))
