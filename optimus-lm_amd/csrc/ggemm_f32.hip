@@ -5,14 +5,19 @@
 // the bf16 kernels: forward, input gradient, weight gradient, and the merged MLP's forms of them (gate
 // and up in one launch with the SwiGLU or its backward in the epilogue, the token gather in the loads).
 //
-// One 64x64 output tile per 256-thread block, contraction steps of 32, two LDS stages: the global
-// loads of step s+1 are in registers' flight while step s is multiplied, and are written to the other
-// stage behind one barrier per step.  These launches are small (the tiny layer: 1.07 GFLOP a product,
-// 7 us of matrix-core time per tile), so what bounds them is the latency of a step's loads and the
-// number of launches.  Tiny layer (2048 tokens, hidden 256, ffn 512, 8 experts, top-2) per step: 15
-// launches of 24-37 us with one stage of 16 and a barrier on each side of the loads, 6 of 9-18 us now.
+// One 64x64 output tile per block of eight wavefronts: four of them (2x2 of 32x32) take the first half of
+// each 64-deep contraction step and four the second, and the two sums are added through LDS at the end.
+// Two LDS stages, one barrier per step; two further steps of both operands are on their way in registers.
+// These launches are small (the tiny layer: 1.07 GFLOP a product, 256 to 288 tiles), so many CUs hold one
+// tile and what bounds them is how much of the matrix core's time one block can use: a wavefront's chain of
+// fragment read -> MFMA, the barrier, the misses.  Tiny layer (2048 tokens, hidden 256, ffn 512, 8
+// experts, top-2), us per launch with four wavefronts, 32-deep steps and one step ahead -> now: gate+up
+// 41 -> 39, down 24 -> 23, down input gradient 25 -> 27, gate/up input gradient 46 -> 44, down weight
+// gradient 23 -> 17, gate/up weight gradients 33 -> 30; four steps ahead without the second group of
+// wavefronts 39, 25, 29, 46, 20, 31.  The row products stay at 64 % of the matrix rate on the CUs that hold
+// two of the 288 tiles.
 //
-// CONTIG operands ([row][c] in memory, c = contraction index) lie in LDS as [row][c] with a 36-float
+// CONTIG operands ([row][c] in memory, c = contraction index) lie in LDS as [row][c] with a 68-float
 // pitch: 16-byte writes and reads, 16 consecutive rows in 16 different 16-byte bank groups.  STRIDED
 // operands ([c][row] in memory: the weight in dgrad, both operands in wgrad) lie as [c][row] with a
 // 68-float pitch, read 4 bytes at a time (one read per 64-cycle MFMA: not what bounds).
@@ -21,7 +26,8 @@
 namespace {
 
 constexpr int TB = 64;      // tile rows and columns
-constexpr int KS = 32;      // contraction step
+constexpr int KS = 64;      // contraction step: 32 indices for each of the two groups of wavefronts
+constexpr int THREADS = 512;
 constexpr int PITCH_C = KS + 4, PITCH_S = TB + 4;
 constexpr int STAGE = TB * PITCH_C > KS * PITCH_S ? TB * PITCH_C : KS * PITCH_S;   // floats per operand tile
 typedef __attribute__((ext_vector_type(4))) float f4;
@@ -41,20 +47,24 @@ struct F32Params {
 };
 
 // One thread's part of a tile and step: 8 floats along c (CONTIG) or along the rows (STRIDED).
-struct Fetched { f4 v[2]; };
-template <int KIND> __device__ __forceinline__ int slot_row(int tid) { return KIND == F_CONTIG ? tid >> 2 : (tid & 7) * 8; }
-template <int KIND> __device__ __forceinline__ int slot_c(int tid) { return KIND == F_CONTIG ? (tid & 3) * 8 : tid >> 3; }
+struct Fetched { f4 v[2]; bool in; };
+template <int KIND> __device__ __forceinline__ int slot_row(int tid) { return KIND == F_CONTIG ? tid >> 3 : (tid & 7) * 8; }
+template <int KIND> __device__ __forceinline__ int slot_c(int tid) { return KIND == F_CONTIG ? (tid & 7) * 8 : tid >> 3; }
 template <int KIND> __device__ __forceinline__ void stash(float *tile, const Fetched &q, int tid) {
     float *p = KIND == F_CONTIG ? tile + slot_row<KIND>(tid) * PITCH_C + slot_c<KIND>(tid)
                                 : tile + slot_c<KIND>(tid) * PITCH_S + slot_row<KIND>(tid);
-    reinterpret_cast<f4 *>(p)[0] = q.v[0];
-    reinterpret_cast<f4 *>(p)[1] = q.v[1];
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    reinterpret_cast<f4 *>(p)[0] = q.in ? q.v[0] : zero;
+    reinterpret_cast<f4 *>(p)[1] = q.in ? q.v[1] : zero;
 }
-// 8 floats at p, the two halves masked
-__device__ __forceinline__ Fetched fetch8(const float *p, bool lo, bool hi) {
+// 8 floats at p (always valid memory: callers clamp); `in` false: zeros take their place when they are
+// stashed.  Extents are multiples of 8, so a slot is inside or outside as a whole.  No load is conditional:
+// at the end of a branch around one the compiler would wait for every load in flight.
+__device__ __forceinline__ Fetched fetch8(const float *p, bool in) {
     Fetched q;
-    q.v[0] = lo ? reinterpret_cast<const f4 *>(p)[0] : f4{0.f, 0.f, 0.f, 0.f};
-    q.v[1] = hi ? reinterpret_cast<const f4 *>(p)[1] : f4{0.f, 0.f, 0.f, 0.f};
+    q.v[0] = reinterpret_cast<const f4 *>(p)[0];
+    q.v[1] = reinterpret_cast<const f4 *>(p)[1];
+    q.in = in;
     return q;
 }
 // Fragment of contraction indices 8s + 4*(lane/32) .. +3 of operand row `row`; element j goes to MFMA j.
@@ -66,30 +76,53 @@ template <int KIND> __device__ __forceinline__ f4 fragment(const float *tile, in
     return v;
 }
 
-// The main loop: `fetch_a(step)` / `fetch_b(step)` deliver this thread's part of a step.
+// The main loop: `fetch_a(step)` / `fetch_b(step)` deliver this thread's part of a step, also past the last
+// one (valid memory, not used).  AHEAD steps of both operands are on their way in registers, since a miss
+// costs more than a step's 1024 cycles of MFMA.
+constexpr int AHEAD = 2;    // (even: a register set always meets the same LDS stage)
 template <int AKIND, int BKIND, typename FA, typename FB>
 __device__ __forceinline__ void multiply(float *lds, int n_steps, int wm, int wn, FA &&fetch_a, FB &&fetch_b, f32x16 &acc) {
-    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, part = tid >> 8;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
     if (n_steps <= 0) return;
-    Fetched a = fetch_a(0), b = fetch_b(0);
-    for (int s = 0; s < n_steps; s++) {
-        float *ta = lds + (s & 1) * 2 * STAGE, *tb = ta + STAGE;
-        stash<AKIND>(ta, a, tid);
-        stash<BKIND>(tb, b, tid);
-        __syncthreads();   // (a stage is rewritten two steps later, behind the barrier of the step between)
-        if (s + 1 < n_steps) { a = fetch_a(s + 1); b = fetch_b(s + 1); }
+    Fetched a[AHEAD], b[AHEAD];
 #pragma unroll
-        for (int g = 0; g < KS / 8; g++) {
-            const f4 fa = fragment<AKIND>(ta, wm + (lane & 31), g, half);
-            const f4 fb = fragment<BKIND>(tb, wn + (lane & 31), g, half);
+    for (int d = 0; d < AHEAD; d++) { a[d] = fetch_a(d); b[d] = fetch_b(d); }
+    for (int s0 = 0;; s0 += AHEAD) {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                // operands swapped: lane l then holds output row wm + l%32 and columns
-                // wn + 8*(r/4) + 4*(l/32) + r%4
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[j], acc, 0, 0, 0);
+        for (int d = 0; d < AHEAD; d++) {
+            if (s0 + d >= n_steps) goto done;
+            float *ta = lds + (d & 1) * 2 * STAGE, *tb = ta + STAGE;
+            stash<AKIND>(ta, a[d], tid);
+            stash<BKIND>(tb, b[d], tid);
+            __syncthreads();   // (a stage is rewritten two steps later, behind the barrier of the step between)
+            a[d] = fetch_a(s0 + d + AHEAD);
+            b[d] = fetch_b(s0 + d + AHEAD);
+#pragma unroll
+            for (int h = 0; h < KS / 16; h++) {
+                const int g = part * (KS / 16) + h;
+                const f4 fa = fragment<AKIND>(ta, wm + (lane & 31), g, half);
+                const f4 fb = fragment<BKIND>(tb, wn + (lane & 31), g, half);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    // operands swapped: lane l then holds output row wm + l%32 and columns
+                    // wn + 8*(r/4) + 4*(l/32) + r%4
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j], fa[j], acc, 0, 0, 0);
+            }
         }
+    }
+done:
+    __syncthreads();
+    float *ex = lds + (tid & 255);
+    if (part) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) ex[r * 256] = acc[r];
+    }
+    __syncthreads();
+    if (!part) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[r] += ex[r * 256];
     }
 }
 
@@ -125,36 +158,40 @@ __device__ __forceinline__ bool find_row_tile(const int32_t *cum, int n_experts,
 // blockIdx.x = row tile (cut per expert), blockIdx.y = column tile (E_SWIGLU: 32 columns of gate and the
 // same 32 of up, side by side in the tile)
 template <int BKIND, int EPI, bool GATHER>
-__global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) {
+__global__ __launch_bounds__(THREADS, 4) void ggemm_f32_rows_kernel(const F32Params p) {
     __shared__ __attribute__((aligned(16))) float lds[4 * STAGE];
     int expert, m0, m_end;
     if (!find_row_tile(p.cum, p.n_experts, blockIdx.x, expert, m0, m_end)) return;   // (the whole block: blockIdx only)
     constexpr int COLS = EPI == E_SWIGLU ? TB / 2 : TB;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int wm = ((wave >> 1) & 1) * 32, wn = (wave & 1) * 32;
     const int n0 = blockIdx.y * COLS;
     const int steps = (p.kc + KS - 1) / KS;
     // A: [row][c]
     const int arow = m0 + slot_row<F_CONTIG>(tid), ac = slot_c<F_CONTIG>(tid);
     const bool a_in = arow < m_end;
     const int64_t a_src = !a_in ? 0 : GATHER ? p.row_index[arow] : arow;
+    const int last = steps * p.phases - 1;
     auto fetch_a = [&](int s) {
+        s = min(s, last);
         const int ph = s >= steps ? 1 : 0, c = (s - ph * steps) * KS + ac;
-        return fetch8(p.A[ph] + a_src * p.lda + c, a_in && c < p.kc, a_in && c + 4 < p.kc);
+        return fetch8((ph ? p.A[1] : p.A[0]) + a_src * p.lda + min(c, p.kc - 8), a_in && c < p.kc);
     };
     // B: W[g] as [n][k] (forward) or [c][col] with c the contraction index (input gradient)
     const int brow = slot_row<BKIND>(tid), bc = slot_c<BKIND>(tid);
     const int64_t b0[2] = {expert * p.strideB[0], expert * p.strideB[1]};
     auto fetch_b = [&](int s) {
+        s = min(s, last);
         const int ph = s >= steps ? 1 : 0, c = (s - ph * steps) * KS + bc;
         if (BKIND == F_CONTIG) {
             const int which = EPI == E_SWIGLU ? brow >> 5 : ph;
             const int n = n0 + (EPI == E_SWIGLU ? brow & 31 : brow);
-            const bool in = n < p.n_cols;
-            return fetch8(p.B[which] + b0[which] + static_cast<int64_t>(n) * p.ldb + c, in && c < p.kc, in && c + 4 < p.kc);
+            return fetch8((which ? p.B[1] + b0[1] : p.B[0] + b0[0]) + static_cast<int64_t>(min(n, p.n_cols - 1)) * p.ldb +
+                              min(c, p.kc - 8), n < p.n_cols && c < p.kc);
         }
         const int n = n0 + brow;
-        return fetch8(p.B[ph] + b0[ph] + static_cast<int64_t>(c) * p.ldb + n, c < p.kc && n < p.n_cols, c < p.kc && n + 4 < p.n_cols);
+        return fetch8((ph ? p.B[1] + b0[1] : p.B[0] + b0[0]) + static_cast<int64_t>(min(c, p.kc - 1)) * p.ldb +
+                          min(n, p.n_cols - 8), c < p.kc && n < p.n_cols);
     };
     f32x16 acc;
     multiply<F_CONTIG, BKIND>(lds, steps * p.phases, wm, wn, fetch_a, fetch_b, acc);
@@ -162,13 +199,13 @@ __global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) 
     if (EPI == E_SWIGLU) {
         // the up half goes to the wavefront that holds the gate half of the same rows and columns
         __syncthreads();
-        float *ex = lds + (wave >> 1) * 16 * 64;
-        if (wn) {
+        float *ex = lds + ((wave >> 1) & 1) * 16 * 64;
+        if (wn && wave < 4) {
 #pragma unroll
             for (int r = 0; r < 16; r++) ex[r * 64 + lane] = acc[r];
         }
         __syncthreads();
-        if (m >= m_end) return;
+        if (m >= m_end || wave >= 4) return;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
             const int n = n0 + q * 8 + (lane >> 5) * 4;
@@ -184,7 +221,7 @@ __global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) 
         }
         return;
     }
-    if (m >= m_end) return;
+    if (m >= m_end || wave >= 4) return;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int n = n0 + wn + q * 8 + (lane >> 5) * 4;
@@ -211,28 +248,34 @@ __global__ __launch_bounds__(256) void ggemm_f32_rows_kernel(const F32Params p) 
 // blockIdx = (column tile of dW, row tile of dW, expert and which of up to two weight gradients):
 // dW[g][n][k] = sum_r dout[r][n] * in[r][k]
 template <bool GATHER>
-__global__ __launch_bounds__(256) void ggemm_f32_wgrad_kernel(const F32Params p) {
+__global__ __launch_bounds__(THREADS, 4) void ggemm_f32_wgrad_kernel(const F32Params p) {
     __shared__ __attribute__((aligned(16))) float lds[4 * STAGE];
     const int expert = blockIdx.z % p.n_experts, which = blockIdx.z / p.n_experts;
     const int r0 = p.cum[expert], r1 = p.cum[expert + 1];
     const int n0 = blockIdx.y * TB, k0 = blockIdx.x * TB;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int wm = ((wave >> 1) & 1) * 32, wn = (wave & 1) * 32;
     const int row = slot_row<F_STRIDED>(tid), c = slot_c<F_STRIDED>(tid);
+    // the loads past the segment (and past the extents) re-read its last row (the last 8 columns)
+    const int a_col = min(n0 + row, p.kc - 8), b_col = min(k0 + row, p.n_cols - 8);
+    const bool a_in = n0 + row < p.kc, b_in = k0 + row < p.n_cols;
     auto fetch_a = [&](int s) {
         const int r = r0 + s * KS + c;
-        return fetch8(p.A[which] + static_cast<int64_t>(r) * p.lda + n0 + row, r < r1 && n0 + row < p.kc, r < r1 && n0 + row + 4 < p.kc);
+        return fetch8(p.A[which] + static_cast<int64_t>(min(r, r1 - 1)) * p.lda + a_col, a_in && r < r1);
     };
+    // GATHER: the source row of this thread's slot AHEAD steps on, looked up one step before it is needed
+    int src = GATHER && r1 > r0 ? p.row_index[min(r0 + c, r1 - 1)] : 0;
     auto fetch_b = [&](int s) {
         const int r = r0 + s * KS + c;
-        const int64_t src = r >= r1 ? 0 : GATHER ? p.row_index[r] : r;
-        return fetch8(p.B[0] + src * p.ldb + k0 + row, r < r1 && k0 + row < p.n_cols, r < r1 && k0 + row + 4 < p.n_cols);
+        const int64_t from = GATHER ? src : min(r, r1 - 1);
+        if (GATHER) src = p.row_index[min(r + KS, r1 - 1)];
+        return fetch8(p.B[0] + from * p.ldb + b_col, b_in && r < r1);
     };
     f32x16 acc;
     multiply<F_STRIDED, F_STRIDED>(lds, (r1 - r0 + KS - 1) / KS, wm, wn, fetch_a, fetch_b, acc);
     float *C = p.C[which] + expert * p.strideC[which];
     const int n = n0 + wm + (lane & 31);
-    if (n >= p.kc) return;
+    if (n >= p.kc || wave >= 4) return;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int k = k0 + wn + q * 8 + (lane >> 5) * 4;
@@ -253,8 +296,8 @@ template <int BKIND, int EPI> int rows_launch(const F32Params &p, int64_t rows, 
     const unsigned n_tiles = tiles_of(p.n_cols, EPI == E_SWIGLU ? TB / 2 : TB);
     if (m_tiles > 0x7fffffffLL || n_tiles > 65535) return OM_ERR_SHAPE;
     const dim3 grid(static_cast<unsigned>(m_tiles), n_tiles);
-    if (p.row_index) ggemm_f32_rows_kernel<BKIND, EPI, true><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
-    else ggemm_f32_rows_kernel<BKIND, EPI, false><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
+    if (p.row_index) ggemm_f32_rows_kernel<BKIND, EPI, true><<<grid, dim3(THREADS), 0, om_stream(stream)>>>(p);
+    else ggemm_f32_rows_kernel<BKIND, EPI, false><<<grid, dim3(THREADS), 0, om_stream(stream)>>>(p);
     return om_launch_status();
 }
 
@@ -383,8 +426,8 @@ int wgrad_f32_launch(int n_sets, const float *const *output_grad, const float *i
     p.n_experts = G; p.n_cols = K; p.kc = N;
     p.accumulate = accumulate;
     const dim3 grid(tiles_of(K), tiles_of(N), n_sets * G);
-    if (input_rows) ggemm_f32_wgrad_kernel<true><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
-    else ggemm_f32_wgrad_kernel<false><<<grid, dim3(256), 0, om_stream(stream)>>>(p);
+    if (input_rows) ggemm_f32_wgrad_kernel<true><<<grid, dim3(THREADS), 0, om_stream(stream)>>>(p);
+    else ggemm_f32_wgrad_kernel<false><<<grid, dim3(THREADS), 0, om_stream(stream)>>>(p);
     return om_launch_status();
 }
 }  // namespace
