@@ -866,6 +866,30 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     }
     __syncthreads();  // the stages are dead: stage 1 becomes the strips, stage 0 the next tile's
 
+    // Weight gradient added to what the output already holds (a gradient buffer that several backward
+    // passes accumulate into): the sum is what an in-place bf16 `grad += dW` gives, two roundings.  The
+    // old values of the whole tile are requested here, ahead of the next tile's operands, into the
+    // registers that the fragments leave free (one strip ahead of its use, each strip waited for a miss:
+    // 32 experts of [2048, 7168], 256 rows each, 820 -> 740 us a launch inside a step).
+    constexpr int OLD_CPR = WN / 8, OLD_ITS = 32 * OLD_CPR / 64;   // as CPRW and ITS of the epilogue
+    u32x4 old[ACCUM ? TM : 1][ACCUM ? OLD_ITS : 1];
+    if (ACCUM) {
+        int lane_o = lane;
+        asm volatile("" : "+v"(lane_o));
+        const uint16_t *src = p.C + expert * p.strideC + n0 + wn * WN + (lane_o % OLD_CPR) * 8;
+        const bool col_in = !EDGE || n0 + wn * WN + (lane_o % OLD_CPR) * 8 < p.n_cols;
+        const int m_first = row_begin + wm * WM + lane_o / OLD_CPR;
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int it = 0; it < OLD_ITS; it++) {
+                const int m = m_first + i * 32 + it * (64 / OLD_CPR);
+                if (!EDGE || (col_in && m < p.kc))
+                    old[ACCUM ? i : 0][ACCUM ? it : 0] =
+                        *reinterpret_cast<const u32x4 *>(src + static_cast<int64_t>(m) * p.ldc);
+            }
+    }
+
     // The next tile's first contraction step is fetched into stage 0 while this tile's results go
     // out (the strips live in stage 1), which takes the cold-miss latency of a tile's first loads
     // off the critical path.
@@ -932,27 +956,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
             wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0] = (m < e_row_end) ? p.row_scale[m] : 0.0f;
         }
     }
-    // Weight gradient added to what the output already holds (a gradient buffer that several
-    // backward passes accumulate into): the old values of a strip are fetched one strip ahead (two
-    // register sets), and the sum is what an in-place bf16 `grad += dW` gives, two roundings.
-    constexpr bool acc_out = ACCUM;
-    u32x4 old2[ACCUM ? 2 : 1][ACCUM ? ITS : 1];
-    auto load_old = [&](int i, int buf) {
-        const int64_t m0 = static_cast<int64_t>(e_row_begin) + wm_e * WM + i * 32;
-#pragma unroll
-        for (int it = 0; it < ITS; it++) {
-            const int q = it * 64 + lane_e;
-            const int64_t o = (m0 + q / CPRW) * p.ldc + col0 + (q % CPRW) * 8;
-            if (m0 + q / CPRW < row_lim)
-                old2[ACCUM ? buf : 0][ACCUM ? it : 0] = *reinterpret_cast<const u32x4 *>(Cb + o);
-        }
-    };
-    if (ACCUM) load_old(0, 0);
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int64_t m0 = static_cast<int64_t>(e_row_begin) + wm_e * WM + i * 32;  // first row of the strip
-        if (ACCUM && i + 1 < TM) load_old(i + 1, (i + 1) & 1);
-        u32x4 *old_out = old2[ACCUM ? (i & 1) : 0];
+        u32x4 *old_out = old[ACCUM ? i : 0];
         if (EPI == EPI_SWIGLU) {
             const float wrow = wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0];   // ROWW: h = w[row] * silu(g) * u, one rounding
 #pragma unroll
@@ -1046,13 +1053,13 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
                 if (m < row_lim) {
                     const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
                     u32x4 v = strip_get(0, q / CPRW, q % CPRW);
-                    if (EPI == EPI_WGRAD && acc_out) {
-                        float fresh[8], old[8];
+                    if (EPI == EPI_WGRAD && ACCUM) {
+                        float fresh[8], prev[8];
                         Elem<uint16_t>::unpack(v, fresh);
-                        Elem<uint16_t>::unpack(old_out[ACCUM ? it : 0], old);
+                        Elem<uint16_t>::unpack(old_out[ACCUM ? it : 0], prev);
 #pragma unroll
                         for (int x = 0; x < 4; x++)
-                            v[x] = pack2_bf16(old[2 * x] + fresh[2 * x], old[2 * x + 1] + fresh[2 * x + 1]);
+                            v[x] = pack2_bf16(prev[2 * x] + fresh[2 * x], prev[2 * x + 1] + fresh[2 * x + 1]);
                     }
                     *reinterpret_cast<u32x4 *>(Cb + o) = v;
                     if (EPI == EPI_SWIGLU) {
