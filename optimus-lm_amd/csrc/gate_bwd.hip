@@ -212,10 +212,15 @@ inline size_t gate_dgrad_lds(int N) {
     return w > DG_STRIPS ? w : DG_STRIPS;
 }
 
-__global__ __launch_bounds__(256) void gate_dgrad_kernel(const float *__restrict__ dlogits,
-                                                         const uint16_t *__restrict__ weight,
-                                                         const uint16_t *base, uint16_t *out, int64_t T,
-                                                         int H, int N) {
+// The dlogits of four 16-slices are fetched together, one batch ahead of their MFMAs, and `base` before the
+// first of them, so that a block waits for one miss and not for one per slice: 8192 tokens, hidden 7168, 256
+// experts 146 -> 113 us, 16384 x 2048, 64 experts 41 -> 36, 3001 x 1000, 12 experts 10.8 -> 6.4.
+// BATCHES * 4 slices of 16 experts; ALIGNED: rows of dlogits are whole 16-byte vectors (N % 4 == 0)
+template <int BATCHES, bool ALIGNED>
+__global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restrict__ dlogits,
+                                                            const uint16_t *__restrict__ weight,
+                                                            const uint16_t *base, uint16_t *out, int64_t T,
+                                                            int H, int N) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h0 = blockIdx.x * DG_HT;
@@ -228,39 +233,67 @@ __global__ __launch_bounds__(256) void gate_dgrad_kernel(const float *__restrict
             v = *reinterpret_cast<const u32x4 *>(weight + static_cast<int64_t>(n) * H + h0 + ch * 8);
         *reinterpret_cast<u32x4 *>(lds + tile_off<DG_HT>(n, ch)) = v;
     }
+    // tokens past the end: the last one's, results unused; experts past the end: zeros
+    const float *drow = dlogits + min(t0 + (lane & 31), T - 1) * N;
+    f32x4 raw[2][4][2];
+    auto fetch = [&](int batch, int set) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int half = 0; half < 2; half++) {
+                const int n = batch * 64 + k * 16 + 8 * (lane >> 5) + 4 * half;
+                if (ALIGNED) {
+                    raw[set][k][half] = *reinterpret_cast<const f32x4 *>(drow + min(n, N - 4));
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) raw[set][k][half][i] = drow[min(n + i, N - 1)];
+                }
+            }
+    };
+    auto packed = [&](int batch, int set, int k) -> bf16x8 {
+        u32x4 v;
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            const int n = batch * 64 + k * 16 + 8 * (lane >> 5) + 4 * half;
+            float d[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) d[i] = n + i < N ? raw[set][k][half][i] : 0.0f;
+            v[2 * half] = pack2(d[0], d[1]);
+            v[2 * half + 1] = pack2(d[2], d[3]);
+        }
+        return __builtin_bit_cast(bf16x8, v);
+    };
+    fetch(0, 0);
+    constexpr int ITS = 32 * (DG_HT / 8) / 64;
+    u32x4 other[ITS];
+    if (base) {
+#pragma unroll
+        for (int it = 0; it < ITS; it++) {
+            const int q = it * 64 + lane;
+            other[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(   // read once
+                base + min(t0 + q / (DG_HT / 8), T - 1) * H + min(h0 + (q % (DG_HT / 8)) * 8, H - 8)));
+        }
+    }
     __syncthreads();
     f32x16 acc[DG_HT / 32];
 #pragma unroll
     for (int b = 0; b < DG_HT / 32; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[b][r] = 0.0f;
-    const int64_t t = t0 + (lane & 31);
-    const float *drow = dlogits + t * N;
-    for (int kk = 0; kk < n_pad; kk += 16) {
-        const int nb = kk + 8 * (lane >> 5);
-        float d[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (t < T) {
-            if ((N & 3) == 0) {   // 16-byte aligned rows
 #pragma unroll
-                for (int half = 0; half < 2; half++)
-                    if (nb + 4 * half < N) {
-                        const f32x4 v = *reinterpret_cast<const f32x4 *>(drow + nb + 4 * half);
+    for (int batch = 0; batch < BATCHES; batch++) {
+        if (batch + 1 < BATCHES) fetch(batch + 1, (batch + 1) & 1);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) d[4 * half + i] = v[i];
-                    }
-            } else {
+        for (int k = 0; k < 4; k++) {
+            const int kk = batch * 64 + k * 16;
+            if (kk >= n_pad) continue;        // (uniform; the weight tile ends here)
+            const bf16x8 fd = packed(batch, batch & 1, k);
 #pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (nb + i < N) d[i] = drow[nb + i];
+            for (int b = 0; b < DG_HT / 32; b++) {
+                const bf16x8 fw = read_frag<DG_HT>(lds, kk, b * 32, lane);
+                // lane l then holds token l % 32 and columns 32 b + 8*(r/4) + 4*(l/32) + r%4
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw, fd, acc[b], 0, 0, 0);
             }
-        }
-        u32x4 packed = {pack2(d[0], d[1]), pack2(d[2], d[3]), pack2(d[4], d[5]), pack2(d[6], d[7])};
-        const bf16x8 fd = __builtin_bit_cast(bf16x8, packed);
-#pragma unroll
-        for (int b = 0; b < DG_HT / 32; b++) {
-            const bf16x8 fw = read_frag<DG_HT>(lds, kk, b * 32, lane);
-            // lane l then holds token l % 32 and columns 32 b + 8*(r/4) + 4*(l/32) + r%4
-            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw, fd, acc[b], 0, 0, 0);
         }
     }
     __syncthreads();   // the weight tile is dead; its memory becomes the strips
@@ -279,7 +312,7 @@ __global__ __launch_bounds__(256) void gate_dgrad_kernel(const float *__restrict
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int it = 0; it < 32 * (DG_HT / 8) / 64; it++) {
+    for (int it = 0; it < ITS; it++) {
         const int q = it * 64 + lane;
         const int row = q / (DG_HT / 8), ch = q % (DG_HT / 8);
         const int64_t tt = t0 + row;
@@ -292,7 +325,7 @@ __global__ __launch_bounds__(256) void gate_dgrad_kernel(const float *__restrict
             const int64_t o = tt * H + h;
             if (base) {
                 float a[8], g[8];
-                Elem<uint16_t>::unpack(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + o)), a);   // read once
+                Elem<uint16_t>::unpack(other[it], a);
                 Elem<uint16_t>::unpack(v, g);
 #pragma unroll
                 for (int i = 0; i < 8; i++) a[i] = a[i] + g[i];
@@ -327,9 +360,17 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
         return OM_OK;
     }
     const dim3 grid((H + DG_HT - 1) / DG_HT, static_cast<unsigned>(t_blocks));
-    gate_dgrad_kernel<<<grid, dim3(256), gate_dgrad_lds(N), om_stream(stream)>>>(
-        dlogits, static_cast<const uint16_t *>(gate_weight), static_cast<const uint16_t *>(base),
-        static_cast<uint16_t *>(dx), T, H, N);
+#define OM_DGRAD(BATCHES, ALIGNED)                                                                          \
+    gate_dgrad_kernel<BATCHES, ALIGNED><<<grid, dim3(256), gate_dgrad_lds(N), om_stream(stream)>>>(          \
+        dlogits, static_cast<const uint16_t *>(gate_weight), static_cast<const uint16_t *>(base),            \
+        static_cast<uint16_t *>(dx), T, H, N)
+    if (N % 4 != 0) {
+        if (N <= 64) OM_DGRAD(1, false);
+        else OM_DGRAD(4, false);
+    } else if (N <= 64) OM_DGRAD(1, true);
+    else if (N <= 128) OM_DGRAD(2, true);
+    else OM_DGRAD(4, true);
+#undef OM_DGRAD
     return om_launch_status();
 }
 
