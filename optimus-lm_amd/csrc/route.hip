@@ -461,22 +461,25 @@ int launch_gate(const void *x, const void *wg, int64_t T, int H, int N, int K, i
 // the auxiliary loss, reference optimus/models/olmoe/modeling_olmoe.py:29-85).  A block walks
 // BAL_TOKENS tokens, one wavefront per token at a time, and leaves one partial row; a second
 // kernel adds the rows in block order, so the result does not depend on scheduling.
-constexpr int BAL_TOKENS = 64;
+// What bounds both is a chain of latencies, not the 4 MB of logits: with four wavefronts a block took 16
+// softmax and top-K selections one after another (46 us at 16384 tokens, 64 experts), and one thread per
+// expert then added 256 rows with one load in flight (66 us).  Sixteen wavefronts per block and 16 loads in
+// flight: 17.5 + 8.6 us.
+constexpr int BAL_TOKENS = 64, BAL_WAVES = 16;
 template <int PER, typename T>
-__global__ __launch_bounds__(256) void balance_stats_kernel(const T *__restrict__ logits,
-                                                            const float *__restrict__ token_weight,
-                                                            int64_t Tn, int N, int K,
-                                                            float *__restrict__ part_prob,
-                                                            float *__restrict__ part_count) {
-    __shared__ float lds_p[4][PER * 64];
-    __shared__ float lds_c[4][PER * 64];
+__global__ __launch_bounds__(BAL_WAVES * 64) void balance_stats_kernel(const T *__restrict__ logits,
+                                                                       const float *__restrict__ token_weight,
+                                                                       int64_t Tn, int N, int K,
+                                                                       float *__restrict__ part_prob,
+                                                                       float *__restrict__ part_count) {
+    __shared__ float lds[BAL_WAVES][PER * 64];   // the probabilities first, then the counts
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float psum[PER];
     float cnt[PER];   // sums of token weights; whole numbers (exact) for 0/1 weights and without weights
 #pragma unroll
     for (int j = 0; j < PER; j++) { psum[j] = 0.0f; cnt[j] = 0.0f; }
     const int64_t t_first = static_cast<int64_t>(blockIdx.x) * BAL_TOKENS;
-    for (int i = wave; i < BAL_TOKENS; i += 4) {
+    for (int i = wave; i < BAL_TOKENS; i += BAL_WAVES) {
         const int64_t t = t_first + i;
         if (t >= Tn) break;
         const float tw = token_weight ? token_weight[t] : 1.0f;   // the token's attention-mask entry
@@ -494,27 +497,51 @@ __global__ __launch_bounds__(256) void balance_stats_kernel(const T *__restrict_
         }
     }
 #pragma unroll
-    for (int j = 0; j < PER; j++) { lds_p[wave][lane + 64 * j] = psum[j]; lds_c[wave][lane + 64 * j] = cnt[j]; }
-    __syncthreads();
-    for (int i = threadIdx.x; i < N; i += 256) {
-        part_prob[static_cast<int64_t>(blockIdx.x) * N + i] = (lds_p[0][i] + lds_p[1][i]) + (lds_p[2][i] + lds_p[3][i]);
-        part_count[static_cast<int64_t>(blockIdx.x) * N + i] = (lds_c[0][i] + lds_c[1][i]) + (lds_c[2][i] + lds_c[3][i]);
+    for (int q = 0; q < 2; q++) {
+        if (q) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PER; j++) lds[wave][lane + 64 * j] = q ? cnt[j] : psum[j];
+        __syncthreads();
+        for (int i = threadIdx.x; i < N; i += BAL_WAVES * 64) {
+            float v[BAL_WAVES];
+#pragma unroll
+            for (int w = 0; w < BAL_WAVES; w++) v[w] = lds[w][i];
+#pragma unroll
+            for (int n = BAL_WAVES / 2; n > 0; n /= 2)
+#pragma unroll
+                for (int w = 0; w < n; w++) v[w] += v[w + n];
+            (q ? part_count : part_prob)[static_cast<int64_t>(blockIdx.x) * N + i] = v[0];
+        }
     }
 }
 
-__global__ __launch_bounds__(256) void balance_reduce_kernel(const float *__restrict__ part_prob,
-                                                             const float *__restrict__ part_count,
-                                                             int n_blocks, int N,
-                                                             float *__restrict__ prob_sum,
-                                                             float *__restrict__ count) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(64) void balance_reduce_kernel(const float *__restrict__ part_prob,
+                                                            const float *__restrict__ part_count,
+                                                            int n_blocks, int N,
+                                                            float *__restrict__ prob_sum,
+                                                            float *__restrict__ count) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
     if (i >= N) return;
     float ps = 0.0f;
     // a block's partial is a sum of at most BAL_TOKENS token weights (whole numbers for 0/1 weights
     // and without weights); adding the partials in double keeps whole-number counts exact at any
     // token count (a hot expert can exceed 2^24 tokens), one rounding to float at the end
     double c = 0.0;
-    for (int b = 0; b < n_blocks; b++) {
+    int b = 0;
+    for (; b + 16 <= n_blocks; b += 16) {
+        float p[16], q[16];
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            p[u] = part_prob[static_cast<int64_t>(b + u) * N + i];
+            q[u] = part_count[static_cast<int64_t>(b + u) * N + i];
+        }
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+            ps += p[u];
+            c += static_cast<double>(q[u]);
+        }
+    }
+    for (; b < n_blocks; b++) {
         ps += part_prob[static_cast<int64_t>(b) * N + i];
         c += static_cast<double>(part_count[static_cast<int64_t>(b) * N + i]);
     }
@@ -755,13 +782,13 @@ extern "C" int om_router_balance_stats_masked(const void *logits, int logits_dty
     float *pp = static_cast<float *>(workspace);
     float *pc = pp + static_cast<int64_t>(nb) * N;
     if (logits_dtype == OM_F32) {
-        OM_DISPATCH_PER(N, (balance_stats_kernel<PER, float><<<nb, 256, 0, st>>>(
+        OM_DISPATCH_PER(N, (balance_stats_kernel<PER, float><<<nb, BAL_WAVES * 64, 0, st>>>(
                                static_cast<const float *>(logits), token_weight, T, N, K, pp, pc)));
     } else {
-        OM_DISPATCH_PER(N, (balance_stats_kernel<PER, uint16_t><<<nb, 256, 0, st>>>(
+        OM_DISPATCH_PER(N, (balance_stats_kernel<PER, uint16_t><<<nb, BAL_WAVES * 64, 0, st>>>(
                                static_cast<const uint16_t *>(logits), token_weight, T, N, K, pp, pc)));
     }
-    balance_reduce_kernel<<<(N + 255) / 256, 256, 0, st>>>(pp, pc, nb, N, prob_sum, count);
+    balance_reduce_kernel<<<(N + 63) / 64, 64, 0, st>>>(pp, pc, nb, N, prob_sum, count);
     return om_launch_status();
 }
 
