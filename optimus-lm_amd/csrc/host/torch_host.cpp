@@ -710,6 +710,11 @@ Tensor route_workspace(const Tensor &x, int64_t T, int64_t H, int64_t N) {
 std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
                                                          at::ScalarType out_dtype, bool one_pass, bool bf16_logits) {
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+    // Up to 2048 tokens the one-pass kernel has at most 64 blocks, each walking all of H: the projection split
+    // over H and a routing launch behind it give the same bits (eight slices added in the one-pass order)
+    // sooner.  us, one launch -> two, hidden 2048 and 64 experts: 64 tokens 22 -> 11, 512 22 -> 15, 2048 24 -> 17,
+    // 4096 24 -> 20, 8192 27 -> 29; hidden 1024 and 32 experts: 512 10.6 -> 8.4, 4096 11.3 -> 12.0; hidden 512 even.
+    if (one_pass && !bf16_logits && T > 0 && T <= 2048 && N <= 64 && H >= 1024 && H % 512 == 0) one_pass = false;
     Tensor logits, weights, experts, x_out;
     {
         at::AutoDispatchBelowADInplaceOrView below;
