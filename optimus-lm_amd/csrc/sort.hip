@@ -8,6 +8,10 @@
 // Ranks come from wavefront ballots (lanes holding the same expert form a mask; rank = popcount of
 // the mask below the lane), per-wave running offsets live in LDS: no atomics, so the result is
 // deterministic.
+// The three launches move a few bytes per pair and wait all the time: a wavefront's steps are a serial chain.
+// Hence eight wavefronts of four steps per block (it was four of eight), and a wavefront's keys and weights
+// fetched at once, not step by step: us, count + scan + scatter, 32768 pairs of 64 experts 9.2 + 6.7 + 21.4 ->
+// 5.3 + 6.3 + 11.6, 9003 pairs of 12 7.0 + 3.1 + 16.3 -> 4.0 + 3.0 + 8.4.
 // Also: the reference's two index operators with their own [expert][column] table layout, one
 // wavefront per column.
 #include "common.h"
@@ -15,9 +19,9 @@
 
 namespace {
 
-constexpr int SORT_THREADS = 256;
+constexpr int SORT_THREADS = 512;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ITERS = 8;                                    // 64-pair steps per wavefront
+constexpr int SORT_ITERS = 4;                                    // 64-pair steps per wavefront
 constexpr int SORT_CHUNK = SORT_THREADS * SORT_ITERS;            // pairs per block
 constexpr int SORT_MAX_NR = 1024;                                // local experts supported
 
@@ -27,10 +31,14 @@ struct RowWeights {
     const void *routing_weights = nullptr;
     float *row_weights = nullptr;
     int bf16 = 0;
-    __device__ __forceinline__ void put(int pos, int64_t pair) const {
-        if (!row_weights) return;
-        row_weights[pos] = bf16 ? bf16_bits_to_f32(static_cast<const uint16_t *>(routing_weights)[pair])
-                                : static_cast<const float *>(routing_weights)[pair];
+    // fetched for all of a wavefront's pairs before the first is placed: a load per placement would be waited for each time
+    __device__ __forceinline__ float get(int64_t pair, int64_t n_pairs) const {
+        if (!row_weights || pair >= n_pairs) return 0.0f;
+        return bf16 ? bf16_bits_to_f32(static_cast<const uint16_t *>(routing_weights)[pair])
+                    : static_cast<const float *>(routing_weights)[pair];
+    }
+    __device__ __forceinline__ void put(int pos, float weight) const {
+        if (row_weights) row_weights[pos] = weight;
     }
 };
 
@@ -54,19 +62,29 @@ __device__ __forceinline__ unsigned long long match_key(int key, int nbits) {
 
 __device__ __forceinline__ unsigned long long lanemask_lt(int lane) { return (1ull << lane) - 1ull; }
 
-// Per-wave histogram of the wave's SORT_ITERS*64 pairs into wave_hist[wave][0..NR).
+// The keys of a wavefront's SORT_ITERS*64 pairs, all loads in flight at once.
 template <typename TI>
-__device__ __forceinline__ int wave_histogram(const TI *selected_experts, int64_t wave_base,
-                                              int64_t n_pairs, int start, int end, int NR, int nbits,
-                                              int lane, volatile int *hist) {
-    int hits = 0;
+__device__ __forceinline__ void wave_keys(const TI *selected_experts, int64_t wave_base, int64_t n_pairs, int start,
+                                          int end, int NR, int lane, int (&key)[SORT_ITERS]) {
+    TI e[SORT_ITERS];
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++) e[it] = selected_experts[min(wave_base + it * 64 + lane, n_pairs - 1)];
+#pragma unroll
     for (int it = 0; it < SORT_ITERS; it++) {
-        const int64_t j = wave_base + it * 64 + lane;
-        const int key = local_key(selected_experts, j, n_pairs, start, end, NR);
-        const unsigned long long m = match_key(key, nbits);
+        const long long v = static_cast<long long>(e[it]);
+        key[it] = wave_base + it * 64 + lane < n_pairs && v >= start && v < end ? static_cast<int>(v - start) : NR;
+    }
+}
+
+// Per-wave histogram of these keys into wave_hist[wave][0..NR).
+__device__ __forceinline__ int wave_histogram(const int (&key)[SORT_ITERS], int NR, int nbits, int lane, volatile int *hist) {
+    int hits = 0;
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++) {
+        const unsigned long long m = match_key(key[it], nbits);
         const bool leader = (__ffsll(static_cast<long long>(m)) - 1) == lane;
-        if (leader && key < NR) hist[key] += __popcll(m);
-        hits += __popcll(__ballot(key < NR));
+        if (leader && key[it] < NR) hist[key[it]] += __popcll(m);
+        hits += __popcll(__ballot(key[it] < NR));
         __builtin_amdgcn_wave_barrier();
     }
     return hits;
@@ -79,10 +97,12 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_count_kernel(const TI *__re
                                                                   int32_t *__restrict__ block_hist) {
     extern __shared__ int lds[];  // [SORT_WAVES][NR]
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t wave_base = static_cast<int64_t>(blockIdx.x) * SORT_CHUNK + wv * (SORT_ITERS * 64);
+    int key[SORT_ITERS];
+    wave_keys(selected_experts, wave_base, n_pairs, start, end, NR, lane, key);
     for (int i = threadIdx.x; i < SORT_WAVES * NR; i += SORT_THREADS) lds[i] = 0;
     __syncthreads();
-    const int64_t wave_base = static_cast<int64_t>(blockIdx.x) * SORT_CHUNK + wv * (SORT_ITERS * 64);
-    wave_histogram(selected_experts, wave_base, n_pairs, start, end, NR, nbits, lane, lds + wv * NR);
+    wave_histogram(key, NR, nbits, lane, lds + wv * NR);
     __syncthreads();
     for (int e = threadIdx.x; e < NR; e += SORT_THREADS) {
         int s = 0;
@@ -169,11 +189,15 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
     extern __shared__ int lds[];  // [SORT_WAVES][NR] then [SORT_WAVES] wave hit counts
     int *wave_hits = lds + SORT_WAVES * NR;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t wave_base = static_cast<int64_t>(blockIdx.x) * SORT_CHUNK + wv * (SORT_ITERS * 64);
+    int key[SORT_ITERS];
+    float weight[SORT_ITERS];
+    wave_keys(selected_experts, wave_base, n_pairs, start, end, NR, lane, key);
+#pragma unroll
+    for (int it = 0; it < SORT_ITERS; it++) weight[it] = rw.get(wave_base + it * 64 + lane, n_pairs);
     for (int i = threadIdx.x; i < SORT_WAVES * NR; i += SORT_THREADS) lds[i] = 0;
     __syncthreads();
-    const int64_t wave_base = static_cast<int64_t>(blockIdx.x) * SORT_CHUNK + wv * (SORT_ITERS * 64);
-    const int hits = wave_histogram(selected_experts, wave_base, n_pairs, start, end, NR, nbits, lane,
-                                    lds + wv * NR);
+    const int hits = wave_histogram(key, NR, nbits, lane, lds + wv * NR);
     if (lane == 0) wave_hits[wv] = hits;
     __syncthreads();
     // counts -> running offsets: off[w][e] = block offset + counts of the waves before w
@@ -192,7 +216,8 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
     // Entries past the number of kept pairs (an expert window keeps fewer than T*K) are given fixed
     // values, so that a caller who sizes its work by T*K instead of reading the count back can tell
     // them apart: output_indices -1 (no row), the other two 0 (a valid token / slot).
-    const int total_kept = cum_expert_counts_ep[n_pairs / K];
+    const int total_kept = cum_expert_counts_ep[static_cast<uint32_t>(n_pairs) / static_cast<uint32_t>(K)];
+#pragma unroll
     for (int it = 0; it < SORT_ITERS; it++) {
         const int64_t j = wave_base + it * 64 + lane;
         if (j < n_pairs && j >= total_kept) {
@@ -200,23 +225,22 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
             input_indices[j] = 0;
             selected_experts_indices[j] = 0;
         }
-        const int key = local_key(selected_experts, j, n_pairs, start, end, NR);
-        const unsigned long long m = match_key(key, nbits);
-        const unsigned long long kept = __ballot(key < NR);
+        const unsigned long long m = match_key(key[it], nbits);
+        const unsigned long long kept = __ballot(key[it] < NR);
         const int oi = oi_base + __popcll(kept & lanemask_lt(lane));
         const bool valid = j < n_pairs;
-        const int64_t t = valid ? j / K : 0;
-        const int k = valid ? static_cast<int>(j - t * K) : 0;
+        const uint32_t t = valid ? static_cast<uint32_t>(j) / static_cast<uint32_t>(K) : 0;   // (pairs are counted in int32)
+        const int k = valid ? static_cast<int>(static_cast<uint32_t>(j) - t * K) : 0;
         if (valid && k == 0) cum_expert_counts_ep[t] = oi;
-        if (key < NR) {
-            const int pos = off[key] + __popcll(m & lanemask_lt(lane));
+        if (key[it] < NR) {
+            const int pos = off[key[it]] + __popcll(m & lanemask_lt(lane));
             __builtin_amdgcn_wave_barrier();
             const bool leader = (__ffsll(static_cast<long long>(m)) - 1) == lane;
-            if (leader) off[key] += __popcll(m);
+            if (leader) off[key[it]] += __popcll(m);
             input_indices[pos] = static_cast<int32_t>(t);
             output_indices[oi] = pos;
             selected_experts_indices[oi] = k;
-            rw.put(pos, j);
+            rw.put(pos, weight[it]);
         } else {
             __builtin_amdgcn_wave_barrier();
         }
@@ -230,8 +254,8 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
 // nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced),
 // one of 6 now.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront)
 // reaches what the three launches take.
-constexpr int SMALL_WAVES = 16;
-constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SORT_ITERS;
+constexpr int SMALL_WAVES = 16, SMALL_ITERS = 8;
+constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SMALL_ITERS;
 constexpr int SMALL_MAX_NR = 256;
 template <typename TI>
 __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
@@ -244,15 +268,18 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     for (int i = tid; i < SMALL_WAVES * NR; i += SMALL_WAVES * 64) off[i / NR][i % NR] = 0;
     const int base = wv * iters * 64;
-    int key[SORT_ITERS];
+    int key[SMALL_ITERS];
 #pragma unroll
-    for (int it = 0; it < SORT_ITERS; it++)
+    for (int it = 0; it < SMALL_ITERS; it++)
         key[it] = it < iters ? local_key(selected_experts, base + it * 64 + lane, n_pairs, start, end, NR) : NR;
+    float weight[SMALL_ITERS];
+#pragma unroll
+    for (int it = 0; it < SMALL_ITERS; it++) weight[it] = it < iters ? rw.get(base + it * 64 + lane, n_pairs) : 0.0f;
     __syncthreads();
     volatile int *mine = off[wv];
     int hits = 0;
 #pragma unroll
-    for (int it = 0; it < SORT_ITERS; it++) {
+    for (int it = 0; it < SMALL_ITERS; it++) {
         if (it >= iters) break;
         const unsigned long long m = match_key(key[it], nbits);
         if (key[it] < NR && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] += __popcll(m);
@@ -288,7 +315,7 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
     for (int w = 0; w < wv; w++) oi_base += wave_hits[w];
     const int kept_all = kept_total;
 #pragma unroll
-    for (int it = 0; it < SORT_ITERS; it++) {
+    for (int it = 0; it < SMALL_ITERS; it++) {
         if (it >= iters) break;
         const int j = base + it * 64 + lane;
         if (j < n_pairs && j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
@@ -310,7 +337,7 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
             input_indices[pos] = t;
             output_indices[oi] = pos;
             selected_experts_indices[oi] = k;
-            rw.put(pos, j);
+            rw.put(pos, weight[it]);
         }
         oi_base += __popcll(kept);
         __builtin_amdgcn_wave_barrier();
