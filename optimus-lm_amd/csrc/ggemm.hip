@@ -179,27 +179,32 @@ __device__ __forceinline__ void unpack4_bf16(u32x2 v, float *f) {
 
 // Row tiles of fwd/dgrad are cut per expert (BM rows each, the last one of an expert partial).
 // One wavefront builds, once per block, a table in LDS from the device-resident cum_token_counts:
-// tile_end[e] = number of row tiles of experts 0..e, seg[e] = cum_token_counts[e].
+// tile_end[e] = number of row tiles of experts 0..e, seg[e] = cum_token_counts[e].  The 256x256 kernels
+// (HALVES) list an expert's last tile apart when at most 128 rows are left for it: tile_end then counts
+// the other tiles, half_end those.
 constexpr int MAX_EXPERTS = 1024;
-template <int BM>
+template <int BM, bool HALVES>
 __device__ __forceinline__ void build_tile_table(const int32_t *cum, int n_experts, int lane,
-                                                 int *tile_end, int *seg) {
-    int base_tiles = 0;
+                                                 int *tile_end, int *half_end, int *seg) {
+    int base_tiles = 0, base_halves = 0;
     for (int e0 = 0; e0 < n_experts; e0 += 64) {
         const int e = e0 + lane;
         int s = 0, cnt = 0;
         if (e < n_experts) { s = cum[e]; cnt = cum[e + 1] - s; }
-        int incl = (cnt + BM - 1) / BM;  // inclusive scan over the wavefront
+        const int half = HALVES && cnt % BM > 0 && cnt % BM <= BM / 2 ? 1 : 0;
+        int incl = (cnt + BM - 1) / BM - half, halves = half;  // inclusive scans over the wavefront
         for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += v;
+            const int v = __shfl_up(incl, o, 64), h = HALVES ? __shfl_up(halves, o, 64) : 0;
+            if (lane >= o) { incl += v; halves += h; }
         }
         if (e < n_experts) {
             tile_end[e] = base_tiles + incl;
+            if (HALVES) half_end[e] = base_halves + halves;
             seg[e] = s;
             if (e == n_experts - 1) seg[n_experts] = s + cnt;
         }
         base_tiles += __shfl(incl, 63, 64);
+        if (HALVES) base_halves += __shfl(halves, 63, 64);
     }
 }
 
@@ -329,6 +334,16 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     int cached_expert = -1;
     __shared__ int tile_end[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
     __shared__ int seg[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS + 1];
+    // A 256-row tile with at most 128 rows is half a tile's work: its lower four wavefronts (one per SIMD) do
+    // all of it, the upper four only fetch their share of B.  A block's share of such tiles comes after its
+    // whole ones, so that the last round of a launch is one of halves.  The step of a half tile is bound by the
+    // latency of its weights and not much shorter than a whole one's, so the gain is that of the rounds: 32
+    // experts of 7168/2048 with 256 rows each on average, us, gate+up 977 -> 923, down input gradient
+    // 582 -> 519, gate/up input gradient 933 -> 904; 64 experts of 2048/1024 with 512 rows, gate+up 378 -> 372,
+    // down 196 -> 189; with 2048 rows each +-1 %.
+    constexpr bool HALVES = BM == 256 && EPI != EPI_WGRAD;
+    __shared__ int half_end[HALVES ? MAX_EXPERTS : 1];
+    int whole_tiles = 0;   // HALVES: the tiles before the halves
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -430,10 +445,13 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         } else {
             constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
             const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
+            const bool half = HALVES && logical >= whole_tiles;
+            if (half) logical -= whole_tiles;
             const int tile_m = logical / tiles_n;
             const int tile_n = logical % tiles_n;
             rot_a = tile_n; rot_b = tile_m & 7;
-            if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane_s, expert, row_begin, row_end)) return false;
+            if (!find_tile<BM>(half ? half_end : tile_end, seg, p.n_experts, tile_m, lane_s, expert, row_begin, row_end)) return false;
+            if (half) row_begin = seg[expert] + (row_end - seg[expert]) / BM * BM;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
             c_len = p.kc;
@@ -809,10 +827,13 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     // counted here from cum_token_counts, so that all XCDs get equal shares of real work.
     int total_tiles = p.total_tiles;
     if (EPI != EPI_WGRAD) {
-        if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
+        if (wave == 0) build_tile_table<BM, HALVES>(p.cum, p.n_experts, lane, tile_end, half_end, seg);
         __syncthreads();
         constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
-        total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+        const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
+        total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * tiles_n;
+        whole_tiles = total_tiles;
+        if (HALVES) total_tiles += __builtin_amdgcn_readfirstlane(half_end[p.n_experts - 1]) * tiles_n;
     }
     const int nbx = gridDim.x / NUM_XCD;
     const int xcd = blockIdx.x % NUM_XCD, slot = blockIdx.x / NUM_XCD;
@@ -825,11 +846,30 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         per = __builtin_amdgcn_readfirstlane(hi) - run_lo;
         rem = 0;
     }
+    // HALVES: XCD x owns an eighth of the whole tiles and an eighth of the halves, both contiguous.  The whole
+    // ones go round its blocks; the last round leaves `spare` blocks without one, which take the first two
+    // rounds of halves, and the rest goes round all blocks.
+    int halves_lo = 0, halves = 0, spare = 0;
+    if (HALVES) {
+        run_lo = static_cast<int>(static_cast<int64_t>(whole_tiles) * xcd / NUM_XCD);
+        per = static_cast<int>(static_cast<int64_t>(whole_tiles) * (xcd + 1) / NUM_XCD) - run_lo;
+        rem = 0;
+        halves_lo = static_cast<int>(static_cast<int64_t>(total_tiles - whole_tiles) * xcd / NUM_XCD);
+        halves = static_cast<int>(static_cast<int64_t>(total_tiles - whole_tiles) * (xcd + 1) / NUM_XCD) - halves_lo;
+        spare = per % nbx ? nbx - per % nbx : 0;
+    }
     const int n_mine = slot < per ? (per - slot + nbx - 1) / nbx : 0;
     const int n_all = n_mine + ((xcd < rem && slot == per % nbx) ? 1 : 0);
     int it = 0;
     // moves the per-tile state to this block's next tile that has rows; false when there is none
     auto next_tile = [&]() -> bool {
+        if (HALVES) {
+            const int k = it++ - n_mine;
+            if (k < 0) return setup_tile(run_lo + slot + (k + n_mine) * nbx);
+            const bool first = spare > 0 && slot >= nbx - spare;
+            const int half = first && k < 2 ? slot - (nbx - spare) + k * spare : 2 * spare + slot + (k - (first ? 2 : 0)) * nbx;
+            return half < halves && setup_tile(whole_tiles + halves_lo + half);
+        }
         while (it < n_all) {
             const int logical = it < n_mine ? run_lo + slot + it * nbx : total_tiles - rem + xcd;
             it++;
@@ -859,6 +899,18 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         fetch_a(1);
         read_group(stage0, 0, 0);
         const int n_steps = loop_steps;
+        if (HALVES && wave_u >= NW / 2 && row_end - row_begin <= BM / 2) {
+            // nothing to multiply: this wavefront's rows of B for every step, and the steps' barriers
+            // (its A rows lie past the expert's rows and nobody reads them)
+            for (int step = 0; step < n_steps; step += 2) {
+                issue_part(step + 1, stage1, A_LOADS, NL);
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+                __syncthreads();
+                issue_part(step + 2, stage0, A_LOADS, NL);
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+                __syncthreads();
+            }
+        } else
         for (int step = 0; step < n_steps; step += 2) {
             half_step(stage0, stage1, step, 0);
             if (!ANY_STEPS || step + 1 < n_steps) half_step(stage1, stage0, step + 1, 1);
