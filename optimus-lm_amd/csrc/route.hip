@@ -77,21 +77,24 @@ __device__ __forceinline__ float fetch_expert_value(const float (&x)[PER], int e
 template <int PER>
 __device__ __forceinline__ void partial_logits(const float *partial, int splits, int64_t Tn, int64_t t, int N, int lane,
                                                float (&x)[PER]) {
+    // eight slices of all the lane's experts in flight, added in slice order; past the end the last valid one again
+    float s[PER];
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int i = lane + 64 * j;
-        x[j] = -INFINITY;
-        if (i >= N) continue;
-        float s = 0.0f;
-        for (int k0 = 0; k0 < splits; k0 += 8) {   // eight loads in flight
-            float v[8];
+    for (int j = 0; j < PER; j++) s[j] = 0.0f;
+    for (int k0 = 0; k0 < splits; k0 += 8) {
+        float v[8][PER];
 #pragma unroll
-            for (int u = 0; u < 8; u++) v[u] = (k0 + u < splits) ? partial[((k0 + u) * Tn + t) * N + i] : 0.0f;
+        for (int u = 0; u < 8; u++)
 #pragma unroll
-            for (int u = 0; u < 8; u++) s += v[u];
-        }
-        x[j] = s;
+            for (int j = 0; j < PER; j++)
+                v[u][j] = partial[(min(k0 + u, splits - 1) * Tn + t) * N + min(lane + 64 * j, N - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+            for (int j = 0; j < PER; j++) s[j] += k0 + u < splits ? v[u][j] : 0.0f;
     }
+#pragma unroll
+    for (int j = 0; j < PER; j++) x[j] = lane + 64 * j < N ? s[j] : -INFINITY;
 }
 
 // logits (lanes past N: -inf) -> softmax probabilities, in place

@@ -529,3 +529,30 @@ def test_few_row_products_stream_the_weights(cuda, counts, N, K, weighted):
         # one bf16 rounding (2^-9 of the value), and sums of K products in another order; h from unrounded g, u
         err = (got[:rows].float().cpu() - want).abs()
         assert (err <= want.abs() * 2 ** -8 + 1e-6 * K ** 0.5).all(), (name, float(err.max()))
+
+
+@pytest.mark.parametrize("counts", [[128, 129, 256, 384, 385, 1, 0, 639], [255, 257, 0, 512, 127, 130, 300, 300]], ids=str)
+def test_half_row_tiles_of_the_256_kernels(cuda, counts):
+    """The 256x256 kernels list an expert's last row tile apart when at most 128 rows are left for it and give
+    it to half of a block's wavefronts, behind the whole tiles: remainders on both sides of 0, 128 and 256,
+    experts with such a tile only, without one, and without rows; more tiles than blocks.  One bf16 rounding of
+    a float32 sum of at most 1024 products (2^-8 of the value, and the order of the sum)."""
+    from optimus import _native as n
+    counts = counts * 6
+    G, N, K, rows = len(counts), 1024, 512, sum(counts)
+    assert rows >= 192 * G and (rows // 256) * (min(N, K) // 256) * 2 >= 256 // 2
+    g = torch.Generator().manual_seed(rows)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    x = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(cuda)
+    dy = torch.randn(rows, N, generator=g).to(torch.bfloat16).to(cuda)
+    w = (torch.randn(G, N, K, generator=g) * 0.05).to(torch.bfloat16).to(cuda)
+    y, dx = torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=cuda), torch.full((rows, K), 7.0, dtype=torch.bfloat16, device=cuda)
+    d, P = cum.to(cuda), n.ptr
+    n.check(n.lib().om_grouped_gemm_fwd(P(x), P(w), P(y), P(d), rows, G, N, K, 0, n.stream()), "fwd")
+    n.check(n.lib().om_grouped_gemm_dgrad(P(dy), P(w), P(dx), P(d), rows, G, N, K, 0, n.stream()), "dgrad")
+    torch.cuda.synchronize()
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        for name, got, want, k in (("fwd", y[s], x[s].float() @ w[e].float().t(), K), ("dgrad", dx[s], dy[s].float() @ w[e].float(), N)):
+            assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6 * k ** 0.5).all(), (name, e)

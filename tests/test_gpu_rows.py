@@ -115,3 +115,22 @@ def test_combine_with_residual_equals_two_steps(cuda, oracle_lib, dtype, wdtype,
     one = torch.empty(T, E, dtype=dtype, device=cuda)
     ops.reduce_ggemm_output_residual(yd, wd, ce, si, oi, res, one)
     assert np.array_equal(bits(one), bits(two))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,N,K,E", [(8, 16, 9, 8), (16, 16, 9, 520), (512, 24, 17, 264), (520, 8, 3, 4104), (3000, 8, 3, 264),
+                                     (1600, 8, 3, 1416)])
+def test_token_sums_on_both_sides_of_the_few_tokens_line(cuda, oracle_lib, dtype, T, N, K, E):
+    """Few tokens run a wavefront per 64-vector chunk with eight rows in flight: more rows per token than that
+    and a remainder, one vector more than a chunk, an expert window that leaves tokens without rows, and
+    sizes on either side of the line.  Same order of the sums: bit-exact."""
+    import pcl_xpu_customops as ops
+    start, end = N // 4, N // 2
+    for lo, hi in ((0, N), (start, end)):
+        se, idx, x, y, w = _setup(T, N, K, E, lo, hi, dtype, oracle_lib)
+        ce, oi = torch.from_numpy(idx["cum_expert_counts_ep"]).to(cuda), torch.from_numpy(idx["output_indices"]).to(cuda)
+        if idx["num_routed_tokens"] == 0:
+            continue
+        hg = torch.empty(T, E, dtype=dtype, device=cuda)
+        ops.shuffle_sub_matrix_reduce(y.to(cuda), ce, oi, hg)
+        assert np.array_equal(bits(hg), oracle_lib.shuffle_sub_matrix_reduce(bits(y), idx["cum_expert_counts_ep"], idx["output_indices"], T))
