@@ -456,6 +456,7 @@ class GradNormPlan:
     clip_grads_with_norm_ compute them, including the roundings to the gradient dtype."""
 
     CHUNK = 1 << 16
+    ONE_LAUNCH_MAX = 24 << 20
 
     def __init__(self, starts, sizes, device, chunk=None):
         # two blocks per CU for a small buffer (a chunk is one block's work), 64 K elements each for a large one
@@ -478,7 +479,10 @@ class GradNormPlan:
         self.n_segs = len(sizes)
         self.chunk_offsets = table.to(device)
         self.seg_first_chunk = torch.tensor(first, dtype=torch.int64).to(device)
-        self.one_launch = bool(_n.lib().om_grad_norm_fits(self.n_chunks, self.n_segs))
+        # (us per step, bf16, three launches and a copy -> one: 3e6 elements 54 -> 31, 1e7 64 -> 61, 2e7 110 -> 109,
+        # 3.1e7 163 -> 164 to 169, 6e7 307 -> 309: from there on the last block's sums are not hidden by anything)
+        self.one_launch = sum(int(sz) for sz in sizes) <= self.ONE_LAUNCH_MAX \
+            and bool(_n.lib().om_grad_norm_fits(self.n_chunks, self.n_segs))
         # one buffer: total norm, clip coefficient, the one-launch kernel's block count (starts at zero)
         self._words = torch.zeros(3, dtype=torch.float32, device=device)
         self.total, self.coef = self._words[0], self._words[1:2]
