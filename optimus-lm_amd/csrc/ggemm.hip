@@ -88,6 +88,7 @@ struct GemmParams {
     int m_tiles_max;            // fwd/dgrad: upper bound on row tiles
     int total_tiles;            // logical tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert
+    int halves_last;            // 256x256 fwd/dgrad: tiles with at most 128 rows are dealt out after the others
 };
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
@@ -180,18 +181,18 @@ __device__ __forceinline__ void unpack4_bf16(u32x2 v, float *f) {
 // Row tiles of fwd/dgrad are cut per expert (BM rows each, the last one of an expert partial).
 // One wavefront builds, once per block, a table in LDS from the device-resident cum_token_counts:
 // tile_end[e] = number of row tiles of experts 0..e, seg[e] = cum_token_counts[e].  The 256x256 kernels
-// (HALVES) list an expert's last tile apart when at most 128 rows are left for it: tile_end then counts
-// the other tiles, half_end those.
+// (HALVES) list an expert's last tile apart when at most 128 rows are left for it and `halves_last` says so:
+// tile_end then counts the other tiles, half_end those.
 constexpr int MAX_EXPERTS = 1024;
 template <int BM, bool HALVES>
-__device__ __forceinline__ void build_tile_table(const int32_t *cum, int n_experts, int lane,
+__device__ __forceinline__ void build_tile_table(const int32_t *cum, int n_experts, int lane, bool halves_last,
                                                  int *tile_end, int *half_end, int *seg) {
     int base_tiles = 0, base_halves = 0;
     for (int e0 = 0; e0 < n_experts; e0 += 64) {
         const int e = e0 + lane;
         int s = 0, cnt = 0;
         if (e < n_experts) { s = cum[e]; cnt = cum[e + 1] - s; }
-        const int half = HALVES && cnt % BM > 0 && cnt % BM <= BM / 2 ? 1 : 0;
+        const int half = HALVES && halves_last && cnt % BM > 0 && cnt % BM <= BM / 2 ? 1 : 0;
         int incl = (cnt + BM - 1) / BM - half, halves = half;  // inclusive scans over the wavefront
         for (int o = 1; o < 64; o <<= 1) {
             const int v = __shfl_up(incl, o, 64), h = HALVES ? __shfl_up(halves, o, 64) : 0;
@@ -827,7 +828,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     // counted here from cum_token_counts, so that all XCDs get equal shares of real work.
     int total_tiles = p.total_tiles;
     if (EPI != EPI_WGRAD) {
-        if (wave == 0) build_tile_table<BM, HALVES>(p.cum, p.n_experts, lane, tile_end, half_end, seg);
+        if (wave == 0) build_tile_table<BM, HALVES>(p.cum, p.n_experts, lane, p.halves_last != 0, tile_end, half_end, seg);
         __syncthreads();
         constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
         const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
@@ -1180,6 +1181,9 @@ int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad f
     const int64_t tiles = static_cast<int64_t>(p.m_tiles_max) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
+    // (with more rows per expert the halves are few, and away from their expert's whole tiles they fetch its weights
+    // once more: a step of 8192 tokens, 1024 rows each on average, is 1.4 % slower with them last)
+    p.halves_last = rows <= static_cast<int64_t>(p.n_experts) * 640;
     ggemm_kernel<BM, BN, Waves<BM>::M, Waves<BM>::N, AKIND, BKIND, EPI, GATHER, ROWW, false, KTAIL, REGLOAD>
         <<<dim3(persistent_blocks<BM>(tiles)), dim3(Waves<BM>::M * Waves<BM>::N * 64), 0, st>>>(p);
     return om_launch_status();
@@ -1190,9 +1194,17 @@ int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad f
 // the CUs (a tiny problem is spread over more CUs by the 128x128 tile).  The 128x128 tile takes any
 // extents and contraction lengths that are multiples of 8: its last column tile and its last
 // contraction step may be partial.
+//
+// "Enough rows", with a nearly empty tile costing less than a whole one (HALVES), is 160 per expert on average,
+// and 112 where an expert's matrix has 4 M weights or more; 192 for the SwiGLU backward of smaller experts.
+// us, 128x128 -> 256x256, even routing / rows spread as exp(0.8 N(0,1)): 32 experts of 7168/2048, 112 rows, gate+up
+// 451 -> 410 / 534 -> 537, gate/up input gradient 445 -> 429 / 603 -> 469; 144 rows 709 -> 458 / 644 -> 568
+// and 763 -> 479 / 688 -> 551; 80 rows 362 -> 395 / 446 -> 522.  64 experts of 2048/1024, 176 rows, all four
+// products 569 -> 439 / 555 -> 542 (SwiGLU backward 104 -> 82 / 101 -> 112), 144 rows 555 -> 456 / 510 -> 531.
 template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t rows) {
     constexpr int div = (EPI == EPI_SWIGLU) ? 2 : 1;
-    if (n_cols % (256 / div) != 0 || kc % 128 != 0 || rows < static_cast<int64_t>(n_experts) * 192) return false;
+    const int enough = static_cast<int64_t>(n_cols) * kc >= (4 << 20) ? 112 : EPI == EPI_SWIGLU_BWD ? 192 : 160;
+    if (n_cols % (256 / div) != 0 || kc % 128 != 0 || rows < static_cast<int64_t>(n_experts) * enough) return false;
     const int64_t tiles = ((rows + 255) / 256) * (n_cols / (256 / div));
     return tiles * 2 >= device_cu_count();
 }
