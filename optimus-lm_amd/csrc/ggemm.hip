@@ -88,7 +88,6 @@ struct GemmParams {
     int m_tiles_max;            // fwd/dgrad: upper bound on row tiles
     int total_tiles;            // logical tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert
-    int halves_last;            // 256x256 fwd/dgrad: tiles with at most 128 rows are dealt out after the others
 };
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
@@ -180,32 +179,27 @@ __device__ __forceinline__ void unpack4_bf16(u32x2 v, float *f) {
 
 // Row tiles of fwd/dgrad are cut per expert (BM rows each, the last one of an expert partial).
 // One wavefront builds, once per block, a table in LDS from the device-resident cum_token_counts:
-// tile_end[e] = number of row tiles of experts 0..e, seg[e] = cum_token_counts[e].  The 256x256 kernels
-// (HALVES) list an expert's last tile apart when at most 128 rows are left for it and `halves_last` says so:
-// tile_end then counts the other tiles, half_end those.
+// tile_end[e] = number of row tiles of experts 0..e, seg[e] = cum_token_counts[e].
 constexpr int MAX_EXPERTS = 1024;
-template <int BM, bool HALVES>
-__device__ __forceinline__ void build_tile_table(const int32_t *cum, int n_experts, int lane, bool halves_last,
-                                                 int *tile_end, int *half_end, int *seg) {
-    int base_tiles = 0, base_halves = 0;
+template <int BM>
+__device__ __forceinline__ void build_tile_table(const int32_t *cum, int n_experts, int lane,
+                                                 int *tile_end, int *seg) {
+    int base_tiles = 0;
     for (int e0 = 0; e0 < n_experts; e0 += 64) {
         const int e = e0 + lane;
         int s = 0, cnt = 0;
         if (e < n_experts) { s = cum[e]; cnt = cum[e + 1] - s; }
-        const int half = HALVES && halves_last && cnt % BM > 0 && cnt % BM <= BM / 2 ? 1 : 0;
-        int incl = (cnt + BM - 1) / BM - half, halves = half;  // inclusive scans over the wavefront
+        int incl = (cnt + BM - 1) / BM;  // inclusive scan over the wavefront
         for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64), h = HALVES ? __shfl_up(halves, o, 64) : 0;
-            if (lane >= o) { incl += v; halves += h; }
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
         }
         if (e < n_experts) {
             tile_end[e] = base_tiles + incl;
-            if (HALVES) half_end[e] = base_halves + halves;
             seg[e] = s;
             if (e == n_experts - 1) seg[n_experts] = s + cnt;
         }
         base_tiles += __shfl(incl, 63, 64);
-        if (HALVES) base_halves += __shfl(halves, 63, 64);
     }
 }
 
@@ -336,15 +330,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     __shared__ int tile_end[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
     __shared__ int seg[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS + 1];
     // A 256-row tile with at most 128 rows is half a tile's work: its lower four wavefronts (one per SIMD) do
-    // all of it, the upper four only fetch their share of B.  A block's share of such tiles comes after its
-    // whole ones, so that the last round of a launch is one of halves.  The step of a half tile is bound by the
-    // latency of its weights and not much shorter than a whole one's, so the gain is that of the rounds: 32
-    // experts of 7168/2048 with 256 rows each on average, us, gate+up 977 -> 923, down input gradient
-    // 582 -> 519, gate/up input gradient 933 -> 904; 64 experts of 2048/1024 with 512 rows, gate+up 378 -> 372,
-    // down 196 -> 189; with 2048 rows each +-1 %.
+    // all of it, the upper four only fetch their share of B.  Its steps stay bound by the latency of its
+    // weights.  Dealing such tiles out after the whole ones, so that a launch's last round is one of halves,
+    // is slower: away from their expert's whole tiles they fetch its weights once more (forward of 3000 tokens,
+    // 64 experts of 2048/1024, 399 -> 445 us a pass, 4096 tokens 529 -> 541, a step of 2048 tokens 1081 -> 1131).
     constexpr bool HALVES = BM == 256 && EPI != EPI_WGRAD;
-    __shared__ int half_end[HALVES ? MAX_EXPERTS : 1];
-    int whole_tiles = 0;   // HALVES: the tiles before the halves
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -446,13 +436,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         } else {
             constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
             const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
-            const bool half = HALVES && logical >= whole_tiles;
-            if (half) logical -= whole_tiles;
             const int tile_m = logical / tiles_n;
             const int tile_n = logical % tiles_n;
             rot_a = tile_n; rot_b = tile_m & 7;
-            if (!find_tile<BM>(half ? half_end : tile_end, seg, p.n_experts, tile_m, lane_s, expert, row_begin, row_end)) return false;
-            if (half) row_begin = seg[expert] + (row_end - seg[expert]) / BM * BM;
+            if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane_s, expert, row_begin, row_end)) return false;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
             c_len = p.kc;
@@ -828,13 +815,10 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
     // counted here from cum_token_counts, so that all XCDs get equal shares of real work.
     int total_tiles = p.total_tiles;
     if (EPI != EPI_WGRAD) {
-        if (wave == 0) build_tile_table<BM, HALVES>(p.cum, p.n_experts, lane, p.halves_last != 0, tile_end, half_end, seg);
+        if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
         __syncthreads();
         constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
-        const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
-        total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * tiles_n;
-        whole_tiles = total_tiles;
-        if (HALVES) total_tiles += __builtin_amdgcn_readfirstlane(half_end[p.n_experts - 1]) * tiles_n;
+        total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     }
     const int nbx = gridDim.x / NUM_XCD;
     const int xcd = blockIdx.x % NUM_XCD, slot = blockIdx.x / NUM_XCD;
@@ -847,30 +831,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         per = __builtin_amdgcn_readfirstlane(hi) - run_lo;
         rem = 0;
     }
-    // HALVES: XCD x owns an eighth of the whole tiles and an eighth of the halves, both contiguous.  The whole
-    // ones go round its blocks; the last round leaves `spare` blocks without one, which take the first two
-    // rounds of halves, and the rest goes round all blocks.
-    int halves_lo = 0, halves = 0, spare = 0;
-    if (HALVES) {
-        run_lo = static_cast<int>(static_cast<int64_t>(whole_tiles) * xcd / NUM_XCD);
-        per = static_cast<int>(static_cast<int64_t>(whole_tiles) * (xcd + 1) / NUM_XCD) - run_lo;
-        rem = 0;
-        halves_lo = static_cast<int>(static_cast<int64_t>(total_tiles - whole_tiles) * xcd / NUM_XCD);
-        halves = static_cast<int>(static_cast<int64_t>(total_tiles - whole_tiles) * (xcd + 1) / NUM_XCD) - halves_lo;
-        spare = per % nbx ? nbx - per % nbx : 0;
-    }
     const int n_mine = slot < per ? (per - slot + nbx - 1) / nbx : 0;
     const int n_all = n_mine + ((xcd < rem && slot == per % nbx) ? 1 : 0);
     int it = 0;
     // moves the per-tile state to this block's next tile that has rows; false when there is none
     auto next_tile = [&]() -> bool {
-        if (HALVES) {
-            const int k = it++ - n_mine;
-            if (k < 0) return setup_tile(run_lo + slot + (k + n_mine) * nbx);
-            const bool first = spare > 0 && slot >= nbx - spare;
-            const int half = first && k < 2 ? slot - (nbx - spare) + k * spare : 2 * spare + slot + (k - (first ? 2 : 0)) * nbx;
-            return half < halves && setup_tile(whole_tiles + halves_lo + half);
-        }
         while (it < n_all) {
             const int logical = it < n_mine ? run_lo + slot + it * nbx : total_tiles - rem + xcd;
             it++;
@@ -1181,9 +1146,6 @@ int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad f
     const int64_t tiles = static_cast<int64_t>(p.m_tiles_max) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
-    // (with more rows per expert the halves are few, and away from their expert's whole tiles they fetch its weights
-    // once more: a step of 8192 tokens, 1024 rows each on average, is 1.4 % slower with them last)
-    p.halves_last = rows <= static_cast<int64_t>(p.n_experts) * 640;
     ggemm_kernel<BM, BN, Waves<BM>::M, Waves<BM>::N, AKIND, BKIND, EPI, GATHER, ROWW, false, KTAIL, REGLOAD>
         <<<dim3(persistent_blocks<BM>(tiles)), dim3(Waves<BM>::M * Waves<BM>::N * 64), 0, st>>>(p);
     return om_launch_status();

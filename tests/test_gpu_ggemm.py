@@ -533,9 +533,8 @@ def test_few_row_products_stream_the_weights(cuda, counts, N, K, weighted):
 
 @pytest.mark.parametrize("counts", [[128, 129, 256, 384, 385, 1, 0, 639], [255, 257, 0, 512, 127, 130, 300, 300]], ids=str)
 def test_half_row_tiles_of_the_256_kernels(cuda, counts):
-    """The 256x256 kernels list an expert's last row tile apart when at most 128 rows are left for it and give
-    it to half of a block's wavefronts, behind the whole tiles: remainders on both sides of 0, 128 and 256,
-    experts with such a tile only, without one, and without rows; more tiles than blocks.  One bf16 rounding of
+    """The 256x256 kernels give a row tile with at most 128 rows to half of a block's wavefronts: remainders
+    on both sides of 0, 128 and 256, experts with such a tile only, without one, and without rows; more tiles than blocks.  One bf16 rounding of
     a float32 sum of at most 1024 products (2^-8 of the value, and the order of the sum)."""
     from optimus import _native as n
     counts = counts * 6
