@@ -1157,15 +1157,21 @@ int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad f
 // extents and contraction lengths that are multiples of 8: its last column tile and its last
 // contraction step may be partial.
 //
-// "Enough rows", with a nearly empty tile costing less than a whole one (HALVES), is 160 per expert on average,
-// and 112 where an expert's matrix has 4 M weights or more; 192 for the SwiGLU backward of smaller experts.
-// us, 128x128 -> 256x256, even routing / rows spread as exp(0.8 N(0,1)): 32 experts of 7168/2048, 112 rows, gate+up
-// 451 -> 410 / 534 -> 537, gate/up input gradient 445 -> 429 / 603 -> 469; 144 rows 709 -> 458 / 644 -> 568
-// and 763 -> 479 / 688 -> 551; 80 rows 362 -> 395 / 446 -> 522.  64 experts of 2048/1024, 176 rows, all four
-// products 569 -> 439 / 555 -> 542 (SwiGLU backward 104 -> 82 / 101 -> 112), 144 rows 555 -> 456 / 510 -> 531.
+// "Enough rows" per expert on average: 160, for the SwiGLU backward, which suffers most from uneven rows, 192; where an
+// expert's matrix has 4 M weights or more, which the 128x128 tile reads once per 128 rows, 128 for gate+up and 112
+// for the plain store.  (Gate+up of smaller experts loses against uneven rows when launched alone, below; in whole
+// passes of 64 experts of 2048/1024 the 256x256 kernel is the better one at 160 to 175 rows: forward of 1330 tokens with
+// popularity as rank^-0.6 2.3 % faster, training steps of 1400 tokens even 0.9 %, of 1330 as rank^-1.2 0.2 %.)
+// Launches alone, us, 128x128 -> 256x256, even routing / rows spread
+// as exp(0.8 N(0,1)).  32 experts of 7168/2048: gate+up at 112 rows 450 -> 399 / 531 -> 569, 144 rows 710 -> 450 /
+// 642 -> 596, SwiGLU backward at 144 rows 348 -> 213 / 329 -> 357, gate/up input gradient at 80 rows 396 -> 420 /
+// 486 -> 446, 112 rows 446 -> 430 / 603 -> 462, down 214 -> 210 / 258 -> 228.  64 experts of 2048/1024 at 176 rows:
+// gate+up 186 -> 169 / 176 -> 199, SwiGLU backward 101 -> 80 / 99 -> 124, down 89 -> 73 / 86 -> 85, gate/up input
+// gradient 179 -> 130 / 183 -> 169; at 112 rows down 64 -> 60 / 65 -> 77.
 template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t rows) {
     constexpr int div = (EPI == EPI_SWIGLU) ? 2 : 1;
-    const int enough = static_cast<int64_t>(n_cols) * kc >= (4 << 20) ? 112 : EPI == EPI_SWIGLU_BWD ? 192 : 160;
+    const bool large = static_cast<int64_t>(n_cols) * kc >= (4 << 20);
+    const int enough = EPI == EPI_SWIGLU_BWD ? 192 : !large ? 160 : EPI == EPI_SWIGLU ? 128 : 112;
     if (n_cols % (256 / div) != 0 || kc % 128 != 0 || rows < static_cast<int64_t>(n_experts) * enough) return false;
     const int64_t tiles = ((rows + 255) / 256) * (n_cols / (256 / div));
     return tiles * 2 >= device_cu_count();
