@@ -474,6 +474,21 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
 
 // ---- autograd plumbing --------------------------------------------------------------------------------
 
+// The nodes below have no forward-mode formula and no batching rule, and their forward runs below the
+// dispatch keys that would ask for one: without this a tangent or a batch dimension is dropped unnoticed.
+// Called first by every entry point with a differentiable input.  (NotImplementedError: what a Python
+// autograd function without `jvp` raises.)
+void refuse_transforms(at::ArrayRef<Tensor> ts) {
+    static constexpr c10::DispatchKeySet functorch({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
+    for (const Tensor &t : ts) {
+        if (!t.defined()) continue;
+        TORCH_CHECK_NOT_IMPLEMENTED(!t._fw_grad(/*level=*/0).defined(),
+                                    "the fused MoE functions have no forward-mode derivative (jvp): use reverse mode");
+        TORCH_CHECK(!t.key_set().has_any(functorch),
+                    "the fused MoE functions cannot run under torch.func transforms (vmap, grad, jvp): use torch.autograd");
+    }
+}
+
 bool any_requires_grad(at::ArrayRef<Tensor> ts) {
     if (!at::GradMode::is_enabled()) return false;
     for (const Tensor &t : ts)
@@ -685,6 +700,7 @@ std::shared_ptr<RouterNode> router_node(const Tensor &x, const Tensor &weight) {
 
 // (logits float32, x)
 std::tuple<Tensor, Tensor> gate_logits(const Tensor &x, const Tensor &weight) {
+    refuse_transforms({x, weight});
     Tensor logits, x_out;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -709,6 +725,7 @@ Tensor route_workspace(const Tensor &x, int64_t T, int64_t H, int64_t N) {
 // to bf16 before the softmax, as a bf16 linear layer returns them.
 std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
                                                          at::ScalarType out_dtype, bool one_pass, bool bf16_logits) {
+    refuse_transforms({x, weight});
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
     // Up to 2048 tokens the one-pass kernel has at most 64 blocks, each walking all of H: the projection split
     // over H and a routing launch behind it give the same bits (eight slices added in the one-pass order)
@@ -754,6 +771,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
 // sigmoid / group-limited router -> (selected_experts int64, routing_weights float32, x)
 std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &weight, const Tensor &bias, int64_t n_group,
                                                  int64_t topk_group, int64_t top_k, bool renorm, double scale) {
+    refuse_transforms({x, weight, bias});
     const int64_t T = x.size(0), N = weight.size(0);
     Tensor logits, weights, experts, x_out;
     {
@@ -885,6 +903,8 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
 Tensor routed_mlp(const Tensor &x, const Tensor &rw, const Tensor &in, const Tensor &cum_ep, const Tensor &out,
                   const Tensor &sel, Tensor cum, const std::optional<Tensor> &residual, bool bound, bool merged,
                   const std::vector<Tensor> &leaves, bool has_shared, const std::optional<Tensor> &one) {
+    refuse_transforms({x, rw, residual.value_or(Tensor())});
+    refuse_transforms(leaves);
     const Call c = begin_call();
     for (const Tensor *t : {&in, &cum_ep, &out, &sel}) require_device(*t);
     if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
@@ -933,6 +953,8 @@ struct CountReadback {
 Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
                    bool sync_free, const std::optional<Tensor> &residual, bool merged, const std::vector<Tensor> &leaves,
                    bool has_shared, const std::optional<Tensor> &one) {
+    refuse_transforms({x, rw, residual.value_or(Tensor())});
+    refuse_transforms(leaves);
     const Call c = begin_call();
     Index ix;
     rw = rw.contiguous();
@@ -993,6 +1015,7 @@ Tensor merged_mlp(const Tensor &x, Tensor cum, bool merged, const std::vector<Te
                   const std::optional<Tensor> &out_rows) {
     variable_list inputs = {x};
     inputs.insert(inputs.end(), leaves.begin(), leaves.end());
+    refuse_transforms(inputs);
     const int64_t G = merged ? 1 : static_cast<int64_t>(leaves.size() / 3);
     MlpWeights w;
     MlpState s;
@@ -1048,6 +1071,7 @@ struct CombineNode : HostNode {      // saves y, rw, sel, in, out
 
 Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const Tensor &sel, const Tensor &in,
                const Tensor &out, const std::optional<Tensor> &residual) {
+    refuse_transforms({y, rw_in, residual.value_or(Tensor())});
     Tensor final, rw = rw_in;
     {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -1,0 +1,71 @@
+"""The C++ host module's entry points where no kernel runs: what they refuse, and how they find the weights."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwAD
+
+from optimus import _native as _n
+
+T, H, I, N, K = 4, 16, 8, 3, 2
+
+
+def _tensors():
+    g = torch.Generator().manual_seed(0)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    i32 = lambda n: torch.zeros(n, dtype=torch.int32)
+    return dict(x=rnd(T, H), weight=rnd(N, H), bias=torch.zeros(N), rw=rnd(T, K), residual=rnd(T, H), y=rnd(T * K, H),
+                gate=rnd(N, I, H), up=rnd(N, I, H), down=rnd(N, H, I),
+                experts=torch.zeros(T, K, dtype=torch.int64), cum=i32(N + 1), cum_ep=i32(T + 1), rows=i32(T * K))
+
+
+def _calls():
+    """entry point -> (call on a dict of tensors, the names of its differentiable inputs)"""
+    h = _n.host()
+    leaves = lambda t: [t["gate"], t["up"], t["down"]]
+    return {
+        "gate_logits": (lambda t: h.gate_logits(t["x"], t["weight"]), ("x", "weight")),
+        "route_softmax": (lambda t: h.route_softmax(t["x"], t["weight"], K, False, torch.bfloat16, False, False),
+                          ("x", "weight")),
+        "route_sigmoid": (lambda t: h.route_sigmoid(t["x"], t["weight"], t["bias"], 1, 1, K, True, 1.0),
+                          ("x", "weight", "bias")),
+        "routed_mlp": (lambda t: h.routed_mlp(t["x"], t["rw"], t["rows"], t["cum_ep"], t["rows"], t["rows"], t["cum"],
+                                              t["residual"], False, True, leaves(t), False, None),
+                       ("x", "rw", "residual", "gate", "up", "down")),
+        "moe_experts": (lambda t: h.moe_experts(t["x"], t["rw"], t["experts"], 0, N, N, False, t["residual"], True,
+                                                leaves(t), False, None),
+                        ("x", "rw", "residual", "gate", "up", "down")),
+        "merged_mlp": (lambda t: h.merged_mlp(t["x"], t["cum"], True, leaves(t), None, None, None),
+                       ("x", "gate", "up", "down")),
+        "combine": (lambda t: h.combine(t["y"], t["rw"], t["cum_ep"], t["rows"], t["rows"], t["rows"], t["residual"]),
+                    ("y", "rw", "residual")),
+    }
+
+
+CASES = [("gate_logits", 2), ("route_softmax", 2), ("route_sigmoid", 3), ("routed_mlp", 6), ("moe_experts", 6),
+         ("merged_mlp", 4), ("combine", 3)]
+
+
+@pytest.mark.parametrize("name,at", [(name, at) for name, n in CASES for at in range(n)])
+def test_forward_mode_is_refused(name, at):
+    """A tangent on any differentiable input raises what an autograd function without a jvp raises; it used to be
+    dropped without a word."""
+    call, inputs = _calls()[name]
+    assert len(inputs) == dict(CASES)[name]
+    t = _tensors()
+    with fwAD.dual_level():
+        t[inputs[at]] = fwAD.make_dual(t[inputs[at]], torch.ones_like(t[inputs[at]]))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            call(t)
+
+
+@pytest.mark.parametrize("name", [name for name, _ in CASES])
+@pytest.mark.parametrize("transform", [torch.vmap, torch.func.grad])
+def test_functorch_transforms_are_refused(name, transform):
+    call, inputs = _calls()[name]
+    t = _tensors()
+    first = torch.stack([t[inputs[0]]] * 2) if transform is torch.vmap else t[inputs[0]]
+
+    def f(v):
+        call({**t, inputs[0]: v})
+        return v.sum()
+    with pytest.raises(RuntimeError, match="torch.func transforms|jvp"):
+        transform(f)(first)
