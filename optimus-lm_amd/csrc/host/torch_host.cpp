@@ -684,11 +684,22 @@ struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits 
     }
 };
 
-void set_outputs(const std::shared_ptr<RouterNode> &node, Tensor *logits, Tensor *weights, Tensor *x) {
+// x as an output: a view of it made where autograd sees views, so that it shares x's version counter (an
+// in-place change of either between forward and backward is noticed by whatever saved the other).
+Tensor pass_through(const Tensor &x) {
+    at::NoGradGuard no_grad;
+    return x.view_as(x);
+}
+
+void set_outputs(const std::shared_ptr<RouterNode> &node, Tensor *logits, Tensor *weights, Tensor &x) {
     int at = 0;
     if (weights) { node->out_weights = at++; torch::autograd::set_history(*weights, node); }
     if (logits) { node->out_logits = at++; torch::autograd::set_history(*logits, node); }
-    if (x) { node->out_x = at++; torch::autograd::set_history(*x, node); }
+    // (an in-place change of a view that is one of several outputs would bypass the node: refused by autograd)
+    if (auto *view = torch::autograd::impl::get_view_autograd_meta(x); view && view->has_bw_view())
+        view->set_creation_meta(torch::autograd::CreationMeta::MULTI_OUTPUT_NODE);
+    node->out_x = at++;
+    torch::autograd::set_history(x, node);
 }
 
 std::shared_ptr<RouterNode> router_node(const Tensor &x, const Tensor &weight) {
@@ -701,15 +712,15 @@ std::shared_ptr<RouterNode> router_node(const Tensor &x, const Tensor &weight) {
 // (logits float32, x)
 std::tuple<Tensor, Tensor> gate_logits(const Tensor &x, const Tensor &weight) {
     refuse_transforms({x, weight});
-    Tensor logits, x_out;
+    Tensor logits;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         logits = gate_logits_forward(begin_call(), x, weight);
-        x_out = x.alias();
     }
+    Tensor x_out = pass_through(x);
     if (any_requires_grad({x, weight})) {
         auto node = router_node(x, weight);
-        set_outputs(node, &logits, nullptr, &x_out);
+        set_outputs(node, &logits, nullptr, x_out);
     }
     return {logits, x_out};
 }
@@ -732,7 +743,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
     // sooner.  us, one launch -> two, hidden 2048 and 64 experts: 64 tokens 22 -> 11, 512 22 -> 15, 2048 24 -> 17,
     // 4096 24 -> 20, 8192 27 -> 29; hidden 1024 and 32 experts: 512 10.6 -> 8.4, 4096 11.3 -> 12.0; hidden 512 even.
     if (one_pass && !bf16_logits && T > 0 && T <= 2048 && N <= 64 && H >= 1024 && H % 512 == 0) one_pass = false;
-    Tensor logits, weights, experts, x_out;
+    Tensor logits, weights, experts;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Call c = begin_call();
@@ -755,15 +766,15 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
             OM(c, om_router_gate_split_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, ptr(logits),
                dtype_code(logits), ptr(weights), dtype_code(weights), experts.data_ptr<int64_t>(), ptr(ws), ws.numel(), c.stream);
         }
-        x_out = x.alias();
     }
+    Tensor x_out = pass_through(x);
     if (any_requires_grad({x, weight})) {
         auto node = router_node(x, weight);
         // (a detached alias: saving an output itself would tie the node to itself)
         node->save(logits.detach());
         node->save(experts);
         node->renorm = renorm;
-        set_outputs(node, &logits, &weights, &x_out);
+        set_outputs(node, &logits, &weights, x_out);
     }
     return {weights, experts, logits, x_out};
 }
@@ -773,7 +784,7 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
                                                  int64_t topk_group, int64_t top_k, bool renorm, double scale) {
     refuse_transforms({x, weight, bias});
     const int64_t T = x.size(0), N = weight.size(0);
-    Tensor logits, weights, experts, x_out;
+    Tensor logits, weights, experts;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Call c = begin_call();
@@ -793,8 +804,8 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
             OM(c, om_router_gate_split_sigmoid_group_topk, ptr(x), ptr(weight), fp(bias), T, x.size(1), N, n_group, topk_group,
                top_k, renorm, scale, fpm(logits), experts.data_ptr<int64_t>(), fpm(weights), ptr(ws), ws.numel(), c.stream);
         }
-        x_out = x.alias();
     }
+    Tensor x_out = pass_through(x);
     if (any_requires_grad({x, weight})) {
         auto node = router_node(x, weight);
         node->save(logits);
@@ -802,7 +813,7 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
         node->renorm = renorm;
         node->sigmoid = true;
         node->scale = scale;
-        set_outputs(node, nullptr, &weights, &x_out);
+        set_outputs(node, nullptr, &weights, x_out);
     }
     return {experts, weights, x_out};
 }

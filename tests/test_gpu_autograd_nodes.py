@@ -1,0 +1,85 @@
+"""The blocks' autograd nodes (csrc/host/torch_host.cpp) against the contract of a torch.autograd.Function:
+in-place changes, saved-tensor hooks, hooks on parameters, repeated backward, threads and streams."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _olmoe(merged=True, fp32_logits=True, dtype=torch.bfloat16, H=256, I=256, N=8, K=2):
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    from optimus.models.common.moe import FastOlmoeParallelSparseMoeBlock
+    from optimus.models.olmoe.configuration_olmoe import OlmoeParallelConfig
+    cfg = OlmoeParallelConfig(hidden_size=H, intermediate_size=I, num_experts=N, num_experts_per_tok=K, norm_topk_prob=True,
+                              use_fast_moe=True, use_merged_mlp_in_fast_moe=merged)
+    cfg.router_logits_fp32 = fp32_logits
+    return FastOlmoeParallelSparseMoeBlock(cfg, ParallelDpPpEpTpMapper()), dtype
+
+
+def _dsv3():
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    from optimus.models.deepseek_v3.configuration_deepseek_v3 import DeepseekV3ParallelConfig
+    from optimus.models.deepseek_v3.modeling_deepseek_v3 import DeepseekV3ParallelMoE
+    cfg = DeepseekV3ParallelConfig(hidden_size=256, moe_intermediate_size=128, n_routed_experts=16,
+                                   num_experts_per_tok=4, n_group=4, topk_group=2, expert_parallelism=2)
+    return DeepseekV3ParallelMoE(cfg, ParallelDpPpEpTpMapper(expert_parallelism=2, rank=1)), torch.bfloat16
+
+
+BLOCKS = {"merged": _olmoe, "per_expert": lambda: _olmoe(merged=False), "model_dtype_logits": lambda: _olmoe(fp32_logits=False),
+          "float32": lambda: _olmoe(dtype=torch.float32), "dsv3": _dsv3}
+
+
+def _block(which, cuda, seed=3):
+    torch.manual_seed(seed)
+    blk, dtype = BLOCKS[which]()
+    for p in blk.parameters():
+        torch.nn.init.normal_(p, std=0.05)
+    return blk.to(cuda).to(dtype)
+
+
+def _data(blk, cuda, tokens=192, seed=11):
+    g = torch.Generator().manual_seed(seed)
+    p = next(blk.parameters())
+    return [torch.randn(2, tokens, 256, generator=g).to(p.dtype).to(cuda) for _ in range(2)]
+
+
+def _out(blk, x):
+    out = blk(x)
+    return out[0] if isinstance(out, tuple) else out
+
+
+def _flat_buffers(blk, cuda):
+    from optimus.optimizers import MixedPrecisionAdamW
+    opt = MixedPrecisionAdamW(blk.parameters(), blk, lr=1e-3, dtype=next(blk.parameters()).dtype, device=cuda)
+    opt.zero_grad()
+    return opt
+
+
+# ---- in-place changes of the hidden states -----------------------------------------------------------
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+@pytest.mark.parametrize("frozen", ["nothing", "gate"])
+def test_hidden_states_changed_before_backward_are_refused(cuda, which, frozen):
+    """The router hands the hidden states through to the experts; what the experts saved still shares the version
+    counter of the caller's tensor.  Nothing may have been added to a live gradient buffer when that is noticed."""
+    blk = _block(which, cuda)
+    if frozen == "gate":
+        blk.gate.requires_grad_(False)
+    opt = _flat_buffers(blk, cuda)
+    x, d = _data(blk, cuda)
+    out = _out(blk, x)
+    x.add_(1)
+    with pytest.raises(RuntimeError, match="modified (by an )?inplace"):
+        out.backward(d)
+    assert float(opt.flat_grad.float().abs().max()) == 0.0
+
+
+def test_router_pass_through_is_a_view_that_cannot_be_changed_in_place(cuda):
+    from optimus import _native as _n
+    x = torch.randn(64, 512, device=cuda).bfloat16().requires_grad_(True)
+    w = torch.randn(8, 512, device=cuda).bfloat16().requires_grad_(True)
+    outs = [_n.host().gate_logits(x, w)[1], _n.host().route_softmax(x, w, 2, True, torch.bfloat16, True, False)[3],
+            _n.host().route_sigmoid(x, w, torch.zeros(8, device=cuda), 1, 1, 2, True, 1.0)[2]]
+    for passed in outs:
+        assert passed.data_ptr() == x.data_ptr() and passed._version == x._version
+        with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
+            passed.add_(1)
