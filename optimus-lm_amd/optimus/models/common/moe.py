@@ -728,12 +728,12 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         """Permutation and RoutedMLPFunction in one call; None when the kernels do not take the operands."""
         merged = isinstance(self.experts, MergedMLP)
         if merged:
-            ex = self.experts._parameters
-            weights = [ex["gate_proj_merged_weight"], ex["up_proj_merged_weight"], ex["down_proj_merged_weight"]]
-            why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
+            # (as attributes: a weight may be parametrized, or a plain tensor that a wrapper has put there)
+            weights = [self.experts.gate_proj_merged_weight, self.experts.up_proj_merged_weight,
+                       self.experts.down_proj_merged_weight]
         else:
             weights = packed_expert_parameters(self.experts)
-            why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
+        why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
         if why is not None:
             if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
                 note_unfused_path("routing weight inside the expert MLP", why)

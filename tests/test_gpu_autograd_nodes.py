@@ -2,6 +2,7 @@
 in-place changes, saved-tensor hooks, hooks on parameters, repeated backward, threads and streams."""
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +84,36 @@ def test_router_pass_through_is_a_view_that_cannot_be_changed_in_place(cuda):
         assert passed.data_ptr() == x.data_ptr() and passed._version == x._version
         with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
             passed.add_(1)
+
+
+# ---- weights that are not plain parameters ------------------------------------------------------------
+class _Doubled(torch.nn.Module):
+    def forward(self, w):
+        return w * 2
+
+
+@pytest.mark.parametrize("how", ["parametrized", "plain_tensor"])
+def test_merged_weight_that_is_no_parameter(cuda, how):
+    """w * 2 in the place of every merged expert weight: the block of doubled weights, gradients reaching w."""
+    names = ("gate_proj_merged_weight", "up_proj_merged_weight", "down_proj_merged_weight")
+    blk, plain = _block("merged", cuda), _block("merged", cuda)
+    with torch.no_grad():
+        for n in names:
+            getattr(plain.experts, n).mul_(2)
+    leaves = []
+    for n in names:
+        w = getattr(blk.experts, n)
+        if how == "parametrized":
+            torch.nn.utils.parametrize.register_parametrization(blk.experts, n, _Doubled())
+            leaves.append(blk.experts.parametrizations[n].original)
+        else:
+            delattr(blk.experts, n)
+            setattr(blk.experts, n, w * 2)
+            leaves.append(w)
+    x, d = _data(blk, cuda)
+    a, b = _out(blk, x), _out(plain, x)
+    assert torch.equal(a, b)
+    a.backward(d)
+    b.backward(d)
+    for n, w in zip(names, leaves):
+        assert torch.equal(w.grad, getattr(plain.experts, n).grad * 2), n

@@ -1,6 +1,7 @@
 """The C++ host module's entry points where no kernel runs: what they refuse, and how they find the weights."""
 import pytest
 import torch
+import torch.nn.utils.parametrize
 import torch.autograd.forward_ad as fwAD
 
 from optimus import _native as _n
@@ -69,3 +70,16 @@ def test_functorch_transforms_are_refused(name, transform):
         return v.sum()
     with pytest.raises(RuntimeError, match="torch.func transforms|jvp"):
         transform(f)(first)
+
+
+def test_block_finds_a_parametrized_merged_weight():
+    """(on the CPU the fused path declines the operands, which it does after it has found the weights)"""
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    from optimus.models.common.moe import FastOlmoeParallelSparseMoeBlock
+    from optimus.models.olmoe.configuration_olmoe import OlmoeParallelConfig
+    cfg = OlmoeParallelConfig(hidden_size=H, intermediate_size=I, num_experts=N, num_experts_per_tok=K, use_fast_moe=True,
+                              use_merged_mlp_in_fast_moe=True)
+    blk = FastOlmoeParallelSparseMoeBlock(cfg, ParallelDpPpEpTpMapper())
+    torch.nn.utils.parametrize.register_parametrization(blk.experts, "gate_proj_merged_weight", torch.nn.Identity())
+    t = _tensors()
+    assert blk._fused_experts_fn(t["x"].float(), t["rw"], t["experts"], None) is None
