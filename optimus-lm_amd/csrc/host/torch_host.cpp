@@ -502,6 +502,26 @@ template <typename N> std::shared_ptr<N> make_node(const variable_list &inputs) 
     return node;
 }
 
+MlpWeights weights_of(at::ArrayRef<Tensor> leaves, bool merged, int64_t n_groups) {
+    if (!merged)
+        return {strided_view(&leaves[0], 3, n_groups), strided_view(&leaves[1], 3, n_groups),
+                strided_view(&leaves[2], 3, n_groups)};
+    if (leaves[0].dim() == 2) return {leaves[0].unsqueeze(0), leaves[1].unsqueeze(0), leaves[2].unsqueeze(0)};
+    return {leaves[0], leaves[1], leaves[2]};
+}
+
+// What a node keeps of one set of expert weights.  The weights themselves are three saved variables (the merged
+// tensors, or the views over the per-expert matrices), and the backward computes with what those unpack to.
+// The parameters are kept beside them only to find a live gradient buffer, so only where they can have one.
+struct ExpertWeights {
+    bool merged = false, single = false;   // single: one MLP's [out, in] matrices
+    int64_t G = 0;
+    size_t n_leaves = 0, at = 0;           // the caller's weight tensors; position of the saved variables
+    std::vector<Tensor> params;
+    // of the per-expert matrices: a view over them has a counter of its own
+    std::vector<std::pair<c10::VariableVersion, uint32_t>> versions;
+};
+
 // A node's backward: kernel errors become the package's own exception type in the thread that called
 // backward().
 struct HostNode : Node {
@@ -527,39 +547,58 @@ struct HostNode : Node {
     std::vector<Tensor> saved() {
         std::vector<Tensor> out;
         out.reserve(vars.size());
-        for (auto &v : vars) out.push_back(v.unpack(shared_from_this()));
+        for (auto &v : vars) {
+            out.push_back(v.unpack(shared_from_this()));
+            if (v.has_hooks() && out.back().defined() && !out.back().is_cuda())
+                throw NativeError("a saved-tensor hook unpacked a tensor that is not on the device it was packed from");
+        }
         return out;
+    }
+    ExpertWeights save_weights(at::ArrayRef<Tensor> leaves, bool merged, const MlpWeights &w) {
+        ExpertWeights e;
+        e.merged = merged;
+        e.single = merged && leaves[0].dim() == 2;
+        e.G = w.G();
+        e.n_leaves = leaves.size();
+        e.at = vars.size();
+        if (merged) for (const Tensor &t : leaves) save(t);
+        else for (const Tensor &t : {w.gate, w.up, w.down}) save(t);
+        for (const Tensor &t : leaves) {
+            e.params.push_back(t.is_leaf() && t.requires_grad() ? t : Tensor());
+            if (!merged) {
+                const auto &counter = torch::autograd::impl::version_counter(t);
+                e.versions.emplace_back(counter, counter.current_version());
+            }
+        }
+        return e;
+    }
+    MlpWeights weights(const ExpertWeights &e, const std::vector<Tensor> &kept) {
+        if (e.merged) return weights_of(at::ArrayRef<Tensor>(&kept[e.at], 3), true, e.G);
+        if (!vars[e.at].has_hooks())       // (what a hook packed is its own: autograd tracks no versions through it either)
+            for (const auto &[counter, saved_version] : e.versions)
+                TORCH_CHECK(counter.current_version() == saved_version,
+                            "one of the variables needed for gradient computation has been modified by an inplace "
+                            "operation: an expert's weight, at version ", counter.current_version(), ", expected ", saved_version);
+        return {kept[e.at], kept[e.at + 1], kept[e.at + 2]};
     }
     void release_variables() override {
         for (auto &v : vars) v.reset_data();
     }
 };
 
-MlpWeights weights_of(const std::vector<Tensor> &leaves, bool merged, size_t first, int64_t n_groups) {
-    MlpWeights w;
-    if (merged) {
-        w = {leaves[first], leaves[first + 1], leaves[first + 2]};
-        if (w.gate.dim() == 2) w = {w.gate.unsqueeze(0), w.up.unsqueeze(0), w.down.unsqueeze(0)};
-    } else {
-        w = {strided_view(&leaves[first], 3, n_groups), strided_view(&leaves[first + 1], 3, n_groups),
-             strided_view(&leaves[first + 2], 3, n_groups)};
-    }
-    return w;
-}
-Sinks sinks_of(const Call &c, const std::vector<Tensor> &leaves, bool merged, size_t first, int64_t n_groups,
-               const MlpWeights &w) {
-    const int64_t n = merged ? 1 : n_groups;
-    return {grad_sink(c, &leaves[first], 3, n, w.gate), grad_sink(c, &leaves[first + 1], 3, n, w.up),
-            grad_sink(c, &leaves[first + 2], 3, n, w.down)};
+Sinks sinks_of(const Call &c, const ExpertWeights &e, const MlpWeights &w) {
+    const int64_t n = e.merged ? 1 : e.G;
+    return {grad_sink(c, &e.params[0], 3, n, w.gate), grad_sink(c, &e.params[1], 3, n, w.up),
+            grad_sink(c, &e.params[2], 3, n, w.down)};
 }
 // gradients in the order of the leaves; undefined for a projection whose gradient went into its live buffer
-void push_grads(variable_list &out, const Sinks &k, bool merged, int64_t n_groups, bool single) {
+void push_grads(variable_list &out, const Sinks &k, const ExpertWeights &e) {
     const Tensor g[3] = {Sinks::fresh(k.gate), Sinks::fresh(k.up), Sinks::fresh(k.down)};
-    if (merged) {
-        for (const Tensor &t : g) out.push_back(single && t.defined() ? t.select(0, 0) : t);
+    if (e.merged) {
+        for (const Tensor &t : g) out.push_back(e.single && t.defined() ? t.select(0, 0) : t);
         return;
     }
-    for (int64_t n = 0; n < n_groups; n++)
+    for (int64_t n = 0; n < e.G; n++)
         for (const Tensor &t : g) out.push_back(t.defined() ? t.select(0, n) : t);
 }
 
@@ -824,18 +863,17 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
 // Inputs in order: hidden_states, routing_weights, residual, routed leaves, shared leaves.
 struct RoutedNode : HostNode {
     Index ix;                        // (without its owners)
-    std::vector<Tensor> leaves;      // the routed weights as the caller holds them, then the shared expert's three
-    MlpWeights w, ws;
-    bool merged = false, has_residual = false, has_shared = false;
-    int64_t G = 0;
+    ExpertWeights routed, shared;
+    bool has_residual = false, has_shared = false;
     std::string name() const override { return "OptimusRoutedExpertsBackward"; }
     variable_list run(variable_list &&grads) override {
-        const size_t n_in = 3 + leaves.size();
+        const size_t n_in = 3 + routed.n_leaves + shared.n_leaves;
         if (!grads[0].defined()) return variable_list(n_in);
         const Call c = begin_call();
         const Tensor dfinal = grads[0].contiguous();
-        // x, rw, row_weights, g, u, h [, shared g, u, h, cum], the index arrays' owners, the weights
+        // x, rw, row_weights, g, u, h [, shared g, u, h, cum], the index arrays' owners, the weights [, the shared ones]
         const std::vector<Tensor> kept = saved();
+        const MlpWeights w = weights(routed, kept), ws = has_shared ? weights(shared, kept) : MlpWeights();
         const MlpState s{Tensor(), kept[3], kept[4], kept[5]};
         size_t at = 6;
         MlpState ss;
@@ -844,21 +882,20 @@ struct RoutedNode : HostNode {
             at = 10;
         }
         Index index = ix;
-        index.owners.assign(kept.begin() + at, kept.begin() + kept.size() - leaves.size());
+        index.owners.assign(kept.begin() + at, kept.begin() + routed.at);
         index.resolve();
-        const size_t n_routed = leaves.size() - (has_shared ? 3 : 0);
         Tensor base;
         Sinks ks;
         if (has_shared) {   // first: its input gradient is the base of the routed experts' per-token sum
-            ks = sinks_of(c, leaves, true, n_routed, 1, ws);
+            ks = sinks_of(c, shared, ws);
             base = merged_backward(c, dfinal, kept[0], ws, iptr(ss.cum), ss, nullptr, ks);
         }
-        const Sinks k = sinks_of(c, leaves, merged, 0, G, w);
+        const Sinks k = sinks_of(c, routed, w);
         auto d = routed_backward(c, dfinal, kept[0], kept[1], index, w, s, kept[2], k, base);
         variable_list out = {d.first, d.second, has_residual ? grads[0] : Tensor()};
         out.reserve(n_in);
-        push_grads(out, k, merged, G, false);
-        if (has_shared) push_grads(out, ks, true, 1, true);
+        push_grads(out, k, routed);
+        if (has_shared) push_grads(out, ks, shared);
         return out;
     }
 };
@@ -868,19 +905,20 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
                       const std::function<void(Index &)> &after_shared = nullptr) {
     variable_list inputs = {x, rw, residual_in};
     inputs.insert(inputs.end(), leaves.begin(), leaves.end());
-    const size_t n_routed = leaves.size() - (has_shared ? 3 : 0);
-    const int64_t G = merged ? leaves[0].size(0) : static_cast<int64_t>(n_routed / 3);
+    const at::ArrayRef<Tensor> all(leaves);
+    const at::ArrayRef<Tensor> routed = all.slice(0, leaves.size() - (has_shared ? 3 : 0)), shared = all.slice(routed.size());
+    const int64_t G = merged ? leaves[0].size(0) : static_cast<int64_t>(routed.size() / 3);
     MlpWeights w, ws;
     MlpState s, ss;
     Tensor row_weights, final, xc, rwc;
     {
         at::AutoDispatchBelowADInplaceOrView below;
-        w = weights_of(leaves, merged, 0, G);
+        w = weights_of(routed, merged, G);
         xc = x.contiguous();
         rwc = rw.contiguous();
         Tensor residual = residual_in.defined() ? residual_in.contiguous() : Tensor();
         if (has_shared) {
-            ws = weights_of(leaves, true, n_routed, 1);
+            ws = weights_of(shared, true, 1);
             residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
         }
         if (after_shared) after_shared(ix);
@@ -888,23 +926,19 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
     }
     if (any_requires_grad(inputs)) {
         auto node = make_node<RoutedNode>(inputs);
-        node->vars.reserve(16 + leaves.size());
+        node->vars.reserve(21);
         node->save(xc.is_same(x) ? x : xc);
         node->save(rwc.is_same(rw) ? rw : rwc);
         for (const Tensor &t : {row_weights, s.g, s.u, s.h}) node->save(t);
         if (has_shared)
             for (const Tensor &t : {ss.g, ss.u, ss.h, one}) node->save(t);
         for (const Tensor &t : ix.owners) node->save(t);
-        for (const Tensor &t : leaves) node->save(t);
+        node->routed = node->save_weights(routed, merged, w);
+        if (has_shared) node->shared = node->save_weights(shared, true, ws);
         ix.owners.clear();
         node->ix = ix;
-        node->leaves = leaves;
-        node->w = w;
-        node->ws = ws;
-        node->merged = merged;
         node->has_residual = residual_in.defined();
         node->has_shared = has_shared;
-        node->G = G;
         torch::autograd::set_history(final, node);
     }
     return final;
@@ -993,19 +1027,17 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
 // The expert MLPs without routing weights (MergedMLPFunction, GroupMLPFunction and their gathered
 // forms).  Inputs in order: x, leaves.
 struct MergedNode : HostNode {
-    std::vector<Tensor> leaves;
-    MlpWeights w;
-    bool merged = false, single = false;
-    int64_t G = 0;
+    ExpertWeights experts;
     std::string name() const override { return "OptimusExpertMlpBackward"; }
     variable_list run(variable_list &&grads) override {
-        if (!grads[0].defined()) return variable_list(1 + leaves.size());
+        if (!grads[0].defined()) return variable_list(1 + experts.n_leaves);
         const Call c = begin_call();
         // x, cum, g, u, h, the gathered forms' index arrays (x_rows, cum_ep, out_rows), the weights
         const std::vector<Tensor> kept = saved();
         const Tensor &xs = kept[0];
         const MlpState s{kept[1], kept[2], kept[3], kept[4]};
-        const Sinks k = sinks_of(c, leaves, merged, 0, G, w);
+        const MlpWeights w = weights(experts, kept);
+        const Sinks k = sinks_of(c, experts, w);
         Tensor dx = merged_backward(c, grads[0], xs, w, iptr(s.cum), s, iptr(kept[5]), k);
         if (kept[5].defined()) {
             ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
@@ -1015,8 +1047,8 @@ struct MergedNode : HostNode {
             dx = sum;
         }
         variable_list out = {dx};
-        out.reserve(1 + leaves.size());
-        push_grads(out, k, merged, G, single);
+        out.reserve(1 + experts.n_leaves);
+        push_grads(out, k, experts);
         return out;
     }
 };
@@ -1039,21 +1071,16 @@ Tensor merged_mlp(const Tensor &x, Tensor cum, bool merged, const std::vector<Te
         for (const auto *t : {&x_rows, &cum_ep, &out_rows}) require_device(t->value_or(Tensor()));
         if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
         s.cum = cum.to(at::kInt).contiguous();
-        w = weights_of(leaves, merged, 0, G);
+        w = weights_of(leaves, merged, G);
         y = merged_forward(c, xc, w, iptr(s.cum), x_rows ? iptr(*x_rows) : nullptr, x_rows ? x_rows->size(0) : xc.size(0), s);
     }
     if (any_requires_grad(inputs)) {
         auto node = make_node<MergedNode>(inputs);
-        node->vars.reserve(8 + leaves.size());
+        node->vars.reserve(11);
         node->save(xc.is_same(x) ? x : xc);
         for (const Tensor &t : {s.cum, s.g, s.u, s.h}) node->save(t);
         for (const auto *t : {&x_rows, &cum_ep, &out_rows}) node->save(t->value_or(Tensor()));
-        for (const Tensor &t : leaves) node->save(t);
-        node->leaves = leaves;
-        node->w = w;
-        node->merged = merged;
-        node->single = merged && leaves[0].dim() == 2;
-        node->G = G;
+        node->experts = node->save_weights(leaves, merged, w);
         torch::autograd::set_history(y, node);
     }
     return y;

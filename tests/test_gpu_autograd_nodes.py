@@ -117,3 +117,62 @@ def test_merged_weight_that_is_no_parameter(cuda, how):
     b.backward(d)
     for n, w in zip(names, leaves):
         assert torch.equal(w.grad, getattr(plain.experts, n).grad * 2), n
+
+
+# ---- saved tensors ------------------------------------------------------------------------------------
+def _grads_of(blk, x):
+    return [x.grad] + [p.grad for p in blk.parameters()]
+
+
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+def test_backward_computes_with_what_saved_tensor_hooks_unpack(cuda, which):
+    """Everything saved is packed to the host; x, every weight and the routing change before the backward, which
+    must give the gradients of the values at the time of the forward."""
+    ref, blk = _block(which, cuda), _block(which, cuda)
+    x, d = _data(blk, cuda)
+    xr, xb = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    _out(ref, xr).backward(d)
+    packed = []
+
+    def pack(t):
+        packed.append(t.data_ptr())
+        return t.detach().to("cpu", copy=True)
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(cuda)):
+        out = _out(blk, xb)
+    weights = [p for n, p in blk.named_parameters()]
+    assert {w.data_ptr() for w in weights if w.dim() == 3} <= set(packed)
+    with torch.no_grad():
+        for w in weights + [xb]:
+            w.mul_(-3)
+    out.backward(d)
+    for a, b in zip(_grads_of(blk, xb), _grads_of(ref, xr)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which,name", [("merged", "experts.up_proj_merged_weight"), ("per_expert", "experts.5.down_proj.weight"),
+                                        ("dsv3", "experts.7.gate_proj.weight"), ("dsv3", "shared_experts.up_proj.weight"),
+                                        ("float32", "experts.down_proj_merged_weight")])
+def test_weight_changed_before_backward_is_refused(cuda, which, name):
+    blk = _block(which, cuda)
+    x, d = _data(blk, cuda)
+    out = _out(blk, x)
+    with torch.no_grad():
+        dict(blk.named_parameters())[name].add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(d)
+
+
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+def test_second_backward_is_refused_or_repeats(cuda, which):
+    blk = _block(which, cuda)
+    opt = _flat_buffers(blk, cuda)
+    x, d = _data(blk, cuda)
+    out = _out(blk, x)
+    out.backward(d, retain_graph=True)
+    once = opt.flat_grad.clone()
+    opt.zero_grad()
+    out.backward(d)
+    assert torch.equal(opt.flat_grad, once) and float(once.float().abs().max()) > 0
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward(d)
+    assert torch.equal(opt.flat_grad, once)
