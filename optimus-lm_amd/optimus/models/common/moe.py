@@ -757,7 +757,7 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
                               instead="running the projection and the routing as separate kernels (same fp32 logits)")
         # (the experts are fed from the router's pass-through of the hidden states, so that their input
         # gradient and the gate's are added in one kernel)
-        weight = self.gate.weight
+        weight = self.gate.weight.contiguous()
         if flat.is_cuda and flat.dtype == weight.dtype and flat.dtype in (torch.bfloat16, torch.float32) \
                 and self.gate.bias is None:
             bf16 = flat.dtype == torch.bfloat16

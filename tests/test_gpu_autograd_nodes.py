@@ -176,3 +176,17 @@ def test_second_backward_is_refused_or_repeats(cuda, which):
     with pytest.raises(RuntimeError, match="second time"):
         out.backward(d)
     assert torch.equal(opt.flat_grad, once)
+
+
+@pytest.mark.parametrize("which", ["merged", "model_dtype_logits", "float32", "dsv3"])
+def test_gate_weight_of_any_strides(cuda, which):
+    blk, ref = _block(which, cuda), _block(which, cuda)
+    gate = blk.gate
+    gate.weight = torch.nn.Parameter(gate.weight.detach().t().contiguous().t())
+    assert not gate.weight.is_contiguous()
+    x, d = _data(blk, cuda)
+    a, b = _out(blk, x), _out(ref, x)
+    assert torch.equal(a, b)
+    a.backward(d)
+    b.backward(d)
+    assert torch.equal(gate.weight.grad, ref.gate.weight.grad)
