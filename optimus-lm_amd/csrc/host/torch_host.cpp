@@ -178,6 +178,18 @@ Tensor strided_view(const Tensor *w, size_t step, int64_t G) {
 
 // ---- weight gradients that live in a flat buffer ----------------------------------------------------
 
+// Whether a hook on the parameter would have to see the incoming gradient.  A hook that was registered and
+// removed leaves its (empty) Python dictionary behind, and so does a deepcopy or a load: asked in Python then.
+bool has_grad_hooks(const Tensor &param) {
+    const size_t n = torch::autograd::impl::hooks(param).size();
+    const bool post = torch::autograd::impl::post_acc_grad_hooks(param) != nullptr;
+    if (n == 0 && !post) return false;
+    py::gil_scoped_acquire gil;
+    const py::object p = py::cast(param), hooks = p.attr("_backward_hooks"), posts = p.attr("_post_accumulate_grad_hooks");
+    return n > (hooks.is_none() ? 0u : 1u) || (post && posts.is_none()) ||   // (the rest: registered from C++)
+           (!hooks.is_none() && py::len(hooks) > 0) || (!posts.is_none() && py::len(posts) > 0);
+}
+
 // param.grad if the weight-gradient kernels may add into it in place: a leaf parameter whose gradient
 // already exists as a dense view of a larger buffer, same dtype and shape, with no hooks that would
 // have to see the incoming gradient; else undefined.
@@ -187,9 +199,7 @@ Tensor live_grad(const Tensor &param) {
     if (!grad.defined() || !grad.is_view() || grad.scalar_type() != param.scalar_type() ||
         grad.sizes() != param.sizes() || !grad.is_cuda() || !grad.is_contiguous() || grad.requires_grad())
         return Tensor();
-    if (!torch::autograd::impl::hooks(param).empty() || torch::autograd::impl::post_acc_grad_hooks(param) != nullptr)
-        return Tensor();
-    return grad;
+    return has_grad_hooks(param) ? Tensor() : grad;
 }
 
 // One projection's gradient: where the GEMM writes it.
@@ -1245,6 +1255,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("moe_experts", &moe_experts);
     m.def("merged_mlp", &merged_mlp);
     m.def("combine", &combine);
+    m.def("live_grad", &live_grad);
     m.def("expert_parameters", &expert_parameters);
     m.def("foreign_grads", &foreign_grads);
     m.def("constant_pitch", [](const std::vector<Tensor> &weights) {

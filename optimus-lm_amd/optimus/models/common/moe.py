@@ -301,15 +301,7 @@ def _live_grad(param):
     that would have to see the incoming gradient; else None."""
     if not accumulate_weight_grads_in_place or torch.is_grad_enabled():
         return None                     # (grad mode is on in backward only under create_graph)
-    if not (isinstance(param, torch.Tensor) and param.is_leaf and param.requires_grad):
-        return None
-    grad = param.grad
-    if grad is None or not grad._is_view() or grad.dtype != param.dtype or grad.shape != param.shape \
-            or not grad.is_cuda or not grad.is_contiguous() or grad.requires_grad:
-        return None
-    if param._backward_hooks or getattr(param, "_post_accumulate_grad_hooks", None):
-        return None
-    return grad
+    return _n.host().live_grad(param)
 
 
 # ----------------------------------------------------------------------------------------------

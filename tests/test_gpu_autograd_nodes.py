@@ -1,5 +1,7 @@
 """The blocks' autograd nodes (csrc/host/torch_host.cpp) against the contract of a torch.autograd.Function:
 in-place changes, saved-tensor hooks, hooks on parameters, repeated backward, threads and streams."""
+import collections
+
 import pytest
 import torch
 import torch.nn.utils.parametrize
@@ -190,3 +192,42 @@ def test_gate_weight_of_any_strides(cuda, which):
     a.backward(d)
     b.backward(d)
     assert torch.equal(gate.weight.grad, ref.gate.weight.grad)
+
+
+# ---- hooks on parameters ------------------------------------------------------------------------------
+@pytest.mark.parametrize("which,name", [("merged", "experts.gate_proj_merged_weight"), ("per_expert", "experts.3.up_proj.weight"),
+                                        ("dsv3", "shared_experts.down_proj.weight")])
+@pytest.mark.parametrize("kind", ["tensor", "post_accumulate"])
+def test_parameter_hooks_see_the_gradient_while_they_are_registered(cuda, which, name, kind):
+    """A live hook gets the gradient of this pass; once it is removed the GEMMs add into the buffer in place again,
+    as they do for a parameter whose hook dictionary a deepcopy left empty."""
+    from optimus import _native as _n
+    blk = _block(which, cuda)
+    opt = _flat_buffers(blk, cuda)
+    p = dict(blk.named_parameters())[name]
+    x, d = _data(blk, cuda)
+    _out(blk, x).backward(d)
+    want = p.grad.clone()
+    seen = []
+    if kind == "tensor":
+        handle = p.register_hook(lambda g: seen.append(g.clone()))
+    else:
+        handle = p.register_post_accumulate_grad_hook(lambda q: seen.append(q.grad.clone()))
+    opt.zero_grad()
+    assert _n.host().live_grad(p) is None
+    _out(blk, x).backward(d)
+    assert len(seen) == 1 and torch.equal(seen[0], want) and torch.equal(p.grad, want)
+    handle.remove()
+    copied = torch.nn.Parameter(p.detach().clone())
+    copied._backward_hooks = collections.OrderedDict()
+    copied.grad = torch.zeros(2 * p.numel(), device=cuda, dtype=p.dtype)[:p.numel()].view_as(p)
+    for q in (p, copied):
+        assert _n.host().live_grad(q).data_ptr() == q.grad.data_ptr()
+    _n.launch_log = []
+    try:
+        opt.zero_grad()
+        _out(blk, x).backward(d)
+    finally:
+        names, _n.launch_log = [e[0] for e in _n.launch_log], None
+    assert sum("wgrad" in n and n.startswith("om_grouped") and not n.endswith("accumulate") for n in names) == 0
+    assert len(seen) == 1 and torch.equal(p.grad, want)
