@@ -74,40 +74,59 @@ void check(int code, const char *what) {
         throw NativeError(std::string(what) + " failed with code " + std::to_string(code) + ": " + om_strerror(code));
 }
 
+// A Python object that may be dropped without the GIL, also while an exception passes.
+struct PyRef {
+    py::object object;
+    ~PyRef() {
+        if (!object) return;
+        py::gil_scoped_acquire gil;
+        object = py::object();
+    }
+};
+
 template <typename F> void launch(const Call &c, const char *name, F &&fn) {
     if (!c.log) {
         check(fn(), name);
         return;
     }
-    py::object start;
+    PyRef start;
     {
         py::gil_scoped_acquire gil;
-        start = py::module_::import("optimus._native").attr("timed_begin")(name);
+        start.object = py::module_::import("optimus._native").attr("timed_begin")(name);
     }
     const int code = fn();
     {
         py::gil_scoped_acquire gil;
-        py::module_::import("optimus._native").attr("timed_end")(name, start);
-        start = py::object();
+        py::module_::import("optimus._native").attr("timed_end")(name, start.object);
     }
     check(code, name);
 }
 #define OM(c, fn, ...) launch(c, #fn, [&] { return fn(__VA_ARGS__); })
 
-// optimus.profilers.record_pcl_function(name) around a scope, when a profiler is set
+// optimus.profilers.record_pcl_function(name) around a scope, when a profiler is set.  What the profiler raises
+// at the scope's end reaches the caller, as from a `with` block; while another exception passes it is reported
+// and dropped.
 struct ProfiledScope {
-    py::object context;
+    PyRef context;
+    int exceptions = std::uncaught_exceptions();
     ProfiledScope(const Call &c, const char *name) {
         if (!c.profile) return;
         py::gil_scoped_acquire gil;
-        context = py::module_::import("optimus.profilers").attr("record_pcl_function")(name);
-        context.attr("__enter__")();
+        py::object entered = py::module_::import("optimus.profilers").attr("record_pcl_function")(name);
+        entered.attr("__enter__")();
+        context.object = std::move(entered);
     }
-    ~ProfiledScope() {
-        if (!context) return;
+    ProfiledScope(const ProfiledScope &) = delete;
+    ~ProfiledScope() noexcept(false) {
+        if (!context.object) return;
         py::gil_scoped_acquire gil;
-        context.attr("__exit__")(py::none(), py::none(), py::none());
-        context = py::object();
+        const py::object entered = std::move(context.object);
+        try {
+            entered.attr("__exit__")(py::none(), py::none(), py::none());
+        } catch (py::error_already_set &e) {
+            if (std::uncaught_exceptions() == exceptions) throw;
+            e.discard_as_unraisable("the end of a profiled scope");
+        }
     }
 };
 
@@ -533,7 +552,7 @@ struct ExpertWeights {
 };
 
 // A node's backward: kernel errors become the package's own exception type in the thread that called
-// backward().
+// backward(), and Python's own (a profiler's) arrive there as they are.
 struct HostNode : Node {
     virtual variable_list run(variable_list &&grads) = 0;
     variable_list apply(variable_list &&grads) override {
@@ -545,10 +564,17 @@ struct HostNode : Node {
             PyObject *cls = module_attr("optimus._native", "NativeLibraryError");
             PyErr_SetString(cls, e.what());
             Py_DECREF(cls);
-            python_error err;
-            err.persist();
-            throw std::move(err);
+            throw_python_error();
+        } catch (py::error_already_set &e) {
+            py::gil_scoped_acquire gil;
+            e.restore();
+            throw_python_error();
         }
+    }
+    [[noreturn]] static void throw_python_error() {   // the one that is set; GIL held
+        python_error err;
+        err.persist();
+        throw std::move(err);
     }
     // Everything the backward needs is saved through SavedVariable, so that saved-tensor hooks (activation
     // checkpointing, offloading) see all of it and a second backward is refused.

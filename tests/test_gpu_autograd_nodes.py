@@ -231,3 +231,64 @@ def test_parameter_hooks_see_the_gradient_while_they_are_registered(cuda, which,
         names, _n.launch_log = [e[0] for e in _n.launch_log], None
     assert sum("wgrad" in n and n.startswith("om_grouped") and not n.endswith("accumulate") for n in names) == 0
     assert len(seen) == 1 and torch.equal(p.grad, want)
+
+
+# ---- Python code called from the host module ----------------------------------------------------------
+@pytest.mark.parametrize("which", ["merged", "float32", "dsv3"])
+@pytest.mark.parametrize("where", ["start", "stop"])
+@pytest.mark.parametrize("direction", ["forward", "backward"])
+def test_an_exception_of_the_profiler_reaches_the_caller(cuda, which, where, direction):
+    import optimus.globals
+    from optimus.profilers import PclProfiler
+
+    class Failing(PclProfiler):
+        armed = False
+
+        def start(self, name, key=""):
+            if self.armed and where == "start":
+                raise LookupError("profiler start")
+            super().start(name, key)
+
+        def stop(self, name):
+            super().stop(name)
+            if self.armed and where == "stop":
+                raise LookupError("profiler stop")
+
+    blk = _block(which, cuda)
+    x, d = _data(blk, cuda)
+    want = _out(blk, x)
+    prof = Failing()
+    optimus.globals.profiler = prof
+    try:
+        _out(blk, x).backward(d)                 # (registers the timers: an unknown one would fail in its turn)
+        prof.armed = direction == "forward"
+        if direction == "forward":
+            with pytest.raises(LookupError, match="profiler " + where):
+                _out(blk, x)
+        else:
+            out = _out(blk, x)
+            prof.armed = True
+            with pytest.raises(LookupError, match="profiler " + where):
+                out.backward(d)
+    finally:
+        optimus.globals.profiler = None
+    assert torch.equal(_out(blk, x), want)       # and the module goes on
+
+
+def test_an_exception_of_the_launch_log_reaches_the_caller(cuda, monkeypatch):
+    from optimus import _native as _n
+    blk = _block("merged", cuda)
+    x, d = _data(blk, cuda)
+    out = _out(blk, x)
+
+    def fail(*a):
+        raise LookupError("log")
+    for name in ("timed_begin", "timed_end"):
+        with monkeypatch.context() as m:
+            m.setattr(_n, name, fail)
+            m.setattr(_n, "launch_log", [])
+            with pytest.raises(LookupError):
+                _out(blk, x)
+            with pytest.raises(LookupError):
+                out.backward(d, retain_graph=True)
+    out.backward(d)
