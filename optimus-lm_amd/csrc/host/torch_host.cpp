@@ -1017,7 +1017,6 @@ struct CountReadback {
     }
     CountReadback(const CountReadback &) = delete;
     int64_t wait() {
-        py::gil_scoped_release nogil;
         if (hipEventSynchronize(copied) != hipSuccess) throw NativeError("reading the routed row count back failed");
         return value.data_ptr<int32_t>()[0];
     }
@@ -1256,31 +1255,35 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             Py_DECREF(cls);
         }
     });
+    // These only allocate and launch: other Python threads run meanwhile (the switches are read under the GIL).
+    const py::call_guard<py::gil_scoped_release> no_gil;
     m.def("build_token_permutation", [](const Tensor &experts, int64_t start, int64_t end) {
         at::AutoDispatchBelowADInplaceOrView below;
         auto r = sort_tensors(begin_call(), experts, start, end);
         return std::make_tuple(r[0], r[1], r[2], r[3], r[4]);
-    });
-    m.def("gate_logits", &gate_logits);
+    }, no_gil);
+    m.def("gate_logits", &gate_logits, no_gil);
     m.def("gate_weight_grad", [](const Tensor &x, const Tensor &w, const Tensor &dlogits) {
         return gate_weight_grad(begin_call(), x, w, dlogits);
-    });
+    }, no_gil);
     m.def("gate_input_grad", [](const Tensor &w, const Tensor &dlogits, const std::optional<Tensor> &other) {
         return gate_input_grad(begin_call(), w, dlogits, other.value_or(Tensor()));
-    });
+    }, no_gil);
     m.def("gate_backward", [](const Tensor &x, const Tensor &w, const Tensor &dlogits, bool need_x, bool need_w,
                               const std::optional<Tensor> &other) {
         return gate_backward(begin_call(), x, w, dlogits, need_x, need_w, other.value_or(Tensor()));
-    });
+    }, no_gil);
     m.def("route_softmax", [](const Tensor &x, const Tensor &w, int64_t top_k, bool renorm, py::object dtype, bool fused,
                               bool bf16_logits) {
-        return route_softmax(x, w, top_k, renorm, torch::python::detail::py_object_to_dtype(dtype), fused, bf16_logits);
+        const at::ScalarType dt = torch::python::detail::py_object_to_dtype(dtype);
+        py::gil_scoped_release nogil;
+        return route_softmax(x, w, top_k, renorm, dt, fused, bf16_logits);
     });
-    m.def("route_sigmoid", &route_sigmoid);
-    m.def("routed_mlp", &routed_mlp);
-    m.def("moe_experts", &moe_experts);
-    m.def("merged_mlp", &merged_mlp);
-    m.def("combine", &combine);
+    m.def("route_sigmoid", &route_sigmoid, no_gil);
+    m.def("routed_mlp", &routed_mlp, no_gil);
+    m.def("moe_experts", &moe_experts, no_gil);
+    m.def("merged_mlp", &merged_mlp, no_gil);
+    m.def("combine", &combine, no_gil);
     m.def("live_grad", &live_grad);
     m.def("expert_parameters", &expert_parameters);
     m.def("foreign_grads", &foreign_grads);

@@ -1,6 +1,10 @@
 """The blocks' autograd nodes (csrc/host/torch_host.cpp) against the contract of a torch.autograd.Function:
 in-place changes, saved-tensor hooks, hooks on parameters, repeated backward, threads and streams."""
 import collections
+import concurrent.futures
+import sys
+import threading
+import time
 
 import pytest
 import torch
@@ -292,3 +296,63 @@ def test_an_exception_of_the_launch_log_reaches_the_caller(cuda, monkeypatch):
             with pytest.raises(LookupError):
                 out.backward(d, retain_graph=True)
     out.backward(d)
+
+
+# ---- threads and streams ------------------------------------------------------------------------------
+def test_forward_calls_let_other_python_threads_run(cuda):
+    """With the interpreter's own switching out of the way, another thread only runs where a call lets the GIL go."""
+    from optimus import _native as _n
+    experts = torch.zeros(512, 8, dtype=torch.int64, device=cuda)
+    call = _n.host().build_token_permutation
+    call(experts, 0, 8)
+    ticks, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            time.sleep(0)                        # (lets the GIL go and asks for it again)
+            ticks[0] += 1
+    t = threading.Thread(target=other)
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(1000)
+    try:
+        t.start()
+        time.sleep(0.01)
+        before, calls = ticks[0], 0
+        while ticks[0] == before and calls < 3000:
+            call(experts, 0, 8)
+            calls += 1
+        assert ticks[0] > before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        t.join()
+
+
+@pytest.mark.parametrize("which", ["merged", "per_expert", "dsv3", "float32"])
+def test_threads_with_streams_of_their_own(cuda, which):
+    """Four threads, each a block, a stream and inputs of its own: the gradients of a single thread."""
+    def work(seed, stream):
+        with torch.cuda.stream(stream):
+            blk = _block_cache[seed]
+            res = []
+            for i in range(6):
+                x, d = _block_data[seed]
+                xi = x.clone().requires_grad_(True)
+                for p in blk.parameters():
+                    p.grad = None
+                out = _out(blk, xi)
+                out.backward(d)
+                res = [out.detach()] + _grads_of(blk, xi)
+            stream.synchronize()
+            return res
+    seeds = range(4)
+    _block_cache = {s: _block(which, cuda, seed=s) for s in seeds}
+    _block_data = {s: _data(_block_cache[s], cuda, seed=s) for s in seeds}
+    torch.cuda.synchronize()
+    want = [work(s, torch.cuda.current_stream()) for s in seeds]
+    streams = [torch.cuda.Stream() for _ in seeds]
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(work, seeds, streams))
+    for a, b in zip(got, want):
+        for u, v in zip(a, b):
+            assert torch.equal(u, v)
