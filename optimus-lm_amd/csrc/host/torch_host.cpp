@@ -555,7 +555,9 @@ struct ExpertWeights {
 // backward(), and Python's own (a profiler's) arrive there as they are.
 struct HostNode : Node {
     virtual variable_list run(variable_list &&grads) = 0;
+    // (one thread at a time unpacks and releases the saved variables, as in the nodes that PyTorch generates)
     variable_list apply(variable_list &&grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
         try {
             at::AutoDispatchBelowADInplaceOrView below;
             return run(std::move(grads));
@@ -618,6 +620,7 @@ struct HostNode : Node {
         return {kept[e.at], kept[e.at + 1], kept[e.at + 2]};
     }
     void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
         for (auto &v : vars) v.reset_data();
     }
 };

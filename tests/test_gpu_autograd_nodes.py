@@ -356,3 +356,28 @@ def test_threads_with_streams_of_their_own(cuda, which):
     for a, b in zip(got, want):
         for u, v in zip(a, b):
             assert torch.equal(u, v)
+
+
+@pytest.mark.parametrize("which", ["merged", "dsv3"])
+def test_two_threads_run_backward_through_one_graph(cuda, which):
+    """Eight passes from four threads through one retained graph, then a pass that releases it beside another: the
+    gradients of one pass each, and in the end the refusal of a second backward, nothing else."""
+    blk = _block(which, cuda)
+    x, d = _data(blk, cuda)
+    x.requires_grad_(True)
+    inputs = [x] + list(blk.parameters())
+    out = _out(blk, x)
+    want = torch.autograd.grad(out, inputs, d, retain_graph=True)
+    grad = lambda retain: torch.autograd.grad(out, inputs, d, retain_graph=retain)
+    torch.cuda.synchronize()
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        for got in pool.map(grad, [True] * 8):
+            for u, v in zip(got, want):
+                assert torch.equal(u, v)
+        ends = [pool.submit(grad, False) for _ in range(4)]
+    done = 0
+    for e in ends:
+        err = e.exception()
+        assert err is None or "second time" in str(err), err
+        done += err is None
+    assert done >= 1
