@@ -549,6 +549,16 @@ struct ExpertWeights {
     std::vector<Tensor> params;
     // of the per-expert matrices: a view over them has a counter of its own
     std::vector<std::pair<c10::VariableVersion, uint32_t>> versions;
+
+    static ExpertWeights of(at::ArrayRef<Tensor> leaves, bool merged) {
+        ExpertWeights e;
+        e.merged = merged;
+        e.single = merged && leaves[0].dim() == 2;
+        e.G = merged ? (e.single ? 1 : leaves[0].size(0)) : static_cast<int64_t>(leaves.size() / 3);
+        e.n_leaves = leaves.size();
+        for (const Tensor &t : leaves) e.params.push_back(t.is_leaf() && t.requires_grad() ? t : Tensor());
+        return e;
+    }
 };
 
 // A node's backward: kernel errors become the package's own exception type in the thread that called
@@ -593,20 +603,16 @@ struct HostNode : Node {
         return out;
     }
     ExpertWeights save_weights(at::ArrayRef<Tensor> leaves, bool merged, const MlpWeights &w) {
-        ExpertWeights e;
-        e.merged = merged;
-        e.single = merged && leaves[0].dim() == 2;
-        e.G = w.G();
-        e.n_leaves = leaves.size();
+        ExpertWeights e = ExpertWeights::of(leaves, merged);
         e.at = vars.size();
-        if (merged) for (const Tensor &t : leaves) save(t);
-        else for (const Tensor &t : {w.gate, w.up, w.down}) save(t);
+        if (merged) {
+            for (const Tensor &t : leaves) save(t);
+            return e;
+        }
+        for (const Tensor &t : {w.gate, w.up, w.down}) save(t);
         for (const Tensor &t : leaves) {
-            e.params.push_back(t.is_leaf() && t.requires_grad() ? t : Tensor());
-            if (!merged) {
-                const auto &counter = torch::autograd::impl::version_counter(t);
-                e.versions.emplace_back(counter, counter.current_version());
-            }
+            const auto &counter = torch::autograd::impl::version_counter(t);
+            e.versions.emplace_back(counter, counter.current_version());
         }
         return e;
     }
@@ -983,22 +989,47 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
     return final;
 }
 
-// RoutedMLPFunction / RoutedAndSharedMLPFunction over index arrays the caller has built
-Tensor routed_mlp(const Tensor &x, const Tensor &rw, const Tensor &in, const Tensor &cum_ep, const Tensor &out,
-                  const Tensor &sel, Tensor cum, const std::optional<Tensor> &residual, bool bound, bool merged,
-                  const std::vector<Tensor> &leaves, bool has_shared, const std::optional<Tensor> &one) {
-    refuse_transforms({x, rw, residual.value_or(Tensor())});
-    refuse_transforms(leaves);
-    const Call c = begin_call();
+// The kernels of RoutedMLPFunction / RoutedAndSharedMLPFunction, for the Python autograd functions: index arrays
+// that the caller has built, weights as [G, out, in] tensors or views.
+Index caller_index(const Tensor &x, const Tensor &in, const Tensor &cum_ep, const Tensor &out, const Tensor &sel, Tensor cum,
+                   bool bound) {
     for (const Tensor *t : {&in, &cum_ep, &out, &sel}) require_device(*t);
     if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
-    cum = cum.to(at::kInt).contiguous();
     Index ix;
-    ix.owners = {cum, cum_ep, in, out, sel};
+    ix.owners = {cum.to(at::kInt).contiguous(), cum_ep, in, out, sel};
     ix.resolve();
     ix.rows = in.size(0);
     ix.bound = bound;
-    return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, one.value_or(Tensor()));
+    return ix;
+}
+// -> final, cum, row_weights, g, u, h
+std::vector<Tensor> routed_mlp_forward(const Tensor &x, const Tensor &rw, const Tensor &in, const Tensor &cum_ep,
+                                       const Tensor &out, const Tensor &sel, const Tensor &cum,
+                                       const std::optional<Tensor> &residual, const std::vector<Tensor> &w) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Index ix = caller_index(x, in, cum_ep, out, sel, cum, false);
+    MlpState s;
+    Tensor row_weights;
+    const Tensor res = residual ? residual->contiguous() : Tensor();
+    Tensor final = routed_forward(begin_call(), x, rw, ix, weights_of(w, true, 0), res, s, row_weights);
+    return {final, ix.owners[0], row_weights, s.g, s.u, s.h};
+}
+// -> dx, d routing_weights, the gradients of the leaves (undefined: added into a live buffer)
+variable_list routed_mlp_backward(const Tensor &dfinal, const Tensor &x, const Tensor &rw, const Tensor &in,
+                                  const Tensor &cum_ep, const Tensor &out, const Tensor &sel, const Tensor &cum,
+                                  const Tensor &row_weights, const Tensor &g, const Tensor &u, const Tensor &h,
+                                  const std::vector<Tensor> &w, const std::vector<Tensor> &leaves, bool merged, bool bound,
+                                  const std::optional<Tensor> &base) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Call c = begin_call();
+    const ExpertWeights e = ExpertWeights::of(leaves, merged);
+    const MlpWeights mw = weights_of(w, true, 0);
+    const Sinks k = sinks_of(c, e, mw);
+    auto d = routed_backward(c, dfinal.contiguous(), x, rw, caller_index(x, in, cum_ep, out, sel, cum, bound), mw,
+                             {Tensor(), g, u, h}, row_weights, k, base.value_or(Tensor()));
+    variable_list grads = {d.first, d.second};
+    push_grads(grads, k, e);
+    return grads;
 }
 
 // Activations of the expert MLP sized by the upper bound T*K instead of the routed rows of an expert
@@ -1062,61 +1093,89 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
     return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, one.value_or(Tensor()));
 }
 
-// The expert MLPs without routing weights (MergedMLPFunction, GroupMLPFunction and their gathered
-// forms).  Inputs in order: x, leaves.
+// Gradients of the expert MLPs without routing weights: dx, then the leaves'.  `x_rows` (with the two arrays
+// of the per-token sum): the MLPs read x through it.
+variable_list merged_mlp_grads(const Call &c, const Tensor &dy, const Tensor &x, const MlpWeights &w, const MlpState &s,
+                               const Tensor &x_rows, const Tensor &cum_ep, const Tensor &out_rows, const ExpertWeights &e) {
+    const Sinks k = sinks_of(c, e, w);
+    Tensor dx = merged_backward(c, dy, x, w, iptr(s.cum), s, iptr(x_rows), k);
+    if (x_rows.defined()) {
+        ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
+        Tensor sum = make(x.sizes(), x);
+        OM(c, om_shuffle_sub_matrix_reduce, ptr(dx), iptr(cum_ep), iptr(out_rows), ptr(sum), x.size(0), x.size(1),
+           dtype_code(x), c.stream);
+        dx = sum;
+    }
+    variable_list grads = {dx};
+    grads.reserve(1 + e.n_leaves);
+    push_grads(grads, k, e);
+    return grads;
+}
+
+// Inputs in order: x, leaves.
 struct MergedNode : HostNode {
     ExpertWeights experts;
     std::string name() const override { return "OptimusExpertMlpBackward"; }
     variable_list run(variable_list &&grads) override {
         if (!grads[0].defined()) return variable_list(1 + experts.n_leaves);
-        const Call c = begin_call();
         // x, cum, g, u, h, the gathered forms' index arrays (x_rows, cum_ep, out_rows), the weights
         const std::vector<Tensor> kept = saved();
-        const Tensor &xs = kept[0];
-        const MlpState s{kept[1], kept[2], kept[3], kept[4]};
-        const MlpWeights w = weights(experts, kept);
-        const Sinks k = sinks_of(c, experts, w);
-        Tensor dx = merged_backward(c, grads[0], xs, w, iptr(s.cum), s, iptr(kept[5]), k);
-        if (kept[5].defined()) {
-            ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
-            Tensor sum = make(xs.sizes(), xs);
-            OM(c, om_shuffle_sub_matrix_reduce, ptr(dx), iptr(kept[6]), iptr(kept[7]), ptr(sum), xs.size(0), xs.size(1),
-               dtype_code(xs), c.stream);
-            dx = sum;
-        }
-        variable_list out = {dx};
-        out.reserve(1 + experts.n_leaves);
-        push_grads(out, k, experts);
-        return out;
+        return merged_mlp_grads(begin_call(), grads[0], kept[0], weights(experts, kept), {kept[1], kept[2], kept[3], kept[4]},
+                                kept[5], kept[6], kept[7], experts);
     }
 };
 
-Tensor merged_mlp(const Tensor &x, Tensor cum, bool merged, const std::vector<Tensor> &leaves,
+// (y, cum, g, u, h) of the expert MLPs; `x_rows`: they read x through it
+std::vector<Tensor> merged_mlp_state(const Tensor &x, Tensor cum, const MlpWeights &w, const Tensor &x_rows) {
+    const Call c = begin_call();
+    MlpState s;
+    require_device(x);
+    require_device(x_rows);
+    if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
+    s.cum = cum.to(at::kInt).contiguous();
+    Tensor y = merged_forward(c, x, w, iptr(s.cum), iptr(x_rows), x_rows.defined() ? x_rows.size(0) : x.size(0), s);
+    return {y, s.cum, s.g, s.u, s.h};
+}
+
+// The kernels of MergedMLPFunction, GroupMLPFunction and their gathered forms, for the Python autograd functions.
+std::vector<Tensor> merged_mlp_forward(const Tensor &x, const Tensor &cum, const std::vector<Tensor> &w,
+                                       const std::optional<Tensor> &x_rows) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return merged_mlp_state(x, cum, weights_of(w, true, 0), x_rows.value_or(Tensor()));
+}
+variable_list merged_mlp_backward(const Tensor &dy, const Tensor &x, const Tensor &cum, const Tensor &g, const Tensor &u,
+                                  const Tensor &h, const std::vector<Tensor> &w, const std::vector<Tensor> &leaves, bool merged,
+                                  const std::optional<Tensor> &x_rows, const std::optional<Tensor> &cum_ep,
+                                  const std::optional<Tensor> &out_rows) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    for (const auto *t : {&cum_ep, &out_rows}) require_device(t->value_or(Tensor()));
+    return merged_mlp_grads(begin_call(), dy, x, weights_of(w, true, 0), {cum, g, u, h}, x_rows.value_or(Tensor()),
+                            cum_ep.value_or(Tensor()), out_rows.value_or(Tensor()), ExpertWeights::of(leaves, merged));
+}
+
+// The expert MLPs without routing weights as one autograd node.
+Tensor merged_mlp(const Tensor &x, const Tensor &cum, bool merged, const std::vector<Tensor> &leaves,
                   const std::optional<Tensor> &x_rows, const std::optional<Tensor> &cum_ep,
                   const std::optional<Tensor> &out_rows) {
     variable_list inputs = {x};
     inputs.insert(inputs.end(), leaves.begin(), leaves.end());
     refuse_transforms(inputs);
-    const int64_t G = merged ? 1 : static_cast<int64_t>(leaves.size() / 3);
     MlpWeights w;
-    MlpState s;
-    Tensor y, xc = x;
+    std::vector<Tensor> state;
+    Tensor xc = x;
     {
         at::AutoDispatchBelowADInplaceOrView below;
-        const Call c = begin_call();
         if (x_rows) xc = x.contiguous();
-        require_device(xc);
-        for (const auto *t : {&x_rows, &cum_ep, &out_rows}) require_device(t->value_or(Tensor()));
-        if (!cum.is_cuda()) cum = cum.to(x.device(), /*non_blocking=*/true);
-        s.cum = cum.to(at::kInt).contiguous();
-        w = weights_of(leaves, merged, G);
-        y = merged_forward(c, xc, w, iptr(s.cum), x_rows ? iptr(*x_rows) : nullptr, x_rows ? x_rows->size(0) : xc.size(0), s);
+        for (const auto *t : {&cum_ep, &out_rows}) require_device(t->value_or(Tensor()));
+        w = weights_of(leaves, merged, static_cast<int64_t>(leaves.size() / 3));
+        state = merged_mlp_state(xc, cum, w, x_rows.value_or(Tensor()));
     }
+    Tensor y = state[0];
     if (any_requires_grad(inputs)) {
         auto node = make_node<MergedNode>(inputs);
         node->vars.reserve(11);
         node->save(xc.is_same(x) ? x : xc);
-        for (const Tensor &t : {s.cum, s.g, s.u, s.h}) node->save(t);
+        for (size_t i = 1; i < state.size(); i++) node->save(state[i]);
         for (const auto *t : {&x_rows, &cum_ep, &out_rows}) node->save(t->value_or(Tensor()));
         node->experts = node->save_weights(leaves, merged, w);
         torch::autograd::set_history(y, node);
@@ -1125,23 +1184,29 @@ Tensor merged_mlp(const Tensor &x, Tensor cum, bool merged, const std::vector<Te
 }
 
 // K6 (GroupGemmOutputReduction[Residual]Function): final[t] = (residual[t] +) sum_k w[t,k] y[pos(t,k)].
+std::pair<Tensor, Tensor> combine_backward(const Tensor &dfinal_in, const Tensor &y, const Tensor &rw, const Tensor &sel,
+                                           const Tensor &in, const Tensor &out) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Call c = begin_call();
+    const Tensor dfinal = dfinal_in.contiguous();
+    Tensor dy = make(y.sizes(), y);
+    // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window
+    // stay zero (the reference pre-zeroes the whole tensor, moe.py:336)
+    Tensor drw = out.size(0) == rw.numel() ? make(rw.sizes(), rw) : at::zeros(rw.sizes(), rw.options());
+    ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_bwd");
+    OM(c, om_reduce_ggemm_output_backward, ptr(dfinal), ptr(y), ptr(rw), iptr(sel), iptr(in), iptr(out), ptr(dy), ptr(drw),
+       out.size(0), rw.size(1), dfinal.size(1), dtype_code(y), dtype_code(rw), c.stream);
+    return {dy, drw};
+}
+
 struct CombineNode : HostNode {      // saves y, rw, sel, in, out
     bool has_residual = false;
     std::string name() const override { return "OptimusCombineBackward"; }
     variable_list run(variable_list &&grads) override {
         if (!grads[0].defined()) return variable_list(3);
-        const Call c = begin_call();
         const std::vector<Tensor> kept = saved();
-        const Tensor dfinal = grads[0].contiguous();
-        const Tensor &ys = kept[0], &rws = kept[1], &sel = kept[2], &in = kept[3], &out = kept[4];
-        Tensor dy = make(ys.sizes(), ys);
-        // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window
-        // stay zero (the reference pre-zeroes the whole tensor, moe.py:336)
-        Tensor drw = out.size(0) == rws.numel() ? make(rws.sizes(), rws) : at::zeros(rws.sizes(), rws.options());
-        ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_bwd");
-        OM(c, om_reduce_ggemm_output_backward, ptr(dfinal), ptr(ys), ptr(rws), iptr(sel), iptr(in), iptr(out), ptr(dy),
-           ptr(drw), out.size(0), rws.size(1), dfinal.size(1), dtype_code(ys), dtype_code(rws), c.stream);
-        return {dy, drw, has_residual ? grads[0] : Tensor()};
+        auto d = combine_backward(grads[0], kept[0], kept[1], kept[2], kept[3], kept[4]);
+        return {d.first, d.second, has_residual ? grads[0] : Tensor()};
     }
 };
 
@@ -1283,10 +1348,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         return route_softmax(x, w, top_k, renorm, dt, fused, bf16_logits);
     });
     m.def("route_sigmoid", &route_sigmoid, no_gil);
-    m.def("routed_mlp", &routed_mlp, no_gil);
+    m.def("routed_mlp_forward", &routed_mlp_forward, no_gil);
+    m.def("routed_mlp_backward", &routed_mlp_backward, no_gil);
     m.def("moe_experts", &moe_experts, no_gil);
     m.def("merged_mlp", &merged_mlp, no_gil);
+    m.def("merged_mlp_forward", &merged_mlp_forward, no_gil);
+    m.def("merged_mlp_backward", &merged_mlp_backward, no_gil);
     m.def("combine", &combine, no_gil);
+    m.def("combine_backward", &combine_backward, no_gil);
+    m.def("expert_view", [](const std::vector<Tensor> &weights) {
+        if (weights.empty()) throw NativeError("no expert weights");
+        at::NoGradGuard no_grad;
+        return strided_view(weights.data(), 1, static_cast<int64_t>(weights.size()));
+    });
     m.def("live_grad", &live_grad);
     m.def("expert_parameters", &expert_parameters);
     m.def("foreign_grads", &foreign_grads);

@@ -203,28 +203,46 @@ def gate_logits_with_passthrough(x, gate):
     return gate(x), x
 
 
-class GateLogitsFunction:
-    """apply(x, weight) -> (fp32 logits of a bf16 gate, x); see fp32_logits_with_passthrough."""
+# The autograd functions below wrap the same kernels, in the same order, as the C++ nodes that the blocks use
+# (csrc/host/torch_host.cpp: gate_logits, route_softmax, merged_mlp, moe_experts, combine): for callers that apply
+# or extend the reference's functions one by one.
+class GateLogitsFunction(torch.autograd.Function):
+    """(fp32 logits, x) of the gate projection.  The second output is the input itself; a caller that
+    feeds the rest of the layer from it makes that part's input gradient arrive here, where the gate's
+    own is added to it inside the input-gradient kernel instead of by a separate accumulation pass."""
 
     @staticmethod
-    def apply(x, weight):
+    def forward(ctx, x, weight):
+        ctx.save_for_backward(x, weight)
+        ctx.set_materialize_grads(False)
         return _n.host().gate_logits(x, weight)
 
+    @staticmethod
+    def backward(ctx, dlogits, x_grad):
+        if dlogits is None:
+            return x_grad, None
+        return _n.host().gate_backward(*ctx.saved_tensors, dlogits, *ctx.needs_input_grad, x_grad)
 
-class GateLogitsF32Function:
-    """apply(x, weight) -> logits = x @ weight.T for a float32 gate (om_router_gate_logits_f32, with both
-    backward products on the float32 gate kernels)."""
+
+class GateLogitsF32Function(torch.autograd.Function):
+    """logits = x @ weight.T for a float32 gate (om_router_gate_logits_f32, with both backward products
+    on the float32 gate kernels)."""
 
     @staticmethod
-    def apply(x, weight):
+    def forward(ctx, x, weight):
+        ctx.save_for_backward(x, weight)
         return _n.host().gate_logits(x, weight)[0]
 
+    @staticmethod
+    def backward(ctx, dlogits):
+        return _n.host().gate_backward(*ctx.saved_tensors, dlogits, *ctx.needs_input_grad, None)
 
-class GateSoftmaxTopkFunction:
-    """The OLMoE router in one launch (om_router_gate_softmax_topk): gate projection with fp32
-    logits, softmax, top-K, optional renormalisation.  apply(x, weight, top_k, norm_topk_prob, out_dtype)
-    returns (routing_weights, selected_experts, router_logits fp32, hidden_states); reference
-    moe.py:456 and :467-471.
+
+class GateSoftmaxTopkFunction(torch.autograd.Function):
+    """The OLMoE router with the gate projection: fp32 logits, softmax, top-K, optional renormalisation,
+    in one launch (om_router_gate_softmax_topk) or, up to 2048 tokens, in two with the same bits
+    (om_router_gate_split_softmax_topk).  Returns (routing_weights, selected_experts, router_logits fp32,
+    hidden_states); reference moe.py:456 and :467-471.
 
     The fourth output is the input itself.  A caller that feeds the experts from it (instead of from
     the tensor it passed in) makes the experts' input gradient arrive here, where the gate's own
@@ -232,8 +250,41 @@ class GateSoftmaxTopkFunction:
     matmul output plus autograd's accumulation kernel."""
 
     @staticmethod
-    def apply(x, weight, top_k, norm_topk_prob, out_dtype):
-        return _n.host().route_softmax(x, weight, top_k, bool(norm_topk_prob), out_dtype, True, False)
+    def forward(ctx, x, weight, top_k, norm_topk_prob, out_dtype):
+        weights, experts, logits, passed = _n.host().route_softmax(x, weight, top_k, bool(norm_topk_prob), out_dtype,
+                                                                   True, False)
+        ctx.save_for_backward(x, weight, logits, experts)
+        ctx.norm_topk_prob = bool(norm_topk_prob)
+        ctx.mark_non_differentiable(experts)
+        # an output nobody differentiates (the logits without an auxiliary loss) arrives as None in
+        # backward instead of a tensor of zeros that would have to be filled and added
+        ctx.set_materialize_grads(False)
+        return weights, experts, logits, passed
+
+    @staticmethod
+    def backward(ctx, weights_grad, _experts_grad, logits_grad, x_grad):
+        x, weight, logits, experts = ctx.saved_tensors
+        if weights_grad is None and logits_grad is None:
+            return x_grad, None, None, None, None
+        dlogits = logits_grad
+        if weights_grad is not None:
+            dlogits = _softmax_topk_backward(logits, experts, weights_grad, ctx.norm_topk_prob)
+            if logits_grad is not None:
+                dlogits = dlogits + logits_grad
+        dx, dw = _n.host().gate_backward(x, weight, dlogits, *ctx.needs_input_grad[:2], x_grad)
+        return dx, dw, None, None, None
+
+
+def _softmax_topk_backward(router_logits, experts, weights_grad, norm_topk_prob):
+    """Gradient of the logits of a softmax top-K router."""
+    T, N = router_logits.shape
+    weights_grad = weights_grad.contiguous()
+    dlogits = torch.empty_like(router_logits)
+    _n.check(_n.lib().om_route_softmax_topk_bwd(
+        _n.ptr(router_logits), _n.dtype_code(router_logits), _n.ptr(experts), _n.ptr(weights_grad),
+        _n.dtype_code(weights_grad), T, N, experts.shape[1], int(norm_topk_prob), _n.ptr(dlogits),
+        _n.stream()), "om_route_softmax_topk_bwd")
+    return dlogits
 
 
 class SoftmaxTopkRouterFunction(torch.autograd.Function):
@@ -258,15 +309,7 @@ class SoftmaxTopkRouterFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, weights_grad, _experts_grad):
-        router_logits, experts = ctx.saved_tensors
-        T, N = router_logits.shape
-        K = experts.shape[1]
-        weights_grad = weights_grad.contiguous()
-        dlogits = torch.empty_like(router_logits)
-        _n.check(_n.lib().om_route_softmax_topk_bwd(
-            _n.ptr(router_logits), _n.dtype_code(router_logits), _n.ptr(experts), _n.ptr(weights_grad),
-            _n.dtype_code(weights_grad), T, N, K, int(ctx.norm_topk_prob), _n.ptr(dlogits),
-            _n.stream()), "om_route_softmax_topk_bwd")
+        dlogits = _softmax_topk_backward(*ctx.saved_tensors, weights_grad, ctx.norm_topk_prob)
         return dlogits, None, None, None
 
 
@@ -346,23 +389,37 @@ class GroupedGemmFunction(torch.autograd.Function):
         return input_grad, (None if acc else weight_grad), None, None, None
 
 
-class MergedMLPFunction:
+def _expert_views(weight_tuple):
+    """[gate, up, down] as [G, out, in] views over the per-expert matrices of a (gate_0, up_0, down_0,
+    gate_1, ...) tuple, which must lie at a constant pitch in one buffer."""
+    return [_n.host().expert_view(list(weight_tuple[j::3])) for j in range(3)]
+
+
+class MergedMLPFunction(torch.autograd.Function):
     """y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment, with the fused kernels:
     gate+up+SwiGLU in one launch forward; backward = down dgrad fused with the SwiGLU backward,
-    one dual-operand dgrad for dx, and three weight-gradient GEMMs.
+    one dual-operand dgrad for dx, and three weight-gradient GEMMs (float32: two launches for them).
 
     Same mathematics as the three GroupedGemmFunction calls and two elementwise ops of the
-    reference's MergedMLP.forward (moe.py:396-405) under autograd; g and u are kept in bf16 for
-    the backward like the reference keeps output_gproj / output_uproj.  float32 modules run the
-    reference's own sequence on the plain fp32 kernels."""
+    reference's MergedMLP.forward (moe.py:396-405) under autograd; g and u are kept in the module's
+    dtype for the backward like the reference keeps output_gproj / output_uproj."""
 
     @staticmethod
-    def apply(x, w_gate, w_up, w_down, cum_token_counts):
+    def forward(ctx, x, w_gate, w_up, w_down, cum_token_counts):
         # a single MLP may hand its three [out, in] weights over as they are
-        return _n.host().merged_mlp(x, cum_token_counts, True, [w_gate, w_up, w_down], None, None, None)
+        ctx.leaves = [w_gate, w_up, w_down]
+        y, *state = _n.host().merged_mlp_forward(x, cum_token_counts, ctx.leaves, None)
+        ctx.save_for_backward(x, *state, *ctx.leaves)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        *saved, w_gate, w_up, w_down = ctx.saved_tensors
+        return (*_n.host().merged_mlp_backward(dy, *saved, [w_gate, w_up, w_down], ctx.leaves, True, None, None, None),
+                None)
 
 
-class GatheredMergedMLPFunction:
+class GatheredMergedMLPFunction(torch.autograd.Function):
     """PrepareInputForGroupGemmFunction followed by MergedMLPFunction (reference moe.py:217-282 and
     :396-405) without the gathered copy of the activations: the gate/up forward GEMM and the two
     gate/up weight-gradient GEMMs read hidden_states through input_indices.  Bit-identical to the
@@ -370,32 +427,61 @@ class GatheredMergedMLPFunction:
     gradients (shuffle_sub_matrix_reduce)."""
 
     @staticmethod
-    def apply(hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate, w_up, w_down,
-              cum_token_counts):
-        return _n.host().merged_mlp(hidden_states, cum_token_counts, True, [w_gate, w_up, w_down],
-                                    input_indices, cum_expert_counts_ep, output_indices)
+    def forward(ctx, hidden_states, input_indices, cum_expert_counts_ep, output_indices, w_gate, w_up, w_down,
+                cum_token_counts):
+        hidden_states = hidden_states.contiguous()
+        ctx.leaves = [w_gate, w_up, w_down]
+        y, *state = _n.host().merged_mlp_forward(hidden_states, cum_token_counts, ctx.leaves, input_indices)
+        ctx.save_for_backward(input_indices, cum_expert_counts_ep, output_indices, hidden_states, *state, *ctx.leaves)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        *saved, w_gate, w_up, w_down = ctx.saved_tensors
+        dx, *dws = _n.host().merged_mlp_backward(dy, *saved[3:], [w_gate, w_up, w_down], ctx.leaves, True, *saved[:3])
+        return (dx, None, None, None, *dws, None)
 
 
-class GroupMLPFunction:
+class GroupMLPFunction(torch.autograd.Function):
     """Un-merged layout of the reference (moe.py:43-161): weights arrive as 3*N separate
     [out, in] tensors (gate_0, up_0, down_0, gate_1, ...).  They must sit at one constant pitch
     inside a single buffer (true for parameters re-pointed into MixedPrecisionAdamW.flat_param and
     after pack_expert_weights); the same fused kernels then run on strided views, no copies."""
 
     @staticmethod
-    def apply(input, cum_token_counts, use_triton_path, *weight_tuple):
-        return _n.host().merged_mlp(input, cum_token_counts, False, list(weight_tuple), None, None, None)
+    def forward(ctx, input, cum_token_counts, use_triton_path, *weight_tuple):
+        ctx.leaves = list(weight_tuple)
+        views = _expert_views(weight_tuple)
+        y, *state = _n.host().merged_mlp_forward(input, cum_token_counts, views, None)
+        ctx.save_for_backward(input, *state, *views)
+        return y
+
+    @staticmethod
+    def backward(ctx, output_grad):
+        *saved, wg, wu, wd = ctx.saved_tensors
+        dx, *dws = _n.host().merged_mlp_backward(output_grad, *saved, [wg, wu, wd], ctx.leaves, False, None, None, None)
+        return (dx, None, None, *dws)
 
 
-class GatheredGroupMLPFunction:
+class GatheredGroupMLPFunction(torch.autograd.Function):
     """GroupMLPFunction on hidden_states[input_indices] without the gathered copy (see
     GatheredMergedMLPFunction); weights as in GroupMLPFunction."""
 
     @staticmethod
-    def apply(hidden_states, input_indices, cum_expert_counts_ep, output_indices, cum_token_counts,
-              *weight_tuple):
-        return _n.host().merged_mlp(hidden_states, cum_token_counts, False, list(weight_tuple),
-                                    input_indices, cum_expert_counts_ep, output_indices)
+    def forward(ctx, hidden_states, input_indices, cum_expert_counts_ep, output_indices, cum_token_counts,
+                *weight_tuple):
+        hidden_states = hidden_states.contiguous()
+        ctx.leaves = list(weight_tuple)
+        views = _expert_views(weight_tuple)
+        y, *state = _n.host().merged_mlp_forward(hidden_states, cum_token_counts, views, input_indices)
+        ctx.save_for_backward(input_indices, cum_expert_counts_ep, output_indices, hidden_states, *state, *views)
+        return y
+
+    @staticmethod
+    def backward(ctx, output_grad):
+        *saved, wg, wu, wd = ctx.saved_tensors
+        dx, *dws = _n.host().merged_mlp_backward(output_grad, *saved[3:], [wg, wu, wd], ctx.leaves, False, *saved[:3])
+        return (dx, None, None, None, None, *dws)
 
 
 def routed_mlp_unfit_reason(hidden_states, routing_weights, w_gate, w_down):
@@ -419,7 +505,7 @@ def routed_mlp_kernel_fits(hidden_states, routing_weights, w_gate, w_down):
     return routed_mlp_unfit_reason(hidden_states, routing_weights, w_gate, w_down) is None
 
 
-class RoutedMLPFunction:
+class RoutedMLPFunction(torch.autograd.Function):
     """The expert half of the block in one function: PrepareInputForGroupGemmFunction, the SwiGLU
     MLP of every expert and GroupGemmOutputReductionFunction (reference moe.py:217-405), with both
     row permutations and the routing weight folded into the GEMMs:
@@ -439,17 +525,31 @@ class RoutedMLPFunction:
     3*G per-expert matrices of GroupMLPFunction."""
 
     @staticmethod
-    def apply(hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-              selected_experts_indices, cum_token_counts, residual, n_merged, *weights):
+    def forward(ctx, hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
+                selected_experts_indices, cum_token_counts, residual, n_merged, *weights):
         # n_merged: True = merged weights; False = per-expert weights; "bound" forms of both say that
         # the index arrays are sized by an upper bound of the routed rows (expert_computation)
-        return _n.host().routed_mlp(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                                    output_indices, selected_experts_indices, cum_token_counts, residual,
-                                    n_merged in ("merged_bound", "per_expert_bound"),
-                                    n_merged in (True, "merged_bound"), list(weights), False, None)
+        ctx.rows_is_bound = n_merged in ("merged_bound", "per_expert_bound")
+        ctx.n_merged = n_merged in (True, "merged_bound")
+        ctx.has_residual = residual is not None
+        ctx.leaves = list(weights)
+        views = ctx.leaves if ctx.n_merged else _expert_views(weights)
+        index = (input_indices, cum_expert_counts_ep, output_indices, selected_experts_indices)
+        hidden_states, routing_weights = hidden_states.contiguous(), routing_weights.contiguous()
+        final, *state = _n.host().routed_mlp_forward(hidden_states, routing_weights, *index, cum_token_counts, residual,
+                                                     views)
+        ctx.save_for_backward(hidden_states, routing_weights, *index, *state, *views)
+        return final
+
+    @staticmethod
+    def backward(ctx, dfinal):
+        *saved, wg, wu, wd = ctx.saved_tensors
+        dx, drw, *dws = _n.host().routed_mlp_backward(dfinal, *saved, [wg, wu, wd], ctx.leaves, ctx.n_merged,
+                                                      ctx.rows_is_bound, None)
+        return (dx, drw, None, None, None, None, None, dfinal if ctx.has_residual else None, None, *dws)
 
 
-class RoutedAndSharedMLPFunction:
+class RoutedAndSharedMLPFunction(torch.autograd.Function):
     """shared_mlp(x) + the routed experts' weighted sum (reference modeling_deepseek_v3.py:265,
     `self.moe(...) + self.shared_experts(residuals)`) as one function: RoutedMLPFunction over the
     per-expert weights with the shared MLP's output as its residual.  Same kernels and bits forward
@@ -462,12 +562,30 @@ class RoutedAndSharedMLPFunction:
     down [out, in] matrices."""
 
     @staticmethod
-    def apply(hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
-              selected_experts_indices, cum_token_counts, rows_is_bound, *weights):
+    def forward(ctx, hidden_states, routing_weights, input_indices, cum_expert_counts_ep, output_indices,
+                selected_experts_indices, cum_token_counts, rows_is_bound, *weights):
+        ctx.leaves, ctx.shared_leaves = list(weights[:-3]), list(weights[-3:])
+        ctx.rows_is_bound = bool(rows_is_bound)
+        views = _expert_views(ctx.leaves)
+        index = (input_indices, cum_expert_counts_ep, output_indices, selected_experts_indices)
+        hidden_states, routing_weights = hidden_states.contiguous(), routing_weights.contiguous()
         one = single_segment_counts(hidden_states.shape[0], hidden_states.device)
-        return _n.host().routed_mlp(hidden_states, routing_weights, input_indices, cum_expert_counts_ep,
-                                    output_indices, selected_experts_indices, cum_token_counts, None,
-                                    bool(rows_is_bound), False, list(weights), True, one)
+        y_shared, *shared_state = _n.host().merged_mlp_forward(hidden_states, one, ctx.shared_leaves, None)
+        final, *state = _n.host().routed_mlp_forward(hidden_states, routing_weights, *index, cum_token_counts, y_shared,
+                                                     views)
+        ctx.save_for_backward(hidden_states, routing_weights, *index, *state, *views, *shared_state, *ctx.shared_leaves)
+        return final
+
+    @staticmethod
+    def backward(ctx, dfinal):
+        saved = ctx.saved_tensors
+        routed, views, shared_state, shared = saved[:11], saved[11:14], saved[14:18], saved[18:]
+        # first the shared MLP: its input gradient is the base of the routed experts' per-token sum
+        base, *dws_shared = _n.host().merged_mlp_backward(dfinal, routed[0], *shared_state, list(shared), ctx.shared_leaves,
+                                                          True, None, None, None)
+        dx, drw, *dws = _n.host().routed_mlp_backward(dfinal, *routed, list(views), ctx.leaves, False, ctx.rows_is_bound,
+                                                      base)
+        return (dx, drw, None, None, None, None, None, None, *dws, *dws_shared)
 
 
 def has_constant_pitch(weights):
@@ -497,6 +615,12 @@ def packed_expert_parameters(experts):
         pack_expert_weights(experts)
         params = _n.host().expert_parameters(experts)
     return params
+
+
+def group_mlp(x, cum_token_counts, experts, input_indices=None, cum_expert_counts_ep=None, output_indices=None):
+    """The expert MLPs of a ModuleList on x (GroupMLPFunction), or on x[input_indices] (GatheredGroupMLPFunction)."""
+    return _n.host().merged_mlp(x, cum_token_counts, False, packed_expert_parameters(experts), input_indices,
+                                cum_expert_counts_ep, output_indices)
 
 
 class PrepareInputForGroupGemmFunction(torch.autograd.Function):
@@ -531,21 +655,25 @@ class PrepareInputForGroupGemmFunction(torch.autograd.Function):
         return hidden_states_grad, None, None, None, None, None, None, None
 
 
-class GroupGemmOutputReductionFunction:
+class GroupGemmOutputReductionFunction(torch.autograd.Function):
     """K6: final[t] = sum_k w[t,k] * ggemm_output[pos(t,k)] in fp32, one rounding; backward gives
     ggemm_output_grad and routing_weights_grad (reference moe.py:284-377).  The four trailing
     flags are accepted and ignored.  routing_weights may be fp32 while activations are bf16."""
 
     @staticmethod
-    def apply(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-              input_indices, output_indices,
-              use_ref_path_fwd=False, use_ref_path_bwd=False,
-              use_triton_path_fwd=False, use_triton_path_bwd=False):
-        return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-                                 input_indices, output_indices, None)
+    def forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                input_indices, output_indices,
+                use_ref_path_fwd=False, use_ref_path_bwd=False,
+                use_triton_path_fwd=False, use_triton_path_bwd=False):
+        return _combine_forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                                input_indices, output_indices, None)
+
+    @staticmethod
+    def backward(ctx, final_hidden_states_grad):
+        return (*_n.host().combine_backward(final_hidden_states_grad, *ctx.saved_tensors), *(None,) * 8)
 
 
-class GroupGemmOutputReductionResidualFunction:
+class GroupGemmOutputReductionResidualFunction(torch.autograd.Function):
     """residual + GroupGemmOutputReductionFunction(...) in one pass: the combined sum is rounded to
     the activation dtype and then added to `residual` (both roundings of the two-step form).  Used
     for the decoder layer's residual connection (modeling_olmoe.py:415) and for the DeepSeek-V3
@@ -553,10 +681,23 @@ class GroupGemmOutputReductionResidualFunction:
     `residual` unchanged and into the combine's backward."""
 
     @staticmethod
-    def apply(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-              input_indices, output_indices, residual):
-        return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
-                                 input_indices, output_indices, residual)
+    def forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                input_indices, output_indices, residual):
+        return _combine_forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                                input_indices, output_indices, residual)
+
+    @staticmethod
+    def backward(ctx, final_hidden_states_grad):
+        return (*_n.host().combine_backward(final_hidden_states_grad, *ctx.saved_tensors), None, None, None, None,
+                final_hidden_states_grad)
+
+
+def _combine_forward(ctx, ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices, input_indices,
+                     output_indices, residual):
+    routing_weights = routing_weights.contiguous()
+    ctx.save_for_backward(ggemm_output, routing_weights, selected_experts_indices, input_indices, output_indices)
+    return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices, input_indices,
+                             output_indices, residual)
 
 
 # ----------------------------------------------------------------------------------------------
@@ -576,18 +717,18 @@ class MergedMLP(nn.Module):
         self.down_proj_merged_weight = torch.nn.Parameter(
             torch.empty((self.num_experts_per_rank, config.hidden_size, config.intermediate_size)))
 
+    def _weights(self):
+        return [self.gate_proj_merged_weight, self.up_proj_merged_weight, self.down_proj_merged_weight]
+
     def forward(self, input, cum_token_counts):
-        return MergedMLPFunction.apply(input, self.gate_proj_merged_weight, self.up_proj_merged_weight,
-                                       self.down_proj_merged_weight, cum_token_counts)
+        return _n.host().merged_mlp(input, cum_token_counts, True, self._weights(), None, None, None)
 
     def forward_gathered(self, hidden_states, input_indices, cum_expert_counts_ep, output_indices,
                          cum_token_counts):
         """forward(hidden_states[input_indices], cum_token_counts) with the gather folded into the
         GEMMs; the two index arrays after input_indices serve the backward's per-token reduction."""
-        return GatheredMergedMLPFunction.apply(hidden_states, input_indices, cum_expert_counts_ep,
-                                               output_indices, self.gate_proj_merged_weight,
-                                               self.up_proj_merged_weight, self.down_proj_merged_weight,
-                                               cum_token_counts)
+        return _n.host().merged_mlp(hidden_states, cum_token_counts, True, self._weights(), input_indices,
+                                    cum_expert_counts_ep, output_indices)
 
 
 def expert_computation(hidden_states, routing_weights, selected_experts, expert_start_idx,
@@ -646,13 +787,8 @@ def expert_computation(hidden_states, routing_weights, selected_experts, expert_
         ggemm_input = PrepareInputForGroupGemmFunction.apply(hidden_states, input_indices,
                                                              cum_expert_counts_ep, output_indices)
         ggemm_output = experts_fn(ggemm_input, cum_token_counts)
-    if residual is not None:
-        return GroupGemmOutputReductionResidualFunction.apply(
-            ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices, input_indices,
-            output_indices, residual)
-    return GroupGemmOutputReductionFunction.apply(ggemm_output, routing_weights, cum_expert_counts_ep,
-                                                  selected_experts_indices, input_indices,
-                                                  output_indices)
+    return _n.host().combine(ggemm_output, routing_weights, cum_expert_counts_ep, selected_experts_indices,
+                             input_indices, output_indices, residual)
 
 
 class FastOlmoeParallelSparseMoeBlock(nn.Module):
@@ -704,25 +840,22 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
     def _experts_fn(self, ggemm_input, cum_token_counts):
         if isinstance(self.experts, MergedMLP):
             return self.experts(ggemm_input, cum_token_counts)
-        return GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
-                                      *packed_expert_parameters(self.experts))
+        return group_mlp(ggemm_input, cum_token_counts, self.experts)
 
     def _gathered_experts_fn(self, hidden_states, input_indices, cum_expert_counts_ep, output_indices,
                              cum_token_counts):
         if isinstance(self.experts, MergedMLP):
             return self.experts.forward_gathered(hidden_states, input_indices, cum_expert_counts_ep,
                                                  output_indices, cum_token_counts)
-        return GatheredGroupMLPFunction.apply(hidden_states, input_indices, cum_expert_counts_ep,
-                                              output_indices, cum_token_counts,
-                                              *packed_expert_parameters(self.experts))
+        return group_mlp(hidden_states, cum_token_counts, self.experts, input_indices, cum_expert_counts_ep,
+                         output_indices)
 
     def _fused_experts_fn(self, hidden_states, routing_weights, selected_experts, residual):
         """Permutation and RoutedMLPFunction in one call; None when the kernels do not take the operands."""
         merged = isinstance(self.experts, MergedMLP)
         if merged:
             # (as attributes: a weight may be parametrized, or a plain tensor that a wrapper has put there)
-            weights = [self.experts.gate_proj_merged_weight, self.experts.up_proj_merged_weight,
-                       self.experts.down_proj_merged_weight]
+            weights = self.experts._weights()
         else:
             weights = packed_expert_parameters(self.experts)
         why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])

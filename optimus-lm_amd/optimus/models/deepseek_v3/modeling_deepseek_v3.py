@@ -42,8 +42,8 @@ class DeepseekV3ParallelMLP(nn.Module):
         lead = hidden_states.shape[:-1]
         x2 = hidden_states.reshape(-1, hidden_states.shape[-1]).contiguous()
         cum = _moe.single_segment_counts(x2.shape[0], x2.device)
-        y = _moe.MergedMLPFunction.apply(x2, self.gate_proj.weight, self.up_proj.weight,
-                                         self.down_proj.weight, cum)
+        y = _n.host().merged_mlp(x2, cum, True, [self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight],
+                                 None, None, None)
         return y.reshape(*lead, -1)
 
     def set_parameters_from_full_module(self, module):
@@ -139,14 +139,12 @@ class DeepseekV3ParallelMoE(nn.Module):
             self.use_activation_checkpointing_for_moe = config.activation_checkpointing_level & (1 << 0)
 
     def _experts_fn(self, ggemm_input, cum_token_counts):
-        return _moe.GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
-                                           *_moe.packed_expert_parameters(self.experts))
+        return _moe.group_mlp(ggemm_input, cum_token_counts, self.experts)
 
     def _gathered_experts_fn(self, hidden_states, input_indices, cum_expert_counts_ep, output_indices,
                              cum_token_counts):
-        return _moe.GatheredGroupMLPFunction.apply(hidden_states, input_indices, cum_expert_counts_ep,
-                                                   output_indices, cum_token_counts,
-                                                   *_moe.packed_expert_parameters(self.experts))
+        return _moe.group_mlp(hidden_states, cum_token_counts, self.experts, input_indices, cum_expert_counts_ep,
+                              output_indices)
 
     def _routed_kernels_fit(self, hidden_states, routing_weights):
         w0, d0 = self.experts[0].gate_proj.weight, self.experts[0].down_proj.weight

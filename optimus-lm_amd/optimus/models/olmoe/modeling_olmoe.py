@@ -13,6 +13,7 @@ import torch
 import torch.nn as nn
 from torch.utils.checkpoint import checkpoint as torch_activation_checkpoint
 
+from optimus import _native as _n
 from optimus.models.common import moe as _moe
 from optimus.models.common.norm import ParallelRMSNorm
 from optimus.models.common.ral_functions import (  # noqa: F401  (same names as the reference module)
@@ -36,8 +37,8 @@ class OlmoeParallelMLP(nn.Module):
         lead = x.shape[:-1]
         x2 = x.reshape(-1, x.shape[-1]).contiguous()
         cum = _moe.single_segment_counts(x2.shape[0], x2.device)
-        y = _moe.MergedMLPFunction.apply(x2, self.gate_proj.weight, self.up_proj.weight,
-                                         self.down_proj.weight, cum)
+        y = _n.host().merged_mlp(x2, cum, True, [self.gate_proj.weight, self.up_proj.weight, self.down_proj.weight],
+                                 None, None, None)
         return y.reshape(*lead, -1)
 
 
@@ -68,8 +69,7 @@ class OlmoeParallelSparseMoeBlock(nn.Module):
             raise NotImplementedError("force_uniform_routing is not part of this build")
 
     def _experts_fn(self, ggemm_input, cum_token_counts):
-        return _moe.GroupMLPFunction.apply(ggemm_input, cum_token_counts, False,
-                                           *_moe.packed_expert_parameters(self.experts))
+        return _moe.group_mlp(ggemm_input, cum_token_counts, self.experts)
 
     def forward(self, hidden_states):
         batch_size, sequence_length, hidden_dim = hidden_states.shape

@@ -380,3 +380,119 @@ def test_two_threads_run_backward_through_one_graph(cuda, which):
         assert err is None or "second time" in str(err), err
         done += err is None
     assert done >= 1
+
+
+# ---- the public autograd functions beside the nodes ---------------------------------------------------
+def _grad_results(outs, inputs, seed=5):
+    g = torch.Generator().manual_seed(seed)
+    outs = [o for o in outs if o.requires_grad]
+    ds = [torch.randn(o.shape, generator=g).to(o.dtype).to(o.device) for o in outs]
+    return [o.detach() for o in outs] + list(torch.autograd.grad(outs, inputs, ds))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_router_functions_equal_the_nodes(cuda, dtype):
+    from optimus import _native as _n
+    from optimus.models.common import moe
+    g = torch.Generator().manual_seed(0)
+    x = torch.randn(300, 512, generator=g).to(dtype).to(cuda).requires_grad_(True)
+    w = (torch.randn(8, 512, generator=g) * 0.05).to(dtype).to(cuda).requires_grad_(True)
+    pairs = [(lambda: moe.GateLogitsFunction.apply(x, w), lambda: _n.host().gate_logits(x, w))]
+    if dtype == torch.float32:
+        pairs.append((lambda: [moe.GateLogitsF32Function.apply(x, w)], lambda: [_n.host().gate_logits(x, w)[0]]))
+    pairs.append((lambda: moe.GateSoftmaxTopkFunction.apply(x, w, 2, True, dtype),
+                  lambda: _n.host().route_softmax(x, w, 2, True, dtype, True, False)))
+    for ours, node in pairs:
+        for a, b in zip(_grad_results(ours(), [x, w]), _grad_results(node(), [x, w])):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("live", [False, True])
+def test_expert_functions_equal_the_nodes(cuda, dtype, live):
+    """Merged and per-expert weights, gathered and not, fresh gradients and live ones."""
+    from optimus import _native as _n
+    from optimus.models.common import moe
+    T, K, G, H, I = 100, 2, 4, 64, 72
+    g = torch.Generator().manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(cuda)
+    experts = torch.randint(0, G, (T, 1), generator=g) + torch.arange(K)
+    cum, cum_ep, rows, out_rows, sel = moe.build_token_permutation((experts % G).to(cuda), 0, G)
+    x = rnd(T, H).to(dtype).requires_grad_(True)
+    rw = rnd(T, K).abs().to(dtype).requires_grad_(True)
+    res = rnd(T, H).to(dtype).requires_grad_(True)
+    merged = [(rnd(G, o, i) * 0.1).to(dtype).requires_grad_(True) for o, i in ((I, H), (I, H), (H, I))]
+    bank = [m.detach().clone() for m in merged]
+    each = [bank[j][n].detach().requires_grad_(True) for n in range(G) for j in range(3)]
+    shared = [(rnd(o, i) * 0.1).to(dtype).requires_grad_(True) for o, i in ((I, H), (I, H), (H, I))]
+    one = moe.single_segment_counts(T, cuda)
+    host = _n.host()
+    gathered = (rows, cum_ep, out_rows)
+    cases = {   # (function, node, activations, weights)
+        "merged": (lambda v: moe.MergedMLPFunction.apply(v, *merged, cum), lambda v: host.merged_mlp(v, cum, True, merged, None, None, None), merged),
+        "per_expert": (lambda v: moe.GroupMLPFunction.apply(v, cum, False, *each), lambda v: host.merged_mlp(v, cum, False, each, None, None, None), each),
+        "single": (lambda v: moe.MergedMLPFunction.apply(v, *shared, moe.single_segment_counts(v.shape[0], cuda)),
+                   lambda v: host.merged_mlp(v, moe.single_segment_counts(v.shape[0], cuda), True, shared, None, None, None), shared),
+        "gathered": (lambda v: moe.GatheredMergedMLPFunction.apply(x, *gathered, *merged, cum), lambda v: host.merged_mlp(x, cum, True, merged, *gathered), merged),
+        "gathered_per_expert": (lambda v: moe.GatheredGroupMLPFunction.apply(x, *gathered, cum, *each),
+                                lambda v: host.merged_mlp(x, cum, False, each, *gathered), each)}
+    xg = x.detach()[rows.long()].requires_grad_(True)
+    y = rnd(T * K, H).to(dtype).requires_grad_(True)
+    combine = {"combine": (moe.GroupGemmOutputReductionFunction, None, [y, rw]),
+               "combine_residual": (moe.GroupGemmOutputReductionResidualFunction, res, [y, rw, res])}
+
+    def results(out, acts, weights):
+        if not live:
+            return _grad_results([out], acts + list(weights))
+        for w in weights:                        # (several weights in one buffer: per-expert sinks need a constant pitch)
+            w.grad = None
+        if len(weights) == 3 * G:
+            for j in range(3):
+                buf = torch.ones(2, G, *weights[j].shape, device=cuda, dtype=dtype)[0]
+                for n in range(G):
+                    weights[3 * n + j].grad = buf[n]
+        else:
+            for w in weights:
+                w.grad = torch.ones(2, *w.shape, device=cuda, dtype=dtype)[0]
+        kept = [w.grad for w in weights]
+        for a in acts:
+            a.grad = None
+        out.backward(torch.ones_like(out) * 0.5)
+        assert all(w.grad is k for w, k in zip(weights, kept))
+        return [out.detach()] + [a.grad for a in acts] + [w.grad.clone() for w in weights]
+
+    for name, (ours, node, weights) in cases.items():
+        act = x if name.startswith("gathered") else xg
+        for a, b in zip(results(ours(act), [act], weights), results(node(act), [act], weights)):
+            assert torch.equal(a, b), name
+    for name, (cls, residual, ins) in combine.items():
+        extra = () if residual is None else (residual,)
+        for a, b in zip(_grad_results([cls.apply(y, rw, cum_ep, sel, rows, out_rows, *extra)], ins),
+                        _grad_results([host.combine(y, rw, cum_ep, sel, rows, out_rows, residual)], ins)):
+            assert torch.equal(a, b), name
+    if dtype == torch.float32:
+        return
+    routed = {
+        "routed": (lambda: moe.RoutedMLPFunction.apply(x, rw, rows, cum_ep, out_rows, sel, cum, res, True, *merged),
+                   lambda: host.moe_experts(x, rw, (experts % G).to(cuda), 0, G, G, False, res, True, merged, False, None),
+                   [x, rw, res], merged),
+        "routed_per_expert": (lambda: moe.RoutedMLPFunction.apply(x, rw, rows, cum_ep, out_rows, sel, cum, None, False, *each),
+                              lambda: host.moe_experts(x, rw, (experts % G).to(cuda), 0, G, G, False, None, False, each, False, None),
+                              [x, rw], each)}
+    for name, (ours, node, acts, weights) in routed.items():
+        for a, b in zip(results(ours(), acts, weights), results(node(), acts, weights)):
+            assert torch.equal(a, b), name
+    for w in each + shared:
+        w.grad = None
+    both = lambda f: _grad_results([f], [x, rw] + each + shared)
+    for a, b in zip(both(moe.RoutedAndSharedMLPFunction.apply(x, rw, rows, cum_ep, out_rows, sel, cum, False, *each, *shared)),
+                    both(host.moe_experts(x, rw, (experts % G).to(cuda), 0, G, G, False, None, False, each + shared, True, one))):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+def test_forward_mode_through_a_block_is_refused(cuda, which):
+    blk = _block(which, cuda)
+    x, d = _data(blk, cuda)
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+        _out(blk, torch.autograd.forward_ad.make_dual(x, d))

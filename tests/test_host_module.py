@@ -28,9 +28,6 @@ def _calls():
                           ("x", "weight")),
         "route_sigmoid": (lambda t: h.route_sigmoid(t["x"], t["weight"], t["bias"], 1, 1, K, True, 1.0),
                           ("x", "weight", "bias")),
-        "routed_mlp": (lambda t: h.routed_mlp(t["x"], t["rw"], t["rows"], t["cum_ep"], t["rows"], t["rows"], t["cum"],
-                                              t["residual"], False, True, leaves(t), False, None),
-                       ("x", "rw", "residual", "gate", "up", "down")),
         "moe_experts": (lambda t: h.moe_experts(t["x"], t["rw"], t["experts"], 0, N, N, False, t["residual"], True,
                                                 leaves(t), False, None),
                         ("x", "rw", "residual", "gate", "up", "down")),
@@ -41,8 +38,8 @@ def _calls():
     }
 
 
-CASES = [("gate_logits", 2), ("route_softmax", 2), ("route_sigmoid", 3), ("routed_mlp", 6), ("moe_experts", 6),
-         ("merged_mlp", 4), ("combine", 3)]
+CASES = [("gate_logits", 2), ("route_softmax", 2), ("route_sigmoid", 3), ("moe_experts", 6), ("merged_mlp", 4),
+         ("combine", 3)]
 
 
 @pytest.mark.parametrize("name,at", [(name, at) for name, n in CASES for at in range(n)])
@@ -83,3 +80,16 @@ def test_block_finds_a_parametrized_merged_weight():
     torch.nn.utils.parametrize.register_parametrization(blk.experts, "gate_proj_merged_weight", torch.nn.Identity())
     t = _tensors()
     assert blk._fused_experts_fn(t["x"].float(), t["rw"], t["experts"], None) is None
+
+
+def test_the_functions_are_autograd_functions():
+    """Callers subclass them, and call their forward and backward."""
+    from optimus.models.common import moe
+    for name in ("GateLogitsFunction", "GateLogitsF32Function", "GateSoftmaxTopkFunction", "SoftmaxTopkRouterFunction",
+                 "GroupedGemmFunction", "MergedMLPFunction", "GatheredMergedMLPFunction", "GroupMLPFunction",
+                 "GatheredGroupMLPFunction", "RoutedMLPFunction", "RoutedAndSharedMLPFunction",
+                 "PrepareInputForGroupGemmFunction", "GroupGemmOutputReductionFunction",
+                 "GroupGemmOutputReductionResidualFunction"):
+        cls = getattr(moe, name)
+        assert issubclass(cls, torch.autograd.Function), name
+        assert "forward" in vars(cls) and "backward" in vars(cls), name
