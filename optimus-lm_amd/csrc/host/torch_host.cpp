@@ -14,6 +14,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 #include <c10/hip/HIPStream.h>
@@ -209,16 +210,26 @@ bool has_grad_hooks(const Tensor &param) {
            (!hooks.is_none() && py::len(hooks) > 0) || (!posts.is_none() && py::len(posts) > 0);
 }
 
+// Whether the running backward pass accumulates into param.grad: torch.autograd.grad() returns gradients instead,
+// and backward(inputs=...) leaves the parameters alone that it does not name.
+bool accumulates_into(const Tensor &param) {
+    const auto *tasks = torch::autograd::get_current_graph_task_exec_info();
+    if (!tasks || tasks->empty()) return true;            // backward() of everything
+    const auto accumulator = torch::autograd::impl::try_get_grad_accumulator(param);
+    const auto it = tasks->find(accumulator.get());
+    return it != tasks->end() && it->second.needed_ && !it->second.captures_;
+}
+
 // param.grad if the weight-gradient kernels may add into it in place: a leaf parameter whose gradient
-// already exists as a dense view of a larger buffer, same dtype and shape, with no hooks that would
-// have to see the incoming gradient; else undefined.
+// already exists as a dense view of a larger buffer, same dtype and shape, in a pass that accumulates into it
+// and with no hooks that would have to see the incoming gradient; else undefined.
 Tensor live_grad(const Tensor &param) {
     if (!param.defined() || !param.is_leaf() || !param.requires_grad()) return Tensor();
     const Tensor &grad = param.grad();
     if (!grad.defined() || !grad.is_view() || grad.scalar_type() != param.scalar_type() ||
         grad.sizes() != param.sizes() || !grad.is_cuda() || !grad.is_contiguous() || grad.requires_grad())
         return Tensor();
-    return has_grad_hooks(param) ? Tensor() : grad;
+    return !accumulates_into(param) || has_grad_hooks(param) ? Tensor() : grad;
 }
 
 // One projection's gradient: where the GEMM writes it.

@@ -496,3 +496,27 @@ def test_forward_mode_through_a_block_is_refused(cuda, which):
     x, d = _data(blk, cuda)
     with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
         _out(blk, torch.autograd.forward_ad.make_dual(x, d))
+
+
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+def test_only_a_pass_that_accumulates_adds_into_live_gradients(cuda, which):
+    """torch.autograd.grad returns gradients and leaves .grad alone; backward(inputs=...) adds only where it is told."""
+    blk = _block(which, cuda)
+    opt = _flat_buffers(blk, cuda)
+    x, d = _data(blk, cuda)
+    x.requires_grad_(True)
+    params = list(blk.parameters())
+    out = _out(blk, x)
+    out.backward(d, retain_graph=True)
+    want = [p.grad.clone() for p in params]
+    dx = x.grad.clone()
+    opt.zero_grad()
+    got = torch.autograd.grad(out, [x] + params, d, retain_graph=True)
+    only_x = torch.autograd.grad(out, x, d, retain_graph=True)[0]
+    assert float(opt.flat_grad.float().abs().max()) == 0.0
+    for a, b in zip(got, [dx] + want):
+        assert torch.equal(a, b)
+    assert torch.equal(only_x, dx)
+    out.backward(d, inputs=[params[1]])
+    for i, p in enumerate(params):
+        assert torch.equal(p.grad, want[i] if i == 1 else torch.zeros_like(p))
