@@ -568,6 +568,27 @@ int om_moe_row_weights_grad(const float *row_dot, int parts, const int32_t *sele
                             void *routing_weights_grad, int64_t RT, int K, int weights_dtype,
                             void *stream);
 
+/* The four forward / input-gradient products of a block for callers that know `rows` only as a bound: under an
+ * expert window the count of routed rows stays on the device, and rows is T*K.  Outputs, launches and checks go by
+ * `rows`; which kernel runs goes by `expected_rows` (0 <= expected_rows <= rows, e.g. T*K times the window's share of
+ * the experts), with the rules that the plain forms apply to rows.  Any expected_rows gives correct results.      */
+int om_grouped_gemm_fwd_bound(const void *input, const void *weight, void *output,
+                              const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int N,
+                              int K, int64_t w_stride, void *stream);
+int om_merged_mlp_gate_up_fwd_weighted_bound(const void *x, const int32_t *x_rows, int64_t src_rows,
+                                             const void *w_gate, const void *w_up, const float *row_weights,
+                                             void *g, void *u, void *h, const int32_t *cum_token_counts,
+                                             int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                             int64_t w_stride, void *stream);
+int om_merged_mlp_down_dgrad_weighted_bound(const void *dy, const int32_t *dy_rows, int64_t src_rows,
+                                            const void *w_down, const void *g, const void *u,
+                                            const float *row_weights, void *dg, void *du, float *row_dot,
+                                            const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
+                                            int G, int I, int H, int64_t w_stride, void *stream);
+int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void *w_gate, const void *w_up,
+                                      void *dx, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
+                                      int G, int I, int H, int64_t w_stride, void *stream);
+
 /* Weight gradients added to a gradient buffer in place.  In the reference's training set-up every
  * p.grad is a view of the optimizer's flat gradient buffer (optimus/optimizers.py:105-111) that is
  * zeroed in place (:117-118), and micro-batches accumulate into it (dist_train.py:154): autograd

@@ -1177,16 +1177,17 @@ template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t
     return tiles * 2 >= device_cu_count();
 }
 
+// `rows` sizes the launch, `expected` (rows, or fewer where rows is a bound) selects the kernel.
 template <int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
-int launch_rows_auto(GemmParams &p, int64_t rows, hipStream_t st) {
-    if (uses_big_tile<EPI>(p.n_cols, p.kc, p.n_experts, rows))
+int launch_rows_auto(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
+    if (uses_big_tile<EPI>(p.n_cols, p.kc, p.n_experts, expected))
         return launch_rows<256, 256, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
     if (p.n_cols % 8 != 0 || p.kc % 8 != 0) return OM_ERR_SHAPE;
     if (p.kc % 64 != 0) return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW, true>(p, rows, st);
     // Few rows per expert (fewer than 256 on average): the launch streams weights that are used once, and the
     // kernels that keep two steps of them in flight are 4-10 % faster; with more rows the direct-load kernels
     // are (4-9 % at 2000 rows per expert), so each regime gets its own.
-    if (rows < static_cast<int64_t>(p.n_experts) * 256)
+    if (expected < static_cast<int64_t>(p.n_experts) * 256)
         return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW, false, true>(p, rows, st);
     return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
 }
@@ -1196,7 +1197,13 @@ int launch_rows_auto(GemmParams &p, int64_t rows, hipStream_t st) {
 extern "C" int om_grouped_gemm_fwd(const void *input, const void *weight, void *output,
                                    const int32_t *cum_token_counts, int64_t rows, int G, int N, int K,
                                    int64_t w_stride, void *stream) {
-    if (rows < 0 || G < 1 || !mult(N, 8) || !mult(K, 8)) return OM_ERR_SHAPE;
+    return om_grouped_gemm_fwd_bound(input, weight, output, cum_token_counts, rows, rows, G, N, K, w_stride, stream);
+}
+
+extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, void *output,
+                                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
+                                         int N, int K, int64_t w_stride, void *stream) {
+    if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(N, 8) || !mult(K, 8)) return OM_ERR_SHAPE;
     if (rows == 0) return OM_OK;
     if (!input || !weight || !output || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(input) || !om_aligned16(weight) || !om_aligned16(output)) return OM_ERR_ALIGN;
@@ -1209,10 +1216,11 @@ extern "C" int om_grouped_gemm_fwd(const void *input, const void *weight, void *
     p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(rows, G, N))
-        return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, G, N, K, p.strideB, om_stream(stream));
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N))
+        return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, p.strideB,
+                                   om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
-    return launch_rows_auto<CONTIG, CONTIG, EPI_STORE>(p, rows, om_stream(stream));
+    return launch_rows_auto<CONTIG, CONTIG, EPI_STORE>(p, rows, expected_rows, om_stream(stream));
 }
 
 extern "C" int om_grouped_gemm_dgrad(const void *output_grad, const void *weight, void *input_grad,
@@ -1232,7 +1240,7 @@ extern "C" int om_grouped_gemm_dgrad(const void *output_grad, const void *weight
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = K; p.kc = N; p.phases = 1;
-    return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, om_stream(stream));
+    return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, rows, om_stream(stream));
 }
 
 namespace {
@@ -1359,9 +1367,9 @@ namespace {
 // `row_weights` != null (needs x_rows): h = row_weights[r] * silu(g) * u
 int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate,
                        const void *w_up, const float *row_weights, void *g, void *u, void *h,
-                       const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
+                       const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I, int H,
                        int64_t w_stride, void *stream) {
-    if (rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
     if (rows == 0) return OM_OK;
     if (!x || !w_gate || !w_up || !g || !u || !h || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(x) || !om_aligned16(w_gate) || !om_aligned16(w_up) || !om_aligned16(g) ||
@@ -1382,13 +1390,14 @@ int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, c
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(rows, G, 2 * I))
-        return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, G, I, H,
-                                       p.strideB, om_stream(stream));
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I))
+        return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, expected, G, I,
+                                       H, p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
-    if (row_weights) return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A, true>(p, rows, om_stream(stream));
-    if (x_rows) return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A>(p, rows, om_stream(stream));
-    return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU>(p, rows, om_stream(stream));
+    if (row_weights)
+        return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A, true>(p, rows, expected, om_stream(stream));
+    if (x_rows) return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A>(p, rows, expected, om_stream(stream));
+    return launch_rows_auto<CONTIG, CONTIG, EPI_SWIGLU>(p, rows, expected, om_stream(stream));
 }
 }  // namespace
 
@@ -1396,7 +1405,7 @@ extern "C" int om_merged_mlp_gate_up_fwd(const void *x, const void *w_gate, cons
                                          void *u, void *h, const int32_t *cum_token_counts,
                                          int64_t rows, int G, int I, int H, int64_t w_stride,
                                          void *stream) {
-    return gate_up_fwd_launch(x, nullptr, 0, w_gate, w_up, nullptr, g, u, h, cum_token_counts, rows, G, I,
+    return gate_up_fwd_launch(x, nullptr, 0, w_gate, w_up, nullptr, g, u, h, cum_token_counts, rows, rows, G, I,
                               H, w_stride, stream);
 }
 
@@ -1408,7 +1417,7 @@ extern "C" int om_merged_mlp_gate_up_fwd_gathered(const void *x, const int32_t *
     if (rows > 0 && !x_rows) return OM_ERR_NULL;
     if (src_rows < 1 && rows > 0) return OM_ERR_SHAPE;
     return gate_up_fwd_launch(x, x_rows, src_rows, w_gate, w_up, nullptr, g, u, h, cum_token_counts, rows,
-                              G, I, H, w_stride, stream);
+                              rows, G, I, H, w_stride, stream);
 }
 
 extern "C" int om_merged_mlp_gate_up_fwd_weighted(const void *x, const int32_t *x_rows, int64_t src_rows,
@@ -1416,10 +1425,20 @@ extern "C" int om_merged_mlp_gate_up_fwd_weighted(const void *x, const int32_t *
                                                   const float *row_weights, void *g, void *u, void *h,
                                                   const int32_t *cum_token_counts, int64_t rows, int G,
                                                   int I, int H, int64_t w_stride, void *stream) {
+    return om_merged_mlp_gate_up_fwd_weighted_bound(x, x_rows, src_rows, w_gate, w_up, row_weights, g, u, h,
+                                                    cum_token_counts, rows, rows, G, I, H, w_stride, stream);
+}
+
+extern "C" int om_merged_mlp_gate_up_fwd_weighted_bound(const void *x, const int32_t *x_rows, int64_t src_rows,
+                                                        const void *w_gate, const void *w_up,
+                                                        const float *row_weights, void *g, void *u, void *h,
+                                                        const int32_t *cum_token_counts, int64_t rows,
+                                                        int64_t expected_rows, int G, int I, int H, int64_t w_stride,
+                                                        void *stream) {
     if (rows > 0 && (!x_rows || !row_weights)) return OM_ERR_NULL;
     if (src_rows < 1 && rows > 0) return OM_ERR_SHAPE;
     return gate_up_fwd_launch(x, x_rows, src_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts,
-                              rows, G, I, H, w_stride, stream);
+                              rows, expected_rows, G, I, H, w_stride, stream);
 }
 
 namespace {
@@ -1432,9 +1451,9 @@ static_assert(256 / Waves<256>::N == ROW_DOT_COLS && 128 / Waves<128>::N == ROW_
 // scaled by row_weights[r] and row_dot receives the partial sums of (dy W) * silu(g) * u
 int down_dgrad_launch(const void *dy, const int32_t *dy_rows, int64_t src_rows, const void *w_down,
                       const void *g, const void *u, const float *row_weights, void *dg, void *du,
-                      float *row_dot, const int32_t *cum_token_counts, int64_t rows, int G, int I, int H,
-                      int64_t w_stride, void *stream) {
-    if (rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+                      float *row_dot, const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I,
+                      int H, int64_t w_stride, void *stream) {
+    if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
     if (rows == 0) return OM_OK;
     if (!dy || !w_down || !g || !u || !dg || !du || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(dy) || !om_aligned16(w_down) || !om_aligned16(g) || !om_aligned16(u) ||
@@ -1457,8 +1476,9 @@ int down_dgrad_launch(const void *dy, const int32_t *dy_rows, int64_t src_rows, 
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
-    if (dy_rows) return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD, GATHER_A, true>(p, rows, om_stream(stream));
-    return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD>(p, rows, om_stream(stream));
+    if (dy_rows)
+        return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD, GATHER_A, true>(p, rows, expected, om_stream(stream));
+    return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD>(p, rows, expected, om_stream(stream));
 }
 }  // namespace
 
@@ -1467,7 +1487,7 @@ extern "C" int om_merged_mlp_down_dgrad(const void *dy, const void *w_down, cons
                                         int64_t rows, int G, int I, int H, int64_t w_stride,
                                         void *stream) {
     return down_dgrad_launch(dy, nullptr, 0, w_down, g, u, nullptr, dg, du, nullptr, cum_token_counts, rows,
-                             G, I, H, w_stride, stream);
+                             rows, G, I, H, w_stride, stream);
 }
 
 extern "C" int om_merged_mlp_row_dot_parts(int I) {
@@ -1481,17 +1501,35 @@ extern "C" int om_merged_mlp_down_dgrad_weighted(const void *dy, const int32_t *
                                                  float *row_dot, const int32_t *cum_token_counts,
                                                  int64_t rows, int G, int I, int H, int64_t w_stride,
                                                  void *stream) {
+    return om_merged_mlp_down_dgrad_weighted_bound(dy, dy_rows, src_rows, w_down, g, u, row_weights, dg, du, row_dot,
+                                                   cum_token_counts, rows, rows, G, I, H, w_stride, stream);
+}
+
+extern "C" int om_merged_mlp_down_dgrad_weighted_bound(const void *dy, const int32_t *dy_rows, int64_t src_rows,
+                                                       const void *w_down, const void *g, const void *u,
+                                                       const float *row_weights, void *dg, void *du,
+                                                       float *row_dot, const int32_t *cum_token_counts,
+                                                       int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                       int64_t w_stride, void *stream) {
     if (rows > 0 && (!dy_rows || !row_weights || !row_dot)) return OM_ERR_NULL;
     if (src_rows < 1 && rows > 0) return OM_ERR_SHAPE;
     return down_dgrad_launch(dy, dy_rows, src_rows, w_down, g, u, row_weights, dg, du, row_dot,
-                             cum_token_counts, rows, G, I, H, w_stride, stream);
+                             cum_token_counts, rows, expected_rows, G, I, H, w_stride, stream);
 }
 
 extern "C" int om_merged_mlp_gate_up_dgrad(const void *dg, const void *du, const void *w_gate,
                                            const void *w_up, void *dx, const int32_t *cum_token_counts,
                                            int64_t rows, int G, int I, int H, int64_t w_stride,
                                            void *stream) {
-    if (rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    return om_merged_mlp_gate_up_dgrad_bound(dg, du, w_gate, w_up, dx, cum_token_counts, rows, rows, G, I, H, w_stride,
+                                             stream);
+}
+
+extern "C" int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void *w_gate,
+                                                 const void *w_up, void *dx, const int32_t *cum_token_counts,
+                                                 int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                 int64_t w_stride, void *stream) {
+    if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
     if (rows == 0) return OM_OK;
     if (!dg || !du || !w_gate || !w_up || !dx || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(dg) || !om_aligned16(du) || !om_aligned16(w_gate) || !om_aligned16(w_up) ||
@@ -1509,5 +1547,5 @@ extern "C" int om_merged_mlp_gate_up_dgrad(const void *dg, const void *du, const
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = H; p.kc = I; p.phases = 2;
-    return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, om_stream(stream));
+    return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, expected_rows, om_stream(stream));
 }

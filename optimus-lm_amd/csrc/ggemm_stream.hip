@@ -198,12 +198,12 @@ template <bool SWIGLU, bool WIDE> __global__ __launch_bounds__(WAVES * 64, WIDE 
     else stream_tile<SWIGLU, 4, 1, WIDE ? 2 : 1>(p, expert, row0, row_end, n0, part);
 }
 
-template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, hipStream_t st) {
+template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, int64_t expected, hipStream_t st) {
     const int64_t hit = rows < p.n_experts ? rows : p.n_experts;
     const int64_t tiles = hit + rows / ROWS < rows ? hit + rows / ROWS : rows;   // >= sum of ceil(rows of an expert / ROWS)
     const int cols = SWIGLU ? 16 : 32;
     const dim3 grid((p.n_cols + cols - 1) / cols, static_cast<unsigned>(tiles)), block(WAVES * 64);
-    if (rows > 16 * static_cast<int64_t>(p.n_experts)) stream_kernel<SWIGLU, true><<<grid, block, 0, st>>>(p);
+    if (expected > 16 * static_cast<int64_t>(p.n_experts)) stream_kernel<SWIGLU, true><<<grid, block, 0, st>>>(p);
     else stream_kernel<SWIGLU, false><<<grid, block, 0, st>>>(p);
     return om_launch_status();
 }
@@ -211,22 +211,27 @@ template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, hipStream
 }  // namespace
 
 // The line between these kernels and the tiled ones (tiled -> here, us, gate+up + down):
-//   up to two rows per expert on average: hidden 2048, ffn 1024, 64 experts, top-8: 1 token 22 + 12.3 -> 13.7 + 7.1,
+//   fewer than two rows per expert on average: hidden 2048, ffn 1024, 64 experts, top-8: 1 token 22 + 12.3 -> 13.7 + 7.1,
 //   2 tokens 24 + 14.1 -> 25 + 13.5, 3 tokens 35 + 20 -> 34 + 17, 8 tokens even, 16 tokens even + 40 -> 43; 37
-//   tokens (4.6 rows) 111 + 43 -> 111 + 48, hidden 7168, ffn 2048 at 8 rows 321 + 165 -> 360 + 174: tiled above two;
+//   tokens (4.6 rows) 111 + 43 -> 111 + 48, hidden 7168, ffn 2048 at 8 rows 321 + 165 -> 360 + 174: tiled from two on;
+//   the same for a window of 32 experts of 7168 / 2048 whose rows are only expected (T tokens of top-8 of 256, six
+//   draws of weights and tokens, whole pass): 40 tokens -3.5 to +3.6 %, 56 tokens -7 to +3 %, 9 tokens 241 -> 220;
 //   more rows where the tiles cannot fill the chip (fewer tiles than CUs): one expert of hidden 7168, ffn 2048
 //   with 64 rows 65 + 21 -> 40 + 14; 12 experts of hidden 1000, ffn 712 with 192 rows 19 + 11.6 -> 10.8 + 5.4;
 //   beyond 64 rows of one expert the weights are streamed again per row tile: 128 rows 65 + 21 -> 43 + 25.
+// `rows`: those to expect where only a bound is known.  (Going by the bound, eight times as many, the window of 32
+// experts of 1024 / 256 ran its gate+up product on tiles at 4 rows per expert and on 256x256 ones at 62: forward of
+// 128 tokens 82.3 -> 78.4 us, 256 86.5 -> 83.3, 1000 105.6 -> 102.3, 2000 112 -> 109; 512 91.6 -> 94.2.)
 bool om_ggemm_streams(int64_t rows, int n_experts, int cols) {
     if (rows > 64 + 16 * static_cast<int64_t>(n_experts)) return false;
-    if (rows <= 2 * static_cast<int64_t>(n_experts)) return true;
+    if (rows < 2 * static_cast<int64_t>(n_experts)) return true;
     const int64_t hit = rows < n_experts ? rows : n_experts;
     return (hit + rows / 128) * ((cols + 127) / 128) <= 256;
 }
 
 int om_ggemm_stream_gate_up(const void *x, const int32_t *x_rows, const void *w_gate, const void *w_up,
-                            const float *row_weights, void *g, void *u, void *h, const int32_t *cum, int64_t rows, int G,
-                            int I, int H, int64_t w_stride, hipStream_t st) {
+                            const float *row_weights, void *g, void *u, void *h, const int32_t *cum, int64_t rows, int64_t expected,
+                            int G, int I, int H, int64_t w_stride, hipStream_t st) {
     StreamParams p = {};
     p.x = static_cast<const uint16_t *>(x);
     p.w[0] = static_cast<const uint16_t *>(w_gate);
@@ -239,11 +244,11 @@ int om_ggemm_stream_gate_up(const void *x, const int32_t *x_rows, const void *w_
     p.row_scale = row_weights;
     p.w_stride = w_stride;
     p.n_experts = G; p.n_cols = I; p.kc = H;
-    return launch<true>(p, rows, st);
+    return launch<true>(p, rows, expected, st);
 }
 
-int om_ggemm_stream_fwd(const void *x, const void *w, void *out, const int32_t *cum, int64_t rows, int G, int N, int K,
-                        int64_t w_stride, hipStream_t st) {
+int om_ggemm_stream_fwd(const void *x, const void *w, void *out, const int32_t *cum, int64_t rows, int64_t expected, int G,
+                        int N, int K, int64_t w_stride, hipStream_t st) {
     StreamParams p = {};
     p.x = static_cast<const uint16_t *>(x);
     p.w[0] = p.w[1] = static_cast<const uint16_t *>(w);
@@ -251,5 +256,5 @@ int om_ggemm_stream_fwd(const void *x, const void *w, void *out, const int32_t *
     p.cum = cum;
     p.w_stride = w_stride;
     p.n_experts = G; p.n_cols = N; p.kc = K;
-    return launch<false>(p, rows, st);
+    return launch<false>(p, rows, expected, st);
 }

@@ -103,6 +103,8 @@ template <typename F> void launch(const Call &c, const char *name, F &&fn) {
     check(code, name);
 }
 #define OM(c, fn, ...) launch(c, #fn, [&] { return fn(__VA_ARGS__); })
+// the form of fn that takes a bound and the rows to expect, logged as fn
+#define OM_BOUND(c, fn, ...) launch(c, #fn, [&] { return fn##_bound(__VA_ARGS__); })
 
 // optimus.profilers.record_pcl_function(name) around a scope, when a profiler is set.  What the profiler raises
 // at the scope's end reaches the caller, as from a `with` block; while another exception passes it is reported
@@ -283,6 +285,8 @@ struct Index {
     const float *row_weights = nullptr;   // the routing weight of every sorted row (one-buffer form only)
     int64_t rows = 0;               // entries of the three last: the routed rows, or an upper bound of them
     bool bound = false;
+    int64_t expected = -1;          // with a bound: the rows to expect, where they can be told
+    int64_t to_choose_by() const { return bound && expected >= 0 ? expected : rows; }
 };
 
 std::vector<Tensor> sort_tensors(const Call &c, const Tensor &experts, int64_t start, int64_t end) {
@@ -464,9 +468,10 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
             weights = fp(row_weights);
             OM(c, om_moe_row_weights, ptr(rw), ix.sel, ix.in, ix.out, fpm(row_weights), rows, K, dtype_code(rw), c.stream);
         }
-        OM(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
-           ptr(s.u), ptr(s.h), ix.cum, rows, G, I, H, pitch, c.stream);
-        OM(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, G, H, I, expert_stride(w.down), c.stream);
+        OM_BOUND(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
+                 ptr(s.u), ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, c.stream);
+        OM_BOUND(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
+                 expert_stride(w.down), c.stream);
     }
     ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_fwd");
     OM(c, om_sum_ggemm_output, ptr(y), ix.cum_ep, ix.out, ptr(residual), ptr(final), T, H, OM_BF16, c.stream);
@@ -490,14 +495,15 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
             if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
             Tensor row_dot = make({parts, rows}, x, at::kFloat);
             wgrad(c, dfinal, s.h, k.down, ix.cum, rows, G, H, I, WgradRows::OUTPUT_GRAD, ix.in, T);
-            OM(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
-               ix.row_weights ? ix.row_weights : fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows, G, I, H, expert_stride(w.down), c.stream);
+            OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
+                     ix.row_weights ? ix.row_weights : fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows,
+                     ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
             OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
                c.stream);
             wgrad(c, dg, x, k.gate, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
             wgrad(c, du, x, k.up, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
-            OM(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows, G, I,
-               H, expert_stride(w.gate), c.stream);
+            OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
+                     ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
         } else {   // nothing routed to these experts: fresh weight gradients are zero, live ones stay as they are
             for (const Sink *sk : {&k.down, &k.gate, &k.up})
                 if (!sk->accumulate) {
@@ -1093,6 +1099,9 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
         const int64_t I = leaves[0].size(-2), H = x.size(1);
         if (sync_free || ix.rows * (3 * I + H) * 2 <= BOUND_ROWS_BYTES) {
             ix.bound = true;
+            // the kernels are chosen by the window's share of the pairs, not by all of them
+            ix.expected = std::max<int64_t>(1, ix.rows * (end - start) / n_total);
+            ix.expected = std::min(ix.expected, ix.rows);
         } else {
             // read the count back (as the reference does), behind the shared expert's kernels: they do not
             // need it, and while the GPU runs them the host waits for a copy that was enqueued before them

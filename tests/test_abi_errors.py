@@ -210,6 +210,24 @@ def test_routing_weight_folded_into_the_expert_mlp(lib):
     assert lib.om_moe_row_weights_grad(None, 16, None, None, None, None, 0, 8, F32, None) == OK
 
 
+def test_products_over_a_bound_of_the_rows(lib):
+    """0 <= expected_rows <= rows; everything else as the plain forms."""
+    for expected in (-1, 4097):
+        assert lib.om_grouped_gemm_fwd_bound(P, P, P, P, 4096, expected, 64, 2048, 1024, 0, None) == SHAPE
+        assert lib.om_merged_mlp_gate_up_fwd_weighted_bound(P, P, 512, P, P, P, P, P, P, P, 4096, expected, 64, 1024, 2048, 0,
+                                                            None) == SHAPE
+        assert lib.om_merged_mlp_down_dgrad_weighted_bound(P, P, 512, P, P, P, P, P, P, P, P, 4096, expected, 64, 1024, 2048, 0,
+                                                           None) == SHAPE
+        assert lib.om_merged_mlp_gate_up_dgrad_bound(P, P, P, P, P, P, 4096, expected, 64, 1024, 2048, 0, None) == SHAPE
+    assert lib.om_grouped_gemm_fwd_bound(P, None, P, P, 4096, 64, 64, 2048, 1024, 0, None) == NULL
+    assert lib.om_grouped_gemm_fwd_bound(None, None, None, None, 0, 0, 64, 2048, 1024, 0, None) == OK
+    assert lib.om_merged_mlp_gate_up_fwd_weighted_bound(P, None, 512, P, P, P, P, P, P, P, 4096, 64, 64, 1024, 2048, 0,
+                                                        None) == NULL
+    assert lib.om_merged_mlp_down_dgrad_weighted_bound(P, P, 512, P, P, P, P, P, ODD, P, P, 4096, 64, 64, 1024, 2048, 0,
+                                                       None) == ALIGN
+    assert lib.om_merged_mlp_gate_up_dgrad_bound(P, P, P, P, None, P, 4096, 64, 64, 1024, 2048, 0, None) == NULL
+
+
 def test_check_raises_with_the_library_text():
     with pytest.raises(n.NativeLibraryError, match="dtype"):
         n.check(DTYPE, "om_adamw_step")

@@ -555,3 +555,58 @@ def test_half_row_tiles_of_the_256_kernels(cuda, counts):
         s = slice(int(cum[e]), int(cum[e + 1]))
         for name, got, want, k in (("fwd", y[s], x[s].float() @ w[e].float().t(), K), ("dgrad", dx[s], dy[s].float() @ w[e].float(), N)):
             assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6 * k ** 0.5).all(), (name, e)
+
+
+@pytest.mark.parametrize("expected", [0, 9, 100, 1087, 3000, 9000])
+@pytest.mark.parametrize("N,K", [(1024, 512), (200, 328)])
+def test_products_over_a_bound_of_the_rows(cuda, expected, N, K):
+    """Outputs sized by a bound of the rows, the kernel chosen by the rows to expect (streamed weights, both loads
+    of the 128x128 tile, 256x256): right for any expectation, nothing written past the rows there are.  A row far
+    from the expected ones included; bounds as in test_few_row_products_stream_the_weights."""
+    from optimus import _native as n
+    counts, bound = [0, 1, 300, 0, 17, 64, 700, 5], 9000
+    G, rows, T = len(counts), sum(counts), 211
+    g = torch.Generator().manual_seed(expected + N)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    bf = lambda *s, f=1.0: (torch.randn(*s, generator=g) * f).to(torch.bfloat16).to(cuda)
+    x, dy = bf(T, K), bf(T, K)
+    index = torch.zeros(bound, dtype=torch.int32)
+    index[:rows] = torch.randint(0, T, (rows,), generator=g).int()
+    scale = torch.rand(bound, generator=g).to(cuda)
+    wg, wu, wd = bf(G, N, K, f=0.05), bf(G, N, K, f=0.05), bf(G, K, N, f=0.05)
+    new = lambda c: torch.full((bound, c), 7.0, dtype=torch.bfloat16, device=cuda)
+    G_, U, Hh, dG, dU, Y, dX = new(N), new(N), new(N), new(N), new(N), new(K), new(K)
+    parts = n.lib().om_merged_mlp_row_dot_parts(N)
+    dot = torch.full((parts, bound), 7.0, device=cuda)
+    d, ix, P, st = cum.to(cuda), index.to(cuda), n.ptr, n.stream()
+    L = n.lib()
+    n.check(L.om_merged_mlp_gate_up_fwd_weighted_bound(P(x), P(ix), T, P(wg), P(wu), P(scale), P(G_), P(U), P(Hh), P(d), bound,
+                                                       expected, G, N, K, 0, st), "gate_up")
+    n.check(L.om_grouped_gemm_fwd_bound(P(Hh), P(wd), P(Y), P(d), bound, expected, G, K, N, 0, st), "down")
+    n.check(L.om_merged_mlp_down_dgrad_weighted_bound(P(dy), P(ix), T, P(wd), P(G_), P(U), P(scale), P(dG), P(dU), P(dot), P(d),
+                                                      bound, expected, G, N, K, 0, st), "down_dgrad")
+    n.check(L.om_merged_mlp_gate_up_dgrad_bound(P(dG), P(dU), P(wg), P(wu), P(dX), P(d), bound, expected, G, N, K, 0, st), "dx")
+    torch.cuda.synchronize()
+    for t in (G_, U, Hh, dG, dU, Y, dX):
+        assert (t[rows:] == 7.0).all()
+    assert (dot[:, rows:] == 7.0).all()
+    xr, dyr, sc = x[ix[:rows].long()].float(), dy[ix[:rows].long()].float(), scale[:rows, None]
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        g_, u_ = xr[s] @ wg[e].float().t(), xr[s] @ wu[e].float().t()
+        gb, ub = G_[s].float(), U[s].float()
+        sig = torch.sigmoid(gb)
+        dh = dyr[s] @ wd[e].float()
+        pre = sc[s] * dh
+        want = {"g": (G_[s], g_, K), "u": (U[s], u_, K), "h": (Hh[s], sc[s] * torch.nn.functional.silu(g_) * u_, K),
+                "y": (Y[s], Hh[s].float() @ wd[e].float().t(), N), "du": (dU[s], pre * gb * sig, K),
+                "dg": (dG[s], pre * ub * sig * (1 + gb * (1 - sig)), K),
+                "dx": (dX[s], dG[s].float() @ wg[e].float() + dU[s].float() @ wu[e].float(), 2 * N)}
+        for name, (got, ref, k) in want.items():
+            rel = 2 ** -7 + 2 ** -12 if name in ("du", "dg") else 2 ** -8
+            # (the order of the sum enters du and dg through a factor of at most |g|, |u| (1 + |g|))
+            factor = 1 + (gb.abs() + ub.abs() * (1 + gb.abs()) if name in ("du", "dg") else 0)
+            assert ((got.float() - ref).abs() <= ref.abs() * rel + 1e-6 * k ** 0.5 * factor).all(), (name, e)
+        terms = dh * gb * sig * ub
+        assert ((dot[:, s].sum(0) - terms.sum(1)).abs() <= (2 ** -8 + 1e-5) * terms.abs().sum(1) + 1e-6).all(), e
