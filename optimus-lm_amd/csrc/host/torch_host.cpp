@@ -1049,11 +1049,19 @@ variable_list routed_mlp_backward(const Tensor &dfinal, const Tensor &x, const T
     return grads;
 }
 
-// Activations of the expert MLP sized by the upper bound T*K instead of the routed rows of an expert
-// window cost expert_parallelism times their memory, and save the host the wait for the count.  Up to
-// this many bytes of them the wait costs more than the memory (a decode batch's are a few MB; 64 MB is
-// 0.02 % of the card).
-constexpr int64_t BOUND_ROWS_BYTES = 64 << 20;
+// Activations of the expert MLP sized by the upper bound T*K instead of the routed rows of an expert window cost
+// expert_parallelism times their memory, and save the host the wait for the count.  What the wait costs, whole
+// passes, us, count read -> bound: forward of 1024/256 experts 64 tokens 89.6 -> 82.5, 1000 tokens 109 -> 104, of
+// 7168/2048 16 tokens 255 -> 254, 512 tokens 583 -> 576; training steps of 1024/256 16 tokens 412 -> 402, of 7168/2048
+// 64 tokens 2435 -> 2432.
+// Without gradients the memory lives for the call only: 64 MB, 0.02 % of the card.  Where a backward follows every
+// layer keeps it, so there the limit is also a 32nd of the layer's own expert weights: whatever the depth of a model,
+// at most 3 % of what its weights take.
+constexpr int64_t BOUND_ROWS_BYTES = 64 << 20, BOUND_ROWS_WEIGHTS = 32;
+bool sized_by_bound(int64_t rows, int64_t G, int64_t I, int64_t H, bool needs_grad) {
+    const int64_t activations = rows * (3 * I + H) * 2, weights = 3 * G * I * H * 2;
+    return activations <= BOUND_ROWS_BYTES && (!needs_grad || activations <= weights / BOUND_ROWS_WEIGHTS);
+}
 
 // One device integer on its way to the host.
 struct CountReadback {
@@ -1080,7 +1088,7 @@ struct CountReadback {
 };
 
 // Sort (with the routing weights laid out per sorted row) and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
-// sync_free: never read the routed-row count of an expert window back.
+// sync_free: never read the routed-row count of an expert window back (else up to a limit: sized_by_bound).
 Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
                    bool sync_free, const std::optional<Tensor> &residual, bool merged, const std::vector<Tensor> &leaves,
                    bool has_shared, const std::optional<Tensor> &one) {
@@ -1097,7 +1105,8 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
     const bool windowed = !(start == 0 && end == n_total);
     if (windowed) {
         const int64_t I = leaves[0].size(-2), H = x.size(1);
-        if (sync_free || ix.rows * (3 * I + H) * 2 <= BOUND_ROWS_BYTES) {
+        const Tensor res = residual.value_or(Tensor());
+        if (sync_free || sized_by_bound(ix.rows, end - start, I, H, any_requires_grad({x, rw, res}) || any_requires_grad(leaves))) {
             ix.bound = true;
             // the kernels are chosen by the window's share of the pairs, not by all of them
             ix.expected = std::max<int64_t>(1, ix.rows * (end - start) / n_total);
@@ -1381,6 +1390,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         at::NoGradGuard no_grad;
         return strided_view(weights.data(), 1, static_cast<int64_t>(weights.size()));
     });
+    m.def("sized_by_bound", &sized_by_bound);
     m.def("live_grad", &live_grad);
     m.def("expert_parameters", &expert_parameters);
     m.def("foreign_grads", &foreign_grads);

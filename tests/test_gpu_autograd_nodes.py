@@ -520,3 +520,23 @@ def test_only_a_pass_that_accumulates_adds_into_live_gradients(cuda, which):
     out.backward(d, inputs=[params[1]])
     for i, p in enumerate(params):
         assert torch.equal(p.grad, want[i] if i == 1 else torch.zeros_like(p))
+
+
+def test_a_training_step_keeps_no_activations_of_other_ranks_pairs(cuda):
+    """An expert window of 8 of 16 experts: what a forward pass keeps for backward is sized by the rows routed here
+    (the bound would be over twice that), a forward without gradients may use the bound."""
+    blk = _block("dsv3", cuda)
+    x, _ = _data(blk, cuda, tokens=1024)
+    with torch.no_grad():
+        experts, _w = blk.gate(x)
+    here = int((experts >= 8).sum())
+    T, H, I = 2048, 256, 128
+    x.requires_grad_(True)
+    _out(blk, x)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = _out(blk, x)
+    kept = torch.cuda.memory_allocated() - before
+    # g, u, h of the routed and the shared expert, the output, routing and index arrays (T rows of 16 + 6 * 4 words)
+    assert kept <= 1.1 * (2 * 3 * I * (here + T) + 2 * T * H + 4 * T * 64) < 2 * 3 * I * (4 * T + T)
+    del out

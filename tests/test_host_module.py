@@ -93,3 +93,12 @@ def test_the_functions_are_autograd_functions():
         cls = getattr(moe, name)
         assert issubclass(cls, torch.autograd.Function), name
         assert "forward" in vars(cls) and "backward" in vars(cls), name
+
+
+@pytest.mark.parametrize("G,I,H", [(32, 2048, 7168), (32, 256, 1024), (1, 8, 8)])
+def test_window_activations_sized_by_a_bound_are_limited(G, I, H):
+    """64 MB while nothing is kept for a backward; with one, also a 32nd of the layer's expert weights."""
+    f, row = _n.host().sized_by_bound, 2 * (3 * I + H)
+    free, kept = (64 << 20) // row, min(64 << 20, 6 * G * I * H // 32) // row
+    assert f(free, G, I, H, False) and not f(free + 1, G, I, H, False)
+    assert f(kept, G, I, H, True) and not f(kept + 1, G, I, H, True)
