@@ -282,8 +282,8 @@ def bench_other_configs(args, device, with_cpu, only=None):
     import torch
     import synthetic_configs as sc
     from optimus.mapper import ParallelDpPpEpTpMapper
-    from optimus.models.common.moe import (MergedMLPFunction, RoutedMLPFunction, SoftmaxTopkRouterFunction,
-                                           expert_computation)
+    from optimus import _native
+    from optimus.models.common.moe import SoftmaxTopkRouterFunction
     steps = max(3, min(args.steps, 10))
     out = {}
 
@@ -363,16 +363,15 @@ def bench_other_configs(args, device, with_cpu, only=None):
         logits = inp["logits"].to(device)
         t = {k: inp[k].to(device).requires_grad_(True) for k in ("x", "w_gate", "w_up", "w_down")}
         dout = inp["dout"].to(device)
-        routed = lambda hs, rw, ii, cum_ep, oi, si, cum, res: RoutedMLPFunction.apply(
-            hs, rw, ii, cum_ep, oi, si, cum, res, True, t["w_gate"], t["w_up"], t["w_down"])
-        fn = lambda gi, cum: MergedMLPFunction.apply(gi, t["w_gate"], t["w_up"], t["w_down"], cum)
+        weights = [t["w_gate"], t["w_up"], t["w_down"]]
 
         def step_c4():
             for v in t.values():
                 v.grad = None
             w, e = SoftmaxTopkRouterFunction.apply(logits, c["K"], False, torch.bfloat16)
-            o = expert_computation(t["x"], w.detach().requires_grad_(True), e, 0, c["N"], fn, c["N"],
-                                   routed_experts_fn=routed)
+            # (the call behind a block's router: permutation, experts and combine)
+            o = _native.host().moe_experts(t["x"], w.detach().requires_grad_(True), e, 0, c["N"], c["N"], False, None, True,
+                                           weights, False, None)
             o.backward(dout)
         ms, per = _timed_steps(step_c4, args.warmup, steps)
         flops = 18.0 * c["T"] * c["K"] * c["H"] * c["I"]
@@ -395,7 +394,7 @@ def bench_other_configs(args, device, with_cpu, only=None):
                         "permutation, expert GEMMs, combine; fwd+bwd)",
             "rows_per_expert": {"min": int(counts.min()), "median": int(counts.median()), "max": int(counts.max()),
                                 "experts_with_at_most_8_rows": int((counts <= 8).sum())}})
-        del t, logits, dout
+        del t, weights, logits, dout
 
     # ---- C5 -----------------------------------------------------------------------------------
     if only in (None, "C5"):

@@ -188,12 +188,14 @@ def test_fast_block_float32_c1(cuda, merged):
         assert max_abs(a, gref) <= 1e-4 * max(1.0, float(gref.abs().max())), (k, max_abs(a, gref))
 
 
-@pytest.mark.parametrize("path", ["separate", "fused"])
+@pytest.mark.parametrize("path", ["separate", "fused", "block"])
 def test_fast_block_injected_logits_skewed(cuda, path):
     """C4: Zipf-skewed routing injected at the functional level (router logits given): many experts
-    get 0-8 rows, a few get hundreds.  Expert computation only (router excluded), fwd+bwd, both as
-    the reference's sequence of separate functions (K4, MergedMLP, K6) and as the blocks' default
-    (RoutedMLPFunction: gather and routing weight inside the expert GEMMs), each against fp32."""
+    get 0-8 rows, a few get hundreds.  Expert computation only (router excluded), fwd+bwd, as the
+    reference's sequence of separate functions (K4, MergedMLP, K6), as RoutedMLPFunction (gather and
+    routing weight inside the expert GEMMs) on index arrays built apart, and as the blocks run it (the
+    permutation inside the same call), each against fp32."""
+    from optimus import _native
     from optimus.models.common.moe import (SoftmaxTopkRouterFunction, MergedMLPFunction, RoutedMLPFunction,
                                            expert_computation)
     inp = sc.moe_inputs("C4")
@@ -212,7 +214,11 @@ def test_fast_block_injected_logits_skewed(cuda, path):
     if path == "fused":
         routed = lambda hs, rw, ii, cum_ep, oi, si, cum, res: RoutedMLPFunction.apply(
             hs, rw, ii, cum_ep, oi, si, cum, res, True, t["w_gate"], t["w_up"], t["w_down"])
-    out = expert_computation(t["x"], wd, e, 0, c["N"], fn, c["N"], routed_experts_fn=routed)
+    block = None
+    if path == "block":
+        block = lambda hs, rw, ee, res: _native.host().moe_experts(
+            hs, rw, ee, 0, c["N"], c["N"], False, res, True, [t["w_gate"], t["w_up"], t["w_down"]], False, None)
+    out = expert_computation(t["x"], wd, e, 0, c["N"], fn, c["N"], routed_experts_fn=routed, fused_experts_fn=block)
     out.backward(inp["dout"].to(cuda))
     r = {k: inp[k].float().requires_grad_(True) for k in ("x", "w_gate", "w_up", "w_down")}
     wr = w_ref.float().requires_grad_(True)

@@ -19,20 +19,25 @@ from util import mean_rel
 pytestmark = pytest.mark.gpu
 
 ALLOWED = 1.0     # times the reference sequence's own distance from float32 (measured: 0.54-0.92)
-_cpu_side = {}    # config name -> the two CPU evaluations (shared by the two GPU forms)
+_cpu_side = {}    # config name -> the two CPU evaluations (shared by the GPU forms)
 
 
 def _gpu_expert_path(cuda, inp, w, e, fuse):
+    from optimus import _native
     from optimus.models.common.moe import MergedMLPFunction, RoutedMLPFunction, expert_computation
     c = inp["cfg"]
     t = {k: inp[k].to(cuda).requires_grad_(True) for k in ("x", "w_gate", "w_up", "w_down")}
     wd = w.to(cuda).requires_grad_(True)
     fn = lambda gi, cum: MergedMLPFunction.apply(gi, t["w_gate"], t["w_up"], t["w_down"], cum)
-    routed = None
-    if fuse:
+    routed = block = None
+    if fuse == "block":
+        block = lambda hs, rw, ee, res: _native.host().moe_experts(
+            hs, rw, ee, 0, c["N"], c["N"], False, res, True, [t["w_gate"], t["w_up"], t["w_down"]], False, None)
+    elif fuse:
         routed = lambda hs, rw, ii, cum_ep, oi, si, cum, res: RoutedMLPFunction.apply(
             hs, rw, ii, cum_ep, oi, si, cum, res, True, t["w_gate"], t["w_up"], t["w_down"])
-    out = expert_computation(t["x"], wd, e.to(cuda), 0, c["N"], fn, c["N"], routed_experts_fn=routed)
+    out = expert_computation(t["x"], wd, e.to(cuda), 0, c["N"], fn, c["N"], routed_experts_fn=routed,
+                             fused_experts_fn=block)
     out.backward(inp["dout"].to(cuda))
     torch.cuda.synchronize()
     grads = {k: v.grad.float().cpu() for k, v in t.items()}
@@ -41,7 +46,7 @@ def _gpu_expert_path(cuda, inp, w, e, fuse):
 
 
 @pytest.mark.parametrize("name,scale", [("C1", 1.0), ("C3", 0.125), ("C4", 1.0)])
-@pytest.mark.parametrize("fuse", [False, True], ids=["separate_functions", "routing_weight_in_mlp"])
+@pytest.mark.parametrize("fuse", [False, True, "block"], ids=["separate_functions", "routing_weight_in_mlp", "as_the_blocks_run_it"])
 def test_not_further_from_float32_than_the_reference_sequence_in_bf16(cuda, name, scale, fuse):
     inp = sc.moe_inputs(name, scale_tokens=scale)
     c = inp["cfg"]
