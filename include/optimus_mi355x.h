@@ -463,7 +463,7 @@ int om_grouped_gemm_wgrad(const void *output_grad, const void *input, void *weig
 /* The same three products for float32 modules (GroupedGemmFunction runs in the module's dtype,
  * moe.py:174-178, :201-210; the reference's small CPU-runnable configuration is float32): fp32
  * operands, fp32 MFMA accumulation, fp32 results.  N and K multiples of 8, w_stride a multiple
- * of 4.  Built for parity at fp32 accuracy, not tuned.                                       */
+ * of 4.                                                                                      */
 int om_grouped_gemm_fwd_f32(const float *input, const float *weight, float *output,
                             const int32_t *cum_token_counts, int64_t rows, int G, int N, int K,
                             int64_t w_stride, void *stream);

@@ -1,6 +1,7 @@
 """ctypes binding of liboptimus_mi355x.so, the C-ABI library of HIP kernels.
 
-This is the only place that touches the library.  Tensors are passed as raw device pointers
+Python code reaches the library through this module only, and the C++ host module (csrc/host/torch_host.cpp), which
+launches the blocks' kernels itself, is loaded here too (host()).  Tensors are passed as raw device pointers
 (`tensor.data_ptr()`), the stream is PyTorch's current HIP stream.  There is no fallback: if
 the library is missing or a call returns an error code, an exception is raised.
 """

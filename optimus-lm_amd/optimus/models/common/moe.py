@@ -743,15 +743,18 @@ def expert_computation(hidden_states, routing_weights, selected_experts, expert_
     cum_token_counts, residual)` may do gather, experts and combine in one function
     (RoutedMLPFunction); it returns None when its kernels do not take the operands.
     `fused_experts_fn(hidden_states, routing_weights, selected_experts, residual)` does the same
-    including the permutation, whose arrays then never become Python objects.
+    including the permutation, whose arrays then never become Python objects: what the blocks pass
+    (moe_experts of the host module); `routed_experts_fn` serves callers with an expert function of
+    their own.
 
-    Under an expert window the number of routed rows is only known on the device.  By default it is
-    read back once, like the reference does (moe.py:520).  With `sync_free_window` and a
-    `routed_experts_fn` nothing is read back: the index arrays keep their T*K entries (om_moe_sort
-    marks the unused tail), the activations of the expert MLP are allocated for T*K rows, of which
-    only the routed ones are computed, and the function is called with `rows_is_bound=True`.  That
-    makes the step capturable in a HIP graph at the price of expert_parallelism times the
-    activation memory."""
+    Under an expert window the number of routed rows is only known on the device.  It is read back
+    once, like the reference does (moe.py:520), by the fused function only where activations for all
+    T*K pairs would take too much memory (sized_by_bound).  With `sync_free_window` and a
+    `routed_experts_fn`, or a block's `sync_free_expert_window`, nothing is ever read back: the index
+    arrays keep their T*K entries (om_moe_sort marks the unused tail), the activations of the expert
+    MLP are allocated for T*K rows, of which only the routed ones are computed, and the function is
+    called with `rows_is_bound=True`.  That makes the step capturable in a HIP graph at the price of
+    expert_parallelism times the activation memory."""
     if fused_experts_fn is not None:
         final = fused_experts_fn(hidden_states, routing_weights, selected_experts, residual)
         if final is not None:
@@ -860,7 +863,7 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
             weights = packed_expert_parameters(self.experts)
         why = routed_mlp_unfit_reason(hidden_states, routing_weights, weights[0], weights[2])
         if why is not None:
-            if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
+            if hidden_states.dtype == torch.bfloat16:    # (float32 modules apply the weight in the combine, by design)
                 note_unfused_path("routing weight inside the expert MLP", why)
             return None
         return _n.host().moe_experts(hidden_states, routing_weights, selected_experts, self.expert_start_idx,

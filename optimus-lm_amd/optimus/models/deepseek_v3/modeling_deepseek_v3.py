@@ -54,7 +54,8 @@ class SigmoidGroupTopkRouterFunction(torch.autograd.Function):
     """(topk_indices, topk_weights) from fp32 router logits: reference
     modeling_deepseek_v3.py:150-180 (selection, no grad) and :185-191 (weights).  Index order
     within a token is (choice score desc, expert index asc); the reference leaves it unspecified
-    (torch.topk(sorted=False))."""
+    (torch.topk(sorted=False)).  For callers with logits of their own: DeepseekV3ParallelTopkRouter
+    routes in the launch that ends the gate projection."""
 
     @staticmethod
     def forward(ctx, router_logits, bias, n_group, topk_group, top_k, norm_topk_prob, scale):
@@ -156,7 +157,7 @@ class DeepseekV3ParallelMoE(nn.Module):
         params = _moe.packed_expert_parameters(self.experts)
         why = _moe.routed_mlp_unfit_reason(hidden_states, routing_weights, params[0], params[2])
         if why is not None:
-            if hidden_states.dtype == torch.bfloat16:    # (float32 modules run unfused by design)
+            if hidden_states.dtype == torch.bfloat16:    # (float32 modules apply the weight in the combine, by design)
                 _moe.note_unfused_path("routing weight inside the expert MLP", why)
             return None
         one = None

@@ -459,7 +459,9 @@ class GradNormPlan:
     ONE_LAUNCH_MAX = 24 << 20
 
     def __init__(self, starts, sizes, device, chunk=None):
-        # two blocks per CU for a small buffer (a chunk is one block's work), 64 K elements each for a large one
+        # two blocks per CU for a small buffer (a chunk is one block's work), 64 K elements each for a large one.  The
+        # chunk groups the float32 partial sums: a buffer of less than 2^24 elements gets another grouping than
+        # with 64 K elements throughout, and with it a norm, a clip coefficient and an update that can differ in the last place
         if chunk is None:
             chunk = min(self.CHUNK, max(4096, 1 << (sum(int(sz) for sz in sizes) // 512).bit_length()))
         chunk = int(chunk)
