@@ -496,7 +496,7 @@ def test_few_row_products_stream_the_weights(cuda, counts, N, K, weighted):
     from optimus import _native as n
     G, rows = len(counts), sum(counts)
     # (the rule: otherwise the tiled kernels run)
-    assert rows <= 64 + 16 * G and (rows <= 2 * G or (min(rows, G) + rows // 128) * ((2 * N + 127) // 128) <= 256)
+    assert rows <= 64 + 16 * G and (rows < 2 * G or (min(rows, G) + rows // 128) * ((2 * N + 127) // 128) <= 256)
     g = torch.Generator().manual_seed(rows + N + K)
     cum = torch.zeros(G + 1, dtype=torch.int32)
     cum[1:] = torch.cumsum(torch.tensor(counts), 0)
