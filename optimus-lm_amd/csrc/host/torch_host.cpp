@@ -586,7 +586,6 @@ struct HostNode : Node {
     variable_list apply(variable_list &&grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
         try {
-            at::AutoDispatchBelowADInplaceOrView below;
             return run(std::move(grads));
         } catch (const NativeError &e) {
             py::gil_scoped_acquire gil;
@@ -609,6 +608,7 @@ struct HostNode : Node {
     // checkpointing, offloading) see all of it and a second backward is refused.
     std::vector<SavedVariable> vars;
     void save(const Tensor &t) { vars.emplace_back(t, false); }
+    // (to be called where autograd records: a hook may run a whole forward pass, as checkpointing does)
     std::vector<Tensor> saved() {
         std::vector<Tensor> out;
         out.reserve(vars.size());
@@ -761,8 +761,9 @@ struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits 
         auto grad = [&](int at) { return at >= 0 && at < static_cast<int>(grads.size()) ? grads[at] : Tensor(); };
         Tensor logits_grad = grad(out_logits), weights_grad = grad(out_weights), x_grad = grad(out_x);
         if (!logits_grad.defined() && !weights_grad.defined()) return {x_grad, Tensor()};
-        const Call c = begin_call();
         const std::vector<Tensor> kept = saved();
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
         const Tensor &xs = kept[0], &ws = kept[1];
         Tensor dlogits = logits_grad;
         if (weights_grad.defined()) {
@@ -931,10 +932,11 @@ struct RoutedNode : HostNode {
     variable_list run(variable_list &&grads) override {
         const size_t n_in = 3 + routed.n_leaves + shared.n_leaves;
         if (!grads[0].defined()) return variable_list(n_in);
-        const Call c = begin_call();
-        const Tensor dfinal = grads[0].contiguous();
         // x, rw, row_weights, g, u, h [, shared g, u, h, cum], the index arrays' owners, the weights [, the shared ones]
         const std::vector<Tensor> kept = saved();
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Call c = begin_call();
+        const Tensor dfinal = grads[0].contiguous();
         const MlpWeights w = weights(routed, kept), ws = has_shared ? weights(shared, kept) : MlpWeights();
         const MlpState s{Tensor(), kept[3], kept[4], kept[5]};
         size_t at = 6;
@@ -1149,6 +1151,7 @@ struct MergedNode : HostNode {
         if (!grads[0].defined()) return variable_list(1 + experts.n_leaves);
         // x, cum, g, u, h, the gathered forms' index arrays (x_rows, cum_ep, out_rows), the weights
         const std::vector<Tensor> kept = saved();
+        at::AutoDispatchBelowADInplaceOrView below;
         return merged_mlp_grads(begin_call(), grads[0], kept[0], weights(experts, kept), {kept[1], kept[2], kept[3], kept[4]},
                                 kept[5], kept[6], kept[7], experts);
     }

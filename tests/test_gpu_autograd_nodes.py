@@ -9,6 +9,7 @@ import time
 import pytest
 import torch
 import torch.nn.utils.parametrize
+import torch.utils.checkpoint
 
 pytestmark = pytest.mark.gpu
 
@@ -540,3 +541,30 @@ def test_a_training_step_keeps_no_activations_of_other_ranks_pairs(cuda):
     # g, u, h of the routed and the shared expert, the output, routing and index arrays (T rows of 16 + 6 * 4 words)
     assert kept <= 1.1 * (2 * 3 * I * (here + T) + 2 * T * H + 4 * T * 64) < 2 * 3 * I * (4 * T + T)
     del out
+
+
+# ---- activation checkpointing around a block ----------------------------------------------------------
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_checkpointed_region_around_a_block(cuda, which, reentrant):
+    """torch's layers before the block in one checkpointed region: the recomputation starts when the block's node
+    unpacks what it saved, and has to record those layers too."""
+    blk = _block(which, cuda)
+    dtype = next(blk.parameters()).dtype
+    torch.manual_seed(1)
+    before = torch.nn.Sequential(torch.nn.Linear(256, 256, bias=False), torch.nn.GELU(), torch.nn.LayerNorm(256)).to(cuda).to(dtype)
+    x, d = _data(blk, cuda)
+    region = lambda v: _out(blk, before(v))
+    params = list(before.parameters()) + list(blk.parameters())
+
+    def grads(f):
+        v = x.clone().requires_grad_(True)
+        for p in params:
+            p.grad = None
+        out = f(v)
+        out.backward(d)
+        return [out.detach(), v.grad] + [p.grad for p in params]
+    want = grads(region)
+    got = grads(lambda v: torch.utils.checkpoint.checkpoint(region, v, use_reentrant=reentrant))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
