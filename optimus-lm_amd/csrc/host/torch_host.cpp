@@ -12,6 +12,7 @@
 // buffer gets it added there by the GEMM and an undefined gradient returned.
 #include <torch/extension.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/engine.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/graph_task.h>
@@ -232,6 +233,25 @@ Tensor live_grad(const Tensor &param) {
         grad.sizes() != param.sizes() || !grad.is_cuda() || !grad.is_contiguous() || grad.requires_grad())
         return Tensor();
     return !accumulates_into(param) || has_grad_hooks(param) ? Tensor() : grad;
+}
+
+// At the end of the running backward pass: order the caller's stream behind what this stream has been given.  A
+// gradient that a GEMM adds into its live buffer never reaches autograd, which orders the caller's stream only
+// behind gradients that it accumulates itself; the forward may have run on another stream than its caller's.
+void order_live_gradients() {
+    if (!torch::autograd::get_current_graph_task_exec_info()) return;   // (not in a backward pass)
+    const auto stream = c10::hip::getCurrentHIPStream();
+    torch::autograd::Engine::get_default_engine().queue_callback([stream] {
+        const auto caller = c10::hip::getCurrentHIPStream(stream.device_index());
+        if (caller.stream() == stream.stream()) return;
+        const c10::DeviceGuard device(stream.device());
+        hipEvent_t done = nullptr;
+        const bool ok = hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess &&
+                        hipEventRecord(done, stream.stream()) == hipSuccess &&
+                        hipStreamWaitEvent(caller.stream(), done, 0) == hipSuccess;
+        if (done) (void)hipEventDestroy(done);
+        if (!ok) throw NativeError("ordering the caller's stream behind the weight gradients failed");
+    });
 }
 
 // One projection's gradient: where the GEMM writes it.
@@ -650,8 +670,10 @@ struct HostNode : Node {
 
 Sinks sinks_of(const Call &c, const ExpertWeights &e, const MlpWeights &w) {
     const int64_t n = e.merged ? 1 : e.G;
-    return {grad_sink(c, &e.params[0], 3, n, w.gate), grad_sink(c, &e.params[1], 3, n, w.up),
-            grad_sink(c, &e.params[2], 3, n, w.down)};
+    Sinks k = {grad_sink(c, &e.params[0], 3, n, w.gate), grad_sink(c, &e.params[1], 3, n, w.up),
+               grad_sink(c, &e.params[2], 3, n, w.down)};
+    if (k.gate.accumulate || k.up.accumulate || k.down.accumulate) order_live_gradients();
+    return k;
 }
 // gradients in the order of the leaves; undefined for a projection whose gradient went into its live buffer
 void push_grads(variable_list &out, const Sinks &k, const ExpertWeights &e) {
@@ -1394,7 +1416,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         return strided_view(weights.data(), 1, static_cast<int64_t>(weights.size()));
     });
     m.def("sized_by_bound", &sized_by_bound);
-    m.def("live_grad", &live_grad);
+    m.def("live_grad", [](const Tensor &param) {
+        Tensor grad = live_grad(param);
+        if (grad.defined()) order_live_gradients();
+        return grad;
+    });
     m.def("expert_parameters", &expert_parameters);
     m.def("foreign_grads", &foreign_grads);
     m.def("constant_pitch", [](const std::vector<Tensor> &weights) {

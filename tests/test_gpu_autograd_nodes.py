@@ -568,3 +568,27 @@ def test_checkpointed_region_around_a_block(cuda, which, reentrant):
     got = grads(lambda v: torch.utils.checkpoint.checkpoint(region, v, use_reentrant=reentrant))
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which", sorted(BLOCKS))
+def test_callers_stream_waits_for_gradients_added_in_place(cuda, which):
+    """Forward on a side stream that is busy, backward called from the current one, no gradient but the in-place ones:
+    what the caller's stream reads next is the finished sum."""
+    blk = _block(which, cuda)
+    blk.gate.requires_grad_(False)
+    opt = _flat_buffers(blk, cuda)
+    x, d = _data(blk, cuda)
+    other = _out(blk, x)                             # (keeps the parameters' accumulation nodes on this stream)
+    _out(blk, x).backward(d)
+    want = opt.flat_grad.clone()
+    opt.zero_grad()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = _out(blk, x)
+        torch.cuda._sleep(100_000_000)               # (some 50 ms)
+    out.backward(d)
+    got = opt.flat_grad.clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and float(want.float().abs().max()) > 0
+    del other
