@@ -1328,24 +1328,34 @@ std::vector<Tensor> expert_parameters(py::handle experts) {
 
 // The .grad of every parameter of `model` whose id() is not in `owned` and that has one, each parameter
 // once.  For a plain nn.Module tree this walks the modules' dictionaries (a step of a small optimizer spent
-// 20 us in the generator behind model.parameters()); anything that overrides the traversal is asked itself.
-void walk_parameters(PyObject *module, std::unordered_set<PyObject *> &modules, const std::function<void(PyObject *)> &visit) {
-    if (!modules.insert(module).second) return;
+// 20 us in the generator behind model.parameters()); where anything overrides the traversal, on the model's class,
+// on the model itself or on the class of a module inside it, model.parameters() is asked.
+PyObject *module_base() {   // torch.nn.Module (kept for good)
+    static PyObject *base = py::object(py::module_::import("torch.nn").attr("Module")).release().ptr();
+    return base;
+}
+bool walk_parameters(PyObject *module, std::unordered_set<PyObject *> &modules, const std::function<void(PyObject *)> &visit) {
+    if (!modules.insert(module).second) return true;
+    static PyObject *named_modules = PyUnicode_InternFromString("named_modules");
+    const py::object ours = py::reinterpret_steal<py::object>(PyObject_GetAttr(reinterpret_cast<PyObject *>(Py_TYPE(module)), named_modules));
+    const py::object base = py::reinterpret_steal<py::object>(PyObject_GetAttr(module_base(), named_modules));
+    if (!ours || !base) { PyErr_Clear(); return false; }
+    if (ours.ptr() != base.ptr()) return false;
     for (const char *name : {"_parameters", "_modules"}) {
         py::object d = py::reinterpret_steal<py::object>(PyObject_GetAttrString(module, name));
         if (!d) throw py::error_already_set();
         PyObject *key, *value;
         Py_ssize_t at = 0;
-        if (!PyDict_Check(d.ptr())) throw py::type_error("nn.Module dictionary expected");
+        if (!PyDict_Check(d.ptr())) return false;
         while (PyDict_Next(d.ptr(), &at, &key, &value)) {
             if (value == Py_None) continue;
             if (name[1] == 'p') visit(value);
-            else walk_parameters(value, modules, visit);
+            else if (!walk_parameters(value, modules, visit)) return false;
         }
     }
+    return true;
 }
 py::list foreign_grads(py::object model, py::set owned) {
-    static PyObject *base = py::object(py::module_::import("torch.nn").attr("Module")).release().ptr();   // (kept for good)
     py::list out;
     std::unordered_set<PyObject *> modules, seen;
     auto visit = [&](PyObject *p) {
@@ -1356,12 +1366,17 @@ py::list foreign_grads(py::object model, py::set owned) {
         if (!grad) throw py::error_already_set();
         if (!grad.is_none()) out.append(grad);
     };
-    bool plain = py::isinstance(model, py::handle(base));
-    for (const char *name : {"parameters", "named_parameters", "_named_members", "named_modules"})
-        plain = plain && py::type::of(model).attr(name).ptr() == py::handle(base).attr(name).ptr();
-    if (plain) walk_parameters(model.ptr(), modules, visit);
-    else
-        for (py::handle p : model.attr("parameters")()) visit(p.ptr());
+    const py::handle base(module_base());
+    bool plain = py::isinstance(model, base);
+    if (plain) {
+        const py::dict own = model.attr("__dict__");
+        for (const char *name : {"parameters", "named_parameters", "_named_members", "named_modules"})
+            plain = plain && !own.contains(name) && py::type::of(model).attr(name).ptr() == base.attr(name).ptr();
+    }
+    if (plain && walk_parameters(model.ptr(), modules, visit)) return out;
+    out = py::list();
+    seen.clear();
+    for (py::handle p : model.attr("parameters")()) visit(p.ptr());
     return out;
 }
 

@@ -102,3 +102,34 @@ def test_window_activations_sized_by_a_bound_are_limited(G, I, H):
     free, kept = (64 << 20) // row, min(64 << 20, 6 * G * I * H // 32) // row
     assert f(free, G, I, H, False) and not f(free + 1, G, I, H, False)
     assert f(kept, G, I, H, True) and not f(kept + 1, G, I, H, True)
+
+
+class _Hiding(torch.nn.Sequential):
+    def named_modules(self, memo=None, prefix="", remove_duplicate=True):
+        yield prefix, self
+        yield prefix + ".0", self[0]
+
+
+def _models():
+    lin = lambda: torch.nn.Linear(3, 2)
+    shared = lin()
+    plain = torch.nn.Sequential(lin(), torch.nn.ModuleDict({"a": shared, "b": torch.nn.Sequential(shared, lin())}))
+    on_class = _Hiding(lin(), lin())
+    inside = torch.nn.Sequential(lin(), _Hiding(lin(), lin()))
+    on_itself = torch.nn.Sequential(lin(), lin())
+    on_itself.parameters = lambda: iter([on_itself[0].weight])
+    stranger = type("Model", (), {"parameters": lambda self: iter(list(plain.parameters())[:3])})()
+    return dict(plain=plain, on_class=on_class, inside=inside, on_itself=on_itself, stranger=stranger)
+
+
+@pytest.mark.parametrize("which", sorted(_models()))
+def test_foreign_gradients_are_those_of_the_models_own_traversal(which):
+    model = _models()[which]
+    params = list(model.parameters())
+    every = [p for m in ([model] if isinstance(model, torch.nn.Module) else []) for p in torch.nn.Module.parameters(m)] or params
+    for p in every[1:]:
+        p.grad = torch.ones_like(p)
+    owned = {id(params[-1])}
+    want = [p.grad for p in params if id(p) not in owned and p.grad is not None]
+    got = _n.host().foreign_grads(model, owned)
+    assert [id(g) for g in got] == [id(g) for g in want]
