@@ -126,9 +126,17 @@ def _models():
 def test_foreign_gradients_are_those_of_the_models_own_traversal(which):
     model = _models()[which]
     params = list(model.parameters())
-    every = [p for m in ([model] if isinstance(model, torch.nn.Module) else []) for p in torch.nn.Module.parameters(m)] or params
-    for p in every[1:]:
+
+    def fill(module):                                # (also what an override hides)
+        for p in module._parameters.values():
+            p.grad = torch.ones_like(p)
+        for m in module._modules.values():
+            fill(m)
+    if isinstance(model, torch.nn.Module):
+        fill(model)
+    for p in params:
         p.grad = torch.ones_like(p)
+    params[0].grad = None
     owned = {id(params[-1])}
     want = [p.grad for p in params if id(p) not in owned and p.grad is not None]
     got = _n.host().foreign_grads(model, owned)
