@@ -1299,30 +1299,53 @@ Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const
 
 // ---- Python module ----------------------------------------------------------------------------------
 
-// The (gate, up, down) weights of a ModuleList of expert MLPs in GroupMLPFunction's order.  Walks the
-// modules' dictionaries: nn.Module attribute access costs about a microsecond each, and a DeepSeek-V3
-// share has 96 of these.
-std::vector<Tensor> expert_parameters(py::handle experts) {
-    static PyObject *s_modules = PyUnicode_InternFromString("_modules"), *s_parameters = PyUnicode_InternFromString("_parameters"),
-                    *s_weight = PyUnicode_InternFromString("weight");
-    static PyObject *names[3] = {PyUnicode_InternFromString("gate_proj"), PyUnicode_InternFromString("up_proj"),
-                                 PyUnicode_InternFromString("down_proj")};
-    auto in_dict = [](py::handle owner, PyObject *dict_name, PyObject *key) -> py::object {   // null when absent
-        py::object d = py::reinterpret_steal<py::object>(PyObject_GetAttr(owner.ptr(), dict_name));
-        if (!d) throw py::error_already_set();
-        if (!PyDict_Check(d.ptr())) return py::object();
-        return py::reinterpret_borrow<py::object>(PyDict_GetItemWithError(d.ptr(), key));
-    };
-    std::vector<Tensor> out;
-    py::object children = experts.attr("_modules");
-    for (auto item : py::cast<py::dict>(children))
-        for (PyObject *name : names) {
-            py::object lin = in_dict(item.second, s_modules, name);
-            if (!lin) lin = py::getattr(item.second, name);
-            py::object weight = in_dict(lin, s_parameters, s_weight);
-            if (!weight) weight = lin.attr("weight");
-            out.push_back(weight.cast<Tensor>());
+PyObject *module_base() {   // torch.nn.Module (kept for good)
+    static PyObject *base = py::object(py::module_::import("torch.nn").attr("Module")).release().ptr();
+    return base;
+}
+
+// Attributes of nn.Module objects, one name: out of the module's `dictionary` (_parameters or _modules) where that is
+// what attribute access would end at, which costs a microsecond each; as an attribute where the class or the object
+// has the name itself (a property, a tensor put there) or the class brings its own attribute access.
+struct ModuleAttribute {
+    PyObject *name, *dictionary;
+    PyTypeObject *type = nullptr;   // the last type seen, and whether it leaves the name to the dictionaries
+    bool plain = false;
+    ModuleAttribute(const char *n, const char *d) : name(PyUnicode_InternFromString(n)), dictionary(PyUnicode_InternFromString(d)) {}
+    py::object of(py::handle owner) {
+        PyObject *o = owner.ptr();
+        if (Py_TYPE(o) != type) {
+            type = Py_TYPE(o);
+            auto *base = reinterpret_cast<PyTypeObject *>(module_base());
+            plain = PyType_IsSubtype(type, base) && !_PyType_Lookup(type, name);
+            for (const char *hook : {"__getattr__", "__getattribute__"}) {
+                const py::str h(hook);
+                plain = plain && _PyType_Lookup(type, h.ptr()) == _PyType_Lookup(base, h.ptr());
+            }
         }
+        if (plain) {
+            PyObject **own = _PyObject_GetDictPtr(o);
+            if (own && *own && !PyDict_GetItemWithError(*own, name)) {
+                PyObject *d = PyDict_GetItemWithError(*own, dictionary);      // borrowed, as all of these
+                PyObject *value = d && PyDict_Check(d) ? PyDict_GetItemWithError(d, name) : nullptr;
+                if (value) return py::reinterpret_borrow<py::object>(value);
+            }
+            if (PyErr_Occurred()) throw py::error_already_set();
+        }
+        py::object value = py::reinterpret_steal<py::object>(PyObject_GetAttr(o, name));
+        if (!value) throw py::error_already_set();
+        return value;
+    }
+};
+
+// The (gate, up, down) weights of a ModuleList of expert MLPs in GroupMLPFunction's order (a DeepSeek-V3 share has 96).
+std::vector<Tensor> expert_parameters(py::handle experts) {
+    ModuleAttribute projections[3] = {{"gate_proj", "_modules"}, {"up_proj", "_modules"}, {"down_proj", "_modules"}};
+    ModuleAttribute weight("weight", "_parameters");
+    std::vector<Tensor> out;
+    const py::object children = experts.attr("_modules");
+    for (auto item : py::cast<py::dict>(children))
+        for (ModuleAttribute &projection : projections) out.push_back(weight.of(projection.of(item.second)).cast<Tensor>());
     return out;
 }
 
@@ -1330,10 +1353,6 @@ std::vector<Tensor> expert_parameters(py::handle experts) {
 // once.  For a plain nn.Module tree this walks the modules' dictionaries (a step of a small optimizer spent
 // 20 us in the generator behind model.parameters()); where anything overrides the traversal, on the model's class,
 // on the model itself or on the class of a module inside it, model.parameters() is asked.
-PyObject *module_base() {   // torch.nn.Module (kept for good)
-    static PyObject *base = py::object(py::module_::import("torch.nn").attr("Module")).release().ptr();
-    return base;
-}
 bool walk_parameters(PyObject *module, std::unordered_set<PyObject *> &modules, const std::function<void(PyObject *)> &visit) {
     if (!modules.insert(module).second) return true;
     static PyObject *named_modules = PyUnicode_InternFromString("named_modules");

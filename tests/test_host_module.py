@@ -141,3 +141,58 @@ def test_foreign_gradients_are_those_of_the_models_own_traversal(which):
     want = [p.grad for p in params if id(p) not in owned and p.grad is not None]
     got = _n.host().foreign_grads(model, owned)
     assert [id(g) for g in got] == [id(g) for g in want]
+
+
+class _Mlp(torch.nn.Module):
+    def __init__(self, make):
+        super().__init__()
+        self.gate_proj, self.up_proj, self.down_proj = make(), make(), make()
+
+
+class _Property(torch.nn.Linear):
+    @property
+    def weight(self):
+        return self._parameters["weight"] * 2
+
+
+class _OwnAccess(torch.nn.Linear):
+    def __getattr__(self, name):
+        return torch.ones(1) if name == "weight" and "made" in self.__dict__ else super().__getattr__(name)
+
+
+def _own_access():
+    lin = _OwnAccess(3, 2)
+    lin.made = True
+    return lin
+
+
+def _shadowed():
+    lin = torch.nn.Linear(3, 2)
+    lin.__dict__["weight"] = torch.zeros(2, 3)
+    return lin
+
+
+@pytest.mark.parametrize("make", [lambda: torch.nn.Linear(3, 2), _own_access, _shadowed,
+                                  lambda: torch.nn.utils.parametrize.register_parametrization(torch.nn.Linear(3, 2), "weight",
+                                                                                              torch.nn.Identity())],
+                         ids=["plain", "own_access", "on_the_object", "parametrized"])
+def test_expert_weights_are_what_attribute_access_gives(make):
+    experts = torch.nn.ModuleList([_Mlp(make), _Mlp(lambda: torch.nn.Linear(3, 2)), _Mlp(make)])
+    got = _n.host().expert_parameters(experts)
+    want = [getattr(e, n).weight for e in experts for n in ("gate_proj", "up_proj", "down_proj")]
+    assert len(got) == 9 and all(torch.equal(a, b) for a, b in zip(got, want))
+    missing = torch.nn.ModuleList([_Mlp(torch.nn.Identity)])
+    with pytest.raises(AttributeError, match="weight"):
+        _n.host().expert_parameters(missing)
+
+
+def test_expert_weights_through_a_property():
+    def make():
+        lin = _Property.__new__(_Property)
+        torch.nn.Module.__init__(lin)
+        lin._parameters["weight"] = torch.nn.Parameter(torch.randn(2, 3))
+        return lin
+    experts = torch.nn.ModuleList([_Mlp(make)])
+    got = _n.host().expert_parameters(experts)
+    for a, name in zip(got, ("gate_proj", "up_proj", "down_proj")):
+        assert torch.equal(a, getattr(experts[0], name)._parameters["weight"] * 2)
