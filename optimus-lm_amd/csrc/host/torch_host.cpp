@@ -360,6 +360,18 @@ int64_t shared_pitch(const MlpWeights &w) {
     return s;
 }
 
+// Operands that the expert kernels would misread: they trust shapes and device.
+void require_mlp_operands(const Tensor &x, const MlpWeights &w) {
+    const auto gate = w.gate.sizes();
+    if (gate.size() != 3 || x.dim() != 2 || x.size(1) != gate[2] || w.up.sizes() != gate ||
+        w.down.sizes() != at::IntArrayRef({gate[0], gate[2], gate[1]}))
+        throw NativeError("expert MLP: expected activations [rows, hidden], gate and up weights [experts, ffn, hidden] and down "
+                          "weights [experts, hidden, ffn]");
+    for (const Tensor *t : {&w.gate, &w.up, &w.down})
+        if (!t->is_cuda())
+            throw NativeError("the HIP kernels need device tensors (got CPU expert weights); there is no CPU fallback");
+}
+
 void gemm_dtype(const Tensor &a, const Tensor &b, const Tensor &c) {
     const auto dt = a.scalar_type();
     TORCH_CHECK_TYPE((dt == at::kBFloat16 || dt == at::kFloat) && b.scalar_type() == dt && c.scalar_type() == dt,
@@ -373,6 +385,7 @@ float *fpm(const Tensor &t) { return static_cast<float *>(ptr(t)); }
 // y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment; with x_rows the MLP input is x[x_rows]
 Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const int32_t *cum, const int32_t *x_rows,
                       int64_t rows, MlpState &s) {
+    require_mlp_operands(x, w);
     require_device(x);
     gemm_dtype(x, w.gate, w.up);
     gemm_dtype(x, w.gate, w.down);
@@ -467,6 +480,12 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
 // The routed half of a bf16 block: gather, weighted SwiGLU MLP, unweighted sum of a token's rows.
 Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const Index &ix, const MlpWeights &w,
                       const Tensor &residual, MlpState &s, Tensor &row_weights) {
+    require_mlp_operands(x, w);
+    if (rw.dim() != 2 || rw.size(0) != x.size(0)) throw NativeError("routing weights: expected [tokens, top_k]");
+    if (residual.defined()) {
+        if (residual.sizes() != x.sizes()) throw NativeError("residual: expected the shape of the hidden states");
+        require_bf16(residual);
+    }
     require_device(x);
     require_device(rw);
     require_device(residual);
@@ -696,6 +715,15 @@ void require_gate_shape(const Tensor &weight, const char *what) {
                           "); there is no library fallback");
 }
 
+// Operands that the gate's kernels would misread: they take both in one type and trust the shapes.
+void require_gate_operands(const Tensor &x, const Tensor &weight) {
+    TORCH_CHECK_TYPE(x.scalar_type() == weight.scalar_type() && (x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat),
+                     "router gate: activations and weight must both be bfloat16 or both float32 (got ", x.scalar_type(), ", ",
+                     weight.scalar_type(), ")");
+    if (x.dim() != 2 || weight.dim() != 2 || x.size(1) != weight.size(1))
+        throw NativeError("router gate: expected activations [tokens, hidden] and a weight [experts, hidden]");
+}
+
 Tensor gate_weight_grad(const Call &c, const Tensor &x, const Tensor &weight, Tensor dlogits) {
     require_gate_shape(weight, "gate weight gradient");
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
@@ -836,6 +864,7 @@ std::shared_ptr<RouterNode> router_node(const Tensor &x, const Tensor &weight) {
 // (logits float32, x)
 std::tuple<Tensor, Tensor> gate_logits(const Tensor &x, const Tensor &weight) {
     refuse_transforms({x, weight});
+    require_gate_operands(x, weight);
     Tensor logits;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -861,6 +890,7 @@ Tensor route_workspace(const Tensor &x, int64_t T, int64_t H, int64_t N) {
 std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
                                                          at::ScalarType out_dtype, bool one_pass, bool bf16_logits) {
     refuse_transforms({x, weight});
+    require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
     // Up to 2048 tokens the one-pass kernel has at most 64 blocks, each walking all of H: the projection split
     // over H and a routing launch behind it give the same bits (eight slices added in the one-pass order)
@@ -907,7 +937,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
 std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &weight, const Tensor &bias, int64_t n_group,
                                                  int64_t topk_group, int64_t top_k, bool renorm, double scale) {
     refuse_transforms({x, weight, bias});
+    require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0);
+    TORCH_CHECK_TYPE(bias.scalar_type() == at::kFloat, "router bias must be float32 (got ", bias.scalar_type(), ")");
+    if (bias.numel() != N) throw NativeError("router bias: expected one value per expert");
     Tensor logits, weights, experts;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -1118,6 +1151,8 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
                    bool has_shared, const std::optional<Tensor> &one) {
     refuse_transforms({x, rw, residual.value_or(Tensor())});
     refuse_transforms(leaves);
+    if (experts.dim() != 2 || x.dim() != 2 || experts.size(0) != x.size(0) || rw.sizes() != experts.sizes())
+        throw NativeError("expected hidden states [tokens, hidden], and routing weights and expert indices [tokens, top_k]");
     const Call c = begin_call();
     Index ix;
     rw = rw.contiguous();
@@ -1181,6 +1216,7 @@ struct MergedNode : HostNode {
 
 // (y, cum, g, u, h) of the expert MLPs; `x_rows`: they read x through it
 std::vector<Tensor> merged_mlp_state(const Tensor &x, Tensor cum, const MlpWeights &w, const Tensor &x_rows) {
+    require_mlp_operands(x, w);
     const Call c = begin_call();
     MlpState s;
     require_device(x);
@@ -1267,6 +1303,12 @@ struct CombineNode : HostNode {      // saves y, rw, sel, in, out
 Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const Tensor &sel, const Tensor &in,
                const Tensor &out, const std::optional<Tensor> &residual) {
     refuse_transforms({y, rw_in, residual.value_or(Tensor())});
+    if (y.dim() != 2 || rw_in.dim() != 2 || cum_ep.numel() != rw_in.size(0) + 1)
+        throw NativeError("combine: expected expert outputs [rows, hidden], routing weights [tokens, top_k], tokens + 1 offsets");
+    if (residual) {
+        if (residual->sizes() != at::IntArrayRef({rw_in.size(0), y.size(1)})) throw NativeError("combine: expected a residual [tokens, hidden]");
+        TORCH_CHECK_TYPE(residual->scalar_type() == y.scalar_type(), "combine: the residual must have the expert outputs' type");
+    }
     Tensor final, rw = rw_in;
     {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -95,6 +95,26 @@ def test_the_functions_are_autograd_functions():
         assert "forward" in vars(cls) and "backward" in vars(cls), name
 
 
+@pytest.mark.parametrize("name,changes", [
+    ("gate_logits", dict(x=lambda t: t.float())), ("gate_logits", dict(weight=lambda t: t.float())),
+    ("gate_logits", dict(weight=lambda t: t[:, :8])), ("gate_logits", dict(x=lambda t: t[0])),
+    ("route_softmax", dict(x=lambda t: t.float())), ("route_softmax", dict(weight=lambda t: t[:, :8].contiguous())),
+    ("route_sigmoid", dict(weight=lambda t: t.float())), ("route_sigmoid", dict(bias=lambda t: t.double())),
+    ("route_sigmoid", dict(bias=lambda t: t[:2])),
+    ("moe_experts", dict(experts=lambda t: t[:2])), ("moe_experts", dict(rw=lambda t: t[:, :1])), ("moe_experts", dict(x=lambda t: t[:2])),
+    ("merged_mlp", dict(x=lambda t: t[:, :8])), ("merged_mlp", dict(up=lambda t: t[:1])),
+    ("merged_mlp", dict(down=lambda t: t.transpose(1, 2))), ("merged_mlp", dict(gate=lambda t: t[:, :4])),
+    ("combine", dict(cum_ep=lambda t: t[:-1])), ("combine", dict(residual=lambda t: t[:, :8])),
+    ("combine", dict(residual=lambda t: t.float())), ("combine", dict(rw=lambda t: t[0]))])
+def test_operands_that_a_kernel_would_misread_are_refused(name, changes):
+    """Before anything is launched, whatever the device."""
+    call, _ = _calls()[name]
+    t = _tensors()
+    t.update({k: f(t[k]) for k, f in changes.items()})
+    with pytest.raises((_n.NativeLibraryError, TypeError), match="expected|must"):
+        call(t)
+
+
 @pytest.mark.parametrize("G,I,H", [(32, 2048, 7168), (32, 256, 1024), (1, 8, 8)])
 def test_window_activations_sized_by_a_bound_are_limited(G, I, H):
     """64 MB while nothing is kept for a backward; with one, also a 32nd of the layer's expert weights."""
