@@ -299,7 +299,13 @@ struct Index {
             row_weights = reinterpret_cast<const float *>(sel + TK);
         } else {
             cum = iptr(owners[0]); cum_ep = iptr(owners[1]); in = iptr(owners[2]); out = iptr(owners[3]); sel = iptr(owners[4]);
+            row_weights = nullptr;
         }
+    }
+    Index without_arrays() const {  // what a node keeps beside the saved owners: no pointer outlives the forward pass
+        Index ix;
+        ix.NR = NR; ix.T = T; ix.TK = TK; ix.rows = rows; ix.bound = bound; ix.expected = expected;
+        return ix;
     }
     const int32_t *cum = nullptr, *cum_ep = nullptr, *in = nullptr, *out = nullptr, *sel = nullptr;
     const float *row_weights = nullptr;   // the routing weight of every sorted row (one-buffer form only)
@@ -980,7 +986,7 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
 // The expert half of a bf16 block (see routed_forward), with an optional residual or shared expert.
 // Inputs in order: hidden_states, routing_weights, residual, routed leaves, shared leaves.
 struct RoutedNode : HostNode {
-    Index ix;                        // (without its owners)
+    Index ix;                        // (without its arrays)
     ExpertWeights routed, shared;
     bool has_residual = false, has_shared = false;
     std::string name() const override { return "OptimusRoutedExpertsBackward"; }
@@ -1054,8 +1060,7 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
         for (const Tensor &t : ix.owners) node->save(t);
         node->routed = node->save_weights(routed, merged, w);
         if (has_shared) node->shared = node->save_weights(shared, true, ws);
-        ix.owners.clear();
-        node->ix = ix;
+        node->ix = ix.without_arrays();
         node->has_residual = residual_in.defined();
         node->has_shared = has_shared;
         torch::autograd::set_history(final, node);
