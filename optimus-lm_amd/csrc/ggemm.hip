@@ -1,22 +1,40 @@
 // Grouped expert GEMMs on bf16 MFMA (v_mfma_f32_32x32x16_bf16), fp32 accumulation.
 //
-// One kernel template covers every product of the merged MLP.  An output tile BM x BN is
-// computed by WAVES_M x WAVES_N wavefronts; each wavefront owns a (BM/WAVES_M) x (BN/WAVES_N)
-// sub-tile as a grid of 32x32 MFMA accumulators.  Operands are staged through LDS in steps of
-// 64 along the contraction index c with direct global->LDS loads (global_load_lds_dwordx4: no
-// register staging, no ds_write), two LDS stages, one barrier per step: the loads of step s+1
-// are in flight while step s is multiplied.
+// One kernel template covers every product of the merged MLP.  An output tile of 256x256 (8 wavefronts) or 128x128
+// (4) is worked by a grid of wavefronts two high; each has 32x32 MFMA accumulators in two columns.  Operands are
+// staged through LDS in steps of 64 along the contraction index c with direct global->LDS loads
+// (global_load_lds_dwordx4: no register staging, no ds_write), two stages.
 //
 // An operand is either
 //   CONTIG  — stored [row][c] with c contiguous (activations in fwd/dgrad, weights in fwd):
-//             LDS keeps 128-byte rows with the 16-byte chunks XOR-permuted per row; a fragment
-//             is one ds_read_b128 per lane;
+//             fragments are one ds_read_b128 per lane;
 //   STRIDED — stored [c][row] with row contiguous (weights in dgrad, both operands in wgrad):
-//             LDS keeps the tile as it lies in memory (chunks XOR-permuted per c-row); fragments
-//             come from the gfx950 transposing LDS read (ds_read_b64_tr_b16), two per lane.
-// A direct load writes LDS at (wave-uniform base + lane*16), so the permutation is applied by
-// choosing which global chunk each lane fetches.  The per-lane order of the 8 contraction
-// indices is the same for both kinds, so they can be mixed in one MFMA.
+//             fragments come from the gfx950 transposing LDS read (ds_read_b64_tr_b16), two per lane.
+// A stage is made of units of 8 KB: 64 rows x 64 c with 128-byte rows (CONTIG), or 64 c x 64 rows with 128-byte c-rows
+// (STRIDED), their 16-byte chunks XOR-permuted so that fragment reads meet no bank conflict.  A direct load writes LDS
+// at (wave-uniform base + lane*16), so the permutation is applied by choosing which global chunk each lane fetches.
+// The per-lane order of the 8 contraction indices is the same for both kinds, so they can be mixed in one MFMA.
+//
+// Main loop.  What bounds a step is how long its loads have to arrive.  With one barrier a step, that waits for all of
+// them, they have 0.6 to 0.9 of a step, and a step of the 256x256 tile took 1.5 us at full clock where its MFMAs take
+// 0.85; the 128x128 kernels, two blocks per CU, spent three quarters of their time waiting.  So a step's buffers are
+// given back piecemeal.  A wavefront keeps all of its B fragments of a step in registers (64 c x 64 columns) and works
+// through the row units of A one after the other (a phase: 8 MFMAs); it reads the fragments of the next phase, and in
+// the later phases B of the next step, under the MFMAs of this one.  Two barriers a step, P in the middle and Q at its
+// end, separate three groups of loads:
+//   after Q(t-1)  B of step t was read during step t-1, as was A's first unit: both are loaded for step t+2, and
+//                 (256x256) A's last unit, free since Q(t-1), for step t+1;
+//   after P(t)    A's remaining units of step t are free: loaded for step t+2.
+// A wavefront passes P and Q once all but its 8 youngest loads have landed (a whole step's worth), so every load has 1
+// to 1.5 steps.  The waits are written as assembly, and so are the loads: with the builtin the compiler waits for every
+// load in flight before a barrier, since it cannot tell which LDS bytes they will write.
+// Measured on one box against the single-barrier loop, us: 3001 tokens, hidden 1000, ffn 712, 12 experts, top-3
+// (128x128): down 32.6 -> 28.6, gate/up input gradient 55.7 -> 46.8, weight gradients 34 -> 31; decode of 37 tokens,
+// 64 experts of 2048/1024, 112.7 -> 104.4 and 57.0 -> 50.8 (that loop with its operands staged through registers two
+// steps ahead); 32 experts of 7168/2048 with 0 to 2849 rows (256x256): gate+up 967 -> 859, gate/up input gradient 959
+// -> 886; 64 experts of 2048/1024 with 2048 rows, where the power limit sets the rate, 1020 -> 1004 and 521 -> 518.
+//
+// A tile's rows are worked in units of 64 (32 per wavefront row), and units past the expert's last row cost no MFMA.
 //
 // Variable rows per expert: the M extent of fwd/dgrad is cut into tiles per expert.  Each block
 // scans the device-resident cum_token_counts once into an LDS table (row tiles up to and including
@@ -33,6 +51,7 @@
 // combine (the SwiGLU epilogue scales h by the weight of its row; the SwiGLU-backward epilogue
 // scales dh by it and produces the per-row sums that make up the weight's gradient).
 #include "common.h"
+#include <type_traits>
 
 namespace {
 
@@ -53,16 +72,8 @@ enum {
 };
 
 constexpr int BK = 64;  // contraction step, elements
-// Shares (in eighths) of a step's direct loads issued after the barrier / with 16-slices 0, 1, 2 of
-// the step.  Forward and input-gradient products (row-major activations): the A loads right after
-// the barrier, the B loads behind the first MFMAs.  Weight gradients (both operands read along the
-// contraction rows): the A loads behind the first MFMAs, the B loads one slice later.  Measured per
-// kernel on one box: the weight gradients gain 4 % with their split and the others lose 1-2 % with
-// it; an even spread over the step, everything in one place, or cutting through the A loads are
-// all 2-7 % worse on the whole layer.
-constexpr int LD_SHARE_T = 4, LD_SHARE_0 = 4, LD_SHARE_1 = 0, LD_SHARE_2 = 0;       // fwd / dgrad
-constexpr int LDW_SHARE_T = 0, LDW_SHARE_0 = 4, LDW_SHARE_1 = 4, LDW_SHARE_2 = 0;   // wgrad
 constexpr int NUM_XCD = 8;
+constexpr int QUEUE_PITCH = 32;   // ints between the tile counters of two XCDs: a 128-byte line each
 
 struct GemmParams {
     // operands; for the two-phase products (gate+up) index 1 is the second pair
@@ -85,19 +96,13 @@ struct GemmParams {
     int n_cols;                 // output columns (fwd/dgrad) — tiles along N = n_cols / BN_OUT
     int kc;                     // contraction length per phase (fwd/dgrad), multiple of 8
     int phases;                 // 1 or 2
-    int m_tiles_max;            // fwd/dgrad: upper bound on row tiles
-    int total_tiles;            // logical tiles of the launch (the blocks loop over them)
+    int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert
+    int32_t *queue;             // null, or NUM_XCD counters QUEUE_PITCH apart, zero before the launch
 };
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
 typedef __attribute__((address_space(3))) void *lds_void_ptr;
-typedef const __attribute__((address_space(1))) void *glb_void_ptr;
-
-// 16 bytes global -> LDS; LDS address = lds_base (wave-uniform) + lane*16.
-__device__ __forceinline__ void load16_to_lds(const void *gptr, char *lds_base) {
-    __builtin_amdgcn_global_load_lds((glb_void_ptr)gptr, (lds_void_ptr)lds_base, 16, 0, 0);
-}
 
 // A block-uniform 64-bit value, pinned to scalar registers (the compiler cannot always prove that
 // per-tile state carried around the tile loop is uniform).
@@ -107,47 +112,12 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// ---- CONTIG tile: R rows x 64 c; 128-byte rows; chunk position = chunk ^ swz(row) ----------
-// (row >> 1) & 7: measured conflict-free for ds_read_b128 with 32 consecutive rows per half-wave
-// (counter SQ_LDS_BANK_CONFLICT = 0, 4 cycles per read); period 16, so rows 32 apart share it.
+// CONTIG unit (64 rows x 64 c, 128-byte rows): chunk position = chunk ^ swz(row), measured conflict-free for
+// ds_read_b128 with 32 consecutive rows per half-wave; period 16, so rows 32 apart share it.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
-__device__ __forceinline__ int contig_off(int row, int ch) { return row * 128 + ((ch ^ swz(row)) << 4); }
-
-// The chunk (8 contraction indices) that lane `lane` of direct load `grp` of a CONTIG tile fetches: the
-// load fills LDS rows grp*8 .. grp*8+7, lane -> (row grp*8 + lane/8, position lane%8 = chunk ^ swz(row)).
-__device__ __forceinline__ int contig_chunk(int grp, int lane) { return (lane & 7) ^ ((grp * 4 + (lane >> 4)) & 7); }
-
-// ---- STRIDED tile: 64 c-rows x R rows-of-the-operand; R*2-byte c-rows; chunk position =
-//      chunk ^ ((crow & 3) << 2): the four c-rows a transposing read touches land in four
-//      different 64-byte bank windows -------------------------------------------------------
-template <int R> __device__ __forceinline__ int strided_off(int crow, int ch) {
-    return crow * (R * 2) + ((ch ^ ((crow & 3) << 2)) << 4);
-}
-
-template <int KIND, int R> struct TileBytes { static constexpr int value = R * 128; };  // both kinds
-
-__device__ __forceinline__ bf16x8 lds_read_frag_contig(const char *tile, int row, int ch) {
-    const u32x4 v = *reinterpret_cast<const u32x4 *>(tile + contig_off(row, ch));
-    return __builtin_bit_cast(bf16x8, v);
-}
-
-// Transposing read: lanes 4r..4r+3 of a 16-lane group address c-row r, 4 consecutive rows-of-the-
-// operand each; lane i receives operand row i at c-rows 0..3.
-template <int R>
-__device__ __forceinline__ bf16x8 lds_read_frag_strided(const char *tile, int c0, int m0, int lane) {
-    const int i = lane & 15;
-    const int r = i >> 2, q = i & 3;
-    const int mb = ((lane >> 4) & 1) * 16;
-    const int g2 = lane >> 5;
-    const int m = m0 + mb + 4 * q;
-    const int cr = c0 + 8 * g2 + r;  // (cr & 3) == (cr + 4) & 3
-    const char *p = tile + strided_off<R>(cr, m >> 3) + (m & 7) * 2;
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 4 * R * 2));
-    typedef __attribute__((ext_vector_type(8))) short s16x8;
-    s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(bf16x8, v);
-}
+// STRIDED unit (64 c-rows x 64 columns, 128-byte c-rows): the four c-rows of a transposing read, two of which share a
+// 256-byte bank row, land in four different 64-byte windows
+__device__ __forceinline__ int unit_swz(int crow) { return ((crow >> 1) & 1) << 2; }
 
 __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
     typedef __attribute__((ext_vector_type(2))) float f32x2;
@@ -278,158 +248,112 @@ __device__ __forceinline__ void wgrad_xcd_run(const int32_t *cum, int n_experts,
     if (xcd == 0) lo = 0;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE,
-          bool ROWW = false, bool ACCUM = false, bool KTAIL = false, bool REGLOAD = false>
-// (second launch bound: two wavefronts per SIMD, i.e. at most 256 registers, for the 128x128 tile, whose two
-// blocks per CU depend on it; the 256x256 tile's 8 wavefronts imply it already)
-__global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
-    static_assert(!ACCUM || EPI == EPI_WGRAD, "only the weight gradient adds into its output");
-    // KTAIL: forward / input-gradient products whose contraction length is not a multiple of 64 (the last
-    // step of a phase is partial); a kernel of its own, so that the others carry none of its handling
-    static_assert(!KTAIL || (BM == 128 && EPI != EPI_WGRAD && AKIND == CONTIG), "partial last contraction step: 128x128 forward / input gradient");
-    // REGLOAD: forward / input-gradient products whose experts hold few rows, where a launch is a stream of
-    // weights that are used once.  Both operands go through registers instead of direct global->LDS loads: the
-    // weights (B) are fetched TWO contraction steps ahead into two register sets, the activations (A, which
-    // mostly hit in L2) one step ahead, and are written to the LDS stage that has become free before the
-    // barrier that ends a step.  With direct loads the look-ahead cannot exceed one step: the compiler
-    // waits for every outstanding load before a barrier, since it cannot tell which LDS bytes a direct load
-    // in flight will write.  Same LDS layout, same order of the sums: bit-identical results.
-    static_assert(!REGLOAD || (BM == 128 && EPI != EPI_WGRAD && !KTAIL), "register-staged operands: 128x128 forward / input gradient");
+// 16 bytes per lane global -> LDS at lds_base + OFS + lane * 16.  Written as assembly so that the compiler neither
+// waits for such a load nor takes it for an LDS access: the main loop's own waits and barriers order them.
+// dma16_if: nothing is loaded with fewer than two steps `left` (block-uniform); the branch lies inside the assembly, so that a step stays one block
+// for the compiler's scheduler.
+template <int OFS> __device__ __forceinline__ void dma16(const void *base, uint32_t lane_bytes, uint32_t lds_base) {
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(lds_base), "v"(lane_bytes), "s"(base), "n"(OFS) : "scc");
+}
+template <int OFS>
+__device__ __forceinline__ void dma16_if(int left, const void *base, uint32_t lane_bytes, uint32_t lds_base) {
+    asm volatile("s_cmp_lt_i32 %4, 2\n\ts_cbranch_scc1 .Lom_skip%=\n\ts_add_u32 m0, %0, %3\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %1, %2\n.Lom_skip%=:"
+                 :: "s"(lds_base), "v"(lane_bytes), "s"(base), "n"(OFS), "s"(left) : "scc");
+}
+// This wavefront's direct loads but the N youngest have landed, and its LDS reads are back.
+template <int N> __device__ __forceinline__ void wait_loads(uint32_t lds) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N), "s"(lds) : "memory");
+}
+// The same inside a tile's main loop, by the number of steps that follow: N2 with two or more, N1 with one, else 0.
+template <int N2, int N1> __device__ __forceinline__ void wait_step_loads(int left, uint32_t lds) {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_cmp_ge_i32 %2, 2\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(%1)\n\t"
+                 "s_cmp_ge_i32 %2, 1\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(0)\n.Lom_wait%=:"
+                 :: "n"(N2), "n"(N1), "s"(left), "s"(lds) : "memory", "scc");
+}
+__device__ __forceinline__ void block_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int V> using IntC = std::integral_constant<int, V>;
+
+// EDGE: output extents and contraction lengths that are any multiple of 8: the last tile along an extent and the last
+// step of a phase may be partial (loads past them are clamped, A is zeroed, stores are masked).  The 256x256 kernels are
+// launched on whole tiles and steps only and carry none of that.
+// (second launch bound: two wavefronts per SIMD, i.e. at most 256 registers, for the 128x128 tile, whose two blocks per
+// CU depend on it; the 256x256 tile's 8 wavefronts imply it already)
+template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool ACCUM = false,
+          bool EDGE = false>
+__global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
+    constexpr int BN = BM, WAVES_N = BN / 64, NW = 2 * WAVES_N;
+    constexpr int TM = BM / 64, TN = 2;     // row units of a tile, accumulators of a wavefront in each
     static_assert(GATHER == GATHER_NONE || (GATHER == GATHER_A && AKIND == CONTIG && EPI != EPI_WGRAD) ||
                       (GATHER == GATHER_B && BKIND == STRIDED && EPI == EPI_WGRAD) ||
                       (GATHER == GATHER_WA && AKIND == STRIDED && EPI == EPI_WGRAD), "gather variants");
+    static_assert(!ACCUM || EPI == EPI_WGRAD, "only the weight gradient adds into its output");
     static_assert(!ROWW || EPI == EPI_SWIGLU || EPI == EPI_SWIGLU_BWD, "row weights belong to the SwiGLU epilogues");
-    constexpr int NW = WAVES_M * WAVES_N;
-    // The 128x128 tile takes output extents that are any multiple of 8: its last tile along an
-    // extent may be partial (loads past the extent are clamped, stores masked).  The 256x256 tile is
-    // only launched on whole tiles and carries none of that.
-    constexpr bool EDGE = BM == 128;
-    // Contraction steps are taken in pairs (static stage names).  The weight gradient, whose step
-    // count follows the expert's rows, and the 128x128 tile end an odd count with a single step; the
-    // 256x256 forward / input-gradient kernels are only launched on even counts.
-    constexpr bool ANY_STEPS = EPI == EPI_WGRAD || EDGE;
-    constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // wavefront sub-tile
-    constexpr int TM = WM / 32, TN = WN / 32;            // 32x32 accumulators per wavefront
-    constexpr int A_BYTES = TileBytes<AKIND, BM>::value;
-    constexpr int B_BYTES = TileBytes<BKIND, BN>::value;
-    constexpr int A_LOADS = BM / 8 / NW;                 // direct loads per wavefront per step
-    constexpr int B_LOADS = BN / 8 / NW;
-    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile/wave mismatch");
-    // two statically distinct stages: the compiler can then tell that a fragment read of one
-    // stage does not depend on the loads in flight to the other
-    __shared__ __attribute__((aligned(1024))) char stage0[A_BYTES + B_BYTES];
-    __shared__ __attribute__((aligned(1024))) char stage1[A_BYTES + B_BYTES];
-    // wgrad through an index: the current expert's slice of the index is kept in LDS (filled when
-    // the block moves to another expert) for the look-up that a tile's first loads wait for; the
-    // look-ups inside the main loop run one step ahead and go to global memory (reading them from
-    // LDS measured 20 % slower: they queue with the fragment reads)
+    constexpr bool WGRAD = EPI == EPI_WGRAD;
     constexpr bool GATHER_W = GATHER == GATHER_B || GATHER == GATHER_WA;
+    constexpr int UNIT = 8192;             // bytes of an operand unit: 64 rows (CONTIG) or 64 columns (STRIDED) x 64 c
+    constexpr int UA = TM, UB = BN / 64;   // units of a step
+    constexpr int L = 8 / NW;              // direct loads per wavefront per unit
+    constexpr int A_STAGE = UA * UNIT, B_STAGE = UB * UNIT;
+    constexpr int B0 = 2 * A_STAGE;        // A of even and odd steps, then B of even and odd steps
+    __shared__ __attribute__((aligned(1024))) char lds[2 * A_STAGE + 2 * B_STAGE];
     constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
     __shared__ int idx_cache[IDX_CACHE];
     int cached_expert = -1;
-    __shared__ int tile_end[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
-    __shared__ int seg[EPI == EPI_WGRAD ? 1 : MAX_EXPERTS + 1];
-    // A 256-row tile with at most 128 rows is half a tile's work: its lower four wavefronts (one per SIMD) do
-    // all of it, the upper four only fetch their share of B.  Its steps stay bound by the latency of its
-    // weights.  Dealing such tiles out after the whole ones, so that a launch's last round is one of halves,
-    // is slower: away from their expert's whole tiles they fetch its weights once more (forward of 3000 tokens,
-    // 64 experts of 2048/1024, 399 -> 445 us a pass, 4096 tokens 529 -> 541, a step of 2048 tokens 1081 -> 1131).
-    constexpr bool HALVES = BM == 256 && EPI != EPI_WGRAD;
+    __shared__ int tile_end[WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
+    __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];
 
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);   // the same value in a scalar register
 
     // ---- per-tile state (set by setup_tile) ---------------------------------------------------
-    int expert = 0, row_begin = 0, row_end = 0;  // fwd/dgrad: rows of this tile's expert segment
-    int n0 = 0;                                  // first output column (LDS B row 0)
-    int c_begin = 0, c_len = 0;                  // contraction range
-    int steps_per_phase = 0, total_steps = 0;
-    int loop_steps = 0;   // steps the main loop takes (see setup_tile)
-    // Tiles that run together on an XCD share operand slices.  Walking the contraction index from
-    // 0 in all of them makes them ask L2 for the same lines at the same time, and all wait for the
-    // same fill; a small per-tile offset `rot` lets one tile fetch a slice and the sharers hit it.
-    int rot = 0;
-    auto rotated = [&](int sp) {   // sp in [0, steps_per_phase)
-        const int r = sp + rot;
-        return r >= steps_per_phase ? r - steps_per_phase : r;
-    };
-
-    // ---- per-lane source offsets of the direct loads (elements, without the c0 term) ------------
-    // CONTIG : lane -> (row = group*8 + lane/8, chunk = (lane%8) ^ swz(row))
-    // STRIDED: lane -> (crow = group*(64/CPR) + lane/CPR, chunk = (lane%CPR) ^ ((crow&3)<<2))
-    // A load's address is (operand pointer + block-uniform 64-bit tile base) + a 32-bit per-lane
-    // offset: the wide part stays in scalar registers (the load takes a scalar base and a 32-bit
-    // vector offset), so operands of any size cost no vector arithmetic.  The per-lane part covers
-    // one tile (BM rows, or 64 contraction rows) — except for rows fetched through an index, whose
-    // lane offset is index * pitch: such a source must span < 2^31 elements (checked on the host).
-    int a_off[A_LOADS], b_off[B_LOADS];
-    int64_t a_base = 0, b_base = 0;   // elements, block-uniform
-    int a_crow[A_LOADS];  // STRIDED A in wgrad: c-row of the lane's slot (for the zero fill)
-    int b_crow[B_LOADS];
-    int b_src[GATHER == GATHER_B ? B_LOADS : 1];   // GATHER_B: source rows of the next B loads
-    int a_src[GATHER == GATHER_WA ? A_LOADS : 1];  // GATHER_WA: source rows of the next A loads
-#pragma unroll
-    for (int i = 0; i < A_LOADS; i++) {
-        constexpr int CPR = BM / 8;
-        a_crow[i] = (AKIND == CONTIG) ? 0 : (wave * A_LOADS + i) * (64 / CPR) + lane / CPR;
-    }
-#pragma unroll
-    for (int i = 0; i < B_LOADS; i++) {
-        constexpr int CPR = BN / 8;
-        const int grp = wave * B_LOADS + i;
-        b_crow[i] = (BKIND == CONTIG) ? 0 : grp * (64 / CPR) + lane / CPR;
-    }
-
+    int expert = 0, row_begin = 0, row_end = 0, n0 = 0, c_begin = 0, c_len = 0;
+    int steps_per_phase = 0, c_wrap = 0, n_steps = 0, rot = 0;
+    int active = TM;      // row units that hold rows of the expert
+    // the slot of this wavefront's direct load l of a unit: row (CONTIG) or contraction row (STRIDED) and chunk
+    auto slot = [&](int l) { return (wave * L + l) * 8 + (lane >> 3); };
+    uint32_t a_off[AKIND == CONTIG ? UA : 1][L];   // bytes from the step's base: CONTIG, the row of each unit
+    uint32_t b_off[EDGE ? UB : 1][L];         // CONTIG as above; STRIDED, the column
+    const char *a_tile[2] = {}, *b_tile[2] = {};   // base addresses of the tile's operands (two phases), block-uniform
+    int tail_c0 = -1;     // first contraction index of the partial step, if the tile has one
+    int src[GATHER_W ? 3 : 1][L];             // GATHER_W: source rows of this lane's slots, steps t, t + 1, t + 2
     const int lda32 = static_cast<int>(p.lda), ldb32 = static_cast<int>(p.ldb);
-    // GATHER_B: the B rows that contraction step `step` needs, looked up one step ahead of the
-    // loads that use them (plain loads: they land before the next wait for the direct loads).
-    auto index_of = [&](int step, int c0, int c) -> int {   // c0: the step's first row (block-uniform)
-        if (step == 0 && c0 + BK <= IDX_CACHE) return idx_cache[GATHER_W ? c : 0];
-        return p.row_index[c_begin + c];
-    };
-    auto load_b_src = [&](int step) {
-        if (GATHER != GATHER_B || step >= loop_steps) return;
-        const int c0 = (step < steps_per_phase ? rotated(step) : step) * BK;
-        // One 4-byte read per B load (measured faster than one read per wavefront plus lane
-        // permutes, which queue behind the fragment reads).  Kept as read: any arithmetic on the
-        // value here would put the wait for it here too.
+    constexpr bool TWO_PHASE = EPI == EPI_STORE && BKIND == STRIDED;   // the merged MLP's dx = dg Wg + du Wu
+    const int64_t b_unit = static_cast<int64_t>(EPI == EPI_SWIGLU ? 32 : 64) * p.ldb * 2;   // CONTIG: bytes between units
+    const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)lds));
+    const uint32_t wave_lds = __builtin_amdgcn_readfirstlane(lds_addr + wave * (L * 1024));
+
+    // Contraction steps run from `rot` to the end of the range and on from its start (both phases alike).
+    auto next_c0 = [&](int c0) { return c0 + BK >= c_wrap ? 0 : c0 + BK; };
+    // GATHER_W: the source rows of the step at c0; the first IDX_CACHE of an expert's rows come from LDS
+    auto look_up = [&](int c0, int (&out)[L]) {
+        if (!GATHER_W) return;
 #pragma unroll
-        for (int i = 0; i < B_LOADS; i++) {
-            const int c = min(c0 + b_crow[i], c_len - 1);   // past the segment: any valid row (A is zeroed)
-            b_src[GATHER == GATHER_B ? i : 0] = index_of(step, c0, c);
+        for (int l = 0; l < L; l++) {
+            const int c = min(c0 + slot(l), c_len - 1);
+            if (c0 + BK <= IDX_CACHE) {
+                out[l] = idx_cache[c];
+            } else {   // (waited for here: at the join the compiler would wait for the direct loads too, on either path)
+                int v = p.row_index[c_begin + c];
+                asm volatile("" : "+v"(v));
+                out[l] = v;
+            }
         }
     };
 
-    auto load_a_src = [&](int step) {   // GATHER_WA: the same for the A rows
-        if (GATHER != GATHER_WA || step >= loop_steps) return;
-        const int c0 = (step < steps_per_phase ? rotated(step) : step) * BK;
-#pragma unroll
-        for (int i = 0; i < A_LOADS; i++) {
-            const int c = min(c0 + a_crow[i], c_len - 1);   // past the segment: any valid row (zeroed in LDS)
-            a_src[GATHER == GATHER_WA ? i : 0] = index_of(step, c0, c);
-        }
-    };
-
-    // Which tile `logical` is, and the load offsets for it.  False: the tile lies past the last
-    // row block (the launch sizes the tile count from an upper bound on the routed rows).
     auto setup_tile = [&](int logical) -> bool {
-        int rot_a, rot_b;  // position among the tiles sharing this tile's A / B operand
-        // lane-derived terms are recomputed per tile rather than kept live across the main loop
-        int lane_s = lane;
-        asm volatile("" : "+v"(lane_s));
-        if (EPI == EPI_WGRAD) {
-            // tiles are numbered expert-major: an XCD works on whole experts (all tiles of dW[g]
-            // share the expert's rows of both operands)
+        int rot_a, rot_b;
+        if (WGRAD) {
             const int tiles_n = (p.n_cols + BN - 1) / BN;
             expert = logical / p.tiles_e;
             const int tile = logical - expert * p.tiles_e;
             const int tm = tile / tiles_n, tn = tile % tiles_n;
             rot_a = tn; rot_b = tm;
-            row_begin = tm * BM;  // row of dW
-            row_end = 0;
+            row_begin = tm * BM;
+            row_end = p.kc;
             n0 = tn * BN;
             c_begin = p.cum[expert];
             c_len = p.cum[expert + 1] - c_begin;
@@ -439,12 +363,11 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
             const int tile_m = logical / tiles_n;
             const int tile_n = logical % tiles_n;
             rot_a = tile_n; rot_b = tile_m & 7;
-            if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane_s, expert, row_begin, row_end)) return false;
+            if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
             c_len = p.kc;
         }
-        // block-uniform values: keep them in scalar registers
         expert = __builtin_amdgcn_readfirstlane(expert);
         row_begin = __builtin_amdgcn_readfirstlane(row_begin);
         row_end = __builtin_amdgcn_readfirstlane(row_end);
@@ -452,399 +375,255 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         c_begin = __builtin_amdgcn_readfirstlane(c_begin);
         c_len = __builtin_amdgcn_readfirstlane(c_len);
         steps_per_phase = (c_len + BK - 1) / BK;
-        total_steps = steps_per_phase * p.phases;
-        loop_steps = ANY_STEPS ? total_steps : ((total_steps + 1) & ~1);
+        n_steps = steps_per_phase * p.phases;
         rot = (rot_a + rot_b) % (steps_per_phase > 0 ? steps_per_phase : 1);
+        c_wrap = steps_per_phase * BK;
+        tail_c0 = (WGRAD || EDGE) && c_wrap != c_len ? c_wrap - BK : -1;
+        active = WGRAD && !EDGE ? TM : min((row_end - row_begin + 63) >> 6, TM);
+        int lane_s = lane;
+        asm volatile("" : "+v"(lane_s));   // recomputed per tile, not kept across the main loop
+        const int ch8 = lane_s & 7;
 #pragma unroll
-        for (int i = 0; i < A_LOADS; i++) {
-            const int grp = wave * A_LOADS + i;
+        for (int l = 0; l < L; l++) {
+            const int r = (wave * L + l) * 8 + (lane_s >> 3);
             if (AKIND == CONTIG) {
-                const int row = grp * 8 + (lane_s >> 3);
-                const int ch = (lane_s & 7) ^ swz(row);
-                int m = row_begin + row;
-                if (m >= row_end) m = row_end - 1;  // rows past the segment: valid memory, result unused
-                if (GATHER == GATHER_A) m = p.row_index[m];
-                else m -= row_begin;                // the tile's first row is part of a_base
-                a_off[i] = m * lda32 + ch * 8;
-            } else {
-                constexpr int CPR = BM / 8;
-                const int ch = (lane_s % CPR) ^ ((a_crow[i] & 3) << 2);
-                // (a partial last tile: chunks past the extent re-read its last chunk; masked on store)
-                a_off[i] = EDGE ? min(row_begin + ch * 8, p.kc - 8) : row_begin + ch * 8;  // + (contraction row within the step) * lda per step
-            }
-        }
+                const int ch = ch8 ^ swz(r);
 #pragma unroll
-        for (int i = 0; i < B_LOADS; i++) {
-            const int grp = wave * B_LOADS + i;
-            if (BKIND == CONTIG) {
-                const int row = grp * 8 + (lane_s >> 3);
-                const int ch = (lane_s & 7) ^ swz(row);
-                // output columns past n_cols (a partial last column tile) re-read the last one; their
-                // results are masked on store
-                const int n_last = EDGE ? p.n_cols - 1 - n0 : BN;
-                if (EPI == EPI_SWIGLU) {
-                    // LDS rows alternate 32 gate rows / 32 up rows; the up matrix is B[1]
-                    const int blk = row >> 5;
-                    const int n = (blk >> 1) * 32 + (row & 31);
-                    b_off[i] = min(n, n_last) * ldb32 + ch * 8;
-                } else {
-                    b_off[i] = min(row, n_last) * ldb32 + ch * 8;
+                for (int u = 0; u < UA; u++) {
+                    int m = min(row_begin + u * 64 + r, row_end - 1);   // rows past the segment: valid memory, result unused
+                    if (GATHER == GATHER_A) m = p.row_index[m];
+                    else m -= row_begin;
+                    a_off[u][l] = (static_cast<uint32_t>(m) * lda32 + ch * 8) * 2u;
                 }
             } else {
-                constexpr int CPR = BN / 8;
-                const int ch = (lane_s % CPR) ^ ((b_crow[i] & 3) << 2);
-                const int col8 = EDGE ? min(ch * 8, p.n_cols - 8 - n0) : ch * 8;   // (partial last column tile, as above)
-                // fwd/dgrad: the lane's contraction row within a step never changes, so it is part of
-                // the offset; wgrad clamps the row into the expert's segment per step
-                b_off[i] = col8 + (EPI == EPI_WGRAD ? 0 : b_crow[i] * ldb32);
+                a_off[0][l] = (ch8 ^ unit_swz(r)) * 16;    // bytes of the column within the unit
+            }
+            if (BKIND == CONTIG) {
+                const int ch = ch8 ^ swz(r);
+                // EPI_SWIGLU: a unit holds 32 gate rows and the same 32 up rows (see B_first)
+                constexpr int PER_UNIT = EPI == EPI_SWIGLU ? 32 : 64;
+                const int n = EPI == EPI_SWIGLU ? (r & 31) : r;
+#pragma unroll
+                for (int u = 0; u < (EDGE ? UB : 1); u++)
+                    b_off[u][l] = (static_cast<uint32_t>(EDGE ? min(u * PER_UNIT + n, p.n_cols - 1 - n0) : n) * ldb32 + ch * 8) * 2u;
+            } else {
+                const int col = (ch8 ^ unit_swz(r)) * 8;
+#pragma unroll
+                for (int u = 0; u < (EDGE ? UB : 1); u++)
+                    b_off[u][l] = (EDGE ? min(u * 64 + col, p.n_cols - 8 - n0) : col) * 2;
             }
         }
-        // block-uniform parts of the addresses (scalar registers)
-        if (AKIND == CONTIG) a_base = GATHER == GATHER_A ? 0 : static_cast<int64_t>(row_begin) * p.lda;
-        else a_base = 0;   // wgrad: the contraction rows enter per step (step_base)
-        if (BKIND == CONTIG) b_base = expert * p.strideB + static_cast<int64_t>(n0) * p.ldb;
-        else b_base = (EPI == EPI_WGRAD ? 0 : expert * p.strideB) + n0;
+        const int64_t a_base = AKIND == CONTIG ? (GATHER == GATHER_A ? 0 : static_cast<int64_t>(row_begin) * p.lda)
+                                               : row_begin + (GATHER == GATHER_WA ? 0 : static_cast<int64_t>(c_begin) * p.lda);
+        const int64_t b_base = BKIND == CONTIG ? expert * p.strideB + static_cast<int64_t>(n0) * p.ldb
+                               : WGRAD ? n0 + (GATHER == GATHER_B ? 0 : static_cast<int64_t>(c_begin) * p.ldb)
+                                       : expert * p.strideB + n0;
+        // EPI_SWIGLU: LDS rows 0..31 of a unit are gate rows, 32..63 up rows; a wavefront's loads lie in one of the two
+        const uint16_t *B_first = EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? p.B[1] : p.B[0];
+        a_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(p.A[0] + a_base)));
+        b_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(B_first + b_base)));
+        if (TWO_PHASE) {
+            a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.A[1] : p.A[0]) + a_base)));
+            b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.B[1] : p.B[0]) + b_base)));
+        }
         if (GATHER_W && expert != cached_expert) {
-            // every wavefront is past the barrier that ends the previous tile's main loop, so no
-            // one still reads the cache; `expert` is block-uniform, so all take this branch together
+            // every wavefront is past the barrier that ends the previous tile's main loop, so no one still reads
+            // the cache; `expert` is block-uniform, so all take this branch together
             const int n_cached = min(c_len, IDX_CACHE);
             for (int i = tid; i < n_cached; i += NW * 64) idx_cache[GATHER_W ? i : 0] = p.row_index[c_begin + i];
             cached_expert = expert;
             __syncthreads();
         }
-        load_b_src(0);
-        load_a_src(0);
+        if (GATHER_W && n_steps > 0) {
+            const int c0 = rot * BK, c1 = next_c0(c0);
+            look_up(c0, src[0]);
+            look_up(c1, src[GATHER_W ? 1 : 0]);
+            look_up(next_c0(c1), src[GATHER_W ? 2 : 0]);
+        }
         return true;
     };
 
-    // Loads of contraction step `step` into `stage`.
-    // Loads [lo, hi) of the step's list (A loads first, then B loads); lo and hi are constants
-    // after unrolling.
-    u32x4 rb[REGLOAD ? 2 : 1][REGLOAD ? B_LOADS : 1];   // REGLOAD: B of steps s+1 and s+2 (set = step % 2)
-    u32x4 ra[REGLOAD ? A_LOADS : 1];                    //          A of step s+1
-    auto issue_part = [&](int step, char *stage, int lo, int hi) {
-        if (REGLOAD) return;                               // (no direct loads in these kernels)
-        if (step >= loop_steps) return;                    // nothing left to fetch for this tile
-        const int ph = (step >= steps_per_phase) ? 1 : 0;  // at most two phases
-        const int sp = step - ph * steps_per_phase;
-        int c0 = (sp < steps_per_phase ? rotated(sp) : sp) * BK;
-        if (!ANY_STEPS && c0 > c_len - BK) c0 = c_len - BK;
-        // KTAIL kernels take contraction lengths that are any multiple of 8: the last step of a phase
-        // may hold fewer than 64 indices.  Its loads past the end re-read the last valid 8 indices (c-row)
-        // instead, and the A slots they fill are zeroed in LDS before the step is multiplied (zero_tail).
-        const bool c_tail = KTAIL && c0 + BK > c_len;   // block-uniform
-        const int c_chunks = (c_len - c0) >> 3;                           // 8-index chunks the step holds
-        // first contraction row that this step's STRIDED loads may touch, folded into the scalar base
-        // (rows are clamped into the segment, so the base is clamped the same way)
-        const int c_lo = (EPI == EPI_WGRAD) ? max(min(c0, c_len - 1), 0) : c0;
-        const int64_t a_step = uniform64(a_base + ((AKIND == STRIDED && GATHER != GATHER_WA) ? static_cast<int64_t>(c_begin + c_lo) * p.lda : 0));
-        const int64_t b_step = uniform64(b_base + ((BKIND == STRIDED && GATHER != GATHER_B) ? static_cast<int64_t>(c_begin + c_lo) * p.ldb : 0));
-        const char *Ap = reinterpret_cast<const char *>((p.phases > 1 && ph ? p.A[1] : p.A[0]) + a_step);
-        const char *Bp = reinterpret_cast<const char *>(
-            ((EPI != EPI_SWIGLU && p.phases > 1 && ph) ? p.B[1] : p.B[0]) + b_step);
-        const char *Bup = reinterpret_cast<const char *>(p.B[1] + b_step);
-        char *sa = stage + wave * (A_LOADS * 1024);
-        char *sb = stage + A_BYTES + wave * (B_LOADS * 1024);
+    // ---- direct loads of one unit into the buffers of parity P; base: a_step / b_step of the unit's step -------
+    auto a_step = [&](int c0, int t) -> const char * {
+        const char *q = TWO_PHASE && t >= steps_per_phase ? a_tile[1] : a_tile[0];
+        if (GATHER == GATHER_WA) return q;
+        return q + (AKIND == CONTIG ? static_cast<uint64_t>(static_cast<uint32_t>(c0)) * 2 : static_cast<uint64_t>(static_cast<uint32_t>(c0)) * static_cast<uint32_t>(lda32 * 2));
+    };
+    auto b_step = [&](int c0, int t) -> const char * {
+        const char *q = TWO_PHASE && t >= steps_per_phase ? b_tile[1] : b_tile[0];
+        if (GATHER == GATHER_B) return q;
+        return q + (BKIND == CONTIG ? static_cast<uint64_t>(static_cast<uint32_t>(c0)) * 2 : static_cast<uint64_t>(static_cast<uint32_t>(c0)) * static_cast<uint32_t>(ldb32 * 2));
+    };
+    // bytes of the contraction row (STRIDED): rows past the range re-read its last row (A is zeroed there)
+    auto crow_bytes = [&](int c0, int l, int ld32, const int (&rows)[L], bool indexed) -> uint32_t {
+        if (indexed) return static_cast<uint32_t>(rows[l]) * (ld32 * 2u);
+        const uint32_t r = static_cast<uint32_t>(slot(l)) * (ld32 * 2u);
+        return WGRAD || EDGE ? min(r, static_cast<uint32_t>(min(c_len - 1 - c0, BK)) * (ld32 * 2u)) : r;
+    };
+    // CONTIG, a partial last step: its chunks past the end re-read the last one (A's are zeroed)
+    auto tail_bytes = [&](int c0, int l) -> uint32_t {
+        return EDGE ? max(((lane & 7) ^ swz(slot(l))) - (((c_len - c0) >> 3) - 1), 0) * 16 : 0;
+    };
+    auto issue_a = [&](int left, const char *base, int c0, auto par, auto unit, const int (&rows)[L]) {
+        constexpr int P = decltype(par)::value, U = decltype(unit)::value;
 #pragma unroll
-        for (int i = 0; i < A_LOADS; i++) {
-            if (i < lo || i >= hi) continue;
-            uint32_t off;  // bytes from the step's scalar base
-            if (AKIND == CONTIG) {
-                off = static_cast<uint32_t>(a_off[i] + c0) * 2u;
-                if (c_tail) off -= static_cast<uint32_t>(max(contig_chunk(wave_u * A_LOADS + i, lane) - (c_chunks - 1), 0)) * 16u;
-            } else {
-                int c = c0 + a_crow[i];
-                if (EPI == EPI_WGRAD) c = min(c, c_len - 1);  // stay in the segment; zeroed below
-                if (GATHER == GATHER_WA)
-                    off = static_cast<uint32_t>(a_off[i] + a_src[GATHER == GATHER_WA ? i : 0] * lda32) * 2u;
-                else
-                    off = static_cast<uint32_t>(a_off[i] + (c - c_lo) * lda32) * 2u;
-            }
-            load16_to_lds(Ap + off, sa + i * 1024);
-        }
-        if (hi >= A_LOADS && lo < A_LOADS) load_a_src(step + 1);   // this step's A loads are out
-#pragma unroll
-        for (int i = 0; i < B_LOADS; i++) {
-            if (A_LOADS + i < lo || A_LOADS + i >= hi) continue;
+        for (int l = 0; l < L; l++) {
             uint32_t off;
-            if (BKIND == CONTIG) {
-                off = static_cast<uint32_t>(b_off[i] + c0) * 2u;
-                if (c_tail) off -= static_cast<uint32_t>(max(contig_chunk(wave_u * B_LOADS + i, lane) - (c_chunks - 1), 0)) * 16u;
-            } else {
-                if (GATHER == GATHER_B) {
-                    off = static_cast<uint32_t>(b_off[i] + b_src[GATHER == GATHER_B ? i : 0] * ldb32) * 2u;
-                } else if (EPI == EPI_WGRAD) {
-                    const int c = min(c0 + b_crow[i], c_len - 1);
-                    off = static_cast<uint32_t>(b_off[i] + (c - c_lo) * ldb32) * 2u;
-                } else {
-                    // loop-invariant: kept opaque so that it stays a 32-bit register next to a scalar
-                    // base (hoisted, it becomes a zero-extended 64-bit pair per load)
-                    int o = b_off[i];
-                    asm volatile("" : "+v"(o));
-                    off = static_cast<uint32_t>(o) * 2u;
-                    if (c_tail) off -= static_cast<uint32_t>(max(c0 + b_crow[i] - (c_len - 1), 0) * ldb32) * 2u;
-                }
-            }
-            // EPI_SWIGLU: a load covers 8 LDS rows inside one 32-row block, all gate or all up rows, so
-            // the choice of the matrix is uniform over the wavefront (scalar base, 32-bit lane offset)
-            const bool up_rows = EPI == EPI_SWIGLU && ((((wave_u * B_LOADS + i) * 8) >> 5) & 1);
-            load16_to_lds((up_rows ? Bup : Bp) + off, sb + i * 1024);
-        }
-        if (hi >= A_LOADS + B_LOADS && lo < A_LOADS + B_LOADS) load_b_src(step + 1);   // this step's B loads are out
-    };
-    constexpr int NL = A_LOADS + B_LOADS;
-    auto issue_loads = [&](int step, char *stage) { issue_part(step, stage, 0, NL); };
-    // REGLOAD: the loads of a step into registers, and from there into an LDS stage.  The loads are issued
-    // unconditionally (past a tile's last step they re-read its last step, unused): inside a branch they
-    // would make the compiler wait for all loads at the join, and the look-ahead would be gone.
-    auto fetch_a = [&](int step) {
-        if (!REGLOAD) return;
-        step = min(step, loop_steps - 1);
-        const int ph = (step >= steps_per_phase) ? 1 : 0;
-        const int c0 = rotated(step - ph * steps_per_phase) * BK;
-        const char *Ap = reinterpret_cast<const char *>((p.phases > 1 && ph ? p.A[1] : p.A[0]) + uniform64(a_base));
-#pragma unroll
-        for (int i = 0; i < A_LOADS; i++)
-            ra[REGLOAD ? i : 0] = *reinterpret_cast<const u32x4 *>(Ap + static_cast<uint32_t>(a_off[i] + c0) * 2u);
-    };
-    auto fetch_b = [&](int step, int set) {
-        if (!REGLOAD) return;
-        step = min(step, loop_steps - 1);
-        const int ph = (step >= steps_per_phase) ? 1 : 0;
-        const int c0 = rotated(step - ph * steps_per_phase) * BK;
-        const int64_t b_step = uniform64(b_base + (BKIND == STRIDED ? static_cast<int64_t>(c_begin + c0) * p.ldb : 0));
-        const char *Bp = reinterpret_cast<const char *>(
-            ((EPI != EPI_SWIGLU && p.phases > 1 && ph) ? p.B[1] : p.B[0]) + b_step);
-        const char *Bup = reinterpret_cast<const char *>(p.B[1] + b_step);
-#pragma unroll
-        for (int i = 0; i < B_LOADS; i++) {
-            uint32_t off;
-            if (BKIND == CONTIG) {
-                off = static_cast<uint32_t>(b_off[i] + c0) * 2u;
-            } else {
-                int o = b_off[i];
-                asm volatile("" : "+v"(o));
-                off = static_cast<uint32_t>(o) * 2u;
-            }
-            const bool up_rows = EPI == EPI_SWIGLU && ((((wave_u * B_LOADS + i) * 8) >> 5) & 1);
-            rb[REGLOAD ? set : 0][REGLOAD ? i : 0] = *reinterpret_cast<const u32x4 *>((up_rows ? Bup : Bp) + off);
+            if (AKIND == CONTIG) off = a_off[AKIND == CONTIG ? U : 0][l] - tail_bytes(c0, l);
+            else off = crow_bytes(c0, l, lda32, rows, GATHER == GATHER_WA) +
+                       (EDGE ? min(a_off[0][l] + U * 128, static_cast<uint32_t>(p.kc - 8 - row_begin) * 2) : a_off[0][l]);
+            const char *q = AKIND == CONTIG || EDGE ? base : base + U * 128;
+            if (l == 0) dma16_if<P * A_STAGE + U * UNIT>(left, q, off, wave_lds);
+            else dma16_if<P * A_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
         }
     };
-    // (a wavefront writes the 1 KB blocks that its direct loads would fill: base + lane * 16)
-    auto commit_a = [&](int step, char *stage) {
-        if (!REGLOAD || step >= loop_steps) return;
-        char *sa = stage + wave * (A_LOADS * 1024) + lane * 16;
+    auto issue_b = [&](int left, const char *base, int c0, auto par, auto unit, const int (&rows)[L]) {
+        constexpr int P = decltype(par)::value, U = decltype(unit)::value;
 #pragma unroll
-        for (int i = 0; i < A_LOADS; i++) *reinterpret_cast<u32x4 *>(sa + i * 1024) = ra[REGLOAD ? i : 0];
-    };
-    auto commit_b = [&](int step, char *stage, int set) {
-        if (!REGLOAD || step >= loop_steps) return;
-        char *sb = stage + A_BYTES + wave * (B_LOADS * 1024) + lane * 16;
-#pragma unroll
-        for (int i = 0; i < B_LOADS; i++) *reinterpret_cast<u32x4 *>(sb + i * 1024) = rb[REGLOAD ? set : 0][REGLOAD ? i : 0];
-    };
-    // The direct loads of a step are spread over the MFMAs of a whole step rather than issued in
-    // one burst: the texture path of a CU accepts about one 1 KB load per wavefront every ~220
-    // cycles, and a wavefront that has to wait for it cannot issue its MFMAs meanwhile.  Shares of
-    // the NL loads: after the barrier of step s (stage free), then with slices 0, 1, 2 of step s+1.
-    constexpr bool WG = EPI == EPI_WGRAD;
-    constexpr int LD_T = NL * (WG ? LDW_SHARE_T : LD_SHARE_T) / 8, LD_0 = NL * (WG ? LDW_SHARE_0 : LD_SHARE_0) / 8;
-    constexpr int LD_1 = NL * (WG ? LDW_SHARE_1 : LD_SHARE_1) / 8;
-    constexpr int LD_2 = NL - LD_T - LD_0 - LD_1;
-    static_assert(LD_SHARE_T + LD_SHARE_0 + LD_SHARE_1 + LD_SHARE_2 == 8 &&
-                      LDW_SHARE_T + LDW_SHARE_0 + LDW_SHARE_1 + LDW_SHARE_2 == 8 && LD_2 >= 0, "load shares");
-    // wgrad: zero the A c-rows past the end of the expert's rows (after the loads have landed,
-    // before the barrier).  B holds finite in-segment data there, so the products vanish.
-    auto zero_tail = [&](int step, char *stage) {
-        if ((EPI != EPI_WGRAD && !KTAIL) || step >= loop_steps) return;   // (nothing was fetched for a step past the last)
-        if (EPI != EPI_WGRAD) {
-            // KTAIL: the last step of a phase holds fewer than 64 indices (A is CONTIG here): zero the
-            // chunks past the end
-            const int ph = (step >= steps_per_phase) ? 1 : 0;
-            const int c0 = rotated(step - ph * steps_per_phase) * BK;
-            if (c0 + BK <= c_len) return;
-            const int c_chunks = (c_len - c0) >> 3;
-            char *sa = stage + wave * (A_LOADS * 1024);
-#pragma unroll
-            for (int i = 0; i < A_LOADS; i++)
-                if (contig_chunk(wave_u * A_LOADS + i, lane) >= c_chunks)
-                    *reinterpret_cast<u32x4 *>(sa + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
-            return;
+        for (int l = 0; l < L; l++) {
+            uint32_t off = b_off[EDGE ? U : 0][l];
+            if (BKIND == CONTIG) off -= tail_bytes(c0, l);
+            else off += crow_bytes(c0, l, ldb32, rows, GATHER == GATHER_B);
+            const char *q = EDGE ? base : BKIND == CONTIG ? base + U * b_unit : base + U * 128;
+            if (l == 0) dma16_if<B0 + P * B_STAGE + U * UNIT>(left, q, off, wave_lds);
+            else dma16_if<B0 + P * B_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
         }
-        const int c0 = (step < steps_per_phase ? rotated(step) : step) * BK;
-        if (c0 + BK <= c_len) return;
-        char *sa = stage + wave * (A_LOADS * 1024);
+    };
+    auto issue_b_all = [&](const char *base, int c0, auto par, const int (&rows)[L]) {
+        issue_b(2, base, c0, par, IntC<0>{}, rows);
+        issue_b(2, base, c0, par, IntC<1>{}, rows);
+        if constexpr (UB == 4) { issue_b(2, base, c0, par, IntC<2>{}, rows); issue_b(2, base, c0, par, IntC<3>{}, rows); }
+    };
+    // zero what lies past the contraction range in A (B holds finite data there, so the products vanish):
+    // this wavefront's own slots of a unit, after its loads have landed and before the barrier
+    auto zero_tail = [&](int c0, auto par, auto unit) {
+        if ((!WGRAD && !EDGE) || c0 != tail_c0) return;
+        char *q = lds + decltype(par)::value * A_STAGE + decltype(unit)::value * UNIT + wave * (L * 1024) + lane * 16;
 #pragma unroll
-        for (int i = 0; i < A_LOADS; i++)
-            if (c0 + a_crow[i] >= c_len)
-                *reinterpret_cast<u32x4 *>(sa + i * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+        for (int l = 0; l < L; l++) {
+            const int c = AKIND == CONTIG ? ((lane & 7) ^ swz(slot(l))) * 8 : slot(l);
+            if (c0 + c >= c_len) *reinterpret_cast<u32x4 *>(q + l * 1024) = u32x4{0, 0, 0, 0};
+        }
     };
 
-    f32x16 acc[TM][TN];
-
-    // ---- fragment addresses (bytes within a stage), loop-invariant ------------------------------
-    // CONTIG : addr(i, kk) = c_base + i*4096 + c_kofs[kk]      (rows i*32 apart share the swizzle)
-    // STRIDED: addr(i, kk) = s_base[i] + kk*16*R*2 (+ 4*R*2 for the second transposing read)
-    const int lrow32 = lane & 31, g2 = lane >> 5;
-    int c_kofs[BK / 16];
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; kk++) c_kofs[kk] = ((kk * 2 + g2) ^ swz(lrow32)) << 4;
-    const int a_cbase = (wm * WM + lrow32) * 128;
-    const int b_cbase = A_BYTES + (wn * WN + lrow32) * 128;
-    int a_sbase[TM], b_sbase[TN];
-    {
-        const int i16 = lane & 15;
-        const int r = i16 >> 2, q = i16 & 3, mb = ((lane >> 4) & 1) * 16;
-        const int cr = 8 * g2 + r;
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int m = wm * WM + i * 32 + mb + 4 * q;
-            a_sbase[i] = strided_off<BM>(cr, m >> 3) + (m & 7) * 2;
-        }
-#pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int m = wn * WN + j * 32 + mb + 4 * q;
-            b_sbase[j] = A_BYTES + strided_off<BN>(cr, m >> 3) + (m & 7) * 2;
-        }
-    }
-    typedef __attribute__((ext_vector_type(8))) short s16x8;
-    auto read_a = [&](const char *stage, int i, int kk) -> bf16x8 {
+    // ---- fragments --------------------------------------------------------------------------------
+    int a_frag[AKIND == CONTIG ? 4 : 1], b_frag[BKIND == CONTIG ? 4 : 2];   // byte addresses within a unit region
+    auto set_fragments = [&]() {
+        int lane_f = lane;
+        asm volatile("" : "+v"(lane_f));   // recomputed per tile, not kept across the epilogue
+        const int lrow32 = lane_f & 31, g2 = lane_f >> 5;
+        const int q16 = lane_f & 3, r16 = (lane_f & 15) >> 2, mb = ((lane_f >> 4) & 1) * 16;
+        const int cr = 8 * g2 + r16;
         if (AKIND == CONTIG) {
-            return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(stage + a_cbase + i * 4096 + c_kofs[kk]));
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) a_frag[AKIND == CONTIG ? kk : 0] = (wm * 32 + lrow32) * 128 + (((kk * 2 + g2) ^ swz(lrow32)) << 4);
         } else {
-            const char *ptr = stage + a_sbase[i] + kk * (16 * BM * 2);
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ptr));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ptr + 4 * BM * 2));
-            return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            const int m = wm * 32 + mb + 4 * q16;
+            a_frag[0] = cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
         }
-    };
-    auto read_b = [&](const char *stage, int j, int kk) -> bf16x8 {
         if (BKIND == CONTIG) {
-            return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(stage + b_cbase + j * 4096 + c_kofs[kk]));
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++) b_frag[BKIND == CONTIG ? kk : 0] = B0 + wn * UNIT + lrow32 * 128 + (((kk * 2 + g2) ^ swz(lrow32)) << 4);
         } else {
-            const char *ptr = stage + b_sbase[j] + kk * (16 * BN * 2);
-            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ptr));
-            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ptr + 4 * BN * 2));
-            return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const int m = j * 32 + mb + 4 * q16;
+                b_frag[j] = B0 + wn * UNIT + cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
+            }
         }
     };
-
-    // ---- main loop ------------------------------------------------------------------------------
-    // Two LDS stages; the loads of step s+2 are issued as soon as every wavefront has taken its
-    // last fragments of step s out of LDS.  Fragments are double buffered in registers: the reads
-    // of 16-slice kk+1 are interleaved with the MFMAs of slice kk, and the first slice of the next
-    // stage is read under the MFMAs of the last slice of this one, so the wavefront never waits on
-    // LDS latency with an empty MFMA pipe.
-    bf16x8 fa[2][TM], fb[2][TN];
-    auto read_group = [&](const char *stage, int kk, int buf) {
-#pragma unroll
-        for (int i = 0; i < TM; i++) fa[buf][i] = read_a(stage, i, kk);
-#pragma unroll
-        for (int j = 0; j < TN; j++) fb[buf][j] = read_b(stage, j, kk);
+    auto read_tr = [&](const char *q) -> bf16x8 {
+        typedef __attribute__((ext_vector_type(8))) short s16x8;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q + 4 * 128));
+        return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    auto mfma_group = [&](int buf) {
+    bf16x8 fa[2][4], fb[2][TN][4];
+    f32x16 acc[TM][TN];
+    auto read_a = [&](auto par, auto unit) {
+        constexpr int O = decltype(par)::value * A_STAGE + decltype(unit)::value * UNIT, buf = decltype(unit)::value & 1;
 #pragma unroll
-        for (int i = 0; i < TM; i++)
+        for (int kk = 0; kk < 4; kk++) {
+            if (AKIND == CONTIG) fa[buf][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + a_frag[AKIND == CONTIG ? kk : 0] + O));
+            else fa[buf][kk] = read_tr(lds + a_frag[0] + O + kk * 2048);
+        }
+    };
+    auto read_b = [&](auto par, auto k_lo, auto k_hi) {
+        constexpr int P = decltype(par)::value, O = P * B_STAGE;
+#pragma unroll
+        for (int kk = decltype(k_lo)::value; kk < decltype(k_hi)::value; kk++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 4096));
+                else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 2048);
+            }
+    };
+    auto multiply = [&](auto par, auto unit) {
+        constexpr int P = decltype(par)::value, I = decltype(unit)::value;
+#pragma unroll
+        for (int kk = 0; kk < 4; kk++)
 #pragma unroll
             for (int j = 0; j < TN; j++)
                 // operands swapped: the lane then holds 4 consecutive output columns per row
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[buf][j], fa[buf][i], acc[i][j], 0, 0, 0);
+                acc[I][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[P][j][kk], fa[I & 1][kk], acc[I][j], 0, 0, 0);
     };
-    // Scheduling hint for one 16-slice: MFMA first, then the LDS reads of the next slice two at a
-    // time behind the leading MFMAs, `nl` direct loads spread evenly, the remaining MFMAs last.
-    // The wait for the previous slice's fragments then sits ahead of the first MFMA with no newer
-    // LDS read in front of it (the compiler always waits for a zero LDS counter here because the
-    // direct loads count as possible LDS accesses), and the last read of a slice has several MFMAs
-    // behind it to hide its latency.
-    constexpr int DS_READS = TM * (AKIND == CONTIG ? 1 : 2) + TN * (BKIND == CONTIG ? 1 : 2);
-    auto interleave_loads = [&](int nl) {
-        constexpr int NM = TM * TN;
-        constexpr int DS_PER = (DS_READS + NM - 2) / (NM - 1) < 2 ? 2 : (DS_READS + NM - 2) / (NM - 1);
-        int placed = 0, ds_left = DS_READS;
+    // one MFMA, then the LDS reads of the next phase behind the leading MFMAs, the rest of the MFMAs last
+    auto schedule = [&](auto reads) {
+        constexpr int R = decltype(reads)::value, PER = R > 7 ? (R + 6) / 7 : (R > 0 ? 1 : 0);
+        int left = R;
 #pragma unroll
-        for (int r = 0; r < NM; r++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // 1 MFMA
-            // (the builtin wants literal counts; the conditions fold after unrolling)
+        for (int m = 0; m < 8; m++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
 #pragma unroll
-            for (int q = 0; q < DS_PER; q++)
-                if (ds_left > 0) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); ds_left--; }
-            const int want = ((r + 1) * nl + NM - 1) / NM;   // loads due by now
-            if (want - placed >= 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // 1 VMEM read
-            if (want - placed >= 2) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            if (want - placed >= 3) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            if (want - placed >= 4) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            placed = want;
+            for (int q = 0; q < PER; q++)
+                if (left > 0) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); left--; }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto interleave = [&]() { interleave_loads(0); };
-    // one contraction step on `cur`; `nxt` holds step s+1 when this returns (par = s % 2)
-    auto half_step = [&](char *cur, char *nxt, int s, int par) {
-#pragma unroll
-        for (int kk = 0; kk < BK / 16 - 1; kk++) {
-            // the rest of the loads of step s+1 (their stage was released in the previous step)
-            const int lo = LD_T + (kk > 0 ? LD_0 : 0) + (kk > 1 ? LD_1 : 0);
-            const int n = kk == 0 ? LD_0 : (kk == 1 ? LD_1 : LD_2);
-            issue_part(s + 1, nxt, lo, lo + n);
-            // REGLOAD: B of step s+2 into the register set that held B of step s (written to LDS a step ago);
-            // issued after the A loads of step s+1 (below, behind the barrier of the previous step), so that
-            // the wait for those leaves these in flight
-            if (REGLOAD && kk == 0) fetch_b(s + 2, par);
-            read_group(cur, kk + 1, (kk + 1) & 1);
-            mfma_group(kk & 1);
-            if (REGLOAD) { if (kk == 0) interleave_loads(B_LOADS); else interleave(); }
-            else if (n > 0) interleave_loads(n); else interleave();
-        }
-        if (!REGLOAD) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's loads of step s+1 landed
-        commit_a(s + 1, nxt);                // (REGLOAD: the compiler's own waits: all loads but the B_LOADS youngest)
-        commit_b(s + 1, nxt, par ^ 1);
-        zero_tail(s + 1, nxt);
-        __syncthreads();                     // everyone's did, and nobody reads `cur` any more
-        issue_part(s + 2, cur, 0, LD_T);
-        fetch_a(s + 2);
-        read_group(nxt, 0, 0);
-        mfma_group((BK / 16 - 1) & 1);
-        if (REGLOAD) interleave_loads(A_LOADS); else if (LD_T > 0) interleave_loads(LD_T); else interleave();
-    };
-    // ---- persistent block: walks its share of the logical tiles --------------------------------
-    // Hardware places block b on XCD b % 8.  XCD x owns the contiguous run [x*per, (x+1)*per) of
-    // tiles and its blocks take them round-robin, so the tiles in flight on an XCD at any moment
-    // are neighbours and share operand slices in that XCD's L2; the total % 8 tiles left over go
-    // one each to the blocks of the least loaded slot.
-    // fwd/dgrad: the launch is sized for an upper bound on the row tiles; the tiles that exist are
-    // counted here from cum_token_counts, so that all XCDs get equal shares of real work.
+    constexpr int RA = AKIND == CONTIG ? 4 : 8, RB = BKIND == CONTIG ? 8 : 16;   // LDS reads of a unit of A, of a step of B
+
     int total_tiles = p.total_tiles;
-    if (EPI != EPI_WGRAD) {
+    if (!WGRAD) {
         if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
         __syncthreads();
         constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
         total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     }
     const int nbx = gridDim.x / NUM_XCD;
-    const int xcd = blockIdx.x % NUM_XCD, slot = blockIdx.x / NUM_XCD;
+    const int xcd = blockIdx.x % NUM_XCD, slot_x = blockIdx.x / NUM_XCD;
     int per = total_tiles / NUM_XCD, rem = total_tiles - per * NUM_XCD;
-    int run_lo = xcd * per;   // first tile of this XCD's run
-    if (EPI == EPI_WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
+    int run_lo = xcd * per;
+    if (WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
         int lo, hi;
         wgrad_xcd_run(p.cum, p.n_experts, p.tiles_e, BK, xcd, NUM_XCD, lane, lo, hi);
         run_lo = __builtin_amdgcn_readfirstlane(lo);
         per = __builtin_amdgcn_readfirstlane(hi) - run_lo;
         rem = 0;
     }
-    const int n_mine = slot < per ? (per - slot + nbx - 1) / nbx : 0;
-    const int n_all = n_mine + ((xcd < rem && slot == per % nbx) ? 1 : 0);
+    const int n_mine = slot_x < per ? (per - slot_x + nbx - 1) / nbx : 0;
+    const int n_all = n_mine + ((xcd < rem && slot_x == per % nbx) ? 1 : 0);
     int it = 0;
-    // moves the per-tile state to this block's next tile that has rows; false when there is none
     auto next_tile = [&]() -> bool {
         while (it < n_all) {
-            const int logical = it < n_mine ? run_lo + slot + it * nbx : total_tiles - rem + xcd;
+            const int logical = it < n_mine ? run_lo + slot_x + it * nbx : total_tiles - rem + xcd;
             it++;
             if (setup_tile(logical)) return true;
         }
         return false;
     };
+    constexpr IntC<0> c0_{}; constexpr IntC<1> c1_{}; constexpr IntC<2> c2_{}; constexpr IntC<3> c3_{}; constexpr IntC<4> c4_{};
+    // step 0 of a tile, all of it
+    auto prefetch = [&]() {
+        if (n_steps == 0) return;
+        const int c0 = rot * BK;
+        const char *qa = a_step(c0, 0), *qb = b_step(c0, 0);
+        issue_b_all(qb, c0, c0_, src[0]);
+        issue_a(2, qa, c0, c0_, c0_, src[0]);
+        issue_a(2, qa, c0, c0_, c1_, src[0]);
+        if constexpr (TM == 4) { issue_a(2, qa, c0, c0_, c2_, src[0]); issue_a(2, qa, c0, c0_, c3_, src[0]); }
+    };
     bool have = next_tile();
-    bool prefetched = false;   // the loads of step 0 of the current tile are already in flight
+    if (have) prefetch();
     while (have) {
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -852,95 +631,156 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-    // Steps are taken in pairs so the stage names are static; an odd step count ends with a single
-    // step.
-    if (loop_steps > 0) {
-        if (!prefetched) { issue_loads(0, stage0); fetch_a(0); fetch_b(0, 0); fetch_b(1, 1); }
-        if (!REGLOAD) __builtin_amdgcn_s_waitcnt(0x0F70);
-        commit_a(0, stage0);
-        commit_b(0, stage0, 0);
-        zero_tail(0, stage0);
-        __syncthreads();
-        issue_part(1, stage1, 0, LD_T);
-        fetch_a(1);
-        read_group(stage0, 0, 0);
-        const int n_steps = loop_steps;
-        if (HALVES && wave_u >= NW / 2 && row_end - row_begin <= BM / 2) {
-            // nothing to multiply: this wavefront's rows of B for every step, and the steps' barriers
-            // (its A rows lie past the expert's rows and nobody reads them)
-            for (int step = 0; step < n_steps; step += 2) {
-                issue_part(step + 1, stage1, A_LOADS, NL);
-                __builtin_amdgcn_s_waitcnt(0x0F70);
-                __syncthreads();
-                issue_part(step + 2, stage0, A_LOADS, NL);
-                __builtin_amdgcn_s_waitcnt(0x0F70);
-                __syncthreads();
-            }
-        } else
-        for (int step = 0; step < n_steps; step += 2) {
-            half_step(stage0, stage1, step, 0);
-            if (!ANY_STEPS || step + 1 < n_steps) half_step(stage1, stage0, step + 1, 1);
-        }
-    }
-    __syncthreads();  // the stages are dead: stage 1 becomes the strips, stage 0 the next tile's
 
-    // Weight gradient added to what the output already holds (a gradient buffer that several backward
-    // passes accumulate into): the sum is what an in-place bf16 `grad += dW` gives, two roundings.  The
-    // old values of the whole tile are requested here, ahead of the next tile's operands, into the
-    // registers that the fragments leave free (one strip ahead of its use, each strip waited for a miss:
-    // 32 experts of [2048, 7168], 256 rows each, 820 -> 740 us a launch inside a step).
-    constexpr int OLD_CPR = WN / 8, OLD_ITS = 32 * OLD_CPR / 64;   // as CPRW and ITS of the epilogue
+    if (n_steps > 0) {
+        // c0 and operand addresses of the steps t + 1 and t + 2 (t: the step being multiplied)
+        const int cs0 = rot * BK;
+        int cs1 = next_c0(cs0), cs2 = next_c0(cs1), cst = cs0;
+        const char *pa1 = a_step(cs1, 1), *pa2 = a_step(cs2, 2), *pb2 = b_step(cs2, 2);
+        // One contraction step of parity P (see the comment above the kernel).  Past the last step nothing is loaded, and
+        // what is read for it is not used.
+        auto step = [&](auto par, auto full, int t) {
+            constexpr int P = decltype(par)::value;
+            constexpr bool FULL = decltype(full)::value;
+            const int left = __builtin_amdgcn_readfirstlane(n_steps - 1 - t);
+            constexpr IntC<P> same{}; constexpr IntC<P ^ 1> other{};
+            const int (&s2)[L] = src[GATHER_W ? 2 : 0];
+            int src3[L] = {};   // source rows of step t + 3
+            const int cs3 = next_c0(cs2);
+            if constexpr (TM == 2) {
+                issue_b(left, pb2, cs2, same, c0_, s2);
+                issue_b(left, pb2, cs2, same, c1_, s2);
+                issue_a(left, pa2, cs2, same, c0_, s2);
+                read_a(same, c1_);
+                multiply(same, c0_);
+                schedule(IntC<RA>{});
+                wait_step_loads<8, 2>(left, lds_addr);
+                zero_tail(cs1, other, c0_);
+                block_barrier();
+                if (GATHER_W && left >= 2) look_up(cs3, src3);
+                issue_a(left, pa2, cs2, same, c1_, s2);
+                read_a(other, c0_);
+                read_b(other, c0_, c4_);
+                if (FULL || active > 1) multiply(same, c1_);
+                schedule(IntC<RA + RB>{});
+                wait_step_loads<8, 0>(left, lds_addr);
+                zero_tail(cs1, other, c1_);
+                block_barrier();
+            } else {
+                // phase 0
+                issue_b(left, pb2, cs2, same, c0_, s2);
+                issue_b(left, pb2, cs2, same, c1_, s2);
+                issue_a(left, pa2, cs2, same, c0_, s2);
+                read_a(same, c1_);
+                multiply(same, c0_);
+                schedule(IntC<RA>{});
+                // phase 1
+                issue_b(left, pb2, cs2, same, c2_, s2);
+                issue_b(left, pb2, cs2, same, c3_, s2);
+                issue_a(left + 1, pa1, cs1, other, c3_, src[GATHER_W ? 1 : 0]);
+                read_a(same, c2_);
+                if (FULL || active > 1) multiply(same, c1_);
+                schedule(IntC<RA>{});
+                wait_step_loads<8, 3>(left, lds_addr);
+                zero_tail(cs1, other, c0_);
+                zero_tail(cst, same, c3_);
+                block_barrier();
+                // phase 2
+                if (GATHER_W && left >= 2) look_up(cs3, src3);
+                issue_a(left, pa2, cs2, same, c1_, s2);
+                read_a(same, c3_);
+                read_b(other, c0_, c2_);
+                if (FULL || active > 2) multiply(same, c2_);
+                schedule(IntC<RA + RB / 2>{});
+                // phase 3
+                issue_a(left, pa2, cs2, same, c2_, s2);
+                read_a(other, c0_);
+                read_b(other, c2_, c4_);
+                if (FULL || active > 3) multiply(same, c3_);
+                schedule(IntC<RA + RB / 2>{});
+                wait_step_loads<8, 1>(left, lds_addr);
+                zero_tail(cs1, other, c1_);
+                zero_tail(cs1, other, c2_);
+                block_barrier();
+            }
+            if (GATHER_W) {
+#pragma unroll
+                for (int l = 0; l < L; l++) { src[0][l] = src[GATHER_W ? 1 : 0][l]; src[GATHER_W ? 1 : 0][l] = src[GATHER_W ? 2 : 0][l]; src[GATHER_W ? 2 : 0][l] = src3[l]; }
+            }
+            cst = cs1;
+            cs1 = cs2;
+            cs2 = cs3;
+            pa1 = pa2;
+            pa2 = a_step(cs2, t + 3);
+            pb2 = b_step(cs2, t + 3);
+        };
+        // the units of step 1 that the loop does not load itself
+        if (n_steps > 1) {
+            const char *pb1 = b_step(cs1, 1);
+            issue_b_all(pb1, cs1, c1_, src[GATHER_W ? 1 : 0]);
+            issue_a(2, pa1, cs1, c1_, c0_, src[GATHER_W ? 1 : 0]);
+            issue_a(2, pa1, cs1, c1_, c1_, src[GATHER_W ? 1 : 0]);
+            if constexpr (TM == 4) { issue_a(2, pa1, cs1, c1_, c2_, src[GATHER_W ? 1 : 0]); wait_loads<7>(lds_addr); }
+            else wait_loads<8>(lds_addr);
+        } else {
+            wait_loads<0>(lds_addr);
+        }
+        zero_tail(cs0, c0_, c0_);
+        zero_tail(cs0, c0_, c1_);
+        if constexpr (TM == 4) { zero_tail(cs0, c0_, c2_); zero_tail(cs0, c0_, c3_); }
+        block_barrier();
+        set_fragments();
+        read_a(c0_, c0_);
+        read_b(c0_, c0_, c4_);
+        block_barrier();   // (their buffers are the first that step 0 loads into)
+        auto loop = [&](auto full) {
+            for (int t = 0; t < n_steps; t += 2) {
+                step(c0_, full, t);
+                if (t + 1 < n_steps) step(c1_, full, t + 1);
+            }
+        };
+        if (active == TM) loop(std::true_type{});
+        else loop(std::false_type{});
+    }
+    __syncthreads();  // the odd steps' buffers become the strips, the even steps' the next tile's
+
+    constexpr int OLD_CPR = 64 / 8, OLD_ITS = 32 * OLD_CPR / 64;   // as CPRW and ITS of the epilogue
     u32x4 old[ACCUM ? TM : 1][ACCUM ? OLD_ITS : 1];
     if (ACCUM) {
         int lane_o = lane;
         asm volatile("" : "+v"(lane_o));
-        const uint16_t *src = p.C + expert * p.strideC + n0 + wn * WN + (lane_o % OLD_CPR) * 8;
-        const bool col_in = !EDGE || n0 + wn * WN + (lane_o % OLD_CPR) * 8 < p.n_cols;
-        const int m_first = row_begin + wm * WM + lane_o / OLD_CPR;
+        const uint16_t *from = p.C + expert * p.strideC + n0 + wn * 64 + (lane_o % OLD_CPR) * 8;
+        const bool col_in = !EDGE || n0 + wn * 64 + (lane_o % OLD_CPR) * 8 < p.n_cols;
+        const int m_first = row_begin + wm * 32 + lane_o / OLD_CPR;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int it = 0; it < OLD_ITS; it++) {
-                const int m = m_first + i * 32 + it * (64 / OLD_CPR);
+                const int m = m_first + i * 64 + it * (64 / OLD_CPR);
                 if (!EDGE || (col_in && m < p.kc))
                     old[ACCUM ? i : 0][ACCUM ? it : 0] =
-                        *reinterpret_cast<const u32x4 *>(src + static_cast<int64_t>(m) * p.ldc);
+                        *reinterpret_cast<const u32x4 *>(from + static_cast<int64_t>(m) * p.ldc);
             }
     }
 
-    // The next tile's first contraction step is fetched into stage 0 while this tile's results go
-    // out (the strips live in stage 1), which takes the cold-miss latency of a tile's first loads
-    // off the critical path.
-    const int e_expert = expert, e_row_begin = row_begin, e_row_end = row_end, e_n0 = n0;
+    const int e_expert = expert, e_row_begin = row_begin, e_row_end = row_end, e_n0 = n0, e_active = active;
     have = next_tile();
-    prefetched = have && loop_steps > 0;
-    if (prefetched) { issue_loads(0, stage0); fetch_a(0); fetch_b(0, 0); fetch_b(1, 1); }
+    if (have) prefetch();
 
     // ---- epilogue ------------------------------------------------------------------------------
-    // Accumulator element r of lane l is output row (l % 32), column (r/4)*8 + (l/32)*4 + (r%4) of
-    // its 32x32 block: a lane holds 4 consecutive columns of ONE row, and the 64 lanes of a store
-    // would touch 32 different rows.  Each wavefront therefore turns its results around through a
-    // private LDS strip (32 rows x COLS bf16, row pitch COLS*2+8 bytes so that both the 8-byte
-    // writes in accumulator layout and the 8-byte reads in row layout are conflict-free) and moves
-    // 16 bytes per lane to and from global memory, 64 lanes covering whole 256-byte row segments.
-    // The fused SwiGLU backward reads g and u in the same row layout.
-    // The epilogue's lane-derived addresses are the same for every tile; recompute them per tile
-    // (a few VALU ops) instead of letting them be hoisted out of the tile loop, where they would
-    // stay live across the main loop and spill.
-    int lane_e = lane, wave_e = __builtin_amdgcn_readfirstlane(wave);
+    int lane_e = lane, wave_e = wave;
     asm volatile("" : "+v"(lane_e), "+s"(wave_e));
-    constexpr int COLS = (EPI == EPI_SWIGLU) ? WN / 2 : WN;   // output columns of this wavefront
+    constexpr int COLS = (EPI == EPI_SWIGLU) ? 32 : 64;   // output columns of this wavefront
     constexpr int PITCH = COLS * 2 + 8;
     constexpr int STRIP = 32 * PITCH;
     constexpr int NSTRIP = (EPI == EPI_SWIGLU) ? 3 : 1;
-    static_assert(NW * NSTRIP * STRIP <= A_BYTES + B_BYTES, "strips must fit in one stage");
+    static_assert(NW / 2 * NSTRIP * STRIP <= A_STAGE && NW / 2 * NSTRIP * STRIP <= B_STAGE, "strips must fit beside the even steps' buffers");
     const int wm_e = wave_e / WAVES_N, wn_e = wave_e % WAVES_N;
-    char *strip = stage1 + wave_e * (NSTRIP * STRIP);
+    char *strip = lds + (wave_e < NW / 2 ? A_STAGE : B0 + B_STAGE) + (wave_e % (NW / 2)) * (NSTRIP * STRIP);
     const int lrow = lane_e & 31;
     const int lcol = (lane_e >> 5) * 4;
     constexpr int CPRW = COLS / 8;            // 16-byte chunks per strip row
     constexpr int ITS = 32 * CPRW / 64;       // chunks per lane per strip
-    // write 4 consecutive columns (as bf16) of row lrow at column `col` of strip `which`
     auto strip_put = [&](int which, int col, float v0, float v1, float v2, float v3) {
         u32x2 v;
         v[0] = pack2_bf16(v0, v1);
@@ -958,44 +798,38 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    const int col0 = (EPI == EPI_SWIGLU) ? e_n0 + (wn_e * WN) / 2 : e_n0 + wn_e * WN;   // first output column
-    uint16_t *Cb = p.C + (EPI == EPI_WGRAD ? e_expert * p.strideC : 0);
-    // Rows this wavefront may touch in global memory: the expert's rows (the weight gradient: the
-    // rows of dW), none at all for a lane whose 8 columns lie past the last output column (a partial
-    // last column tile; extents are multiples of 8, so a lane's 16-byte chunk is in or out as a whole).
-    const int row_lim = !EDGE ? (EPI == EPI_WGRAD ? 0x7fffffff : e_row_end)
-                              : (col0 + (lane_e % (COLS / 8)) * 8 < p.n_cols) ? (EPI == EPI_WGRAD ? p.kc : e_row_end) : 0;
-    // ROWW forward: the weights of this lane's row in every strip, fetched together up front
+    const int col0 = e_n0 + wn_e * COLS;   // first output column
+    uint16_t *Cb = p.C + (WGRAD ? e_expert * p.strideC : 0);
+    const int row_lim = EDGE && col0 + (lane_e % (COLS / 8)) * 8 >= p.n_cols ? 0 : e_row_end;
     float wrow_all[(ROWW && EPI == EPI_SWIGLU) ? TM : 1];
     if (ROWW && EPI == EPI_SWIGLU) {
 #pragma unroll
         for (int i = 0; i < TM; i++) {
-            const int64_t m = static_cast<int64_t>(e_row_begin) + wm_e * WM + i * 32 + lrow;
+            const int64_t m = static_cast<int64_t>(e_row_begin) + (2 * i + wm_e) * 32 + lrow;
             wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0] = (m < e_row_end) ? p.row_scale[m] : 0.0f;
         }
     }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-        const int64_t m0 = static_cast<int64_t>(e_row_begin) + wm_e * WM + i * 32;  // first row of the strip
+        if (i >= e_active) break;
+        const int64_t m0 = static_cast<int64_t>(e_row_begin) + (2 * i + wm_e) * 32;  // first row of the strip
         u32x4 *old_out = old[ACCUM ? i : 0];
         if (EPI == EPI_SWIGLU) {
             const float wrow = wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0];   // ROWW: h = w[row] * silu(g) * u, one rounding
 #pragma unroll
-            for (int j = 0; j < TN; j += 2)
+            for (int rq = 0; rq < 4; rq++) {
+                float hv[4];
 #pragma unroll
-                for (int rq = 0; rq < 4; rq++) {
-                    float hv[4];
-#pragma unroll
-                    for (int x = 0; x < 4; x++) {
-                        const float gv = acc[i][j][rq * 4 + x], uv = acc[i][j + 1][rq * 4 + x];
-                        hv[x] = (gv * fast_sigmoid(gv)) * uv;
-                        if (ROWW) hv[x] *= wrow;
-                    }
-                    const int col = (j / 2) * 32 + rq * 8 + lcol;
-                    strip_put(0, col, acc[i][j][rq * 4], acc[i][j][rq * 4 + 1], acc[i][j][rq * 4 + 2], acc[i][j][rq * 4 + 3]);
-                    strip_put(1, col, acc[i][j + 1][rq * 4], acc[i][j + 1][rq * 4 + 1], acc[i][j + 1][rq * 4 + 2], acc[i][j + 1][rq * 4 + 3]);
-                    strip_put(2, col, hv[0], hv[1], hv[2], hv[3]);
+                for (int x = 0; x < 4; x++) {
+                    const float gv = acc[i][0][rq * 4 + x], uv = acc[i][1][rq * 4 + x];
+                    hv[x] = (gv * fast_sigmoid(gv)) * uv;
+                    if (ROWW) hv[x] *= wrow;
                 }
+                const int col = rq * 8 + lcol;
+                strip_put(0, col, acc[i][0][rq * 4], acc[i][0][rq * 4 + 1], acc[i][0][rq * 4 + 2], acc[i][0][rq * 4 + 3]);
+                strip_put(1, col, acc[i][1][rq * 4], acc[i][1][rq * 4 + 1], acc[i][1][rq * 4 + 2], acc[i][1][rq * 4 + 3]);
+                strip_put(2, col, hv[0], hv[1], hv[2], hv[3]);
+            }
         } else {
 #pragma unroll
             for (int j = 0; j < TN; j++)
@@ -1006,14 +840,17 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         }
         strip_sync();
         if (EPI == EPI_SWIGLU_BWD) {
-            u32x4 gq[ITS], uq[ITS];
+            constexpr int GRP = 2;   // g and u in flight for half a strip: with all of it the 256x256 kernel spills
+            u32x4 gq[GRP], uq[GRP];
             // ROWW: lane l fetches the weight of strip row l % 32 along with the g/u loads; the
             // lanes that work on a row pick it up with a lane read
             float w_strip = 0.0f;
             if (ROWW && m0 + (lane_e & 31) < e_row_end) w_strip = p.row_scale[m0 + (lane_e & 31)];
 #pragma unroll
-            for (int it = 0; it < ITS; it++) {
-                const int q = it * 64 + lane_e;
+            for (int i0 = 0; i0 < ITS; i0 += GRP) {
+#pragma unroll
+            for (int it = 0; it < GRP; it++) {
+                const int q = (i0 + it) * 64 + lane_e;
                 const int64_t m = m0 + q / CPRW;
                 if (m < row_lim) {
                     const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
@@ -1023,8 +860,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
                 }
             }
 #pragma unroll
-            for (int it = 0; it < ITS; it++) {
-                const int q = it * 64 + lane_e;
+            for (int it = 0; it < GRP; it++) {
+                const int q = (i0 + it) * 64 + lane_e;
                 const int64_t m = m0 + q / CPRW;
                 float dot = 0.0f;   // ROWW: this lane's part of sum_i dh[m][i] * silu(g[m][i]) * u[m][i]
                 const float wr = ROWW ? __shfl(w_strip, q / CPRW, 64) : 1.0f;
@@ -1063,6 +900,8 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
                     if (q % CPRW == 0 && m < row_lim) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
+            }
         } else {
 #pragma unroll
             for (int it = 0; it < ITS; it++) {
@@ -1071,7 +910,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
                 if (m < row_lim) {
                     const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
                     u32x4 v = strip_get(0, q / CPRW, q % CPRW);
-                    if (EPI == EPI_WGRAD && ACCUM) {
+                    if (WGRAD && ACCUM) {
                         float fresh[8], prev[8];
                         Elem<uint16_t>::unpack(v, fresh);
                         Elem<uint16_t>::unpack(old_out[ACCUM ? it : 0], prev);
@@ -1089,7 +928,7 @@ __global__ __launch_bounds__(WAVES_M *WAVES_N * 64, BM == 128 ? 2 : 1) void ggem
         }
         strip_sync();  // the strip is rewritten by the next i
     }
-    __syncthreads();  // the strips alias stage 1, which the next tile loads into
+    __syncthreads();  // the strips alias the odd steps' buffers, which the next tile loads into
     }  // tile loop
 }
 
@@ -1132,27 +971,23 @@ template <int BM> unsigned persistent_blocks(int64_t tiles) {
     return static_cast<unsigned>(per_xcd * NUM_XCD);
 }
 
-template <int BM> struct Waves {
-    static constexpr int M = 2;                       // 256x256: 2 x 4 wavefronts of 128x64;
-    static constexpr int N = (BM == 256) ? 4 : 2;    // 128x128: 2 x 2 wavefronts of 64x64
-};
+template <int BM> constexpr int WAVES_N = BM / 64;        // 256x256: 2 x 4 wavefronts, 128x128: 2 x 2
+template <int BM> constexpr int THREADS = 2 * WAVES_N<BM> * 64;
 
-template <int BM, int BN, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool KTAIL = false,
-          bool REGLOAD = false>
+template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
 int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad family
-    constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
+    constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BM / 2 : BM;
     if (p.n_experts > MAX_EXPERTS) return OM_ERR_SHAPE;   // the tile table lives in LDS
-    p.m_tiles_max = static_cast<int>((rows + BM - 1) / BM + p.n_experts);
-    const int64_t tiles = static_cast<int64_t>(p.m_tiles_max) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+    const int64_t m_tiles_max = (rows + BM - 1) / BM + p.n_experts;
+    const int64_t tiles = m_tiles_max * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
-    p.total_tiles = static_cast<int>(tiles);
-    ggemm_kernel<BM, BN, Waves<BM>::M, Waves<BM>::N, AKIND, BKIND, EPI, GATHER, ROWW, false, KTAIL, REGLOAD>
-        <<<dim3(persistent_blocks<BM>(tiles)), dim3(Waves<BM>::M * Waves<BM>::N * 64), 0, st>>>(p);
+    ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128>
+        <<<dim3(persistent_blocks<BM>(tiles)), dim3(THREADS<BM>), 0, st>>>(p);
     return om_launch_status();
 }
 
 // The tile shape launch_rows_auto picks: 256x256 when the output columns are a whole number of such
-// tiles, the contraction a whole number of step pairs, the experts hold enough rows to fill them, and there are enough of them for at least half
+// tiles, the contraction a whole number of steps, the experts hold enough rows to fill them, and there are enough of them for at least half
 // the CUs (a tiny problem is spread over more CUs by the 128x128 tile).  The 128x128 tile takes any
 // extents and contraction lengths that are multiples of 8: its last column tile and its last
 // contraction step may be partial.
@@ -1172,7 +1007,7 @@ template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t
     constexpr int div = (EPI == EPI_SWIGLU) ? 2 : 1;
     const bool large = static_cast<int64_t>(n_cols) * kc >= (4 << 20);
     const int enough = EPI == EPI_SWIGLU_BWD ? 192 : !large ? 160 : EPI == EPI_SWIGLU ? 128 : 112;
-    if (n_cols % (256 / div) != 0 || kc % 128 != 0 || rows < static_cast<int64_t>(n_experts) * enough) return false;
+    if (n_cols % (256 / div) != 0 || kc % BK != 0 || rows < static_cast<int64_t>(n_experts) * enough) return false;
     const int64_t tiles = ((rows + 255) / 256) * (n_cols / (256 / div));
     return tiles * 2 >= device_cu_count();
 }
@@ -1181,15 +1016,9 @@ template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t
 template <int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
 int launch_rows_auto(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
     if (uses_big_tile<EPI>(p.n_cols, p.kc, p.n_experts, expected))
-        return launch_rows<256, 256, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
+        return launch_rows<256, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
     if (p.n_cols % 8 != 0 || p.kc % 8 != 0) return OM_ERR_SHAPE;
-    if (p.kc % 64 != 0) return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW, true>(p, rows, st);
-    // Few rows per expert (fewer than 256 on average): the launch streams weights that are used once, and the
-    // kernels that keep two steps of them in flight are 4-10 % faster; with more rows the direct-load kernels
-    // are (4-9 % at 2000 rows per expert), so each regime gets its own.
-    if (expected < static_cast<int64_t>(p.n_experts) * 256)
-        return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW, false, true>(p, rows, st);
-    return launch_rows<128, 128, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
+    return launch_rows<128, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
 }
 
 }  // namespace
@@ -1276,18 +1105,16 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
-    const dim3 grid_big(persistent_blocks<256>(tiles)), block_big(Waves<256>::M * Waves<256>::N * 64);
-    const dim3 grid_small(persistent_blocks<128>(tiles)), block_small(256);
     // ACCUM (C[g] = bf16(float(C[g]) + float(bf16(acc))) instead of C[g] = acc) is a template
     // parameter: the plain kernels carry none of it
 #define OM_WGRAD(GATHER_KIND, ACC)                                                                               \
     do {                                                                                                         \
         if (big)                                                                                                 \
-            ggemm_kernel<256, 256, Waves<256>::M, Waves<256>::N, STRIDED, STRIDED, EPI_WGRAD, GATHER_KIND, false, \
-                         ACC><<<grid_big, block_big, 0, st>>>(p);                                                \
+            ggemm_kernel<256, STRIDED, STRIDED, EPI_WGRAD, GATHER_KIND, false, ACC>                              \
+                <<<dim3(persistent_blocks<256>(tiles)), dim3(THREADS<256>), 0, st>>>(p);                         \
         else                                                                                                     \
-            ggemm_kernel<128, 128, 2, 2, STRIDED, STRIDED, EPI_WGRAD, GATHER_KIND, false, ACC>                    \
-                <<<grid_small, block_small, 0, st>>>(p);                                                         \
+            ggemm_kernel<128, STRIDED, STRIDED, EPI_WGRAD, GATHER_KIND, false, ACC, true>                        \
+                <<<dim3(persistent_blocks<128>(tiles)), dim3(THREADS<128>), 0, st>>>(p);                         \
     } while (0)
     if (accumulate) {
         if (gather == GATHER_NONE) OM_WGRAD(GATHER_NONE, true);
@@ -1445,7 +1272,7 @@ namespace {
 // columns of the intermediate size that one wavefront's epilogue covers (both tile shapes): the
 // granularity of the row_dot partial sums
 constexpr int ROW_DOT_COLS = 64;
-static_assert(256 / Waves<256>::N == ROW_DOT_COLS && 128 / Waves<128>::N == ROW_DOT_COLS, "row_dot layout");
+static_assert(256 / WAVES_N<256> == ROW_DOT_COLS && 128 / WAVES_N<128> == ROW_DOT_COLS, "row_dot layout");
 
 // `dy_rows` != null: sorted row r of dy is row dy_rows[r] of a [src_rows, H] matrix, the result is
 // scaled by row_weights[r] and row_dot receives the partial sums of (dy W) * silu(g) * u

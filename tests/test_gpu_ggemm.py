@@ -557,6 +557,37 @@ def test_half_row_tiles_of_the_256_kernels(cuda, counts):
             assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6 * k ** 0.5).all(), (name, e)
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320])
+def test_row_units_and_step_counts_of_the_256_kernels(cuda, K):
+    """1 to 5 contraction steps (the loads run two steps ahead, so the first and last two of a tile are special), rows on
+    both sides of every multiple of 64 (the units in which a tile's rows are worked), and in the weight gradient
+    contractions of 0 to 513 rows.  One bf16 rounding of a float32 sum (2^-8 of the value, and the order of the sum)."""
+    from optimus import _native as n
+    counts = [64, 65, 127, 129, 191, 192, 193, 255, 256, 257, 320, 0, 1, 448, 513, 300] * 3
+    G, N, rows = len(counts), 1024, sum(counts)
+    assert rows >= 192 * G and (rows // 256) * (N // 256) * 2 >= 256
+    g = torch.Generator().manual_seed(K)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    x = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(cuda)
+    z = torch.randn(rows, N, generator=g).to(torch.bfloat16).to(cuda)
+    w = (torch.randn(G, N, K, generator=g) * 0.05).to(torch.bfloat16).to(cuda)
+    wt = (torch.randn(G, K, N, generator=g) * 0.05).to(torch.bfloat16).to(cuda)
+    y, dx = (torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    dw = torch.full((G, N, 512), 7.0, dtype=torch.bfloat16, device=cuda)
+    d, P = cum.to(cuda), n.ptr
+    n.check(n.lib().om_grouped_gemm_fwd(P(x), P(w), P(y), P(d), rows, G, N, K, 0, n.stream()), "fwd")
+    n.check(n.lib().om_grouped_gemm_dgrad(P(x), P(wt), P(dx), P(d), rows, G, K, N, 0, n.stream()), "dgrad")
+    v = z[:, :512].contiguous()
+    n.check(n.lib().om_grouped_gemm_wgrad(P(z), P(v), P(dw), P(d), rows, G, N, 512, 0, n.stream()), "wgrad")
+    torch.cuda.synchronize()
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        for name, got, want, k in (("fwd", y[s], x[s].float() @ w[e].float().t(), K), ("dgrad", dx[s], x[s].float() @ wt[e].float(), K),
+                                   ("wgrad", dw[e], z[s].float().t() @ v[s].float(), counts[e])):
+            assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5 * max(k, 1) ** 0.5).all(), (name, e)
+
+
 @pytest.mark.parametrize("expected", [0, 9, 100, 1087, 3000, 9000])
 @pytest.mark.parametrize("N,K", [(1024, 512), (200, 328)])
 def test_products_over_a_bound_of_the_rows(cuda, expected, N, K):
