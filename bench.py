@@ -66,6 +66,7 @@ GEMM_ENTRY_PRODUCTS = {     # C-ABI entry -> number of [rows x N x K] products p
     "om_merged_mlp_down_dgrad": 1, "om_merged_mlp_gate_up_dgrad": 2, "om_grouped_gemm_dgrad": 1,
     "om_grouped_gemm_wgrad_accumulate": 1, "om_grouped_gemm_wgrad_gathered_accumulate": 1,
     "om_grouped_gemm_wgrad_gathered_out_accumulate": 1,
+    "om_grouped_gemm_wgrad_merged": 3, "om_grouped_gemm_wgrad_merged_accumulate": 3,
 }
 
 
@@ -384,7 +385,7 @@ def bench_other_configs(args, device, with_cpu, only=None):
         per_launch = {   # weight bytes each entry point streams (reads, or writes for the weight gradients)
             "om_merged_mlp_gate_up_fwd_weighted": one_pass * 2 / 3, "om_grouped_gemm_fwd": one_pass / 3,
             "om_merged_mlp_down_dgrad_weighted": one_pass / 3, "om_merged_mlp_gate_up_dgrad": one_pass * 2 / 3,
-            "om_grouped_gemm_wgrad_gathered": one_pass * 2 / 3, "om_grouped_gemm_wgrad_gathered_out": one_pass / 3}
+            "om_grouped_gemm_wgrad_merged": one_pass}
         out["C4"] = entry(c["T"], ms, per, flops, wbytes, bound="hbm",
                           traffic=measured_traffic_bytes("C4:all_expert_gemm_launches"), extra={
             "weight_stream_gb_per_s_by_entry_point": {

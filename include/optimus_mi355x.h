@@ -613,6 +613,22 @@ int om_grouped_gemm_wgrad_f32_accumulate(const float *output_grad, const float *
                                          const int32_t *cum_token_counts, int64_t rows, int G, int N,
                                          int K, int64_t w_stride, void *stream);
 
+/* The three weight gradients of a merged MLP (in one launch where they are small): dw_down [G,H,I] = dout^T h, dw_gate [G,I,H] = dg^T x and
+ * dw_up = du^T x over each expert's rows, or added to what the three hold (`_accumulate`, as above).  dout_rows / x_rows
+ * (may be null): row r of dout / x is row dout_rows[r] / x_rows[r] of a [src_rows, H] matrix.  Strides: elements between
+ * experts, 0 for packed.  I and H multiples of 8.                                                                    */
+int om_grouped_gemm_wgrad_merged(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
+                                 const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
+                                 void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                 int64_t rows, int G, int I, int H, int64_t down_stride, int64_t gate_stride,
+                                 int64_t up_stride, void *stream);
+int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const int32_t *dout_rows, const void *h,
+                                            const void *dg, const void *du, const void *x,
+                                            const int32_t *x_rows, int64_t src_rows, void *dw_down,
+                                            void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                            int64_t rows, int G, int I, int H, int64_t down_stride,
+                                            int64_t gate_stride, int64_t up_stride, void *stream);
+
 /* The merged MLP of a float32 module (moe.py:396-405 and its autograd), the forms of the bf16 entry points
  * above: gate and up in one launch with h = silu(g) * u formed in the epilogue, the SwiGLU backward in the
  * epilogue of dh = dy W_down, dx as one accumulation over both products, and both weight gradients in one

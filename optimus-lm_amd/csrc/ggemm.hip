@@ -62,7 +62,8 @@ enum {
     GATHER_NONE = 0,
     GATHER_A = 1,    // fwd/dgrad: A rows
     GATHER_B = 2,    // wgrad: contraction rows of B
-    GATHER_WA = 3    // wgrad: contraction rows of A
+    GATHER_WA = 3,   // wgrad: contraction rows of A
+    MERGED = 4       // the three weight gradients of a merged MLP in one launch (see WgradSet)
 };
 enum {
     EPI_STORE = 0,        // C = acc
@@ -73,7 +74,15 @@ enum {
 
 constexpr int BK = 64;  // contraction step, elements
 constexpr int NUM_XCD = 8;
-constexpr int QUEUE_PITCH = 32;   // ints between the tile counters of two XCDs: a 128-byte line each
+
+// MERGED: one weight gradient C[e] (+)= A^T B over expert e's rows; A [rows, m], B [rows, n], C [m, n] per expert.
+struct WgradSet {
+    const uint16_t *A, *B;
+    uint16_t *C;
+    const int32_t *a_rows, *b_rows;   // at most one not null: rows taken through an index
+    int64_t strideC;
+    int m, n;
+};
 
 struct GemmParams {
     // operands; for the two-phase products (gate+up) index 1 is the second pair
@@ -97,8 +106,8 @@ struct GemmParams {
     int kc;                     // contraction length per phase (fwd/dgrad), multiple of 8
     int phases;                 // 1 or 2
     int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
-    int tiles_e;                // wgrad: tiles per expert
-    int32_t *queue;             // null, or NUM_XCD counters QUEUE_PITCH apart, zero before the launch
+    int tiles_e;                // wgrad: tiles per expert (MERGED: of all three)
+    WgradSet set[3];            // MERGED
 };
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
@@ -288,11 +297,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     constexpr int TM = BM / 64, TN = 2;     // row units of a tile, accumulators of a wavefront in each
     static_assert(GATHER == GATHER_NONE || (GATHER == GATHER_A && AKIND == CONTIG && EPI != EPI_WGRAD) ||
                       (GATHER == GATHER_B && BKIND == STRIDED && EPI == EPI_WGRAD) ||
-                      (GATHER == GATHER_WA && AKIND == STRIDED && EPI == EPI_WGRAD), "gather variants");
+                      ((GATHER == GATHER_WA || GATHER == MERGED) && AKIND == STRIDED && EPI == EPI_WGRAD), "gather variants");
     static_assert(!ACCUM || EPI == EPI_WGRAD, "only the weight gradient adds into its output");
     static_assert(!ROWW || EPI == EPI_SWIGLU || EPI == EPI_SWIGLU_BWD, "row weights belong to the SwiGLU epilogues");
     constexpr bool WGRAD = EPI == EPI_WGRAD;
-    constexpr bool GATHER_W = GATHER == GATHER_B || GATHER == GATHER_WA;
+    constexpr bool GATHER_W = GATHER == GATHER_B || GATHER == GATHER_WA || GATHER == MERGED;
     constexpr int UNIT = 8192;             // bytes of an operand unit: 64 rows (CONTIG) or 64 columns (STRIDED) x 64 c
     constexpr int UA = TM, UB = BN / 64;   // units of a step
     constexpr int L = 8 / NW;              // direct loads per wavefront per unit
@@ -301,7 +310,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     __shared__ __attribute__((aligned(1024))) char lds[2 * A_STAGE + 2 * B_STAGE];
     constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
     __shared__ int idx_cache[IDX_CACHE];
-    int cached_expert = -1;
+    int cached_expert = -1;            // (MERGED: and product)
     __shared__ int tile_end[WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
     __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];
 
@@ -320,7 +329,10 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     const char *a_tile[2] = {}, *b_tile[2] = {};   // base addresses of the tile's operands (two phases), block-uniform
     int tail_c0 = -1;     // first contraction index of the partial step, if the tile has one
     int src[GATHER_W ? 3 : 1][L];             // GATHER_W: source rows of this lane's slots, steps t, t + 1, t + 2
-    const int lda32 = static_cast<int>(p.lda), ldb32 = static_cast<int>(p.ldb);
+    // of the current product (MERGED: set by setup_tile, otherwise the launch's)
+    int lda32 = static_cast<int>(p.lda), ldb32 = static_cast<int>(p.ldb), n_cols = p.n_cols, m_rows = p.kc, product = 0;
+    const int32_t *row_index = p.row_index;
+    bool a_indexed = GATHER == GATHER_WA, b_indexed = GATHER == GATHER_B;
     constexpr bool TWO_PHASE = EPI == EPI_STORE && BKIND == STRIDED;   // the merged MLP's dx = dg Wg + du Wu
     const int64_t b_unit = static_cast<int64_t>(EPI == EPI_SWIGLU ? 32 : 64) * p.ldb * 2;   // CONTIG: bytes between units
     const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)lds));
@@ -330,14 +342,14 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     auto next_c0 = [&](int c0) { return c0 + BK >= c_wrap ? 0 : c0 + BK; };
     // GATHER_W: the source rows of the step at c0; the first IDX_CACHE of an expert's rows come from LDS
     auto look_up = [&](int c0, int (&out)[L]) {
-        if (!GATHER_W) return;
+        if (!GATHER_W || (GATHER == MERGED && !row_index)) return;
 #pragma unroll
         for (int l = 0; l < L; l++) {
             const int c = min(c0 + slot(l), c_len - 1);
             if (c0 + BK <= IDX_CACHE) {
                 out[l] = idx_cache[c];
             } else {   // (waited for here: at the join the compiler would wait for the direct loads too, on either path)
-                int v = p.row_index[c_begin + c];
+                int v = row_index[c_begin + c];
                 asm volatile("" : "+v"(v));
                 out[l] = v;
             }
@@ -347,13 +359,23 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     auto setup_tile = [&](int logical) -> bool {
         int rot_a, rot_b;
         if (WGRAD) {
-            const int tiles_n = (p.n_cols + BN - 1) / BN;
             expert = logical / p.tiles_e;
-            const int tile = logical - expert * p.tiles_e;
+            int tile = logical - expert * p.tiles_e;
+            if (GATHER == MERGED) {
+                const int each = p.tiles_e / 3;     // (the three have the same extents, one of them transposed)
+                product = __builtin_amdgcn_readfirstlane(tile / each);
+                tile -= product * each;
+                const WgradSet &w = p.set[product];
+                m_rows = w.m; n_cols = w.n;
+                lda32 = m_rows; ldb32 = n_cols;
+                a_indexed = w.a_rows != nullptr; b_indexed = w.b_rows != nullptr;
+                row_index = a_indexed ? w.a_rows : w.b_rows;
+            }
+            const int tiles_n = (n_cols + BN - 1) / BN;
             const int tm = tile / tiles_n, tn = tile % tiles_n;
             rot_a = tn; rot_b = tm;
             row_begin = tm * BM;
-            row_end = p.kc;
+            row_end = m_rows;
             n0 = tn * BN;
             c_begin = p.cum[expert];
             c_len = p.cum[expert + 1] - c_begin;
@@ -410,28 +432,30 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 const int col = (ch8 ^ unit_swz(r)) * 8;
 #pragma unroll
                 for (int u = 0; u < (EDGE ? UB : 1); u++)
-                    b_off[u][l] = (EDGE ? min(u * 64 + col, p.n_cols - 8 - n0) : col) * 2;
+                    b_off[u][l] = (EDGE ? min(u * 64 + col, n_cols - 8 - n0) : col) * 2;
             }
         }
         const int64_t a_base = AKIND == CONTIG ? (GATHER == GATHER_A ? 0 : static_cast<int64_t>(row_begin) * p.lda)
-                                               : row_begin + (GATHER == GATHER_WA ? 0 : static_cast<int64_t>(c_begin) * p.lda);
+                                               : row_begin + (a_indexed ? 0 : static_cast<int64_t>(c_begin) * lda32);
         const int64_t b_base = BKIND == CONTIG ? expert * p.strideB + static_cast<int64_t>(n0) * p.ldb
-                               : WGRAD ? n0 + (GATHER == GATHER_B ? 0 : static_cast<int64_t>(c_begin) * p.ldb)
+                               : WGRAD ? n0 + (b_indexed ? 0 : static_cast<int64_t>(c_begin) * ldb32)
                                        : expert * p.strideB + n0;
         // EPI_SWIGLU: LDS rows 0..31 of a unit are gate rows, 32..63 up rows; a wavefront's loads lie in one of the two
-        const uint16_t *B_first = EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? p.B[1] : p.B[0];
-        a_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(p.A[0] + a_base)));
+        const uint16_t *A_first = GATHER == MERGED ? p.set[product].A : p.A[0];
+        const uint16_t *B_first = GATHER == MERGED ? p.set[product].B : EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? p.B[1] : p.B[0];
+        a_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(A_first + a_base)));
         b_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(B_first + b_base)));
         if (TWO_PHASE) {
             a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.A[1] : p.A[0]) + a_base)));
             b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.B[1] : p.B[0]) + b_base)));
         }
-        if (GATHER_W && expert != cached_expert) {
+        const int cache_key = GATHER == MERGED ? expert * 2 + (row_index != p.set[1].b_rows ? 1 : 0) : expert;
+        if (GATHER_W && (GATHER != MERGED || row_index) && cache_key != cached_expert) {
             // every wavefront is past the barrier that ends the previous tile's main loop, so no one still reads
             // the cache; `expert` is block-uniform, so all take this branch together
             const int n_cached = min(c_len, IDX_CACHE);
-            for (int i = tid; i < n_cached; i += NW * 64) idx_cache[GATHER_W ? i : 0] = p.row_index[c_begin + i];
-            cached_expert = expert;
+            for (int i = tid; i < n_cached; i += NW * 64) idx_cache[GATHER_W ? i : 0] = row_index[c_begin + i];
+            cached_expert = cache_key;
             __syncthreads();
         }
         if (GATHER_W && n_steps > 0) {
@@ -446,12 +470,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     // ---- direct loads of one unit into the buffers of parity P; base: a_step / b_step of the unit's step -------
     auto a_step = [&](int c0, int t) -> const char * {
         const char *q = TWO_PHASE && t >= steps_per_phase ? a_tile[1] : a_tile[0];
-        if (GATHER == GATHER_WA) return q;
+        if (WGRAD && a_indexed) return q;
         return q + (AKIND == CONTIG ? static_cast<uint64_t>(static_cast<uint32_t>(c0)) * 2 : static_cast<uint64_t>(static_cast<uint32_t>(c0)) * static_cast<uint32_t>(lda32 * 2));
     };
     auto b_step = [&](int c0, int t) -> const char * {
         const char *q = TWO_PHASE && t >= steps_per_phase ? b_tile[1] : b_tile[0];
-        if (GATHER == GATHER_B) return q;
+        if (WGRAD && b_indexed) return q;
         return q + (BKIND == CONTIG ? static_cast<uint64_t>(static_cast<uint32_t>(c0)) * 2 : static_cast<uint64_t>(static_cast<uint32_t>(c0)) * static_cast<uint32_t>(ldb32 * 2));
     };
     // bytes of the contraction row (STRIDED): rows past the range re-read its last row (A is zeroed there)
@@ -470,8 +494,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         for (int l = 0; l < L; l++) {
             uint32_t off;
             if (AKIND == CONTIG) off = a_off[AKIND == CONTIG ? U : 0][l] - tail_bytes(c0, l);
-            else off = crow_bytes(c0, l, lda32, rows, GATHER == GATHER_WA) +
-                       (EDGE ? min(a_off[0][l] + U * 128, static_cast<uint32_t>(p.kc - 8 - row_begin) * 2) : a_off[0][l]);
+            else off = crow_bytes(c0, l, lda32, rows, a_indexed) +
+                       (EDGE ? min(a_off[0][l] + U * 128, static_cast<uint32_t>(m_rows - 8 - row_begin) * 2) : a_off[0][l]);
             const char *q = AKIND == CONTIG || EDGE ? base : base + U * 128;
             if (l == 0) dma16_if<P * A_STAGE + U * UNIT>(left, q, off, wave_lds);
             else dma16_if<P * A_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
@@ -483,7 +507,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         for (int l = 0; l < L; l++) {
             uint32_t off = b_off[EDGE ? U : 0][l];
             if (BKIND == CONTIG) off -= tail_bytes(c0, l);
-            else off += crow_bytes(c0, l, ldb32, rows, GATHER == GATHER_B);
+            else off += crow_bytes(c0, l, ldb32, rows, b_indexed);
             const char *q = EDGE ? base : BKIND == CONTIG ? base + U * b_unit : base + U * 128;
             if (l == 0) dma16_if<B0 + P * B_STAGE + U * UNIT>(left, q, off, wave_lds);
             else dma16_if<B0 + P * B_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
@@ -749,21 +773,24 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     if (ACCUM) {
         int lane_o = lane;
         asm volatile("" : "+v"(lane_o));
-        const uint16_t *from = p.C + expert * p.strideC + n0 + wn * 64 + (lane_o % OLD_CPR) * 8;
-        const bool col_in = !EDGE || n0 + wn * 64 + (lane_o % OLD_CPR) * 8 < p.n_cols;
+        const uint16_t *from = (GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + expert * p.strideC) + n0 + wn * 64 + (lane_o % OLD_CPR) * 8;
+        const bool col_in = !EDGE || n0 + wn * 64 + (lane_o % OLD_CPR) * 8 < n_cols;
+        const int64_t ldc = GATHER == MERGED ? n_cols : p.ldc;
         const int m_first = row_begin + wm * 32 + lane_o / OLD_CPR;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int it = 0; it < OLD_ITS; it++) {
                 const int m = m_first + i * 64 + it * (64 / OLD_CPR);
-                if (!EDGE || (col_in && m < p.kc))
+                if (!EDGE || (col_in && m < m_rows))
                     old[ACCUM ? i : 0][ACCUM ? it : 0] =
-                        *reinterpret_cast<const u32x4 *>(from + static_cast<int64_t>(m) * p.ldc);
+                        *reinterpret_cast<const u32x4 *>(from + static_cast<int64_t>(m) * ldc);
             }
     }
 
-    const int e_expert = expert, e_row_begin = row_begin, e_row_end = row_end, e_n0 = n0, e_active = active;
+    uint16_t *Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + (WGRAD ? expert * p.strideC : 0);
+    const int64_t e_ldc = GATHER == MERGED ? n_cols : p.ldc;
+    const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_n0 = n0, e_active = active;
     have = next_tile();
     if (have) prefetch();
 
@@ -799,8 +826,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
     const int col0 = e_n0 + wn_e * COLS;   // first output column
-    uint16_t *Cb = p.C + (WGRAD ? e_expert * p.strideC : 0);
-    const int row_lim = EDGE && col0 + (lane_e % (COLS / 8)) * 8 >= p.n_cols ? 0 : e_row_end;
+    const int row_lim = EDGE && col0 + (lane_e % (COLS / 8)) * 8 >= e_n_cols ? 0 : e_row_end;
     float wrow_all[(ROWW && EPI == EPI_SWIGLU) ? TM : 1];
     if (ROWW && EPI == EPI_SWIGLU) {
 #pragma unroll
@@ -908,7 +934,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 const int q = it * 64 + lane_e;
                 const int64_t m = m0 + q / CPRW;
                 if (m < row_lim) {
-                    const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
+                    const int64_t o = m * e_ldc + col0 + (q % CPRW) * 8;
                     u32x4 v = strip_get(0, q / CPRW, q % CPRW);
                     if (WGRAD && ACCUM) {
                         float fresh[8], prev[8];
@@ -1073,6 +1099,11 @@ extern "C" int om_grouped_gemm_dgrad(const void *output_grad, const void *weight
 }
 
 namespace {
+// 256x256 tiles for the weight gradients unless the `matrices` of [n, k] have too few to occupy half the CUs
+bool wgrad_big_tile(int n, int k, int64_t matrices) {
+    return n % 256 == 0 && k % 256 == 0 && matrices * (n / 256) * (k / 256) * 2 >= device_cu_count();
+}
+
 // weight gradient; gather == GATHER_B: contraction row c of `input` is row index[c] of a
 // [src_rows, K] matrix; gather == GATHER_WA: contraction row c of `output_grad` is row index[c] of a
 // [src_rows, N] matrix (the token gather folded into the loads)
@@ -1098,9 +1129,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
         return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = K; p.kc = N; p.phases = 1;
     hipStream_t st = om_stream(stream);
-    // 256x256 tiles unless they are too few to occupy half the CUs
-    const bool big = N % 256 == 0 && K % 256 == 0 &&
-                     static_cast<int64_t>(G) * (N / 256) * (K / 256) * 2 >= device_cu_count();
+    const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
@@ -1187,6 +1216,89 @@ extern "C" int om_grouped_gemm_wgrad_gathered_out_accumulate(const void *output_
     if (src_rows < 1) return OM_ERR_SHAPE;
     return wgrad_launch(output_grad, input, output_grad_rows, GATHER_WA, src_rows, weight_grad,
                         cum_token_counts, rows, G, N, K, w_stride, stream, true);
+}
+
+namespace {
+// dW_down (+)= dout^T h, dW_gate (+)= dg^T x, dW_up (+)= du^T x, in one launch where that saves rounds of tiles: those of an
+// expert's three gradients come one after the other.
+int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du, const void *x,
+                        const int32_t *x_rows, int64_t src_rows, void *dw_down, void *dw_gate, void *dw_up,
+                        const int32_t *cum_token_counts, int64_t rows, int G, int I, int H, int64_t down_stride,
+                        int64_t gate_stride, int64_t up_stride, bool accumulate, void *stream) {
+    if (rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    if (!dw_down || !dw_gate || !dw_up || !cum_token_counts || (rows > 0 && (!dout || !h || !dg || !du || !x))) return OM_ERR_NULL;
+    if ((dout_rows || x_rows) && src_rows < 1) return OM_ERR_SHAPE;
+    GemmParams p = {};
+    const int64_t packed = static_cast<int64_t>(I) * H;
+    auto set = [&](int i, const void *a, const int32_t *a_rows, const void *b, const int32_t *b_rows, void *c, int64_t stride, int m, int n) {
+        p.set[i] = {static_cast<const uint16_t *>(a), static_cast<const uint16_t *>(b), static_cast<uint16_t *>(c), a_rows, b_rows,
+                    stride ? stride : packed, m, n};
+        return om_aligned16(a) && om_aligned16(b) && om_aligned16(c) && pitch_ok(p.set[i].strideC);
+    };
+    if (!set(0, dout, dout_rows, h, nullptr, dw_down, down_stride, H, I) || !set(1, dg, nullptr, x, x_rows, dw_gate, gate_stride, I, H) ||
+        !set(2, du, nullptr, x, x_rows, dw_up, up_stride, I, H))
+        return OM_ERR_ALIGN;
+    if (!fits_span(rows * H) || !fits_span(rows * I) || ((dout_rows || x_rows) && !fits_gather(src_rows * H))) return OM_ERR_SHAPE;
+    for (const WgradSet &s : p.set)
+        if (!fits_span(s.strideC * G)) return OM_ERR_SHAPE;
+    p.cum = cum_token_counts;
+    p.rows = rows; p.n_experts = G; p.phases = 1;
+    const bool big = wgrad_big_tile(H, I, 3 * static_cast<int64_t>(G));
+    const int tile = big ? 256 : 128;
+    const int64_t each = static_cast<int64_t>((H + tile - 1) / tile) * ((I + tile - 1) / tile), tiles = 3 * each * G;
+    if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
+    // One launch where it saves rounds of tiles, and more of them than the tenth that its kernel is slower by (its operands
+    // are chosen per tile): 12 experts of 1000x712, 576 tiles a product on 512 blocks, 103 -> 72 us; 8 of 256x512, 64
+    // tiles, 38 -> 16.  One of 7168x2048, 224 tiles on 256 blocks and as many rounds either way, 698 -> 774; 64 of
+    // 2048x1024 with 2048 rows, 2048 tiles, 1620 -> 1701.  With few rows an expert, where a launch is stores and its ends
+    // weigh more, one launch as well: those 64 experts with 64 rows each on average, a step of 512 tokens 717 -> 696.
+    const int64_t blocks = static_cast<int64_t>(device_cu_count()) * (big ? 1 : 2);
+    auto rounds = [](int64_t t, int64_t b) { return (t + b - 1) / b; };
+    const bool big_alone = wgrad_big_tile(H, I, G);
+    const int64_t alone = static_cast<int64_t>((H + (big_alone ? 255 : 127)) / (big_alone ? 256 : 128)) *
+                          ((I + (big_alone ? 255 : 127)) / (big_alone ? 256 : 128)) * G;
+    const int64_t blocks_alone = static_cast<int64_t>(device_cu_count()) * (big_alone ? 1 : 2);
+    if (rows > 256 * static_cast<int64_t>(G) && big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone)) {
+        const int gather_d = dout_rows ? GATHER_WA : GATHER_NONE, gather_x = x_rows ? GATHER_B : GATHER_NONE;
+        int code = wgrad_launch(dout, h, dout_rows, gather_d, dout_rows ? src_rows : 0, dw_down, cum_token_counts, rows, G, H, I,
+                                down_stride, stream, accumulate);
+        if (code == OM_OK)
+            code = wgrad_launch(dg, x, x_rows, gather_x, x_rows ? src_rows : 0, dw_gate, cum_token_counts, rows, G, I, H,
+                                gate_stride, stream, accumulate);
+        if (code == OM_OK)
+            code = wgrad_launch(du, x, x_rows, gather_x, x_rows ? src_rows : 0, dw_up, cum_token_counts, rows, G, I, H,
+                                up_stride, stream, accumulate);
+        return code;
+    }
+    p.tiles_e = static_cast<int>(3 * each);
+    p.total_tiles = static_cast<int>(tiles);
+    const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
+    hipStream_t st = om_stream(stream);
+    if (big && accumulate) ggemm_kernel<256, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, true><<<grid, block, 0, st>>>(p);
+    else if (big) ggemm_kernel<256, STRIDED, STRIDED, EPI_WGRAD, MERGED><<<grid, block, 0, st>>>(p);
+    else if (accumulate) ggemm_kernel<128, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, true, true><<<grid, block, 0, st>>>(p);
+    else ggemm_kernel<128, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, false, true><<<grid, block, 0, st>>>(p);
+    return om_launch_status();
+}
+}  // namespace
+
+extern "C" int om_grouped_gemm_wgrad_merged(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
+                                            const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
+                                            void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                            int64_t rows, int G, int I, int H, int64_t down_stride,
+                                            int64_t gate_stride, int64_t up_stride, void *stream) {
+    return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
+                               cum_token_counts, rows, G, I, H, down_stride, gate_stride, up_stride, false, stream);
+}
+
+extern "C" int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const int32_t *dout_rows, const void *h,
+                                                       const void *dg, const void *du, const void *x,
+                                                       const int32_t *x_rows, int64_t src_rows, void *dw_down,
+                                                       void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                                       int64_t rows, int G, int I, int H, int64_t down_stride,
+                                                       int64_t gate_stride, int64_t up_stride, void *stream) {
+    return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
+                               cum_token_counts, rows, G, I, H, down_stride, gate_stride, up_stride, true, stream);
 }
 
 namespace {

@@ -454,6 +454,27 @@ struct Sinks {
     static Tensor fresh(const Sink &s) { return s.accumulate ? Tensor() : s.grad; }
 };
 
+// All three weight gradients of a bf16 merged MLP: one call where all are written or all are added into their sinks.
+// dout_rows / x_rows: rows of dout / x taken through an index.
+void wgrads(const Call &c, const Tensor &dout, const int32_t *dout_rows, const Tensor &h, const Tensor &dg, const Tensor &du,
+            const Tensor &x, const int32_t *x_rows, const Sinks &k, const int32_t *cum, int64_t rows, int64_t G, int64_t I,
+            int64_t H) {
+    if (k.gate.accumulate == k.up.accumulate && k.gate.accumulate == k.down.accumulate) {
+        const int64_t src_rows = dout_rows ? dout.size(0) : x.size(0);
+#define OM_W(fn)                                                                                                        \
+    OM(c, fn, ptr(dout), dout_rows, ptr(h), ptr(dg), ptr(du), ptr(x), x_rows, src_rows, ptr(k.down.grad), ptr(k.gate.grad), \
+       ptr(k.up.grad), cum, rows, G, I, H, k.down.pitch, k.gate.pitch, k.up.pitch, c.stream)
+        if (k.gate.accumulate) OM_W(om_grouped_gemm_wgrad_merged_accumulate);
+        else OM_W(om_grouped_gemm_wgrad_merged);
+#undef OM_W
+        return;
+    }
+    wgrad(c, dout, h, k.down, cum, rows, G, H, I, dout_rows ? WgradRows::OUTPUT_GRAD : WgradRows::PLAIN, dout_rows, dout.size(0));
+    const WgradRows kind = x_rows ? WgradRows::INPUT : WgradRows::PLAIN;
+    wgrad(c, dg, x, k.gate, cum, rows, G, I, H, kind, x_rows, x.size(0));
+    wgrad(c, du, x, k.up, cum, rows, G, I, H, kind, x_rows, x.size(0));
+}
+
 // Backward of merged_forward: returns dx (of the gathered matrix when x_rows is set); the weight
 // gradients go into the sinks.
 Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeights &w, const int32_t *cum,
@@ -472,12 +493,9 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
            expert_stride(w.gate), expert_stride(w.up), c.stream);
         return dx;
     }
-    wgrad(c, dy, s.h, k.down, cum, rows, G, H, I);
     OM(c, om_merged_mlp_down_dgrad, ptr(dy), ptr(w.down), ptr(s.g), ptr(s.u), ptr(dg), ptr(du), cum, rows, G, I, H,
        expert_stride(w.down), c.stream);
-    const WgradRows kind = x_rows && rows > 0 ? WgradRows::INPUT : WgradRows::PLAIN;
-    wgrad(c, dg, x, k.gate, cum, rows, G, I, H, kind, x_rows, x.size(0));
-    wgrad(c, du, x, k.up, cum, rows, G, I, H, kind, x_rows, x.size(0));
+    wgrads(c, dy, nullptr, s.h, dg, du, x, rows > 0 ? x_rows : nullptr, k, cum, rows, G, I, H);
     OM(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx), cum, rows, G, I, H,
        expert_stride(w.gate), c.stream);
     return dx;
@@ -539,14 +557,12 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
             const int parts = om_merged_mlp_row_dot_parts(I);
             if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
             Tensor row_dot = make({parts, rows}, x, at::kFloat);
-            wgrad(c, dfinal, s.h, k.down, ix.cum, rows, G, H, I, WgradRows::OUTPUT_GRAD, ix.in, T);
             OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
                      ix.row_weights ? ix.row_weights : fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows,
                      ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
             OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
                c.stream);
-            wgrad(c, dg, x, k.gate, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
-            wgrad(c, du, x, k.up, ix.cum, rows, G, I, H, WgradRows::INPUT, ix.in, T);
+            wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, G, I, H);
             OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
                      ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
         } else {   // nothing routed to these experts: fresh weight gradients are zero, live ones stay as they are

@@ -72,6 +72,45 @@ def test_accumulate_entry_points_equal_gemm_then_add(cuda, form, kind, G, rows, 
     assert (bits(acc) == bits(expect)).all()
 
 
+# both tile shapes, one launch and three, extents that no tile divides, experts without rows, one with more rows than the
+# block keeps indices of in LDS
+@pytest.mark.parametrize("kind,G,rows,I,H", [("ragged", 8, 4096, 512, 256), ("ragged", 12, 9003, 712, 1000), ("empties", 16, 777, 128, 256),
+                                             ("ragged", 64, 4096, 1024, 2048), ("uniform", 22, 11000, 512, 1024), ("onehot", 5, 5000, 256, 512),
+                                             ("uniform", 1, 300, 264, 136), ("ragged", 3, 5, 8, 72), ("uniform", 4, 0, 128, 128)])
+@pytest.mark.parametrize("indexed", [False, True])
+def test_three_weight_gradients_of_a_merged_mlp(cuda, indexed, kind, G, rows, I, H):
+    """One bf16 rounding of a float32 sum over an expert's rows (2^-8 of the value, and the order of the sum); the
+    accumulating form equals torch's in-place add of what the writing form gives, bit for bit."""
+    from optimus import _native as n
+    g = torch.Generator().manual_seed(rows + I)
+    T = max(rows // 2, 8)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(cuda)
+    dout, x, h, dg, du = rnd(T if indexed else max(rows, 1), H), rnd(T if indexed else max(rows, 1), H), rnd(max(rows, 1), I), rnd(max(rows, 1), I), rnd(max(rows, 1), I)
+    idx = torch.randint(0, T, (max(rows, 1),), generator=g, dtype=torch.int32).to(cuda)
+    cum = _counts(kind, G, rows) if rows else torch.zeros(G + 1, dtype=torch.int32)
+    d, P, ix = cum.to(cuda), n.ptr, idx if indexed else None
+    pitch = I * H + 64
+    old = [rnd(G * pitch) for _ in range(3)]
+    fresh, acc = [torch.full_like(o, 7.0) for o in old], [o.clone() for o in old]
+    p = lambda t: None if t is None else P(t)
+    for suffix, out in (("", fresh), ("_accumulate", acc)):
+        _call("om_grouped_gemm_wgrad_merged" + suffix, P(dout), p(ix), P(h), P(dg), P(du), P(x), p(ix), T, *(P(o) for o in out),
+              P(d), rows, G, I, H, pitch, pitch, pitch)
+    torch.cuda.synchronize()
+    dr, xr = (t[idx.long()] if indexed else t for t in (dout, x))
+    for i, (a, b, m, k) in enumerate(((dr, h, H, I), (dg, xr, I, H), (du, xr, I, H))):
+        view = lambda t: torch.as_strided(t, (G, m, k), (pitch, k, 1))
+        for e in range(G):
+            s = slice(int(cum[e]), int(cum[e + 1]))
+            want = a[s].float().t() @ b[s].float()
+            err = (view(fresh[i])[e].float() - want).abs()
+            assert (err <= want.abs() * 2 ** -8 + 2e-5 * max(s.stop - s.start, 1) ** 0.5).all(), (i, e)
+        expect = old[i].clone()
+        view(expect).add_(view(fresh[i]))
+        assert (bits(acc[i]) == bits(expect)).all(), i
+        assert (torch.as_strided(fresh[i], (G, 64), (pitch, 1), I * H) == 7.0).all()
+
+
 def test_accumulate_f32(cuda):
     from optimus import _native as n
     g = torch.Generator().manual_seed(5)
