@@ -649,6 +649,25 @@ int om_merged_mlp_gate_up_wgrad_f32(const float *dg, const float *du, const floa
                                     int64_t rows, int G, int I, int H, int64_t gate_stride, int64_t up_stride,
                                     int accumulate, void *stream);
 
+/* The end of the float32 merged MLP's backward in one launch: dx = dg W_gate + du W_up (rows as dg), dw_down = dy^T h,
+ * dw_gate = dg^T x and dw_up = du^T x (`_accumulate`: added to what the three hold).  None depends on another, and the
+ * launches of a small layer leave most of the chip idle each.  x_rows as above.                                      */
+int om_grouped_gemm_wgrad_merged_dgrad_f32(const float *dy, const float *h, const float *dg, const float *du,
+                                           const float *x, const int32_t *x_rows, int64_t src_rows,
+                                           const float *w_gate, const float *w_up, float *dx, float *dw_down,
+                                           float *dw_gate, float *dw_up, const int32_t *cum_token_counts,
+                                           int64_t rows, int G, int I, int H, int64_t gate_stride,
+                                           int64_t up_stride, int64_t dw_down_stride, int64_t dw_gate_stride,
+                                           int64_t dw_up_stride, void *stream);
+int om_grouped_gemm_wgrad_merged_dgrad_f32_accumulate(const float *dy, const float *h, const float *dg,
+                                                      const float *du, const float *x, const int32_t *x_rows,
+                                                      int64_t src_rows, const float *w_gate, const float *w_up,
+                                                      float *dx, float *dw_down, float *dw_gate, float *dw_up,
+                                                      const int32_t *cum_token_counts, int64_t rows, int G,
+                                                      int I, int H, int64_t gate_stride, int64_t up_stride,
+                                                      int64_t dw_down_stride, int64_t dw_gate_stride,
+                                                      int64_t dw_up_stride, void *stream);
+
 /* Stand-alone SwiGLU glue (moe.py:401-402 forward; moe.py:37-41 and :133-147 backward),
  * for callers that keep the three GEMMs separate.  n elements, dtype OM_F32 or OM_BF16.   */
 int om_swiglu_fwd(const void *g, const void *u, void *h, int64_t n, int dtype, void *stream);

@@ -484,11 +484,22 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
     Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx = make({rows, H}, x);
     ProfiledScope scope(c, "1moeblock--7gmlp_bwd");
     if (x.scalar_type() == at::kFloat) {
-        wgrad_f32(c, dy, s.h, k.down, cum, rows, G, H, I);
         OM(c, om_merged_mlp_down_dgrad_f32, fp(dy), fp(w.down), fp(s.g), fp(s.u), fpm(dg), fpm(du), cum, rows, G, I, H,
            expert_stride(w.down), c.stream);
-        OM(c, om_merged_mlp_gate_up_wgrad_f32, fp(dg), fp(du), fp(x), rows ? x_rows : nullptr, x.size(0), fpm(k.gate.grad),
-           fpm(k.up.grad), cum, rows, G, I, H, k.gate.pitch, k.up.pitch, k.gate.accumulate | k.up.accumulate << 1, c.stream);
+        const int32_t *rows_of_x = rows ? x_rows : nullptr;
+        if (k.gate.accumulate == k.up.accumulate && k.gate.accumulate == k.down.accumulate) {
+#define OM_W(fn)                                                                                                           \
+    OM(c, fn, fp(dy), fp(s.h), fp(dg), fp(du), fp(x), rows_of_x, x.size(0), fp(w.gate), fp(w.up), fpm(dx), fpm(k.down.grad), \
+       fpm(k.gate.grad), fpm(k.up.grad), cum, rows, G, I, H, expert_stride(w.gate), expert_stride(w.up), k.down.pitch,         \
+       k.gate.pitch, k.up.pitch, c.stream)
+            if (k.gate.accumulate) OM_W(om_grouped_gemm_wgrad_merged_dgrad_f32_accumulate);
+            else OM_W(om_grouped_gemm_wgrad_merged_dgrad_f32);
+#undef OM_W
+            return dx;
+        }
+        wgrad_f32(c, dy, s.h, k.down, cum, rows, G, H, I);
+        OM(c, om_merged_mlp_gate_up_wgrad_f32, fp(dg), fp(du), fp(x), rows_of_x, x.size(0), fpm(k.gate.grad), fpm(k.up.grad), cum,
+           rows, G, I, H, k.gate.pitch, k.up.pitch, k.gate.accumulate | k.up.accumulate << 1, c.stream);
         OM(c, om_merged_mlp_gate_up_dgrad_f32, fp(dg), fp(du), fp(w.gate), fp(w.up), fpm(dx), cum, rows, G, I, H,
            expert_stride(w.gate), expert_stride(w.up), c.stream);
         return dx;

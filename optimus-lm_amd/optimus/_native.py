@@ -169,6 +169,10 @@ SIGNATURES = {
     "om_merged_mlp_gate_up_dgrad_f32": (c_int, [c_void_p] * 6 + [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_void_p]),
     "om_merged_mlp_gate_up_wgrad_f32": (c_int, [c_void_p] * 4 + [c_i64] + [c_void_p] * 3 +
                                         [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_int, c_void_p]),
+    "om_grouped_gemm_wgrad_merged_dgrad_f32": (c_int, [c_void_p] * 6 + [c_i64] + [c_void_p] * 7
+                                              + [c_i64, c_int, c_int, c_int] + [c_i64] * 5 + [c_void_p]),
+    "om_grouped_gemm_wgrad_merged_dgrad_f32_accumulate": (c_int, [c_void_p] * 6 + [c_i64] + [c_void_p] * 7 +
+                                                          [c_i64, c_int, c_int, c_int] + [c_i64] * 5 + [c_void_p]),
     "om_swiglu_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_void_p]),
     "om_swiglu_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int,
                               c_void_p]),

@@ -247,6 +247,56 @@ def test_grouped_gemm_float32(cuda, kind, G, rows, N, K):
         assert float(wd.grad[empty.to(cuda)].abs().max()) == 0.0
 
 
+# row tiles of 32 and of 64, contractions of 1 to 5 steps of 32 and partial ones, more rows in an expert than the kernel keeps
+# indices of in LDS, no rows at all
+@pytest.mark.parametrize("counts,I,H", [([31, 32, 33, 0, 1, 63, 64, 65], 40, 72), ([96, 97, 128, 160, 159, 5], 160, 96), ([1100, 7, 300], 64, 32),
+                                        ([512, 530, 490, 515, 700, 300, 512, 537], 512, 256), ([2000, 2048], 136, 520), ([0, 0, 0], 64, 64)])
+@pytest.mark.parametrize("indexed", [False, True])
+def test_float32_input_and_weight_gradients_in_one_launch(cuda, indexed, counts, I, H):
+    """dx and the three weight gradients (written, and added to old values) against float64, and forward and SwiGLU backward of
+    the same sizes: a few float32 roundings of the absolute sum."""
+    from optimus import _native as n
+    g = torch.Generator().manual_seed(sum(counts) + I)
+    G, rows = len(counts), sum(counts)
+    R, T = max(rows, 1), max(rows // 2, 4)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(cuda)
+    x, idx = rnd(T if indexed else R, H), torch.randint(0, T, (R,), generator=g, dtype=torch.int32).to(cuda)
+    dy, h, dg, du, wg, wu, wd = rnd(R, H), rnd(R, I), rnd(R, I), rnd(R, I), rnd(G, I, H) * 0.05, rnd(G, I, H) * 0.05, rnd(G, H, I) * 0.05
+    gq, uq, hq, dgq, duq, dx = rnd(R, I), rnd(R, I), rnd(R, I), rnd(R, I), rnd(R, I), rnd(R, H)
+    shapes = ((G, H, I), (G, I, H), (G, I, H))
+    fresh, old = [torch.full(s, 7.0, device=cuda) for s in shapes], [rnd(*s) for s in shapes]
+    acc, d, P, L = [o.clone() for o in old], cum.to(cuda), n.ptr, n.lib()
+    ix = P(idx) if indexed else None
+    for suffix, out in (("", fresh), ("_accumulate", acc)):
+        n.check(getattr(L, "om_grouped_gemm_wgrad_merged_dgrad_f32" + suffix)(
+            P(dy), P(h), P(dg), P(du), P(x), ix, T, P(wg), P(wu), P(dx), *(P(o) for o in out), P(d), rows, G, I, H, 0, 0, 0, 0, 0, n.stream()), "bwd")
+    n.check(L.om_merged_mlp_gate_up_fwd_f32(P(x), ix, T, P(wg), P(wu), P(gq), P(uq), P(hq), P(d), rows, G, I, H, 0, 0, n.stream()), "fwd")
+    n.check(L.om_merged_mlp_down_dgrad_f32(P(dy), P(wd), P(gq), P(uq), P(dgq), P(duq), P(d), rows, G, I, H, 0, n.stream()), "dgrad")
+    torch.cuda.synchronize()
+    D = lambda t: t.double()
+
+    def close(name, got, want, scale, roundings=2e-6):
+        assert ((D(got) - want).abs() <= roundings * scale + 1e-30).all(), name
+    xr = x[idx.long()] if indexed else x
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        for i, (a, b) in enumerate(((dy, h), (dg, xr), (du, xr))):
+            want, scale = D(a[s]).t() @ D(b[s]), D(a[s]).abs().t() @ D(b[s]).abs()
+            close(("dw", i, e), fresh[i][e], want, scale)
+            assert torch.equal(acc[i][e], old[i][e] + fresh[i][e])
+        close(("dx", e), dx[s], D(dg[s]) @ D(wg[e]) + D(du[s]) @ D(wu[e]), D(dg[s]).abs() @ D(wg[e]).abs() + D(du[s]).abs() @ D(wu[e]).abs())
+        for name, got, w in (("g", gq, wg), ("u", uq, wu)):
+            close((name, e), got[s], D(xr[s]) @ D(w[e]).t(), D(xr[s]).abs() @ D(w[e]).abs().t())
+        dh, G64, U64 = D(dy[s]) @ D(wd[e]), D(gq[s]), D(uq[s])
+        sg, size = torch.sigmoid(G64), D(dy[s]).abs() @ D(wd[e]).abs()
+        # (the factors beside dh: a few roundings of their own)
+        close(("du", e), duq[s], dh * G64 * sg, size * (G64 * sg).abs(), 4e-6)
+        close(("dg", e), dgq[s], dh * U64 * sg * (1 + G64 * (1 - sg)), size * U64.abs() * sg * (1 + G64.abs()), 4e-6)
+        close(("h", e), hq[s], G64 * sg * U64, (G64 * U64).abs() * sg, 4e-6)
+
+
 # sizes of the seeded sweeps: multiples of 128, and multiples of 8 only (partial last tiles along every
 # extent, a last contraction step with 8 to 56 indices)
 SWEEP_SIZES = {"multiples_of_128": ([128, 256, 384, 512, 1024], [128, 256, 384, 640, 1024]),
