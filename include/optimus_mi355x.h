@@ -180,7 +180,8 @@ int om_router_gate_logits_split(const void *x, const void *gate_weight, int64_t 
                                 void *stream);
 
 /* The whole router for a bf16 gate of any shape (N <= 256, H a multiple of 8): the projection split over
- * slices of H, then one launch that adds the slices in order, writes the logits and routes.
+ * slices of H, then one launch that adds the slices in order, writes the logits and routes (both in one launch for
+ * more than 512 tokens, at most 64 experts and an H that is a multiple of 512; the same bits).
  *   om_router_gate_split_softmax_topk       : the softmax router above; logits_out in logits_dtype (OM_BF16:
  *       rounded to bf16 before the softmax, the logits of a bf16 linear layer)
  *   om_router_gate_split_sigmoid_group_topk : the DeepSeek-V3 router (om_route_sigmoid_group_topk below)

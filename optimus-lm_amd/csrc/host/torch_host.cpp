@@ -925,11 +925,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
     refuse_transforms({x, weight});
     require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
-    // Up to 2048 tokens the one-pass kernel has at most 64 blocks, each walking all of H: the projection split
-    // over H and a routing launch behind it give the same bits (eight slices added in the one-pass order)
-    // sooner.  us, one launch -> two, hidden 2048 and 64 experts: 64 tokens 22 -> 11, 512 22 -> 15, 2048 24 -> 17,
-    // 4096 24 -> 20, 8192 27 -> 29; hidden 1024 and 32 experts: 512 10.6 -> 8.4, 4096 11.3 -> 12.0; hidden 512 even.
-    if (one_pass && !bf16_logits && T > 0 && T <= 2048 && N <= 64 && H >= 1024 && H % 512 == 0) one_pass = false;
+    // Few tokens: one CU would take in all of the gate weight, the projection split over the chip and a launch behind it
+    // are sooner (om_router_gate_split_softmax_topk, which has the figures).
+    if (one_pass && T <= 512 && N <= 64 && H >= 1024 && H % 512 == 0) one_pass = false;
     Tensor logits, weights, experts;
     {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -439,6 +439,204 @@ __global__ __launch_bounds__(WAVES * 64) void gate_route_kernel(
     }
 }
 
+// Within each row of 16 lanes.  The sum adds lanes 8 apart first, then 4, 2 and 1, as the last steps of wave_sum do.
+#define OM_ROW_STEP(x, ctrl) __builtin_amdgcn_update_dpp(0, x, ctrl, 0xf, 0xf, true)
+__device__ __forceinline__ float row_max(float v) {
+    v = fmaxf(v, __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x128)));    // row_ror:8
+    v = fmaxf(v, __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x124)));    // row_ror:4
+    v = fmaxf(v, __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x4E)));     // quad_perm [2,3,0,1]
+    return fmaxf(v, __int_as_float(OM_ROW_STEP(__float_as_int(v), 0xB1)));  // quad_perm [1,0,3,2]
+}
+__device__ __forceinline__ int row_min(int v) {
+    v = min(v, OM_ROW_STEP(v, 0x128));
+    v = min(v, OM_ROW_STEP(v, 0x124));
+    v = min(v, OM_ROW_STEP(v, 0x4E));
+    return min(v, OM_ROW_STEP(v, 0xB1));
+}
+__device__ __forceinline__ float row_sum(float v) {
+    v += __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x128));
+    v += __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x124));
+    v += __int_as_float(OM_ROW_STEP(__float_as_int(v), 0x4E));
+    return v + __int_as_float(OM_ROW_STEP(__float_as_int(v), 0xB1));
+}
+#undef OM_ROW_STEP
+
+// softmax_in_place and select_topk for four tokens in a wavefront, a row of 16 lanes each: lane l of a row holds
+// the logits of experts l + 16 * j in p[j] (past N: -inf), the lane of rank r < K <= 16 gets the r-th winner.  The same
+// bits as with a wavefront per token: the sum pairs the same experts, the selection order is total.
+// One CU routes the 32 tokens of a block, so it is vector-instruction issue that counts: a round of selection is
+// about as many instructions here for four tokens as there for one.
+template <int Q>
+__device__ __forceinline__ void row_softmax_topk(float (&p)[Q], int N, int K, int l16, float &my_v, int &my_i) {
+    float mx = p[0];
+#pragma unroll
+    for (int j = 1; j < Q; j++) mx = fmaxf(mx, p[j]);
+    mx = row_max(mx);
+#pragma unroll
+    for (int j = 0; j < Q; j++) p[j] = l16 + 16 * j < N ? expf(p[j] - mx) : 0.0f;
+    const float sum = row_sum(Q == 4 ? (p[0] + p[2]) + (p[1] + p[3]) : p[0] + p[1]);
+#pragma unroll
+    for (int j = 0; j < Q; j++) p[j] = l16 + 16 * j < N ? p[j] / sum : -INFINITY;
+    my_v = 0.0f;
+    my_i = 0;
+    for (int r = 0; r < K; r++) {
+        float bv = -INFINITY;
+        int bi = 0x7fffffff;
+#pragma unroll
+        for (int j = 0; j < Q; j++)
+            if (p[j] > bv) { bv = p[j]; bi = l16 + 16 * j; }   // ascending experts: the first maximum wins
+        const float m = row_max(bv);
+        const int i = row_min(bv == m ? bi : 0x7fffffff);
+        if (l16 == r) { my_v = m; my_i = i; }
+#pragma unroll
+        for (int j = 0; j < Q; j++)
+            if (l16 + 16 * j == i) p[j] = -INFINITY;           // taken
+    }
+}
+
+// The same for at most 64 experts and hidden sizes that are multiples of 512.  What bounds it is how fast a CU takes in
+// 32 rows of x and the whole gate weight (256 KB for 64 experts at hidden 2048), so everything comes by direct loads of
+// whole 64-byte row pieces, two steps ahead, through a ring of three steps in LDS: a step is 32 columns of each of eight
+// slices of H, a slice has a wavefront for each 32 experts (NB), and those share the slice's rows of x.  Slices are added
+// in their order, whatever the number of tokens.  TL: the logits' type; bf16 logits are rounded before the softmax, as a
+// bf16 linear layer returns them.
+// us with the routing (before: eight wavefronts over eight slices with fragments straight from global memory, 32-byte
+// pieces of 64 rows at a time): 64 experts, hidden 2048: 4096 tokens 10.7 (22.0), 16384 tokens 23.6 (38.0: 2.8 TB/s of x
+// now); 32 experts, hidden 1024: 512 tokens 4.9 (9.0), 16384 tokens 11.0 (20.6).
+typedef __attribute__((address_space(3))) char *lds_bytes;
+// 16 bytes from each lane's address to LDS at m0 + 16 * lane.  Outside the compiler's view: the code waits itself.
+__device__ __forceinline__ void dma16(const char *lane_address, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(lane_address) : "memory");
+}
+
+template <int NB, typename TL, typename TW, bool ROUTE>
+__global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg,
+                                                                     int64_t Tn, int H, int N, int K, int renorm,
+                                                                     TL *__restrict__ logits_out, TW *__restrict__ weights_out,
+                                                                     int64_t *__restrict__ experts_out) {
+    constexpr int NP = NB * 32, SLICES = 8, WAVES = NB * SLICES, SLOTS = 3;
+    constexpr int UNITS = 2 + 2 * NB;                       // 1 KB loads (16 rows of 64 bytes) of a slice's step: x, then weight
+    constexpr int LOADS = UNITS / NB;                       // of which each wavefront issues
+    constexpr int SLICE_BYTES = UNITS * 1024, STEP_BYTES = SLICES * SLICE_BYTES;
+    constexpr int LD = NP + 8;                              // (the two halves of a wavefront store to different banks)
+    static_assert(SLOTS * STEP_BYTES >= SLICES * 32 * LD * 4, "the partial sums take the ring's place");
+    __shared__ __attribute__((aligned(1024))) char lds[SLOTS * STEP_BYTES];
+    float (*part)[32][LD] = reinterpret_cast<float (*)[32][LD]>(lds);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int slice = wave / NB, nb = wave % NB;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 32;
+    const int steps = H / (SLICES * 32);                    // at least two
+    const int r32 = lane & 31;
+    // Chunk c (16 bytes) of a 64-byte row r is stored at c ^ (r / 4 % 4): fragment reads of 16 rows use every bank once.
+    const char *src[LOADS];
+    uint32_t dst[LOADS];
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes)lds));
+#pragma unroll
+    for (int l = 0; l < LOADS; l++) {
+        const int unit = nb * LOADS + l, row = (unit < 2 ? unit : unit - 2) * 16 + (lane >> 2);
+        const int column = slice * (H / SLICES) + ((lane & 3) ^ (lane >> 4)) * 8;
+        // rows past the end (tokens, experts): valid memory, results unused
+        src[l] = reinterpret_cast<const char *>(unit < 2 ? x + min(t0 + row, Tn - 1) * H + column
+                                                         : wg + static_cast<int64_t>(min(row, N - 1)) * H + column);
+        dst[l] = lds0 + slice * SLICE_BYTES + unit * 1024;
+    }
+    auto issue = [&](int step, int slot) {
+#pragma unroll
+        for (int l = 0; l < LOADS; l++) dma16(src[l] + step * 64, dst[l] + slot * STEP_BYTES);
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
+    issue(0, 0);
+    issue(1, 1);
+    int slot = 0, free_slot = 2;
+    for (int s = 0; s < steps; s++) {
+        // This wavefront's part of step s has landed (step s + 1 may be outstanding); behind the barrier everyone's has, and
+        // everyone has read step s - 1, whose slot takes step s + 2.
+        if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 2 < steps) issue(s + 2, free_slot);
+        const char *at = lds + slot * STEP_BYTES + slice * SLICE_BYTES + r32 * 64;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int o = ((u * 2 + (lane >> 5)) ^ (r32 >> 2 & 3)) << 4;
+            const u32x4 a = *reinterpret_cast<const u32x4 *>(at + o);
+            const u32x4 b = *reinterpret_cast<const u32x4 *>(at + 2048 + nb * 2048 + o);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+        }
+        free_slot = slot;
+        slot = slot == SLOTS - 1 ? 0 : slot + 1;
+    }
+    __syncthreads();                                        // every step has been read
+    // accumulator element r of lane l: token (r/4)*8 + (l/32)*4 + r%4, expert nb*32 + l%32
+#pragma unroll
+    for (int r = 0; r < 16; r++) part[slice][(r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)][nb * 32 + r32] = acc[r];
+    __syncthreads();
+    if (!ROUTE || K <= 16) {                                // a row of 16 lanes per token
+        constexpr int Q = NP / 16;
+        const int l16 = lane & 15, tk = wave * 4 + (lane >> 4);
+        if (wave >= 8) return;
+        float p[Q];
+#pragma unroll
+        for (int j = 0; j < Q; j++) p[j] = part[0][tk][l16 + 16 * j];
+#pragma unroll
+        for (int s = 1; s < SLICES; s++)
+#pragma unroll
+            for (int j = 0; j < Q; j++) p[j] += part[s][tk][l16 + 16 * j];
+        const bool inside = t0 + tk < Tn;
+#pragma unroll
+        for (int j = 0; j < Q; j++) {
+            const int n = l16 + 16 * j;
+            if (logits_out && inside && n < N) Elem<TL>::store(logits_out + (t0 + tk) * N + n, p[j]);
+            if (sizeof(TL) == 2) p[j] = bf16_bits_to_f32(f32_to_bf16_bits(p[j]));
+            if (n >= N) p[j] = -INFINITY;
+        }
+        if (!ROUTE) return;
+        float w; int e;
+        row_softmax_topk<Q>(p, N, K, l16, w, e);
+        if (renorm) w = w / row_sum(l16 < K ? w : 0.0f);
+        if (inside && l16 < K) {
+            Elem<TW>::store(weights_out + (t0 + tk) * K + l16, w);
+            experts_out[(t0 + tk) * K + l16] = e;
+        }
+        return;
+    }
+    for (int tk = wave; tk < 32 && t0 + tk < Tn; tk += WAVES) {   // a wavefront per token
+        float p[1] = {-INFINITY};
+        if (lane < N) {
+            p[0] = part[0][tk][lane];
+#pragma unroll
+            for (int s = 1; s < SLICES; s++) p[0] += part[s][tk][lane];
+            if (logits_out) Elem<TL>::store(logits_out + (t0 + tk) * N + lane, p[0]);
+            if (sizeof(TL) == 2) p[0] = bf16_bits_to_f32(f32_to_bf16_bits(p[0]));
+        }
+        softmax_in_place<1>(N, lane, p);
+        float w; int e;
+        select_topk<1>(p, N, K, lane, w, e);
+        if (renorm) w = w / wave_sum(lane < K ? w : 0.0f);
+        if (lane < K) {
+            Elem<TW>::store(weights_out + (t0 + tk) * K + lane, w);
+            experts_out[(t0 + tk) * K + lane] = e;
+        }
+    }
+}
+
+// shapes of gate_route_slices_kernel
+inline bool gate_slices_fit(int H, int N) { return N <= 64 && H % 512 == 0; }
+
+template <typename TL, typename TW, bool ROUTE>
+int launch_gate_slices(const void *x, const void *wg, int64_t T, int H, int N, int K, int renorm, void *logits_out,
+                       void *weights_out, int64_t *experts_out, hipStream_t st) {
+    const unsigned nb = static_cast<unsigned>((T + 31) / 32);
+    const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(wg);
+    TL *lo = static_cast<TL *>(logits_out);
+    TW *wo = static_cast<TW *>(weights_out);
+    if (N <= 32) gate_route_slices_kernel<1, TL, TW, ROUTE><<<nb, 512, 0, st>>>(xp, wp, T, H, N, K, renorm, lo, wo, experts_out);
+    else gate_route_slices_kernel<2, TL, TW, ROUTE><<<nb, 1024, 0, st>>>(xp, wp, T, H, N, K, renorm, lo, wo, experts_out);
+    return om_launch_status();
+}
+
 template <bool ROUTE, typename TW>
 int launch_gate(const void *x, const void *wg, int64_t T, int H, int N, int K, int renorm,
                 float *logits_out, void *weights_out, int64_t *experts_out, hipStream_t st) {
@@ -451,9 +649,11 @@ int launch_gate(const void *x, const void *wg, int64_t T, int H, int N, int K, i
         gate_route_kernel<NB, WAVES, UNR, PER, TW, ROUTE><<<nb, WAVES * 64, 0, st>>>(             \
             xp, wp, T, H, N, K, renorm, logits_out, wo, experts_out);                             \
     } while (0)
-    if (N <= 32) OM_GATE(1, 8, 4, 1);
-    else if (N <= 64) OM_GATE(2, 8, 4, 1);
-    else if (N <= 128) OM_GATE(4, 8, 2, 2);
+    if (N <= 64) {
+        if (!gate_slices_fit(H, N)) return OM_ERR_SHAPE;
+        return launch_gate_slices<float, TW, ROUTE>(x, wg, T, H, N, K, renorm, logits_out, weights_out, experts_out, st);
+    }
+    if (N <= 128) OM_GATE(4, 8, 2, 2);
     else OM_GATE(8, 4, 1, 4);
 #undef OM_GATE
     return om_launch_status();
@@ -694,16 +894,19 @@ extern "C" int om_router_gate_softmax_topk(const void *x, const void *gate_weigh
 
 namespace {
 // What the two entry points below have in common: the projection's slices into the workspace.
-int gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, void *workspace, int64_t workspace_bytes,
-                  void *stream, int &splits) {
+int gate_operands(const void *x, const void *gate_weight, int64_t T, int H, int N, const void *workspace,
+                  int64_t workspace_bytes) {
     const int64_t need = om_router_gate_route_workspace_bytes(T, H, N);
     if (need < 0) return static_cast<int>(need);
     if (!x || !gate_weight || !workspace) return OM_ERR_NULL;
     if (!om_aligned16(x) || !om_aligned16(gate_weight) || !om_aligned16(workspace)) return OM_ERR_ALIGN;
-    if (workspace_bytes < need) return OM_ERR_WORKSPACE;
-    splits = om_gate_route_splits(T, H, N);
+    return workspace_bytes < need ? OM_ERR_WORKSPACE : OM_OK;
+}
+
+int gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, void *workspace, void *stream) {
+    const int splits = om_gate_route_splits(T, H, N);
     om_launch_gate_partials(x, gate_weight, T, H, N, splits, static_cast<float *>(workspace), om_stream(stream));
-    return OM_OK;
+    return splits;
 }
 }  // namespace
 
@@ -716,10 +919,22 @@ extern "C" int om_router_gate_split_softmax_topk(const void *x, const void *gate
     if (T < 0 || N < 1 || K < 1 || K > N || K > 64) return OM_ERR_SHAPE;
     if (T == 0) return OM_OK;
     if (!logits_out || !weights_out || !experts_out) return OM_ERR_NULL;
-    int splits = 0;
-    const int rc = gate_partials(x, gate_weight, T, H, N, workspace, workspace_bytes, stream, splits);
+    const int rc = gate_operands(x, gate_weight, T, H, N, workspace, workspace_bytes);
     if (rc != OM_OK) return rc;
     hipStream_t st = om_stream(stream);
+    // One launch or two: with the gate weight out of the caches (after a forward's expert weights) one CU waits for it longer
+    // than many do.  A whole MoE forward of 64 experts, hidden 2048, us, one launch -> two: 1 token 43.7 -> 41.8, 37 tokens
+    // 173.7 -> 171.8; 512 tokens (with the backward) 700 -> 701; 4096 tokens 520.7 -> 524.2.  In the caches, the router alone:
+    // 1 token 7.7 -> 7.8, 512 tokens 8.1 -> 12.2, 4096 tokens 10.7 -> 19.0, and at hidden 7168 15.5 -> 11.5, 16.2 -> 18.5 and
+    // 25.8 -> 26.7.  Below hidden 1024 the weight is small: 512, 32 experts, 512 tokens 4.4 -> 9.2.
+    if (gate_slices_fit(H, N) && (T > 512 || H < 1024)) {
+#define OM_GS(TL, TW) \
+    launch_gate_slices<TL, TW, true>(x, gate_weight, T, H, N, K, norm_topk_prob, logits_out, weights_out, experts_out, st)
+        if (logits_dtype == OM_F32) return weights_dtype == OM_F32 ? OM_GS(float, float) : OM_GS(float, uint16_t);
+        return weights_dtype == OM_F32 ? OM_GS(uint16_t, float) : OM_GS(uint16_t, uint16_t);
+#undef OM_GS
+    }
+    const int splits = gate_partials(x, gate_weight, T, H, N, workspace, stream);
     const unsigned nb = token_blocks(T);
     const float *part = static_cast<const float *>(workspace);
 #define OM_PR(TL, TW)                                                                                     \
@@ -744,9 +959,9 @@ extern "C" int om_router_gate_split_sigmoid_group_topk(const void *x, const void
         return OM_ERR_SHAPE;
     if (T == 0) return OM_OK;
     if (!bias || !logits_out || !experts_out || !weights_out) return OM_ERR_NULL;
-    int splits = 0;
-    const int rc = gate_partials(x, gate_weight, T, H, N, workspace, workspace_bytes, stream, splits);
+    const int rc = gate_operands(x, gate_weight, T, H, N, workspace, workspace_bytes);
     if (rc != OM_OK) return rc;
+    const int splits = gate_partials(x, gate_weight, T, H, N, workspace, stream);
     hipStream_t st = om_stream(stream);
     const unsigned nb = token_blocks(T);
     const float scale = static_cast<float>(routed_scaling_factor);

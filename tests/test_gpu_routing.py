@@ -464,3 +464,34 @@ def test_split_gate_router_equals_its_steps(cuda, T, H, N, K, bf16_logits):
     assert bool(((logits.double() - ref).abs() <= bound + 1e-30).all())
     if not bf16_logits and N <= 64 and H % 512 == 0:
         assert torch.equal(logits, fp32_logits(x, w))       # eight slices in order: the one-pass kernel's bits
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 512, 64, 8), (31, 1024, 33, 16), (33, 512, 17, 1), (65, 1536, 64, 17), (64, 2048, 32, 32),
+                                     (95, 512, 5, 4), (513, 4608, 50, 6), (512, 4608, 50, 6),
+                                     (8200, 512, 64, 8)])
+@pytest.mark.parametrize("renorm", [False, True])
+@pytest.mark.parametrize("one_pass,bf16_logits", [(True, False), (False, False), (False, True)])
+def test_one_launch_gate_router(cuda, T, H, N, K, renorm, one_pass, bf16_logits):
+    """The one-launch router of up to 64 experts: edges of its 32 tokens, experts that do not fill their
+    block of 32, the selections on rows of 16 lanes and (more than 16) on whole wavefronts, equal
+    logits (two experts with the same weights) and a token without a number.  The logits against
+    float64 products, the routing bit for bit against the router on the same logits."""
+    from optimus import _native as n
+    from optimus.models.common.moe import SoftmaxTopkRouterFunction
+    x, w = _gate_inputs(T, H, N, seed=T + H + N)
+    w[N // 2] = w[0]
+    if T > 2:
+        x[T // 2, 3] = float("nan")
+    x, w = x.to(cuda), w.to(cuda)
+    we, e, logits, _ = n.host().route_softmax(x, w, K, renorm, torch.float32, one_pass, bf16_logits)
+    w2, e2 = SoftmaxTopkRouterFunction.apply(logits, K, renorm, torch.float32)
+    assert torch.equal(e, e2) and torch.equal(we.view(torch.int32), w2.view(torch.int32))
+    ok = torch.ones(T, dtype=torch.bool, device=cuda)
+    if T > 2:
+        ok[T // 2] = False
+        assert bool(logits[T // 2].isnan().all())
+    assert torch.equal(logits[ok, N // 2], logits[ok, 0])
+    ref = x[ok].double() @ w.double().t()
+    # an fp32 sum of H exact products in any order, then (bf16) one rounding of 2^-9
+    bound = 8 * 2.0 ** -24 * (x[ok].double().abs() @ w.double().abs().t()) + (2.0 ** -8 * ref.abs() if bf16_logits else 0)
+    assert bool(((logits[ok].double() - ref).abs() <= bound + 1e-30).all())
