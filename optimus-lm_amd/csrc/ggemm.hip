@@ -107,6 +107,7 @@ struct GemmParams {
     int phases;                 // 1 or 2
     int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert (MERGED: of all three)
+    bool spread;                // wgrad: every XCD has an eighth of each expert's tiles (spread_tiles)
     WgradSet set[3];            // MERGED
 };
 
@@ -209,6 +210,34 @@ __device__ __forceinline__ bool find_tile(const int *tile_end, const int *seg, i
 // the expert's rows of both operands, and with near-uniform routing whole experts per XCD (what
 // equal tile counts give) is the better cut.  Every wavefront computes the two boundaries it needs
 // by itself from cum_token_counts (two strided passes, no LDS, no barrier).
+//
+// An expert with many tiles keeps an XCD busy for several rounds of its blocks, all of them multiplying
+// (many rows) or all of them storing (few); the XCD that holds the few-row experts is then bound by what one
+// XCD can store.  So where an eighth of an expert's tiles is a third of a round or more (spread_tiles) every XCD takes an eighth
+// of each expert, neighbouring columns of tiles along the longer extent, which share the whole panel along the shorter
+// one; and the experts come in the order of their rows, the rounds running over the blocks to and fro, so that the sums of
+// a block's tiles differ little (expert_order).
+// us, against contiguous runs of equal work per XCD (wgrad_xcd_run) with each XCD's tiles expert by expert: 32 experts of 2048/7168,
+// accumulating: 256 rows each 515 -> 509, 2048 rows 1947 -> 1788; 12510 rows, between 0 and 2663 an expert, 708 -> 568;
+// rows as 1 / rank, mean 512, 778 -> 689.  Writing only: 64 rows each 230 -> 254, 512 rows 548 -> 550, the uneven ones 567 -> 459
+// and 694 -> 570.  64 experts' three gradients of 1024/2048 in one launch (96 tiles), 4096 rows as rank^-1.2: 229 -> 211.
+// Not with 32 tiles an expert, one round of an XCD: 64 experts of 1024/2048, 256 rows each 118 -> 141, 2048 rows
+// 484 -> 589 (each XCD then reads the short panel of all experts).  Nor with half of an XCD's blocks going through the experts
+// backwards, to have some multiply while others store: 568 -> 590.
+constexpr int SPREAD_MAX_EXPERTS = 256;
+// order[i]: the expert with the i-th most rows.  The whole block, with a barrier at the end.
+__device__ __forceinline__ void expert_order(const int32_t *cum, int n_experts, int tid, int threads, int *order) {
+    for (int e = tid; e < n_experts; e += threads) {
+        const int rows = cum[e + 1] - cum[e];
+        int rank = 0;
+        for (int j = 0; j < n_experts; j++) {
+            const int other = cum[j + 1] - cum[j];
+            rank += other > rows || (other == rows && j < e) ? 1 : 0;
+        }
+        order[rank] = e;
+    }
+    __syncthreads();
+}
 constexpr int WGRAD_EPILOGUE_STEPS = 3;   // a tile's stores take about as long as 3 steps
 constexpr int WGRAD_BALANCE_MAX_EXPERTS = 4096;
 __device__ __forceinline__ int wgrad_tile_units(int rows, int bk) {
@@ -311,6 +340,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
     __shared__ int idx_cache[IDX_CACHE];
     int cached_expert = -1;            // (MERGED: and product)
+    constexpr bool SPREADS = WGRAD && BM == 256;
+    __shared__ int order[SPREADS ? SPREAD_MAX_EXPERTS : 1];
     __shared__ int tile_end[WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
     __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];
 
@@ -372,7 +403,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 row_index = a_indexed ? w.a_rows : w.b_rows;
             }
             const int tiles_n = (n_cols + BN - 1) / BN;
-            const int tm = tile / tiles_n, tn = tile % tiles_n;
+            int tm = tile / tiles_n, tn = tile % tiles_n;
+            if (SPREADS && p.spread && n_cols > m_rows) {   // columns of tiles instead of rows
+                const int tiles_m = m_rows / BM;
+                tn = tile / tiles_m;
+                tm = tile % tiles_m;
+            }
             rot_a = tn; rot_b = tm;
             row_begin = tm * BM;
             row_end = m_rows;
@@ -617,7 +653,10 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     const int xcd = blockIdx.x % NUM_XCD, slot_x = blockIdx.x / NUM_XCD;
     int per = total_tiles / NUM_XCD, rem = total_tiles - per * NUM_XCD;
     int run_lo = xcd * per;
-    if (WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
+    const bool spread = SPREADS && p.spread;
+    if (spread) {
+        expert_order(p.cum, p.n_experts, tid, NW * 64, order);
+    } else if (WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
         int lo, hi;
         wgrad_xcd_run(p.cum, p.n_experts, p.tiles_e, BK, xcd, NUM_XCD, lane, lo, hi);
         run_lo = __builtin_amdgcn_readfirstlane(lo);
@@ -625,13 +664,19 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         rem = 0;
     }
     const int n_mine = slot_x < per ? (per - slot_x + nbx - 1) / nbx : 0;
-    const int n_all = n_mine + ((xcd < rem && slot_x == per % nbx) ? 1 : 0);
+    const int n_all = spread ? (per + nbx - 1) / nbx : n_mine + ((xcd < rem && slot_x == per % nbx) ? 1 : 0);
     int it = 0;
     auto next_tile = [&]() -> bool {
         while (it < n_all) {
-            const int logical = it < n_mine ? run_lo + slot_x + it * nbx : total_tiles - rem + xcd;
+            int logical = it < n_mine ? run_lo + slot_x + it * nbx : total_tiles - rem + xcd;
+            if (spread) {
+                const int q = it * nbx + (it & 1 ? nbx - 1 - slot_x : slot_x), eighth = p.tiles_e / NUM_XCD, i = q / eighth;
+                logical = q < per ? __builtin_amdgcn_readfirstlane(order[SPREADS ? i : 0]) * p.tiles_e + xcd * eighth + (q - i * eighth) : -1;
+            }
             it++;
-            if (setup_tile(logical)) return true;
+            if (spread && logical < 0) continue;
+            // (nothing to add for an expert without rows)
+            if (setup_tile(logical) && !(ACCUM && n_steps == 0)) return true;
         }
         return false;
     };
@@ -1104,6 +1149,11 @@ bool wgrad_big_tile(int n, int k, int64_t matrices) {
     return n % 256 == 0 && k % 256 == 0 && matrices * (n / 256) * (k / 256) * 2 >= device_cu_count();
 }
 
+// Whether each XCD takes an eighth of every expert's tiles (see expert_order): 12 tiles of it at least.
+bool spread_tiles(bool big, int tiles_e, int n_experts) {
+    return big && tiles_e % NUM_XCD == 0 && tiles_e >= 12 * NUM_XCD && n_experts <= SPREAD_MAX_EXPERTS;
+}
+
 // weight gradient; gather == GATHER_B: contraction row c of `input` is row index[c] of a
 // [src_rows, K] matrix; gather == GATHER_WA: contraction row c of `output_grad` is row index[c] of a
 // [src_rows, N] matrix (the token gather folded into the loads)
@@ -1131,6 +1181,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     hipStream_t st = om_stream(stream);
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
+    p.spread = spread_tiles(big, p.tiles_e, G);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
@@ -1271,6 +1322,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
         return code;
     }
     p.tiles_e = static_cast<int>(3 * each);
+    p.spread = spread_tiles(big, p.tiles_e, G);
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);

@@ -111,6 +111,38 @@ def test_three_weight_gradients_of_a_merged_mlp(cuda, indexed, kind, G, rows, I,
         assert (torch.as_strided(fresh[i], (G, 64), (pitch, 1), I * H) == 7.0).all()
 
 
+# matrices of 96 and more 256x256 tiles, a multiple of eight of them: the XCDs share every expert's tiles, the experts come
+# by rows.  Equal rows, one expert, more experts than a round has blocks, all rows on one, wide and tall matrices.
+@pytest.mark.parametrize("kind,G,rows,N,K", [("uniform", 1, 100, 2048, 3072), ("ragged", 33, 1500, 2048, 3072), ("empties", 6, 900, 3072, 2048),
+                                             ("onehot", 5, 700, 4096, 2048), ("uniform", 4, 512, 3072, 2048), ("uniform", 3, 0, 2048, 3072)])
+@pytest.mark.parametrize("gathered", [False, True])
+def test_weight_gradients_spread_over_the_xcds(cuda, gathered, kind, G, rows, N, K):
+    """The same bound as above: one bf16 rounding of a float32 sum over the expert's rows; accumulated bit for bit as
+    torch's in-place add of it."""
+    from optimus import _native as n
+    g = torch.Generator().manual_seed(rows + G)
+    T = max(rows // 2, 8)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(cuda)
+    dout, x = rnd(max(rows, 1), N), rnd(T if gathered else max(rows, 1), K)
+    idx = torch.randint(0, T, (max(rows, 1),), generator=g, dtype=torch.int32).to(cuda)
+    cum = _counts(kind, G, rows) if rows else torch.zeros(G + 1, dtype=torch.int32)
+    d, P = cum.to(cuda), n.ptr
+    old = torch.randn(G, N, K, device=cuda).to(torch.bfloat16)
+    fresh, acc = torch.full_like(old, 7.0), old.clone()
+    for suffix, out in (("", fresh), ("_accumulate", acc)):
+        if gathered:
+            _call("om_grouped_gemm_wgrad_gathered" + suffix, P(dout), P(x), P(idx), T, P(out), P(d), rows, G, N, K, 0)
+        else:
+            _call("om_grouped_gemm_wgrad" + suffix, P(dout), P(x), P(out), P(d), rows, G, N, K, 0)
+    xr = x[idx.long()] if gathered else x
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        want = dout[s].float().t() @ xr[s].float()
+        err = (fresh[e].float() - want).abs()
+        assert (err <= want.abs() * 2 ** -8 + 2e-5 * max(s.stop - s.start, 1) ** 0.5).all(), e
+    assert (bits(acc) == bits(old.add_(fresh))).all()
+
+
 def test_accumulate_f32(cuda):
     from optimus import _native as n
     g = torch.Generator().manual_seed(5)
