@@ -84,6 +84,9 @@ struct WgradSet {
     int m, n;
 };
 
+template <int BM> constexpr int WAVES_N = BM / 64;        // 256x256: 2 x 4 wavefronts, 128x128: 2 x 2
+template <int BM> constexpr int THREADS = 2 * WAVES_N<BM> * 64;
+
 struct GemmParams {
     // operands; for the two-phase products (gate+up) index 1 is the second pair
     const uint16_t *A[2];
@@ -107,7 +110,7 @@ struct GemmParams {
     int phases;                 // 1 or 2
     int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert (MERGED: of all three)
-    bool spread;                // wgrad: every XCD has an eighth of each expert's tiles (spread_tiles)
+    int share;                  // XCDs that share an expert's tiles; 0: contiguous runs of tiles per XCD
     WgradSet set[3];            // MERGED
 };
 
@@ -202,6 +205,84 @@ __device__ __forceinline__ bool find_tile(const int *tile_end, const int *seg, i
     return false;
 }
 
+// Launches with large experts (p.share != 0) share each expert among several XCDs.  An expert of many tiles, XCD by XCD, would
+// keep one XCD busy for several rounds of its blocks, all of them multiplying (many rows) or all of them moving the
+// weights (few), and those with the few-row experts are then bound by what one XCD can load or store.
+// So the experts are taken in the order of their rows; `share` XCDs have each a part of every expert of a group; with
+// two or more groups (share < 8) the experts go to them to and fro; and a part is neighbouring columns of tiles along the longer
+// extent (row products: the columns of the weight matrix, which its part of the weights then crosses once).
+// The rounds run over the XCD's blocks to and fro as well, so that the sums of a block's tiles differ little.
+// us, contiguous runs of equal work per XCD -> shared, 32 experts of 2048/7168.  12510 rows, between 0 and 2663 an expert (in a
+// training pass): gate+up 865 -> 792, down 431 -> 415, SwiGLU backward 541 -> 437, gate/up input gradient 908 -> 789,
+// accumulating weight gradients 715 -> 590.  Alone, rows as 1 / rank with mean 64 / 512 / 2048, even rows with mean 512 / 2048:
+// gate+up 490 -> 422, 1001 -> 1027, 3619 -> 3565, 796 -> 835, 3312 -> 2992; gate/up input gradient 548 -> 432, 1071 -> 1020,
+// 3771 -> 3588, 916 -> 821, 3674 -> 3100; SwiGLU backward 287 -> 277, 566 -> 562, 1817 -> 1943, 427 -> 438, 1630 -> 1647; weight
+// gradients, writing 224 -> 245, 688 -> 570, 1936 -> 1736, 529 -> 544, 1770 -> 1668, accumulating 444 -> 399, 757 -> 689, 2069 -> 1821,
+// 676 -> 664, 1920 -> 1787.  Smaller experts lose what they share in the caches: 64 of 1024/2048, even, 512 rows,
+// four XCDs, gate+up 257 -> 269, all eight 307; the weight gradients, one round of an XCD each, 170 -> 179 and 205.  Nor is
+// it better to mix experts of many and of few rows in time: alternating them, weight gradients 590 -> 670.
+constexpr int SHARE_MAX_EXPERTS = 256;
+// order[i]: the expert with the i-th most rows.  The whole block, with a barrier at the end.
+__device__ __forceinline__ void expert_order(const int32_t *cum, int n_experts, int tid, int lane, int *order) {
+    static_assert(SHARE_MAX_EXPERTS <= THREADS<128>, "a thread per expert");
+    if (tid - lane < n_experts) {
+        const int e = min(tid, n_experts - 1), mine = cum[e + 1] - cum[e];
+        int rank = 0;
+        for (int j0 = 0; j0 < n_experts; j0 += 64) {
+            const int j = min(j0 + lane, n_experts - 1), rows = j0 + lane < n_experts ? cum[j + 1] - cum[j] : -1;
+#pragma unroll 16
+            for (int l = 0; l < 64; l++) {
+                const int other = __builtin_amdgcn_readlane(rows, l);
+                rank += other > mine || (other == mine && j0 + l < e) ? 1 : 0;
+            }
+        }
+        if (tid < n_experts) order[rank] = e;
+    }
+    __syncthreads();
+}
+// First tile of the part of an XCD in the i-th expert of `order`; where `share` does not divide them the XCDs take turns
+// with the odd ones.
+__device__ __forceinline__ int part_begin(int tiles, int i, int member, int share) {
+    return (member * tiles + (i * 5 & (share - 1))) / share;
+}
+// An expert of `order` as an XCD sees it: its rows, and what turns the XCD's tile number into the expert's.
+struct Part { int expert, row_begin, row_end, shift; };
+// part[i], and tile_end[i] = number of tiles, of the first i + 1 experts in `order`, that are this XCD's.  tiles_of(rows): of an expert.  One wavefront.
+template <typename TILES>
+__device__ __forceinline__ void build_part_table(const int32_t *cum, const int *order, int n_experts, int share, int xcd, int lane,
+                                                 TILES tiles_of, int *tile_end, Part *part) {
+    const int groups = NUM_XCD / share, member = xcd % share;
+    int base_tiles = 0;
+    for (int i0 = 0; i0 < n_experts; i0 += 64) {
+        const int i = i0 + lane, there = i % groups, group = (i / groups) & 1 ? groups - 1 - there : there;
+        const int e = order[min(i, n_experts - 1)], begin = cum[e], end = cum[e + 1], tiles = tiles_of(end - begin);
+        const int first = part_begin(tiles, i, member, share);
+        const int mine = i < n_experts && group == xcd / share ? part_begin(tiles, i, member + 1, share) - first : 0;
+        int incl = mine;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
+        }
+        if (i < n_experts) {
+            tile_end[i] = base_tiles + incl;
+            part[i] = {e, begin, end, first - (base_tiles + incl - mine)};
+        }
+        base_tiles += __shfl(incl, 63, 64);
+    }
+}
+// The part that tile `at` of the XCD (less than the last tile_end) belongs to.
+__device__ __forceinline__ Part find_part(const int *tile_end, const Part *part, int n_experts, int lane, int at) {
+    int i = 0;
+    asm volatile("" : "+v"(lane));   // addresses recomputed per tile, not kept across the main loop
+    for (int i0 = 0; i0 < n_experts; i0 += 64) {
+        const unsigned long long vote = __ballot(i0 + lane < n_experts && at < tile_end[min(i0 + lane, n_experts - 1)]);
+        if (vote) { i = i0 + __ffsll(static_cast<long long>(vote)) - 1; break; }
+    }
+    const Part p = part[__builtin_amdgcn_readfirstlane(i)];
+    return {__builtin_amdgcn_readfirstlane(p.expert), __builtin_amdgcn_readfirstlane(p.row_begin),
+            __builtin_amdgcn_readfirstlane(p.row_end), __builtin_amdgcn_readfirstlane(p.shift)};
+}
+
 // Weight gradient: the tiles of expert e cost about (contraction steps of e + a few steps' worth of
 // epilogue) each, so with skewed routing equal tile counts per XCD are far from equal work.  The
 // tiles are numbered expert-major; boundary j of 0..8 is the tile at which j/8 of the launch's work
@@ -210,34 +291,6 @@ __device__ __forceinline__ bool find_tile(const int *tile_end, const int *seg, i
 // the expert's rows of both operands, and with near-uniform routing whole experts per XCD (what
 // equal tile counts give) is the better cut.  Every wavefront computes the two boundaries it needs
 // by itself from cum_token_counts (two strided passes, no LDS, no barrier).
-//
-// An expert with many tiles keeps an XCD busy for several rounds of its blocks, all of them multiplying
-// (many rows) or all of them storing (few); the XCD that holds the few-row experts is then bound by what one
-// XCD can store.  So where an eighth of an expert's tiles is a third of a round or more (spread_tiles) every XCD takes an eighth
-// of each expert, neighbouring columns of tiles along the longer extent, which share the whole panel along the shorter
-// one; and the experts come in the order of their rows, the rounds running over the blocks to and fro, so that the sums of
-// a block's tiles differ little (expert_order).
-// us, against contiguous runs of equal work per XCD (wgrad_xcd_run) with each XCD's tiles expert by expert: 32 experts of 2048/7168,
-// accumulating: 256 rows each 515 -> 509, 2048 rows 1947 -> 1788; 12510 rows, between 0 and 2663 an expert, 708 -> 568;
-// rows as 1 / rank, mean 512, 778 -> 689.  Writing only: 64 rows each 230 -> 254, 512 rows 548 -> 550, the uneven ones 567 -> 459
-// and 694 -> 570.  64 experts' three gradients of 1024/2048 in one launch (96 tiles), 4096 rows as rank^-1.2: 229 -> 211.
-// Not with 32 tiles an expert, one round of an XCD: 64 experts of 1024/2048, 256 rows each 118 -> 141, 2048 rows
-// 484 -> 589 (each XCD then reads the short panel of all experts).  Nor with half of an XCD's blocks going through the experts
-// backwards, to have some multiply while others store: 568 -> 590.
-constexpr int SPREAD_MAX_EXPERTS = 256;
-// order[i]: the expert with the i-th most rows.  The whole block, with a barrier at the end.
-__device__ __forceinline__ void expert_order(const int32_t *cum, int n_experts, int tid, int threads, int *order) {
-    for (int e = tid; e < n_experts; e += threads) {
-        const int rows = cum[e + 1] - cum[e];
-        int rank = 0;
-        for (int j = 0; j < n_experts; j++) {
-            const int other = cum[j + 1] - cum[j];
-            rank += other > rows || (other == rows && j < e) ? 1 : 0;
-        }
-        order[rank] = e;
-    }
-    __syncthreads();
-}
 constexpr int WGRAD_EPILOGUE_STEPS = 3;   // a tile's stores take about as long as 3 steps
 constexpr int WGRAD_BALANCE_MAX_EXPERTS = 4096;
 __device__ __forceinline__ int wgrad_tile_units(int rows, int bk) {
@@ -340,15 +393,17 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
     __shared__ int idx_cache[IDX_CACHE];
     int cached_expert = -1;            // (MERGED: and product)
-    constexpr bool SPREADS = WGRAD && BM == 256;
-    __shared__ int order[SPREADS ? SPREAD_MAX_EXPERTS : 1];
-    __shared__ int tile_end[WGRAD ? 1 : MAX_EXPERTS];   // see build_tile_table
+    constexpr bool SHARES = !WGRAD || !EDGE;            // whether the launch may be one with p.share != 0
+    __shared__ int order[SHARES ? SHARE_MAX_EXPERTS : 1];
+    __shared__ __attribute__((aligned(16))) Part part[SHARES ? SHARE_MAX_EXPERTS : 1];
+    __shared__ int tile_end[!WGRAD ? MAX_EXPERTS : SHARES ? SHARE_MAX_EXPERTS : 1];   // see build_tile_table, build_part_table
     __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
+    const int xcd = blockIdx.x % NUM_XCD;
     // ---- per-tile state (set by setup_tile) ---------------------------------------------------
     int expert = 0, row_begin = 0, row_end = 0, n0 = 0, c_begin = 0, c_len = 0;
     int steps_per_phase = 0, c_wrap = 0, n_steps = 0, rot = 0;
@@ -387,11 +442,27 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         }
     };
 
+    auto tiles_of = [&](int rows) {
+        constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
+        return WGRAD ? p.tiles_e : (rows + BM - 1) / BM * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+    };
+    // p.share: `logical` counts this XCD's tiles, otherwise the launch's
     auto setup_tile = [&](int logical) -> bool {
         int rot_a, rot_b;
         if (WGRAD) {
-            expert = logical / p.tiles_e;
-            int tile = logical - expert * p.tiles_e;
+            int tile;
+            if (SHARES && p.share) {
+                const Part q = find_part(tile_end, part, p.n_experts, lane, logical);
+                expert = q.expert;
+                tile = logical + q.shift;
+                c_begin = q.row_begin;
+                c_len = q.row_end - q.row_begin;
+            } else {
+                expert = logical / p.tiles_e;
+                tile = logical - expert * p.tiles_e;
+                c_begin = p.cum[expert];
+                c_len = p.cum[expert + 1] - c_begin;
+            }
             if (GATHER == MERGED) {
                 const int each = p.tiles_e / 3;     // (the three have the same extents, one of them transposed)
                 product = __builtin_amdgcn_readfirstlane(tile / each);
@@ -404,7 +475,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             }
             const int tiles_n = (n_cols + BN - 1) / BN;
             int tm = tile / tiles_n, tn = tile % tiles_n;
-            if (SPREADS && p.spread && n_cols > m_rows) {   // columns of tiles instead of rows
+            if (SHARES && p.share && n_cols > m_rows) {   // columns of tiles instead of rows
                 const int tiles_m = m_rows / BM;
                 tn = tile / tiles_m;
                 tm = tile % tiles_m;
@@ -413,15 +484,20 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             row_begin = tm * BM;
             row_end = m_rows;
             n0 = tn * BN;
-            c_begin = p.cum[expert];
-            c_len = p.cum[expert + 1] - c_begin;
         } else {
             constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
             const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
-            const int tile_m = logical / tiles_n;
-            const int tile_n = logical % tiles_n;
+            int tile_m = logical / tiles_n, tile_n = logical % tiles_n;
+            if (p.share) {
+                const Part q = find_part(tile_end, part, p.n_experts, lane, logical);
+                const int tile = logical + q.shift, tiles_m = (q.row_end - q.row_begin + BM - 1) / BM;
+                tile_n = tile / tiles_m;
+                tile_m = tile - tile_n * tiles_m;
+                expert = q.expert;
+                row_begin = q.row_begin + tile_m * BM;
+                row_end = q.row_end;
+            } else if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
             rot_a = tile_n; rot_b = tile_m & 7;
-            if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
             c_len = p.kc;
@@ -642,39 +718,40 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     constexpr int RA = AKIND == CONTIG ? 4 : 8, RB = BKIND == CONTIG ? 8 : 16;   // LDS reads of a unit of A, of a step of B
 
-    int total_tiles = p.total_tiles;
-    if (!WGRAD) {
-        if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
+    const int nbx = gridDim.x / NUM_XCD, slot_x = blockIdx.x / NUM_XCD;
+    int total_tiles = p.total_tiles, per = 0, rem = 0, run_lo = 0;
+    if (SHARES && p.share) {
+        expert_order(p.cum, p.n_experts, tid, lane, order);
+        if (wave == 0) build_part_table(p.cum, order, p.n_experts, p.share, xcd, lane, tiles_of, tile_end, part);
         __syncthreads();
-        constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
-        total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+        per = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]);
+    } else {
+        if (!WGRAD) {
+            if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
+            __syncthreads();
+            constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
+            total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+        }
+        per = total_tiles / NUM_XCD;
+        rem = total_tiles - per * NUM_XCD;
+        run_lo = xcd * per;
+        if (WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
+            int lo, hi;
+            wgrad_xcd_run(p.cum, p.n_experts, p.tiles_e, BK, xcd, NUM_XCD, lane, lo, hi);
+            run_lo = __builtin_amdgcn_readfirstlane(lo);
+            per = __builtin_amdgcn_readfirstlane(hi) - run_lo;
+            rem = 0;
+        }
     }
-    const int nbx = gridDim.x / NUM_XCD;
-    const int xcd = blockIdx.x % NUM_XCD, slot_x = blockIdx.x / NUM_XCD;
-    int per = total_tiles / NUM_XCD, rem = total_tiles - per * NUM_XCD;
-    int run_lo = xcd * per;
-    const bool spread = SPREADS && p.spread;
-    if (spread) {
-        expert_order(p.cum, p.n_experts, tid, NW * 64, order);
-    } else if (WGRAD && p.n_experts <= WGRAD_BALANCE_MAX_EXPERTS) {
-        int lo, hi;
-        wgrad_xcd_run(p.cum, p.n_experts, p.tiles_e, BK, xcd, NUM_XCD, lane, lo, hi);
-        run_lo = __builtin_amdgcn_readfirstlane(lo);
-        per = __builtin_amdgcn_readfirstlane(hi) - run_lo;
-        rem = 0;
-    }
-    const int n_mine = slot_x < per ? (per - slot_x + nbx - 1) / nbx : 0;
-    const int n_all = spread ? (per + nbx - 1) / nbx : n_mine + ((xcd < rem && slot_x == per % nbx) ? 1 : 0);
+    // the block's place in round `it` of its XCD
+    auto place = [&](int it) { return SHARES && p.share && (it & 1) ? nbx - 1 - slot_x : slot_x; };
+    const int n_mine = per / nbx + (place(per / nbx) < per % nbx ? 1 : 0);
+    const int n_all = n_mine + ((xcd < rem && slot_x == per % nbx) ? 1 : 0);
     int it = 0;
     auto next_tile = [&]() -> bool {
         while (it < n_all) {
-            int logical = it < n_mine ? run_lo + slot_x + it * nbx : total_tiles - rem + xcd;
-            if (spread) {
-                const int q = it * nbx + (it & 1 ? nbx - 1 - slot_x : slot_x), eighth = p.tiles_e / NUM_XCD, i = q / eighth;
-                logical = q < per ? __builtin_amdgcn_readfirstlane(order[SPREADS ? i : 0]) * p.tiles_e + xcd * eighth + (q - i * eighth) : -1;
-            }
+            const int logical = it < n_mine ? run_lo + place(it) + it * nbx : total_tiles - rem + xcd;
             it++;
-            if (spread && logical < 0) continue;
             // (nothing to add for an expert without rows)
             if (setup_tile(logical) && !(ACCUM && n_steps == 0)) return true;
         }
@@ -1042,13 +1119,20 @@ template <int BM> unsigned persistent_blocks(int64_t tiles) {
     return static_cast<unsigned>(per_xcd * NUM_XCD);
 }
 
-template <int BM> constexpr int WAVES_N = BM / 64;        // 256x256: 2 x 4 wavefronts, 128x128: 2 x 2
-template <int BM> constexpr int THREADS = 2 * WAVES_N<BM> * 64;
+
+// XCDs that share an expert's row products: from 8 M weights a matrix on, four, or all eight with few experts, which two
+// groups of XCDs could not divide evenly.  One expert alone needs no sharing: its tiles are alike.
+inline int rows_share(const GemmParams &p, int64_t expected) {
+    if (p.n_experts < 2 || p.n_experts > SHARE_MAX_EXPERTS || static_cast<int64_t>(p.n_cols) * p.kc < (8 << 20)) return 0;
+    if (expected < 32 * static_cast<int64_t>(p.n_experts)) return 0;
+    return p.n_experts >= 16 ? 4 : NUM_XCD;
+}
 
 template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
-int launch_rows(GemmParams &p, int64_t rows, hipStream_t st) {  // fwd / dgrad family
+int launch_rows(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {  // fwd / dgrad family
     constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BM / 2 : BM;
     if (p.n_experts > MAX_EXPERTS) return OM_ERR_SHAPE;   // the tile table lives in LDS
+    p.share = rows_share(p, expected);
     const int64_t m_tiles_max = (rows + BM - 1) / BM + p.n_experts;
     const int64_t tiles = m_tiles_max * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
@@ -1087,9 +1171,9 @@ template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t
 template <int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
 int launch_rows_auto(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
     if (uses_big_tile<EPI>(p.n_cols, p.kc, p.n_experts, expected))
-        return launch_rows<256, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
+        return launch_rows<256, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, expected, st);
     if (p.n_cols % 8 != 0 || p.kc % 8 != 0) return OM_ERR_SHAPE;
-    return launch_rows<128, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, st);
+    return launch_rows<128, AKIND, BKIND, EPI, GATHER, ROWW>(p, rows, expected, st);
 }
 
 }  // namespace
@@ -1149,9 +1233,9 @@ bool wgrad_big_tile(int n, int k, int64_t matrices) {
     return n % 256 == 0 && k % 256 == 0 && matrices * (n / 256) * (k / 256) * 2 >= device_cu_count();
 }
 
-// Whether each XCD takes an eighth of every expert's tiles (see expert_order): 12 tiles of it at least.
-bool spread_tiles(bool big, int tiles_e, int n_experts) {
-    return big && tiles_e % NUM_XCD == 0 && tiles_e >= 12 * NUM_XCD && n_experts <= SPREAD_MAX_EXPERTS;
+// XCDs that share an expert's weight gradient: all, where an eighth of its tiles is about a third of a round or more.
+int wgrad_share(bool big, int tiles_e, int n_experts) {
+    return big && tiles_e >= 12 * NUM_XCD && n_experts <= SHARE_MAX_EXPERTS ? NUM_XCD : 0;
 }
 
 // weight gradient; gather == GATHER_B: contraction row c of `input` is row index[c] of a
@@ -1181,7 +1265,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     hipStream_t st = om_stream(stream);
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
-    p.spread = spread_tiles(big, p.tiles_e, G);
+    p.share = wgrad_share(big, p.tiles_e, G);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
@@ -1322,7 +1406,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
         return code;
     }
     p.tiles_e = static_cast<int>(3 * each);
-    p.spread = spread_tiles(big, p.tiles_e, G);
+    p.share = wgrad_share(big, p.tiles_e, G);
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);

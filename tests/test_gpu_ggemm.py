@@ -638,6 +638,34 @@ def test_row_units_and_step_counts_of_the_256_kernels(cuda, K):
             assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 2e-5 * max(k, 1) ** 0.5).all(), (name, e)
 
 
+# weights of 8 M elements and more: several XCDs share an expert, four with 16 experts or more, all eight with fewer.  Both
+# tile sizes, columns of tiles that neither divides, more experts than a wavefront has lanes, experts without rows, one with all.
+@pytest.mark.parametrize("kind,G,rows,N,K", [("uniform", 16, 4000, 4096, 2048), ("ragged", 33, 6500, 4096, 2048), ("ragged", 17, 700, 4104, 2056),
+                                             ("empties", 20, 5000, 2048, 4096), ("onehot", 3, 900, 4352, 2048), ("ragged", 5, 1700, 2056, 4104),
+                                             ("ragged", 70, 9000, 2048, 4096), ("uniform", 2, 64, 4096, 2048)])
+def test_row_products_of_shared_experts(cuda, kind, G, rows, N, K):
+    """Every tile once: forward, input gradient and the gate/up product against float32 products of each expert's
+    rows; one bf16 rounding of a float32 sum (2^-8 of the value, and the order of the sum)."""
+    from optimus import _native as n
+    cum = _counts(kind, G, rows)
+    bf = lambda *s, f=1.0: (torch.randn(*s, device=cuda) * f).to(torch.bfloat16)
+    torch.manual_seed(G)
+    x, dy, w, w2 = bf(rows, K), bf(rows, N), bf(G, N, K, f=0.02), bf(G, N, K, f=0.02)
+    y, g, u, h = (torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(4))
+    dx, d, P = torch.full((rows, K), 7.0, dtype=torch.bfloat16, device=cuda), cum.to(cuda), n.ptr
+    n.check(n.lib().om_grouped_gemm_fwd(P(x), P(w), P(y), P(d), rows, G, N, K, 0, n.stream()), "fwd")
+    n.check(n.lib().om_grouped_gemm_dgrad(P(dy), P(w), P(dx), P(d), rows, G, N, K, 0, n.stream()), "dgrad")
+    n.check(n.lib().om_merged_mlp_gate_up_fwd(P(x), P(w), P(w2), P(g), P(u), P(h), P(d), rows, G, N, K, 0, n.stream()), "gate/up")
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        first = x[s].float() @ w[e].float().t()
+        for name, got, want, k in (("fwd", y[s], first, K), ("dgrad", dx[s], dy[s].float() @ w[e].float(), N), ("gate", g[s], first, K),
+                                   ("up", u[s], x[s].float() @ w2[e].float().t(), K)):
+            assert ((got.float() - want).abs() <= want.abs() * 2 ** -8 + 1e-6 * k ** 0.5).all(), (name, e)
+    silu = torch.nn.functional.silu(g.float()) * u.float()    # h is formed before g and u are rounded: three roundings
+    assert ((h.float() - silu).abs() <= silu.abs() * 2 ** -6 + (g.float().abs() + 1) * (u.float().abs() + 1) * 2 ** -7).all()
+
+
 @pytest.mark.parametrize("expected", [0, 9, 100, 1087, 3000, 9000])
 @pytest.mark.parametrize("N,K", [(1024, 512), (200, 328)])
 def test_products_over_a_bound_of_the_rows(cuda, expected, N, K):
