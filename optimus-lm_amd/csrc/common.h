@@ -82,6 +82,16 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
+// Direct load of 16 bytes from each lane's address to LDS at lds + 16 * lane.  Outside the compiler's view: the code waits
+// for it itself (vmcnt counts it).
+__device__ __forceinline__ void dma16_lane(const char *lane_address, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(lane_address) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(char *shared) {
+    typedef __attribute__((address_space(3))) char *lds_bytes;
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes)shared));
+}
+
 // 1 / (1 + e^-x) with the hardware exponential and reciprocal (about 1 ulp each, far inside one
 // bf16 rounding of the results it feeds).  An IEEE division here costs ten instructions per
 // element, and the SwiGLU epilogues are bound by vector-ALU issue.

@@ -17,6 +17,8 @@
 // x is read once (2 B per element), dlogits comes from L2 for all but the first column slice.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(256) void gate_wgrad_reduce_kernel(const float *__r
 inline int gate_wgrad_splits(int64_t T, int H) {
     const int64_t stages = (T + TC - 1) / TC;
     const int slices = (H + HT - 1) / HT;
-    int64_t want = (2 * 256 + slices - 1) / slices;   // ~2 blocks per CU
+    int64_t want = 2 * 256 / slices;   // two blocks per CU, all at once
     if (want > stages / 2) want = stages / 2;
     if (want < 1) want = 1;
     if (want > 256) want = 256;
@@ -336,6 +338,129 @@ __global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restr
     }
 }
 
+// The same for more than 64 experts, a multiple of 16 of them: with many experts a block's dlogits and weights are more
+// than its results.  A block of eight wavefronts keeps the dlogits of its 256 tokens in registers (bf16, MFMA layout) and goes
+// through a range of 64-column slices of the weight, which come by direct loads two slices ahead through a ring of three;
+// `base` comes one slice ahead.  What is left to bound it is `base` and dx.
+// us, `base` and weights out of the caches, 256 experts, before (128 tokens x 128 columns a block, dlogits in fp32 once per 128
+// columns) -> now: hidden 7168, 64 tokens 18.9 -> 11.3, 512 tokens 19.7 -> 16.4, 8192 tokens 113.9 -> 71.0 (4.0 TB/s of base,
+// dx and dlogits); hidden 1624, 8176 tokens 45.3 -> 36.6; 128 experts, hidden 4096, 4096 tokens 29.3 -> 24.3.
+constexpr int DW_HT = 64, DW_TOK = 256, DW_PITCH = DW_HT * 2 + 8;
+
+// NK * 16 >= N experts; grid (column ranges of `tiles` slices, T / 256)
+template <int NK, bool BASE>
+__global__ __launch_bounds__(512) void gate_dgrad_wide_kernel(const float *__restrict__ dlogits, const uint16_t *__restrict__ weight,
+                                                              const uint16_t *base, uint16_t *out, int64_t T, int H, int N, int tiles) {
+    constexpr int SLOTS = 3, SLOT = NK * 16 * DW_HT * 2, LOADS = SLOT / 1024 / 8, ITS = 32 * (DW_HT / 8) / 64;
+    __shared__ __attribute__((aligned(1024))) char lds[SLOTS * SLOT + 8 * 32 * DW_PITCH];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int64_t t0 = static_cast<int64_t>(blockIdx.y) * DW_TOK + wave * 32;
+    const int first = blockIdx.x * tiles, steps = min(tiles, (H + DW_HT - 1) / DW_HT - first);
+    char *strip = lds + SLOTS * SLOT + wave * (32 * DW_PITCH);
+    // chunk c (16 bytes) of weight row n at c ^ 4 * (n / 2 % 2): the four rows of a transposing read in different banks
+    const uint32_t lds0 = lds_address(lds);
+    const uint16_t *src[LOADS];
+    int col[LOADS];
+#pragma unroll
+    for (int l = 0; l < LOADS; l++) {
+        const int n = (wave * LOADS + l) * 8 + (lane >> 3);
+        col[l] = first * DW_HT + ((lane & 7) ^ (((n >> 1) & 1) << 2)) * 8;
+        src[l] = weight + static_cast<int64_t>(min(n, N - 1)) * H;     // (rows past the end are not multiplied)
+    }
+    auto issue = [&](int s, int slot) {          // columns past the end: the last chunk again, results unused
+#pragma unroll
+        for (int l = 0; l < LOADS; l++)
+            dma16_lane(reinterpret_cast<const char *>(src[l] + min(col[l] + s * DW_HT, H - 8)), lds0 + slot * SLOT + (wave * LOADS + l) * 1024);
+    };
+    issue(0, 0);
+    if (steps > 1) issue(1, 1);
+    u32x4 other[2][ITS];
+    auto fetch_base = [&](int s, int set) {
+#pragma unroll
+        for (int it = 0; it < ITS; it++) {
+            const int q = it * 64 + lane;
+            other[set][it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(   // read once
+                base + min(t0 + q / (DW_HT / 8), T - 1) * H + min((first + s) * DW_HT + (q % (DW_HT / 8)) * 8, H - 8)));
+        }
+    };
+    if (BASE) fetch_base(0, 0);
+    bf16x8 fd[NK];                               // tokens past the end: the last one's, results unused
+    const float *drow = dlogits + min(t0 + (lane & 31), T - 1) * N + 8 * (lane >> 5);
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+        const f32x4 lo = *reinterpret_cast<const f32x4 *>(drow + min(k * 16, N - 16));
+        const f32x4 hi = *reinterpret_cast<const f32x4 *>(drow + min(k * 16, N - 16) + 4);
+        fd[k] = __builtin_bit_cast(bf16x8, u32x4{pack2(lo[0], lo[1]), pack2(lo[2], lo[3]), pack2(hi[0], hi[1]), pack2(hi[2], hi[3])});
+    }
+    const int r16 = (lane & 15) >> 2, cr = 8 * (lane >> 5) + r16, m = ((lane >> 4) & 1) * 16 + 4 * (lane & 3);
+    int frag[2];
+#pragma unroll
+    for (int b = 0; b < 2; b++) frag[b] = cr * 128 + ((((b * 32 + m) >> 3) ^ (((cr >> 1) & 1) << 2)) << 4) + (m & 7) * 2;
+    int slot = 0, free_slot = 2;
+    auto step = [&](int s, int set) {
+        // The wavefront's weights of step s have landed: younger are the next step's, and `base`'s loads of this one (stores
+        // may be skipped and do not count).  Behind the barrier everyone's have, and everyone has read step s - 1.
+        if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS + (BASE ? ITS : 0)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (BASE && s + 1 < steps) fetch_base(s + 1, set ^ 1);
+        f32x16 acc[2];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[b][r] = 0.0f;
+        const char *tile = lds + slot * SLOT;
+#pragma unroll
+        for (int k = 0; k < NK; k++) {
+            if (k * 16 >= N) continue;           // (uniform)
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                const char *p = tile + frag[b] + k * 2048;
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p + 4 * 128));
+                const bf16x8 fw = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                // lane l then holds token l % 32 and columns 32 b + 8*(r/4) + 4*(l/32) + r%4
+                acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw, fd[k], acc[b], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int rq = 0; rq < 4; rq++) {
+                const u32x2 v = {pack2(acc[b][rq * 4], acc[b][rq * 4 + 1]), pack2(acc[b][rq * 4 + 2], acc[b][rq * 4 + 3])};
+                *reinterpret_cast<u32x2 *>(strip + (lane & 31) * DW_PITCH + (b * 32 + rq * 8 + (lane >> 5) * 4) * 2) = v;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int it = 0; it < ITS; it++) {
+            const int q = it * 64 + lane, row = q / (DW_HT / 8), ch = q % (DW_HT / 8);
+            const int64_t tt = t0 + row;
+            const int h = (first + s) * DW_HT + ch * 8;
+            const char *sp = strip + row * DW_PITCH + ch * 16;
+            const u32x2 lo = *reinterpret_cast<const u32x2 *>(sp), hi = *reinterpret_cast<const u32x2 *>(sp + 8);
+            u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
+            if (BASE) {
+                float a[8], g[8];
+                Elem<uint16_t>::unpack(other[set][it], a);
+                Elem<uint16_t>::unpack(v, g);
+#pragma unroll
+                for (int i = 0; i < 8; i++) a[i] = a[i] + g[i];
+                v = Elem<uint16_t>::pack(a);
+            }
+            if (tt < T && h < H) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out + tt * H + h));
+        }
+        if (s + 2 < steps) issue(s + 2, free_slot);
+        free_slot = slot;
+        slot = slot == SLOTS - 1 ? 0 : slot + 1;
+    };
+    for (int s = 0; s < steps; s += 2) {
+        step(s, 0);
+        if (s + 1 < steps) step(s + 1, 1);
+    }
+}
+
 }  // namespace
 
 extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weight, const void *base,
@@ -345,6 +470,21 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
     if (!dlogits || !gate_weight || !dx) return OM_ERR_NULL;
     if (!om_aligned16(dlogits) || !om_aligned16(gate_weight) || !om_aligned16(dx) || !om_aligned16(base))
         return OM_ERR_ALIGN;
+    hipStream_t st = om_stream(stream);
+    const float *dl = dlogits;
+    const uint16_t *w = static_cast<const uint16_t *>(gate_weight), *bp = static_cast<const uint16_t *>(base);
+    uint16_t *dp = static_cast<uint16_t *>(dx);
+    const int64_t wide_blocks = (T + DW_TOK - 1) / DW_TOK;
+    if (N > 64 && N % 16 == 0 && wide_blocks <= 65535) {
+        const int slices = (H + DW_HT - 1) / DW_HT, ranges = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(slices, 256 / wide_blocks)));
+        const int tiles = (slices + ranges - 1) / ranges;
+        const dim3 grid((slices + tiles - 1) / tiles, static_cast<unsigned>(wide_blocks));
+        if (N <= 128 && base) gate_dgrad_wide_kernel<8, true><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
+        else if (N <= 128) gate_dgrad_wide_kernel<8, false><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
+        else if (base) gate_dgrad_wide_kernel<16, true><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
+        else gate_dgrad_wide_kernel<16, false><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
+        return om_launch_status();
+    }
     const int64_t t_blocks = (T + DG_TOK - 1) / DG_TOK;
     if (t_blocks > 65535) {
         // the token blocks ride on the grid's second dimension: split long inputs into several launches
@@ -361,9 +501,7 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
     }
     const dim3 grid((H + DG_HT - 1) / DG_HT, static_cast<unsigned>(t_blocks));
 #define OM_DGRAD(BATCHES, ALIGNED)                                                                          \
-    gate_dgrad_kernel<BATCHES, ALIGNED><<<grid, dim3(256), gate_dgrad_lds(N), om_stream(stream)>>>(          \
-        dlogits, static_cast<const uint16_t *>(gate_weight), static_cast<const uint16_t *>(base),            \
-        static_cast<uint16_t *>(dx), T, H, N)
+    gate_dgrad_kernel<BATCHES, ALIGNED><<<grid, dim3(256), gate_dgrad_lds(N), st>>>(dl, w, bp, dp, T, H, N)
     if (N % 4 != 0) {
         if (N <= 64) OM_DGRAD(1, false);
         else OM_DGRAD(4, false);

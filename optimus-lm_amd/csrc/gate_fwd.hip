@@ -12,6 +12,8 @@
 // the blocks still fill the chip through the split of H.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef const __attribute__((address_space(1))) void *glb_ptr;
@@ -36,10 +38,9 @@ __global__ __launch_bounds__(256) void gate_logits_split_kernel(const uint16_t *
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t t0 = static_cast<int64_t>(blockIdx.x) * GT + wave * 32;
     const int h_begin = blockIdx.y * h_per_split;
-    const int steps = h_per_split / GK;
-    // H is any multiple of 8: the last step of the last slice may hold fewer than 64 columns.  Its token
+    // H is any multiple of 8: the last slice may be shorter and its last step may hold fewer than 64 columns.  Its token
     // fragments past the end are zeros, its weight loads past the end re-read the last 8 columns.
-    const int h_len = min(H - h_begin, h_per_split);
+    const int h_len = min(H - h_begin, h_per_split), steps = (h_len + GK - 1) / GK;
     // token fragment: lane l holds token t0 + l % 32, 8 consecutive h starting at 8 * (l / 32)
     int64_t ta = t0 + (lane & 31);
     if (ta >= T) ta = T - 1;                    // rows past the end: valid memory, result unused
@@ -128,6 +129,98 @@ __global__ __launch_bounds__(256) void gate_logits_split_kernel(const uint16_t *
     }
 }
 
+// The same for more than 64 experts, where a step's weights (32 KB for 256) are most of what a CU takes in: 128 tokens and all
+// experts per block of eight wavefronts (64 x 64 of the logits each, NB = 4: 32 x 64), tokens and weights both by direct loads of
+// whole 128-byte rows, two steps ahead, through a ring of three.  Rows, chunks and the last step as above, but that the
+// tokens' chunks past the end are zeroed in LDS.
+// us with the launch that adds the slices, weights out of the caches, 256 experts (before: four wavefronts of 32 tokens x 256
+// experts, tokens straight from global memory in MFMA layout one step ahead, twice as many slices where those had to divide the
+// steps): hidden 7168, 64 tokens 23.0 -> 14.5, 512 tokens 32.3 -> 18.0, 8192 tokens 87.2 -> 59.4; hidden 1624, 8176 tokens
+// 120.2 -> 34.2.  128 experts, hidden 4096, 4096 tokens 33.6 -> 25.1.
+template <int NB>
+__global__ __launch_bounds__(512) void gate_logits_wide_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int64_t T,
+                                                               int H, int N, int h_per_split, float *__restrict__ partial) {
+    constexpr int NP = NB * 32, SLOTS = 3, WN = NP / 64, TM = GT / 32 / (8 / WN), TN = 2;
+    constexpr int UNITS = (GT + NP) / 8, LOADS = UNITS / 8;   // 1 KB direct loads of a step, tokens first, and a wavefront's
+    constexpr int STEP = (GT + NP) * 128;
+    __shared__ __attribute__((aligned(1024))) char lds[SLOTS * STEP];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int wm = wave / WN, wn = wave % WN;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.x) * GT;
+    const int h_begin = blockIdx.y * h_per_split, h_len = min(H - h_begin, h_per_split), steps = (h_len + GK - 1) / GK;
+    const uint32_t lds0 = lds_address(lds);
+    const char *src[LOADS];
+    int chunk[LOADS];
+#pragma unroll
+    for (int l = 0; l < LOADS; l++) {
+        const int unit = wave * LOADS + l, row = unit * 8 + (lane >> 3);
+        chunk[l] = (lane & 7) ^ ((row >> 1) & 7);
+        // rows past the end (tokens, experts): valid memory, results unused
+        src[l] = reinterpret_cast<const char *>(row < GT ? x + min(t0 + row, T - 1) * H + h_begin
+                                                         : w + static_cast<int64_t>(min(row - GT, N - 1)) * H + h_begin);
+    }
+    auto issue = [&](int s, int slot) {
+        const int last = ((h_len - s * GK) >> 3) - 1;         // chunks past the end: the last one again
+#pragma unroll
+        for (int l = 0; l < LOADS; l++)
+            dma16_lane(src[l] + s * (GK * 2) + min(chunk[l], last) * 16, lds0 + slot * STEP + (wave * LOADS + l) * 1024);
+    };
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    issue(0, 0);
+    if (steps > 1) issue(1, 1);
+    int slot = 0, free_slot = 2;
+    for (int s = 0; s < steps; s++) {
+        // This wavefront's part of step s has landed; behind the barrier everyone's has, and everyone has read step s - 1,
+        // whose slot takes step s + 2.
+        if (s + 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if ((s + 1) * GK > h_len) {
+#pragma unroll
+            for (int l = 0; l < LOADS; l++)
+                if (wave * LOADS + l < GT / 8 && s * GK + chunk[l] * 8 >= h_len)
+                    *reinterpret_cast<u32x4 *>(lds + slot * STEP + (wave * LOADS + l) * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (s + 2 < steps) issue(s + 2, free_slot);
+        const char *xs = lds + slot * STEP, *ws = xs + GT * 128;
+#pragma unroll
+        for (int u = 0; u < GK / 16; u++) {
+            bf16x8 fx[TM], fw[TN];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+                fx[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(xs + w_off((wm * TM + i) * 32 + (lane & 31), u * 2 + (lane >> 5))));
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+                fw[j] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(ws + w_off((wn * TN + j) * 32 + (lane & 31), u * 2 + (lane >> 5))));
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fx[i], fw[j], acc[i][j], 0, 0, 0);
+        }
+        free_slot = slot;
+        slot = slot == SLOTS - 1 ? 0 : slot + 1;
+    }
+    // accumulator element r of lane l: token 8*(r/4) + 4*(l/32) + r%4, expert l%32
+    float *out = partial + static_cast<int64_t>(blockIdx.y) * T * N;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int64_t t = t0 + (wm * TM + i) * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const int n = (wn * TN + j) * 32 + (lane & 31);
+                if (t < T && n < N) out[t * N + n] = acc[i][j][r];
+            }
+        }
+}
+
 // logits = sum over the slices of H, in slice order
 __global__ __launch_bounds__(256) void gate_logits_reduce_kernel(const float *__restrict__ partial,
                                                                  int splits, int64_t tn,
@@ -149,19 +242,14 @@ inline bool gate_split_shape_ok(int64_t T, int H, int N) {
     return T >= 0 && T <= 0x7fffffffLL && N >= 1 && N <= 256 && H >= 8 && H % 8 == 0;
 }
 
-// Slices of H: enough blocks for one per CU when the token count alone does not give them, each
-// slice a whole number of 64-wide steps, the last of which may be partial (the fp32 partials cost
-// 8 B per logit and slice).  At most 32: 64 tokens, hidden 7168, 256 experts 22 us with 16 slices, 19 with 28.
+// Slices of H: a block per CU, and no more (the fp32 partials cost 8 B per logit and slice).  At most 32: 64 tokens, hidden 7168, 256 experts 22 us with 16 slices, 19 with 28.
+// A slice is a whole number of 64-wide steps, the last one may be shorter and its last step partial.
 inline int gate_split_count(int64_t T, int H) {
-    const int64_t token_blocks = (T + GT - 1) / GT;
+    const int64_t token_blocks = std::max<int64_t>((T + GT - 1) / GT, 1);
     const int steps = (H + GK - 1) / GK;
-    int best = 1;
-    for (int s = 1; s <= 32 && s <= steps; s++)
-        if (steps % s == 0) {
-            best = s;
-            if (token_blocks * s >= 256) break;
-        }
-    return best;
+    const int want = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(32, 256 / token_blocks)));
+    const int each = (steps + want - 1) / want;
+    return (steps + each - 1) / each;
 }
 
 }  // namespace
@@ -169,18 +257,17 @@ inline int gate_split_count(int64_t T, int H) {
 // Behind a routing kernel that adds the slices itself: eight of them where the steps divide (the order of
 // the sums is then that of om_router_gate_softmax_topk, bit for bit), else as above.
 int om_gate_route_splits(int64_t T, int H, int N) {
-    const int steps = (H + GK - 1) / GK;
-    return N <= 64 && H % 512 == 0 && steps % 8 == 0 ? 8 : gate_split_count(T, H);
+    return N <= 64 && H % 512 == 0 ? 8 : gate_split_count(T, H);
 }
 
 void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, int splits, float *ws,
                              hipStream_t st) {
     const dim3 grid(static_cast<unsigned>((T + GT - 1) / GT), splits);
     const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(gate_weight);
-    const int hps = (H + GK - 1) / GK / splits * GK;   // a whole number of steps; the last slice may end early
+    const int hps = ((H + GK - 1) / GK + splits - 1) / splits * GK;
     if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
-    else if (N <= 128) gate_logits_split_kernel<4><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
-    else gate_logits_split_kernel<8><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    else if (N <= 128) gate_logits_wide_kernel<4><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    else gate_logits_wide_kernel<8><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);
 }
 
 extern "C" int64_t om_router_gate_route_workspace_bytes(int64_t T, int H, int N) {

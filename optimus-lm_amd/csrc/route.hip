@@ -503,12 +503,6 @@ __device__ __forceinline__ void row_softmax_topk(float (&p)[Q], int N, int K, in
 // us with the routing (before: eight wavefronts over eight slices with fragments straight from global memory, 32-byte
 // pieces of 64 rows at a time): 64 experts, hidden 2048: 4096 tokens 10.7 (22.0), 16384 tokens 23.6 (38.0: 2.8 TB/s of x
 // now); 32 experts, hidden 1024: 512 tokens 4.9 (9.0), 16384 tokens 11.0 (20.6).
-typedef __attribute__((address_space(3))) char *lds_bytes;
-// 16 bytes from each lane's address to LDS at m0 + 16 * lane.  Outside the compiler's view: the code waits itself.
-__device__ __forceinline__ void dma16(const char *lane_address, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(lane_address) : "memory");
-}
-
 template <int NB, typename TL, typename TW, bool ROUTE>
 __global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg,
                                                                      int64_t Tn, int H, int N, int K, int renorm,
@@ -530,7 +524,7 @@ __global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint1
     // Chunk c (16 bytes) of a 64-byte row r is stored at c ^ (r / 4 % 4): fragment reads of 16 rows use every bank once.
     const char *src[LOADS];
     uint32_t dst[LOADS];
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes)lds));
+    const uint32_t lds0 = lds_address(lds);
 #pragma unroll
     for (int l = 0; l < LOADS; l++) {
         const int unit = nb * LOADS + l, row = (unit < 2 ? unit : unit - 2) * 16 + (lane >> 2);
@@ -542,7 +536,7 @@ __global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint1
     }
     auto issue = [&](int step, int slot) {
 #pragma unroll
-        for (int l = 0; l < LOADS; l++) dma16(src[l] + step * 64, dst[l] + slot * STEP_BYTES);
+        for (int l = 0; l < LOADS; l++) dma16_lane(src[l] + step * 64, dst[l] + slot * STEP_BYTES);
     };
     f32x16 acc;
 #pragma unroll

@@ -495,3 +495,32 @@ def test_one_launch_gate_router(cuda, T, H, N, K, renorm, one_pass, bf16_logits)
     # an fp32 sum of H exact products in any order, then (bf16) one rounding of 2^-9
     bound = 8 * 2.0 ** -24 * (x[ok].double().abs() @ w.double().abs().t()) + (2.0 ** -8 * ref.abs() if bf16_logits else 0)
     assert bool(((logits[ok].double() - ref).abs() <= bound + 1e-30).all())
+
+
+@pytest.mark.parametrize("T,H,N", [(1, 8, 65), (127, 72, 100), (129, 64, 128), (257, 128, 129), (256, 1624, 256), (640, 200, 160), (300, 7168, 80),
+                                   (33000, 136, 256)])
+@pytest.mark.parametrize("base", [False, True])
+def test_gate_of_many_experts(cuda, T, H, N, base):
+    """Projection and input gradient of more than 64 experts: edges of the blocks of 128 and 256 tokens, one to three steps
+    of 64 columns and a partial last one, slices of unequal length, experts that do not fill their tiles; with `base` the
+    sum has a second rounding."""
+    from optimus import _native as n
+    L, P = n.lib(), n.ptr
+    x, w = _gate_inputs(T, H, N, seed=T + H + N)
+    g = torch.Generator().manual_seed(N)
+    dl = torch.randn(T, N, generator=g)
+    x, w, dl = x.to(cuda), w.to(cuda), dl.to(cuda)
+    logits, dx = torch.full((T, N), 7.0, device=cuda), torch.full((T + 1, H), 7.0, dtype=torch.bfloat16, device=cuda)
+    size = L.om_router_gate_logits_split_workspace_bytes(T, H, N)
+    ws = torch.empty(size, dtype=torch.uint8, device=cuda)
+    n.check(L.om_router_gate_logits_split(P(x), P(w), T, H, N, P(logits), P(ws), size, n.stream()), "logits")
+    n.check(L.om_router_gate_dgrad(P(dl), P(w), P(x) if base else None, P(dx), T, H, N, n.stream()), "dgrad")
+    # a rounding of 2^-24 of the sum so far for every 16 columns and every slice
+    bound = (H / 16 + 33) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30
+    assert bool(((logits.double() - x.double() @ w.double().t()).abs() <= bound).all())
+    d16 = dl.to(torch.bfloat16).double()
+    exact = d16 @ w.double()
+    total = exact + x.double() if base else exact
+    bound = 2e-6 * (d16.abs() @ w.double().abs()) + exact.abs() * 2.0 ** -8 + (total.abs() * 2.0 ** -8 if base else 0) + 1e-30
+    assert bool(((dx[:T].double() - total).abs() <= bound).all())
+    assert bool((dx[T] == 7.0).all())
