@@ -156,6 +156,122 @@ __global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restr
         }
 }
 
+// The same for more than 128 experts, a multiple of 4 of them: 256 rows and 256 columns of dW per block of eight wavefronts (64 x
+// 128 each), so that the fp32 dlogits are read once per 256 columns, in steps of 32 tokens.  x comes by direct loads two steps
+// ahead through a ring of three, the dlogits through registers, two steps ahead too, and a pair of buffers.  Every step loads,
+// past the last one that one again, so that the number of loads in flight is known.
+// us with the launch that adds the ranges, x out of the caches, before (128 columns a block, both operands through registers
+// one stage ahead) -> now, 256 experts: hidden 7168, 64 tokens 19.3 -> 16.4, 2048 tokens 57 -> 41, 8192 tokens 115 -> 72; hidden
+// 1624, 8176 tokens 60 -> 42.  160 experts, hidden 5120, 4096 tokens 56 -> 37.
+constexpr int WW_HT = 256, WW_TC = 32;
+__global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__restrict__ x, const float *__restrict__ dlogits, int64_t T,
+                                                              int H, int N, int64_t tokens_per_split, float *__restrict__ partial) {
+    constexpr int SLOTS = 3, XS = WW_TC * WW_HT * 2, DS = WW_TC * 256 * 2, XL = XS / 1024 / 8, DL = WW_TC * 256 / 4 / 512;
+    constexpr int TM = 2, TN = 4;
+    __shared__ __attribute__((aligned(1024))) char lds[SLOTS * XS + 2 * DS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int h0 = blockIdx.x * WW_HT;
+    const int64_t t_begin = static_cast<int64_t>(blockIdx.y) * tokens_per_split;
+    const int tokens = static_cast<int>(max(min(tokens_per_split, T - t_begin), static_cast<int64_t>(0)));
+    const int steps = (tokens + WW_TC - 1) / WW_TC;
+    float *out = partial + static_cast<int64_t>(blockIdx.y) * N * H;
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    if (steps > 0) {
+        const uint32_t lds0 = lds_address(lds);
+        char *const ds = lds + SLOTS * XS;
+        auto x_row = [&](int l) { return (wave * XL + l) * 2 + (lane >> 5); };
+        auto issue_x = [&](int s, int slot) {     // rows and columns past the end: valid memory; the rows are zeroed, the columns unused
+            const int step = min(s, steps - 1) * WW_TC;
+#pragma unroll
+            for (int l = 0; l < XL; l++) {
+                const int row = x_row(l), col = h0 + ((lane & 31) ^ ((row & 3) << 2)) * 8;
+                dma16_lane(reinterpret_cast<const char *>(x + (t_begin + min(step + row, tokens - 1)) * H + min(col, H - 8)),
+                           lds0 + slot * XS + (wave * XL + l) * 1024);
+            }
+        };
+        f32x4 dq[2][DL];
+        auto fetch_d = [&](int s, int set) {
+            const int step = min(s, steps - 1) * WW_TC;
+#pragma unroll
+            for (int j = 0; j < DL; j++) {
+                const int q = j * 512 + tid;
+                dq[set][j] = *reinterpret_cast<const f32x4 *>(dlogits + (t_begin + min(step + q / 64, tokens - 1)) * N + min(q % 64 * 4, N - 4));
+            }
+        };
+        auto stash_d = [&](int s, int set) {      // tokens and experts past the end: zeros
+#pragma unroll
+            for (int j = 0; j < DL; j++) {
+                const int q = j * 512 + tid, crow = q / 64, n = q % 64 * 4;
+                const bool inside = s * WW_TC + crow < tokens && n < N;
+                const f32x4 d = dq[set][j];
+                const u32x2 v = {inside ? pack2(d[0], d[1]) : 0u, inside ? pack2(d[2], d[3]) : 0u};
+                *reinterpret_cast<u32x2 *>(ds + (s & 1) * DS + tile_off<256>(crow, n >> 3) + (n & 7) * 2) = v;
+            }
+        };
+        issue_x(0, 0);
+        fetch_d(0, 0);
+        stash_d(0, 0);
+        fetch_d(1, 1);
+        issue_x(1, 1);
+        fetch_d(2, 0);
+        int slot = 0, free_slot = 2;
+        auto step = [&](int s, int set) {         // set: the dlogits of step s + 1
+            // This wavefront's part of x of step s has landed: younger are the dlogits of steps s + 1 and s + 2 and x of s + 1.
+            // Behind the barrier everyone's has, the dlogits of step s are there, and step s - 1 has been read.
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XL + DL) : "memory");
+            if ((s + 1) * WW_TC > tokens) {
+#pragma unroll
+                for (int l = 0; l < XL; l++)
+                    if (s * WW_TC + x_row(l) >= tokens) *reinterpret_cast<u32x4 *>(lds + slot * XS + (wave * XL + l) * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            stash_d(s + 1, set);
+            issue_x(s + 2, free_slot);
+            fetch_d(s + 3, set);
+            const char *xs = lds + slot * XS, *dd = ds + (s & 1) * DS;
+#pragma unroll
+            for (int kk = 0; kk < WW_TC / 16; kk++) {
+                bf16x8 fd[TM], fx[TN];
+#pragma unroll
+                for (int i = 0; i < TM; i++) fd[i] = read_frag<256>(dd, kk * 16, wm * 64 + i * 32, lane);
+#pragma unroll
+                for (int j = 0; j < TN; j++) fx[j] = read_frag<256>(xs, kk * 16, wn * 128 + j * 32, lane);
+#pragma unroll
+                for (int i = 0; i < TM; i++)
+#pragma unroll
+                    for (int j = 0; j < TN; j++)
+                        // lane l then holds column h = l % 32 and rows n = 8*(r/4) + 4*(l/32) + r%4
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fd[i], fx[j], acc[i][j], 0, 0, 0);
+            }
+            free_slot = slot;
+            slot = slot == SLOTS - 1 ? 0 : slot + 1;
+        };
+        for (int s = 0; s < steps; s += 2) {
+            step(s, 1);
+            if (s + 1 < steps) step(s + 1, 0);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load into LDS outlives the block
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int n = wm * 64 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+                const int h = h0 + wn * 128 + j * 32 + (lane & 31);
+                if (n < N && h < H) out[static_cast<int64_t>(n) * H + h] = acc[i][j][r];
+            }
+        }
+}
+
 // dW = sum over splits, in split order; 4 elements per thread.
 template <typename T>
 __global__ __launch_bounds__(256) void gate_wgrad_reduce_kernel(const float *__restrict__ partial,
@@ -182,11 +298,13 @@ __global__ __launch_bounds__(256) void gate_wgrad_reduce_kernel(const float *__r
     }
 }
 
-// Token ranges: enough blocks to fill the chip twice over, at least two stages each.
-inline int gate_wgrad_splits(int64_t T, int H) {
+inline bool gate_wgrad_wide(int N) { return N > 128 && N % 4 == 0; }
+
+// Token ranges: the blocks that the chip holds at once (two per CU, one of the wide kernel's), at least two stages of tokens each.
+inline int gate_wgrad_splits(int64_t T, int H, int N) {
     const int64_t stages = (T + TC - 1) / TC;
-    const int slices = (H + HT - 1) / HT;
-    int64_t want = 2 * 256 / slices;   // two blocks per CU, all at once
+    const int ht = gate_wgrad_wide(N) ? WW_HT : HT, blocks = gate_wgrad_wide(N) ? 256 : 512;
+    int64_t want = blocks / ((H + ht - 1) / ht);
     if (want > stages / 2) want = stages / 2;
     if (want < 1) want = 1;
     if (want > 256) want = 256;
@@ -514,7 +632,7 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
 
 extern "C" int64_t om_router_gate_wgrad_workspace_bytes(int64_t T, int H, int N) {
     if (!gate_wgrad_shape_ok(T, H, N)) return OM_ERR_SHAPE;
-    return static_cast<int64_t>(gate_wgrad_splits(T, H)) * N * H * 4;
+    return static_cast<int64_t>(gate_wgrad_splits(T, H, N)) * N * H * 4;
 }
 
 extern "C" int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t T, int H, int N,
@@ -526,7 +644,7 @@ extern "C" int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t
     if (T > 0 && (!x || !dlogits)) return OM_ERR_NULL;
     if (!om_aligned16(x) || !om_aligned16(dlogits) || !om_aligned16(dweight) || !om_aligned16(workspace))
         return OM_ERR_ALIGN;
-    const int splits = gate_wgrad_splits(T, H);
+    const int splits = gate_wgrad_splits(T, H, N);
     const int64_t nh = static_cast<int64_t>(N) * H;
     if (workspace_bytes < splits * nh * 4) return OM_ERR_WORKSPACE;
     hipStream_t st = om_stream(stream);
@@ -535,7 +653,9 @@ extern "C" int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t
     const dim3 grid((H + HT - 1) / HT, splits);
     const uint16_t *xp = static_cast<const uint16_t *>(x);
     float *ws = static_cast<float *>(workspace);
-    if (N <= 32)
+    if (gate_wgrad_wide(N))
+        gate_wgrad_wide_kernel<<<dim3((H + WW_HT - 1) / WW_HT, splits), dim3(512), 0, st>>>(xp, dlogits, T, H, N, tokens_per_split, ws);
+    else if (N <= 32)
         gate_wgrad_kernel<1><<<grid, dim3(256), 0, st>>>(xp, dlogits, T, H, N, tokens_per_split, ws);
     else if (N <= 64)
         gate_wgrad_kernel<2><<<grid, dim3(256), 0, st>>>(xp, dlogits, T, H, N, tokens_per_split, ws);

@@ -498,10 +498,10 @@ def test_one_launch_gate_router(cuda, T, H, N, K, renorm, one_pass, bf16_logits)
 
 
 @pytest.mark.parametrize("T,H,N", [(1, 8, 65), (127, 72, 100), (129, 64, 128), (257, 128, 129), (256, 1624, 256), (640, 200, 160), (300, 7168, 80),
-                                   (33000, 136, 256)])
+                                   (33000, 136, 256), (700, 264, 132), (1000, 520, 250)])
 @pytest.mark.parametrize("base", [False, True])
 def test_gate_of_many_experts(cuda, T, H, N, base):
-    """Projection and input gradient of more than 64 experts: edges of the blocks of 128 and 256 tokens, one to three steps
+    """Projection and both gradients of more than 64 experts: edges of the blocks of 128 and 256 tokens, one to three steps
     of 64 columns and a partial last one, slices of unequal length, experts that do not fill their tiles; with `base` the
     sum has a second rounding."""
     from optimus import _native as n
@@ -524,3 +524,12 @@ def test_gate_of_many_experts(cuda, T, H, N, base):
     bound = 2e-6 * (d16.abs() @ w.double().abs()) + exact.abs() * 2.0 ** -8 + (total.abs() * 2.0 ** -8 if base else 0) + 1e-30
     assert bool(((dx[:T].double() - total).abs() <= bound).all())
     assert bool((dx[T] == 7.0).all())
+    if base:
+        return
+    dw = torch.full((N + 1, H), 7.0, device=cuda)
+    size = L.om_router_gate_wgrad_workspace_bytes(T, H, N)
+    ws = torch.empty(size, dtype=torch.uint8, device=cuda)
+    n.check(L.om_router_gate_wgrad(P(x), P(dl), T, H, N, P(dw), 0, P(ws), size, n.stream()), "wgrad")
+    bound = (T / 16 + 300) * 2.0 ** -24 * (d16.abs().t() @ x.double().abs()) + 1e-30
+    assert bool(((dw[:N].double() - d16.t() @ x.double()).abs() <= bound).all())
+    assert bool((dw[N] == 7.0).all())
