@@ -110,6 +110,7 @@ struct GemmParams {
     int phases;                 // 1 or 2
     int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert (MERGED: of all three)
+    bool stream;                // wgrad: the gradients do not fit the caches (see CACHED_WEIGHTS)
     int share;                  // XCDs that share an expert's tiles; 0: contiguous runs of tiles per XCD
     WgradSet set[3];            // MERGED
 };
@@ -353,6 +354,14 @@ __device__ __forceinline__ void dma16_if(int left, const void *base, uint32_t la
                  "global_load_lds_dwordx4 %1, %2\n.Lom_skip%=:"
                  :: "s"(lds_base), "v"(lane_bytes), "s"(base), "n"(OFS), "s"(left) : "scc");
 }
+// dma16_if of data that is read once: kept out of the caches where `once` is set
+template <int OFS>
+__device__ __forceinline__ void dma16_if_once(int left, int once, const void *base, uint32_t lane_bytes, uint32_t lds_base) {
+    asm volatile("s_cmp_lt_i32 %4, 2\n\ts_cbranch_scc1 .Lom_skip%=\n\ts_add_u32 m0, %0, %3\n\ts_cmp_eq_u32 %5, 0\n\t"
+                 "s_cbranch_scc1 .Lom_keep%=\n\tglobal_load_lds_dwordx4 %1, %2 nt\n\ts_branch .Lom_skip%=\n.Lom_keep%=:\n\t"
+                 "global_load_lds_dwordx4 %1, %2\n.Lom_skip%=:"
+                 :: "s"(lds_base), "v"(lane_bytes), "s"(base), "n"(OFS), "s"(left), "s"(once) : "scc");
+}
 // This wavefront's direct loads but the N youngest have landed, and its LDS reads are back.
 template <int N> __device__ __forceinline__ void wait_loads(uint32_t lds) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N), "s"(lds) : "memory");
@@ -373,7 +382,7 @@ template <int V> using IntC = std::integral_constant<int, V>;
 // (second launch bound: two wavefronts per SIMD, i.e. at most 256 registers, for the 128x128 tile, whose two blocks per
 // CU depend on it; the 256x256 tile's 8 wavefronts imply it already)
 template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool ACCUM = false,
-          bool EDGE = false>
+          bool EDGE = false, bool ONCE = false>
 __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
     constexpr int BN = BM, WAVES_N = BN / 64, NW = 2 * WAVES_N;
     constexpr int TM = BM / 64, TN = 2;     // row units of a tile, accumulators of a wavefront in each
@@ -408,6 +417,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     int expert = 0, row_begin = 0, row_end = 0, n0 = 0, c_begin = 0, c_len = 0;
     int steps_per_phase = 0, c_wrap = 0, n_steps = 0, rot = 0;
     int active = TM;      // row units that hold rows of the expert
+    int once = 0;         // ONCE: whether no other row tile reads the expert's weights
     // the slot of this wavefront's direct load l of a unit: row (CONTIG) or contraction row (STRIDED) and chunk
     auto slot = [&](int l) { return (wave * L + l) * 8 + (lane >> 3); };
     uint32_t a_off[AKIND == CONTIG ? UA : 1][L];   // bytes from the step's base: CONTIG, the row of each unit
@@ -497,6 +507,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 row_begin = q.row_begin + tile_m * BM;
                 row_end = q.row_end;
             } else if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
+            if (ONCE) once = __builtin_amdgcn_readfirstlane(row_end - row_begin <= BM && (p.share ? tile_m == 0 : row_begin == seg[expert]) ? 1 : 0);
             rot_a = tile_n; rot_b = tile_m & 7;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
@@ -621,7 +632,9 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             if (BKIND == CONTIG) off -= tail_bytes(c0, l);
             else off += crow_bytes(c0, l, ldb32, rows, b_indexed);
             const char *q = EDGE ? base : BKIND == CONTIG ? base + U * b_unit : base + U * 128;
-            if (l == 0) dma16_if<B0 + P * B_STAGE + U * UNIT>(left, q, off, wave_lds);
+            if (ONCE && l == 0) dma16_if_once<B0 + P * B_STAGE + U * UNIT>(left, once, q, off, wave_lds);
+            else if (ONCE) dma16_if_once<B0 + P * B_STAGE + U * UNIT + 1024>(left, once, q, off, wave_lds);
+            else if (l == 0) dma16_if<B0 + P * B_STAGE + U * UNIT>(left, q, off, wave_lds);
             else dma16_if<B0 + P * B_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
         }
     };
@@ -1066,7 +1079,13 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                         for (int x = 0; x < 4; x++)
                             v[x] = pack2_bf16(prev[2 * x] + fresh[2 * x], prev[2 * x + 1] + fresh[2 * x + 1]);
                     }
-                    *reinterpret_cast<u32x4 *>(Cb + o) = v;
+                    if (WGRAD && !EDGE && p.stream) {
+                        asm volatile("");   // (or the compiler makes one ordinary store of the two)
+                        __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(Cb + o));
+                        asm volatile("");
+                    } else {
+                        *reinterpret_cast<u32x4 *>(Cb + o) = v;
+                    }
                     if (EPI == EPI_SWIGLU) {
                         *reinterpret_cast<u32x4 *>(p.C1 + o) = strip_get(1, q / CPRW, q % CPRW);
                         *reinterpret_cast<u32x4 *>(p.C2 + o) = strip_get(2, q / CPRW, q % CPRW);
@@ -1120,6 +1139,16 @@ template <int BM> unsigned persistent_blocks(int64_t tiles) {
 }
 
 
+// Elements of the weights, or of their gradients, that the caches (256 MB, and more passes through them) cannot hold from one use to the
+// next.  From there on they are kept out: the 128x128 row products load the weights of an expert with one row tile without leaving
+// them there, the 256x256 weight gradients are stored past them; what the caches held instead was written back or fetched again under
+// the next products.  us, 64 experts of 1024/2048: 37 tokens gate+up 104 -> 93 (5.8 TB/s of weights), down 50 -> 44;
+// 512 tokens, uneven, gate/up input gradient behind the weight gradients 167 -> 104, those 209 -> 214; 32 experts of 2048/7168, 64
+// rows in all, 146 -> 133 and 84 -> 75.  Weights that do fit lose by it (32 experts of 376/1720, 733 tokens: forward 113 -> 117),
+// and so do those that a second row tile reads (12 experts of 712/1000, 750 rows each: gate+up 51 -> 82 when all were
+// loaded so) and the saved g and u of the forward (prefill of 4096 tokens, gate+up 344 -> 354).
+constexpr int64_t CACHED_WEIGHTS = 128 << 20;
+
 // XCDs that share an expert's row products: from 8 M weights a matrix on, four, or all eight with few experts, which two
 // groups of XCDs could not divide evenly.  One expert alone needs no sharing: its tiles are alike.
 inline int rows_share(const GemmParams &p, int64_t expected) {
@@ -1136,8 +1165,12 @@ int launch_rows(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
     const int64_t m_tiles_max = (rows + BM - 1) / BM + p.n_experts;
     const int64_t tiles = m_tiles_max * ((p.n_cols + BN_OUT - 1) / BN_OUT);
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
-    ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128>
-        <<<dim3(persistent_blocks<BM>(tiles)), dim3(THREADS<BM>), 0, st>>>(p);
+    const dim3 grid(persistent_blocks<BM>(tiles)), block(THREADS<BM>);
+    const int64_t weights = static_cast<int64_t>(p.n_experts) * p.n_cols * p.kc * (EPI == EPI_SWIGLU ? 2 : p.phases);
+    if (BM == 128 && weights >= CACHED_WEIGHTS)
+        ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128, BM == 128><<<grid, block, 0, st>>>(p);
+    else
+        ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128><<<grid, block, 0, st>>>(p);
     return om_launch_status();
 }
 
@@ -1266,6 +1299,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
     p.share = wgrad_share(big, p.tiles_e, G);
+    p.stream = static_cast<int64_t>(G) * N * K >= CACHED_WEIGHTS;
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
@@ -1407,6 +1441,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     }
     p.tiles_e = static_cast<int>(3 * each);
     p.share = wgrad_share(big, p.tiles_e, G);
+    p.stream = 3 * packed * G >= CACHED_WEIGHTS;
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);
