@@ -102,7 +102,9 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 // The grouped products of few rows per expert (ggemm_stream.hip): the rule, and the launches that the entry
 // points of ggemm.hip make under it.  Arguments are checked by the caller.  `expected`: the rows to choose by,
 // `rows` where they are known and fewer where `rows` is a bound.
-bool om_ggemm_streams(int64_t rows, int n_experts, int cols);   // cols: weight rows per expert (gate and up: both)
+bool om_ggemm_streams(int64_t rows, int n_experts, int cols, int kc);   // cols: weight rows per expert (gate and up: both)
+// Elements of weights, or of their gradients, that the caches cannot hold from one use to the next (see ggemm.hip).
+constexpr int64_t CACHED_WEIGHTS = 128 << 20;
 int om_ggemm_stream_gate_up(const void *x, const int32_t *x_rows, const void *w_gate, const void *w_up,
                             const float *row_weights, void *g, void *u, void *h, const int32_t *cum, int64_t rows, int64_t expected,
                             int G, int I, int H, int64_t w_stride, hipStream_t st);

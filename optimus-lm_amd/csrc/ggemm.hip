@@ -43,7 +43,8 @@
 // contraction range of expert g; rows past its end are zero-filled in LDS.
 //
 // Block order: consecutive block ids go to different XCDs (8 per chip, each with its own L2), so
-// block ids are remapped to give every XCD a contiguous run of tiles, which share operand tiles.
+// block ids are remapped to give every XCD a contiguous run of tiles, which share operand tiles, or, with large experts,
+// a part of each expert (GemmParams::share).
 //
 // Two things that surround the expert GEMMs in the layer are folded into them (template parameters
 // GATHER and ROWW): the token gather (an operand's rows are fetched through an index: the A rows of
@@ -1139,15 +1140,14 @@ template <int BM> unsigned persistent_blocks(int64_t tiles) {
 }
 
 
-// Elements of the weights, or of their gradients, that the caches (256 MB, and more passes through them) cannot hold from one use to the
-// next.  From there on they are kept out: the 128x128 row products load the weights of an expert with one row tile without leaving
-// them there, the 256x256 weight gradients are stored past them; what the caches held instead was written back or fetched again under
+// CACHED_WEIGHTS: the caches hold 256 MB, and more than the weights passes through them.  From there on the weights are
+// kept out of them: the 128x128 row products load those of an expert with one row tile without leaving them there, the
+// 256x256 weight gradients are stored past them; what the caches held instead was written back or fetched again under
 // the next products.  us, 64 experts of 1024/2048: 37 tokens gate+up 104 -> 93 (5.8 TB/s of weights), down 50 -> 44;
 // 512 tokens, uneven, gate/up input gradient behind the weight gradients 167 -> 104, those 209 -> 214; 32 experts of 2048/7168, 64
 // rows in all, 146 -> 133 and 84 -> 75.  Weights that do fit lose by it (32 experts of 376/1720, 733 tokens: forward 113 -> 117),
 // and so do those that a second row tile reads (12 experts of 712/1000, 750 rows each: gate+up 51 -> 82 when all were
 // loaded so) and the saved g and u of the forward (prefill of 4096 tokens, gate+up 344 -> 354).
-constexpr int64_t CACHED_WEIGHTS = 128 << 20;
 
 // XCDs that share an expert's row products: from 8 M weights a matrix on, four, or all eight with few experts, which two
 // groups of XCDs could not divide evenly.  One expert alone needs no sharing: its tiles are alike.
@@ -1233,7 +1233,7 @@ extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, 
     p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N))
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N, K))
         return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, p.strideB,
                                    om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
@@ -1500,7 +1500,7 @@ int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, c
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I))
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I, H))
         return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, expected, G, I,
                                        H, p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
