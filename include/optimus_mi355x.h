@@ -442,7 +442,7 @@ int om_rmsnorm_bwd(const void *dy, const void *h, const void *weight, const floa
  * serves per-expert nn.Linear weights that sit at a constant pitch inside one flat buffer
  * (a multiple of 8 elements, else OM_ERR_ALIGN).  N and K must be multiples of 8, the size of a
  * 16-byte vector (the 256x256 tile serves extents that are multiples of 256 with a contraction that
- * is a multiple of 128; the 128x128 tile everything else, with a partial last tile where an extent
+ * is a multiple of 64; the 128x128 tile everything else, with a partial last tile where an extent
  * is not a multiple of 128 and a zero-filled last contraction step where the contraction length is
  * not a multiple of 64).
  * Tensors
@@ -597,7 +597,7 @@ int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void
  * epilogue:  weight_grad = cast(float(weight_grad) + float(cast(dW)))  in the gradient's dtype,
  * the bits of the in-place add on a freshly rounded dW, without dW being written or re-read.
  * Arguments as the entry points of the same name without the suffix; weight_grad is read and
- * written (every element, also those of experts without rows).                               */
+ * written (where an expert has no rows there is nothing to add, and its elements may be left alone). */
 int om_grouped_gemm_wgrad_accumulate(const void *output_grad, const void *input, void *weight_grad,
                                      const int32_t *cum_token_counts, int64_t rows, int G, int N, int K,
                                      int64_t w_stride, void *stream);
