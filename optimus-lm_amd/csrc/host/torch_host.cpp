@@ -1,8 +1,8 @@
 // The host side of the MoE block in C++: allocations, launches of the C-ABI entry points and the
 // autograd nodes around them, as the Python module `optimus_torch_host`.
 //
-// What bounded the small calls was the interpreter: a training step of the tiny layer is 22 launches of
-// 2-14 us each, and enqueueing them through ctypes and Python autograd functions took 510 us.  Here a
+// What bounded the small calls was the interpreter: a training step of the tiny layer was 22 launches
+// (15 now) of 2-14 us each, and enqueueing them through ctypes and Python autograd functions took 510 us.  Here a
 // layer is two autograd nodes (router, experts) whose forward and backward run without the interpreter:
 // each reads the three run-time switches of the Python modules once (launch log, profiler, in-place
 // weight gradients) and then only allocates and launches.
