@@ -272,6 +272,20 @@ __device__ __forceinline__ void build_part_table(const int32_t *cum, const int *
         base_tiles += __shfl(incl, 63, 64);
     }
 }
+// first[e]: row tiles of the experts before e.  One wavefront.
+template <int BM> __device__ __forceinline__ void build_first_tiles(const int32_t *cum, int n_experts, int lane, int *first) {
+    int base_tiles = 0;
+    for (int e0 = 0; e0 < n_experts; e0 += 64) {
+        const int e = min(e0 + lane, n_experts - 1), tiles = e0 + lane < n_experts ? (cum[e + 1] - cum[e] + BM - 1) / BM : 0;
+        int incl = tiles;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += v;
+        }
+        if (e0 + lane < n_experts) first[e] = base_tiles + incl - tiles;
+        base_tiles += __shfl(incl, 63, 64);
+    }
+}
 // The part that tile `at` of the XCD (less than the last tile_end) belongs to.
 __device__ __forceinline__ Part find_part(const int *tile_end, const Part *part, int n_experts, int lane, int at) {
     int i = 0;
@@ -407,7 +421,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     __shared__ int order[SHARES ? SHARE_MAX_EXPERTS : 1];
     __shared__ __attribute__((aligned(16))) Part part[SHARES ? SHARE_MAX_EXPERTS : 1];
     __shared__ int tile_end[!WGRAD ? MAX_EXPERTS : SHARES ? SHARE_MAX_EXPERTS : 1];   // see build_tile_table, build_part_table
-    __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];
+    __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];   // see build_tile_table; p.share: build_first_tiles
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -498,7 +512,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         } else {
             constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
             const int tiles_n = (p.n_cols + BN_OUT - 1) / BN_OUT;
-            int tile_m = logical / tiles_n, tile_n = logical % tiles_n;
+            int tile_m = logical / tiles_n, tile_n = logical % tiles_n, row_tile = tile_m;
             if (p.share) {
                 const Part q = find_part(tile_end, part, p.n_experts, lane, logical);
                 const int tile = logical + q.shift, tiles_m = (q.row_end - q.row_begin + BM - 1) / BM;
@@ -507,9 +521,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 expert = q.expert;
                 row_begin = q.row_begin + tile_m * BM;
                 row_end = q.row_end;
+                row_tile = __builtin_amdgcn_readfirstlane(seg[expert]) + tile_m;
             } else if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
             if (ONCE) once = __builtin_amdgcn_readfirstlane(row_end - row_begin <= BM && (p.share ? tile_m == 0 : row_begin == seg[expert]) ? 1 : 0);
-            rot_a = tile_n; rot_b = tile_m & 7;
+            // (`row_tile` among all experts' with and without p.share: the sums begin at the same step, the same bits)
+            rot_a = tile_n; rot_b = row_tile & 7;
             n0 = tile_n * BN_OUT;
             c_begin = 0;
             c_len = p.kc;
@@ -737,6 +753,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     if (SHARES && p.share) {
         expert_order(p.cum, p.n_experts, tid, lane, order);
         if (wave == 0) build_part_table(p.cum, order, p.n_experts, p.share, xcd, lane, tiles_of, tile_end, part);
+        if constexpr (!WGRAD) { if (wave == 1) build_first_tiles<BM>(p.cum, p.n_experts, lane, seg); }
         __syncthreads();
         per = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]);
     } else {

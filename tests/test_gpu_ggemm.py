@@ -669,6 +669,49 @@ def test_row_products_of_shared_experts(cuda, kind, G, rows, N, K):
     assert ((h.float() - silu).abs() <= silu.abs() * 2 ** -6 + (g.float().abs() + 1) * (u.float().abs() + 1) * 2 ** -7).all()
 
 
+# (rows per expert: enough to share, on 128x128 tiles; extents that tiles and steps divide and do not)
+@pytest.mark.parametrize("kind,G,rows,I,H", [("ragged", 16, 1500, 2048, 4096), ("empties", 5, 500, 2056, 4104), ("ragged", 33, 1100, 2056, 4104)])
+def test_sharing_experts_leaves_the_bits(cuda, kind, G, rows, I, H):
+    """Experts divided among XCDs or not (fewer rows expected): the products of the merged MLP add in the same order."""
+    from optimus import _native as n
+    torch.manual_seed(G)
+    bf = lambda *s, f=1.0: (torch.randn(*s, device=cuda) * f).to(torch.bfloat16)
+    x, dy, wg, wu, wd = bf(rows, H), bf(rows, H), bf(G, I, H, f=0.02), bf(G, I, H, f=0.02), bf(G, H, I, f=0.02)
+    d, index, scale = _counts(kind, G, rows).to(cuda), torch.randperm(rows, device=cuda, dtype=torch.int32), torch.rand(rows, device=cuda)
+    P, L, parts, out = n.ptr, n.lib(), n.lib().om_merged_mlp_row_dot_parts(I), []
+    for expected in (32 * G - 1, rows):
+        g, u, h, dg, du = (torch.empty(rows, I, dtype=torch.bfloat16, device=cuda) for _ in range(5))
+        y, dx, dot = torch.empty_like(x), torch.empty_like(x), torch.empty(parts, rows, device=cuda)
+        n.check(L.om_merged_mlp_gate_up_fwd_weighted_bound(P(x), P(index), rows, P(wg), P(wu), P(scale), P(g), P(u), P(h), P(d), rows,
+                                                           expected, G, I, H, 0, n.stream()), "gate/up")
+        n.check(L.om_grouped_gemm_fwd_bound(P(h), P(wd), P(y), P(d), rows, expected, G, H, I, 0, n.stream()), "down")
+        n.check(L.om_merged_mlp_down_dgrad_weighted_bound(P(dy), P(index), rows, P(wd), P(g), P(u), P(scale), P(dg), P(du), P(dot), P(d),
+                                                          rows, expected, G, I, H, 0, n.stream()), "down dgrad")
+        n.check(L.om_merged_mlp_gate_up_dgrad_bound(P(dg), P(du), P(wg), P(wu), P(dx), P(d), rows, expected, G, I, H, 0, n.stream()), "dx")
+        out.append((g, u, h, y, dg, du, dot, dx))
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(*out)):
+        assert torch.equal(a, b), i
+
+
+def test_sharing_experts_leaves_the_bits_of_large_tiles(cuda):
+    """The same on 256x256 tiles: an expert's rows as the last row tiles of a launch of one expert, which is not shared;
+    as many tiles before them, modulo the period of the steps that sums begin at (8)."""
+    from optimus import _native as n
+    G, rows, N, K = 9, 4500, 2048, 4096
+    torch.manual_seed(3)
+    x, w = torch.randn(rows, K, device=cuda).to(torch.bfloat16), (torch.randn(G, N, K, device=cuda) * 0.02).to(torch.bfloat16)
+    cum, y, P, before = _counts("ragged", G, rows), torch.empty(rows, N, dtype=torch.bfloat16, device=cuda), n.ptr, 0
+    n.check(n.lib().om_grouped_gemm_fwd(P(x), P(w), P(y), P(cum.to(cuda)), rows, G, N, K, 0, n.stream()), "fwd")
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        xe = torch.cat([torch.zeros((before % 8 + 16) * 256, K, dtype=torch.bfloat16, device=cuda), x[s]])
+        ye, ce = torch.empty(len(xe), N, dtype=torch.bfloat16, device=cuda), torch.tensor([0, len(xe)], dtype=torch.int32, device=cuda)
+        n.check(n.lib().om_grouped_gemm_fwd(P(xe), P(w[e]), P(ye), P(ce), len(xe), 1, N, K, 0, n.stream()), "one expert")
+        assert torch.equal(ye[len(xe) - (s.stop - s.start):], y[s]), e
+        before += (s.stop - s.start + 255) // 256
+
+
 @pytest.mark.parametrize("expected", [0, 9, 100, 1087, 3000, 9000])
 @pytest.mark.parametrize("N,K", [(1024, 512), (200, 328)])
 def test_products_over_a_bound_of_the_rows(cuda, expected, N, K):
