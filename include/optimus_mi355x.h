@@ -617,7 +617,8 @@ int om_grouped_gemm_wgrad_f32_accumulate(const float *output_grad, const float *
 /* The three weight gradients of a merged MLP (in one launch where they are small): dw_down [G,H,I] = dout^T h, dw_gate [G,I,H] = dg^T x and
  * dw_up = du^T x over each expert's rows, or added to what the three hold (`_accumulate`, as above).  dout_rows / x_rows
  * (may be null): row r of dout / x is row dout_rows[r] / x_rows[r] of a [src_rows, H] matrix.  Strides: elements between
- * experts, 0 for packed.  I and H multiples of 8.                                                                    */
+ * experts, 0 for packed.  I and H multiples of 8.  Outputs may lie between one another; where they have memory in common
+ * (weights that are one parameter) they are written, or added to, one after another: down, gate, up.                  */
 int om_grouped_gemm_wgrad_merged(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
                                  const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
                                  void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
@@ -633,7 +634,7 @@ int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const int32_t *dou
 /* The merged MLP of a float32 module (moe.py:396-405 and its autograd), the forms of the bf16 entry points
  * above: gate and up in one launch with h = silu(g) * u formed in the epilogue, the SwiGLU backward in the
  * epilogue of dh = dy W_down, dx as one accumulation over both products, and both weight gradients in one
- * launch (`accumulate` bit 0: add into dw_gate, bit 1: into dw_up).  x_rows (may be null): row r of x is row
+ * launch (`accumulate` bit 0: add into dw_gate, bit 1: into dw_up; gate before up where the two have memory in common).  x_rows (may be null): row r of x is row
  * x_rows[r] of a [src_rows, H] matrix.  I and H multiples of 8.                                             */
 int om_merged_mlp_gate_up_fwd_f32(const float *x, const int32_t *x_rows, int64_t src_rows, const float *w_gate,
                                   const float *w_up, float *g, float *u, float *h, const int32_t *cum_token_counts,
@@ -652,7 +653,8 @@ int om_merged_mlp_gate_up_wgrad_f32(const float *dg, const float *du, const floa
 
 /* The end of the float32 merged MLP's backward in one launch: dx = dg W_gate + du W_up (rows as dg), dw_down = dy^T h,
  * dw_gate = dg^T x and dw_up = du^T x (`_accumulate`: added to what the three hold).  None depends on another, and the
- * launches of a small layer leave most of the chip idle each.  x_rows as above.                                      */
+ * launches of a small layer leave most of the chip idle each.  x_rows as above; weight gradients with memory in common
+ * one after another (down, gate, up).                                                                                 */
 int om_grouped_gemm_wgrad_merged_dgrad_f32(const float *dy, const float *h, const float *dg, const float *du,
                                            const float *x, const int32_t *x_rows, int64_t src_rows,
                                            const float *w_gate, const float *w_up, float *dx, float *dw_down,

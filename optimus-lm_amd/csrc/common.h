@@ -92,6 +92,23 @@ __device__ __forceinline__ uint32_t lds_address(char *shared) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes)shared));
 }
 
+// Whether two arrays of n blocks (`bytes` each, `pitch` bytes apart, positive) have a byte in common: block by block, since
+// the gradients of per-expert modules in a flat buffer lie between one another.
+inline bool om_blocks_overlap(const void *a, int64_t a_pitch, int64_t a_bytes, const void *b, int64_t b_pitch, int64_t b_bytes, int n) {
+    const int64_t d = static_cast<int64_t>(reinterpret_cast<uintptr_t>(b)) - static_cast<int64_t>(reinterpret_cast<uintptr_t>(a));
+    if (d >= (n - 1) * a_pitch + a_bytes || d + (n - 1) * b_pitch + b_bytes <= 0) return false;
+    // is there a block j in [lo, hi] of b with -b_bytes < d + j * b_pitch - at < a_bytes, `at` the offset of a block of a?
+    auto floor_div = [](int64_t x, int64_t y) { return x >= 0 ? x / y : -((-x + y - 1) / y); };
+    auto hit = [&](int64_t at, int64_t lo, int64_t hi) {
+        const int64_t first = floor_div(at - d - b_bytes, b_pitch) + 1, last = floor_div(at - d + a_bytes - 1, b_pitch);
+        return (first > lo ? first : lo) <= (last < hi ? last : hi);
+    };
+    if (a_pitch == b_pitch) return hit(0, 1 - n, n - 1);   // (only the difference of the block numbers matters)
+    for (int i = 0; i < n; i++)
+        if (hit(i * a_pitch, 0, n - 1)) return true;
+    return false;
+}
+
 // 1 / (1 + e^-x) with the hardware exponential and reciprocal (about 1 ulp each, far inside one
 // bf16 rounding of the results it feeds).  An IEEE division here costs ten instructions per
 // element, and the SwiGLU epilogues are bound by vector-ALU issue.

@@ -1444,7 +1444,14 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     const int64_t alone = static_cast<int64_t>((H + (big_alone ? 255 : 127)) / (big_alone ? 256 : 128)) *
                           ((I + (big_alone ? 255 : 127)) / (big_alone ? 256 : 128)) * G;
     const int64_t blocks_alone = static_cast<int64_t>(device_cu_count()) * (big_alone ? 1 : 2);
-    if (rows > 256 * static_cast<int64_t>(G) && big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone)) {
+    // Gradients with memory in common (two of the weights are one parameter) are written, or added to, one after another.
+    bool overlap = false;
+    for (int i = 0; i < 3; i++) {
+        const WgradSet &a = p.set[i], &b = p.set[(i + 1) % 3];
+        overlap |= om_blocks_overlap(a.C, a.strideC * 2, packed * 2, b.C, b.strideC * 2, packed * 2, G);
+    }
+    const bool no_fewer_rounds = big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone);
+    if (overlap || (rows > 256 * static_cast<int64_t>(G) && no_fewer_rounds)) {
         const int gather_d = dout_rows ? GATHER_WA : GATHER_NONE, gather_x = x_rows ? GATHER_B : GATHER_NONE;
         int code = wgrad_launch(dout, h, dout_rows, gather_d, dout_rows ? src_rows : 0, dw_down, cum_token_counts, rows, G, H, I,
                                 down_stride, stream, accumulate);

@@ -617,6 +617,16 @@ int wgrad_set(F32Wgrad &w, int s, const float *dout, const float *in, const int3
     if (!fits31(w.strideC[s] * G) || !fits31((in_rows ? src_rows : rows) * K) || !fits31(rows * N)) return OM_ERR_SHAPE;
     return OM_OK;
 }
+// Whether the gradients of two sets have memory in common (their weights are one parameter): they are then written, or added
+// to, in launches one after another.
+bool wgrad_sets_overlap(const F32Wgrad &w) {
+    for (int a = 0; a < w.sets; a++)
+        for (int b = a + 1; b < w.sets; b++)
+            if (om_blocks_overlap(w.C[a], w.strideC[a] * 4, 4 * static_cast<int64_t>(w.n[a]) * w.k[a], w.C[b], w.strideC[b] * 4,
+                                  4 * static_cast<int64_t>(w.n[b]) * w.k[b], w.n_experts))
+                return true;
+    return false;
+}
 int64_t wgrad_blocks(const F32Wgrad &w, int tile_rows) {
     int64_t blocks = 0;
     for (int s = 0; s < w.sets; s++) blocks += tiles_of(w.n[s], tile_rows) * tiles_of(w.k[s], TN) * w.n_experts;
@@ -635,6 +645,14 @@ int wgrad_f32_launch(int n_sets, const float *const *output_grad, const float *i
         if (code != OM_OK) return code;
     }
     w.cum = cum_token_counts; w.n_experts = G; w.sets = n_sets; w.accumulate = accumulate;
+    if (wgrad_sets_overlap(w)) {
+        for (int s = 0; s < n_sets; s++) {
+            const int code = wgrad_f32_launch(1, output_grad + s, input, input_rows, src_rows, weight_grad + s, cum_token_counts, rows, G,
+                                              N, K, w_stride + s, stream, (accumulate >> s) & 1);
+            if (code != OM_OK) return code;
+        }
+        return OM_OK;
+    }
     const bool high = two_high(wgrad_blocks(w, 64), wgrad_blocks(w, 32));
     const int64_t blocks = wgrad_blocks(w, high ? 64 : 32);
     if (blocks > 0x7fffffffLL) return OM_ERR_SHAPE;
@@ -691,6 +709,15 @@ int backward_f32_launch(const float *dy, const float *h, const float *dg, const 
     if (code == OM_OK) code = wgrad_set(w, 2, du, x, x_rows, src_rows, dw_up, dw_up_stride, rows, G, I, H);
     if (code != OM_OK) return code;
     w.cum = cum_token_counts; w.n_experts = G; w.sets = 3; w.accumulate = accumulate ? 7 : 0;
+    if (wgrad_sets_overlap(w)) {
+        const float *dout[2] = {dg, du};
+        float *dw[2] = {dw_gate, dw_up};
+        const int64_t strides[2] = {dw_gate_stride, dw_up_stride};
+        if (rows > 0) code = rows_launch<F_STRIDED, E_STORE>(p, rows, stream);
+        if (code == OM_OK) code = wgrad_f32_launch(1, &dy, h, nullptr, 0, &dw_down, cum_token_counts, rows, G, H, I, &dw_down_stride, stream, accumulate);
+        if (code == OM_OK) code = wgrad_f32_launch(2, dout, x, x_rows, src_rows, dw, cum_token_counts, rows, G, I, H, strides, stream, accumulate ? 3 : 0);
+        return code;
+    }
     const int n_tiles = rows > 0 ? static_cast<int>(tiles_of(p.n_cols, TN)) : 1;
     auto row_blocks = [&](int tile_rows) { return rows > 0 ? rows_blocks(p, rows, TN, tile_rows) : 0; };
     // 64-row tiles unless the input gradient's few long ones would be the last to end: the tiny layer with 64 rows an expert

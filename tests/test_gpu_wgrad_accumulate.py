@@ -160,6 +160,83 @@ def test_accumulate_f32(cuda):
     assert torch.equal(acc, old + fresh)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tied", [(0, 0, 1), (0, 1, 0), (0, 1, 1), (0, 0, 0)])     # gate, up, down: which parameter
+@pytest.mark.parametrize("G,rows,I", [(8, 700, 256), (3, 3000, 512), (1, 129, 200)])
+def test_weights_that_are_one_parameter(cuda, G, rows, I, tied, dtype):
+    """Projections that share a parameter add into one live gradient: the sum of the gradients that separate parameters get,
+    in the order down, gate, up; bit for bit."""
+    from optimus.models.common.moe import MergedMLPFunction
+    g = torch.Generator().manual_seed(rows + sum(tied))
+    H = I if tied[2] in tied[:2] else I + 56
+    rnd = lambda *s, f=1.0: (torch.randn(*s, generator=g) * f).to(dtype).to(cuda)
+    x, dy, cum = rnd(rows, H), rnd(rows, H), _counts("ragged", G, rows).to(cuda)
+    shapes = [(G, I, H), (G, I, H), (G, H, I)]
+    values = {t: rnd(*shapes[tied.index(t)], f=0.05) for t in sorted(set(tied))}
+    old = {t: rnd(*values[t].shape) for t in values}
+
+    def run(weights):
+        xd = x.clone().requires_grad_(True)
+        MergedMLPFunction.apply(xd, *weights, cum).backward(dy)
+        torch.cuda.synchronize()
+        return xd.grad
+
+    def live(value, grad):                   # a parameter whose gradient lies in a larger buffer
+        p = torch.nn.Parameter(value.clone())
+        flat = torch.full((grad.numel() + 64,), 7.0, dtype=dtype, device=cuda)
+        p.grad = flat[:grad.numel()].view_as(grad)
+        p.grad.copy_(grad)
+        return p
+
+    separate = [torch.nn.Parameter(values[t].clone()) for t in tied]
+    dx = run(separate)
+    for _ in range(3):
+        one = {t: live(values[t], old[t]) for t in values}
+        buffers = {t: one[t].grad.data_ptr() for t in one}
+        assert torch.equal(run([one[t] for t in tied]), dx)
+        for t in values:
+            want = old[t].clone()
+            for i in (2, 0, 1):
+                if tied[i] == t:
+                    want += separate[i].grad
+            assert one[t].grad.data_ptr() == buffers[t] and (bits(one[t].grad) == bits(want)).all(), t
+
+
+# gate, up and down gradients of each expert between one another in one buffer, and the same with gate and up in one place
+@pytest.mark.parametrize("pitches,offsets", [((3, 3, 3), (0, 1, 2)), ((3, 3, 3), (0, 0, 2)), ((2, 2, 1), (0, 1, 12)), ((2, 4, 1), (0, 0, 24))])
+def test_interleaved_gradients(cuda, pitches, offsets):
+    """bf16 and float32 entry points on gradients at multiples of I * H in one buffer, against one product at a time."""
+    from optimus import _native as n
+    G, rows, I, H = 6, 500, 128, 192
+    for dtype in (torch.bfloat16, torch.float32):
+        g = torch.Generator().manual_seed(sum(pitches))
+        rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(cuda)
+        dout, x, h, dg, du, wg, wu = rnd(rows, H), rnd(rows, H), rnd(rows, I), rnd(rows, I), rnd(rows, I), rnd(G, I, H), rnd(G, I, H)
+        cum, P, M, dx, f = _counts("ragged", G, rows).to(cuda), n.ptr, I * H, torch.empty_like(x), "_f32" if dtype == torch.float32 else ""
+        got = rnd(32 * M)
+        want = got.clone()
+        at = lambda t: [P(t[o * M:]) for o in offsets]
+        if f:
+            _call("om_grouped_gemm_wgrad_merged_dgrad_f32_accumulate", P(dout), P(h), P(dg), P(du), P(x), None, 0, P(wg), P(wu), P(dx),
+                  at(got)[2], at(got)[0], at(got)[1], P(cum), rows, G, I, H, 0, 0, pitches[2] * M, pitches[0] * M, pitches[1] * M)
+        else:
+            _call("om_grouped_gemm_wgrad_merged_accumulate", P(dout), None, P(h), P(dg), P(du), P(x), None, 0, at(got)[2], at(got)[0],
+                  at(got)[1], P(cum), rows, G, I, H, pitches[2] * M, pitches[0] * M, pitches[1] * M)
+        for i, a, b, N, K in ((2, dout, h, H, I), (0, dg, x, I, H), (1, du, x, I, H)):
+            _call(f"om_grouped_gemm_wgrad{f}_accumulate", P(a), P(b), at(want)[i], P(cum), rows, G, N, K, pitches[i] * M)
+        torch.cuda.synchronize()
+        assert (bits(got) == bits(want)).all()
+        if f:
+            two = want.clone()
+            got = want.clone()
+            _call("om_merged_mlp_gate_up_wgrad_f32", P(dg), P(du), P(x), None, 0, at(got)[0], at(got)[1], P(cum), rows, G, I, H,
+                  pitches[0] * M, pitches[1] * M, 3)
+            for i, a in ((0, dg), (1, du)):
+                _call("om_grouped_gemm_wgrad_f32_accumulate", P(a), P(x), at(two)[i], P(cum), rows, G, I, H, pitches[i] * M)
+            torch.cuda.synchronize()
+            assert (bits(got) == bits(two)).all()
+
+
 def _olmoe_block(cuda, merged, fast=True, dtype=torch.bfloat16, seed=3):
     from optimus.mapper import ParallelDpPpEpTpMapper
     from optimus.models.common.moe import FastOlmoeParallelSparseMoeBlock
