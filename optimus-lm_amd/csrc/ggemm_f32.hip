@@ -102,7 +102,7 @@ template <int COLS, int AKIND, int KIND> __device__ __forceinline__ void dma_slo
 
 // This lane's source of one operand, stepped through the contraction.  Steps 0 .. steps - 1 are `stride` bytes apart; with
 // a second phase the next `steps` follow at `second` bytes from the first ones.  A phase's last step may hold fewer than KS
-// indices: `back` bytes less there re-read valid data (A is zeroed where it does).
+// indices: `back` bytes less there re-read valid data (zeroed in LDS).
 struct Source {
     const char *at;
     int64_t stride, jump;       // jump: from a phase's last step to the next one's first
@@ -112,11 +112,12 @@ struct Source {
 };
 
 // The main loop.  load_a() / load_b(i): this lane's addresses of the step that is loaded next; advance(): to the one after
-// it; tail_of(t): does step t hold fewer than KS indices; a_past: does the lane's slot of A then lie past them (the slot then holds other data, and B finite data: zeros make the products vanish).
+// it; tail_of(t): does step t hold fewer than KS indices; a_past, b_past: do the lane's slots then lie past them.  Those hold
+// other data and are zeroed, of both operands: zeros of one alone would turn an infinity of the other into a NaN.
 // acc: this wavefront's 32x32 block (columns 32 * (wave & 1), rows 32 * the next bit with MW 2) over its half of every step.
 template <int MW, int AKIND, int BKIND, typename FA, typename FB, typename FN, typename FT>
 __device__ __forceinline__ void multiply(char *lds, int n_steps, FA &&load_a, FB &&load_b, FN &&advance, FT &&tail_of, bool a_past,
-                                         f32x16 &acc) {
+                                         const bool (&b_past)[Tile<MW>::B_LOADS], f32x16 &acc) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     constexpr int SLOT = Tile<MW>::SLOT, A_BYTES = Tile<MW>::A_BYTES, B_LOADS = Tile<MW>::B_LOADS, LOADS = 1 + B_LOADS;
     constexpr int S = KS / 16;                           // fragments of 8 indices per wavefront and step
@@ -136,7 +137,13 @@ __device__ __forceinline__ void multiply(char *lds, int n_steps, FA &&load_a, FB
         advance();
     };
     auto zero = [&](int t, auto slot) {
-        if (tail_of(t) && a_past) *reinterpret_cast<f4 *>(lds + decltype(slot)::value * SLOT + wave * 1024 + lane * 16) = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (!tail_of(t)) return;
+        char *own = lds + decltype(slot)::value * SLOT + lane * 16;
+        const f4 zeros = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (a_past) *reinterpret_cast<f4 *>(own + wave * 1024) = zeros;
+#pragma unroll
+        for (int i = 0; i < B_LOADS; i++)
+            if (b_past[i]) *reinterpret_cast<f4 *>(own + A_BYTES + (wave * B_LOADS + i) * 1024) = zeros;
     };
     // fragment addresses; element j of fragment s goes to MFMA 4 * s + j
     int a_frag[S], b_frag[S];
@@ -281,6 +288,7 @@ __device__ __forceinline__ void rows_tile(const F32Params &p, char *lds, int row
     const int left_in_tail = p.kc - (steps - 1) * KS;    // indices in a phase's last step
     constexpr int B_LOADS = Tile<MW>::B_LOADS;
     Source a, b[B_LOADS];
+    bool b_past[B_LOADS];
     const float *B0 = p.B[0] + expert * p.strideB[0], *B1 = p.phases > 1 || EPI == E_SWIGLU ? p.B[1] + expert * p.strideB[1] : B0;
     int a_row, a_chunk;
     dma_slot<Tile<MW>::ROWS, F_CONTIG, F_CONTIG>(wave, lane, a_row, a_chunk);
@@ -301,9 +309,11 @@ __device__ __forceinline__ void rows_tile(const F32Params &p, char *lds, int row
             const int n = min(n0 + (EPI == E_SWIGLU ? r & 31 : r), p.n_cols - 1);
             b[i].at = reinterpret_cast<const char *>((EPI == E_SWIGLU && r >= 32 ? B1 : B0) + static_cast<int64_t>(n) * p.ldb) + ch * 16;
             b[i].back = max(ch * 4 + 4 - left_in_tail, 0) * 4;
+            b_past[i] = ch * 4 >= left_in_tail;
         } else {
             b[i].at = reinterpret_cast<const char *>(B0 + static_cast<int64_t>(r) * p.ldb + min(n0 + ch * 4, p.n_cols - 4));
             b[i].back = static_cast<uint32_t>(max(r - (left_in_tail - 1), 0)) * static_cast<uint32_t>(p.ldb) * 4u;
+            b_past[i] = r >= left_in_tail;
         }
     }
     int at = 0;                                          // the step of the phase that is loaded next
@@ -319,7 +329,7 @@ __device__ __forceinline__ void rows_tile(const F32Params &p, char *lds, int row
     };
     auto tail_of = [&](int t) { return tail >= 0 && (t == tail || t - steps == tail); };
     f32x16 acc;
-    multiply<MW, F_CONTIG, BKIND>(lds, steps * p.phases, load_a, load_b, advance, tail_of, a_chunk * 4 >= left_in_tail, acc);
+    multiply<MW, F_CONTIG, BKIND>(lds, steps * p.phases, load_a, load_b, advance, tail_of, a_chunk * 4 >= left_in_tail, b_past, acc);
     finish<MW>(lds, acc);
     // 8 threads to a row: 8 neighbouring columns each (E_SWIGLU: 4 of gate and the same 4 of up)
     const int part = threadIdx.x & 7, row = threadIdx.x >> 3, n = n0 + part * (EPI == E_SWIGLU ? 4 : 8);
@@ -368,12 +378,13 @@ __device__ __forceinline__ void wgrad_tile(const F32Wgrad &p, char *lds, int *id
         for (int i = threadIdx.x; i < min(len, IDX_CACHE); i += Tile<MW>::THREADS) idx_cache[i] = b_rows[r0 + i];
         __syncthreads();
     }
-    // columns past the extent re-read its last 4; rows past the segment its last row (A is zeroed there)
+    // columns past the extent re-read its last 4; rows past the segment its last row (zeroed in LDS)
     constexpr int B_LOADS = Tile<MW>::B_LOADS;
     const int steps = (len + KS - 1) / KS, tail = len % KS ? steps - 1 : -1;
     const int left_in_tail = len - (steps - 1) * KS;     // rows in the last step
     Source a, b[B_LOADS];
     int a_c, b_c[B_LOADS];
+    bool b_past[B_LOADS];
     auto set = [&](Source &s, const float *base, int ld, int c, int col) {
         s.at = reinterpret_cast<const char *>(base + static_cast<int64_t>(c) * ld + min(col, ld - 4));
         s.stride = s.jump = static_cast<int64_t>(KS) * ld * 4;
@@ -385,6 +396,7 @@ __device__ __forceinline__ void wgrad_tile(const F32Wgrad &p, char *lds, int *id
 #pragma unroll
     for (int i = 0; i < B_LOADS; i++) {
         dma_slot<TN, F_STRIDED, F_STRIDED>(wave * B_LOADS + i, lane, b_c[i], chunk);
+        b_past[i] = b_c[i] >= left_in_tail;
         set(b[i], p.B[set_id] + (b_rows ? 0 : static_cast<int64_t>(r0) * n_cols), n_cols, b_rows ? 0 : b_c[i], k0 + chunk * 4);
     }
     int at = 0;
@@ -410,7 +422,7 @@ __device__ __forceinline__ void wgrad_tile(const F32Wgrad &p, char *lds, int *id
     };
     auto tail_of = [&](int t) { return t == tail; };
     f32x16 acc;
-    multiply<MW, F_STRIDED, F_STRIDED>(lds, steps, load_a, load_b, advance, tail_of, a_c >= left_in_tail, acc);
+    multiply<MW, F_STRIDED, F_STRIDED>(lds, steps, load_a, load_b, advance, tail_of, a_c >= left_in_tail, b_past, acc);
     finish<MW>(lds, acc);
     const bool add = (p.accumulate >> set_id) & 1;
     const int row = threadIdx.x >> 3, k = k0 + (threadIdx.x & 7) * 8;

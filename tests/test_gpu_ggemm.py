@@ -247,6 +247,62 @@ def test_grouped_gemm_float32(cuda, kind, G, rows, N, K):
         assert float(wd.grad[empty.to(cuda)].abs().max()) == 0.0
 
 
+# contractions of which the last step (32) is partial, of both operands; one and two row-tile heights
+@pytest.mark.parametrize("counts,I,H", [([40, 7, 0, 33], 72, 40), ([700, 129], 264, 328), ([1, 2, 3, 95], 8, 104)])
+def test_float32_infinities_stay_infinities(cuda, counts, I, H):
+    """An infinity in the last contraction index of either operand gives what float64 products give: it meets no zero that
+    stands for an index past the end."""
+    from optimus import _native as n
+    g = torch.Generator().manual_seed(I)
+    G, rows = len(counts), sum(counts)
+    cum = torch.zeros(G + 1, dtype=torch.int32)
+    cum[1:] = torch.cumsum(torch.tensor(counts), 0)
+    inf, P, L, d, st = float("inf"), n.ptr, n.lib(), cum.to(cuda), n.stream()
+    last = (cum[1:] - 1)[torch.tensor(counts) > 0].long()     # each expert's last row
+    mats = lambda r, c: torch.rand(r, c, generator=g) + 0.5   # (no zero beside an infinity)
+    x, dy, h, dg, du = mats(rows, H), mats(rows, H), mats(rows, I), mats(rows, I), mats(rows, I)
+    wg, wu, wd = (torch.rand(G, *s, generator=g) + 0.5 for s in ((I, H), (I, H), (H, I)))
+    wg[:, I // 2, H - 1], wu[:, I - 1, H - 1], wd[:, H - 1, 0] = inf, -inf, inf
+    same = lambda got, want, name: (torch.testing.assert_close(got.double().cpu(), want, rtol=1e-5, atol=0.0, equal_nan=True, msg=name))
+
+    def run(name, *a):
+        n.check(getattr(L, name)(*a, st), name)
+        torch.cuda.synchronize()
+    dev = lambda *ts: [t.to(cuda) for t in ts]
+    new = lambda *s: torch.full(s, 7.0, device=cuda)
+    X, DY, HH, DG, DU, WG, WU, WD = dev(x, dy, h, dg, du, wg, wu, wd)
+    per_expert = lambda f: torch.cat([f(slice(int(cum[e]), int(cum[e + 1])), e) for e in range(G)])
+    up = lambda t: t.double()
+    # the weights' infinities: forward, input gradient of one matrix, gate and up, both of them in one accumulation
+    y = new(rows, I)
+    run("om_grouped_gemm_fwd_f32", P(X), P(WG), P(y), P(d), rows, G, I, H, 0)
+    same(y, per_expert(lambda s, e: up(x[s]) @ up(wg[e]).t()), "fwd")
+    dx = new(rows, I)
+    run("om_grouped_gemm_dgrad_f32", P(DY), P(WD), P(dx), P(d), rows, G, H, I, 0)
+    same(dx, per_expert(lambda s, e: up(dy[s]) @ up(wd[e])), "dgrad")
+    gq, uq, hq = new(rows, I), new(rows, I), new(rows, I)
+    run("om_merged_mlp_gate_up_fwd_f32", P(X), None, 0, P(WG), P(WU), P(gq), P(uq), P(hq), P(d), rows, G, I, H, 0, 0)
+    same(gq, per_expert(lambda s, e: up(x[s]) @ up(wg[e]).t()), "gate")
+    same(uq, per_expert(lambda s, e: up(x[s]) @ up(wu[e]).t()), "up")
+    dx = new(rows, H)
+    run("om_merged_mlp_gate_up_dgrad_f32", P(DG), P(DU), P(WG), P(WU), P(dx), P(d), rows, G, I, H, 0, 0)
+    same(dx, per_expert(lambda s, e: up(dg[s]) @ up(wg[e]) + up(du[s]) @ up(wu[e])), "dx")
+    # the activations' infinities: weight gradients, alone and in the backward's one launch
+    x[last, 3], h[last, I - 1], dg[last, 1] = inf, -inf, -inf
+    X, HH, DG = dev(x, h, dg)
+    dw = lambda a, b: torch.stack([up(a[s]).t() @ up(b[s]) for s in (slice(int(cum[e]), int(cum[e + 1])) for e in range(G))])
+    out = new(G, H, I)
+    run("om_grouped_gemm_wgrad_f32", P(DY), P(HH), P(out), P(d), rows, G, H, I, 0)
+    same(out, dw(dy, h), "wgrad")
+    index = torch.arange(rows, dtype=torch.int32, device=cuda)
+    for ix in (None, P(index)):
+        down, gate, upw = new(G, H, I), new(G, I, H), new(G, I, H)
+        run("om_grouped_gemm_wgrad_merged_dgrad_f32", P(DY), P(HH), P(DG), P(DU), P(X), ix, rows, P(WG), P(WU), P(dx), P(down), P(gate),
+            P(upw), P(d), rows, G, I, H, 0, 0, 0, 0, 0)
+        for name, got, want in (("down", down, dw(dy, h)), ("gate", gate, dw(dg, x)), ("up", upw, dw(du, x))):
+            same(got, want, name)
+
+
 # row tiles of 32 and of 64, contractions of 1 to 5 steps of 32 and partial ones, more rows in an expert than the kernel keeps
 # indices of in LDS, no rows at all
 @pytest.mark.parametrize("counts,I,H", [([31, 32, 33, 0, 1, 63, 64, 65], 40, 72), ([96, 97, 128, 160, 159, 5], 160, 96), ([1100, 7, 300], 64, 32),
