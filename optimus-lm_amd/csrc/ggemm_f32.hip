@@ -645,11 +645,15 @@ int64_t wgrad_blocks(const F32Wgrad &w, int tile_rows) {
     return blocks;
 }
 
+// Weight gradients over the same rows times experts that are accepted: what these entry points refuse, not a bound of the
+// launch (`blocks` is that).  The whole backward takes the experts that its gate and up gradients take.
+constexpr int64_t MAX_GRADIENTS = 65535;
+
 // n_sets 1 or 2: dW[s] (+)= dout[s]^T in, over the same rows of `input` (through input_rows when given)
 int wgrad_f32_launch(int n_sets, const float *const *output_grad, const float *input, const int32_t *input_rows,
                      int64_t src_rows, float *const *weight_grad, const int32_t *cum_token_counts, int64_t rows, int G,
                      int N, int K, const int64_t *w_stride, void *stream, int accumulate) {
-    if (rows < 0 || G < 1 || n_sets * static_cast<int64_t>(G) > 65535 || !mult8(N) || !mult8(K)) return OM_ERR_SHAPE;
+    if (rows < 0 || G < 1 || n_sets * static_cast<int64_t>(G) > MAX_GRADIENTS || !mult8(N) || !mult8(K)) return OM_ERR_SHAPE;
     if (!cum_token_counts) return OM_ERR_NULL;
     F32Wgrad w = {};
     for (int s = 0; s < n_sets; s++) {
@@ -710,7 +714,7 @@ int backward_f32_launch(const float *dy, const float *h, const float *dg, const 
                         float *dw_up, const int32_t *cum_token_counts, int64_t rows, int G, int I, int H, int64_t gate_stride,
                         int64_t up_stride, int64_t dw_down_stride, int64_t dw_gate_stride, int64_t dw_up_stride, bool accumulate,
                         void *stream) {
-    if (rows < 0 || G < 1 || 3 * static_cast<int64_t>(G) > 65535 || !mult8(I) || !mult8(H)) return OM_ERR_SHAPE;
+    if (rows < 0 || G < 1 || 2 * static_cast<int64_t>(G) > MAX_GRADIENTS || !mult8(I) || !mult8(H)) return OM_ERR_SHAPE;
     if (x_rows && rows > 0 && src_rows < 1) return OM_ERR_SHAPE;
     if (!cum_token_counts) return OM_ERR_NULL;
     F32Params p = {};

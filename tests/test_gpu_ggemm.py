@@ -247,6 +247,35 @@ def test_grouped_gemm_float32(cuda, kind, G, rows, N, K):
         assert float(wd.grad[empty.to(cuda)].abs().max()) == 0.0
 
 
+def test_float32_backward_of_many_experts(cuda):
+    """30000 experts, a few of them with rows: bounded by the launch's blocks alone."""
+    from optimus import _native as n
+    G, rows, I, H = 30000, 64, 8, 16
+    g = torch.Generator().manual_seed(1)
+    owner = torch.sort(torch.randint(0, G, (rows,), generator=g)).values
+    cum = torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(owner, minlength=G).cumsum(0)]).to(torch.int32).to(cuda)
+    x, dy, wg, wu, wd = (torch.randn(*s, generator=g).to(cuda) for s in ((rows, H), (rows, H), (G, I, H), (G, I, H), (G, H, I)))
+    ws = [torch.nn.Parameter(w) for w in (wg, wu, wd)]
+    from optimus.models.common.moe import MergedMLPFunction
+    xd = x.clone().requires_grad_(True)
+    MergedMLPFunction.apply(xd, *ws, cum).backward(dy)
+    D, ref = (lambda t: t.detach().double()), [torch.zeros_like(w, dtype=torch.float64) for w in ws]
+    for r in range(rows):
+        e = int(owner[r])
+        a, b = D(wg[e]) @ D(x[r]), D(wu[e]) @ D(x[r])
+        s = torch.sigmoid(a)
+        dh = D(wd[e]).t() @ D(dy[r])
+        da, db = dh * b * s * (1 + a * (1 - s)), dh * a * s
+        ref[0][e] += torch.outer(da, D(x[r]))
+        ref[1][e] += torch.outer(db, D(x[r]))
+        ref[2][e] += torch.outer(D(dy[r]), a * s * b)
+        want = D(wg[e]).t() @ da + D(wu[e]).t() @ db
+        # float32 sums of 8 to 16 products behind three of their own: 2e-6 of the largest, as elsewhere, times their number
+        assert (D(xd.grad[r]) - want).abs().max() <= 1e-5 * (1 + want.abs().max())
+    for w, want in zip(ws, ref):
+        assert (D(w.grad) - want).abs().max() <= 1e-5 * (1 + want.abs().max())
+
+
 # contractions of which the last step (32) is partial, of both operands; one and two row-tile heights
 @pytest.mark.parametrize("counts,I,H", [([40, 7, 0, 33], 72, 40), ([700, 129], 264, 328), ([1, 2, 3, 95], 8, 104)])
 def test_float32_infinities_stay_infinities(cuda, counts, I, H):
