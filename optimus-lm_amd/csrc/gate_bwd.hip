@@ -159,13 +159,14 @@ __global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restr
 // The same for more than 128 experts, a multiple of 4 of them: 256 rows and 256 columns of dW per block of eight wavefronts (64 x
 // 128 each), so that the fp32 dlogits are read once per 256 columns, in steps of 32 tokens.  x comes by direct loads two steps
 // ahead through a ring of three, the dlogits through registers, two steps ahead too, and a pair of buffers.  Every step loads,
-// past the last one that one again, so that the number of loads in flight is known.
+// past the last one that one again, so that the number of loads in flight is known.  The dlogits' loads are among those that the
+// wait counts: `dlogits` is not __restrict__, so that the compiler may not move them over the assembly's memory clobbers.
 // us with the launch that adds the ranges, x out of the caches, before (128 columns a block, both operands through registers
 // one stage ahead) -> now, 256 experts: hidden 7168, 64 tokens 19.3 -> 16.4, 2048 tokens 57 -> 41, 8192 tokens 115 -> 72; hidden
 // 1624, 8176 tokens 60 -> 42.  160 experts, hidden 5120, 4096 tokens 56 -> 37.
 constexpr int WW_HT = 256, WW_TC = 32;
-__global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__restrict__ x, const float *__restrict__ dlogits, int64_t T,
-                                                              int H, int N, int64_t tokens_per_split, float *__restrict__ partial) {
+__global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__restrict__ x, const float *dlogits, int64_t T, int H,
+                                                              int N, int64_t tokens_per_split, float *__restrict__ partial) {
     constexpr int SLOTS = 3, XS = WW_TC * WW_HT * 2, DS = WW_TC * 256 * 2, XL = XS / 1024 / 8, DL = WW_TC * 256 / 4 / 512;
     constexpr int TM = 2, TN = 4;
     __shared__ __attribute__((aligned(1024))) char lds[SLOTS * XS + 2 * DS];
@@ -459,7 +460,8 @@ __global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restr
 // The same for more than 64 experts, a multiple of 16 of them: with many experts a block's dlogits and weights are more
 // than its results.  A block of eight wavefronts keeps the dlogits of its 256 tokens in registers (bf16, MFMA layout) and goes
 // through a range of 64-column slices of the weight, which come by direct loads two slices ahead through a ring of three;
-// `base` comes one slice ahead.  What is left to bound it is `base` and dx.
+// `base` comes one slice ahead (not __restrict__: its loads are counted by a wait and must stay between the assembly
+// statements around them).  What is left to bound it is `base` and dx.
 // us, `base` and weights out of the caches, 256 experts, before (128 tokens x 128 columns a block, dlogits in fp32 once per 128
 // columns) -> now: hidden 7168, 64 tokens 18.9 -> 11.3, 512 tokens 19.7 -> 16.4, 8192 tokens 113.9 -> 71.0 (4.0 TB/s of base,
 // dx and dlogits); hidden 1624, 8176 tokens 45.3 -> 36.6; 128 experts, hidden 4096, 4096 tokens 29.3 -> 24.3.
