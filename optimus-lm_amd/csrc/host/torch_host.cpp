@@ -926,8 +926,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
     require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
     // Few tokens: one CU would take in all of the gate weight, the projection split over the chip and a launch behind it
-    // are sooner (om_router_gate_split_softmax_topk, which has the figures).
-    if (one_pass && T <= 512 && N <= 64 && H >= 1024 && H % 512 == 0) one_pass = false;
+    // are sooner; with many selections it depends (om_router_gate_split_softmax_topk, which has the figures and decides).
+    if (one_pass && N <= 64 && H % 512 == 0 && (top_k > 16 || (T <= 512 && H >= 1024))) one_pass = false;
     Tensor logits, weights, experts;
     {
         at::AutoDispatchBelowADInplaceOrView below;

@@ -921,7 +921,14 @@ extern "C" int om_router_gate_split_softmax_topk(const void *x, const void *gate
     // 173.7 -> 171.8; 512 tokens (with the backward) 700 -> 701; 4096 tokens 520.7 -> 524.2.  In the caches, the router alone:
     // 1 token 7.7 -> 7.8, 512 tokens 8.1 -> 12.2, 4096 tokens 10.7 -> 19.0, and at hidden 7168 15.5 -> 11.5, 16.2 -> 18.5 and
     // 25.8 -> 26.7.  Below hidden 1024 the weight is small: 512, 32 experts, 512 tokens 4.4 -> 9.2.
-    if (gate_slices_fit(H, N) && (T > 512 || H < 1024)) {
+    // More than 16 selections take a wavefront per token, of a block's 32 tokens two or four to each of its wavefronts: one launch
+    // only where its blocks (256 at a time) fill their last round by three quarters and there are 16 wavefronts, or for a few
+    // tokens of a small weight.  One -> two, 64 experts, hidden 2048, 32 selections: 600 tokens 24.3 -> 16.2, 4500 27.2 -> 31.2, 8192 28.8 ->
+    // 37.9, 12000 53.9 -> 51.4, 16384 56.5 -> 66.7; 60 selections, hidden 4096: 6000 49.1 -> 46.3, 8192 52.2 -> 57.0; 32 experts, 24
+    // selections, hidden 2048: 600 24.8 -> 13.0, 8192 28.0 -> 27.4, 12000 53.2 -> 38.9; hidden 512, 40 of 62: 4 tokens 10.1 -> 12.4, 20 of
+    // 40: 52 tokens 15.4 -> 9.5.
+    const bool one_launch = K <= 16 ? T > 512 || H < 1024 : H < 1024 && T <= 16 ? true : N > 32 && (T - 1) % 8192 >= 6144;
+    if (gate_slices_fit(H, N) && one_launch) {
 #define OM_GS(TL, TW) \
     launch_gate_slices<TL, TW, true>(x, gate_weight, T, H, N, K, norm_topk_prob, logits_out, weights_out, experts_out, st)
         if (logits_dtype == OM_F32) return weights_dtype == OM_F32 ? OM_GS(float, float) : OM_GS(float, uint16_t);

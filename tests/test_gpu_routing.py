@@ -497,6 +497,27 @@ def test_one_launch_gate_router(cuda, T, H, N, K, renorm, one_pass, bf16_logits)
     assert bool(((logits[ok].double() - ref).abs() <= bound + 1e-30).all())
 
 
+@pytest.mark.parametrize("T,H,N,K,one", [(513, 1024, 64, 16, True), (513, 1024, 64, 17, False), (16, 512, 40, 20, True), (17, 512, 40, 20, False),
+                                         (6144, 512, 33, 33, False), (6145, 512, 33, 33, True), (8192, 1024, 64, 17, True),
+                                         (8193, 512, 64, 40, False), (8192, 512, 32, 17, False)])
+def test_router_of_many_selections(cuda, T, H, N, K, one):
+    """Where more than 16 experts are selected the two launches stay where they are the faster ones (seen by the workspace, which
+    one launch leaves alone); the same bits either way."""
+    from optimus import _native as n
+    x, w = (t.to(cuda) for t in _gate_inputs(T, H, N, seed=T + K))
+    size = n.lib().om_router_gate_route_workspace_bytes(T, H, N)
+    ws = torch.full((size,), 77, dtype=torch.uint8, device=cuda)
+    new = lambda *s, dt=torch.float32: torch.empty(*s, dtype=dt, device=cuda)
+    a, b = ((new(T, N), new(T, K), new(T, K, dt=torch.int64)) for _ in range(2))
+    P = n.ptr
+    n.check(n.lib().om_router_gate_split_softmax_topk(P(x), P(w), T, H, N, K, 1, P(a[0]), n.OM_F32, P(a[1]), n.OM_F32, P(a[2]), P(ws), size,
+                                                      n.stream()), "split")
+    n.check(n.lib().om_router_gate_softmax_topk(P(x), P(w), T, H, N, K, 1, P(b[0]), P(b[1]), n.OM_F32, P(b[2]), n.stream()), "one pass")
+    for u, v in zip(a, b):
+        assert torch.equal(u, v)
+    assert bool((ws == 77).all()) == one
+
+
 @pytest.mark.parametrize("T,H,N", [(1, 8, 65), (127, 72, 100), (129, 64, 128), (257, 128, 129), (256, 1624, 256), (640, 200, 160), (300, 7168, 80),
                                    (33000, 136, 256), (700, 264, 132), (1000, 520, 250)])
 @pytest.mark.parametrize("base", [False, True])
