@@ -242,13 +242,29 @@ inline bool gate_split_shape_ok(int64_t T, int H, int N) {
     return T >= 0 && T <= 0x7fffffffLL && N >= 1 && N <= 256 && H >= 8 && H % 8 == 0;
 }
 
-// Slices of H: a block per CU, and no more (the fp32 partials cost 8 B per logit and slice).  At most 32: 64 tokens, hidden 7168, 256 experts 22 us with 16 slices, 19 with 28.
-// A slice is a whole number of 64-wide steps, the last one may be shorter and its last step partial.
-inline int gate_split_count(int64_t T, int H) {
+// Slices of H: a block per CU, and no more (the fp32 partials cost 8 B per logit and slice).  At most 32: 64 tokens, hidden 7168,
+// 256 experts 22 us with 16 slices, 19 with 28.  A slice is a whole number of 64-wide steps, the last one may be shorter and
+// its last step partial.
+// Up to 64 experts several blocks share a CU.  From 33 blocks of tokens on (below, more slices cost what they give) the
+// count with the least time by this account is taken: a step of the busiest CU's k blocks takes 730 ns with one of them, 900 k -
+// 700 with more, a slice's partials 3 ps per logit (fitted to 270 shapes of 8 to 61 experts, hidden 336 to 6440, 1 to 8 slices
+// each).  us, a block per CU -> now: 8 experts, hidden 4104, 11000 tokens 28.8 -> 19.4, 18000 50.5 -> 28.5; 40 experts,
+// hidden 4928, 6677 tokens 24.4 -> 21.5; 61 experts, hidden 6440, 18000 tokens 89.7 -> 59.1, 22000 133 -> 102; hidden 336, 22000
+// tokens 15.5, one slice in both; at worst 8 experts, hidden 336, 5000 tokens 6.5 -> 7.1.
+inline int gate_split_count(int64_t T, int H, int N) {
     const int64_t token_blocks = std::max<int64_t>((T + GT - 1) / GT, 1);
     const int steps = (H + GK - 1) / GK;
-    const int want = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(32, 256 / token_blocks)));
-    const int each = (steps + want - 1) / want;
+    auto steps_each = [&](int slices) { return (steps + slices - 1) / slices; };
+    int want = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(32, 256 / token_blocks)));
+    if (N <= 64 && token_blocks > 32) {
+        int64_t least = INT64_MAX;
+        for (int s = 1; s <= std::min(8, steps); s++) {
+            const int64_t k = (token_blocks * s + 255) / 256;
+            const int64_t picoseconds = steps_each(s) * 1000 * (k == 1 ? 730 : 900 * k - 700) + s * 3 * T * N;
+            if (picoseconds < least) { least = picoseconds; want = s; }
+        }
+    }
+    const int each = steps_each(want);
     return (steps + each - 1) / each;
 }
 
@@ -257,7 +273,7 @@ inline int gate_split_count(int64_t T, int H) {
 // Behind a routing kernel that adds the slices itself: eight of them where the steps divide (the order of
 // the sums is then that of om_router_gate_softmax_topk, bit for bit), else as above.
 int om_gate_route_splits(int64_t T, int H, int N) {
-    return N <= 64 && H % 512 == 0 ? 8 : gate_split_count(T, H);
+    return N <= 64 && H % 512 == 0 ? 8 : gate_split_count(T, H, N);
 }
 
 void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, int splits, float *ws,
@@ -277,7 +293,7 @@ extern "C" int64_t om_router_gate_route_workspace_bytes(int64_t T, int H, int N)
 
 extern "C" int64_t om_router_gate_logits_split_workspace_bytes(int64_t T, int H, int N) {
     if (!gate_split_shape_ok(T, H, N)) return OM_ERR_SHAPE;
-    return static_cast<int64_t>(gate_split_count(T, H)) * T * N * 4;
+    return static_cast<int64_t>(gate_split_count(T, H, N)) * T * N * 4;
 }
 
 extern "C" int om_router_gate_logits_split(const void *x, const void *gate_weight, int64_t T, int H, int N,
@@ -287,7 +303,7 @@ extern "C" int om_router_gate_logits_split(const void *x, const void *gate_weigh
     if (T == 0) return OM_OK;
     if (!x || !gate_weight || !logits_out || !workspace) return OM_ERR_NULL;
     if (!om_aligned16(x) || !om_aligned16(gate_weight) || !om_aligned16(workspace)) return OM_ERR_ALIGN;
-    const int splits = gate_split_count(T, H);
+    const int splits = gate_split_count(T, H, N);
     const int64_t tn = T * N;
     if (workspace_bytes < splits * tn * 4) return OM_ERR_WORKSPACE;
     hipStream_t st = om_stream(stream);

@@ -518,6 +518,21 @@ def test_router_of_many_selections(cuda, T, H, N, K, one):
     assert bool((ws == 77).all()) == one
 
 
+@pytest.mark.parametrize("T,H,N,slices", [(4096, 1000, 12, 8), (4097, 1000, 12, 6), (6677, 4928, 40, 8), (8193, 1000, 12, 6), (11000, 4104, 8, 5), (18000, 4104, 8, 3), (18000, 336, 61, 1),
+                                          (16513, 2920, 61, 3), (33000, 72, 64, 1)])
+def test_gate_of_many_tokens(cuda, T, H, N, slices):
+    """Up to 64 experts: as many slices of the hidden size as the busiest CU is done with soonest; the logits against float64."""
+    from optimus import _native as n
+    L, P = n.lib(), n.ptr
+    x, w = (t.to(cuda) for t in _gate_inputs(T, H, N, seed=T + N))
+    size = L.om_router_gate_logits_split_workspace_bytes(T, H, N)
+    assert size == slices * T * N * 4
+    ws, logits = torch.empty(size, dtype=torch.uint8, device=cuda), torch.full((T + 1, N), 7.0, device=cuda)
+    n.check(L.om_router_gate_logits_split(P(x), P(w), T, H, N, P(logits), P(ws), size, n.stream()), "logits")
+    bound = (H / 16 + 33) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30   # as in test_gate_of_many_experts
+    assert bool(((logits[:T].double() - x.double() @ w.double().t()).abs() <= bound).all()) and bool((logits[T] == 7.0).all())
+
+
 @pytest.mark.parametrize("T,H,N", [(1, 8, 65), (127, 72, 100), (129, 64, 128), (257, 128, 129), (256, 1624, 256), (640, 200, 160), (300, 7168, 80),
                                    (33000, 136, 256), (700, 264, 132), (1000, 520, 250)])
 @pytest.mark.parametrize("base", [False, True])
