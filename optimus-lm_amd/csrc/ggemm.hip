@@ -1283,8 +1283,14 @@ bool wgrad_big_tile(int n, int k, int64_t matrices) {
     return n % 256 == 0 && k % 256 == 0 && matrices * (n / 256) * (k / 256) * 2 >= device_cu_count();
 }
 
-// XCDs that share an expert's weight gradient: all, where an eighth of its tiles is about a third of a round or more.
-int wgrad_share(bool big, int tiles_e, int n_experts) {
+// XCDs that share an expert's weight gradient: all, where an eighth of its tiles is about a third of a round or more.  With few
+// rows the writing form is stores alone, which whole experts per XCD do better; the accumulating form leaves out the experts
+// without rows, and the rest has to be shared.  The three of 32 experts of 2048/7168 in one launch, us, shared -> not, rows even /
+// as 1 / rank^1.2, writing: 8 rows in all 538 -> 483 / 531 -> 505, 128 rows 540 -> 524 / 531 -> 524, 512 rows 541 -> 523 / 550 -> 583,
+// 2048 rows 625 -> 634 / 632 -> 684; accumulating: 1 row 114 -> 254, 64 rows 913 -> 1043 / 667 -> 768.  64 experts of 1024/2048,
+// writing: 64 rows 161 -> 148 / 159 -> 132, 512 rows 162 -> 158 / 156 -> 161, 2048 rows 166 -> 164 / 177 -> 175.
+int wgrad_share(bool big, int tiles_e, int n_experts, int64_t rows, bool accumulate) {
+    if (!accumulate && rows < 16 * static_cast<int64_t>(n_experts)) return 0;
     return big && tiles_e >= 12 * NUM_XCD && n_experts <= SHARE_MAX_EXPERTS ? NUM_XCD : 0;
 }
 
@@ -1315,7 +1321,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     hipStream_t st = om_stream(stream);
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
-    p.share = wgrad_share(big, p.tiles_e, G);
+    p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
     p.stream = static_cast<int64_t>(G) * N * K >= CACHED_WEIGHTS;
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
@@ -1437,7 +1443,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     // are chosen per tile): 12 experts of 1000x712, 576 tiles a product on 512 blocks, 103 -> 72 us; 8 of 256x512, 64
     // tiles, 38 -> 16.  One of 7168x2048, 224 tiles on 256 blocks and as many rounds either way, 698 -> 774; 64 of
     // 2048x1024 with 2048 rows, 2048 tiles, 1620 -> 1701.  With few rows an expert, where a launch is stores and its ends
-    // weigh more, one launch as well: those 64 experts with 64 rows each on average, a step of 512 tokens 717 -> 696.
+    // weigh more, one launch as well: those 64 experts with 64 rows each on average, a step of 512 tokens 717 -> 696. 
     const int64_t blocks = static_cast<int64_t>(device_cu_count()) * (big ? 1 : 2);
     auto rounds = [](int64_t t, int64_t b) { return (t + b - 1) / b; };
     const bool big_alone = wgrad_big_tile(H, I, G);
@@ -1464,7 +1470,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
         return code;
     }
     p.tiles_e = static_cast<int>(3 * each);
-    p.share = wgrad_share(big, p.tiles_e, G);
+    p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
     p.stream = 3 * packed * G >= CACHED_WEIGHTS;
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
