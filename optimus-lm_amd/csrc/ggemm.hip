@@ -1443,7 +1443,11 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     // are chosen per tile): 12 experts of 1000x712, 576 tiles a product on 512 blocks, 103 -> 72 us; 8 of 256x512, 64
     // tiles, 38 -> 16.  One of 7168x2048, 224 tiles on 256 blocks and as many rounds either way, 698 -> 774; 64 of
     // 2048x1024 with 2048 rows, 2048 tiles, 1620 -> 1701.  With few rows an expert, where a launch is stores and its ends
-    // weigh more, one launch as well: those 64 experts with 64 rows each on average, a step of 512 tokens 717 -> 696. 
+    // weigh more, one launch as well: those 64 experts with 64 rows each on average, a step of 512 tokens 717 -> 696.  But not with
+    // many rounds of 128x128 tiles, beside which the ends weigh little.  One -> three launches, us: 64 experts of 1048x1712, 48 rounds,
+    // writing 64 rows in all 219 -> 204, 2048 rows 251 -> 244, 8192 rows 361 -> 330, accumulating 299 -> 290, 354 -> 357, 440 -> 415; 16 of
+    // 1104x3736, 26 rounds, writing 64 rows 132 -> 118, 2048 203 -> 179, accumulating 193 -> 210, 253 -> 244; 16 of 688x2304, 11 rounds, writing
+    // 50 -> 53, 72 -> 67; 48 of 520x1400, 16 rounds (18 in three), writing 67 -> 69, 70 -> 70, accumulating 95 -> 104, 97 -> 111.
     const int64_t blocks = static_cast<int64_t>(device_cu_count()) * (big ? 1 : 2);
     auto rounds = [](int64_t t, int64_t b) { return (t + b - 1) / b; };
     const bool big_alone = wgrad_big_tile(H, I, G);
@@ -1457,7 +1461,8 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
         overlap |= om_blocks_overlap(a.C, a.strideC * 2, packed * 2, b.C, b.strideC * 2, packed * 2, G);
     }
     const bool no_fewer_rounds = big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone);
-    if (overlap || (rows > 256 * static_cast<int64_t>(G) && no_fewer_rounds)) {
+    const bool many_rounds = !big && rounds(tiles, blocks) > (accumulate ? 32 : 16);
+    if (overlap || (no_fewer_rounds && (many_rounds || rows > 256 * static_cast<int64_t>(G)))) {
         const int gather_d = dout_rows ? GATHER_WA : GATHER_NONE, gather_x = x_rows ? GATHER_B : GATHER_NONE;
         int code = wgrad_launch(dout, h, dout_rows, gather_d, dout_rows ? src_rows : 0, dw_down, cum_token_counts, rows, G, H, I,
                                 down_stride, stream, accumulate);

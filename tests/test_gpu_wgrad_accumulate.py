@@ -76,7 +76,9 @@ def test_accumulate_entry_points_equal_gemm_then_add(cuda, form, kind, G, rows, 
 # block keeps indices of in LDS
 @pytest.mark.parametrize("kind,G,rows,I,H", [("ragged", 8, 4096, 512, 256), ("ragged", 12, 9003, 712, 1000), ("empties", 16, 777, 128, 256),
                                              ("ragged", 64, 4096, 1024, 2048), ("uniform", 22, 11000, 512, 1024), ("onehot", 5, 5000, 256, 512),
-                                             ("uniform", 1, 300, 264, 136), ("ragged", 3, 5, 8, 72), ("uniform", 4, 0, 128, 128)])
+                                             ("uniform", 1, 300, 264, 136), ("ragged", 3, 5, 8, 72), ("uniform", 4, 0, 128, 128),
+                                             # (more than 16 rounds of tiles: three launches that write, one that adds)
+                                             ("ragged", 700, 2000, 136, 136)])
 @pytest.mark.parametrize("indexed", [False, True])
 def test_three_weight_gradients_of_a_merged_mlp(cuda, indexed, kind, G, rows, I, H):
     """One bf16 rounding of a float32 sum over an expert's rows (2^-8 of the value, and the order of the sum); the
