@@ -754,6 +754,39 @@ def test_row_products_of_shared_experts(cuda, kind, G, rows, N, K):
     assert ((h.float() - silu).abs() <= silu.abs() * 2 ** -6 + (g.float().abs() + 1) * (u.float().abs() + 1) * 2 ** -7).all()
 
 
+# four XCDs (16 experts and more) and all eight to an expert, 256x256 and 128x128 tiles, extents that neither divides
+@pytest.mark.parametrize("kind,G,rows,I,H", [("ragged", 16, 6000, 2048, 4096), ("ragged", 5, 3300, 4096, 2048), ("ragged", 16, 1500, 2056, 4104),
+                                             ("empties", 6, 600, 2048, 4096), ("onehot", 3, 900, 2056, 4104)])
+def test_backward_products_of_shared_experts(cuda, kind, G, rows, I, H):
+    """SwiGLU backward (rows through an index, weighted, with the partial sums of the weights' gradient) and the two-phase
+    input gradient over a bound of the rows: bounds as in test_products_over_a_bound_of_the_rows, nothing past the last row."""
+    from optimus import _native as n
+    torch.manual_seed(rows)
+    bf = lambda *s, f=1.0: (torch.randn(*s, device=cuda) * f).to(torch.bfloat16)
+    bound, cum = rows + 45, _counts(kind, G, rows)
+    dy, wg, wu, wd, g, u = bf(rows // 2, H), bf(G, I, H, f=0.02), bf(G, I, H, f=0.02), bf(G, H, I, f=0.02), bf(bound, I), bf(bound, I)
+    index = torch.randint(0, rows // 2, (bound,), device=cuda, dtype=torch.int32)
+    scale, new = torch.rand(bound, device=cuda), lambda c: torch.full((bound, c), 7.0, dtype=torch.bfloat16, device=cuda)
+    dg, du, dx, d, P, L = new(I), new(I), new(H), cum.to(cuda), n.ptr, n.lib()
+    dot = torch.full((L.om_merged_mlp_row_dot_parts(I), bound), 7.0, device=cuda)
+    n.check(L.om_merged_mlp_down_dgrad_weighted_bound(P(dy), P(index), rows // 2, P(wd), P(g), P(u), P(scale), P(dg), P(du), P(dot), P(d), bound,
+                                                      rows, G, I, H, 0, n.stream()), "down dgrad")
+    n.check(L.om_merged_mlp_gate_up_dgrad_bound(P(dg), P(du), P(wg), P(wu), P(dx), P(d), bound, rows, G, I, H, 0, n.stream()), "dx")
+    torch.cuda.synchronize()
+    assert all((t[rows:] == 7.0).all() for t in (dg, du, dx)) and (dot[:, rows:] == 7.0).all()
+    for e in range(G):
+        s = slice(int(cum[e]), int(cum[e + 1]))
+        gb, ub, dh = g[s].float(), u[s].float(), dy[index[s].long()].float() @ wd[e].float()
+        sig, pre = torch.sigmoid(gb), scale[s, None] * dh
+        factor = 1 + gb.abs() + ub.abs() * (1 + gb.abs())
+        for name, got, want, rel, room in (("du", du[s], pre * gb * sig, 2 ** -7 + 2 ** -12, H ** 0.5 * factor),
+                                           ("dg", dg[s], pre * ub * sig * (1 + gb * (1 - sig)), 2 ** -7 + 2 ** -12, H ** 0.5 * factor),
+                                           ("dx", dx[s], dg[s].float() @ wg[e].float() + du[s].float() @ wu[e].float(), 2 ** -8, (2 * I) ** 0.5)):
+            assert ((got.float() - want).abs() <= want.abs() * rel + 1e-6 * room).all(), (name, e)
+        terms = dh * gb * sig * ub
+        assert ((dot[:, s].sum(0) - terms.sum(1)).abs() <= (2 ** -8 + 1e-5) * terms.abs().sum(1) + 1e-6).all(), e
+
+
 # (rows per expert: enough to share, on 128x128 tiles; extents that tiles and steps divide and do not)
 @pytest.mark.parametrize("kind,G,rows,I,H", [("ragged", 16, 1500, 2048, 4096), ("empties", 5, 500, 2056, 4104), ("ragged", 33, 1100, 2056, 4104)])
 def test_sharing_experts_leaves_the_bits(cuda, kind, G, rows, I, H):

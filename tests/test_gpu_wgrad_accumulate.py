@@ -114,8 +114,9 @@ def test_three_weight_gradients_of_a_merged_mlp(cuda, indexed, kind, G, rows, I,
 
 
 # matrices of 96 and more 256x256 tiles, a multiple of eight of them: the XCDs share every expert's tiles, the experts come
-# by rows.  Equal rows, one expert, more experts than a round has blocks, all rows on one, wide and tall matrices.
-@pytest.mark.parametrize("kind,G,rows,N,K", [("uniform", 1, 100, 2048, 3072), ("ragged", 33, 1500, 2048, 3072), ("empties", 6, 900, 3072, 2048),
+# by rows.  Equal rows, one expert (with fewer than 128 tiles: the 128x128 kernel), more experts than a round has blocks, all
+# rows on one, wide and tall matrices.
+@pytest.mark.parametrize("kind,G,rows,N,K", [("uniform", 1, 100, 2048, 3072), ("uniform", 1, 100, 4096, 2048), ("ragged", 33, 1500, 2048, 3072), ("empties", 6, 900, 3072, 2048),
                                              ("onehot", 5, 700, 4096, 2048), ("uniform", 4, 512, 3072, 2048), ("uniform", 3, 0, 2048, 3072),
                                              # (the line below which only the accumulating form is shared)
                                              ("ragged", 33, 527, 2048, 3072), ("ragged", 33, 528, 2048, 3072)])
