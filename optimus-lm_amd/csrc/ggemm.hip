@@ -355,14 +355,9 @@ __device__ __forceinline__ void wgrad_xcd_run(const int32_t *cum, int n_experts,
     if (xcd == 0) lo = 0;
 }
 
-// 16 bytes per lane global -> LDS at lds_base + OFS + lane * 16.  Written as assembly so that the compiler neither
-// waits for such a load nor takes it for an LDS access: the main loop's own waits and barriers order them.
-// dma16_if: nothing is loaded with fewer than two steps `left` (block-uniform); the branch lies inside the assembly, so that a step stays one block
-// for the compiler's scheduler.
-template <int OFS> __device__ __forceinline__ void dma16(const void *base, uint32_t lane_bytes, uint32_t lds_base) {
-    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(lds_base), "v"(lane_bytes), "s"(base), "n"(OFS) : "scc");
-}
+// 16 bytes per lane global -> LDS at lds_base + OFS + lane * 16, nothing with fewer than two steps `left` (block-uniform).
+// Written as assembly so that the compiler neither waits for such a load nor takes it for an LDS access: the main loop's own
+// waits and barriers order them.  The branch lies inside, so that a step stays one block for the compiler's scheduler.
 template <int OFS>
 __device__ __forceinline__ void dma16_if(int left, const void *base, uint32_t lane_bytes, uint32_t lds_base) {
     asm volatile("s_cmp_lt_i32 %4, 2\n\ts_cbranch_scc1 .Lom_skip%=\n\ts_add_u32 m0, %0, %3\n\ts_nop 0\n\t"
