@@ -1179,7 +1179,8 @@ int launch_rows(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     const dim3 grid(persistent_blocks<BM>(tiles)), block(THREADS<BM>);
     const int64_t weights = static_cast<int64_t>(p.n_experts) * p.n_cols * p.kc * (EPI == EPI_SWIGLU ? 2 : p.phases);
-    if (BM == 128 && weights >= CACHED_WEIGHTS)
+    if (BM == 128 && om_weights_pass_caches(p.B[0], weights, p.ldb, p.strideB) &&
+        om_weights_pass_caches(p.B[1], weights, p.ldb, p.strideB))   // (one matrix: a null B[1], nothing to check)
         ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128, BM == 128><<<grid, block, 0, st>>>(p);
     else
         ggemm_kernel<BM, AKIND, BKIND, EPI, GATHER, ROWW, false, BM == 128><<<grid, block, 0, st>>>(p);
@@ -1245,7 +1246,8 @@ extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, 
     p.strideB = w_stride ? w_stride : static_cast<int64_t>(N) * K;
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N, K))
+    const bool past_caches = om_weights_pass_caches(weight, static_cast<int64_t>(G) * N * K, K, p.strideB);
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N, past_caches))
         return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, p.strideB,
                                    om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
@@ -1530,7 +1532,9 @@ int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, c
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I, H))
+    const int64_t weights = 2 * static_cast<int64_t>(G) * I * H;
+    const bool past_caches = om_weights_pass_caches(w_gate, weights, H, p.strideB) && om_weights_pass_caches(w_up, weights, H, p.strideB);
+    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I, past_caches))
         return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, expected, G, I,
                                        H, p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;

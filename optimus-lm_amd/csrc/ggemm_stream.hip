@@ -216,7 +216,7 @@ template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, int64_t e
 //   tokens (4.6 rows) 111 + 43 -> 111 + 48, hidden 7168, ffn 2048 at 8 rows 321 + 165 -> 360 + 174: tiled from two on;
 //   the same for a window of 32 experts of 7168 / 2048 whose rows are only expected (T tokens of top-8 of 256, six
 //   draws of weights and tokens, whole pass): 40 tokens -3.5 to +3.6 %, 56 tokens -7 to +3 %, 9 tokens 241 -> 220;
-//   fewer than half a row per expert where the tiled kernels load the weights past the caches (CACHED_WEIGHTS), which the
+//   fewer than half a row per expert where the tiled kernels load the weights past the caches (om_weights_pass_caches), which the
 //   figures above are without: whole forward of 4 tokens 80 (here 95), 8 tokens 115 (132), 15 tokens 140 (160); the window of
 //   32 experts, 20 tokens 246, 172, 178 (255, 179, 200), 60 tokens 275, 261, 244 (317, 266, 263); 2 and 9 tokens even;
 //   more rows where the tiles cannot fill the chip (fewer tiles than CUs): one expert of hidden 7168, ffn 2048
@@ -225,9 +225,8 @@ template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, int64_t e
 // `rows`: those to expect where only a bound is known.  (Going by the bound, eight times as many, the window of 32
 // experts of 1024 / 256 ran its gate+up product on tiles at 4 rows per expert and on 256x256 ones at 62: forward of
 // 128 tokens 82.3 -> 78.4 us, 256 86.5 -> 83.3, 1000 105.6 -> 102.3, 2000 112 -> 109; 512 91.6 -> 94.2.)
-bool om_ggemm_streams(int64_t rows, int n_experts, int cols, int kc) {
+bool om_ggemm_streams(int64_t rows, int n_experts, int cols, bool past_caches) {
     if (rows > 64 + 16 * static_cast<int64_t>(n_experts)) return false;
-    const bool past_caches = static_cast<int64_t>(n_experts) * cols * kc >= CACHED_WEIGHTS;
     if (rows < (past_caches ? n_experts / 2 : 2 * static_cast<int64_t>(n_experts))) return true;
     const int64_t hit = rows < n_experts ? rows : n_experts;
     return (hit + rows / 128) * ((cols + 127) / 128) <= 256;

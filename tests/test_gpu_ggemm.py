@@ -729,7 +729,7 @@ def test_row_units_and_step_counts_of_the_256_kernels(cuda, K):
                                              ("empties", 20, 5000, 2048, 4096), ("onehot", 3, 900, 4352, 2048), ("ragged", 5, 1700, 2056, 4104),
                                              ("ragged", 70, 9000, 2048, 4096), ("uniform", 2, 64, 4096, 2048),
                                              # (not shared, but too much for the caches: experts with one row tile, with several)
-                                             ("ragged", 64, 3000, 1024, 2048), ("onehot", 40, 129, 2056, 1640),
+                                             ("ragged", 64, 3000, 1024, 2048), ("onehot", 40, 129, 2056, 1640), ("ragged", 40, 129, 2056, 1664),
                                              ("ragged", 64, 33, 1024, 2048), ("uniform", 64, 31, 1024, 2048)])
 def test_row_products_of_shared_experts(cuda, kind, G, rows, N, K):
     """Every tile once: forward, input gradient and the gate/up product against float32 products of each expert's
