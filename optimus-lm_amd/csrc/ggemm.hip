@@ -1152,13 +1152,16 @@ template <int BM> unsigned persistent_blocks(int64_t tiles) {
 }
 
 
-// CACHED_WEIGHTS: the caches hold 256 MB, and more than the weights passes through them.  From there on the weights are
-// kept out of them: the 128x128 row products load those of an expert with one row tile without leaving them there, the
-// 256x256 weight gradients are stored past them; what the caches held instead was written back or fetched again under
+// CACHED_WEIGHTS: the caches hold 256 MB, and more than a launch's weights passes through them.  From there on (gate and up: 64 M
+// elements each) the weights are kept out of them: the 128x128 row products load those of an expert with one row tile without
+// leaving them there (rows of whole lines: om_weights_pass_caches), the 256x256 weight gradients are stored past them; what the caches held instead was written back or fetched again under
 // the next products.  us, 64 experts of 1024/2048: 37 tokens gate+up 104 -> 93 (5.8 TB/s of weights), down 50 -> 44;
 // 512 tokens, uneven, gate/up input gradient behind the weight gradients 167 -> 104, those 209 -> 214; 32 experts of 2048/7168, 64
-// rows in all, 146 -> 133 and 84 -> 75.  Weights that do fit lose by it (32 experts of 376/1720, 733 tokens: forward 113 -> 117),
-// and so do those that a second row tile reads (12 experts of 712/1000, 750 rows each: gate+up 51 -> 82 when all were
+// rows in all, 146 -> 133 and 84 -> 75.  Around the line, whole forward of 37 tokens, 64 experts, ffn 1024, nothing -> all three
+// matrices past the caches: hidden 512 54 -> 58, 768 80 -> 76, 1280 119 -> 108, 1536 136 -> 116, 2048 169 -> 147, 3072 238 -> 206 (1280
+// with the line 109); training steps of 512 tokens, gradients written: hidden 256 (48 M in all three) 171 -> 169, 512 239 -> 204 (the line
+// leaves that out), 1024 377 -> 325, 1792 624 -> 542; added, within 1.5 %.  What loses by it are weights
+// that a second row tile reads (12 experts of 712/1000, 750 rows each: gate+up 51 -> 82 when all were
 // loaded so) and the saved g and u of the forward (prefill of 4096 tokens, gate+up 344 -> 354).
 
 // XCDs that share an expert's row products: from 8 M weights a matrix on, four, or all eight with few experts, which two
@@ -1286,6 +1289,9 @@ bool wgrad_big_tile(int n, int k, int64_t matrices) {
 // as 1 / rank^1.2, writing: 8 rows in all 538 -> 483 / 531 -> 505, 128 rows 540 -> 524 / 531 -> 524, 512 rows 541 -> 523 / 550 -> 583,
 // 2048 rows 625 -> 634 / 632 -> 684; accumulating: 1 row 114 -> 254, 64 rows 913 -> 1043 / 667 -> 768.  64 experts of 1024/2048,
 // writing: 64 rows 161 -> 148 / 159 -> 132, 512 rows 162 -> 158 / 156 -> 161, 2048 rows 166 -> 164 / 177 -> 175.
+// Around 12 tiles per XCD the two are near each other, even rows a little better alone and uneven ones shared: 64 rows an expert,
+// not shared -> shared, even / uneven, writing: 48 tiles (64 experts of 1024/1024) 97 -> 100 / 110 -> 115, 72 149 -> 145 / 161 -> 152, 84 172 ->
+// 168 / 175 -> 173, 96 199 -> 187 / 193 -> 195, 120 239 -> 231 / 245 -> 243, 144 275 -> 284 / 293 -> 284.
 int wgrad_share(bool big, int tiles_e, int n_experts, int64_t rows, bool accumulate) {
     if (!accumulate && rows < 16 * static_cast<int64_t>(n_experts)) return 0;
     return big && tiles_e >= 12 * NUM_XCD && n_experts <= SHARE_MAX_EXPERTS ? NUM_XCD : 0;

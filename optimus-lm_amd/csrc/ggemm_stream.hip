@@ -218,7 +218,9 @@ template <bool SWIGLU> int launch(const StreamParams &p, int64_t rows, int64_t e
 //   draws of weights and tokens, whole pass): 40 tokens -3.5 to +3.6 %, 56 tokens -7 to +3 %, 9 tokens 241 -> 220;
 //   fewer than half a row per expert where the tiled kernels load the weights past the caches (om_weights_pass_caches), which the
 //   figures above are without: whole forward of 4 tokens 80 (here 95), 8 tokens 115 (132), 15 tokens 140 (160); the window of
-//   32 experts, 20 tokens 246, 172, 178 (255, 179, 200), 60 tokens 275, 261, 244 (317, 266, 263); 2 and 9 tokens even;
+//   32 experts, 20 tokens 246, 172, 178 (255, 179, 200), 60 tokens 275, 261, 244 (317, 266, 263); 2 and 9 tokens even; at half a row an expert
+//   itself 64 experts of ffn 1024 are even on average (4 tokens, hidden 1024 51.8 (49.4), 1536 68.0 (63.7), 1792 74.6 (75.5), 2048 83.5
+//   (91.4), 3072 111 (109)), at one row 2 to 9 % better;
 //   more rows where the tiles cannot fill the chip (fewer tiles than CUs): one expert of hidden 7168, ffn 2048
 //   with 64 rows 65 + 21 -> 40 + 14; 12 experts of hidden 1000, ffn 712 with 192 rows 19 + 11.6 -> 10.8 + 5.4;
 //   beyond 64 rows of one expert the weights are streamed again per row tile: 128 rows 65 + 21 -> 43 + 25.
