@@ -122,10 +122,11 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 bool om_ggemm_streams(int64_t rows, int n_experts, int cols, bool past_caches);   // cols: weight rows per expert (gate and up: both)
 // Elements of weights, or of their gradients, that the caches cannot hold from one use to the next (see ggemm.hip).
 constexpr int64_t CACHED_WEIGHTS = 128 << 20;
-// Whether the tiled kernels load a launch's weights (`elements` in all, rows `pitch` apart) past the caches: only where the
-// 128-byte pieces that they load are whole lines.  A line of two pieces would be fetched twice, which the caches otherwise
+// Whether the tiled kernels load a launch's weights (`elements` in all, rows `pitch` apart) past the caches, or store its weight
+// gradients so: only where the 128-byte pieces that they load or store are whole lines.  A line of two pieces would be fetched twice, which the caches otherwise
 // spare: forward of 64 experts, ffn 1024, us, through the caches -> past them: hidden 2600, 37 tokens 225 -> 243, 512 tokens 283 -> 326, hidden
-// 2624 207 -> 181, 249 -> 241; 16 experts of 7000/2040, 2 tokens 280 -> 328, of 7168/2048 231 -> 208.
+// 2624 207 -> 181, 249 -> 241; 16 experts of 7000/2040, 2 tokens 280 -> 328, of 7168/2048 231 -> 208.  Written gradients
+// 16 bytes off a line: 32 experts of 2048/7168, 128 rows 597 -> 1552, on a line 576 -> 524.
 inline bool om_weights_pass_caches(const void *w, int64_t elements, int64_t pitch, int64_t expert_pitch) {
     return elements >= CACHED_WEIGHTS && pitch % 64 == 0 && expert_pitch % 64 == 0 && reinterpret_cast<uintptr_t>(w) % 128 == 0;
 }

@@ -111,7 +111,7 @@ struct GemmParams {
     int phases;                 // 1 or 2
     int total_tiles;            // wgrad: tiles of the launch (the blocks loop over them)
     int tiles_e;                // wgrad: tiles per expert (MERGED: of all three)
-    bool stream;                // wgrad: the gradients do not fit the caches (see CACHED_WEIGHTS)
+    bool stream;                // wgrad: the gradients are stored past the caches (see CACHED_WEIGHTS)
     int share;                  // XCDs that share an expert's tiles; 0: contiguous runs of tiles per XCD
     WgradSet set[3];            // MERGED
 };
@@ -1325,7 +1325,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
     p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
-    p.stream = static_cast<int64_t>(G) * N * K >= CACHED_WEIGHTS;
+    p.stream = om_weights_pass_caches(weight_grad, static_cast<int64_t>(G) * N * K, K, p.strideC);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
@@ -1479,7 +1479,8 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     }
     p.tiles_e = static_cast<int>(3 * each);
     p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
-    p.stream = 3 * packed * G >= CACHED_WEIGHTS;
+    p.stream = true;
+    for (const WgradSet &s : p.set) p.stream &= om_weights_pass_caches(s.C, 3 * packed * G, s.n, s.strideC);
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);

@@ -148,6 +148,23 @@ def test_weight_gradients_spread_over_the_xcds(cuda, gathered, kind, G, rows, N,
     assert (bits(acc) == bits(old.add_(fresh))).all()
 
 
+@pytest.mark.parametrize("offset", [0, 8, 32])
+def test_large_gradients_off_a_line(cuda, offset):
+    """Gradients that the caches cannot hold, on a 128-byte line (stored past the caches) and off it: the same bits."""
+    from optimus import _native as n
+    G, rows, I, H = 45, 500, 1024, 1024
+    torch.manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)
+    dout, x, h, dg, du, d, P = rnd(rows, H), rnd(rows, H), rnd(rows, I), rnd(rows, I), rnd(rows, I), _counts("ragged", G, rows).to(cuda), n.ptr
+    out = [torch.full((G * I * H + 64,), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(3)]
+    _call("om_grouped_gemm_wgrad_merged", P(dout), None, P(h), P(dg), P(du), P(x), None, 0, *(P(o[offset:]) for o in out), P(d), rows, G, I, H, 0, 0, 0)
+    for o, a, b in zip(out, (dout, dg, du), (h, x, x)):
+        one = torch.empty(G, I, H, dtype=torch.bfloat16, device=cuda)
+        _call("om_grouped_gemm_wgrad", P(a), P(b), P(one), P(d), rows, G, H, I, 0)
+        assert torch.equal(o[offset:offset + one.numel()].view_as(one), one)
+        assert (o[:offset] == 7.0).all() and (o[offset + one.numel():] == 7.0).all()
+
+
 def test_accumulate_f32(cuda):
     from optimus import _native as n
     g = torch.Generator().manual_seed(5)
