@@ -464,11 +464,17 @@ __global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restr
 // statements around them).  What is left to bound it is `base` and dx.
 // us, `base` and weights out of the caches, 256 experts, before (128 tokens x 128 columns a block, dlogits in fp32 once per 128
 // columns) -> now: hidden 7168, 64 tokens 18.9 -> 11.3, 512 tokens 19.7 -> 16.4, 8192 tokens 113.9 -> 71.0 (4.0 TB/s of base,
-// dx and dlogits); hidden 1624, 8176 tokens 45.3 -> 36.6; 128 experts, hidden 4096, 4096 tokens 29.3 -> 24.3.
+// dx and dlogits); 128 experts, hidden 4096, 4096 tokens 29.3 -> 24.3.  Hidden sizes that are not a multiple of 64, `base` and
+// dx past the caches / through them: 256 experts, hidden 7000, 8192 tokens (133 before) 135 / 98, 1624, 17000 tokens (69) 65 / 50;
+// 128 experts, hidden 7000, 8192 tokens (91) 130 / 76.  With everything in the caches, as a repeated call alone finds it, the
+// kernel before was the faster one from 200 tokens up to about 6 M elements (256 experts, hidden 2048, 1024 tokens 10.3 against
+// 12.0); behind a layer's expert products, which leave the gate's weight to memory, 16.0 against 12.9.
 constexpr int DW_HT = 64, DW_TOK = 256, DW_PITCH = DW_HT * 2 + 8;
 
 // NK * 16 >= N experts; grid (column ranges of `tiles` slices, T / 256)
-template <int NK, bool BASE>
+// LINES: the 128-byte pieces of `base` and dx that a slice takes are whole lines and pass the caches by; a line of two pieces would
+// be moved twice.
+template <int NK, bool BASE, bool LINES>
 __global__ __launch_bounds__(512) void gate_dgrad_wide_kernel(const float *__restrict__ dlogits, const uint16_t *__restrict__ weight,
                                                               const uint16_t *base, uint16_t *out, int64_t T, int H, int N, int tiles) {
     constexpr int SLOTS = 3, SLOT = NK * 16 * DW_HT * 2, LOADS = SLOT / 1024 / 8, ITS = 32 * (DW_HT / 8) / 64;
@@ -499,8 +505,9 @@ __global__ __launch_bounds__(512) void gate_dgrad_wide_kernel(const float *__res
 #pragma unroll
         for (int it = 0; it < ITS; it++) {
             const int q = it * 64 + lane;
-            other[set][it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(   // read once
-                base + min(t0 + q / (DW_HT / 8), T - 1) * H + min((first + s) * DW_HT + (q % (DW_HT / 8)) * 8, H - 8)));
+            const u32x4 *from = reinterpret_cast<const u32x4 *>(
+                base + min(t0 + q / (DW_HT / 8), T - 1) * H + min((first + s) * DW_HT + (q % (DW_HT / 8)) * 8, H - 8));
+            other[set][it] = LINES ? __builtin_nontemporal_load(from) : *from;   // read once
         }
     };
     if (BASE) fetch_base(0, 0);
@@ -569,7 +576,11 @@ __global__ __launch_bounds__(512) void gate_dgrad_wide_kernel(const float *__res
                 for (int i = 0; i < 8; i++) a[i] = a[i] + g[i];
                 v = Elem<uint16_t>::pack(a);
             }
-            if (tt < T && h < H) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out + tt * H + h));
+            if (tt < T && h < H) {
+                u32x4 *to = reinterpret_cast<u32x4 *>(out + tt * H + h);
+                if (LINES) __builtin_nontemporal_store(v, to);
+                else *to = v;
+            }
         }
         if (s + 2 < steps) issue(s + 2, free_slot);
         free_slot = slot;
@@ -599,10 +610,17 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
         const int slices = (H + DW_HT - 1) / DW_HT, ranges = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(slices, 256 / wide_blocks)));
         const int tiles = (slices + ranges - 1) / ranges;
         const dim3 grid((slices + tiles - 1) / tiles, static_cast<unsigned>(wide_blocks));
-        if (N <= 128 && base) gate_dgrad_wide_kernel<8, true><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
-        else if (N <= 128) gate_dgrad_wide_kernel<8, false><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
-        else if (base) gate_dgrad_wide_kernel<16, true><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
-        else gate_dgrad_wide_kernel<16, false><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles);
+        const bool lines = H % 64 == 0 && reinterpret_cast<uintptr_t>(base) % 128 == 0 && reinterpret_cast<uintptr_t>(dx) % 128 == 0;
+#define OM_WIDE(NK, BASE)                                                                                        \
+    do {                                                                                                         \
+        if (lines) gate_dgrad_wide_kernel<NK, BASE, true><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles); \
+        else gate_dgrad_wide_kernel<NK, BASE, false><<<grid, dim3(512), 0, st>>>(dl, w, bp, dp, T, H, N, tiles); \
+    } while (0)
+        if (N <= 128 && base) OM_WIDE(8, true);
+        else if (N <= 128) OM_WIDE(8, false);
+        else if (base) OM_WIDE(16, true);
+        else OM_WIDE(16, false);
+#undef OM_WIDE
         return om_launch_status();
     }
     const int64_t t_blocks = (T + DG_TOK - 1) / DG_TOK;

@@ -534,7 +534,7 @@ def test_gate_of_many_tokens(cuda, T, H, N, slices):
 
 
 @pytest.mark.parametrize("T,H,N", [(1, 8, 65), (127, 72, 100), (129, 64, 128), (257, 128, 129), (256, 1624, 256), (640, 200, 160), (300, 7168, 80),
-                                   (33000, 136, 256), (700, 264, 132), (1000, 520, 250)])
+                                   (33000, 136, 256), (700, 264, 132), (1000, 520, 250), (700, 192, 96)])
 @pytest.mark.parametrize("base", [False, True])
 def test_gate_of_many_experts(cuda, T, H, N, base):
     """Projection and both gradients of more than 64 experts: edges of the blocks of 128 and 256 tokens, one to three steps
