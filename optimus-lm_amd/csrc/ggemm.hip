@@ -1302,7 +1302,7 @@ int wgrad_share(bool big, int tiles_e, int n_experts, int64_t rows, bool accumul
 // [src_rows, N] matrix (the token gather folded into the loads)
 int wgrad_launch(const void *output_grad, const void *input, const int32_t *index, int gather,
                  int64_t src_rows, void *weight_grad, const int32_t *cum_token_counts, int64_t rows, int G,
-                 int N, int K, int64_t w_stride, void *stream, bool accumulate = false) {
+                 int N, int K, int64_t w_stride, void *stream, bool accumulate = false, int64_t expected = -1) {
     if (rows < 0 || G < 1 || !mult(N, 8) || !mult(K, 8)) return OM_ERR_SHAPE;
     // rows == 0 (nothing routed to these experts): the activations may be empty tensors without
     // storage; the launch then only writes zeros
@@ -1324,7 +1324,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     hipStream_t st = om_stream(stream);
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
-    p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
+    p.share = wgrad_share(big, p.tiles_e, G, expected < 0 ? rows : expected, accumulate);
     p.stream = om_weights_pass_caches(weight_grad, static_cast<int64_t>(G) * N * K, K, p.strideC);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
@@ -1418,9 +1418,9 @@ namespace {
 // expert's three gradients come one after the other.
 int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du, const void *x,
                         const int32_t *x_rows, int64_t src_rows, void *dw_down, void *dw_gate, void *dw_up,
-                        const int32_t *cum_token_counts, int64_t rows, int G, int I, int H, int64_t down_stride,
+                        const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I, int H, int64_t down_stride,
                         int64_t gate_stride, int64_t up_stride, bool accumulate, void *stream) {
-    if (rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
     if (!dw_down || !dw_gate || !dw_up || !cum_token_counts || (rows > 0 && (!dout || !h || !dg || !du || !x))) return OM_ERR_NULL;
     if ((dout_rows || x_rows) && src_rows < 1) return OM_ERR_SHAPE;
     GemmParams p = {};
@@ -1465,20 +1465,20 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     }
     const bool no_fewer_rounds = big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone);
     const bool many_rounds = !big && rounds(tiles, blocks) > (accumulate ? 32 : 16);
-    if (overlap || (no_fewer_rounds && (many_rounds || rows > 256 * static_cast<int64_t>(G)))) {
+    if (overlap || (no_fewer_rounds && (many_rounds || expected > 256 * static_cast<int64_t>(G)))) {
         const int gather_d = dout_rows ? GATHER_WA : GATHER_NONE, gather_x = x_rows ? GATHER_B : GATHER_NONE;
         int code = wgrad_launch(dout, h, dout_rows, gather_d, dout_rows ? src_rows : 0, dw_down, cum_token_counts, rows, G, H, I,
-                                down_stride, stream, accumulate);
+                                down_stride, stream, accumulate, expected);
         if (code == OM_OK)
             code = wgrad_launch(dg, x, x_rows, gather_x, x_rows ? src_rows : 0, dw_gate, cum_token_counts, rows, G, I, H,
-                                gate_stride, stream, accumulate);
+                                gate_stride, stream, accumulate, expected);
         if (code == OM_OK)
             code = wgrad_launch(du, x, x_rows, gather_x, x_rows ? src_rows : 0, dw_up, cum_token_counts, rows, G, I, H,
-                                up_stride, stream, accumulate);
+                                up_stride, stream, accumulate, expected);
         return code;
     }
     p.tiles_e = static_cast<int>(3 * each);
-    p.share = wgrad_share(big, p.tiles_e, G, rows, accumulate);
+    p.share = wgrad_share(big, p.tiles_e, G, expected, accumulate);
     p.stream = true;
     for (const WgradSet &s : p.set) p.stream &= om_weights_pass_caches(s.C, 3 * packed * G, s.n, s.strideC);
     p.total_tiles = static_cast<int>(tiles);
@@ -1498,7 +1498,7 @@ extern "C" int om_grouped_gemm_wgrad_merged(const void *dout, const int32_t *dou
                                             int64_t rows, int G, int I, int H, int64_t down_stride,
                                             int64_t gate_stride, int64_t up_stride, void *stream) {
     return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
-                               cum_token_counts, rows, G, I, H, down_stride, gate_stride, up_stride, false, stream);
+                               cum_token_counts, rows, rows, G, I, H, down_stride, gate_stride, up_stride, false, stream);
 }
 
 extern "C" int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const int32_t *dout_rows, const void *h,
@@ -1508,7 +1508,26 @@ extern "C" int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const i
                                                        int64_t rows, int G, int I, int H, int64_t down_stride,
                                                        int64_t gate_stride, int64_t up_stride, void *stream) {
     return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
-                               cum_token_counts, rows, G, I, H, down_stride, gate_stride, up_stride, true, stream);
+                               cum_token_counts, rows, rows, G, I, H, down_stride, gate_stride, up_stride, true, stream);
+}
+
+extern "C" int om_grouped_gemm_wgrad_merged_bound(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
+                                            const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
+                                            void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                            int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t down_stride,
+                                            int64_t gate_stride, int64_t up_stride, void *stream) {
+    return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
+                               cum_token_counts, rows, expected_rows, G, I, H, down_stride, gate_stride, up_stride, false, stream);
+}
+
+extern "C" int om_grouped_gemm_wgrad_merged_accumulate_bound(const void *dout, const int32_t *dout_rows, const void *h,
+                                                       const void *dg, const void *du, const void *x,
+                                                       const int32_t *x_rows, int64_t src_rows, void *dw_down,
+                                                       void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                                       int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t down_stride,
+                                                       int64_t gate_stride, int64_t up_stride, void *stream) {
+    return wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up,
+                               cum_token_counts, rows, expected_rows, G, I, H, down_stride, gate_stride, up_stride, true, stream);
 }
 
 namespace {

@@ -455,15 +455,15 @@ struct Sinks {
 };
 
 // All three weight gradients of a bf16 merged MLP: one call where all are written or all are added into their sinks.
-// dout_rows / x_rows: rows of dout / x taken through an index.
+// dout_rows / x_rows: rows of dout / x taken through an index.  `expected`: the rows to choose launches by, where `rows` is a bound.
 void wgrads(const Call &c, const Tensor &dout, const int32_t *dout_rows, const Tensor &h, const Tensor &dg, const Tensor &du,
-            const Tensor &x, const int32_t *x_rows, const Sinks &k, const int32_t *cum, int64_t rows, int64_t G, int64_t I,
-            int64_t H) {
+            const Tensor &x, const int32_t *x_rows, const Sinks &k, const int32_t *cum, int64_t rows, int64_t expected, int64_t G,
+            int64_t I, int64_t H) {
     if (k.gate.accumulate == k.up.accumulate && k.gate.accumulate == k.down.accumulate) {
         const int64_t src_rows = dout_rows ? dout.size(0) : x.size(0);
 #define OM_W(fn)                                                                                                        \
-    OM(c, fn, ptr(dout), dout_rows, ptr(h), ptr(dg), ptr(du), ptr(x), x_rows, src_rows, ptr(k.down.grad), ptr(k.gate.grad), \
-       ptr(k.up.grad), cum, rows, G, I, H, k.down.pitch, k.gate.pitch, k.up.pitch, c.stream)
+    OM_BOUND(c, fn, ptr(dout), dout_rows, ptr(h), ptr(dg), ptr(du), ptr(x), x_rows, src_rows, ptr(k.down.grad), ptr(k.gate.grad), \
+             ptr(k.up.grad), cum, rows, expected, G, I, H, k.down.pitch, k.gate.pitch, k.up.pitch, c.stream)
         if (k.gate.accumulate) OM_W(om_grouped_gemm_wgrad_merged_accumulate);
         else OM_W(om_grouped_gemm_wgrad_merged);
 #undef OM_W
@@ -506,7 +506,7 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
     }
     OM(c, om_merged_mlp_down_dgrad, ptr(dy), ptr(w.down), ptr(s.g), ptr(s.u), ptr(dg), ptr(du), cum, rows, G, I, H,
        expert_stride(w.down), c.stream);
-    wgrads(c, dy, nullptr, s.h, dg, du, x, rows > 0 ? x_rows : nullptr, k, cum, rows, G, I, H);
+    wgrads(c, dy, nullptr, s.h, dg, du, x, rows > 0 ? x_rows : nullptr, k, cum, rows, rows, G, I, H);
     OM(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx), cum, rows, G, I, H,
        expert_stride(w.gate), c.stream);
     return dx;
@@ -573,7 +573,7 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
                      ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
             OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
                c.stream);
-            wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, G, I, H);
+            wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, ix.to_choose_by(), G, I, H);
             OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
                      ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
         } else {   // nothing routed to these experts: fresh weight gradients are zero, live ones stay as they are

@@ -163,6 +163,10 @@ SIGNATURES = {
                                      [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_void_p]),
     "om_grouped_gemm_wgrad_merged_accumulate": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 4 +
                                                 [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_void_p]),
+    "om_grouped_gemm_wgrad_merged_bound": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 4 +
+                                           [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_void_p]),
+    "om_grouped_gemm_wgrad_merged_accumulate_bound": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 4 +
+                                                      [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_void_p]),
     "om_merged_mlp_gate_up_fwd_f32": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 6 +
                                       [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_void_p]),
     "om_merged_mlp_down_dgrad_f32": (c_int, [c_void_p] * 7 + [c_i64, c_int, c_int, c_int, c_i64, c_void_p]),

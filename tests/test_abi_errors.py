@@ -219,12 +219,17 @@ def test_products_over_a_bound_of_the_rows(lib):
         assert lib.om_merged_mlp_down_dgrad_weighted_bound(P, P, 512, P, P, P, P, P, P, P, P, 4096, expected, 64, 1024, 2048, 0,
                                                            None) == SHAPE
         assert lib.om_merged_mlp_gate_up_dgrad_bound(P, P, P, P, P, P, 4096, expected, 64, 1024, 2048, 0, None) == SHAPE
+        for form in (lib.om_grouped_gemm_wgrad_merged_bound, lib.om_grouped_gemm_wgrad_merged_accumulate_bound):
+            assert form(P, P, P, P, P, P, P, 512, P, P, P, P, 4096, expected, 64, 1024, 2048, 0, 0, 0, None) == SHAPE
     assert lib.om_grouped_gemm_fwd_bound(P, None, P, P, 4096, 64, 64, 2048, 1024, 0, None) == NULL
     assert lib.om_grouped_gemm_fwd_bound(None, None, None, None, 0, 0, 64, 2048, 1024, 0, None) == OK
     assert lib.om_merged_mlp_gate_up_fwd_weighted_bound(P, None, 512, P, P, P, P, P, P, P, 4096, 64, 64, 1024, 2048, 0,
                                                         None) == NULL
     assert lib.om_merged_mlp_down_dgrad_weighted_bound(P, P, 512, P, P, P, P, P, ODD, P, P, 4096, 64, 64, 1024, 2048, 0,
                                                        None) == ALIGN
+    assert lib.om_grouped_gemm_wgrad_merged_bound(P, P, P, P, P, P, P, 512, P, P, None, P, 4096, 64, 64, 1024, 2048, 0, 0, 0, None) == NULL
+    assert lib.om_grouped_gemm_wgrad_merged_accumulate_bound(P, P, P, P, P, P, P, 512, P, ODD, P, P, 4096, 64, 64, 1024, 2048, 0, 0, 0,
+                                                             None) == ALIGN
     assert lib.om_merged_mlp_gate_up_dgrad_bound(P, P, P, P, None, P, 4096, 64, 64, 1024, 2048, 0, None) == NULL
 
 

@@ -148,6 +148,43 @@ def test_weight_gradients_spread_over_the_xcds(cuda, gathered, kind, G, rows, N,
     assert (bits(acc) == bits(old.add_(fresh))).all()
 
 
+def _launches(fn):
+    """Kernels that fn launches."""
+    import ctypes
+    from optimus import _native as n
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        fn()
+    nodes = ctypes.c_size_t()
+    count = ctypes.CDLL(n.LIB_PATH).hipGraphGetNodes       # (the runtime that the library is linked with)
+    assert count(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    return nodes.value
+
+
+# 16 experts of 32 tiles a product: as many rounds in one launch as in three, so that only few rows take one launch
+@pytest.mark.parametrize("suffix", ["", "_accumulate"])
+@pytest.mark.parametrize("expected,launches", [(0, 1), (520, 1), (4096, 1), (4097, 3), (4160, 3)])
+def test_launches_go_by_the_rows_to_expect(cuda, suffix, expected, launches):
+    """Where `rows` is a bound, three times and more what there is, the choice is the one that the plain form makes for
+    the rows to expect, and the results are its results."""
+    from optimus import _native as n
+    G, bound, I, H = 16, 4160, 1024, 2048
+    cum = _counts("ragged", G, 520)
+    torch.manual_seed(2)
+    rnd = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)
+    dout, x, h, dg, du, d, P = rnd(bound, H), rnd(bound, H), rnd(bound, I), rnd(bound, I), rnd(bound, I), cum.to(cuda), n.ptr
+    old = [rnd(G, I * H) for _ in range(3)]
+    got, want = [o.clone() for o in old], [o.clone() for o in old]
+    args = lambda out, *rows: (P(dout), None, P(h), P(dg), P(du), P(x), None, 0, *(P(o) for o in out), P(d), *rows, G, I, H, 0, 0, 0)
+    _call("om_grouped_gemm_wgrad_merged" + suffix, *args(want, 520))
+    name = "om_grouped_gemm_wgrad_merged" + suffix + "_bound"
+    _call(name, *args(got, bound, expected))
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert (bits(a) == bits(b)).all()
+    assert _launches(lambda: _call(name, *args(got, bound, expected))) == launches
+
+
 @pytest.mark.parametrize("offset", [0, 8, 32])
 def test_large_gradients_off_a_line(cuda, offset):
     """Gradients that the caches cannot hold, on a 128-byte line (stored past the caches) and off it: the same bits."""
