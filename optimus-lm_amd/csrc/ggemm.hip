@@ -1451,6 +1451,13 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     // writing 64 rows in all 219 -> 204, 2048 rows 251 -> 244, 8192 rows 361 -> 330, accumulating 299 -> 290, 354 -> 357, 440 -> 415; 16 of
     // 1104x3736, 26 rounds, writing 64 rows 132 -> 118, 2048 203 -> 179, accumulating 193 -> 210, 253 -> 244; 16 of 688x2304, 11 rounds, writing
     // 50 -> 53, 72 -> 67; 48 of 520x1400, 16 rounds (18 in three), writing 67 -> 69, 70 -> 70, accumulating 95 -> 104, 97 -> 111.
+    // Nor from 128 rows an expert on with many rounds of 256x256 tiles that are written, of experts that the XCDs share in each launch
+    // (those that they share in one launch only, 128 of 1024x2048, gain by that: uneven 256 rows 992 -> 750).  One -> three, even rows
+    // / as 1 / rank^1.2: 32 of 2048x7168, 84 rounds, 64 rows 583 -> 605 / 662 -> 645, 128 rows 771 -> 755 / 788 -> 753, 256 rows 1171 -> 1058 /
+    // 1198 -> 1060; 16 of them, 42 rounds, 64 rows 296 -> 308 / 329 -> 323, 128 rows 390 -> 380 / 415 -> 395, 256 rows 560 -> 525 / 561 ->
+    // 541; 64 of 2048x4096, 96 rounds, 128 rows 880 -> 870 / 914 -> 912, 256 rows 1322 -> 1245 / 1392 -> 1315; 32 of 1536x5120, 45 rounds,
+    // 128 rows 408 -> 407 / 428 -> 428, 256 rows 605 -> 581 / 603 -> 602; 8 of 2048x7168, 21 rounds, 256 rows 282 -> 307 / 309 -> 308.
+    // Adding, 32 of 2048x7168, 128 rows 1213 -> 1208 / 1276 -> 1272, others slower in three.
     const int64_t blocks = static_cast<int64_t>(device_cu_count()) * (big ? 1 : 2);
     auto rounds = [](int64_t t, int64_t b) { return (t + b - 1) / b; };
     const bool big_alone = wgrad_big_tile(H, I, G);
@@ -1465,7 +1472,8 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     }
     const bool no_fewer_rounds = big == big_alone && 11 * rounds(tiles, blocks) >= 10 * 3 * rounds(alone, blocks_alone);
     const bool many_rounds = !big && rounds(tiles, blocks) > (accumulate ? 32 : 16);
-    if (overlap || (no_fewer_rounds && (many_rounds || expected > 256 * static_cast<int64_t>(G)))) {
+    const bool large = big && !accumulate && rounds(tiles, blocks) > 32 && each >= 12 * NUM_XCD;
+    if (overlap || (no_fewer_rounds && (many_rounds || expected > 256 * static_cast<int64_t>(G) || (large && expected >= 128 * static_cast<int64_t>(G))))) {
         const int gather_d = dout_rows ? GATHER_WA : GATHER_NONE, gather_x = x_rows ? GATHER_B : GATHER_NONE;
         int code = wgrad_launch(dout, h, dout_rows, gather_d, dout_rows ? src_rows : 0, dw_down, cum_token_counts, rows, G, H, I,
                                 down_stride, stream, accumulate, expected);

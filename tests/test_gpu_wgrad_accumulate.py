@@ -185,6 +185,27 @@ def test_launches_go_by_the_rows_to_expect(cuda, suffix, expected, launches):
     assert _launches(lambda: _call(name, *args(got, bound, expected))) == launches
 
 
+# 33 rounds of 256x256 tiles: from 128 rows an expert on the writing form makes three launches
+@pytest.mark.parametrize("rows,suffix,launches", [(3711, "", 1), (3712, "", 3), (3712, "_accumulate", 1)])
+def test_launches_of_large_experts(cuda, rows, suffix, launches):
+    from optimus import _native as n
+    G, I, H = 29, 2048, 3072
+    torch.manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, device=cuda).to(torch.bfloat16)
+    dout, x, h, dg, du, d, P = rnd(rows, H), rnd(rows, H), rnd(rows, I), rnd(rows, I), rnd(rows, I), _counts("ragged", G, rows).to(cuda), n.ptr
+    got = [rnd(G, I * H) for _ in range(3)]
+    want = [o.clone() for o in got]
+    run = lambda: _call("om_grouped_gemm_wgrad_merged" + suffix, P(dout), None, P(h), P(dg), P(du), P(x), None, 0, *(P(o) for o in got),
+                        P(d), rows, G, I, H, 0, 0, 0)
+    run()
+    for o, a, b, m, k in zip(want, (dout, dg, du), (h, x, x), (H, I, I), (I, H, H)):
+        _call("om_grouped_gemm_wgrad" + suffix, P(a), P(b), P(o), P(d), rows, G, m, k, 0)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert _launches(run) == launches
+
+
 @pytest.mark.parametrize("offset", [0, 8, 32])
 def test_large_gradients_off_a_line(cuda, offset):
     """Gradients that the caches cannot hold, on a 128-byte line (stored past the caches) and off it: the same bits."""
