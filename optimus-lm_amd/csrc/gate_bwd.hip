@@ -161,9 +161,12 @@ __global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restr
 // ahead through a ring of three, the dlogits through registers, two steps ahead too, and a pair of buffers.  Every step loads,
 // past the last one that one again, so that the number of loads in flight is known.  The dlogits' loads are among those that the
 // wait counts: `dlogits` is not __restrict__, so that the compiler may not move them over the assembly's memory clobbers.
+// (The compiler's own wait for the dlogits of the next step counts its loads alone, and so waits for x of that step too: of its
+// two steps x has one and a part.)
 // us with the launch that adds the ranges, x out of the caches, before (128 columns a block, both operands through registers
 // one stage ahead) -> now, 256 experts: hidden 7168, 64 tokens 19.3 -> 16.4, 2048 tokens 57 -> 41, 8192 tokens 115 -> 72; hidden
-// 1624, 8176 tokens 60 -> 42.  160 experts, hidden 5120, 4096 tokens 56 -> 37.
+// 1624, 8176 tokens 60 -> 42.  160 experts, hidden 5120, 4096 tokens 56 -> 37.  Without a way out between the two steps of the
+// loop's body: 8192 tokens 77.1 -> 70.8, 160 experts 36.9 -> 34.4, 513 tokens of 4096, 200 experts 23.5 -> 22.0, 8000 tokens 69.0 -> 69.7.
 constexpr int WW_HT = 256, WW_TC = 32;
 __global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__restrict__ x, const float *dlogits, int64_t T, int H,
                                                               int N, int64_t tokens_per_split, float *__restrict__ partial) {
@@ -224,7 +227,8 @@ __global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__
         fetch_d(2, 0);
         int slot = 0, free_slot = 2;
         auto step = [&](int s, int set) {         // set: the dlogits of step s + 1
-            // This wavefront's part of x of step s has landed: younger are the dlogits of steps s + 1 and s + 2 and x of s + 1.
+            // This wavefront's part of x of step s has landed: younger are at least the dlogits of step s + 1, which this step stores
+            // to LDS, and x of s + 1 (the dlogits of s + 2 too, but behind the last steps the compiler may leave out what nothing reads).
             // Behind the barrier everyone's has, the dlogits of step s are there, and step s - 1 has been read.
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XL + DL) : "memory");
             if ((s + 1) * WW_TC > tokens) {
@@ -254,10 +258,12 @@ __global__ __launch_bounds__(512) void gate_wgrad_wide_kernel(const uint16_t *__
             free_slot = slot;
             slot = slot == SLOTS - 1 ? 0 : slot + 1;
         };
-        for (int s = 0; s < steps; s += 2) {
+        int s = 0;
+        for (; s + 1 < steps; s += 2) {   // (where paths join, the compiler waits for every load in flight)
             step(s, 1);
-            if (s + 1 < steps) step(s + 1, 0);
+            step(s + 1, 0);
         }
+        if (s < steps) step(s, 1);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load into LDS outlives the block
     }
 #pragma unroll
