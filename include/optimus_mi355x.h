@@ -631,23 +631,25 @@ int om_grouped_gemm_wgrad_merged_accumulate(const void *dout, const int32_t *dou
                                             int64_t rows, int G, int I, int H, int64_t down_stride,
                                             int64_t gate_stride, int64_t up_stride, void *stream);
 
-/* The merged MLP of a float32 module (moe.py:396-405 and its autograd), the forms of the bf16 entry points
 /* `rows` known as a bound only: the choice of launches goes by expected_rows (0 <= expected_rows <= rows, as above). */
 int om_grouped_gemm_wgrad_merged_bound(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
-                                 const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
-                                 void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
-                                 int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t down_stride, int64_t gate_stride,
-                                 int64_t up_stride, void *stream);
+                                       const void *du, const void *x, const int32_t *x_rows, int64_t src_rows,
+                                       void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                       int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t down_stride,
+                                       int64_t gate_stride, int64_t up_stride, void *stream);
 int om_grouped_gemm_wgrad_merged_accumulate_bound(const void *dout, const int32_t *dout_rows, const void *h,
-                                            const void *dg, const void *du, const void *x,
-                                            const int32_t *x_rows, int64_t src_rows, void *dw_down,
-                                            void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
-                                            int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t down_stride,
-                                            int64_t gate_stride, int64_t up_stride, void *stream);
+                                                  const void *dg, const void *du, const void *x,
+                                                  const int32_t *x_rows, int64_t src_rows, void *dw_down,
+                                                  void *dw_gate, void *dw_up, const int32_t *cum_token_counts,
+                                                  int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                  int64_t down_stride, int64_t gate_stride, int64_t up_stride,
+                                                  void *stream);
+
+/* The merged MLP of a float32 module (moe.py:396-405 and its autograd), the forms of the bf16 entry points
  * above: gate and up in one launch with h = silu(g) * u formed in the epilogue, the SwiGLU backward in the
  * epilogue of dh = dy W_down, dx as one accumulation over both products, and both weight gradients in one
- * launch (`accumulate` bit 0: add into dw_gate, bit 1: into dw_up; gate before up where the two have memory in common).  x_rows (may be null): row r of x is row
- * x_rows[r] of a [src_rows, H] matrix.  I and H multiples of 8.                                             */
+ * launch (`accumulate` bit 0: add into dw_gate, bit 1: into dw_up; gate before up where the two have memory in
+ * common).  x_rows (may be null): row r of x is row x_rows[r] of a [src_rows, H] matrix.  I and H multiples of 8. */
 int om_merged_mlp_gate_up_fwd_f32(const float *x, const int32_t *x_rows, int64_t src_rows, const float *w_gate,
                                   const float *w_up, float *g, float *u, float *h, const int32_t *cum_token_counts,
                                   int64_t rows, int G, int I, int H, int64_t gate_stride, int64_t up_stride,
