@@ -337,7 +337,7 @@ def bench_other_configs(args, device, with_cpu, only=None):
             "graph_replay_ms_per_step": round(graph_ms, 4),
             "graph_replay_tokens_per_s": round(c["T"] / (graph_ms * 1e-3), 1),
             "workload": "C1 tiny MoE layer fwd+bwd (2048 tokens, hidden 256, 8 experts, top-2 renormalised, ffn 512), "
-                        "bf16 on the GPU; 17 launches, bound by enqueueing them "
+                        "bf16 on the GPU; 15 launches, bound by enqueueing them "
                         "(ms_per_step); graph_replay_* is the same step recorded once into a HIP graph"})
         if with_cpu:
             from oracle import moe_layer as L

@@ -180,12 +180,14 @@ int om_router_gate_logits_split(const void *x, const void *gate_weight, int64_t 
                                 void *stream);
 
 /* The whole router for a bf16 gate of any shape (N <= 256, H a multiple of 8): the projection split over
- * slices of H, then one launch that adds the slices in order, writes the logits and routes (both in one launch for
- * more than 512 tokens, at most 64 experts and an H that is a multiple of 512; the same bits).
+ * slices of H, then one launch that adds the slices in order, writes the logits and routes (the softmax router with at
+ * most 64 experts and an H that is a multiple of 512 also in one launch, the same bits: up to 16 selections with more than
+ * 512 tokens or an H below 1024, beyond 16 where the tokens fill the chip's rounds or are a few).
  *   om_router_gate_split_softmax_topk       : the softmax router above; logits_out in logits_dtype (OM_BF16:
  *       rounded to bf16 before the softmax, the logits of a bf16 linear layer)
  *   om_router_gate_split_sigmoid_group_topk : the DeepSeek-V3 router (om_route_sigmoid_group_topk below)
- * workspace: om_router_gate_route_workspace_bytes(T,H,N) bytes, 16-byte aligned (negative = error code). */
+ * workspace: om_router_gate_route_workspace_bytes(T,H,N) bytes, 16-byte aligned (negative = error code); asked for
+ *   whichever form the sizes and K lead to, one launch leaves it alone. */
 int64_t om_router_gate_route_workspace_bytes(int64_t T, int H, int N);
 int om_router_gate_split_softmax_topk(const void *x, const void *gate_weight, int64_t T, int H, int N, int K,
                                       int norm_topk_prob, void *logits_out, int logits_dtype, void *weights_out,

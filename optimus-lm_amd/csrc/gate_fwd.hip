@@ -1,15 +1,16 @@
-// Router gate projection for many experts, logits[t,n] = sum_h x[t,h] * W[n,h] in fp32 from bf16
+// Router gate projection split over slices of the hidden size, logits[t,n] = sum_h x[t,h] * W[n,h] in fp32 from bf16
 // operands (the DeepSeek-V3 router: optimus/models/deepseek_v3/modeling_deepseek_v3.py:160 casts
 // both operands to float32 and calls F.linear; bf16 x bf16 products are exact in fp32, so this is
 // that value up to the order of the sum).
 //
 // With a few hundred experts the gate weight is megabytes (256 x 7168 bf16 = 3.7 MB).  A block that
 // covers 32 tokens re-reads all of it from L2, and that traffic, not the read of x, bounds the
-// launch.  Here a block covers 128 tokens (four wavefronts of 32) and a slice of H; the weight tile
-// of a 64-wide step is fetched once per block into LDS with direct loads and shared by the four
-// wavefronts, the token fragments come straight from global memory in MFMA layout, and the slices
-// of H are added by a second kernel in slice order (deterministic).  Weight traffic falls by 4x,
-// the blocks still fill the chip through the split of H.
+// launch.  Here a block covers 128 tokens and a slice of H; the weight tile of a 64-wide step is
+// fetched once per block into LDS with direct loads and shared by its wavefronts, and the slices of
+// H are added by a second kernel (or the routing's) in slice order (deterministic).  Weight traffic
+// falls by 4x, the blocks still fill the chip through the split of H.
+// Up to 64 experts: gate_logits_split_kernel, four wavefronts of 32 tokens whose token fragments come
+// straight from global memory in MFMA layout, several blocks on a CU.  More: gate_logits_wide_kernel.
 #include "common.h"
 
 #include <algorithm>

@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         }
         strip_sync();
         if (EPI == EPI_SWIGLU_BWD) {
-            constexpr int GRP = 2;   // g and u in flight for half a strip: with all of it the 256x256 kernel spills
+            constexpr int GRP = 2;   // g and u in flight for half a strip: the 256x256 kernels spill 3 and 4 registers, with all of it 67 and 68
             u32x4 gq[GRP], uq[GRP];
             // ROWW: lane l fetches the weight of strip row l % 32 along with the g/u loads; the
             // lanes that work on a row pick it up with a lane read

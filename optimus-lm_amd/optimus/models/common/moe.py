@@ -398,7 +398,8 @@ def _expert_views(weight_tuple):
 class MergedMLPFunction(torch.autograd.Function):
     """y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment, with the fused kernels:
     gate+up+SwiGLU in one launch forward; backward = down dgrad fused with the SwiGLU backward,
-    one dual-operand dgrad for dx, and three weight-gradient GEMMs (float32: two launches for them).
+    one dual-operand dgrad for dx, and three weight-gradient GEMMs (in one launch where that is sooner; float32: in one
+    launch with the dgrad).
 
     Same mathematics as the three GroupedGemmFunction calls and two elementwise ops of the
     reference's MergedMLP.forward (moe.py:396-405) under autograd; g and u are kept in the module's
