@@ -1,7 +1,8 @@
-// Grouped expert GEMMs on bf16 MFMA (v_mfma_f32_32x32x16_bf16), fp32 accumulation.
+// Grouped expert GEMMs on bf16 MFMA (v_mfma_f32_16x16x32_bf16), fp32 accumulation.
 //
 // One kernel template covers every product of the merged MLP.  An output tile of 256x256 (8 wavefronts) or 128x128
-// (4) is worked by a grid of wavefronts two high; each has 32x32 MFMA accumulators in two columns.  Operands are
+// (4) is worked by a grid of wavefronts two high; each has 32 rows of a row unit and 64 columns, as 2 x 4 accumulators of
+// 16x16.  Operands are
 // staged through LDS in steps of 64 along the contraction index c with direct global->LDS loads
 // (global_load_lds_dwordx4: no register staging, no ds_write), two stages.
 //
@@ -19,7 +20,7 @@
 // them, they have 0.6 to 0.9 of a step, and a step of the 256x256 tile took 1.5 us at full clock where its MFMAs take
 // 0.85; the 128x128 kernels, two blocks per CU, spent three quarters of their time waiting.  So a step's buffers are
 // given back piecemeal.  A wavefront keeps all of its B fragments of a step in registers (64 c x 64 columns) and works
-// through the row units of A one after the other (a phase: 8 MFMAs); it reads the fragments of the next phase, and in
+// through the row units of A one after the other (a phase: 16 MFMAs); it reads the fragments of the next phase, and in
 // the later phases B of the next step, under the MFMAs of this one.  Two barriers a step, P in the middle and Q at its
 // end, separate three groups of loads:
 //   after Q(t-1)  B of step t was read during step t-1, as was A's first unit: both are loaded for step t+2, and
@@ -33,6 +34,12 @@
 // 64 experts of 2048/1024, 112.7 -> 104.4 and 57.0 -> 50.8 (that loop with its operands staged through registers two
 // steps ahead); 32 experts of 7168/2048 with 0 to 2849 rows (256x256): gate+up 967 -> 859, gate/up input gradient 959
 // -> 886; 64 experts of 2048/1024 with 2048 rows, where the power limit sets the rate, 1020 -> 1004 and 521 -> 518.
+//
+// The 16x16x32 instruction takes less energy per operation than 32x32x16 (alone, random operands, under the power limit
+// 2.00 against 1.77 PFLOP/s), which is what the large launches are bound by; fragments and accumulators take as many
+// registers, and the sums are the same bits.  Whole passes, us, 32x32x16 -> 16x16x32: 64 experts of 2048/1024, forward of
+// 4096 tokens 522 -> 509, training step of 16384 5344 -> 5287; 32 experts of 7168/2048 and a shared one, 8192 tokens
+// 6169 -> 6005.
 //
 // A tile's rows are worked in units of 64 (32 per wavefront row), and units past the expert's last row cost no MFMA.
 //
@@ -127,12 +134,12 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-// CONTIG unit (64 rows x 64 c, 128-byte rows): chunk position = chunk ^ swz(row), measured conflict-free for
-// ds_read_b128 with 32 consecutive rows per half-wave; period 16, so rows 32 apart share it.
+// CONTIG unit (64 rows x 64 c, 128-byte rows): chunk position = chunk ^ swz(row), conflict-free for ds_read_b128, whose
+// lanes are served sixteen at a time, with 16 consecutive rows; period 16, so rows 16 apart share it.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
-// STRIDED unit (64 c-rows x 64 columns, 128-byte c-rows): the four c-rows of a transposing read, two of which share a
-// 256-byte bank row, land in four different 64-byte windows
-__device__ __forceinline__ int unit_swz(int crow) { return ((crow >> 1) & 1) << 2; }
+// STRIDED unit (64 c-rows x 64 columns, 128-byte c-rows): a transposing read takes 32 bytes of four c-rows for every 16
+// lanes, of c-rows 8 apart for the next 16; the eight pieces land in eight different 32-byte windows of the banks
+__device__ __forceinline__ int unit_swz(int crow) { return (((crow >> 1) & 1) << 2) | (((crow >> 3) & 1) << 1); }
 
 __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
     typedef __attribute__((ext_vector_type(2))) float f32x2;
@@ -668,28 +675,28 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
 
     // ---- fragments --------------------------------------------------------------------------------
-    int a_frag[AKIND == CONTIG ? 4 : 1], b_frag[BKIND == CONTIG ? 4 : 2];   // byte addresses within a unit region
+    int a_frag[2], b_frag[BKIND == CONTIG ? 2 : 4];   // byte addresses within a unit region: CONTIG by kk, STRIDED by block
     auto set_fragments = [&]() {
         int lane_f = lane;
         asm volatile("" : "+v"(lane_f));   // recomputed per tile, not kept across the epilogue
-        const int lrow32 = lane_f & 31, g2 = lane_f >> 5;
-        const int q16 = lane_f & 3, r16 = (lane_f & 15) >> 2, mb = ((lane_f >> 4) & 1) * 16;
-        const int cr = 8 * g2 + r16;
-        if (AKIND == CONTIG) {
+        const int l16 = lane_f & 15, g4 = lane_f >> 4;
+        const int q16 = lane_f & 3, cr = 8 * g4 + (l16 >> 2);
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) a_frag[AKIND == CONTIG ? kk : 0] = (wm * 32 + lrow32) * 128 + (((kk * 2 + g2) ^ swz(lrow32)) << 4);
-        } else {
-            const int m = wm * 32 + mb + 4 * q16;
-            a_frag[0] = cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
+        for (int x = 0; x < 2; x++) {
+            if (AKIND == CONTIG) {
+                a_frag[x] = (wm * 32 + l16) * 128 + (((x * 4 + g4) ^ swz(l16)) << 4);
+            } else {
+                const int m = wm * 32 + x * 16 + 4 * q16;
+                a_frag[x] = cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
+            }
         }
-        if (BKIND == CONTIG) {
 #pragma unroll
-            for (int kk = 0; kk < 4; kk++) b_frag[BKIND == CONTIG ? kk : 0] = B0 + wn * UNIT + lrow32 * 128 + (((kk * 2 + g2) ^ swz(lrow32)) << 4);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int m = j * 32 + mb + 4 * q16;
-                b_frag[j] = B0 + wn * UNIT + cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
+        for (int x = 0; x < (BKIND == CONTIG ? 2 : 4); x++) {
+            if (BKIND == CONTIG) {
+                b_frag[x] = B0 + wn * UNIT + l16 * 128 + (((x * 4 + g4) ^ swz(l16)) << 4);
+            } else {
+                const int m = x * 16 + 4 * q16;
+                b_frag[x] = B0 + wn * UNIT + cr * 128 + (((m >> 3) ^ unit_swz(cr)) << 4) + (m & 7) * 2;
             }
         }
     };
@@ -699,34 +706,38 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(q + 4 * 128));
         return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    bf16x8 fa[2][4], fb[2][TN][4];
-    f32x16 acc[TM][TN];
+    bf16x8 fa[2][2][2], fb[2][4][2];   // [..][16-row block][32 indices]
+    f32x4 acc[TM][2][4];
     auto read_a = [&](auto par, auto unit) {
         constexpr int O = decltype(par)::value * A_STAGE + decltype(unit)::value * UNIT, buf = decltype(unit)::value & 1;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            if (AKIND == CONTIG) fa[buf][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + a_frag[AKIND == CONTIG ? kk : 0] + O));
-            else fa[buf][kk] = read_tr(lds + a_frag[0] + O + kk * 2048);
-        }
+        for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                if (AKIND == CONTIG) fa[buf][i][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + a_frag[kk] + O + i * 2048));
+                else fa[buf][i][kk] = read_tr(lds + a_frag[i] + O + kk * 4096);
+            }
     };
     auto read_b = [&](auto par, auto k_lo, auto k_hi) {
         constexpr int P = decltype(par)::value, O = P * B_STAGE;
 #pragma unroll
         for (int kk = decltype(k_lo)::value; kk < decltype(k_hi)::value; kk++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) {
-                if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 4096));
-                else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 2048);
+            for (int j = 0; j < 4; j++) {
+                if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 2048));
+                else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 4096);
             }
     };
     auto multiply = [&](auto par, auto unit) {
         constexpr int P = decltype(par)::value, I = decltype(unit)::value;
 #pragma unroll
-        for (int kk = 0; kk < 4; kk++)
+        for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-                // operands swapped: the lane then holds 4 consecutive output columns per row
-                acc[I][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[P][j][kk], fa[I & 1][kk], acc[I][j], 0, 0, 0);
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    // operands swapped: the lane then holds 4 consecutive output columns per row
+                    acc[I][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[P][j][kk], fa[I & 1][i][kk], acc[I][i][j], 0, 0, 0);
     };
     // one MFMA, then the LDS reads of the next phase behind the leading MFMAs, the rest of the MFMAs last
     auto schedule = [&](auto reads) {
@@ -734,7 +745,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         int left = R;
 #pragma unroll
         for (int m = 0; m < 8; m++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 #pragma unroll
             for (int q = 0; q < PER; q++)
                 if (left > 0) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); left--; }
@@ -783,7 +794,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         }
         return false;
     };
-    constexpr IntC<0> c0_{}; constexpr IntC<1> c1_{}; constexpr IntC<2> c2_{}; constexpr IntC<3> c3_{}; constexpr IntC<4> c4_{};
+    constexpr IntC<0> c0_{}; constexpr IntC<1> c1_{}; constexpr IntC<2> c2_{}; constexpr IntC<3> c3_{};
     // step 0 of a tile, all of it
     auto prefetch = [&]() {
         if (n_steps == 0) return;
@@ -800,9 +811,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+        for (int j = 0; j < 8; j++) acc[i][j >> 2][j & 3] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     if (n_steps > 0) {
         // c0 and operand addresses of the steps t + 1 and t + 2 (t: the step being multiplied)
@@ -832,7 +841,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
                 issue_a(left, pa2, cs2, same, c1_, s2);
                 read_a(other, c0_);
-                read_b(other, c0_, c4_);
+                read_b(other, c0_, c2_);
                 if (FULL || active > 1) multiply(same, c1_);
                 schedule(IntC<RA + RB>{});
                 wait_step_loads<8, 0>(left, lds_addr);
@@ -861,13 +870,13 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
                 issue_a(left, pa2, cs2, same, c1_, s2);
                 read_a(same, c3_);
-                read_b(other, c0_, c2_);
+                read_b(other, c0_, c1_);
                 if (FULL || active > 2) multiply(same, c2_);
                 schedule(IntC<RA + RB / 2>{});
                 // phase 3
                 issue_a(left, pa2, cs2, same, c2_, s2);
                 read_a(other, c0_);
-                read_b(other, c2_, c4_);
+                read_b(other, c1_, c2_);
                 if (FULL || active > 3) multiply(same, c3_);
                 schedule(IntC<RA + RB / 2>{});
                 wait_step_loads<8, 1>(left, lds_addr);
@@ -903,7 +912,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         block_barrier();
         set_fragments();
         read_a(c0_, c0_);
-        read_b(c0_, c0_, c4_);
+        read_b(c0_, c0_, c2_);
         block_barrier();   // (their buffers are the first that step 0 loads into)
         auto loop = [&](auto full) {
             for (int t = 0; t < n_steps; t += 2) {
@@ -952,15 +961,15 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     static_assert(NW / 2 * NSTRIP * STRIP <= A_STAGE && NW / 2 * NSTRIP * STRIP <= B_STAGE, "strips must fit beside the even steps' buffers");
     const int wm_e = wave_e / WAVES_N, wn_e = wave_e % WAVES_N;
     char *strip = lds + (wave_e < NW / 2 ? A_STAGE : B0 + B_STAGE) + (wave_e % (NW / 2)) * (NSTRIP * STRIP);
-    const int lrow = lane_e & 31;
-    const int lcol = (lane_e >> 5) * 4;
+    const int lrow = lane_e & 15;
+    const int lcol = (lane_e >> 4) * 4;
     constexpr int CPRW = COLS / 8;            // 16-byte chunks per strip row
     constexpr int ITS = 32 * CPRW / 64;       // chunks per lane per strip
-    auto strip_put = [&](int which, int col, float v0, float v1, float v2, float v3) {
+    auto strip_put = [&](int which, int row, int col, f32x4 f) {   // (of a 16x16 block)
         u32x2 v;
-        v[0] = pack2_bf16(v0, v1);
-        v[1] = pack2_bf16(v2, v3);
-        *reinterpret_cast<u32x2 *>(strip + which * STRIP + lrow * PITCH + col * 2) = v;
+        v[0] = pack2_bf16(f[0], f[1]);
+        v[1] = pack2_bf16(f[2], f[3]);
+        *reinterpret_cast<u32x2 *>(strip + which * STRIP + (row + lrow) * PITCH + (col + lcol) * 2) = v;
     };
     auto strip_get = [&](int which, int row, int cc) -> u32x4 {
         const char *q = strip + which * STRIP + row * PITCH + cc * 16;
@@ -975,11 +984,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     const int col0 = e_n0 + wn_e * COLS;   // first output column
     const int row_lim = EDGE && col0 + (lane_e % (COLS / 8)) * 8 >= e_n_cols ? 0 : e_row_end;
-    float wrow_all[(ROWW && EPI == EPI_SWIGLU) ? TM : 1];
+    float wrow_all[(ROWW && EPI == EPI_SWIGLU) ? 2 * TM : 1];
     if (ROWW && EPI == EPI_SWIGLU) {
 #pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int64_t m = static_cast<int64_t>(e_row_begin) + (2 * i + wm_e) * 32 + lrow;
+        for (int i = 0; i < 2 * TM; i++) {
+            const int64_t m = static_cast<int64_t>(e_row_begin) + ((i & ~1) + wm_e) * 32 + (i & 1) * 16 + lrow;
             wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0] = (m < e_row_end) ? p.row_scale[m] : 0.0f;
         }
     }
@@ -989,32 +998,28 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         const int64_t m0 = static_cast<int64_t>(e_row_begin) + (2 * i + wm_e) * 32;  // first row of the strip
         u32x4 *old_out = old[ACCUM ? i : 0];
         if (EPI == EPI_SWIGLU) {
-            const float wrow = wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0];   // ROWW: h = w[row] * silu(g) * u, one rounding
 #pragma unroll
-            for (int rq = 0; rq < 4; rq++) {
-                float hv[4];
+            for (int b = 0; b < 4; b++) {
+                const int half = b >> 1, j = b & 1;
+                const float wrow = wrow_all[(ROWW && EPI == EPI_SWIGLU) ? 2 * i + half : 0];   // ROWW: h = w[row] * silu(g) * u, one rounding
+                const f32x4 gv = acc[i][half][j], uv = acc[i][half][2 + j];
+                f32x4 hv;
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
-                    const float gv = acc[i][0][rq * 4 + x], uv = acc[i][1][rq * 4 + x];
-                    hv[x] = (gv * fast_sigmoid(gv)) * uv;
+                    hv[x] = (gv[x] * fast_sigmoid(gv[x])) * uv[x];
                     if (ROWW) hv[x] *= wrow;
                 }
-                const int col = rq * 8 + lcol;
-                strip_put(0, col, acc[i][0][rq * 4], acc[i][0][rq * 4 + 1], acc[i][0][rq * 4 + 2], acc[i][0][rq * 4 + 3]);
-                strip_put(1, col, acc[i][1][rq * 4], acc[i][1][rq * 4 + 1], acc[i][1][rq * 4 + 2], acc[i][1][rq * 4 + 3]);
-                strip_put(2, col, hv[0], hv[1], hv[2], hv[3]);
+                strip_put(0, half * 16, j * 16, gv);
+                strip_put(1, half * 16, j * 16, uv);
+                strip_put(2, half * 16, j * 16, hv);
             }
         } else {
 #pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int rq = 0; rq < 4; rq++)
-                    strip_put(0, j * 32 + rq * 8 + lcol, acc[i][j][rq * 4], acc[i][j][rq * 4 + 1],
-                              acc[i][j][rq * 4 + 2], acc[i][j][rq * 4 + 3]);
+            for (int b = 0; b < 8; b++) strip_put(0, (b >> 2) * 16, (b & 3) * 16, acc[i][b >> 2][b & 3]);
         }
         strip_sync();
         if (EPI == EPI_SWIGLU_BWD) {
-            constexpr int GRP = 2;   // g and u in flight for half a strip: the 256x256 kernels spill 3 and 4 registers, with all of it 67 and 68
+            constexpr int GRP = 2;   // g and u in flight for half a strip: the 256x256 kernels spill 7 and 8 registers
             u32x4 gq[GRP], uq[GRP];
             // ROWW: lane l fetches the weight of strip row l % 32 along with the g/u loads; the
             // lanes that work on a row pick it up with a lane read
