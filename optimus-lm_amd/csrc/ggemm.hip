@@ -22,13 +22,18 @@
 // given back piecemeal.  A wavefront keeps all of its B fragments of a step in registers (64 c x 64 columns) and works
 // through the row units of A one after the other (a phase: 16 MFMAs); it reads the fragments of the next phase, and in
 // the later phases B of the next step, under the MFMAs of this one.  Two barriers a step, P in the middle and Q at its
-// end, separate three groups of loads:
-//   after Q(t-1)  B of step t was read during step t-1, as was A's first unit: both are loaded for step t+2, and
-//                 (256x256) A's last unit, free since Q(t-1), for step t+1;
-//   after P(t)    A's remaining units of step t are free: loaded for step t+2.
-// A wavefront passes P and Q once all but its 8 youngest loads have landed (a whole step's worth), so every load has 1
-// to 1.5 steps.  The waits are written as assembly, and so are the loads: with the builtin the compiler waits for every
-// load in flight before a barrier, since it cannot tell which LDS bytes they will write.
+// end, give the buffers back:
+//   after Q(t-1)  B of step t was read during step t-1, as was A's first unit: both are free for step t+2, and
+//                 (256x256) A's last unit for step t+1;
+//   after P(t)    A's remaining units of step t are free for step t+2.
+// The loads go out evenly, one for every eight MFMAs (256x256; 128x128 two): eight wavefronts that issue three each at once
+// wait for one another's addresses, and the matrix cores for them.  A wavefront passes P (Q) once all but its 6 (8) youngest
+// loads have landed, so every load has 1 to 1.5 steps.  The waits are written as assembly, and so are the loads: with the
+// builtin the compiler waits for every load in flight before a barrier, since it cannot tell which LDS bytes they will write.
+// Loads at a phase's start, six of a step's eight after Q -> evenly, us: 64 experts of 2048/1024 with 2048 rows, gate+up 950 ->
+// 916, down 493 -> 477, gate/up input gradient 907 -> 883, weight gradients 1465 -> 1446 (added 1583 -> 1545); with 512 rows
+// gate/up input gradient 250 -> 239; 32 experts of 7168/2048, 400 uneven rows, gate+up 847 -> 829, gate/up input gradient 829 ->
+// 805.  (At full clock, on operands of zeros, one product of 8192^3 is slower: 700 -> 757.)
 // Measured on one box against the single-barrier loop, us: 3001 tokens, hidden 1000, ffn 712, 12 experts, top-3
 // (128x128): down 32.6 -> 28.6, gate/up input gradient 55.7 -> 46.8, weight gradients 34 -> 31; decode of 37 tokens,
 // 64 experts of 2048/1024, 112.7 -> 104.4 and 57.0 -> 50.8 (that loop with its operands staged through registers two
@@ -708,30 +713,28 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     bf16x8 fa[2][2][2], fb[2][4][2];   // [..][16-row block][32 indices]
     f32x4 acc[TM][2][4];
-    auto read_a = [&](auto par, auto unit) {
+    auto read_a = [&](auto par, auto unit, auto k_lo, auto k_hi) {
         constexpr int O = decltype(par)::value * A_STAGE + decltype(unit)::value * UNIT, buf = decltype(unit)::value & 1;
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++)
+        for (int kk = decltype(k_lo)::value; kk < decltype(k_hi)::value; kk++)
 #pragma unroll
             for (int i = 0; i < 2; i++) {
                 if (AKIND == CONTIG) fa[buf][i][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + a_frag[kk] + O + i * 2048));
                 else fa[buf][i][kk] = read_tr(lds + a_frag[i] + O + kk * 4096);
             }
     };
-    auto read_b = [&](auto par, auto k_lo, auto k_hi) {
+    // fragments f_lo .. f_hi of the eight (four of every 32 indices)
+    auto read_b = [&](auto par, auto f_lo, auto f_hi) {
         constexpr int P = decltype(par)::value, O = P * B_STAGE;
 #pragma unroll
-        for (int kk = decltype(k_lo)::value; kk < decltype(k_hi)::value; kk++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
+            for (int f = decltype(f_lo)::value; f < decltype(f_hi)::value; f++) {
+                const int kk = f >> 2, j = f & 3;
                 if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 2048));
                 else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 4096);
             }
     };
-    auto multiply = [&](auto par, auto unit) {
-        constexpr int P = decltype(par)::value, I = decltype(unit)::value;
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++)
+    auto multiply = [&](auto par, auto unit, auto k) {
+        constexpr int P = decltype(par)::value, I = decltype(unit)::value, kk = decltype(k)::value;
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
@@ -745,7 +748,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         int left = R;
 #pragma unroll
         for (int m = 0; m < 8; m++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
 #pragma unroll
             for (int q = 0; q < PER; q++)
                 if (left > 0) { __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); left--; }
@@ -795,6 +798,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         return false;
     };
     constexpr IntC<0> c0_{}; constexpr IntC<1> c1_{}; constexpr IntC<2> c2_{}; constexpr IntC<3> c3_{};
+    constexpr IntC<4> c4_{}; constexpr IntC<6> c6_{}; constexpr IntC<8> c8_{};
     // step 0 of a tile, all of it
     auto prefetch = [&]() {
         if (n_steps == 0) return;
@@ -828,57 +832,79 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             const int (&s2)[L] = src[GATHER_W ? 2 : 0];
             int src3[L] = {};   // source rows of step t + 3
             const int cs3 = next_c0(cs2);
+            constexpr IntC<RA / 2> ra{}; constexpr IntC<RA / 2 + RB / (TM == 2 ? 2 : 4)> rab{};
             if constexpr (TM == 2) {
                 issue_b(left, pb2, cs2, same, c0_, s2);
+                read_a(same, c1_, c0_, c1_);
+                multiply(same, c0_, c0_);
+                schedule(ra);
                 issue_b(left, pb2, cs2, same, c1_, s2);
-                issue_a(left, pa2, cs2, same, c0_, s2);
-                read_a(same, c1_);
-                multiply(same, c0_);
-                schedule(IntC<RA>{});
-                wait_step_loads<8, 2>(left, lds_addr);
+                read_a(same, c1_, c1_, c2_);
+                multiply(same, c0_, c1_);
+                schedule(ra);
+                wait_step_loads<6, 2>(left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 block_barrier();
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
+                issue_a(left, pa2, cs2, same, c0_, s2);
+                read_a(other, c0_, c0_, c1_);
+                read_b(other, c0_, c4_);
+                if (FULL || active > 1) multiply(same, c1_, c0_);
+                schedule(rab);
                 issue_a(left, pa2, cs2, same, c1_, s2);
-                read_a(other, c0_);
-                read_b(other, c0_, c2_);
-                if (FULL || active > 1) multiply(same, c1_);
-                schedule(IntC<RA + RB>{});
+                read_a(other, c0_, c1_, c2_);
+                read_b(other, c4_, c8_);
+                if (FULL || active > 1) multiply(same, c1_, c1_);
+                schedule(rab);
                 wait_step_loads<8, 0>(left, lds_addr);
                 zero_tail(cs1, other, c1_);
                 block_barrier();
             } else {
                 // phase 0
-                issue_b(left, pb2, cs2, same, c0_, s2);
-                issue_b(left, pb2, cs2, same, c1_, s2);
-                issue_a(left, pa2, cs2, same, c0_, s2);
-                read_a(same, c1_);
-                multiply(same, c0_);
-                schedule(IntC<RA>{});
-                // phase 1
-                issue_b(left, pb2, cs2, same, c2_, s2);
-                issue_b(left, pb2, cs2, same, c3_, s2);
                 issue_a(left + 1, pa1, cs1, other, c3_, src[GATHER_W ? 1 : 0]);
-                read_a(same, c2_);
-                if (FULL || active > 1) multiply(same, c1_);
-                schedule(IntC<RA>{});
-                wait_step_loads<8, 3>(left, lds_addr);
+                read_a(same, c1_, c0_, c1_);
+                multiply(same, c0_, c0_);
+                schedule(ra);
+                issue_b(left, pb2, cs2, same, c0_, s2);
+                read_a(same, c1_, c1_, c2_);
+                multiply(same, c0_, c1_);
+                schedule(ra);
+                // phase 1
+                issue_b(left, pb2, cs2, same, c1_, s2);
+                read_a(same, c2_, c0_, c1_);
+                if (FULL || active > 1) multiply(same, c1_, c0_);
+                schedule(ra);
+                issue_b(left, pb2, cs2, same, c2_, s2);
+                read_a(same, c2_, c1_, c2_);
+                if (FULL || active > 1) multiply(same, c1_, c1_);
+                schedule(ra);
+                wait_step_loads<6, 3>(left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 zero_tail(cst, same, c3_);
                 block_barrier();
                 // phase 2
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
-                issue_a(left, pa2, cs2, same, c1_, s2);
-                read_a(same, c3_);
-                read_b(other, c0_, c1_);
-                if (FULL || active > 2) multiply(same, c2_);
-                schedule(IntC<RA + RB / 2>{});
+                issue_b(left, pb2, cs2, same, c3_, s2);
+                read_a(same, c3_, c0_, c1_);
+                read_b(other, c0_, c2_);
+                if (FULL || active > 2) multiply(same, c2_, c0_);
+                schedule(rab);
+                issue_a(left, pa2, cs2, same, c0_, s2);
+                read_a(same, c3_, c1_, c2_);
+                read_b(other, c2_, c4_);
+                if (FULL || active > 2) multiply(same, c2_, c1_);
+                schedule(rab);
                 // phase 3
+                issue_a(left, pa2, cs2, same, c1_, s2);
+                read_a(other, c0_, c0_, c1_);
+                read_b(other, c4_, c6_);
+                if (FULL || active > 3) multiply(same, c3_, c0_);
+                schedule(rab);
                 issue_a(left, pa2, cs2, same, c2_, s2);
-                read_a(other, c0_);
-                read_b(other, c1_, c2_);
-                if (FULL || active > 3) multiply(same, c3_);
-                schedule(IntC<RA + RB / 2>{});
+                read_a(other, c0_, c1_, c2_);
+                read_b(other, c6_, c8_);
+                if (FULL || active > 3) multiply(same, c3_, c1_);
+                schedule(rab);
                 wait_step_loads<8, 1>(left, lds_addr);
                 zero_tail(cs1, other, c1_);
                 zero_tail(cs1, other, c2_);
@@ -911,8 +937,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         if constexpr (TM == 4) { zero_tail(cs0, c0_, c2_); zero_tail(cs0, c0_, c3_); }
         block_barrier();
         set_fragments();
-        read_a(c0_, c0_);
-        read_b(c0_, c0_, c2_);
+        read_a(c0_, c0_, c0_, c2_);
+        read_b(c0_, c0_, c8_);
         block_barrier();   // (their buffers are the first that step 0 loads into)
         auto loop = [&](auto full) {
             for (int t = 0; t < n_steps; t += 2) {
