@@ -26,8 +26,9 @@
 //   after Q(t-1)  B of step t was read during step t-1, as was A's first unit: both are free for step t+2, and
 //                 (256x256) A's last unit for step t+1;
 //   after P(t)    A's remaining units of step t are free for step t+2.
-// The loads go out evenly, one for every eight MFMAs (256x256; 128x128 two): eight wavefronts that issue three each at once
-// wait for one another's addresses, and the matrix cores for them.  A wavefront passes P (Q) once all but its 6 (8) youngest
+// 256x256: the loads go out evenly, one for every eight MFMAs: eight wavefronts that issue three each at once wait for one
+// another's addresses, and the matrix cores for them.  (128x128: as soon as a buffer is free; few rows wait for weights, and
+// evenly a decode batch of 37 took 155 us instead of 150.)  A wavefront passes P (Q) once all but its 6 (8; 128x128 8) youngest
 // loads have landed, so every load has 1 to 1.5 steps.  The waits are written as assembly, and so are the loads: with the
 // builtin the compiler waits for every load in flight before a barrier, since it cannot tell which LDS bytes they will write.
 // Loads at a phase's start, six of a step's eight after Q -> evenly, us: 64 experts of 2048/1024 with 2048 rows, gate+up 950 ->
@@ -153,25 +154,15 @@ __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, h);
 }
 
-// Sum over aligned groups of N neighbouring lanes (N = 4, 8 or 16); every lane of the group gets
-// it.  DPP: swap within pairs, swap pairs within quads, mirror within 8, mirror within 16.
+// Sum over aligned groups of eight neighbouring lanes; every lane of the group gets it.  DPP: swap within pairs, swap
+// pairs within quads, mirror within 8.
 template <int CTRL> __device__ __forceinline__ float dpp_move(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
-template <int N> __device__ __forceinline__ float lane_group_sum(float v) {
-    static_assert(N == 4 || N == 8 || N == 16, "group size");
+__device__ __forceinline__ float eight_lanes_sum(float v) {
     v += dpp_move<0xB1>(v);
     v += dpp_move<0x4E>(v);
-    if (N >= 8) v += dpp_move<0x141>(v);
-    if (N >= 16) v += dpp_move<0x140>(v);
-    return v;
-}
-
-__device__ __forceinline__ void unpack4_bf16(u32x2 v, float *f) {
-    f[0] = __uint_as_float(v[0] << 16);
-    f[1] = __uint_as_float(v[0] & 0xffff0000u);
-    f[2] = __uint_as_float(v[1] << 16);
-    f[3] = __uint_as_float(v[1] & 0xffff0000u);
+    return v + dpp_move<0x141>(v);
 }
 
 // Row tiles of fwd/dgrad are cut per expert (BM rows each, the last one of an expert partial).
@@ -388,9 +379,11 @@ __device__ __forceinline__ void dma16_if_once(int left, int once, const void *ba
 template <int N> __device__ __forceinline__ void wait_loads(uint32_t lds) {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N), "s"(lds) : "memory");
 }
-// The same inside a tile's main loop, by the number of steps that follow: N2 with two or more, N1 with one, else 0.
+// The same inside a tile's main loop, by the number of steps that follow: N2 with two or more, N1 with one, 0 with none;
+// no load is waited for with a negative number.
 template <int N2, int N1> __device__ __forceinline__ void wait_step_loads(int left, uint32_t lds) {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_cmp_ge_i32 %2, 2\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(%1)\n\t"
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_cmp_lt_i32 %2, 0\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(%0)\n\t"
+                 "s_cmp_ge_i32 %2, 2\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(%1)\n\t"
                  "s_cmp_ge_i32 %2, 1\n\ts_cbranch_scc1 .Lom_wait%=\n\ts_waitcnt vmcnt(0)\n.Lom_wait%=:"
                  :: "n"(N2), "n"(N1), "s"(left), "s"(lds) : "memory", "scc");
 }
@@ -799,7 +792,22 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     constexpr IntC<0> c0_{}; constexpr IntC<1> c1_{}; constexpr IntC<2> c2_{}; constexpr IntC<3> c3_{};
     constexpr IntC<4> c4_{}; constexpr IntC<6> c6_{}; constexpr IntC<8> c8_{};
-    // step 0 of a tile, all of it
+    // Step 0 of a tile, and (second) of step 1 what does not go where the strips of the epilogue lie (A's last units).
+    // EARLY: both are loaded ahead of the epilogue's stores, and the tile's first step does not wait for those: the memory
+    // counter runs in order, so before this a tile began when the last one's 128 KB had been accepted.  Weight gradients
+    // alone, us: 64 experts of 2048/1024, 512 tokens, uneven 200 -> 180 (the pass 603 -> 599, bound by what memory takes),
+    // 16384 tokens 1447 -> 1415; 32 experts of 7168/2048, 400 uneven rows, 1364 -> 1314, added 1814 -> 1783.  The row products,
+    // with more steps to a tile, gain nothing by it (1 % slower in gate+up of 512 rows).
+    constexpr int FIRST = 6;                  // loads of step 1 in second()
+    constexpr bool EARLY = WGRAD;
+    auto second = [&]() {
+        if (n_steps == 1) return;
+        const int c1 = next_c0(rot * BK);
+        const char *qa1 = a_step(c1, 1), *qb1 = b_step(c1, 1);
+        issue_b_all(qb1, c1, c1_, src[GATHER_W ? 1 : 0]);
+        issue_a(2, qa1, c1, c1_, c0_, src[GATHER_W ? 1 : 0]);
+        if constexpr (TM == 4) issue_a(2, qa1, c1, c1_, c1_, src[GATHER_W ? 1 : 0]);
+    };
     auto prefetch = [&]() {
         if (n_steps == 0) return;
         const int c0 = rot * BK;
@@ -808,7 +816,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         issue_a(2, qa, c0, c0_, c0_, src[0]);
         issue_a(2, qa, c0, c0_, c1_, src[0]);
         if constexpr (TM == 4) { issue_a(2, qa, c0, c0_, c2_, src[0]); issue_a(2, qa, c0, c0_, c3_, src[0]); }
+        if (EARLY) second();
     };
+    // 16-byte stores that a wavefront makes at least for a tile all of whose rows exist: they follow the next tile's prefetch,
+    // and its first step does not wait for them
+    constexpr int STORES = EDGE || !EARLY ? 0 : 16;
+    bool stores_follow = false;
     bool have = next_tile();
     if (have) prefetch();
     while (have) {
@@ -822,6 +835,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         const int cs0 = rot * BK;
         int cs1 = next_c0(cs0), cs2 = next_c0(cs1), cst = cs0;
         const char *pa1 = a_step(cs1, 1), *pa2 = a_step(cs2, 2), *pb2 = b_step(cs2, 2);
+        // steps that follow step 0, for the wait in its middle: nothing to wait for where all that it needs is here
+        const int left0 = __builtin_amdgcn_readfirstlane((STORES && stores_follow) || n_steps == 1 ? -1 : n_steps - 1);
         // One contraction step of parity P (see the comment above the kernel).  Past the last step nothing is loaded, and
         // what is read for it is not used.
         auto step = [&](auto par, auto full, int t) {
@@ -835,28 +850,28 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             constexpr IntC<RA / 2> ra{}; constexpr IntC<RA / 2 + RB / (TM == 2 ? 2 : 4)> rab{};
             if constexpr (TM == 2) {
                 issue_b(left, pb2, cs2, same, c0_, s2);
+                issue_b(left, pb2, cs2, same, c1_, s2);
+                issue_a(left, pa2, cs2, same, c0_, s2);
                 read_a(same, c1_, c0_, c1_);
                 multiply(same, c0_, c0_);
                 schedule(ra);
-                issue_b(left, pb2, cs2, same, c1_, s2);
                 read_a(same, c1_, c1_, c2_);
                 multiply(same, c0_, c1_);
                 schedule(ra);
-                wait_step_loads<6, 2>(left, lds_addr);
+                wait_step_loads<8, 2>(t == 0 ? left0 : left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 block_barrier();
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
-                issue_a(left, pa2, cs2, same, c0_, s2);
+                issue_a(left, pa2, cs2, same, c1_, s2);
                 read_a(other, c0_, c0_, c1_);
                 read_b(other, c0_, c4_);
                 if (FULL || active > 1) multiply(same, c1_, c0_);
                 schedule(rab);
-                issue_a(left, pa2, cs2, same, c1_, s2);
                 read_a(other, c0_, c1_, c2_);
                 read_b(other, c4_, c8_);
                 if (FULL || active > 1) multiply(same, c1_, c1_);
                 schedule(rab);
-                wait_step_loads<8, 0>(left, lds_addr);
+                wait_step_loads<8, 0>(left - (left == 0), lds_addr);
                 zero_tail(cs1, other, c1_);
                 block_barrier();
             } else {
@@ -878,7 +893,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 read_a(same, c2_, c1_, c2_);
                 if (FULL || active > 1) multiply(same, c1_, c1_);
                 schedule(ra);
-                wait_step_loads<6, 3>(left, lds_addr);
+                wait_step_loads<6, 3>(t == 0 ? left0 : left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 zero_tail(cst, same, c3_);
                 block_barrier();
@@ -905,7 +920,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 read_b(other, c6_, c8_);
                 if (FULL || active > 3) multiply(same, c3_, c1_);
                 schedule(rab);
-                wait_step_loads<8, 1>(left, lds_addr);
+                wait_step_loads<8, 1>(left - (left == 0), lds_addr);
                 zero_tail(cs1, other, c1_);
                 zero_tail(cs1, other, c2_);
                 block_barrier();
@@ -921,21 +936,15 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             pa2 = a_step(cs2, t + 3);
             pb2 = b_step(cs2, t + 3);
         };
-        // the units of step 1 that the loop does not load itself
-        if (n_steps > 1) {
-            const char *pb1 = b_step(cs1, 1);
-            issue_b_all(pb1, cs1, c1_, src[GATHER_W ? 1 : 0]);
-            issue_a(2, pa1, cs1, c1_, c0_, src[GATHER_W ? 1 : 0]);
-            issue_a(2, pa1, cs1, c1_, c1_, src[GATHER_W ? 1 : 0]);
-            if constexpr (TM == 4) { issue_a(2, pa1, cs1, c1_, c2_, src[GATHER_W ? 1 : 0]); wait_loads<7>(lds_addr); }
-            else wait_loads<8>(lds_addr);
-        } else {
-            wait_loads<0>(lds_addr);
-        }
+        if (!EARLY) second();
+        if (STORES && stores_follow) wait_loads<STORES>(lds_addr);
+        else if (n_steps > 1) wait_loads<FIRST>(lds_addr);
+        else wait_loads<0>(lds_addr);
         zero_tail(cs0, c0_, c0_);
         zero_tail(cs0, c0_, c1_);
         if constexpr (TM == 4) { zero_tail(cs0, c0_, c2_); zero_tail(cs0, c0_, c3_); }
         block_barrier();
+        if (n_steps > 1) issue_a(2, pa1, cs1, c1_, IntC<TM == 4 ? 2 : 1>{}, src[GATHER_W ? 1 : 0]);   // (the strips are done with)
         set_fragments();
         read_a(c0_, c0_, c0_, c2_);
         read_b(c0_, c0_, c8_);
@@ -949,197 +958,197 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         if (active == TM) loop(std::true_type{});
         else loop(std::false_type{});
     }
-    __syncthreads();  // the odd steps' buffers become the strips, the even steps' the next tile's
+    __syncthreads();
 
-    constexpr int OLD_CPR = 64 / 8, OLD_ITS = 32 * OLD_CPR / 64;   // as CPRW and ITS of the epilogue
-    u32x4 old[ACCUM ? TM : 1][ACCUM ? OLD_ITS : 1];
-    if (ACCUM) {
-        int lane_o = lane;
-        asm volatile("" : "+v"(lane_o));
-        const uint16_t *from = (GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + expert * p.strideC) + n0 + wn * 64 + (lane_o % OLD_CPR) * 8;
-        const bool col_in = !EDGE || n0 + wn * 64 + (lane_o % OLD_CPR) * 8 < n_cols;
-        const int64_t ldc = GATHER == MERGED ? n_cols : p.ldc;
-        const int m_first = row_begin + wm * 32 + lane_o / OLD_CPR;
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int it = 0; it < OLD_ITS; it++) {
-                const int m = m_first + i * 64 + it * (64 / OLD_CPR);
-                if (!EDGE || (col_in && m < m_rows))
-                    old[ACCUM ? i : 0][ACCUM ? it : 0] =
-                        *reinterpret_cast<const u32x4 *>(from + static_cast<int64_t>(m) * ldc);
-            }
-    }
-
-    uint16_t *Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + (WGRAD ? expert * p.strideC : 0);
-    const int64_t e_ldc = GATHER == MERGED ? n_cols : p.ldc;
-    const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_n0 = n0, e_active = active;
-    have = next_tile();
-    if (have) prefetch();
-
-    // ---- epilogue ------------------------------------------------------------------------------
+    // ---- epilogue, while the next tile's first steps are loaded --------------------------------------------------------------
+    // Each wavefront turns its accumulators around 16 rows at a time in a strip of its own (128-byte rows, 64 columns; in
+    // the last units of odd steps' A) and moves 16-byte chunks of 8 neighbouring columns, eight lanes to a row.
     int lane_e = lane, wave_e = wave;
     asm volatile("" : "+v"(lane_e), "+s"(wave_e));
-    constexpr int COLS = (EPI == EPI_SWIGLU) ? 32 : 64;   // output columns of this wavefront
-    constexpr int PITCH = COLS * 2 + 8;
-    constexpr int STRIP = 32 * PITCH;
-    constexpr int NSTRIP = (EPI == EPI_SWIGLU) ? 3 : 1;
-    static_assert(NW / 2 * NSTRIP * STRIP <= A_STAGE && NW / 2 * NSTRIP * STRIP <= B_STAGE, "strips must fit beside the even steps' buffers");
     const int wm_e = wave_e / WAVES_N, wn_e = wave_e % WAVES_N;
-    char *strip = lds + (wave_e < NW / 2 ? A_STAGE : B0 + B_STAGE) + (wave_e % (NW / 2)) * (NSTRIP * STRIP);
-    const int lrow = lane_e & 15;
-    const int lcol = (lane_e >> 4) * 4;
-    constexpr int CPRW = COLS / 8;            // 16-byte chunks per strip row
-    constexpr int ITS = 32 * CPRW / 64;       // chunks per lane per strip
-    auto strip_put = [&](int which, int row, int col, f32x4 f) {   // (of a 16x16 block)
-        u32x2 v;
-        v[0] = pack2_bf16(f[0], f[1]);
-        v[1] = pack2_bf16(f[2], f[3]);
-        *reinterpret_cast<u32x2 *>(strip + which * STRIP + (row + lrow) * PITCH + (col + lcol) * 2) = v;
-    };
-    auto strip_get = [&](int which, int row, int cc) -> u32x4 {
-        const char *q = strip + which * STRIP + row * PITCH + cc * 16;
-        const u32x2 lo = *reinterpret_cast<const u32x2 *>(q);
-        const u32x2 hi = *reinterpret_cast<const u32x2 *>(q + 8);
-        return u32x4{lo[0], lo[1], hi[0], hi[1]};
+    constexpr int COLS = (EPI == EPI_SWIGLU) ? 32 : 64;   // output columns of this wavefront (EPI_SWIGLU: gate and up, side by side)
+    static_assert(NW * 2048 <= (TM == 4 ? 2 : 1) * UNIT, "strips must fit into the units that prefetch leaves out");
+    const int strip = 2 * A_STAGE - NW * 2048 + wave_e * 2048;   // bytes from lds; 2 KB, its 16-byte chunks XOR-permuted by row
+    int put_at[2], get_at[2];   // of blocks 0 and 1 (2 and 3: the other half of the row); of 8 rows and the other 8
+    {
+        const int row = lane_e & 15, g4 = lane_e >> 4;
+#pragma unroll
+        for (int j = 0; j < 2; j++) put_at[j] = strip + row * 128 + (((j * 2 + (g4 >> 1)) ^ swz(row)) << 4) + (g4 & 1) * 8;
+#pragma unroll
+        for (int x = 0; x < 2; x++) get_at[x] = strip + (x * 8 + (lane_e >> 3)) * 128 + (((lane_e & 7) ^ swz(x * 8 + (lane_e >> 3))) << 4);
+    }
+    auto strip_put = [&](auto block, f32x4 f) {
+        constexpr int J = decltype(block)::value;
+        *reinterpret_cast<u32x2 *>(lds + (put_at[J & 1] ^ (J >= 2 ? 64 : 0))) = u32x2{pack2_bf16(f[0], f[1]), pack2_bf16(f[2], f[3])};
     };
     auto strip_sync = [&]() {  // LDS operations of one wavefront are performed in order
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
-    const int col0 = e_n0 + wn_e * COLS;   // first output column
-    const int row_lim = EDGE && col0 + (lane_e % (COLS / 8)) * 8 >= e_n_cols ? 0 : e_row_end;
-    float wrow_all[(ROWW && EPI == EPI_SWIGLU) ? 2 * TM : 1];
+    // four blocks side by side: chunks 0 and 1 of the strip's rows
+    auto turn = [&](f32x4 b0, f32x4 b1, f32x4 b2, f32x4 b3, u32x4 (&chunk)[2]) {
+        strip_put(c0_, b0); strip_put(c1_, b1); strip_put(c2_, b2); strip_put(c3_, b3);
+        strip_sync();
+#pragma unroll
+        for (int x = 0; x < 2; x++) chunk[x] = *reinterpret_cast<const u32x4 *>(lds + get_at[x]);
+        strip_sync();
+    };
+    const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_active = active;
+    const int col0 = n0 + wn_e * COLS;   // first output column
+    const int chunk_col = (lane_e & (COLS / 8 - 1)) * 8, chunk_row = lane_e >> 3;
+    auto chunk_m = [&](int i, int x) { return (2 * i + wm_e) * 32 + x * 8 + chunk_row; };   // row within the tile; x 0 .. 3
+    const bool all_rows = !EDGE && (WGRAD || e_row_begin + BM <= e_row_end);
+    const int row_lim = EDGE && col0 + chunk_col >= e_n_cols ? 0 : e_row_end;
+    uint16_t *Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + (WGRAD ? expert * p.strideC : 0);
+    const int64_t e_ldc = GATHER == MERGED ? n_cols : p.ldc;
+    // a chunk's element: block-uniform, and this lane's part of it
+    const int64_t tile_at = uniform64(static_cast<int64_t>(e_row_begin + wm_e * 32) * e_ldc + col0);
+    const uint32_t lane_at = static_cast<uint32_t>(chunk_row) * static_cast<uint32_t>(e_ldc) + chunk_col;
+    auto chunk_at = [&](auto *base, int i, int x) { return base + (tile_at + (i * 64 + x * 8) * e_ldc) + lane_at; };
+    float weight[ROWW && EPI == EPI_SWIGLU ? TM : 1][2];   // of the rows of this lane's accumulators; here, so that they do not wait for the prefetch
     if (ROWW && EPI == EPI_SWIGLU) {
 #pragma unroll
-        for (int i = 0; i < 2 * TM; i++) {
-            const int64_t m = static_cast<int64_t>(e_row_begin) + ((i & ~1) + wm_e) * 32 + (i & 1) * 16 + lrow;
-            wrow_all[(ROWW && EPI == EPI_SWIGLU) ? i : 0] = (m < e_row_end) ? p.row_scale[m] : 0.0f;
-        }
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+                weight[ROWW && EPI == EPI_SWIGLU ? i : 0][x] =
+                    p.row_scale[min(e_row_begin + (2 * i + wm_e) * 32 + x * 16 + (lane_e & 15), e_row_end - 1)];
     }
+    have = next_tile();
+    u32x4 old[ACCUM ? TM : 1][ACCUM ? 4 : 1];
+    if (ACCUM) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                // (EDGE: rows and columns past the matrix: its last ones, not used; a load in a branch would be waited for with all others)
+                const uint16_t *from = EDGE ? Cb + static_cast<int64_t>(min(e_row_begin + chunk_m(i, x), e_row_end - 1)) * e_ldc + min(col0 + chunk_col, e_n_cols - 8)
+                                            : chunk_at(Cb, i, x);
+                old[ACCUM ? i : 0][ACCUM ? x : 0] = *reinterpret_cast<const u32x4 *>(from);
+            }
+    }
+    if (have) prefetch();
+    if (ACCUM && EDGE) {   // (waited for once: between stores that may not be made the compiler would wait for all of them)
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) asm volatile("" : "+v"(old[ACCUM ? i : 0][ACCUM ? x : 0]));
+    }
+    stores_follow = all_rows;
+    auto rows_out = [&](auto past_caches) {   // (two loops: of a branch at each store the compiler knows less about what is under way)
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         if (i >= e_active) break;
-        const int64_t m0 = static_cast<int64_t>(e_row_begin) + (2 * i + wm_e) * 32;  // first row of the strip
-        u32x4 *old_out = old[ACCUM ? i : 0];
         if (EPI == EPI_SWIGLU) {
+            f32x4 h[2][2];
+            u32x4 chunk[3][2];
+            // gate and up of a row in one strip row: the lanes of its first half store to g, the others to u
+            uint16_t *const gu = lane_e & 4 ? p.C1 : p.C;
+            // a strip is written again as soon as its reads are issued; what they bring is stored one strip later
+            auto store_gu = [&](int x) {
 #pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const int half = b >> 1, j = b & 1;
-                const float wrow = wrow_all[(ROWW && EPI == EPI_SWIGLU) ? 2 * i + half : 0];   // ROWW: h = w[row] * silu(g) * u, one rounding
-                const f32x4 gv = acc[i][half][j], uv = acc[i][half][2 + j];
-                f32x4 hv;
+                for (int y = 0; y < 2; y++)
+                    if (all_rows || e_row_begin + chunk_m(i, x * 2 + y) < row_lim)
+                        *reinterpret_cast<u32x4 *>(chunk_at(gu, i, x * 2 + y)) = chunk[x][y];
+            };
 #pragma unroll
-                for (int x = 0; x < 4; x++) {
-                    hv[x] = (gv[x] * fast_sigmoid(gv[x])) * uv[x];
-                    if (ROWW) hv[x] *= wrow;
-                }
-                strip_put(0, half * 16, j * 16, gv);
-                strip_put(1, half * 16, j * 16, uv);
-                strip_put(2, half * 16, j * 16, hv);
+            for (int x = 0; x < 2; x++) {
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int y = 0; y < 4; y++) {
+                        const float gv = acc[i][x][j][y], uv = acc[i][x][2 + j][y];
+                        h[x][j][y] = (gv * fast_sigmoid(gv)) * uv;
+                        if (ROWW) h[x][j][y] *= weight[ROWW ? i : 0][x];   // h = w[row] * silu(g) * u, one rounding
+                    }
+                turn(acc[i][x][0], acc[i][x][1], acc[i][x][2], acc[i][x][3], chunk[x]);
+            }
+            store_gu(0);
+            // h of the unit's upper 16 rows beside that of its lower ones
+            turn(h[0][0], h[0][1], h[1][0], h[1][1], chunk[2]);
+            store_gu(1);
+#pragma unroll
+            for (int y = 0; y < 2; y++) {
+                const int upper = lane_e & 4 ? 16 : 0;
+                if (all_rows || e_row_begin + chunk_m(i, y) + upper < row_lim)
+                    *reinterpret_cast<u32x4 *>(chunk_at(p.C2, i, y) + upper * e_ldc) = chunk[2][y];
             }
         } else {
+            u32x4 chunk[2];
+            u32x4 gq[EPI == EPI_SWIGLU_BWD ? 2 : 1], uq[EPI == EPI_SWIGLU_BWD ? 2 : 1];
+            float wr[2] = {1.0f, 1.0f};
 #pragma unroll
-            for (int b = 0; b < 8; b++) strip_put(0, (b >> 2) * 16, (b & 3) * 16, acc[i][b >> 2][b & 3]);
-        }
-        strip_sync();
-        if (EPI == EPI_SWIGLU_BWD) {
-            constexpr int GRP = 2;   // g and u in flight for half a strip: the 256x256 kernels spill 7 and 8 registers
-            u32x4 gq[GRP], uq[GRP];
-            // ROWW: lane l fetches the weight of strip row l % 32 along with the g/u loads; the
-            // lanes that work on a row pick it up with a lane read
-            float w_strip = 0.0f;
-            if (ROWW && m0 + (lane_e & 31) < e_row_end) w_strip = p.row_scale[m0 + (lane_e & 31)];
+            for (int x = 0; x < 4; x++) {
+                if (EPI == EPI_SWIGLU_BWD && x % 2 == 0) {
+                    // g, u (and the weights) of half a unit.  They have no reader after this one: past the caches (-1 to -3 %)
 #pragma unroll
-            for (int i0 = 0; i0 < ITS; i0 += GRP) {
-#pragma unroll
-            for (int it = 0; it < GRP; it++) {
-                const int q = (i0 + it) * 64 + lane_e;
-                const int64_t m = m0 + q / CPRW;
-                if (m < row_lim) {
-                    const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
-                    // g and u have no reader after this one: keep them out of the caches (-1 to -3 %)
-                    gq[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p.G + o));
-                    uq[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p.U + o));
-                }
-            }
-#pragma unroll
-            for (int it = 0; it < GRP; it++) {
-                const int q = (i0 + it) * 64 + lane_e;
-                const int64_t m = m0 + q / CPRW;
-                float dot = 0.0f;   // ROWW: this lane's part of sum_i dh[m][i] * silu(g[m][i]) * u[m][i]
-                const float wr = ROWW ? __shfl(w_strip, q / CPRW, 64) : 1.0f;
-                if (m < row_lim) {
-                    float dh[8], gv[8], uv[8], dg[8], du[8];
-                    Elem<uint16_t>::unpack(strip_get(0, q / CPRW, q % CPRW), dh);
-                    Elem<uint16_t>::unpack(gq[it], gv);
-                    Elem<uint16_t>::unpack(uq[it], uv);
-#pragma unroll
-                    for (int x = 0; x < 8; x++) {
-                        const float sg = fast_sigmoid(gv[x]);
-                        const float sl = gv[x] * sg;
-                        if (ROWW) {
-                            // acc is the gradient of w * silu(g) * u: the routing weight's gradient
-                            // is its product with silu(g) * u, the activation's gets the factor w
-                            dot += dh[x] * (sl * uv[x]);
-                            dh[x] *= wr;
+                    for (int y = 0; y < 2; y++) {
+                        const int m = e_row_begin + chunk_m(i, x + y);
+                        if (all_rows || m < row_lim) {
+                            gq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(p.G, i, x + y)));
+                            uq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(p.U, i, x + y)));
+                            if (ROWW) wr[y] = p.row_scale[m];
                         }
-                        du[x] = dh[x] * sl;
-                        dg[x] = (dh[x] * uv[x]) * (sg * (1.0f + gv[x] * (1.0f - sg)));
                     }
-                    const int64_t o = m * p.ldc + col0 + (q % CPRW) * 8;
-                    u32x4 vg, vu;
+                }
+                if (x % 2 == 0) turn(acc[i][x >> 1][0], acc[i][x >> 1][1], acc[i][x >> 1][2], acc[i][x >> 1][3], chunk);
+                u32x4 v = chunk[x & 1];
+                const int m = e_row_begin + chunk_m(i, x);
+                if (EPI == EPI_SWIGLU_BWD) {
+                    float dot = 0.0f;   // ROWW: this lane's part of sum_i dh[m][i] * silu(g[m][i]) * u[m][i]
+                    if (all_rows || m < row_lim) {
+                        float dh[8], gv[8], uv[8], dg[8], du[8];
+                        Elem<uint16_t>::unpack(v, dh);
+                        Elem<uint16_t>::unpack(gq[x & 1], gv);
+                        Elem<uint16_t>::unpack(uq[x & 1], uv);
 #pragma unroll
-                    for (int x = 0; x < 4; x++) {
-                        vg[x] = pack2_bf16(dg[2 * x], dg[2 * x + 1]);
-                        vu[x] = pack2_bf16(du[2 * x], du[2 * x + 1]);
+                        for (int y = 0; y < 8; y++) {
+                            const float sg = fast_sigmoid(gv[y]);
+                            const float sl = gv[y] * sg;
+                            if (ROWW) {
+                                // acc is the gradient of w * silu(g) * u: the routing weight's gradient
+                                // is its product with silu(g) * u, the activation's gets the factor w
+                                dot += dh[y] * (sl * uv[y]);
+                                dh[y] *= wr[x & 1];
+                            }
+                            du[y] = dh[y] * sl;
+                            dg[y] = (dh[y] * uv[y]) * (sg * (1.0f + gv[y] * (1.0f - sg)));
+                        }
+                        u32x4 vg, vu;
+#pragma unroll
+                        for (int y = 0; y < 4; y++) {
+                            vg[y] = pack2_bf16(dg[2 * y], dg[2 * y + 1]);
+                            vu[y] = pack2_bf16(du[2 * y], du[2 * y + 1]);
+                        }
+                        *reinterpret_cast<u32x4 *>(chunk_at(p.C, i, x)) = vg;
+                        *reinterpret_cast<u32x4 *>(chunk_at(p.C1, i, x)) = vu;
                     }
-                    *reinterpret_cast<u32x4 *>(p.C + o) = vg;
-                    *reinterpret_cast<u32x4 *>(p.C1 + o) = vu;
-                }
-                if (ROWW) {
-                    // the CPRW lanes of a row are neighbours: add them up in a fixed order and let
-                    // the first one store the sum for this wavefront's column range
-                    dot = lane_group_sum<CPRW>(dot);
-                    if (q % CPRW == 0 && m < row_lim) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            }
-        } else {
-#pragma unroll
-            for (int it = 0; it < ITS; it++) {
-                const int q = it * 64 + lane_e;
-                const int64_t m = m0 + q / CPRW;
-                if (m < row_lim) {
-                    const int64_t o = m * e_ldc + col0 + (q % CPRW) * 8;
-                    u32x4 v = strip_get(0, q / CPRW, q % CPRW);
-                    if (WGRAD && ACCUM) {
+                    if (ROWW) {   // this wavefront's column range of the row: its eight lanes in a fixed order
+                        dot = eight_lanes_sum(dot);
+                        if ((lane_e & 7) == 0 && m < row_lim) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
+                    }
+                    if (x & 1) __builtin_amdgcn_sched_barrier(0);
+                } else if (all_rows || m < row_lim) {   // (all_rows: known to the compiler where old values are waited for)
+                    if (ACCUM) {
                         float fresh[8], prev[8];
                         Elem<uint16_t>::unpack(v, fresh);
-                        Elem<uint16_t>::unpack(old_out[ACCUM ? it : 0], prev);
+                        Elem<uint16_t>::unpack(old[ACCUM ? i : 0][ACCUM ? x : 0], prev);
 #pragma unroll
-                        for (int x = 0; x < 4; x++)
-                            v[x] = pack2_bf16(prev[2 * x] + fresh[2 * x], prev[2 * x + 1] + fresh[2 * x + 1]);
+                        for (int y = 0; y < 4; y++)
+                            v[y] = pack2_bf16(prev[2 * y] + fresh[2 * y], prev[2 * y + 1] + fresh[2 * y + 1]);
                     }
-                    if (WGRAD && !EDGE && p.stream) {
-                        asm volatile("");   // (or the compiler makes one ordinary store of the two)
-                        __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(Cb + o));
-                        asm volatile("");
-                    } else {
-                        *reinterpret_cast<u32x4 *>(Cb + o) = v;
-                    }
-                    if (EPI == EPI_SWIGLU) {
-                        *reinterpret_cast<u32x4 *>(p.C1 + o) = strip_get(1, q / CPRW, q % CPRW);
-                        *reinterpret_cast<u32x4 *>(p.C2 + o) = strip_get(2, q / CPRW, q % CPRW);
-                    }
+                    u32x4 *to = reinterpret_cast<u32x4 *>(chunk_at(Cb, i, x));
+                    if (decltype(past_caches)::value) __builtin_nontemporal_store(v, to);
+                    else *to = v;
+                    if (ACCUM) __builtin_amdgcn_sched_barrier(0);   // (all of them at once spill registers)
                 }
             }
         }
-        strip_sync();  // the strip is rewritten by the next i
     }
-    __syncthreads();  // the strips alias the odd steps' buffers, which the next tile loads into
+    };
+    if (WGRAD && !EDGE && p.stream) rows_out(std::true_type{});
+    else rows_out(std::false_type{});
     }  // tile loop
 }
 
