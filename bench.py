@@ -67,6 +67,9 @@ GEMM_ENTRY_PRODUCTS = {     # C-ABI entry -> number of [rows x N x K] products p
     "om_grouped_gemm_wgrad_accumulate": 1, "om_grouped_gemm_wgrad_gathered_accumulate": 1,
     "om_grouped_gemm_wgrad_gathered_out_accumulate": 1,
     "om_grouped_gemm_wgrad_merged": 3, "om_grouped_gemm_wgrad_merged_accumulate": 3,
+    # with a shared expert's rows as well
+    "om_merged_mlp_gate_up_fwd_weighted_dense": 2, "om_grouped_gemm_fwd_dense": 1,
+    "om_merged_mlp_down_dgrad_weighted_dense": 1, "om_merged_mlp_gate_up_dgrad_dense": 2,
 }
 
 

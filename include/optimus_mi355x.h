@@ -592,6 +592,43 @@ int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void
                                       void *dx, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
                                       int G, int I, int H, int64_t w_stride, void *stream);
 
+/* One more expert of the same extents beside the routed ones, with all of its `rows` known: the shared expert of a
+ * DeepSeek-V3 layer (modeling_deepseek_v3.py:265), whose rows are not permuted and not weighted.  Its products run in the
+ * routed experts' launch where that is faster, else in one of their own ahead of it; the results do not depend on
+ * it beyond the order of the sums.  Fields by entry point (others are ignored; dense matrices, 16-byte aligned):
+ *   ..._gate_up_fwd_weighted_dense : a[0] = x [rows, H]; w = gate, up [I, H]; c = g, u, h [rows, I]
+ *   om_grouped_gemm_fwd_dense      : a[0] = input [rows, K]; w[0] [N, K]; c[0] = output [rows, N]
+ *   ..._down_dgrad_weighted_dense  : a[0] = dy [rows, H]; w[0] = down [H, I]; g, u [rows, I]; c = dg, du [rows, I]
+ *   ..._gate_up_dgrad_dense        : a = dg, du [rows, I]; w = gate, up [I, H]; c[0] = dx [rows, H]
+ *   cum: device {0, rows}, for a launch of its own.  The other arguments as in the _bound forms.           */
+typedef struct {
+    const void *a[2], *w[2];
+    void *c[3];
+    const void *g, *u;
+    const int32_t *cum;
+    int64_t rows;
+} om_dense_expert;
+/* 1 if the gate+up product of a dense expert with dense_rows rows would run in the routed experts' launch. */
+int om_merged_mlp_dense_rides(int64_t expected_rows, int G, int I, int H, int64_t dense_rows);
+int om_merged_mlp_gate_up_fwd_weighted_dense(const void *x, const int32_t *x_rows, int64_t src_rows,
+                                             const void *w_gate, const void *w_up, const float *row_weights,
+                                             void *g, void *u, void *h, const int32_t *cum_token_counts,
+                                             int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                             int64_t w_stride, const om_dense_expert *dense, void *stream);
+int om_grouped_gemm_fwd_dense(const void *input, const void *weight, void *output,
+                              const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int N,
+                              int K, int64_t w_stride, const om_dense_expert *dense, void *stream);
+int om_merged_mlp_down_dgrad_weighted_dense(const void *dy, const int32_t *dy_rows, int64_t src_rows,
+                                            const void *w_down, const void *g, const void *u,
+                                            const float *row_weights, void *dg, void *du, float *row_dot,
+                                            const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
+                                            int G, int I, int H, int64_t w_stride, const om_dense_expert *dense,
+                                            void *stream);
+int om_merged_mlp_gate_up_dgrad_dense(const void *dg, const void *du, const void *w_gate, const void *w_up,
+                                      void *dx, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
+                                      int G, int I, int H, int64_t w_stride, const om_dense_expert *dense,
+                                      void *stream);
+
 /* Weight gradients added to a gradient buffer in place.  In the reference's training set-up every
  * p.grad is a view of the optimizer's flat gradient buffer (optimus/optimizers.py:105-111) that is
  * zeroed in place (:117-118), and micro-batches accumulate into it (dist_train.py:154): autograd

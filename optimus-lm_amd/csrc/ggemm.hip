@@ -98,6 +98,15 @@ struct WgradSet {
     int m, n;
 };
 
+// DENSE: one more expert behind the others, with operands and outputs of its own and all of its rows known to the host (the
+// shared expert beside a window of routed ones).  Its rows are not taken through an index and have the weight 1.
+struct DenseExpert {
+    const uint16_t *A[2], *B[2];
+    uint16_t *C, *C1, *C2;
+    const uint16_t *G, *U;
+    int rows;
+};
+
 template <int BM> constexpr int WAVES_N = BM / 64;        // 256x256: 2 x 4 wavefronts, 128x128: 2 x 2
 template <int BM> constexpr int THREADS = 2 * WAVES_N<BM> * 64;
 
@@ -127,6 +136,7 @@ struct GemmParams {
     bool stream;                // wgrad: the gradients are stored past the caches (see CACHED_WEIGHTS)
     int share;                  // XCDs that share an expert's tiles; 0: contiguous runs of tiles per XCD
     WgradSet set[3];            // MERGED
+    DenseExpert dense;          // DENSE
 };
 
 typedef __attribute__((address_space(3))) s16x4 *lds_s16x4_ptr;
@@ -397,13 +407,14 @@ template <int V> using IntC = std::integral_constant<int, V>;
 // (second launch bound: two wavefronts per SIMD, i.e. at most 256 registers, for the 128x128 tile, whose two blocks per
 // CU depend on it; the 256x256 tile's 8 wavefronts imply it already)
 template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool ACCUM = false,
-          bool EDGE = false, bool ONCE = false>
+          bool EDGE = false, bool ONCE = false, bool DENSE = false>
 __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
     constexpr int BN = BM, WAVES_N = BN / 64, NW = 2 * WAVES_N;
     constexpr int TM = BM / 64, TN = 2;     // row units of a tile, accumulators of a wavefront in each
     static_assert(GATHER == GATHER_NONE || (GATHER == GATHER_A && AKIND == CONTIG && EPI != EPI_WGRAD) ||
                       (GATHER == GATHER_B && BKIND == STRIDED && EPI == EPI_WGRAD) ||
                       ((GATHER == GATHER_WA || GATHER == MERGED) && AKIND == STRIDED && EPI == EPI_WGRAD), "gather variants");
+    static_assert(!DENSE || (BM == 128 && EPI != EPI_WGRAD), "few rows per expert");
     static_assert(!ACCUM || EPI == EPI_WGRAD, "only the weight gradient adds into its output");
     static_assert(!ROWW || EPI == EPI_SWIGLU || EPI == EPI_SWIGLU_BWD, "row weights belong to the SwiGLU epilogues");
     constexpr bool WGRAD = EPI == EPI_WGRAD;
@@ -432,6 +443,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     int expert = 0, row_begin = 0, row_end = 0, n0 = 0, c_begin = 0, c_len = 0;
     int steps_per_phase = 0, c_wrap = 0, n_steps = 0, rot = 0;
     int active = TM;      // row units that hold rows of the expert
+    bool dense = false;   // DENSE: whether the tile is the dense expert's
     int once = 0;         // ONCE: whether no other row tile reads the expert's weights
     // the slot of this wavefront's direct load l of a unit: row (CONTIG) or contraction row (STRIDED) and chunk
     auto slot = [&](int l) { return (wave * L + l) * 8 + (lane >> 3); };
@@ -522,8 +534,18 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 row_begin = q.row_begin + tile_m * BM;
                 row_end = q.row_end;
                 row_tile = __builtin_amdgcn_readfirstlane(seg[expert]) + tile_m;
-            } else if (!find_tile<BM>(tile_end, seg, p.n_experts, tile_m, lane, expert, row_begin, row_end)) return false;
-            if (ONCE) once = __builtin_amdgcn_readfirstlane(row_end - row_begin <= BM && (p.share ? tile_m == 0 : row_begin == seg[expert]) ? 1 : 0);
+            } else if (!find_tile<BM>(tile_end, seg, p.n_experts + DENSE, tile_m, lane, expert, row_begin, row_end)) return false;
+            int first_row = p.share ? 0 : seg[expert];   // (p.share: not used)
+            if (DENSE) {
+                dense = __builtin_amdgcn_readfirstlane(expert) == p.n_experts;
+                if (dense) {
+                    row_tile -= tile_end[p.n_experts - 1];
+                    row_begin = row_tile * BM;
+                    row_end = p.dense.rows;
+                    first_row = 0;
+                }
+            }
+            if (ONCE) once = __builtin_amdgcn_readfirstlane(row_end - row_begin <= BM && (p.share ? tile_m == 0 : row_begin == first_row) ? 1 : 0);
             // (`row_tile` among all experts' with and without p.share: the sums begin at the same step, the same bits)
             rot_a = tile_n; rot_b = row_tile & 7;
             n0 = tile_n * BN_OUT;
@@ -553,8 +575,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
 #pragma unroll
                 for (int u = 0; u < UA; u++) {
                     int m = min(row_begin + u * 64 + r, row_end - 1);   // rows past the segment: valid memory, result unused
-                    if (GATHER == GATHER_A) m = p.row_index[m];
-                    else m -= row_begin;
+                    if (GATHER == GATHER_A && !dense) m = p.row_index[m];
+                    else if (GATHER != GATHER_A) m -= row_begin;
                     a_off[u][l] = (static_cast<uint32_t>(m) * lda32 + ch * 8) * 2u;
                 }
             } else {
@@ -577,17 +599,20 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         }
         const int64_t a_base = AKIND == CONTIG ? (GATHER == GATHER_A ? 0 : static_cast<int64_t>(row_begin) * p.lda)
                                                : row_begin + (a_indexed ? 0 : static_cast<int64_t>(c_begin) * lda32);
-        const int64_t b_base = BKIND == CONTIG ? expert * p.strideB + static_cast<int64_t>(n0) * p.ldb
+        const int64_t matrix = dense ? 0 : expert * p.strideB;
+        const int64_t b_base = BKIND == CONTIG ? matrix + static_cast<int64_t>(n0) * p.ldb
                                : WGRAD ? n0 + (b_indexed ? 0 : static_cast<int64_t>(c_begin) * ldb32)
-                                       : expert * p.strideB + n0;
+                                       : matrix + n0;
         // EPI_SWIGLU: LDS rows 0..31 of a unit are gate rows, 32..63 up rows; a wavefront's loads lie in one of the two
-        const uint16_t *A_first = GATHER == MERGED ? p.set[product].A : p.A[0];
-        const uint16_t *B_first = GATHER == MERGED ? p.set[product].B : EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? p.B[1] : p.B[0];
+        const int second = EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? 1 : 0;
+        const uint16_t *A_first = GATHER == MERGED ? p.set[product].A : dense ? p.dense.A[0] : p.A[0];
+        const uint16_t *B_first = GATHER == MERGED ? p.set[product].B : dense ? p.dense.B[second] : p.B[second];
         a_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(A_first + a_base)));
         b_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(B_first + b_base)));
         if (TWO_PHASE) {
-            a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.A[1] : p.A[0]) + a_base)));
-            b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((p.phases > 1 ? p.B[1] : p.B[0]) + b_base)));
+            const int phase = p.phases > 1 ? 1 : 0;
+            a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((dense ? p.dense.A[phase] : p.A[phase]) + a_base)));
+            b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((dense ? p.dense.B[phase] : p.B[phase]) + b_base)));
         }
         const int cache_key = GATHER == MERGED ? expert * 2 + (row_index != p.set[1].b_rows ? 1 : 0) : expert;
         if (GATHER_W && (GATHER != MERGED || row_index) && cache_key != cached_expert) {
@@ -643,14 +668,15 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     auto issue_b = [&](int left, const char *base, int c0, auto par, auto unit, const int (&rows)[L]) {
         constexpr int P = decltype(par)::value, U = decltype(unit)::value;
+        const int past = ONCE ? __builtin_amdgcn_readfirstlane(once) : 0;
 #pragma unroll
         for (int l = 0; l < L; l++) {
             uint32_t off = b_off[EDGE ? U : 0][l];
             if (BKIND == CONTIG) off -= tail_bytes(c0, l);
             else off += crow_bytes(c0, l, ldb32, rows, b_indexed);
             const char *q = EDGE ? base : BKIND == CONTIG ? base + U * b_unit : base + U * 128;
-            if (ONCE && l == 0) dma16_if_once<B0 + P * B_STAGE + U * UNIT>(left, once, q, off, wave_lds);
-            else if (ONCE) dma16_if_once<B0 + P * B_STAGE + U * UNIT + 1024>(left, once, q, off, wave_lds);
+            if (ONCE && l == 0) dma16_if_once<B0 + P * B_STAGE + U * UNIT>(left, past, q, off, wave_lds);
+            else if (ONCE) dma16_if_once<B0 + P * B_STAGE + U * UNIT + 1024>(left, past, q, off, wave_lds);
             else if (l == 0) dma16_if<B0 + P * B_STAGE + U * UNIT>(left, q, off, wave_lds);
             else dma16_if<B0 + P * B_STAGE + U * UNIT + 1024>(left, q, off, wave_lds);
         }
@@ -762,8 +788,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         if (!WGRAD) {
             if (wave == 0) build_tile_table<BM>(p.cum, p.n_experts, lane, tile_end, seg);
             __syncthreads();
+            if (DENSE) {
+                if (tid == 0) tile_end[p.n_experts] = tile_end[p.n_experts - 1] + (p.dense.rows + BM - 1) / BM;
+                __syncthreads();
+            }
             constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? BN / 2 : BN;
-            total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+            total_tiles = __builtin_amdgcn_readfirstlane(tile_end[p.n_experts - 1 + DENSE]) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
         }
         per = total_tiles / NUM_XCD;
         rem = total_tiles - per * NUM_XCD;
@@ -1000,7 +1030,9 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     auto chunk_m = [&](int i, int x) { return (2 * i + wm_e) * 32 + x * 8 + chunk_row; };   // row within the tile; x 0 .. 3
     const bool all_rows = !EDGE && (WGRAD || e_row_begin + BM <= e_row_end);
     const int row_lim = EDGE && col0 + chunk_col >= e_n_cols ? 0 : e_row_end;
-    uint16_t *Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : p.C + (WGRAD ? expert * p.strideC : 0);
+    const bool e_dense = dense;
+    uint16_t *const C = e_dense ? p.dense.C : p.C, *const C1 = e_dense ? p.dense.C1 : p.C1;
+    uint16_t *const Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : C + (WGRAD ? expert * p.strideC : 0);
     const int64_t e_ldc = GATHER == MERGED ? n_cols : p.ldc;
     // a chunk's element: block-uniform, and this lane's part of it
     const int64_t tile_at = uniform64(static_cast<int64_t>(e_row_begin + wm_e * 32) * e_ldc + col0);
@@ -1012,7 +1044,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int x = 0; x < 2; x++)
-                weight[ROWW && EPI == EPI_SWIGLU ? i : 0][x] =
+                weight[ROWW && EPI == EPI_SWIGLU ? i : 0][x] = e_dense ? 1.0f :
                     p.row_scale[min(e_row_begin + (2 * i + wm_e) * 32 + x * 16 + (lane_e & 15), e_row_end - 1)];
     }
     have = next_tile();
@@ -1044,7 +1076,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             f32x4 h[2][2];
             u32x4 chunk[3][2];
             // gate and up of a row in one strip row: the lanes of its first half store to g, the others to u
-            uint16_t *const gu = lane_e & 4 ? p.C1 : p.C;
+            uint16_t *const gu = lane_e & 4 ? C1 : C, *const h_out = e_dense ? p.dense.C2 : p.C2;
             // a strip is written again as soon as its reads are issued; what they bring is stored one strip later
             auto store_gu = [&](int x) {
 #pragma unroll
@@ -1072,7 +1104,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             for (int y = 0; y < 2; y++) {
                 const int upper = lane_e & 4 ? 16 : 0;
                 if (all_rows || e_row_begin + chunk_m(i, y) + upper < row_lim)
-                    *reinterpret_cast<u32x4 *>(chunk_at(p.C2, i, y) + upper * e_ldc) = chunk[2][y];
+                    *reinterpret_cast<u32x4 *>(chunk_at(h_out, i, y) + upper * e_ldc) = chunk[2][y];
             }
         } else {
             u32x4 chunk[2];
@@ -1086,9 +1118,9 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                     for (int y = 0; y < 2; y++) {
                         const int m = e_row_begin + chunk_m(i, x + y);
                         if (all_rows || m < row_lim) {
-                            gq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(p.G, i, x + y)));
-                            uq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(p.U, i, x + y)));
-                            if (ROWW) wr[y] = p.row_scale[m];
+                            gq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(e_dense ? p.dense.G : p.G, i, x + y)));
+                            uq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(e_dense ? p.dense.U : p.U, i, x + y)));
+                            if (ROWW && !e_dense) wr[y] = p.row_scale[m];
                         }
                     }
                 }
@@ -1121,12 +1153,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                             vg[y] = pack2_bf16(dg[2 * y], dg[2 * y + 1]);
                             vu[y] = pack2_bf16(du[2 * y], du[2 * y + 1]);
                         }
-                        *reinterpret_cast<u32x4 *>(chunk_at(p.C, i, x)) = vg;
-                        *reinterpret_cast<u32x4 *>(chunk_at(p.C1, i, x)) = vu;
+                        *reinterpret_cast<u32x4 *>(chunk_at(C, i, x)) = vg;
+                        *reinterpret_cast<u32x4 *>(chunk_at(C1, i, x)) = vu;
                     }
                     if (ROWW) {   // this wavefront's column range of the row: its eight lanes in a fixed order
                         dot = eight_lanes_sum(dot);
-                        if ((lane_e & 7) == 0 && m < row_lim) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
+                        if ((lane_e & 7) == 0 && m < row_lim && !e_dense) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
                     }
                     if (x & 1) __builtin_amdgcn_sched_barrier(0);
                 } else if (all_rows || m < row_lim) {   // (all_rows: known to the compiler where old values are waited for)
@@ -1256,6 +1288,47 @@ template <int EPI> bool uses_big_tile(int n_cols, int kc, int n_experts, int64_t
     return tiles * 2 >= device_cu_count();
 }
 
+// Whether a dense expert rides in the launch of the routed ones: where both would be 128x128 tiles.  A shared expert with few
+// rows is a launch of few blocks that each walk all of a long contraction (64 rows of 7168/2048: gate+up 42 us, down 15, in
+// the streaming kernels; 128x128 tiles 65 and 21); beside the routed experts' tiles it costs what its weights take to arrive.
+// Whole passes of 32 of 256 experts and the shared one, us, on its own -> riding.  7168/2048, forward of 16 tokens 211 -> 190, 64
+// 279 -> 231, 128 361 -> 304, 315 431 -> 363; training steps of 16 1225 -> 1097, 128 1795 -> 1670, 400 2233 -> 2175, 1000 2938 ->
+// 2843.  3000/1000, forward of 200 190 -> 154; 1024/256 of 600 94 -> 85, of 100 as before; steps of 3000/1000, 700 tokens 888 -> 810.
+// Not where its own tiles fill the chip: 1200/1000, forward of 5000 267 -> 275.
+template <int EPI> bool dense_rides(const GemmParams &p, int64_t expected, int64_t dense_rows) {
+    constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? 64 : 128;
+    return p.n_experts < MAX_EXPERTS && rows_share(p, expected) == 0 && !uses_big_tile<EPI>(p.n_cols, p.kc, p.n_experts, expected) &&
+           !uses_big_tile<EPI>(p.n_cols, p.kc, 1, dense_rows) &&
+           (dense_rows + 127) / 128 * ((p.n_cols + BN_OUT - 1) / BN_OUT) < 2 * device_cu_count();
+}
+template <int AKIND, int BKIND, int EPI, int GATHER, bool ROWW>
+int launch_rows_dense(GemmParams &p, int64_t rows, hipStream_t st) {
+    constexpr int BN_OUT = (EPI == EPI_SWIGLU) ? 64 : 128;
+    p.share = 0;
+    const int64_t tiles = ((rows + 127) / 128 + p.n_experts + (p.dense.rows + 127) / 128) * ((p.n_cols + BN_OUT - 1) / BN_OUT);
+    if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
+    const dim3 grid(persistent_blocks<128>(tiles)), block(THREADS<128>);
+    const int64_t weights = static_cast<int64_t>(p.n_experts) * p.n_cols * p.kc * (EPI == EPI_SWIGLU ? 2 : p.phases);
+    bool once = true;   // (one matrix: null second pointers, nothing to check)
+    for (int i = 0; i < 2; i++)
+        once &= om_weights_pass_caches(p.B[i], weights, p.ldb, p.strideB) && om_weights_pass_caches(p.dense.B[i], weights, p.ldb, 0);
+    if (once) ggemm_kernel<128, AKIND, BKIND, EPI, GATHER, ROWW, false, true, true, true><<<grid, block, 0, st>>>(p);
+    else ggemm_kernel<128, AKIND, BKIND, EPI, GATHER, ROWW, false, true, false, true><<<grid, block, 0, st>>>(p);
+    return om_launch_status();
+}
+
+// The dense expert of an entry point's arguments; its operands are checked by the launch of its own where it does not ride.
+bool dense_operands(GemmParams &p, const om_dense_expert *d) {
+    for (const void *q : {d->a[0], d->a[1], d->w[0], d->w[1], static_cast<const void *>(d->c[0]), static_cast<const void *>(d->c[1]),
+                          static_cast<const void *>(d->c[2]), d->g, d->u})
+        if (!om_aligned16(q)) return false;
+    p.dense = {{static_cast<const uint16_t *>(d->a[0]), static_cast<const uint16_t *>(d->a[1])},
+               {static_cast<const uint16_t *>(d->w[0]), static_cast<const uint16_t *>(d->w[1])},
+               static_cast<uint16_t *>(d->c[0]), static_cast<uint16_t *>(d->c[1]), static_cast<uint16_t *>(d->c[2]),
+               static_cast<const uint16_t *>(d->g), static_cast<const uint16_t *>(d->u), static_cast<int>(d->rows)};
+    return true;
+}
+
 // `rows` sizes the launch, `expected` (rows, or fewer where rows is a bound) selects the kernel.
 template <int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false>
 int launch_rows_auto(GemmParams &p, int64_t rows, int64_t expected, hipStream_t st) {
@@ -1273,11 +1346,16 @@ extern "C" int om_grouped_gemm_fwd(const void *input, const void *weight, void *
     return om_grouped_gemm_fwd_bound(input, weight, output, cum_token_counts, rows, rows, G, N, K, w_stride, stream);
 }
 
-extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, void *output,
-                                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
-                                         int N, int K, int64_t w_stride, void *stream) {
+namespace {
+int grouped_fwd_launch(const void *input, const void *weight, void *output, const int32_t *cum_token_counts, int64_t rows,
+                       int64_t expected_rows, int G, int N, int K, int64_t w_stride, const om_dense_expert *dense, void *stream) {
     if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(N, 8) || !mult(K, 8)) return OM_ERR_SHAPE;
-    if (rows == 0) return OM_OK;
+    if (dense && (dense->rows < 1 || !fits_gather(dense->rows))) return OM_ERR_SHAPE;
+    if (dense && (!dense->a[0] || !dense->w[0] || !dense->c[0] || !dense->cum)) return OM_ERR_NULL;
+    auto dense_alone = [&]() {
+        return grouped_fwd_launch(dense->a[0], dense->w[0], dense->c[0], dense->cum, dense->rows, dense->rows, 1, N, K, 0, nullptr, stream);
+    };
+    if (rows == 0) return dense ? dense_alone() : OM_OK;
     if (!input || !weight || !output || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(input) || !om_aligned16(weight) || !om_aligned16(output)) return OM_ERR_ALIGN;
     GemmParams p = {};
@@ -1290,11 +1368,34 @@ extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, 
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * K) || !fits_span(rows * N) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
     const bool past_caches = om_weights_pass_caches(weight, static_cast<int64_t>(G) * N * K, K, p.strideB);
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N, past_caches))
+    const bool streams = G <= MAX_EXPERTS && om_ggemm_streams(expected_rows, G, N, past_caches);
+    p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
+    if (dense && !streams && dense_rides<EPI_STORE>(p, expected_rows, dense->rows)) {
+        if (!dense_operands(p, dense)) return OM_ERR_ALIGN;
+        return launch_rows_dense<CONTIG, CONTIG, EPI_STORE, GATHER_NONE, false>(p, rows, om_stream(stream));
+    }
+    if (dense) {
+        const int code = dense_alone();
+        if (code != OM_OK) return code;
+    }
+    if (streams)
         return om_ggemm_stream_fwd(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, p.strideB,
                                    om_stream(stream));
-    p.rows = rows; p.n_experts = G; p.n_cols = N; p.kc = K; p.phases = 1;
     return launch_rows_auto<CONTIG, CONTIG, EPI_STORE>(p, rows, expected_rows, om_stream(stream));
+}
+}  // namespace
+
+extern "C" int om_grouped_gemm_fwd_bound(const void *input, const void *weight, void *output,
+                                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
+                                         int N, int K, int64_t w_stride, void *stream) {
+    return grouped_fwd_launch(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, w_stride, nullptr, stream);
+}
+
+extern "C" int om_grouped_gemm_fwd_dense(const void *input, const void *weight, void *output,
+                                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
+                                         int N, int K, int64_t w_stride, const om_dense_expert *dense, void *stream) {
+    if (!dense) return OM_ERR_NULL;
+    return grouped_fwd_launch(input, weight, output, cum_token_counts, rows, expected_rows, G, N, K, w_stride, dense, stream);
 }
 
 extern "C" int om_grouped_gemm_dgrad(const void *output_grad, const void *weight, void *input_grad,
@@ -1584,9 +1685,15 @@ namespace {
 int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate,
                        const void *w_up, const float *row_weights, void *g, void *u, void *h,
                        const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I, int H,
-                       int64_t w_stride, void *stream) {
+                       int64_t w_stride, void *stream, const om_dense_expert *dense = nullptr) {
     if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
-    if (rows == 0) return OM_OK;
+    if (dense && (dense->rows < 1 || !fits_gather(dense->rows * H))) return OM_ERR_SHAPE;
+    if (dense && (!dense->a[0] || !dense->w[0] || !dense->w[1] || !dense->c[0] || !dense->c[1] || !dense->c[2] || !dense->cum)) return OM_ERR_NULL;
+    auto dense_alone = [&]() {
+        return gate_up_fwd_launch(dense->a[0], nullptr, 0, dense->w[0], dense->w[1], nullptr, dense->c[0], dense->c[1], dense->c[2],
+                                  dense->cum, dense->rows, dense->rows, 1, I, H, 0, stream);
+    };
+    if (rows == 0) return dense ? dense_alone() : OM_OK;
     if (!x || !w_gate || !w_up || !g || !u || !h || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(x) || !om_aligned16(w_gate) || !om_aligned16(w_up) || !om_aligned16(g) ||
         !om_aligned16(u) || !om_aligned16(h))
@@ -1608,7 +1715,17 @@ int gate_up_fwd_launch(const void *x, const int32_t *x_rows, int64_t src_rows, c
         return OM_ERR_SHAPE;
     const int64_t weights = 2 * static_cast<int64_t>(G) * I * H;
     const bool past_caches = om_weights_pass_caches(w_gate, weights, H, p.strideB) && om_weights_pass_caches(w_up, weights, H, p.strideB);
-    if (G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I, past_caches))
+    const bool streams = G <= MAX_EXPERTS && om_ggemm_streams(expected, G, 2 * I, past_caches);
+    if (dense) {
+        p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1; p.rows = rows;
+        if (!streams && dense_rides<EPI_SWIGLU>(p, expected, dense->rows)) {
+            if (!dense_operands(p, dense)) return OM_ERR_ALIGN;
+            return launch_rows_dense<CONTIG, CONTIG, EPI_SWIGLU, GATHER_A, true>(p, rows, om_stream(stream));
+        }
+        const int code = dense_alone();
+        if (code != OM_OK) return code;
+    }
+    if (streams)
         return om_ggemm_stream_gate_up(x, x_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts, rows, expected, G, I,
                                        H, p.strideB, om_stream(stream));
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
@@ -1659,6 +1776,26 @@ extern "C" int om_merged_mlp_gate_up_fwd_weighted_bound(const void *x, const int
                               rows, expected_rows, G, I, H, w_stride, stream);
 }
 
+extern "C" int om_merged_mlp_gate_up_fwd_weighted_dense(const void *x, const int32_t *x_rows, int64_t src_rows,
+                                                        const void *w_gate, const void *w_up,
+                                                        const float *row_weights, void *g, void *u, void *h,
+                                                        const int32_t *cum_token_counts, int64_t rows,
+                                                        int64_t expected_rows, int G, int I, int H, int64_t w_stride,
+                                                        const om_dense_expert *dense, void *stream) {
+    if (!dense || (rows > 0 && (!x_rows || !row_weights))) return OM_ERR_NULL;
+    if (src_rows < 1 && rows > 0) return OM_ERR_SHAPE;
+    return gate_up_fwd_launch(x, x_rows, src_rows, w_gate, w_up, row_weights, g, u, h, cum_token_counts,
+                              rows, expected_rows, G, I, H, w_stride, stream, dense);
+}
+
+extern "C" int om_merged_mlp_dense_rides(int64_t expected_rows, int G, int I, int H, int64_t dense_rows) {
+    if (expected_rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8) || dense_rows < 1) return OM_ERR_SHAPE;
+    GemmParams p = {};
+    p.n_experts = G; p.n_cols = I; p.kc = H;
+    const bool past_caches = 2 * static_cast<int64_t>(G) * I * H >= CACHED_WEIGHTS && H % 64 == 0;   // (as far as sizes say)
+    return !om_ggemm_streams(expected_rows, G, 2 * I, past_caches) && dense_rides<EPI_SWIGLU>(p, expected_rows, dense_rows) ? 1 : 0;
+}
+
 namespace {
 // columns of the intermediate size that one wavefront's epilogue covers (both tile shapes): the
 // granularity of the row_dot partial sums
@@ -1670,9 +1807,15 @@ static_assert(256 / WAVES_N<256> == ROW_DOT_COLS && 128 / WAVES_N<128> == ROW_DO
 int down_dgrad_launch(const void *dy, const int32_t *dy_rows, int64_t src_rows, const void *w_down,
                       const void *g, const void *u, const float *row_weights, void *dg, void *du,
                       float *row_dot, const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I,
-                      int H, int64_t w_stride, void *stream) {
+                      int H, int64_t w_stride, void *stream, const om_dense_expert *dense = nullptr) {
     if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
-    if (rows == 0) return OM_OK;
+    if (dense && (dense->rows < 1 || !fits_gather(dense->rows * H))) return OM_ERR_SHAPE;
+    if (dense && (!dense->a[0] || !dense->w[0] || !dense->c[0] || !dense->c[1] || !dense->g || !dense->u || !dense->cum)) return OM_ERR_NULL;
+    auto dense_alone = [&]() {
+        return down_dgrad_launch(dense->a[0], nullptr, 0, dense->w[0], dense->g, dense->u, nullptr, dense->c[0], dense->c[1], nullptr,
+                                 dense->cum, dense->rows, dense->rows, 1, I, H, 0, stream);
+    };
+    if (rows == 0) return dense ? dense_alone() : OM_OK;
     if (!dy || !w_down || !g || !u || !dg || !du || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(dy) || !om_aligned16(w_down) || !om_aligned16(g) || !om_aligned16(u) ||
         !om_aligned16(dg) || !om_aligned16(du))
@@ -1694,6 +1837,14 @@ int down_dgrad_launch(const void *dy, const int32_t *dy_rows, int64_t src_rows, 
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G) || !fits_gather(src_rows * H))
         return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = I; p.kc = H; p.phases = 1;
+    if (dense) {
+        if (dense_rides<EPI_SWIGLU_BWD>(p, expected, dense->rows)) {
+            if (!dense_operands(p, dense)) return OM_ERR_ALIGN;
+            return launch_rows_dense<CONTIG, STRIDED, EPI_SWIGLU_BWD, GATHER_A, true>(p, rows, om_stream(stream));
+        }
+        const int code = dense_alone();
+        if (code != OM_OK) return code;
+    }
     if (dy_rows)
         return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD, GATHER_A, true>(p, rows, expected, om_stream(stream));
     return launch_rows_auto<CONTIG, STRIDED, EPI_SWIGLU_BWD>(p, rows, expected, om_stream(stream));
@@ -1735,6 +1886,18 @@ extern "C" int om_merged_mlp_down_dgrad_weighted_bound(const void *dy, const int
                              cum_token_counts, rows, expected_rows, G, I, H, w_stride, stream);
 }
 
+extern "C" int om_merged_mlp_down_dgrad_weighted_dense(const void *dy, const int32_t *dy_rows, int64_t src_rows,
+                                                       const void *w_down, const void *g, const void *u,
+                                                       const float *row_weights, void *dg, void *du,
+                                                       float *row_dot, const int32_t *cum_token_counts,
+                                                       int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                       int64_t w_stride, const om_dense_expert *dense, void *stream) {
+    if (!dense || (rows > 0 && (!dy_rows || !row_weights || !row_dot))) return OM_ERR_NULL;
+    if (src_rows < 1 && rows > 0) return OM_ERR_SHAPE;
+    return down_dgrad_launch(dy, dy_rows, src_rows, w_down, g, u, row_weights, dg, du, row_dot,
+                             cum_token_counts, rows, expected_rows, G, I, H, w_stride, stream, dense);
+}
+
 extern "C" int om_merged_mlp_gate_up_dgrad(const void *dg, const void *du, const void *w_gate,
                                            const void *w_up, void *dx, const int32_t *cum_token_counts,
                                            int64_t rows, int G, int I, int H, int64_t w_stride,
@@ -1743,12 +1906,18 @@ extern "C" int om_merged_mlp_gate_up_dgrad(const void *dg, const void *du, const
                                              stream);
 }
 
-extern "C" int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void *w_gate,
-                                                 const void *w_up, void *dx, const int32_t *cum_token_counts,
-                                                 int64_t rows, int64_t expected_rows, int G, int I, int H,
-                                                 int64_t w_stride, void *stream) {
+namespace {
+int gate_up_dgrad_launch(const void *dg, const void *du, const void *w_gate, const void *w_up, void *dx,
+                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I, int H,
+                         int64_t w_stride, const om_dense_expert *dense, void *stream) {
     if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
-    if (rows == 0) return OM_OK;
+    if (dense && (dense->rows < 1 || !fits_gather(dense->rows))) return OM_ERR_SHAPE;
+    if (dense && (!dense->a[0] || !dense->a[1] || !dense->w[0] || !dense->w[1] || !dense->c[0] || !dense->cum)) return OM_ERR_NULL;
+    auto dense_alone = [&]() {
+        return gate_up_dgrad_launch(dense->a[0], dense->a[1], dense->w[0], dense->w[1], dense->c[0], dense->cum, dense->rows,
+                                    dense->rows, 1, I, H, 0, nullptr, stream);
+    };
+    if (rows == 0) return dense ? dense_alone() : OM_OK;
     if (!dg || !du || !w_gate || !w_up || !dx || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(dg) || !om_aligned16(du) || !om_aligned16(w_gate) || !om_aligned16(w_up) ||
         !om_aligned16(dx))
@@ -1765,5 +1934,29 @@ extern "C" int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du,
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = H; p.kc = I; p.phases = 2;
+    if (dense) {
+        if (dense_rides<EPI_STORE>(p, expected_rows, dense->rows)) {
+            if (!dense_operands(p, dense)) return OM_ERR_ALIGN;
+            return launch_rows_dense<CONTIG, STRIDED, EPI_STORE, GATHER_NONE, false>(p, rows, om_stream(stream));
+        }
+        const int code = dense_alone();
+        if (code != OM_OK) return code;
+    }
     return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, expected_rows, om_stream(stream));
+}
+}  // namespace
+
+extern "C" int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du, const void *w_gate,
+                                                 const void *w_up, void *dx, const int32_t *cum_token_counts,
+                                                 int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                 int64_t w_stride, void *stream) {
+    return gate_up_dgrad_launch(dg, du, w_gate, w_up, dx, cum_token_counts, rows, expected_rows, G, I, H, w_stride, nullptr, stream);
+}
+
+extern "C" int om_merged_mlp_gate_up_dgrad_dense(const void *dg, const void *du, const void *w_gate,
+                                                 const void *w_up, void *dx, const int32_t *cum_token_counts,
+                                                 int64_t rows, int64_t expected_rows, int G, int I, int H,
+                                                 int64_t w_stride, const om_dense_expert *dense, void *stream) {
+    if (!dense) return OM_ERR_NULL;
+    return gate_up_dgrad_launch(dg, du, w_gate, w_up, dx, cum_token_counts, rows, expected_rows, G, I, H, w_stride, dense, stream);
 }

@@ -512,9 +512,25 @@ Tensor merged_backward(const Call &c, Tensor dy, const Tensor &x, const MlpWeigh
     return dx;
 }
 
-// The routed half of a bf16 block: gather, weighted SwiGLU MLP, unweighted sum of a token's rows.
+// The shared expert of a block as it goes along with the routed ones, whose extents it has (om_dense_expert).
+struct Alongside {
+    const MlpWeights &w;
+    MlpState &s;             // the forward's; its cum: device {0, tokens}
+    Tensor y;                // its output
+    static bool fits(const MlpWeights &w, const MlpWeights &routed) {
+        return w.I() == routed.I() && w.H() == routed.H() && w.gate.is_contiguous() && w.up.is_contiguous() && w.down.is_contiguous();
+    }
+};
+om_dense_expert dense_expert(std::array<const Tensor *, 2> a, std::array<const Tensor *, 2> w, std::array<const Tensor *, 3> cs,
+                             const MlpState &s, int64_t rows) {
+    auto p = [](const Tensor *t) { return t ? ptr(*t) : nullptr; };
+    return {{p(a[0]), p(a[1])}, {p(w[0]), p(w[1])}, {p(cs[0]), p(cs[1]), p(cs[2])}, ptr(s.g), ptr(s.u), iptr(s.cum), rows};
+}
+
+// The routed half of a bf16 block: gather, weighted SwiGLU MLP, unweighted sum of a token's rows.  `along`: and the shared
+// expert, whose output is the residual.
 Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const Index &ix, const MlpWeights &w,
-                      const Tensor &residual, MlpState &s, Tensor &row_weights) {
+                      Tensor residual, MlpState &s, Tensor &row_weights, Alongside *along = nullptr) {
     require_mlp_operands(x, w);
     if (rw.dim() != 2 || rw.size(0) != x.size(0)) throw NativeError("routing weights: expected [tokens, top_k]");
     if (residual.defined()) {
@@ -542,10 +558,22 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
             weights = fp(row_weights);
             OM(c, om_moe_row_weights, ptr(rw), ix.sel, ix.in, ix.out, fpm(row_weights), rows, K, dtype_code(rw), c.stream);
         }
-        OM_BOUND(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
-                 ptr(s.u), ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, c.stream);
-        OM_BOUND(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
-                 expert_stride(w.down), c.stream);
+        if (along) {
+            MlpState &d = along->s;
+            for (Tensor *t : {&d.g, &d.u, &d.h}) *t = make({T, I}, x);
+            residual = along->y = make({T, H}, x);
+            const om_dense_expert up = dense_expert({&x, nullptr}, {&along->w.gate, &along->w.up}, {&d.g, &d.u, &d.h}, d, T);
+            OM(c, om_merged_mlp_gate_up_fwd_weighted_dense, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g), ptr(s.u),
+               ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, &up, c.stream);
+            const om_dense_expert down = dense_expert({&d.h, nullptr}, {&along->w.down, nullptr}, {&along->y, nullptr, nullptr}, d, T);
+            OM(c, om_grouped_gemm_fwd_dense, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
+               expert_stride(w.down), &down, c.stream);
+        } else {
+            OM_BOUND(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
+                     ptr(s.u), ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, c.stream);
+            OM_BOUND(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
+                     expert_stride(w.down), c.stream);
+        }
     }
     ProfiledScope scope(c, "1moeblock--8gmlp_output_reduction_fwd");
     OM(c, om_sum_ggemm_output, ptr(y), ix.cum_ep, ix.out, ptr(residual), ptr(final), T, H, OM_BF16, c.stream);
@@ -553,10 +581,12 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
 }
 
 // -> (dx, d routing_weights); `base` [T,H]: another gradient of the same hidden states, added to dx
-// inside the per-token sum.
+// inside the per-token sum.  `along`: the shared expert's backward as well, whose input gradient is that base; its weight
+// gradients go into `along_sinks`.
 std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, const Tensor &x, const Tensor &rw,
                                           const Index &ix, const MlpWeights &w, const MlpState &s,
-                                          const Tensor &row_weights, const Sinks &k, const Tensor &base) {
+                                          const Tensor &row_weights, const Sinks &k, Tensor base, Alongside *along = nullptr,
+                                          const Sinks *along_sinks = nullptr) {
     const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
     Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx_rows = make({rows, H}, x);
     // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window stay zero
@@ -568,14 +598,31 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
             const int parts = om_merged_mlp_row_dot_parts(I);
             if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
             Tensor row_dot = make({parts, rows}, x, at::kFloat);
-            OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u),
-                     ix.row_weights ? ix.row_weights : fp(row_weights), ptr(dg), ptr(du), fpm(row_dot), ix.cum, rows,
-                     ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
+            const float *row_w = ix.row_weights ? ix.row_weights : fp(row_weights);
+            Tensor dense_dg, dense_du;
+            if (along) {
+                dense_dg = make({T, I}, x);
+                dense_du = make({T, I}, x);
+                base = make({T, H}, x);
+                const om_dense_expert d = dense_expert({&dfinal, nullptr}, {&along->w.down, nullptr}, {&dense_dg, &dense_du, nullptr}, along->s, T);
+                OM(c, om_merged_mlp_down_dgrad_weighted_dense, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u), row_w, ptr(dg),
+                   ptr(du), fpm(row_dot), ix.cum, rows, ix.to_choose_by(), G, I, H, expert_stride(w.down), &d, c.stream);
+                wgrads(c, dfinal, nullptr, along->s.h, dense_dg, dense_du, x, nullptr, *along_sinks, iptr(along->s.cum), T, T, 1, I, H);
+            } else {
+                OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u), row_w, ptr(dg),
+                         ptr(du), fpm(row_dot), ix.cum, rows, ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
+            }
             OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
                c.stream);
             wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, ix.to_choose_by(), G, I, H);
-            OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
-                     ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
+            if (along) {
+                const om_dense_expert d = dense_expert({&dense_dg, &dense_du}, {&along->w.gate, &along->w.up}, {&base, nullptr, nullptr}, along->s, T);
+                OM(c, om_merged_mlp_gate_up_dgrad_dense, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
+                   ix.to_choose_by(), G, I, H, expert_stride(w.gate), &d, c.stream);
+            } else {
+                OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
+                         ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
+            }
         } else {   // nothing routed to these experts: fresh weight gradients are zero, live ones stay as they are
             for (const Sink *sk : {&k.down, &k.gate, &k.up})
                 if (!sk->accumulate) {
@@ -588,6 +635,15 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
     require_device(base);
     OM(c, om_sum_ggemm_output, ptr(dx_rows), ix.cum_ep, ix.out, ptr(base), ptr(dx), T, H, OM_BF16, c.stream);
     return {dx, drw};
+}
+
+// What merged_forward checks of a shared expert, for one that goes along with the routed experts.
+void require_shared_operands(const Tensor &x, const MlpWeights &w, const Tensor &one, MlpState &s) {
+    require_mlp_operands(x, w);
+    require_device(x);
+    gemm_dtype(x, w.gate, w.up);
+    gemm_dtype(x, w.gate, w.down);
+    s.cum = one;
 }
 
 // ---- autograd plumbing --------------------------------------------------------------------------------
@@ -1036,12 +1092,14 @@ struct RoutedNode : HostNode {
         index.resolve();
         Tensor base;
         Sinks ks;
+        Alongside along{ws, ss, Tensor()};
+        const bool together = has_shared && index.rows > 0 && Alongside::fits(ws, w);
         if (has_shared) {   // first: its input gradient is the base of the routed experts' per-token sum
             ks = sinks_of(c, shared, ws);
-            base = merged_backward(c, dfinal, kept[0], ws, iptr(ss.cum), ss, nullptr, ks);
+            if (!together) base = merged_backward(c, dfinal, kept[0], ws, iptr(ss.cum), ss, nullptr, ks);
         }
         const Sinks k = sinks_of(c, routed, w);
-        auto d = routed_backward(c, dfinal, kept[0], kept[1], index, w, s, kept[2], k, base);
+        auto d = routed_backward(c, dfinal, kept[0], kept[1], index, w, s, kept[2], k, base, together ? &along : nullptr, &ks);
         variable_list out = {d.first, d.second, has_residual ? grads[0] : Tensor()};
         out.reserve(n_in);
         push_grads(out, k, routed);
@@ -1067,12 +1125,17 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
         xc = x.contiguous();
         rwc = rw.contiguous();
         Tensor residual = residual_in.defined() ? residual_in.contiguous() : Tensor();
+        Alongside along{ws, ss, Tensor()};
+        bool together = false;
         if (has_shared) {
             ws = weights_of(shared, true, 1);
-            residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
+            // (the host waits for the rows behind the shared expert's kernels, where it has to)
+            together = !after_shared && xc.size(0) > 0 && Alongside::fits(ws, w);
+            if (together) require_shared_operands(xc, ws, one, ss);
+            else residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
         }
         if (after_shared) after_shared(ix);
-        final = routed_forward(c, xc, rwc, ix, w, residual, s, row_weights);
+        final = routed_forward(c, xc, rwc, ix, w, residual, s, row_weights, together ? &along : nullptr);
     }
     if (any_requires_grad(inputs)) {
         auto node = make_node<RoutedNode>(inputs);
@@ -1204,6 +1267,16 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
             // read the count back (as the reference does), behind the shared expert's kernels: they do not
             // need it, and while the GPU runs them the host waits for a copy that was enqueued before them
             auto count = std::make_shared<CountReadback>(ix.cum + (end - start), c.stream);
+            // unless they are those of the routed experts and, alone, too few for the chip (fewer tiles than three quarters
+            // of its CUs): then that saves more than the wait costs.  Forward passes, us, behind them -> together: 7168/2048 of
+            // 600 tokens (160 tiles) 566 -> 516, 3000/1000 of 1000 (128) 248 -> 234; but 1200/1000 of 3000 (384) 187 -> 191,
+            // 1024/256 of 8000 (252) 146 -> 155.
+            const int64_t tiles = (x.size(0) + 127) / 128 * ((I + 63) / 64);
+            if (has_shared && one && tiles < 192 && om_merged_mlp_dense_rides(ix.rows * (end - start) / n_total, static_cast<int>(end - start),
+                                                               static_cast<int>(I), static_cast<int>(H), x.size(0)) == 1) {
+                ix.rows = count->wait();
+                return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, *one);
+            }
             return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared,
                                   one.value_or(Tensor()), [count](Index &index) { index.rows = count->wait(); });
         }

@@ -1,0 +1,94 @@
+"""The shared expert in the routed experts' launches (om_*_dense): the routed outputs are the bits of the calls without it,
+and the shared expert's those of a call of its own, wherever that runs on the same tiles."""
+import ctypes
+
+import pytest
+import torch
+
+from util import assert_bf16_parity
+
+pytestmark = pytest.mark.gpu
+
+
+class Dense(ctypes.Structure):
+    _fields_ = [("a", ctypes.c_void_p * 2), ("w", ctypes.c_void_p * 2), ("c", ctypes.c_void_p * 3), ("g", ctypes.c_void_p),
+                ("u", ctypes.c_void_p), ("cum", ctypes.c_void_p), ("rows", ctypes.c_int64)]
+
+
+def _ptrs(n, *ts):
+    return (ctypes.c_void_p * n)(*([t.data_ptr() for t in ts] + [None] * (n - len(ts))))
+
+
+# tokens at the edges of 64-row units and 128-row tiles; extents that no tile divides; one expert; experts without rows; a
+# bound of the rows above those routed; 2200 tokens, whose shared expert takes 256x256 tiles of its own
+@pytest.mark.parametrize("T,G,I,H,rows,bound", [(17, 8, 72, 40, 9, 34), (64, 32, 256, 1024, 64, 512), (128, 1, 136, 328, 5, 5),
+                                                (129, 12, 200, 264, 387, 387), (300, 5, 512, 256, 0, 600), (2200, 3, 1024, 2048, 40, 40)])
+def test_dense_expert_beside_the_routed_ones(cuda, T, G, I, H, rows, bound):
+    from optimus import _native
+    lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator().manual_seed(T + G)
+
+    def rnd(*s, scale=1.0):
+        return (torch.randn(*s, generator=gen) * scale).to(torch.bfloat16).to(cuda)
+
+    def new(*s):
+        return torch.full(s, float("nan"), dtype=torch.bfloat16, device=cuda)
+
+    cuts = torch.sort(torch.randint(0, rows + 1, (G - 1,), generator=gen)).values
+    cum = torch.cat([torch.zeros(1), cuts, torch.full((1,), rows)]).to(torch.int32).to(cuda)
+    idx = torch.randint(0, T, (bound,), generator=gen).to(torch.int32).to(cuda)
+    w = torch.rand(bound, generator=gen).to(cuda)
+    one = torch.tensor([0, T], dtype=torch.int32, device=cuda)
+    x, dy = rnd(T, H), rnd(T, H)
+    wg, wu, wd = rnd(G, I, H, scale=0.1), rnd(G, I, H, scale=0.1), rnd(G, H, I, scale=0.1)
+    sg, su, sd = rnd(I, H, scale=0.1), rnd(I, H, scale=0.1), rnd(H, I, scale=0.1)
+    P = lambda t: t.data_ptr()
+    parts = lib.om_merged_mlp_row_dot_parts(I)
+    expected = max(rows, 1) if bound > rows else bound
+
+    def run(dense):
+        r = {k: new(bound, I) for k in ("g", "u", "h", "dg", "du")} | {k: new(bound, H) for k in ("y", "dx")}
+        s = {k: new(T, I) for k in ("g", "u", "h", "dg", "du")} | {k: new(T, H) for k in ("y", "dx")}
+        r["dot"] = torch.zeros(parts, bound, device=cuda)
+        tail = (P(cum), bound, expected, G)
+
+        def call(name, args, dims, a, ws, cs, alone):
+            if dense:
+                d = Dense(_ptrs(2, *a), _ptrs(2, *ws), _ptrs(3, *cs), P(s["g"]), P(s["u"]), P(one), T)
+                assert getattr(lib, name + "_dense")(*args, *tail, *dims, 0, ctypes.addressof(d), st) == 0
+            else:
+                assert getattr(lib, name + "_bound")(*args, *tail, *dims, 0, st) == 0
+                assert alone() == 0
+
+        call("om_merged_mlp_gate_up_fwd_weighted", (P(x), P(idx), T, P(wg), P(wu), P(w), P(r["g"]), P(r["u"]), P(r["h"])), (I, H),
+             (x,), (sg, su), (s["g"], s["u"], s["h"]),
+             lambda: lib.om_merged_mlp_gate_up_fwd(P(x), P(sg), P(su), P(s["g"]), P(s["u"]), P(s["h"]), P(one), T, 1, I, H, 0, st))
+        call("om_grouped_gemm_fwd", (P(r["h"]), P(wd), P(r["y"])), (H, I), (s["h"],), (sd,), (s["y"],),
+             lambda: lib.om_grouped_gemm_fwd(P(s["h"]), P(sd), P(s["y"]), P(one), T, 1, H, I, 0, st))
+        call("om_merged_mlp_down_dgrad_weighted",
+             (P(dy), P(idx), T, P(wd), P(r["g"]), P(r["u"]), P(w), P(r["dg"]), P(r["du"]), P(r["dot"])), (I, H),
+             (dy,), (sd,), (s["dg"], s["du"]),
+             lambda: lib.om_merged_mlp_down_dgrad(P(dy), P(sd), P(s["g"]), P(s["u"]), P(s["dg"]), P(s["du"]), P(one), T, 1, I, H, 0, st))
+        call("om_merged_mlp_gate_up_dgrad", (P(r["dg"]), P(r["du"]), P(wg), P(wu), P(r["dx"])), (I, H), (s["dg"], s["du"]),
+             (sg, su), (s["dx"],),
+             lambda: lib.om_merged_mlp_gate_up_dgrad(P(s["dg"]), P(s["du"]), P(sg), P(su), P(s["dx"]), P(one), T, 1, I, H, 0, st))
+        torch.cuda.synchronize()
+        return r, s
+
+    (r, s), (r0, s0) = run(True), run(False)
+    for k in r:
+        got, want = (r[k][:, :rows], r0[k][:, :rows]) if k == "dot" else (r[k][:rows], r0[k][:rows])
+        assert torch.equal(got, want), k
+        if k != "dot":
+            assert r[k][rows:].isnan().all(), k          # nothing past the routed rows
+    f = lambda *ts: [t.float().cpu() for t in ts]
+    xf, gf, uf, hf, dgf, duf = f(x, s["g"], s["u"], s["h"], s["dg"], s["du"])
+    sgf, suf, sdf = f(sg, su, sd)
+    # each product against float32 on the operands that it had (the bar of a single rounding, as for the other entry points)
+    assert_bf16_parity(s["g"], xf @ sgf.t(), 1.03, 1.8e-3, "dense g")
+    assert_bf16_parity(s["u"], xf @ suf.t(), 1.03, 1.8e-3, "dense u")
+    assert_bf16_parity(s["y"], hf @ sdf.t(), 1.03, 1.8e-3, "dense y")
+    assert_bf16_parity(s["dx"], dgf @ sgf + duf @ suf, 1.03, 1.8e-3, "dense dx")
+    if T > 80:   # (a launch of its own with fewer rows adds a forward product up in another order)
+        for k in s:
+            assert torch.equal(s[k], s0[k]), k
