@@ -1442,6 +1442,46 @@ Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const
     return final;
 }
 
+// ---- optimizer ----------------------------------------------------------------------------------------
+// A step of a small optimizer is two launches of 7 to 10 us; through ctypes, with the operands looked over in Python, they
+// took the host 29 us (22 now, 21 a step among others).
+
+bool flat_buffer(const Tensor &t, int64_t n) { return t.is_cuda() && t.is_contiguous() && t.numel() == n; }
+
+// The update of adamw_step_; false: operands that its Python part refuses (it raises).
+bool adamw_step(const Tensor &param, const Tensor &grad, const Tensor &master, const Tensor &exp_avg, const Tensor &exp_avg_sq,
+                int64_t step, double lr, double beta1, double beta2, double eps, double weight_decay,
+                const std::optional<Tensor> &grad_scale, bool store_scaled_grad) {
+    const int64_t n = master.numel();
+    for (const Tensor *t : {&param, &grad, &master, &exp_avg, &exp_avg_sq})
+        if (!flat_buffer(*t, n)) return false;
+    for (const Tensor *t : {&master, &exp_avg, &exp_avg_sq})
+        if (t->scalar_type() != at::kFloat) return false;
+    const auto dt = param.scalar_type();
+    if (grad.scalar_type() != dt || (dt != at::kBFloat16 && (dt != at::kFloat || param.data_ptr() != master.data_ptr()))) return false;
+    if (grad_scale && (!flat_buffer(*grad_scale, 1) || grad_scale->scalar_type() != at::kFloat)) return false;
+    const Call c = begin_call();
+    if (grad_scale)
+        OM(c, om_adamw_step_clipped, ptr(param), ptr(grad), fpm(master), fpm(exp_avg), fpm(exp_avg_sq), n, lr, beta1, beta2, eps,
+           weight_decay, step, dtype_code(param), fp(*grad_scale), store_scaled_grad, c.stream);
+    else
+        OM(c, om_adamw_step, ptr(param), ptr(grad), fpm(master), fpm(exp_avg), fpm(exp_avg_sq), n, lr, beta1, beta2, eps,
+           weight_decay, step, dtype_code(param), c.stream);
+    return true;
+}
+
+// GradNormPlan's one-launch form; words: total norm, clip coefficient, the kernel's block count.
+void grad_norm(const Tensor &grad, const Tensor &chunk_offsets, int64_t n_chunks, const Tensor &seg_first_chunk, int64_t n_segs,
+               double max_norm, const Tensor &partials, const Tensor &seg_norms, const Tensor &words,
+               const std::optional<Tensor> &norm_out) {
+    require_device(grad);
+    const Call c = begin_call();
+    float *w = fpm(words);
+    OM(c, om_grad_norm, ptr(grad), dtype_code(grad), chunk_offsets.data_ptr<int64_t>(), n_chunks, seg_first_chunk.data_ptr<int64_t>(),
+       n_segs, max_norm, fpm(partials), fpm(seg_norms), w, w + 1, norm_out ? ptr(*norm_out) : nullptr,
+       reinterpret_cast<unsigned *>(w + 2), c.stream);
+}
+
 // ---- Python module ----------------------------------------------------------------------------------
 
 PyObject *module_base() {   // torch.nn.Module (kept for good)
@@ -1594,6 +1634,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         at::NoGradGuard no_grad;
         return strided_view(weights.data(), 1, static_cast<int64_t>(weights.size()));
     });
+    m.def("adamw_step", &adamw_step, no_gil);
+    m.def("grad_norm", &grad_norm, no_gil);
     m.def("sized_by_bound", &sized_by_bound);
     m.def("live_grad", [](const Tensor &param) {
         Tensor grad = live_grad(param);

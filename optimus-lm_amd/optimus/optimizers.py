@@ -417,6 +417,10 @@ def adamw_step_(flat_param, flat_grad, flat_master, flat_exp_avg, flat_exp_avg_s
     optimus/optimizers.py:162-205, as a single HIP pass).  `step` is 1-based (step_id + 1).
     `grad_scale` (device fp32 scalar) folds the gradient clip in: the update uses
     cast(grad * grad_scale), and stores it back into flat_grad if `store_scaled_grad`."""
+    if _n.host().adamw_step(flat_param, flat_grad, flat_master, flat_exp_avg, flat_exp_avg_sq, int(step), float(lr),
+                            float(beta1), float(beta2), float(eps), float(weight_decay), grad_scale, bool(store_scaled_grad)):
+        return
+    # not operands that the kernels take: say which
     _n.require_cuda_contiguous(flat_param, flat_grad, flat_master, flat_exp_avg, flat_exp_avg_sq)
     n = flat_master.numel()
     if flat_grad.numel() != n or flat_exp_avg.numel() != n or flat_exp_avg_sq.numel() != n \
@@ -429,22 +433,10 @@ def adamw_step_(flat_param, flat_grad, flat_master, flat_exp_avg, flat_exp_avg_s
         if flat_param.data_ptr() != flat_master.data_ptr() or flat_grad.dtype != torch.float32:
             raise ValueError("float32 mode: flat_fp32_master_param must alias flat_param and "
                              "flat_grad must be float32 (reference optimizers.py:100-102)")
-        code = _n.OM_F32
-    elif flat_param.dtype == torch.bfloat16 and flat_grad.dtype == torch.bfloat16:
-        code = _n.OM_BF16
-    else:
+    elif flat_param.dtype != torch.bfloat16 or flat_grad.dtype != torch.bfloat16:
         raise TypeError("flat_param / flat_grad must both be bfloat16 or both float32")
-    args = (_n.ptr(flat_param), _n.ptr(flat_grad), _n.ptr(flat_master), _n.ptr(flat_exp_avg),
-            _n.ptr(flat_exp_avg_sq), n, float(lr), float(beta1), float(beta2), float(eps),
-            float(weight_decay), int(step), code)
-    if grad_scale is None:
-        _n.check(_n.lib().om_adamw_step(*args, _n.stream()), "om_adamw_step")
-    else:
-        _n.require_cuda_contiguous(grad_scale)
-        if grad_scale.dtype != torch.float32 or grad_scale.numel() != 1:
-            raise TypeError("grad_scale must be one float32 element on the device")
-        _n.check(_n.lib().om_adamw_step_clipped(*args, _n.ptr(grad_scale), int(bool(store_scaled_grad)),
-                                                _n.stream()), "om_adamw_step_clipped")
+    _n.require_cuda_contiguous(grad_scale)
+    raise TypeError("grad_scale must be one float32 element on the device")
 
 
 class GradNormPlan:
@@ -495,14 +487,11 @@ class GradNormPlan:
         """Returns (total_norm, clip_coef) as 0-dim float32 device tensors (views of one buffer
         that the next call overwrites).  `norm_out`: a 0-dim tensor of the gradient dtype that receives
         the total norm too."""
-        _n.require_cuda_contiguous(flat_grad)
         if self.one_launch:
-            _n.check(_n.lib().om_grad_norm(
-                _n.ptr(flat_grad), _n.dtype_code(flat_grad), _n.ptr(self.chunk_offsets), self.n_chunks,
-                _n.ptr(self.seg_first_chunk), self.n_segs, float(max_norm), _n.ptr(self.partials),
-                _n.ptr(self.seg_norms), _n.ptr(self._words), _n.ptr(self._words) + 4, _n.ptr(norm_out),
-                _n.ptr(self._words) + 8, _n.stream()), "om_grad_norm")
+            _n.host().grad_norm(flat_grad, self.chunk_offsets, self.n_chunks, self.seg_first_chunk, self.n_segs,
+                                float(max_norm), self.partials, self.seg_norms, self._words, norm_out)
             return self.total, self.coef
+        _n.require_cuda_contiguous(flat_grad)
         code = _n.dtype_code(flat_grad)
         lib = _n.lib()
         _n.check(lib.om_grad_sumsq(_n.ptr(flat_grad), code, _n.ptr(self.chunk_offsets), self.n_chunks,
