@@ -82,6 +82,19 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
+// Stores a vector (8 or 16 bytes a lane) past the caches, `bytes` behind a block-uniform address; bytes < 2^31.  Of the cache
+// policies of a store nt alone leaves the lines in the L2s, which write them back in their own order, when the kernel ends or under the
+// next one; with sc1 as well they go on to memory at once.  Weight gradients of 64 experts of 2048/1024, 512 tokens with popularity as
+// rank^-1.2, whole training steps, us: through the caches 656, nt 618, sc1 656, sc0 sc1 658, sc1 nt 593, sc0 sc1 nt 596 (two
+// boxes, one side of each 604 to 606).  No gain for gradients that were just read to be added to.
+template <typename T> __device__ __forceinline__ void store_past_caches(void *base, uint32_t bytes, T v) {
+    constexpr int SC1_NT = 16 | 2;
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00020000);
+    static_assert(sizeof(T) == 16 || sizeof(T) == 8, "one vector a lane");
+    if constexpr (sizeof(T) == 16) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, bytes, 0, SC1_NT);
+    else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rsrc, bytes, 0, SC1_NT);
+}
+
 // Direct load of 16 bytes from each lane's address to LDS at lds + 16 * lane.  Outside the compiler's view: the code waits
 // for it itself (vmcnt counts it).
 __device__ __forceinline__ void dma16_lane(const char *lane_address, uint32_t lds) {

@@ -1171,7 +1171,9 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                             v[y] = pack2_bf16(prev[2 * y] + fresh[2 * y], prev[2 * y + 1] + fresh[2 * y + 1]);
                     }
                     u32x4 *to = reinterpret_cast<u32x4 *>(chunk_at(Cb, i, x));
-                    if (decltype(past_caches)::value) __builtin_nontemporal_store(v, to);
+                    if (decltype(past_caches)::value && !ACCUM)
+                        store_past_caches(Cb + tile_at, (lane_at + static_cast<uint32_t>(i * 64 + x * 8) * static_cast<uint32_t>(e_ldc)) * 2, v);
+                    else if (decltype(past_caches)::value) __builtin_nontemporal_store(v, to);
                     else *to = v;
                     if (ACCUM) __builtin_amdgcn_sched_barrier(0);   // (all of them at once spill registers)
                 }
@@ -1438,6 +1440,8 @@ int wgrad_share(bool big, int tiles_e, int n_experts, int64_t rows, bool accumul
     return big && tiles_e >= 12 * NUM_XCD && n_experts <= SHARE_MAX_EXPERTS ? NUM_XCD : 0;
 }
 
+constexpr int STREAM_MAX_PITCH = 1 << 21;   // elements; 256 rows of a tile span less than the 2^31 bytes of store_past_caches
+
 // weight gradient; gather == GATHER_B: contraction row c of `input` is row index[c] of a
 // [src_rows, K] matrix; gather == GATHER_WA: contraction row c of `output_grad` is row index[c] of a
 // [src_rows, N] matrix (the token gather folded into the loads)
@@ -1466,7 +1470,7 @@ int wgrad_launch(const void *output_grad, const void *input, const int32_t *inde
     const bool big = wgrad_big_tile(N, K, G);
     p.tiles_e = big ? (N / 256) * (K / 256) : ((N + 127) / 128) * ((K + 127) / 128);
     p.share = wgrad_share(big, p.tiles_e, G, expected < 0 ? rows : expected, accumulate);
-    p.stream = om_weights_pass_caches(weight_grad, static_cast<int64_t>(G) * N * K, K, p.strideC);
+    p.stream = K <= STREAM_MAX_PITCH && om_weights_pass_caches(weight_grad, static_cast<int64_t>(G) * N * K, K, p.strideC);
     const int64_t tiles = static_cast<int64_t>(p.tiles_e) * G;
     if (tiles > 0x7fffffffLL) return OM_ERR_SHAPE;
     p.total_tiles = static_cast<int>(tiles);
@@ -1629,7 +1633,7 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     p.tiles_e = static_cast<int>(3 * each);
     p.share = wgrad_share(big, p.tiles_e, G, expected, accumulate);
     p.stream = true;
-    for (const WgradSet &s : p.set) p.stream &= om_weights_pass_caches(s.C, 3 * packed * G, s.n, s.strideC);
+    for (const WgradSet &s : p.set) p.stream &= s.n <= STREAM_MAX_PITCH && om_weights_pass_caches(s.C, 3 * packed * G, s.n, s.strideC);
     p.total_tiles = static_cast<int>(tiles);
     const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);
