@@ -250,59 +250,82 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
 }
 
 // Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (up to 8 x 64)
-// pairs' keys and ranks in registers between the passes.  A decode batch or a small training batch spends
-// nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced),
-// one of 6 now.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront)
-// reaches what the three launches take.
-constexpr int SMALL_WAVES = 16, SMALL_ITERS = 8;
-constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SMALL_ITERS;
+// pairs' keys, weights and ranks in registers between the passes.  A decode batch or a small training batch spends
+// nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced), one of 6 when the
+// caches are warm.  So no step waits for another's loads (ITERS, the 64-pair steps of a wavefront, is known to the compiler, and
+// pairs past the end are read as the last one), the rank of a pair within its expert comes from the counting pass, and
+// only that pass is a chain through LDS: 4096 pairs with cold caches, in a training step of 512 tokens of 64 experts, 15.2 ->
+// 9.8 us.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront) reaches what the three
+// launches take.
+constexpr int SMALL_WAVES = 16, SMALL_MAX_ITERS = 8;
+constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SMALL_MAX_ITERS;
 constexpr int SMALL_MAX_NR = 256;
-template <typename TI>
+template <typename TI, int ITERS>
 __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
-    const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits, int iters,
+    const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
     int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
     int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
     int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
-    __shared__ int off[SMALL_WAVES][SMALL_MAX_NR];   // counts, then running offsets
-    __shared__ int wave_hits[SMALL_WAVES], chunk_total[SMALL_MAX_NR / 64], kept_total;
+    __shared__ int off[SMALL_WAVES][SMALL_MAX_NR];   // counts, then the first position of a wavefront's rows of an expert
+    __shared__ __attribute__((aligned(16))) int wave_hits[SMALL_WAVES], chunk_total[SMALL_MAX_NR / 64];
+    __shared__ int kept_total;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    for (int i = tid; i < SMALL_WAVES * NR; i += SMALL_WAVES * 64) off[i / NR][i % NR] = 0;
-    const int base = wv * iters * 64;
-    int key[SMALL_ITERS];
+    const int base = wv * ITERS * 64 + lane;
+    TI e[ITERS];
 #pragma unroll
-    for (int it = 0; it < SMALL_ITERS; it++)
-        key[it] = it < iters ? local_key(selected_experts, base + it * 64 + lane, n_pairs, start, end, NR) : NR;
-    float weight[SMALL_ITERS];
+    for (int it = 0; it < ITERS; it++) e[it] = selected_experts[min(base + it * 64, n_pairs - 1)];
+    float weight[ITERS] = {};
+    if (rw.row_weights && rw.bf16) {
+        uint16_t bits[ITERS];
 #pragma unroll
-    for (int it = 0; it < SMALL_ITERS; it++) weight[it] = it < iters ? rw.get(base + it * 64 + lane, n_pairs) : 0.0f;
-    __syncthreads();
+        for (int it = 0; it < ITERS; it++) bits[it] = static_cast<const uint16_t *>(rw.routing_weights)[min(base + it * 64, n_pairs - 1)];
+#pragma unroll
+        for (int it = 0; it < ITERS; it++) weight[it] = bf16_bits_to_f32(bits[it]);
+    } else if (rw.row_weights) {
+#pragma unroll
+        for (int it = 0; it < ITERS; it++) weight[it] = static_cast<const float *>(rw.routing_weights)[min(base + it * 64, n_pairs - 1)];
+    }
     volatile int *mine = off[wv];
-    int hits = 0;
+    for (int i = lane; i < NR; i += 64) mine[i] = 0;
+    __builtin_amdgcn_wave_barrier();
+    int key[ITERS], rank[ITERS], before_in_step[ITERS], hits = 0;   // before_in_step: kept pairs of this wavefront before this one
 #pragma unroll
-    for (int it = 0; it < SMALL_ITERS; it++) {
-        if (it >= iters) break;
-        const unsigned long long m = match_key(key[it], nbits);
-        if (key[it] < NR && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] += __popcll(m);
-        hits += __popcll(__ballot(key[it] < NR));
+    for (int it = 0; it < ITERS; it++) {
+        const long long v = static_cast<long long>(e[it]);
+        const bool kept = base + it * 64 < n_pairs && v >= start && v < end;
+        key[it] = kept ? static_cast<int>(v - start) : NR;
+        const unsigned long long m = match_key(key[it], nbits), all = __ballot(kept);
+        const int seen = mine[kept ? key[it] : 0];
+        __builtin_amdgcn_wave_barrier();
+        rank[it] = seen + __popcll(m & lanemask_lt(lane));
+        if (kept && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] = seen + __popcll(m);
+        before_in_step[it] = hits + __popcll(all & lanemask_lt(lane));
+        hits += __popcll(all);
         __builtin_amdgcn_wave_barrier();
     }
     if (lane == 0) wave_hits[wv] = hits;
     __syncthreads();
     // thread e: expert e's total over the wavefronts, exclusive positions of the wavefronts within it
-    int total = 0;
-    if (tid < NR)
+    int total = 0, at[SMALL_WAVES];
+    if (tid < NR) {
+#pragma unroll
+        for (int w = 0; w < SMALL_WAVES; w++) at[w] = off[w][tid];
+#pragma unroll
         for (int w = 0; w < SMALL_WAVES; w++) {
-            const int c = off[w][tid];
-            off[w][tid] = total;
+            const int c = at[w];
+            at[w] = total;
             total += c;
         }
+    }
     const int incl = wave_incl_scan(total, lane);
     if (tid < SMALL_MAX_NR && lane == 63) chunk_total[wv] = incl;
     __syncthreads();
     int before = incl - total;   // rows of the experts before this one
-    for (int w = 0; w < wv && w < SMALL_MAX_NR / 64; w++) before += chunk_total[w];
+#pragma unroll
+    for (int w = 0; w < SMALL_MAX_NR / 64; w++) before += w < wv ? chunk_total[w] : 0;
     if (tid < NR) {
-        for (int w = 0; w < SMALL_WAVES; w++) off[w][tid] += before;
+#pragma unroll
+        for (int w = 0; w < SMALL_WAVES; w++) off[w][tid] = before + at[w];
         cum_token_counts[tid] = before;
         if (tid == NR - 1) {
             cum_token_counts[NR] = before + total;
@@ -312,35 +335,29 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
     }
     __syncthreads();
     int oi_base = 0;
-    for (int w = 0; w < wv; w++) oi_base += wave_hits[w];
+#pragma unroll
+    for (int w = 0; w < SMALL_WAVES; w++) oi_base += w < wv ? wave_hits[w] : 0;
     const int kept_all = kept_total;
 #pragma unroll
-    for (int it = 0; it < SMALL_ITERS; it++) {
-        if (it >= iters) break;
-        const int j = base + it * 64 + lane;
-        if (j < n_pairs && j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
+    for (int it = 0; it < ITERS; it++) {
+        const int j = base + it * 64;
+        if (j >= n_pairs) continue;
+        if (j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
             output_indices[j] = -1;
             input_indices[j] = 0;
             selected_experts_indices[j] = 0;
         }
-        const unsigned long long m = match_key(key[it], nbits);
-        const unsigned long long kept = __ballot(key[it] < NR);
-        const int oi = oi_base + __popcll(kept & lanemask_lt(lane));
-        const bool valid = j < n_pairs;
-        const int t = valid ? j / K : 0, k = valid ? j - t * K : 0;
-        if (valid && k == 0) cum_expert_counts_ep[t] = oi;
-        int pos = 0;
-        if (key[it] < NR) pos = mine[key[it]] + __popcll(m & lanemask_lt(lane));
-        __builtin_amdgcn_wave_barrier();
+        const int oi = oi_base + before_in_step[it];
+        const uint32_t t = static_cast<uint32_t>(j) / static_cast<uint32_t>(K);
+        const int k = j - static_cast<int>(t) * K;
+        if (k == 0) cum_expert_counts_ep[t] = oi;
         if (key[it] < NR) {
-            if ((__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] += __popcll(m);
-            input_indices[pos] = t;
+            const int pos = off[wv][key[it]] + rank[it];
+            input_indices[pos] = static_cast<int32_t>(t);
             output_indices[oi] = pos;
             selected_experts_indices[oi] = k;
             rw.put(pos, weight[it]);
         }
-        oi_base += __popcll(kept);
-        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -472,17 +489,21 @@ int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, in
     const int NR = expert_end_idx - expert_start_idx;
     const int64_t n_pairs = T * K;
     if (n_pairs > 0 && n_pairs <= SMALL_PAIRS && NR <= SMALL_MAX_NR) {
-        const int iters = static_cast<int>((n_pairs + SMALL_WAVES * 64 - 1) / (SMALL_WAVES * 64));
-        if (index_dtype == OM_I64)
-            sort_small_kernel<int64_t><<<1, SMALL_WAVES * 64, 0, st>>>(
-                static_cast<const int64_t *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx,
-                expert_end_idx, NR, key_bits(NR), iters, cum_token_counts, cum_expert_counts_ep, input_indices,
-                output_indices, selected_experts_indices, rw);
-        else
-            sort_small_kernel<int32_t><<<1, SMALL_WAVES * 64, 0, st>>>(
-                static_cast<const int32_t *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx,
-                expert_end_idx, NR, key_bits(NR), iters, cum_token_counts, cum_expert_counts_ep, input_indices,
-                output_indices, selected_experts_indices, rw);
+#define OM_SMALL(TI, ITERS)                                                                                                     \
+    sort_small_kernel<TI, ITERS><<<1, SMALL_WAVES * 64, 0, st>>>(                                                               \
+        static_cast<const TI *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR,          \
+        key_bits(NR), cum_token_counts, cum_expert_counts_ep, input_indices, output_indices, selected_experts_indices, rw)
+#define OM_SMALL_ITERS(TI)                                              \
+    do {                                                                \
+        if (n_pairs <= SMALL_WAVES * 64) OM_SMALL(TI, 1);               \
+        else if (n_pairs <= 2 * SMALL_WAVES * 64) OM_SMALL(TI, 2);      \
+        else if (n_pairs <= 4 * SMALL_WAVES * 64) OM_SMALL(TI, 4);      \
+        else OM_SMALL(TI, SMALL_MAX_ITERS);                             \
+    } while (0)
+        if (index_dtype == OM_I64) OM_SMALL_ITERS(int64_t);
+        else OM_SMALL_ITERS(int32_t);
+#undef OM_SMALL_ITERS
+#undef OM_SMALL
         return om_launch_status();
     }
     const int64_t NB = (n_pairs + SORT_CHUNK - 1) / SORT_CHUNK;

@@ -164,3 +164,13 @@ def test_weighted_sort_on_both_sides_of_the_one_block_line(cuda, oracle_lib, T, 
     want = torch.empty(TR, device=cuda)
     want[pos] = wd[t[pos], si[:TR].long()].float()
     assert torch.equal(rows[:TR], want)
+
+
+@pytest.mark.parametrize("T,N,K,start,end", [
+    (1, 8, 8, 0, 8), (1, 1, 1, 0, 1), (1023, 64, 1, 0, 64), (1024, 64, 1, 0, 64), (1025, 64, 1, 3, 40),
+    (683, 256, 3, 0, 256), (2048, 256, 1, 5, 6), (1366, 12, 3, 0, 12), (512, 64, 8, 8, 16), (4097, 65, 1, 0, 65),
+    (2731, 128, 3, 64, 128), (8191, 7, 1, 0, 7), (4096, 200, 2, 0, 200)])
+def test_one_block_sort_at_its_edges(cuda, oracle_lib, T, N, K, start, end):
+    """Up to 8192 pairs, around 1, 2, 4 and 8 steps a wavefront, experts around whole wavefronts."""
+    for dt in (torch.float32, torch.bfloat16):
+        test_weighted_sort_on_both_sides_of_the_one_block_line(cuda, oracle_lib, T, N, K, start, end, dt)
