@@ -1024,6 +1024,10 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         for (int x = 0; x < 2; x++) chunk[x] = *reinterpret_cast<const u32x4 *>(lds + get_at[x]);
         strip_sync();
     };
+    // The saved g and u of a whole 128x128 tile are loaded at once, ahead of the next tile's look-ups: half a unit at a time they were
+    // four waits in a row.  3001 tokens, hidden 1000, ffn 712, 12 experts, top-3 39.9 -> 37.1 us; 512 tokens, uneven, 64 experts of
+    // 2048/1024 77.5 -> 73.  (256x256: no registers for that.)
+    constexpr bool GU_AHEAD = EPI == EPI_SWIGLU_BWD && TM == 2;
     const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_active = active;
     const int col0 = n0 + wn_e * COLS;   // first output column
     const int chunk_col = (lane_e & (COLS / 8 - 1)) * 8, chunk_row = lane_e >> 3;
@@ -1046,6 +1050,20 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             for (int x = 0; x < 2; x++)
                 weight[ROWW && EPI == EPI_SWIGLU ? i : 0][x] = e_dense ? 1.0f :
                     p.row_scale[min(e_row_begin + (2 * i + wm_e) * 32 + x * 16 + (lane_e & 15), e_row_end - 1)];
+    }
+    u32x4 g_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1], u_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1];
+    float w_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1];
+    if (GU_AHEAD) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) {   // (rows and columns past the tile's: the last ones, not used)
+                const int m = min(e_row_begin + chunk_m(i, x), e_row_end - 1);
+                const int64_t from = static_cast<int64_t>(m) * e_ldc + (EDGE ? min(col0 + chunk_col, e_n_cols - 8) : col0 + chunk_col);
+                g_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.G : p.G) + from));
+                u_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.U : p.U) + from));
+                w_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = ROWW && !e_dense ? p.row_scale[m] : 1.0f;
+            }
     }
     have = next_tile();
     u32x4 old[ACCUM ? TM : 1][ACCUM ? 4 : 1];
@@ -1108,11 +1126,18 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             }
         } else {
             u32x4 chunk[2];
-            u32x4 gq[EPI == EPI_SWIGLU_BWD ? 2 : 1], uq[EPI == EPI_SWIGLU_BWD ? 2 : 1];
+            u32x4 gq[2], uq[2];   // EPI_SWIGLU_BWD
             float wr[2] = {1.0f, 1.0f};
 #pragma unroll
             for (int x = 0; x < 4; x++) {
-                if (EPI == EPI_SWIGLU_BWD && x % 2 == 0) {
+                if (GU_AHEAD && x % 2 == 0) {
+#pragma unroll
+                    for (int y = 0; y < 2; y++) {
+                        gq[y] = g_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
+                        uq[y] = u_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
+                        wr[y] = w_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
+                    }
+                } else if (EPI == EPI_SWIGLU_BWD && x % 2 == 0) {
                     // g, u (and the weights) of half a unit.  They have no reader after this one: past the caches (-1 to -3 %)
 #pragma unroll
                     for (int y = 0; y < 2; y++) {
