@@ -1024,10 +1024,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         for (int x = 0; x < 2; x++) chunk[x] = *reinterpret_cast<const u32x4 *>(lds + get_at[x]);
         strip_sync();
     };
-    // The saved g and u of a whole 128x128 tile are loaded at once, ahead of the next tile's look-ups: half a unit at a time they were
-    // four waits in a row.  3001 tokens, hidden 1000, ffn 712, 12 experts, top-3 39.9 -> 37.1 us; 512 tokens, uneven, 64 experts of
-    // 2048/1024 77.5 -> 73.  (256x256: no registers for that.)
-    constexpr bool GU_AHEAD = EPI == EPI_SWIGLU_BWD && TM == 2;
+    // SwiGLU backward: the saved g and u (and the weights) of two units are loaded ahead of the next tile's look-ups, those of
+    // a further one when its buffer has been used; the fragments' registers are free by now.  Half a unit at a time, behind the next
+    // tile's loads, each was waited for.  us: 3001 tokens, hidden 1000, ffn 712, 12 experts, top-3 (128x128) 39.9 -> 37.1; 512 tokens,
+    // uneven, 64 experts of 2048/1024 77.5 -> 73; 16384 tokens (256x256) 715 -> 660 and less, whole steps of 2048 985 -> 977, 4096
+    // 1546 -> 1524, 16384 uneven 5484 -> 5453 (the power limit keeps the rest), 32 experts of 1024/768, 9000 tokens, 709 -> 700.
+    constexpr bool GU = EPI == EPI_SWIGLU_BWD;
     const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_active = active;
     const int col0 = n0 + wn_e * COLS;   // first output column
     const int chunk_col = (lane_e & (COLS / 8 - 1)) * 8, chunk_row = lane_e >> 3;
@@ -1051,20 +1053,20 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 weight[ROWW && EPI == EPI_SWIGLU ? i : 0][x] = e_dense ? 1.0f :
                     p.row_scale[min(e_row_begin + (2 * i + wm_e) * 32 + x * 16 + (lane_e & 15), e_row_end - 1)];
     }
-    u32x4 g_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1], u_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1];
-    float w_in[GU_AHEAD ? TM : 1][GU_AHEAD ? 4 : 1];
-    if (GU_AHEAD) {
+    u32x4 g_in[GU ? 2 : 1][GU ? 4 : 1], u_in[GU ? 2 : 1][GU ? 4 : 1];   // of even and odd units
+    float w_in[GU ? 2 : 1][GU ? 4 : 1];
+    auto load_gu = [&](int i) {
 #pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int x = 0; x < 4; x++) {   // (rows and columns past the tile's: the last ones, not used)
-                const int m = min(e_row_begin + chunk_m(i, x), e_row_end - 1);
-                const int64_t from = static_cast<int64_t>(m) * e_ldc + (EDGE ? min(col0 + chunk_col, e_n_cols - 8) : col0 + chunk_col);
-                g_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.G : p.G) + from));
-                u_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.U : p.U) + from));
-                w_in[GU_AHEAD ? i : 0][GU_AHEAD ? x : 0] = ROWW && !e_dense ? p.row_scale[m] : 1.0f;
-            }
-    }
+        for (int x = 0; x < 4; x++) {   // (rows and columns past the tile's: the last ones, not used)
+            const int m = min(e_row_begin + chunk_m(i, x), e_row_end - 1), at = GU ? i & 1 : 0, ax = GU ? x : 0;
+            const int64_t from = static_cast<int64_t>(m) * e_ldc + (EDGE ? min(col0 + chunk_col, e_n_cols - 8) : col0 + chunk_col);
+            // no reader after this one: past the caches (-1 to -3 %)
+            g_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.G : p.G) + from));
+            u_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.U : p.U) + from));
+            w_in[at][ax] = ROWW && !e_dense ? p.row_scale[m] : 1.0f;
+        }
+    };
+    if (GU) { load_gu(0); load_gu(1); }
     have = next_tile();
     u32x4 old[ACCUM ? TM : 1][ACCUM ? 4 : 1];
     if (ACCUM) {
@@ -1126,29 +1128,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             }
         } else {
             u32x4 chunk[2];
-            u32x4 gq[2], uq[2];   // EPI_SWIGLU_BWD
-            float wr[2] = {1.0f, 1.0f};
 #pragma unroll
             for (int x = 0; x < 4; x++) {
-                if (GU_AHEAD && x % 2 == 0) {
-#pragma unroll
-                    for (int y = 0; y < 2; y++) {
-                        gq[y] = g_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
-                        uq[y] = u_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
-                        wr[y] = w_in[GU_AHEAD ? i : 0][GU_AHEAD ? x + y : 0];
-                    }
-                } else if (EPI == EPI_SWIGLU_BWD && x % 2 == 0) {
-                    // g, u (and the weights) of half a unit.  They have no reader after this one: past the caches (-1 to -3 %)
-#pragma unroll
-                    for (int y = 0; y < 2; y++) {
-                        const int m = e_row_begin + chunk_m(i, x + y);
-                        if (all_rows || m < row_lim) {
-                            gq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(e_dense ? p.dense.G : p.G, i, x + y)));
-                            uq[y] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(chunk_at(e_dense ? p.dense.U : p.U, i, x + y)));
-                            if (ROWW && !e_dense) wr[y] = p.row_scale[m];
-                        }
-                    }
-                }
                 if (x % 2 == 0) turn(acc[i][x >> 1][0], acc[i][x >> 1][1], acc[i][x >> 1][2], acc[i][x >> 1][3], chunk);
                 u32x4 v = chunk[x & 1];
                 const int m = e_row_begin + chunk_m(i, x);
@@ -1157,8 +1138,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                     if (all_rows || m < row_lim) {
                         float dh[8], gv[8], uv[8], dg[8], du[8];
                         Elem<uint16_t>::unpack(v, dh);
-                        Elem<uint16_t>::unpack(gq[x & 1], gv);
-                        Elem<uint16_t>::unpack(uq[x & 1], uv);
+                        Elem<uint16_t>::unpack(g_in[GU ? i & 1 : 0][GU ? x : 0], gv);
+                        Elem<uint16_t>::unpack(u_in[GU ? i & 1 : 0][GU ? x : 0], uv);
 #pragma unroll
                         for (int y = 0; y < 8; y++) {
                             const float sg = fast_sigmoid(gv[y]);
@@ -1167,7 +1148,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                                 // acc is the gradient of w * silu(g) * u: the routing weight's gradient
                                 // is its product with silu(g) * u, the activation's gets the factor w
                                 dot += dh[y] * (sl * uv[y]);
-                                dh[y] *= wr[x & 1];
+                                dh[y] *= w_in[GU ? i & 1 : 0][GU ? x : 0];
                             }
                             du[y] = dh[y] * sl;
                             dg[y] = (dh[y] * uv[y]) * (sg * (1.0f + gv[y] * (1.0f - sg)));
@@ -1203,6 +1184,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                     if (ACCUM) __builtin_amdgcn_sched_barrier(0);   // (all of them at once spill registers)
                 }
             }
+            if (GU && i + 2 < TM) load_gu(i + 2);
         }
     }
     };
