@@ -827,9 +827,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     // counter runs in order, so before this a tile began when the last one's 128 KB had been accepted.  Weight gradients
     // alone, us: 64 experts of 2048/1024, 512 tokens, uneven 200 -> 180 (the pass 603 -> 599, bound by what memory takes),
     // 16384 tokens 1447 -> 1415; 32 experts of 7168/2048, 400 uneven rows, 1364 -> 1314, added 1814 -> 1783.  The row products,
-    // with more steps to a tile, gain nothing by it (1 % slower in gate+up of 512 rows).
+    // with more steps to a tile, gain nothing by it (1 % slower in gate+up of 512 rows), nor do 128x128 tiles, whose two blocks per CU
+    // cover each other's stores: early, with the stores waited for -> not, us: 12 experts of 1000/712, 9003 rows, 74.3 -> 73.8; 64 of
+    // 1712/1048, 8192 rows, 309 -> 304; 8 of 256/512, 4096 rows, 25.8 -> 25.5 (with a whole tile's eight stores counted 1.5 % slower than early).
     constexpr int FIRST = 6;                  // loads of step 1 in second()
-    constexpr bool EARLY = WGRAD;
+    constexpr bool EARLY = WGRAD && !EDGE;
     auto second = [&]() {
         if (n_steps == 1) return;
         const int c1 = next_c0(rot * BK);
@@ -850,7 +852,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     // 16-byte stores that a wavefront makes at least for a tile all of whose rows exist: they follow the next tile's prefetch,
     // and its first step does not wait for them
-    constexpr int STORES = EDGE || !EARLY ? 0 : 16;
+    constexpr int STORES = EARLY ? 16 : 0;
     bool stores_follow = false;
     bool have = next_tile();
     if (have) prefetch();

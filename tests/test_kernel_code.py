@@ -1,0 +1,48 @@
+"""What the compiler makes of the expert GEMMs (ggemm.hip): properties of the generated code that the kernels' speed or
+their waits rest on and that no result shows."""
+import os
+import re
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "optimus-lm_amd", "csrc")
+# template arguments of ggemm_kernel, in order
+FIELDS = ("BM", "AKIND", "BKIND", "EPI", "GATHER", "ROWW", "ACCUM", "EDGE", "ONCE", "DENSE")
+EPI_WGRAD = 3
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """[(template arguments, assembly lines, notes)] of the library's build."""
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc")
+    import build as library_build
+    out = str(tmp_path_factory.mktemp("asm") / "ggemm.s")
+    flags = [f for f in library_build.HIPCC_FLAGS if f != "-shared"]
+    subprocess.run([hipcc, *flags, "--cuda-device-only", "-S", os.path.join(CSRC, "ggemm.hip"), "-o", out], check=True,
+                   capture_output=True)
+    text = open(out).read()
+    notes = {m.group(1): dict(re.findall(r"\.(\w+_spill_count):\s*(\d+)", m.group(0)))
+             for m in re.finditer(r"\.name:\s+(\S+).*?\.wavefront_size", text, re.S)}
+    found = []
+    for name in sorted(set(re.findall(r"^(\S*ggemm_kernel\S+):", text, re.M))):
+        arguments = dict(zip(FIELDS, map(int, re.findall(r"L[ib](\d+)E", name))))
+        assert len(arguments) == len(FIELDS)
+        start = text.index("\n" + name + ":")
+        found.append((arguments, text[start:text.index(".Lfunc_end", start)].split("\n"), notes[name]))
+    assert len(found) > 30
+    return found
+
+
+def test_step_1_is_loaded_ahead_only_where_the_stores_are_counted(kernels):
+    """Loads of a tile's step 1 in front of the last one's stores are of use where the first wait leaves the stores out;
+    anywhere else they are code, and a wait for what is behind them.  128x128 tiles: as many direct loads in every kernel."""
+    counts = set()
+    for k, lines, _ in kernels:
+        ahead = any("s_waitcnt vmcnt(16) lgkmcnt(0)" in line for line in lines)
+        assert ahead == (k["EPI"] == EPI_WGRAD and not k["EDGE"]), k
+        if k["BM"] == 128:
+            counts.add(sum("global_load_lds_dwordx4" in line and not line.endswith(" nt") for line in lines))
+    assert len(counts) == 1
