@@ -831,6 +831,12 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     // cover each other's stores: early, with the stores waited for -> not, us: 12 experts of 1000/712, 9003 rows, 74.3 -> 73.8; 64 of
     // 1712/1048, 8192 rows, 309 -> 304; 8 of 256/512, 4096 rows, 25.8 -> 25.5 (with a whole tile's eight stores counted 1.5 % slower than early).
     constexpr int FIRST = 6;                  // loads of step 1 in second()
+    constexpr int LAST = TM == 4 ? 2 : 1;     // the unit of A that follows them (TM == 4: and the one behind it, with step 0)
+    // 128x128: what a wavefront loads of that unit goes where its own strip lies, so it need not wait for the others' strips, as it does
+    // with 256x256 tiles (one barrier later; strips of their own in those units gained nothing there).  With few steps to a tile
+    // part of the load's way was waited for.  Behind the barrier -> ahead of the first wait, us: 8 experts of 256/512, 4096 rows, down 13.2
+    // -> 12.9; weight gradients of 64 experts of 1712/1048, 8192 rows, 304 -> 300, added ones of 16 of 1304/600, 4096 rows, 62.8 -> 62.1.
+    constexpr bool OWN_STRIP = TM == 2;
     constexpr bool EARLY = WGRAD && !EDGE;
     auto second = [&]() {
         if (n_steps == 1) return;
@@ -969,14 +975,19 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             pb2 = b_step(cs2, t + 3);
         };
         if (!EARLY) second();
+        auto last = [&]() { if (n_steps > 1) issue_a(2, pa1, cs1, c1_, IntC<LAST>{}, src[GATHER_W ? 1 : 0]); };
+        if (OWN_STRIP) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the strip's reads are back)
+            last();
+        }
         if (STORES && stores_follow) wait_loads<STORES>(lds_addr);
-        else if (n_steps > 1) wait_loads<FIRST>(lds_addr);
+        else if (n_steps > 1) wait_loads<FIRST + (OWN_STRIP ? L : 0)>(lds_addr);
         else wait_loads<0>(lds_addr);
         zero_tail(cs0, c0_, c0_);
         zero_tail(cs0, c0_, c1_);
         if constexpr (TM == 4) { zero_tail(cs0, c0_, c2_); zero_tail(cs0, c0_, c3_); }
         block_barrier();
-        if (n_steps > 1) issue_a(2, pa1, cs1, c1_, IntC<TM == 4 ? 2 : 1>{}, src[GATHER_W ? 1 : 0]);   // (the strips are done with)
+        if (!OWN_STRIP) last();   // (the strips are done with)
         set_fragments();
         read_a(c0_, c0_, c0_, c2_);
         read_b(c0_, c0_, c8_);
@@ -999,7 +1010,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     asm volatile("" : "+v"(lane_e), "+s"(wave_e));
     const int wm_e = wave_e / WAVES_N, wn_e = wave_e % WAVES_N;
     constexpr int COLS = (EPI == EPI_SWIGLU) ? 32 : 64;   // output columns of this wavefront (EPI_SWIGLU: gate and up, side by side)
-    static_assert(NW * 2048 <= (TM == 4 ? 2 : 1) * UNIT, "strips must fit into the units that prefetch leaves out");
+    static_assert(NW * 2048 == (TM - LAST) * UNIT, "strips are the units that second() leaves out");
+    static_assert(!OWN_STRIP || (L * 1024 == 2048 && TM - LAST == 1), "a wavefront's strip is what it loads of that unit");
     const int strip = 2 * A_STAGE - NW * 2048 + wave_e * 2048;   // bytes from lds; 2 KB, its 16-byte chunks XOR-permuted by row
     int put_at[2], get_at[2];   // of blocks 0 and 1 (2 and 3: the other half of the row); of 8 rows and the other 8
     {

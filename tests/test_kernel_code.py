@@ -46,3 +46,11 @@ def test_step_1_is_loaded_ahead_only_where_the_stores_are_counted(kernels):
         if k["BM"] == 128:
             counts.add(sum("global_load_lds_dwordx4" in line and not line.endswith(" nt") for line in lines))
     assert len(counts) == 1
+
+
+def test_first_steps_of_128x128_tiles_are_loaded_ahead_of_the_first_wait(kernels):
+    """All eight loads that step 1 of a tile needs are under way when a wavefront first waits, for step 0."""
+    for k, lines, _ in kernels:
+        if k["BM"] == 128:
+            first = [line.split()[1] for line in lines if re.match(r"\s*s_waitcnt vmcnt\(\d+\) lgkmcnt\(0\)$", line)]
+            assert set(first) == {"vmcnt(8)", "vmcnt(0)"}, k
