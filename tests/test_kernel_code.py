@@ -54,3 +54,11 @@ def test_first_steps_of_128x128_tiles_are_loaded_ahead_of_the_first_wait(kernels
         if k["BM"] == 128:
             first = [line.split()[1] for line in lines if re.match(r"\s*s_waitcnt vmcnt\(\d+\) lgkmcnt\(0\)$", line)]
             assert set(first) == {"vmcnt(8)", "vmcnt(0)"}, k
+
+
+def test_128x128_kernels_have_each_step_once(kernels):
+    """Even and odd steps, of tiles with both row units and of tiles with one: 32 MFMAs a step or 16.  Short launches fetch
+    their code cold."""
+    for k, lines, _ in kernels:
+        if k["BM"] == 128:
+            assert sum("v_mfma_f32_16x16x32_bf16" in line for line in lines) == 2 * (32 + 16), k
