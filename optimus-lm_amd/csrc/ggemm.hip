@@ -270,7 +270,10 @@ __device__ __forceinline__ void build_part_table(const int32_t *cum, const int *
     int base_tiles = 0;
     for (int i0 = 0; i0 < n_experts; i0 += 64) {
         const int i = i0 + lane, there = i % groups, group = (i / groups) & 1 ? groups - 1 - there : there;
-        const int e = order[min(i, n_experts - 1)], begin = cum[e], end = cum[e + 1], tiles = tiles_of(end - begin);
+        const int e = order[min(i, n_experts - 1)];
+        int begin = cum[e], end = cum[e + 1];
+        asm volatile("" : "+v"(begin), "+v"(end));   // waited for here: around their use the compiler would wait for them, and all else, in every tile
+        const int tiles = tiles_of(end - begin);
         const int first = part_begin(tiles, i, member, share);
         const int mine = i < n_experts && group == xcd / share ? part_begin(tiles, i, member + 1, share) - first : 0;
         int incl = mine;
@@ -1086,26 +1089,30 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         }
     };
     if (GU) { load_gu(0); load_gu(1); }
-    have = next_tile();
     u32x4 old[ACCUM ? TM : 1][ACCUM ? 4 : 1];
     if (ACCUM) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int x = 0; x < 4; x++) {
-                // (EDGE: rows and columns past the matrix: its last ones, not used; a load in a branch would be waited for with all others)
+                // (EDGE: rows and columns past the matrix: its last ones, not used)
                 const uint16_t *from = EDGE ? Cb + static_cast<int64_t>(min(e_row_begin + chunk_m(i, x), e_row_end - 1)) * e_ldc + min(col0 + chunk_col, e_n_cols - 8)
                                             : chunk_at(Cb, i, x);
                 old[ACCUM ? i : 0][ACCUM ? x : 0] = *reinterpret_cast<const u32x4 *>(from);
             }
     }
-    if (have) prefetch();
-    if (ACCUM && EDGE) {   // (waited for once: between stores that may not be made the compiler would wait for all of them)
+    have = next_tile();
+    if (ACCUM) {
+        // Waited for here, ahead of the direct loads, which the compiler does not count: behind them each of its waits for an old value was one
+        // for most of the next tile's first steps, and a path that it saw around them made it wait for the stores too, in each tile.  us,
+        // behind -> ahead: 64 experts of 2048/1024, 4096 rows, uneven, 347 -> 328, 131072 rows 1532 -> 1506; 32 of 7168/2048, 12510 rows,
+        // uneven, 1780 -> 1681; 12 of 1000/712, 9003 rows, 85.0 -> 83.1
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int x = 0; x < 4; x++) asm volatile("" : "+v"(old[ACCUM ? i : 0][ACCUM ? x : 0]));
     }
+    if (have) prefetch();
     stores_follow = all_rows;
     auto rows_out = [&](auto past_caches) {   // (two loops: of a branch at each store the compiler knows less about what is under way)
 #pragma unroll

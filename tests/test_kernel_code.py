@@ -62,3 +62,16 @@ def test_128x128_kernels_have_each_step_once(kernels):
     for k, lines, _ in kernels:
         if k["BM"] == 128:
             assert sum("v_mfma_f32_16x16x32_bf16" in line for line in lines) == 2 * (32 + 16), k
+
+
+def test_weight_gradients_start_a_tile_with_stores_under_way(kernels):
+    """From the wait that leaves the last tile's 16 stores out to the first MFMA nothing else waits for memory: what the compiler
+    believes to be still on its way there it would wait for together with the stores."""
+    seen = 0
+    for k, lines, _ in kernels:
+        if k["BM"] == 256 and k["EPI"] == EPI_WGRAD:
+            at = next(i for i, line in enumerate(lines) if "s_waitcnt vmcnt(16) lgkmcnt(0)" in line)
+            until = next(i for i in range(at, len(lines)) if "v_mfma" in lines[i])
+            assert not any("vmcnt(" in line or "scratch_" in line for line in lines[at + 1:until]), k
+            seen += 1
+    assert seen == 8
