@@ -697,7 +697,14 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
 #pragma unroll
         for (int l = 0; l < L; l++) {
             const int c = AKIND == CONTIG ? ((lane & 7) ^ swz(slot(l))) * 8 : slot(l);
-            if (c0 + c >= c_len) *reinterpret_cast<u32x4 *>(q + l * 1024) = u32x4{0, 0, 0, 0};
+            if (c0 + c >= c_len) {
+                // made here: four registers of zeros kept for the whole loop were spilled in the accumulating 256x256 weight gradients, and
+                // registers were short in the others.  us, kept -> made: 64 experts of 2048/1024, 32768 rows, uneven, 1049 -> 1029 (added 1050 ->
+                // 1046), 131072 rows 1401 -> 1379 (1506 -> 1487); 32 of 7168/2048, 12510 rows, uneven, 1277 -> 1259 (1681 -> 1669)
+                uint32_t zero = 0;
+                asm volatile("" : "+v"(zero));
+                *reinterpret_cast<u32x4 *>(q + l * 1024) = u32x4{zero, zero, zero, zero};
+            }
         }
     };
 

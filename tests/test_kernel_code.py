@@ -75,3 +75,9 @@ def test_weight_gradients_start_a_tile_with_stores_under_way(kernels):
             assert not any("vmcnt(" in line or "scratch_" in line for line in lines[at + 1:until]), k
             seen += 1
     assert seen == 8
+
+
+def test_no_vector_register_is_spilled(kernels):
+    for k, lines, notes in kernels:
+        assert int(notes["vgpr_spill_count"]) == 0, k
+        assert not any("scratch_" in line for line in lines), k
