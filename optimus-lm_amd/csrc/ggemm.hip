@@ -1120,6 +1120,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             for (int x = 0; x < 4; x++) asm volatile("" : "+v"(old[ACCUM ? i : 0][ACCUM ? x : 0]));
     }
     if (have) prefetch();
+    // the next tile's first wait counts the stores as younger than its loads: none may move ahead of them
+    if (STORES) asm volatile("; stores from here on" ::: "memory");
     stores_follow = all_rows;
     auto rows_out = [&](auto past_caches) {   // (two loops: of a branch at each store the compiler knows less about what is under way)
 #pragma unroll

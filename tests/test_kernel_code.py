@@ -81,3 +81,15 @@ def test_no_vector_register_is_spilled(kernels):
     for k, lines, notes in kernels:
         assert int(notes["vgpr_spill_count"]) == 0, k
         assert not any("scratch_" in line for line in lines), k
+
+
+def test_counted_stores_stay_behind_the_loads_they_follow(kernels):
+    """The first wait of a tile leaves the 16 youngest operations out, which are the last tile's stores only while none of them
+    stands ahead of the direct loads."""
+    for k, lines, _ in kernels:
+        if k["BM"] == 256 and k["EPI"] == EPI_WGRAD:
+            at = [i for i, line in enumerate(lines) if "stores from here on" in line]
+            assert len(at) == 1, k
+            stores = [i for i, line in enumerate(lines) if re.match(r"\s*(global|buffer)_store_dwordx4", line)]
+            assert len(stores) >= 32 and min(stores) > at[0], k       # past the caches and through them
+            assert max(i for i, line in enumerate(lines) if "global_load_lds" in line) < at[0], k
