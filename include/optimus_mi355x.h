@@ -610,6 +610,9 @@ typedef struct {
 } om_dense_expert;
 /* 1 if the gate+up product of a dense expert with dense_rows rows would run in the routed experts' launch. */
 int om_merged_mlp_dense_rides(int64_t expected_rows, int G, int I, int H, int64_t dense_rows);
+/* Which products of a dense expert with dense_rows rows would run in the routed experts' launches: a sum of these. */
+enum { OM_DENSE_GATE_UP = 1, OM_DENSE_DOWN = 2, OM_DENSE_DOWN_DGRAD = 4, OM_DENSE_GATE_UP_DGRAD = 8 };
+int om_merged_mlp_dense_products(int64_t expected_rows, int G, int I, int H, int64_t dense_rows);
 int om_merged_mlp_gate_up_fwd_weighted_dense(const void *x, const int32_t *x_rows, int64_t src_rows,
                                              const void *w_gate, const void *w_up, const float *row_weights,
                                              void *g, void *u, void *h, const int32_t *cum_token_counts,

@@ -1834,12 +1834,23 @@ extern "C" int om_merged_mlp_gate_up_fwd_weighted_dense(const void *x, const int
                               rows, expected_rows, G, I, H, w_stride, stream, dense);
 }
 
-extern "C" int om_merged_mlp_dense_rides(int64_t expected_rows, int G, int I, int H, int64_t dense_rows) {
+extern "C" int om_merged_mlp_dense_products(int64_t expected_rows, int G, int I, int H, int64_t dense_rows) {
     if (expected_rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8) || dense_rows < 1) return OM_ERR_SHAPE;
-    GemmParams p = {};
-    p.n_experts = G; p.n_cols = I; p.kc = H;
-    const bool past_caches = 2 * static_cast<int64_t>(G) * I * H >= CACHED_WEIGHTS && H % 64 == 0;   // (as far as sizes say)
-    return !om_ggemm_streams(expected_rows, G, 2 * I, past_caches) && dense_rides<EPI_SWIGLU>(p, expected_rows, dense_rows) ? 1 : 0;
+    GemmParams up = {}, down = {};   // of extents [I] x H and [H] x I
+    up.n_experts = down.n_experts = G;
+    up.n_cols = down.kc = I; up.kc = down.n_cols = H;
+    const int64_t weights = static_cast<int64_t>(G) * I * H;     // (whether they pass the caches: as far as sizes say)
+    const bool up_streams = om_ggemm_streams(expected_rows, G, 2 * I, 2 * weights >= CACHED_WEIGHTS && H % 64 == 0);
+    const bool down_streams = om_ggemm_streams(expected_rows, G, H, weights >= CACHED_WEIGHTS && I % 64 == 0);
+    return (!up_streams && dense_rides<EPI_SWIGLU>(up, expected_rows, dense_rows) ? OM_DENSE_GATE_UP : 0) |
+           (!down_streams && dense_rides<EPI_STORE>(down, expected_rows, dense_rows) ? OM_DENSE_DOWN : 0) |
+           (dense_rides<EPI_SWIGLU_BWD>(up, expected_rows, dense_rows) ? OM_DENSE_DOWN_DGRAD : 0) |
+           (dense_rides<EPI_STORE>(down, expected_rows, dense_rows) ? OM_DENSE_GATE_UP_DGRAD : 0);
+}
+
+extern "C" int om_merged_mlp_dense_rides(int64_t expected_rows, int G, int I, int H, int64_t dense_rows) {
+    const int products = om_merged_mlp_dense_products(expected_rows, G, I, H, dense_rows);
+    return products < 0 ? products : products & OM_DENSE_GATE_UP ? 1 : 0;
 }
 
 namespace {

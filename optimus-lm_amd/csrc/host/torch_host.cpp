@@ -517,8 +517,16 @@ struct Alongside {
     const MlpWeights &w;
     MlpState &s;             // the forward's; its cum: device {0, tokens}
     Tensor y;                // its output
-    static bool fits(const MlpWeights &w, const MlpWeights &routed) {
-        return w.I() == routed.I() && w.H() == routed.H() && w.gate.is_contiguous() && w.up.is_contiguous() && w.down.is_contiguous();
+    static bool fits(const MlpWeights &w, int64_t I, int64_t H) {
+        return w.I() == I && w.H() == H && w.gate.is_contiguous() && w.up.is_contiguous() && w.down.is_contiguous();
+    }
+    // Whether one of `products` (OM_DENSE_...) would run in a routed launch.  Where none would, the shared expert goes first, all of
+    // it: what it computes with in between (64 MB of dg and du with 8192 tokens of intermediate size 2048) is used at once and given back.
+    static bool rides(const MlpWeights &w, const MlpWeights &routed, int64_t expected, int64_t tokens, int products) {
+        if (!fits(w, routed.I(), routed.H()) || tokens < 1) return false;
+        const int which = om_merged_mlp_dense_products(expected, static_cast<int>(routed.G()), static_cast<int>(routed.I()),
+                                                       static_cast<int>(routed.H()), tokens);
+        return which > 0 && (which & products);
     }
 };
 om_dense_expert dense_expert(std::array<const Tensor *, 2> a, std::array<const Tensor *, 2> w, std::array<const Tensor *, 3> cs,
@@ -1093,7 +1101,7 @@ struct RoutedNode : HostNode {
         Tensor base;
         Sinks ks;
         Alongside along{ws, ss, Tensor()};
-        const bool together = has_shared && index.rows > 0 && Alongside::fits(ws, w);
+        const bool together = has_shared && index.rows > 0 && Alongside::rides(ws, w, index.to_choose_by(), dfinal.size(0), OM_DENSE_DOWN_DGRAD | OM_DENSE_GATE_UP_DGRAD);
         if (has_shared) {   // first: its input gradient is the base of the routed experts' per-token sum
             ks = sinks_of(c, shared, ws);
             if (!together) base = merged_backward(c, dfinal, kept[0], ws, iptr(ss.cum), ss, nullptr, ks);
@@ -1130,7 +1138,7 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
         if (has_shared) {
             ws = weights_of(shared, true, 1);
             // (the host waits for the rows behind the shared expert's kernels, where it has to)
-            together = !after_shared && xc.size(0) > 0 && Alongside::fits(ws, w);
+            together = !after_shared && Alongside::rides(ws, w, ix.to_choose_by(), xc.size(0), OM_DENSE_GATE_UP | OM_DENSE_DOWN);
             if (together) require_shared_operands(xc, ws, one, ss);
             else residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
         }

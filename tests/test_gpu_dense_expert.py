@@ -92,3 +92,32 @@ def test_dense_expert_beside_the_routed_ones(cuda, T, G, I, H, rows, bound):
     if T > 80:   # (a launch of its own with fewer rows adds a forward product up in another order)
         for k in s:
             assert torch.equal(s[k], s0[k]), k
+
+
+@pytest.mark.parametrize("T,products", [(8192, 0), (600, 15)])
+def test_shared_expert_goes_first_where_nothing_of_it_rides(cuda, T, products):
+    """All of its forward, and all of its backward, stand ahead of the routed experts' then."""
+    from optimus import _native
+    G, K, H, I = 8, 1, 1024, 1024
+    assert _native.lib().om_merged_mlp_dense_products(T * K, G, I, H, T) == products
+    gen = torch.Generator().manual_seed(T)
+
+    def leaf(*s, scale=0.05):
+        return (torch.randn(*s, generator=gen) * scale).to(torch.bfloat16).to(cuda).requires_grad_(True)
+
+    x, rw = leaf(T, H, scale=1.0), torch.rand(T, K, generator=gen).to(cuda).requires_grad_(True)
+    experts = torch.randint(0, G, (T, K), generator=gen).to(cuda)
+    leaves = [leaf(G, I, H), leaf(G, I, H), leaf(G, H, I), leaf(I, H), leaf(I, H), leaf(H, I)]
+    one = torch.tensor([0, T], dtype=torch.int32, device=cuda)
+    _native.launch_log = []
+    try:
+        out = _native.host().moe_experts(x, rw, experts, 0, G, G, False, None, True, leaves, True, one)
+        out.backward(torch.ones_like(out))
+        torch.cuda.synchronize()
+    finally:
+        names, _native.launch_log = [e[0] for e in _native.launch_log], None
+    assert any(n.endswith("_dense") for n in names) == (products != 0)
+    if not products:
+        for last_shared, first_routed in (("om_grouped_gemm_fwd", "om_merged_mlp_gate_up_fwd_weighted"),
+                                          ("om_merged_mlp_gate_up_dgrad", "om_merged_mlp_down_dgrad_weighted")):
+            assert names.index(last_shared) < names.index(first_routed), names
