@@ -1245,6 +1245,21 @@ struct CountReadback {
     }
 };
 
+// Whether the host waits for the row count ahead of the shared expert's kernels: where they are those of the routed experts and,
+// alone, too few for the chip (fewer tiles than three quarters of its CUs) that saves more than the wait costs.  Forward passes, us, behind
+// them -> together: 7168/2048 of 600 tokens (160 tiles) 566 -> 516, 3000/1000 of 1000 (128) 248 -> 234; but 1200/1000 of 3000 (384)
+// 187 -> 191, 1024/256 of 8000 (252) 146 -> 155.
+bool waits_ahead_of_shared(int64_t expected, int64_t G, int64_t I, int64_t H, int64_t tokens, const std::vector<Tensor> &shared) {
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < 1)
+        cus = 256;
+    at::AutoDispatchBelowADInplaceOrView below;
+    const int64_t tiles = (tokens + 127) / 128 * ((I + 63) / 64);
+    return tiles * 4 < cus * 3 && Alongside::fits(weights_of(shared, true, 1), I, H) &&
+           om_merged_mlp_dense_rides(expected, static_cast<int>(G), static_cast<int>(I), static_cast<int>(H), tokens) == 1;
+}
+
 // Sort (with the routing weights laid out per sorted row) and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
 // sync_free: never read the routed-row count of an expert window back (else up to a limit: sized_by_bound).
 Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
@@ -1275,13 +1290,8 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
             // read the count back (as the reference does), behind the shared expert's kernels: they do not
             // need it, and while the GPU runs them the host waits for a copy that was enqueued before them
             auto count = std::make_shared<CountReadback>(ix.cum + (end - start), c.stream);
-            // unless they are those of the routed experts and, alone, too few for the chip (fewer tiles than three quarters
-            // of its CUs): then that saves more than the wait costs.  Forward passes, us, behind them -> together: 7168/2048 of
-            // 600 tokens (160 tiles) 566 -> 516, 3000/1000 of 1000 (128) 248 -> 234; but 1200/1000 of 3000 (384) 187 -> 191,
-            // 1024/256 of 8000 (252) 146 -> 155.
-            const int64_t tiles = (x.size(0) + 127) / 128 * ((I + 63) / 64);
-            if (has_shared && one && tiles < 192 && om_merged_mlp_dense_rides(ix.rows * (end - start) / n_total, static_cast<int>(end - start),
-                                                               static_cast<int>(I), static_cast<int>(H), x.size(0)) == 1) {
+            if (has_shared && one && waits_ahead_of_shared(ix.rows * (end - start) / n_total, end - start, I, H, x.size(0),
+                                                           std::vector<Tensor>(leaves.end() - 3, leaves.end()))) {
                 ix.rows = count->wait();
                 return routed_experts(c, x, rw, ix, residual.value_or(Tensor()), merged, leaves, has_shared, *one);
             }
@@ -1645,6 +1655,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("adamw_step", &adamw_step, no_gil);
     m.def("grad_norm", &grad_norm, no_gil);
     m.def("sized_by_bound", &sized_by_bound);
+    m.def("waits_ahead_of_shared", &waits_ahead_of_shared);
     m.def("live_grad", [](const Tensor &param) {
         Tensor grad = live_grad(param);
         if (grad.defined()) order_live_gradients();

@@ -216,3 +216,20 @@ def test_expert_weights_through_a_property():
     got = _n.host().expert_parameters(experts)
     for a, name in zip(got, ("gate_proj", "up_proj", "down_proj")):
         assert torch.equal(a, getattr(experts[0], name)._parameters["weight"] * 2)
+
+
+def test_row_count_is_waited_for_first_only_where_the_shared_expert_rides():
+    """Fewer 128x128 tiles than three quarters of the CUs, the routed experts' extents, dense matrices."""
+    f, I, H = _n.host().waits_ahead_of_shared, 1000, 3000
+
+    def shared(i, h):
+        return [torch.empty(*s, dtype=torch.bfloat16) for s in ((i, h), (i, h), (h, i))]
+
+    assert f(1000, 32, I, H, 1000, shared(I, H))
+    assert f(1000, 32, I, H, 1000, [w.unsqueeze(0) for w in shared(I, H)])
+    assert not f(1000, 32, I, H, 1000, shared(2 * I, H))                 # two shared experts as one
+    gate, up, down = shared(I, H)
+    assert not f(1000, 32, I, H, 1000, [gate, torch.empty(H, I, dtype=torch.bfloat16).t(), down])
+    tiles_per_block = (I + 63) // 64
+    line = -(-192 // tiles_per_block) * 128                              # 256 CUs
+    assert f(1000, 32, I, H, line - 128, shared(I, H)) and not f(1000, 32, I, H, line, shared(I, H))
