@@ -44,11 +44,19 @@ __device__ __forceinline__ void adam_update(float g, float &m, float &v, float &
 // Every wavefront access is one contiguous span (512 B of the bf16 streams, 1 KB of the fp32 ones).
 constexpr int ADAMW_THREADS = 64;
 constexpr size_t ADAMW_OCCUPANCY_LDS = 13600;   // bytes of dynamic LDS per block: 12 blocks per CU
+// More elements than this are stored past the caches: their 128 MB of states are several times what the L2s hold (32 MB), and what lies there
+// does not serve the next step.  us, through them (nt alone) -> past them, steps in a row / caches filled by others: bf16, 1.3e6 6.9 -> 8.8
+// / 11.1 -> 11.2, 3e6 15.8 -> 17.5 / 20.8 -> 20.4, 6e6 29.0 -> 29.6 / 33.0 -> 32.0, 1e7 48.7 -> 48.5 / 52.8 -> 51.3, 2e7 91.7 -> 90.1 / 94.7 ->
+// 92.7; float32 6.4 -> 9.3 / 11.7 -> 11.7, 15.9 -> 18.2 / 20.4 -> 20.6, 30.0 -> 31.2 / 35.2 -> 34.1, 51.3 -> 51.1 / 55.4 -> 53.6, 99.9 -> 96.8 /
+// 103.9 -> 99.8.
+constexpr int64_t PAST_CACHES = 8 << 20;
 
 template <typename T> __device__ __forceinline__ T stream_load(const T *p) { return __builtin_nontemporal_load(p); }
-// vector c of this thread
-template <typename T, typename P> __device__ __forceinline__ void stream_store(P *p, T v) {
-    store_past_caches(reinterpret_cast<T *>(p) + static_cast<int64_t>(blockIdx.x) * ADAMW_THREADS, threadIdx.x * sizeof(T), v);
+// vector c of this thread; PAST: see PAST_CACHES
+template <bool PAST, typename T, typename P> __device__ __forceinline__ void stream_store(P *p, T v) {
+    T *block = reinterpret_cast<T *>(p) + static_cast<int64_t>(blockIdx.x) * ADAMW_THREADS;
+    if constexpr (PAST) store_past_caches(block, threadIdx.x * sizeof(T), v);
+    else __builtin_nontemporal_store(v, block + threadIdx.x);
 }
 // Keeps a value that is only copied from being recognised as "the value just loaded from there"
 // (the traffic probe writes back what it read and must keep its stores).
@@ -95,7 +103,7 @@ __device__ __forceinline__ void adam_tail(float *master, const float *grad, floa
 // fp32 states are written back as read, param = bf16(master)).
 // TAIL: the lane after the last full vector takes the elements behind it (a branch that the large launches
 // do without: it costs them 1-2 %).
-template <int CLIP, bool MATH, bool TAIL>
+template <int CLIP, bool MATH, bool TAIL, bool PAST>
 __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__restrict__ param,
                                                                       const uint16_t *__restrict__ grad,
                                                                       uint16_t *grad_rw,
@@ -133,7 +141,7 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__r
             u32x2 gs;
             gs[0] = static_cast<uint32_t>(gb[0]) | (static_cast<uint32_t>(gb[1]) << 16);
             gs[1] = static_cast<uint32_t>(gb[2]) | (static_cast<uint32_t>(gb[3]) << 16);
-            stream_store(grad_rw, gs);
+            stream_store<PAST>(grad_rw, gs);
         }
     }
     if (MATH) {
@@ -147,17 +155,17 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_bf16_kernel(uint16_t *__r
         asm volatile("" : : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]));   // the gradient load stays
         opaque(m0); opaque(v0); opaque(w0);
     }
-    stream_store(exp_avg, m0);
-    stream_store(exp_avg_sq, v0);
-    stream_store(master, w0);
+    stream_store<PAST>(exp_avg, m0);
+    stream_store<PAST>(exp_avg_sq, v0);
+    stream_store<PAST>(master, w0);
     u32x2 pk;
     pk[0] = static_cast<uint32_t>(f32_to_bf16_bits(w0[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(w0[1])) << 16);
     pk[1] = static_cast<uint32_t>(f32_to_bf16_bits(w0[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(w0[3])) << 16);
-    stream_store(param, pk);
+    stream_store<PAST>(param, pk);
 }
 
 // fp32 mode: the parameter buffer is the master buffer (16 B read, 12 B written per element).
-template <int CLIP, bool TAIL>
+template <int CLIP, bool TAIL, bool PAST>
 __global__ __launch_bounds__(ADAMW_THREADS) void adamw_f32_kernel(float *__restrict__ master,
                                                                   const float *__restrict__ grad,
                                                                   float *grad_rw,
@@ -181,7 +189,7 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_f32_kernel(float *__restr
     if (CLIP) {
 #pragma unroll
         for (int i = 0; i < 4; i++) g[i] = g[i] * coef;
-        if (CLIP == 2) stream_store(grad_rw, g);
+        if (CLIP == 2) stream_store<PAST>(grad_rw, g);
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -189,9 +197,9 @@ __global__ __launch_bounds__(ADAMW_THREADS) void adamw_f32_kernel(float *__restr
         adam_update(g[i], ma, va, wa, s);
         m[i] = ma; v[i] = va; w[i] = wa;
     }
-    stream_store(exp_avg, m);
-    stream_store(exp_avg_sq, v);
-    stream_store(master, w);
+    stream_store<PAST>(exp_avg, m);
+    stream_store<PAST>(exp_avg_sq, v);
+    stream_store<PAST>(master, w);
 }
 
 }  // namespace
@@ -258,28 +266,29 @@ static int adamw_launch(void *param, void *grad, float *master, float *exp_avg, 
     const size_t lds = small ? 0 : ADAMW_OCCUPANCY_LDS;
     const dim3 block(ADAMW_THREADS);
     // `lo`: first element, `vecs` full vectors and (TAIL) the elements up to `count`
-    auto go = [&](auto tail_tag, unsigned grid, int64_t lo, int64_t vecs, int64_t count) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
+    auto go = [&](auto tail_tag, auto past_tag, unsigned grid, int64_t lo, int64_t vecs, int64_t count) {
+        constexpr bool TAIL = decltype(tail_tag)::value, PAST = decltype(past_tag)::value;
         float *w = master + lo, *m = exp_avg + lo, *v = exp_avg_sq + lo;
         if (param_dtype == OM_BF16) {
             uint16_t *p = static_cast<uint16_t *>(param) + lo, *g = static_cast<uint16_t *>(grad) + lo;
-            if (clip == ADAMW_PROBE) adamw_bf16_kernel<0, false, false><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
-            else if (clip == 0) adamw_bf16_kernel<0, true, TAIL><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
-            else if (clip == 1) adamw_bf16_kernel<1, true, TAIL><<<grid, block, lds, st>>>(p, g, nullptr, grad_scale, w, m, v, vecs, count, s);
-            else adamw_bf16_kernel<2, true, TAIL><<<grid, block, lds, st>>>(p, nullptr, g, grad_scale, w, m, v, vecs, count, s);
+            if (clip == ADAMW_PROBE) adamw_bf16_kernel<0, false, false, PAST><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
+            else if (clip == 0) adamw_bf16_kernel<0, true, TAIL, PAST><<<grid, block, lds, st>>>(p, g, nullptr, nullptr, w, m, v, vecs, count, s);
+            else if (clip == 1) adamw_bf16_kernel<1, true, TAIL, PAST><<<grid, block, lds, st>>>(p, g, nullptr, grad_scale, w, m, v, vecs, count, s);
+            else adamw_bf16_kernel<2, true, TAIL, PAST><<<grid, block, lds, st>>>(p, nullptr, g, grad_scale, w, m, v, vecs, count, s);
         } else {
             float *g = static_cast<float *>(grad) + lo;
-            if (clip == 0) adamw_f32_kernel<0, TAIL><<<grid, block, lds, st>>>(w, g, nullptr, nullptr, m, v, vecs, count, s);
-            else if (clip == 1) adamw_f32_kernel<1, TAIL><<<grid, block, lds, st>>>(w, g, nullptr, grad_scale, m, v, vecs, count, s);
-            else adamw_f32_kernel<2, TAIL><<<grid, block, lds, st>>>(w, nullptr, g, grad_scale, m, v, vecs, count, s);
+            if (clip == 0) adamw_f32_kernel<0, TAIL, PAST><<<grid, block, lds, st>>>(w, g, nullptr, nullptr, m, v, vecs, count, s);
+            else if (clip == 1) adamw_f32_kernel<1, TAIL, PAST><<<grid, block, lds, st>>>(w, g, nullptr, grad_scale, m, v, vecs, count, s);
+            else adamw_f32_kernel<2, TAIL, PAST><<<grid, block, lds, st>>>(w, nullptr, g, grad_scale, m, v, vecs, count, s);
         }
     };
     if (param_dtype == OM_F32 && clip == ADAMW_PROBE) return OM_ERR_DTYPE;
     if (with_tail) {
-        go(std::true_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
+        go(std::true_type(), std::false_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
     } else {
-        if (n_vec > 0) go(std::false_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
-        if (tail > 0 && clip != ADAMW_PROBE) go(std::true_type(), 1u, n_vec * 4, 0, tail);
+        if (n_vec > 0 && n > PAST_CACHES) go(std::false_type(), std::true_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
+        else if (n_vec > 0) go(std::false_type(), std::false_type(), static_cast<unsigned>(blocks), 0, n_vec, n);
+        if (tail > 0 && clip != ADAMW_PROBE) go(std::true_type(), std::false_type(), 1u, n_vec * 4, 0, tail);
     }
     return om_launch_status();
 }

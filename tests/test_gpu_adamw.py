@@ -69,9 +69,8 @@ def test_multi_step_and_fp64_distance(cuda, oracle_lib):
     assert rel.max() <= 1e-6, rel.max()
 
 
-def test_fp32_mode_bit_exact(cuda, oracle_lib):
+def test_fp32_mode_bit_exact(cuda, oracle_lib, n=100003):
     from optimus.optimizers import adamw_step_
-    n = 100003
     st = _state(n)
     grad32 = st["grad"].float()
     w = st["master"].clone().to(cuda); g = grad32.to(cuda)
@@ -83,6 +82,13 @@ def test_fp32_mode_bit_exact(cuda, oracle_lib):
     assert np.array_equal(w.cpu().numpy().view(np.uint32), wo.view(np.uint32))
     assert np.array_equal(m.cpu().numpy().view(np.uint32), mo.view(np.uint32))
     assert np.array_equal(v.cpu().numpy().view(np.uint32), vo.view(np.uint32))
+
+
+# around the line from which on the states are stored past the caches: whole vectors and remainders
+@pytest.mark.parametrize("n", [8 << 20, (8 << 20) + 1, (8 << 20) + 4, (8 << 20) + 7])
+def test_both_store_policies_bit_exact(cuda, oracle_lib, n):
+    test_bf16_bit_exact_vs_oracle(cuda, oracle_lib, n, 0.1)
+    test_fp32_mode_bit_exact(cuda, oracle_lib, n)
 
 
 def test_optimizer_class_matches_kernel(cuda, oracle_lib):
