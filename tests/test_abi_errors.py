@@ -2,6 +2,9 @@
 HIP runtime and answers with a negative OM_ERR_* code — it never throws and never launches on bad
 input.  These calls return from the validation, so they run without a GPU; the pointers are made-up
 addresses that are never dereferenced on the host."""
+import ctypes
+import struct
+
 import pytest
 
 from optimus import _native as n
@@ -231,6 +234,54 @@ def test_products_over_a_bound_of_the_rows(lib):
     assert lib.om_grouped_gemm_wgrad_merged_accumulate_bound(P, P, P, P, P, P, P, 512, P, ODD, P, P, 4096, 64, 64, 1024, 2048, 0, 0, 0,
                                                              None) == ALIGN
     assert lib.om_merged_mlp_gate_up_dgrad_bound(P, P, P, P, None, P, 4096, 64, 64, 1024, 2048, 0, None) == NULL
+
+
+def _dense(rows=64, a=(P, P), w=(P, P), c=(P, P, P), g=P, u=P, cum=P):
+    """An om_dense_expert."""
+    return ctypes.create_string_buffer(struct.pack("10Qq", *(v or 0 for v in (*a, *w, *c, g, u, cum)), rows))
+
+
+# entry point, arguments ahead of cum_token_counts, extents, fields of the dense expert that it reads (a, w, c, whether g and u)
+DENSE = [("om_merged_mlp_gate_up_fwd_weighted_dense", (P, P, 64, P, P, P, P, P, P), (1, 2, 3, False)),
+         ("om_grouped_gemm_fwd_dense", (P, P, P), (1, 1, 1, False)),
+         ("om_merged_mlp_down_dgrad_weighted_dense", (P, P, 64, P, P, P, P, P, P, P), (1, 1, 2, True)),
+         ("om_merged_mlp_gate_up_dgrad_dense", (P, P, P, P, P), (2, 2, 1, False))]
+
+
+@pytest.mark.parametrize("name,args,fields", DENSE)
+def test_products_with_a_dense_expert(lib, name, args, fields):
+    """What the routed operands are refused for in the plain forms, and the dense expert's own; it rides at these sizes."""
+    n_a, n_w, n_c, gu = fields
+
+    def call(dense, args=args, rows=512, expected=128, G=32, I=1024, H=2048, stride=0):
+        return getattr(lib, name)(*args, P, rows, expected, G, I, H, stride, ctypes.addressof(dense) if dense is not None else None, None)
+
+    assert lib.om_merged_mlp_dense_products(128, 32, 1024, 2048, 64) == 15
+    assert call(None) == NULL
+    assert call(_dense(), expected=513) == SHAPE and call(_dense(), expected=-1) == SHAPE
+    assert call(_dense(), I=1004) == SHAPE and call(_dense(), H=2044) == SHAPE and call(_dense(), G=0) == SHAPE
+    assert call(_dense(), stride=1024 * 2048 + 4) == ALIGN
+    assert call(_dense(rows=0)) == SHAPE and call(_dense(rows=1 << 31)) == SHAPE
+    assert call(_dense(cum=None)) == NULL
+    for field, count in (("a", n_a), ("w", n_w), ("c", n_c)):
+        size = {"a": 2, "w": 2, "c": 3}[field]
+        for i in range(count):
+            assert call(_dense(**{field: [None if j == i else P for j in range(size)]})) == NULL, (field, i)
+            assert call(_dense(**{field: [ODD if j == i else P for j in range(size)]})) == ALIGN, (field, i)
+    if gu:
+        assert call(_dense(g=None)) == NULL and call(_dense(u=ODD)) == ALIGN
+    for i, v in enumerate(args):
+        if v == P:
+            assert call(_dense(), args[:i] + (None,) + args[i + 1:]) == NULL, i
+    if name != "om_merged_mlp_down_dgrad_weighted_dense":   # (its last is of 32 bits)
+        assert call(_dense(), args[:-1] + (ODD,)) == ALIGN
+
+
+def test_dense_products(lib):
+    for bad in ((-1, 8, 1024, 1024, 64), (64, 0, 1024, 1024, 64), (64, 8, 1004, 1024, 64), (64, 8, 1024, 1004, 64), (64, 8, 1024, 1024, 0)):
+        assert lib.om_merged_mlp_dense_products(*bad) == SHAPE and lib.om_merged_mlp_dense_rides(*bad) == SHAPE
+    for sizes in ((64, 32, 2048, 7168, 64), (8192, 32, 2048, 7168, 8192), (5000, 32, 1000, 1200, 5000)):
+        assert lib.om_merged_mlp_dense_rides(*sizes) == lib.om_merged_mlp_dense_products(*sizes) & 1
 
 
 def test_check_raises_with_the_library_text():

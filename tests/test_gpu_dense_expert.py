@@ -20,15 +20,22 @@ def _ptrs(n, *ts):
 
 
 # tokens at the edges of 64-row units and 128-row tiles; extents that no tile divides; one expert; experts without rows; a
-# bound of the rows above those routed; 2200 tokens, whose shared expert takes 256x256 tiles of its own
+# bound of the rows above those routed; 2200 tokens, whose shared expert takes 256x256 tiles of its own; 128 M weights a matrix,
+# from which on they are loaded past the caches where one row tile reads them: one, and three, of the shared expert
 @pytest.mark.parametrize("T,G,I,H,rows,bound", [(17, 8, 72, 40, 9, 34), (64, 32, 256, 1024, 64, 512), (128, 1, 136, 328, 5, 5),
-                                                (129, 12, 200, 264, 387, 387), (300, 5, 512, 256, 0, 600), (2200, 3, 1024, 2048, 40, 40)])
+                                                (129, 12, 200, 264, 387, 387), (300, 5, 512, 256, 0, 600), (2200, 3, 1024, 2048, 40, 40),
+                                                (64, 16, 2048, 4096, 200, 200), (300, 16, 2048, 4096, 200, 250)])
 def test_dense_expert_beside_the_routed_ones(cuda, T, G, I, H, rows, bound):
     from optimus import _native
     lib, st = _native.lib(), torch.cuda.current_stream().cuda_stream
     gen = torch.Generator().manual_seed(T + G)
 
+    large = G * I * H >= 128 << 20
+    on_device = torch.Generator(device=cuda).manual_seed(T + G)
+
     def rnd(*s, scale=1.0):
+        if large:
+            return torch.empty(*s, dtype=torch.bfloat16, device=cuda).normal_(0.0, scale, generator=on_device)
         return (torch.randn(*s, generator=gen) * scale).to(torch.bfloat16).to(cuda)
 
     def new(*s):
@@ -45,6 +52,8 @@ def test_dense_expert_beside_the_routed_ones(cuda, T, G, I, H, rows, bound):
     P = lambda t: t.data_ptr()
     parts = lib.om_merged_mlp_row_dot_parts(I)
     expected = max(rows, 1) if bound > rows else bound
+    if large:
+        assert lib.om_merged_mlp_dense_products(expected, G, I, H, T) == 15     # all four products
 
     def run(dense):
         r = {k: new(bound, I) for k in ("g", "u", "h", "dg", "du")} | {k: new(bound, H) for k in ("y", "dx")}
@@ -89,6 +98,12 @@ def test_dense_expert_beside_the_routed_ones(cuda, T, G, I, H, rows, bound):
     assert_bf16_parity(s["u"], xf @ suf.t(), 1.03, 1.8e-3, "dense u")
     assert_bf16_parity(s["y"], hf @ sdf.t(), 1.03, 1.8e-3, "dense y")
     assert_bf16_parity(s["dx"], dgf @ sgf + duf @ suf, 1.03, 1.8e-3, "dense dx")
+    # h from the sums themselves, one rounding; dg and du from the gradient of h rounded, two: independent, sqrt(2) of one at most
+    silu = lambda t: t * torch.sigmoid(t)
+    assert_bf16_parity(s["h"], silu(xf @ sgf.t()) * (xf @ suf.t()), 1.03, 1.8e-3, "dense h")
+    dh, sig = dy.float().cpu() @ sdf, torch.sigmoid(gf)
+    assert_bf16_parity(s["dg"], dh * uf * sig * (1 + gf * (1 - sig)), 1.46, 2.6e-3, "dense dg")
+    assert_bf16_parity(s["du"], dh * silu(gf), 1.46, 2.6e-3, "dense du")
     if T > 80:   # (a launch of its own with fewer rows adds a forward product up in another order)
         for k in s:
             assert torch.equal(s[k], s0[k]), k
