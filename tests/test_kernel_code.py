@@ -78,8 +78,9 @@ def test_weight_gradients_start_a_tile_with_stores_under_way(kernels):
 
 
 def test_no_vector_register_is_spilled(kernels):
+    """Nor more than a few scalar ones, into lanes of a vector register."""
     for k, lines, notes in kernels:
-        assert int(notes["vgpr_spill_count"]) == 0, k
+        assert int(notes["vgpr_spill_count"]) == 0 and int(notes["sgpr_spill_count"]) <= 4, k
         assert not any("scratch_" in line for line in lines), k
 
 
