@@ -756,20 +756,20 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     auto read_b = [&](auto par, auto f_lo, auto f_hi) {
         constexpr int P = decltype(par)::value, O = P * B_STAGE;
 #pragma unroll
-            for (int f = decltype(f_lo)::value; f < decltype(f_hi)::value; f++) {
-                const int kk = f >> 2, j = f & 3;
-                if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 2048));
-                else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 4096);
-            }
+        for (int f = decltype(f_lo)::value; f < decltype(f_hi)::value; f++) {
+            const int kk = f >> 2, j = f & 3;
+            if (BKIND == CONTIG) fb[P][j][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(lds + b_frag[BKIND == CONTIG ? kk : 0] + O + j * 2048));
+            else fb[P][j][kk] = read_tr(lds + b_frag[BKIND == CONTIG ? 0 : j] + O + kk * 4096);
+        }
     };
     auto multiply = [&](auto par, auto unit, auto k) {
         constexpr int P = decltype(par)::value, I = decltype(unit)::value, kk = decltype(k)::value;
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    // operands swapped: the lane then holds 4 consecutive output columns per row
-                    acc[I][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[P][j][kk], fa[I & 1][i][kk], acc[I][i][j], 0, 0, 0);
+            for (int j = 0; j < 4; j++)
+                // operands swapped: the lane then holds 4 consecutive output columns per row
+                acc[I][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[P][j][kk], fa[I & 1][i][kk], acc[I][i][j], 0, 0, 0);
     };
     // one MFMA, then the LDS reads of the next phase behind the leading MFMAs, the rest of the MFMAs last
     auto schedule = [&](auto reads) {
@@ -1129,103 +1129,103 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     stores_follow = all_rows;
     auto rows_out = [&](auto past_caches) {   // (two loops: of a branch at each store the compiler knows less about what is under way)
 #pragma unroll
-    for (int i = 0; i < TM; i++) {
-        if (i >= e_active) break;
-        if (EPI == EPI_SWIGLU) {
-            f32x4 h[2][2];
-            u32x4 chunk[3][2];
-            // gate and up of a row in one strip row: the lanes of its first half store to g, the others to u
-            uint16_t *const gu = lane_e & 4 ? C1 : C, *const h_out = e_dense ? p.dense.C2 : p.C2;
-            // a strip is written again as soon as its reads are issued; what they bring is stored one strip later
-            auto store_gu = [&](int x) {
+        for (int i = 0; i < TM; i++) {
+            if (i >= e_active) break;
+            if (EPI == EPI_SWIGLU) {
+                f32x4 h[2][2];
+                u32x4 chunk[3][2];
+                // gate and up of a row in one strip row: the lanes of its first half store to g, the others to u
+                uint16_t *const gu = lane_e & 4 ? C1 : C, *const h_out = e_dense ? p.dense.C2 : p.C2;
+                // a strip is written again as soon as its reads are issued; what they bring is stored one strip later
+                auto store_gu = [&](int x) {
 #pragma unroll
-                for (int y = 0; y < 2; y++)
-                    if (all_rows || e_row_begin + chunk_m(i, x * 2 + y) < row_lim)
-                        *reinterpret_cast<u32x4 *>(chunk_at(gu, i, x * 2 + y)) = chunk[x][y];
-            };
+                    for (int y = 0; y < 2; y++)
+                        if (all_rows || e_row_begin + chunk_m(i, x * 2 + y) < row_lim)
+                            *reinterpret_cast<u32x4 *>(chunk_at(gu, i, x * 2 + y)) = chunk[x][y];
+                };
 #pragma unroll
-            for (int x = 0; x < 2; x++) {
+                for (int x = 0; x < 2; x++) {
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-#pragma unroll
-                    for (int y = 0; y < 4; y++) {
-                        const float gv = acc[i][x][j][y], uv = acc[i][x][2 + j][y];
-                        h[x][j][y] = (gv * fast_sigmoid(gv)) * uv;
-                        if (ROWW) h[x][j][y] *= weight[ROWW ? i : 0][x];   // h = w[row] * silu(g) * u, one rounding
-                    }
-                turn(acc[i][x][0], acc[i][x][1], acc[i][x][2], acc[i][x][3], chunk[x]);
-            }
-            store_gu(0);
-            // h of the unit's upper 16 rows beside that of its lower ones
-            turn(h[0][0], h[0][1], h[1][0], h[1][1], chunk[2]);
-            store_gu(1);
-#pragma unroll
-            for (int y = 0; y < 2; y++) {
-                const int upper = lane_e & 4 ? 16 : 0;
-                if (all_rows || e_row_begin + chunk_m(i, y) + upper < row_lim)
-                    *reinterpret_cast<u32x4 *>(chunk_at(h_out, i, y) + upper * e_ldc) = chunk[2][y];
-            }
-        } else {
-            u32x4 chunk[2];
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                if (x % 2 == 0) turn(acc[i][x >> 1][0], acc[i][x >> 1][1], acc[i][x >> 1][2], acc[i][x >> 1][3], chunk);
-                u32x4 v = chunk[x & 1];
-                const int m = e_row_begin + chunk_m(i, x);
-                if (EPI == EPI_SWIGLU_BWD) {
-                    float dot = 0.0f;   // ROWW: this lane's part of sum_i dh[m][i] * silu(g[m][i]) * u[m][i]
-                    if (all_rows || m < row_lim) {
-                        float dh[8], gv[8], uv[8], dg[8], du[8];
-                        Elem<uint16_t>::unpack(v, dh);
-                        Elem<uint16_t>::unpack(g_in[GU ? i & 1 : 0][GU ? x : 0], gv);
-                        Elem<uint16_t>::unpack(u_in[GU ? i & 1 : 0][GU ? x : 0], uv);
-#pragma unroll
-                        for (int y = 0; y < 8; y++) {
-                            const float sg = fast_sigmoid(gv[y]);
-                            const float sl = gv[y] * sg;
-                            if (ROWW) {
-                                // acc is the gradient of w * silu(g) * u: the routing weight's gradient
-                                // is its product with silu(g) * u, the activation's gets the factor w
-                                dot += dh[y] * (sl * uv[y]);
-                                dh[y] *= w_in[GU ? i & 1 : 0][GU ? x : 0];
-                            }
-                            du[y] = dh[y] * sl;
-                            dg[y] = (dh[y] * uv[y]) * (sg * (1.0f + gv[y] * (1.0f - sg)));
-                        }
-                        u32x4 vg, vu;
+                    for (int j = 0; j < 2; j++)
 #pragma unroll
                         for (int y = 0; y < 4; y++) {
-                            vg[y] = pack2_bf16(dg[2 * y], dg[2 * y + 1]);
-                            vu[y] = pack2_bf16(du[2 * y], du[2 * y + 1]);
+                            const float gv = acc[i][x][j][y], uv = acc[i][x][2 + j][y];
+                            h[x][j][y] = (gv * fast_sigmoid(gv)) * uv;
+                            if (ROWW) h[x][j][y] *= weight[ROWW ? i : 0][x];   // h = w[row] * silu(g) * u, one rounding
                         }
-                        *reinterpret_cast<u32x4 *>(chunk_at(C, i, x)) = vg;
-                        *reinterpret_cast<u32x4 *>(chunk_at(C1, i, x)) = vu;
-                    }
-                    if (ROWW) {   // this wavefront's column range of the row: its eight lanes in a fixed order
-                        dot = eight_lanes_sum(dot);
-                        if ((lane_e & 7) == 0 && m < row_lim && !e_dense) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
-                    }
-                    if (x & 1) __builtin_amdgcn_sched_barrier(0);
-                } else if (all_rows || m < row_lim) {   // (all_rows: known to the compiler where old values are waited for)
-                    if (ACCUM) {
-                        float fresh[8], prev[8];
-                        Elem<uint16_t>::unpack(v, fresh);
-                        Elem<uint16_t>::unpack(old[ACCUM ? i : 0][ACCUM ? x : 0], prev);
-#pragma unroll
-                        for (int y = 0; y < 4; y++)
-                            v[y] = pack2_bf16(prev[2 * y] + fresh[2 * y], prev[2 * y + 1] + fresh[2 * y + 1]);
-                    }
-                    u32x4 *to = reinterpret_cast<u32x4 *>(chunk_at(Cb, i, x));
-                    if (decltype(past_caches)::value && !ACCUM)
-                        store_past_caches(Cb + tile_at, (lane_at + static_cast<uint32_t>(i * 64 + x * 8) * static_cast<uint32_t>(e_ldc)) * 2, v);
-                    else if (decltype(past_caches)::value) __builtin_nontemporal_store(v, to);
-                    else *to = v;
-                    if (ACCUM) __builtin_amdgcn_sched_barrier(0);   // (all of them at once spill registers)
+                    turn(acc[i][x][0], acc[i][x][1], acc[i][x][2], acc[i][x][3], chunk[x]);
                 }
+                store_gu(0);
+                // h of the unit's upper 16 rows beside that of its lower ones
+                turn(h[0][0], h[0][1], h[1][0], h[1][1], chunk[2]);
+                store_gu(1);
+#pragma unroll
+                for (int y = 0; y < 2; y++) {
+                    const int upper = lane_e & 4 ? 16 : 0;
+                    if (all_rows || e_row_begin + chunk_m(i, y) + upper < row_lim)
+                        *reinterpret_cast<u32x4 *>(chunk_at(h_out, i, y) + upper * e_ldc) = chunk[2][y];
+                }
+            } else {
+                u32x4 chunk[2];
+#pragma unroll
+                for (int x = 0; x < 4; x++) {
+                    if (x % 2 == 0) turn(acc[i][x >> 1][0], acc[i][x >> 1][1], acc[i][x >> 1][2], acc[i][x >> 1][3], chunk);
+                    u32x4 v = chunk[x & 1];
+                    const int m = e_row_begin + chunk_m(i, x);
+                    if (EPI == EPI_SWIGLU_BWD) {
+                        float dot = 0.0f;   // ROWW: this lane's part of sum_i dh[m][i] * silu(g[m][i]) * u[m][i]
+                        if (all_rows || m < row_lim) {
+                            float dh[8], gv[8], uv[8], dg[8], du[8];
+                            Elem<uint16_t>::unpack(v, dh);
+                            Elem<uint16_t>::unpack(g_in[GU ? i & 1 : 0][GU ? x : 0], gv);
+                            Elem<uint16_t>::unpack(u_in[GU ? i & 1 : 0][GU ? x : 0], uv);
+#pragma unroll
+                            for (int y = 0; y < 8; y++) {
+                                const float sg = fast_sigmoid(gv[y]);
+                                const float sl = gv[y] * sg;
+                                if (ROWW) {
+                                    // acc is the gradient of w * silu(g) * u: the routing weight's gradient
+                                    // is its product with silu(g) * u, the activation's gets the factor w
+                                    dot += dh[y] * (sl * uv[y]);
+                                    dh[y] *= w_in[GU ? i & 1 : 0][GU ? x : 0];
+                                }
+                                du[y] = dh[y] * sl;
+                                dg[y] = (dh[y] * uv[y]) * (sg * (1.0f + gv[y] * (1.0f - sg)));
+                            }
+                            u32x4 vg, vu;
+#pragma unroll
+                            for (int y = 0; y < 4; y++) {
+                                vg[y] = pack2_bf16(dg[2 * y], dg[2 * y + 1]);
+                                vu[y] = pack2_bf16(du[2 * y], du[2 * y + 1]);
+                            }
+                            *reinterpret_cast<u32x4 *>(chunk_at(C, i, x)) = vg;
+                            *reinterpret_cast<u32x4 *>(chunk_at(C1, i, x)) = vu;
+                        }
+                        if (ROWW) {   // this wavefront's column range of the row: its eight lanes in a fixed order
+                            dot = eight_lanes_sum(dot);
+                            if ((lane_e & 7) == 0 && m < row_lim && !e_dense) p.row_dot[(col0 / COLS) * p.rows + m] = dot;
+                        }
+                        if (x & 1) __builtin_amdgcn_sched_barrier(0);
+                    } else if (all_rows || m < row_lim) {   // (all_rows: known to the compiler where old values are waited for)
+                        if (ACCUM) {
+                            float fresh[8], prev[8];
+                            Elem<uint16_t>::unpack(v, fresh);
+                            Elem<uint16_t>::unpack(old[ACCUM ? i : 0][ACCUM ? x : 0], prev);
+#pragma unroll
+                            for (int y = 0; y < 4; y++)
+                                v[y] = pack2_bf16(prev[2 * y] + fresh[2 * y], prev[2 * y + 1] + fresh[2 * y + 1]);
+                        }
+                        u32x4 *to = reinterpret_cast<u32x4 *>(chunk_at(Cb, i, x));
+                        if (decltype(past_caches)::value && !ACCUM)
+                            store_past_caches(Cb + tile_at, (lane_at + static_cast<uint32_t>(i * 64 + x * 8) * static_cast<uint32_t>(e_ldc)) * 2, v);
+                        else if (decltype(past_caches)::value) __builtin_nontemporal_store(v, to);
+                        else *to = v;
+                        if (ACCUM) __builtin_amdgcn_sched_barrier(0);   // (all of them at once spill registers)
+                    }
+                }
+                if (GU && i + 2 < TM) load_gu(i + 2);
             }
-            if (GU && i + 2 < TM) load_gu(i + 2);
         }
-    }
     };
     if (WGRAD && !EDGE && p.stream) rows_out(std::true_type{});
     else rows_out(std::false_type{});
