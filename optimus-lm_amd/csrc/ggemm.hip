@@ -150,6 +150,13 @@ __device__ __forceinline__ int64_t uniform64(int64_t v) {
     return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// One of two fields of the kernel's arguments.  Both are read: of a read on either side of a branch the compiler makes one through an
+// address that it chooses, and then reads every argument where it is used instead of all of them, a few at a time, when the kernel starts.
+// 128x128 tiles, us, so -> read together: 8 experts of 256/512, 4096 rows, gate+up 15.0 -> 14.5, down 13.2 -> 12.7, gate/up input gradient
+// 19.0 -> 18.5; 12 of 1000/712, 9003 rows, down 34.0 -> 33.1, SwiGLU backward 38.0 -> 37.4, gate/up input gradient 54.9 -> 53.4; 64 of 2048/1024, 296
+// rows, gate+up 88.9 -> 87.9, down 48.1 -> 47.0.
+template <typename T> __device__ __forceinline__ T pick(bool first, T a, T b) { return first ? a : b; }
+
 // CONTIG unit (64 rows x 64 c, 128-byte rows): chunk position = chunk ^ swz(row), conflict-free for ds_read_b128, whose
 // lanes are served sixteen at a time, with 16 consecutive rows; period 16, so rows 16 apart share it.
 __device__ __forceinline__ int swz(int row) { return (row >> 1) & 7; }
@@ -447,6 +454,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     int steps_per_phase = 0, c_wrap = 0, n_steps = 0, rot = 0;
     int active = TM;      // row units that hold rows of the expert
     bool dense = false;   // DENSE: whether the tile is the dense expert's
+    auto own = [&](auto of_dense, auto of_routed) { return DENSE ? pick(dense, of_dense, of_routed) : of_routed; };
     int once = 0;         // ONCE: whether no other row tile reads the expert's weights
     // the slot of this wavefront's direct load l of a unit: row (CONTIG) or contraction row (STRIDED) and chunk
     auto slot = [&](int l) { return (wave * L + l) * 8 + (lane >> 3); };
@@ -607,15 +615,18 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                                : WGRAD ? n0 + (b_indexed ? 0 : static_cast<int64_t>(c_begin) * ldb32)
                                        : matrix + n0;
         // EPI_SWIGLU: LDS rows 0..31 of a unit are gate rows, 32..63 up rows; a wavefront's loads lie in one of the two
-        const int second = EPI == EPI_SWIGLU && wave * L * 8 >= 32 ? 1 : 0;
-        const uint16_t *A_first = GATHER == MERGED ? p.set[product].A : dense ? p.dense.A[0] : p.A[0];
-        const uint16_t *B_first = GATHER == MERGED ? p.set[product].B : dense ? p.dense.B[second] : p.B[second];
+        const bool second = EPI == EPI_SWIGLU && wave * L * 8 >= 32;
+        const uint16_t *A_first = GATHER == MERGED ? p.set[product].A : own(p.dense.A[0], p.A[0]);
+        const uint16_t *B_first = GATHER == MERGED ? p.set[product].B
+                                : EPI == EPI_SWIGLU ? pick(second, own(p.dense.B[1], p.B[1]), own(p.dense.B[0], p.B[0])) : own(p.dense.B[0], p.B[0]);
         a_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(A_first + a_base)));
         b_tile[0] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(B_first + b_base)));
         if (TWO_PHASE) {
-            const int phase = p.phases > 1 ? 1 : 0;
-            a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((dense ? p.dense.A[phase] : p.A[phase]) + a_base)));
-            b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>((dense ? p.dense.B[phase] : p.B[phase]) + b_base)));
+            const bool two = p.phases > 1;
+            const uint16_t *A_second = pick(two, own(p.dense.A[1], p.A[1]), own(p.dense.A[0], p.A[0]));
+            const uint16_t *B_second = pick(two, own(p.dense.B[1], p.B[1]), own(p.dense.B[0], p.B[0]));
+            a_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(A_second + a_base)));
+            b_tile[1] = reinterpret_cast<const char *>(uniform64(reinterpret_cast<int64_t>(B_second + b_base)));
         }
         const int cache_key = GATHER == MERGED ? expert * 2 + (row_index != p.set[1].b_rows ? 1 : 0) : expert;
         if (GATHER_W && (GATHER != MERGED || row_index) && cache_key != cached_expert) {
@@ -1066,9 +1077,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     const bool all_rows = !EDGE && (WGRAD || e_row_begin + BM <= e_row_end);
     const int row_lim = EDGE && col0 + chunk_col >= e_n_cols ? 0 : e_row_end;
     const bool e_dense = dense;
-    uint16_t *const C = e_dense ? p.dense.C : p.C, *const C1 = e_dense ? p.dense.C1 : p.C1;
+    uint16_t *const C = own(p.dense.C, p.C), *const C1 = own(p.dense.C1, p.C1);
     uint16_t *const Cb = GATHER == MERGED ? p.set[product].C + expert * p.set[product].strideC : C + (WGRAD ? expert * p.strideC : 0);
     const int64_t e_ldc = GATHER == MERGED ? n_cols : p.ldc;
+    uint16_t *const h_out = own(p.dense.C2, p.C2);
+    const uint16_t *const g_saved = own(p.dense.G, p.G), *const u_saved = own(p.dense.U, p.U);
     // a chunk's element: block-uniform, and this lane's part of it
     const int64_t tile_at = uniform64(static_cast<int64_t>(e_row_begin + wm_e * 32) * e_ldc + col0);
     const uint32_t lane_at = static_cast<uint32_t>(chunk_row) * static_cast<uint32_t>(e_ldc) + chunk_col;
@@ -1094,8 +1107,8 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
             const int m = min(e_row_begin + chunk_m(i, x), e_row_end - 1), at = GU ? i & 1 : 0, ax = GU ? x : 0;
             const int64_t from = static_cast<int64_t>(m) * e_ldc + (EDGE ? min(col0 + chunk_col, e_n_cols - 8) : col0 + chunk_col);
             // no reader after this one: past the caches (-1 to -3 %)
-            g_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.G : p.G) + from));
-            u_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>((e_dense ? p.dense.U : p.U) + from));
+            g_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(g_saved + from));
+            u_in[at][ax] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(u_saved + from));
             w_in[at][ax] = ROWW && !e_dense ? p.row_scale[m] : 1.0f;
         }
     };
@@ -1135,7 +1148,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 f32x4 h[2][2];
                 u32x4 chunk[3][2];
                 // gate and up of a row in one strip row: the lanes of its first half store to g, the others to u
-                uint16_t *const gu = lane_e & 4 ? C1 : C, *const h_out = e_dense ? p.dense.C2 : p.C2;
+                uint16_t *const gu = lane_e & 4 ? C1 : C;
                 // a strip is written again as soon as its reads are issued; what they bring is stored one strip later
                 auto store_gu = [&](int x) {
 #pragma unroll
