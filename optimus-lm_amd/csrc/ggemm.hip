@@ -1067,7 +1067,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     // SwiGLU backward: the saved g and u (and the weights) of two units are loaded ahead of the next tile's look-ups, those of
     // a further one when its buffer has been used; the fragments' registers are free by now.  Half a unit at a time, behind the next
     // tile's loads, each was waited for.  us: 3001 tokens, hidden 1000, ffn 712, 12 experts, top-3 (128x128) 39.9 -> 37.1; 512 tokens,
-    // uneven, 64 experts of 2048/1024 77.5 -> 73; 16384 tokens (256x256) 715 -> 660 and less, whole steps of 2048 985 -> 977, 4096
+    // uneven, 64 experts of 2048/1024 as before (77); 16384 tokens (256x256) 715 -> 660 and less, whole steps of 2048 985 -> 977, 4096
     // 1546 -> 1524, 16384 uneven 5484 -> 5453 (the power limit keeps the rest), 32 experts of 1024/768, 9000 tokens, 709 -> 700.
     constexpr bool GU = EPI == EPI_SWIGLU_BWD;
     const int e_n_cols = n_cols, e_row_begin = row_begin, e_row_end = row_end, e_active = active;
