@@ -895,11 +895,11 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
         int cs1 = next_c0(cs0), cs2 = next_c0(cs1), cst = cs0;
         const char *pa1 = a_step(cs1, 1), *pa2 = a_step(cs2, 2), *pb2 = b_step(cs2, 2);
         // steps that follow step 0, for the wait in its middle: nothing to wait for where all that it needs is here.  Asked for in step 0
-        // alone, this makes the compiler copy the loop's first round, with accumulators that need not be zeroed first.  256x256 weight
-        // gradients gain by the copy (one that is carried from step to step instead: 64 experts of 2048/1024, 512 tokens, uneven, 186 -> 192 us);
-        // the 128x128 kernels, a third of whose code it was, do not, and the wait is theirs to skip for a single step only.  us, with ->
-        // without: 12 experts of 1000/712, 9003 rows, down 33.8 -> 33.0, weight gradients 75.1 -> 74.4; 8 of 256/512, 4096 rows, 13.2 -> 12.9 and 17.7 ->
-        // 17.4; 64 of 2048/1024, 296 rows, down 48.0 -> 47.4; other row products within 1 %.
+        // alone, this makes the compiler copy the loop's first round, with accumulators that need not be zeroed first.  The weight gradients
+        // gain by the copy; without it, us: 64 experts of 2048/1024, 512 tokens, uneven, 186 -> 192; added ones of 16 of 1304/600, 4096 rows,
+        // 68.5 -> 70.6, of 12 of 1000/712, 9003 rows, 71.0 -> 72.4.  In the row products of 128x128 tiles it is a third of the code for a wait
+        // that only a single step can skip; with -> without: 12 of 1000/712, 9003 rows, down 33.8 -> 33.0, 8 of 256/512, 4096 rows, 13.2 -> 12.9, 64 of
+        // 2048/1024, 296 rows, 48.0 -> 47.4, others within 1 %.
         const int left0 = __builtin_amdgcn_readfirstlane(stores_follow || n_steps == 1 ? -1 : n_steps - 1);
         // One contraction step of parity P (see the comment above the kernel).  Past the last step nothing is loaded, and
         // what is read for it is not used.
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 read_a(same, c1_, c1_, c2_);
                 multiply(same, c0_, c1_);
                 schedule(ra);
-                wait_step_loads<8, 2>(left, lds_addr);
+                wait_step_loads<8, 2>(WGRAD && t == 0 ? left0 : left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 block_barrier();
                 if (GATHER_W && left >= 2) look_up(cs3, src3);
@@ -957,7 +957,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
                 read_a(same, c2_, c1_, c2_);
                 if (FULL || active > 1) multiply(same, c1_, c1_);
                 schedule(ra);
-                wait_step_loads<6, 3>(STORES && t == 0 ? left0 : left, lds_addr);
+                wait_step_loads<6, 3>(WGRAD && t == 0 ? left0 : left, lds_addr);
                 zero_tail(cs1, other, c0_);
                 zero_tail(cst, same, c3_);
                 block_barrier();
