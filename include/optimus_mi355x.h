@@ -544,7 +544,10 @@ int om_grouped_gemm_wgrad_gathered(const void *output_grad, const void *input,
  *                              (parts = om_merged_mlp_row_dot_parts(I) = ceil(I / 64), fp32 [parts, rows]);
  *                              then as om_merged_mlp_down_dgrad with dh = row_weights[r] * dh'
  *   om_moe_row_weights_grad  : dw[t,k] = sum over parts (in order) of row_dot[part][pos]; entries of
- *                              pairs outside the expert window are not written (pre-zero them)   */
+ *                              pairs outside the expert window are not written (pre-zero them)
+ *   om_sum_ggemm_output_row_weights_grad : om_sum_ggemm_output and, in the same launch, dw[t,k] as above
+ *                              (row_dot [parts, rows]), zero for pairs outside the expert window: all of
+ *                              routing_weights_grad [T,K] is written                              */
 int om_moe_row_weights(const void *routing_weights, const int32_t *selected_experts_indices,
                        const int32_t *input_indices, const int32_t *output_indices,
                        float *row_weights, int64_t RT, int K, int weights_dtype, void *stream);
@@ -570,6 +573,12 @@ int om_moe_row_weights_grad(const float *row_dot, int parts, const int32_t *sele
                             const int32_t *input_indices, const int32_t *output_indices,
                             void *routing_weights_grad, int64_t RT, int K, int weights_dtype,
                             void *stream);
+int om_sum_ggemm_output_row_weights_grad(const void *ggemm_output, const int32_t *cum_expert_counts_ep,
+                                         const int32_t *output_indices, const void *residual,
+                                         void *final_hidden_states, int64_t T, int64_t E, int dtype,
+                                         const float *row_dot, int parts, int64_t rows,
+                                         const int32_t *selected_experts_indices, void *routing_weights_grad,
+                                         int K, int weights_dtype, void *stream);
 
 /* The four forward / input-gradient products of a block for callers that know `rows` only as a bound: under an
  * expert window the count of routed rows stays on the device, and rows is T*K.  Outputs, launches and checks go by

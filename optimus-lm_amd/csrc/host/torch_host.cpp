@@ -597,15 +597,15 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
                                           const Sinks *along_sinks = nullptr) {
     const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
     Tensor dg = make({rows, I}, x), du = make({rows, I}, x), dx_rows = make({rows, H}, x);
-    // the kernel writes the entry of every routed (token, k) pair; pairs outside the expert window stay zero
-    Tensor drw = rows == rw.numel() && !ix.bound ? make(rw.sizes(), rw) : at::zeros(rw.sizes(), rw.options());
+    Tensor drw = rows > 0 ? make(rw.sizes(), rw) : at::zeros(rw.sizes(), rw.options());
+    Tensor row_dot;
+    const int parts = om_merged_mlp_row_dot_parts(I);
+    if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
     Tensor dx = make(x.sizes(), x);
     {
         ProfiledScope scope(c, "1moeblock--7gmlp_bwd");
         if (rows > 0) {
-            const int parts = om_merged_mlp_row_dot_parts(I);
-            if (parts < 1) check(parts, "om_merged_mlp_row_dot_parts");
-            Tensor row_dot = make({parts, rows}, x, at::kFloat);
+            row_dot = make({parts, rows}, x, at::kFloat);
             const float *row_w = ix.row_weights ? ix.row_weights : fp(row_weights);
             Tensor dense_dg, dense_du;
             if (along) {
@@ -620,8 +620,6 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
                 OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u), row_w, ptr(dg),
                          ptr(du), fpm(row_dot), ix.cum, rows, ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
             }
-            OM(c, om_moe_row_weights_grad, fp(row_dot), parts, ix.sel, ix.in, ix.out, ptr(drw), rows, K, dtype_code(drw),
-               c.stream);
             wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, ix.to_choose_by(), G, I, H);
             if (along) {
                 const om_dense_expert d = dense_expert({&dense_dg, &dense_du}, {&along->w.gate, &along->w.up}, {&base, nullptr, nullptr}, along->s, T);
@@ -641,7 +639,11 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
     }
     ProfiledScope scope(c, "1moeblock--6gmlp_input_prep_bwd");
     require_device(base);
-    OM(c, om_sum_ggemm_output, ptr(dx_rows), ix.cum_ep, ix.out, ptr(base), ptr(dx), T, H, OM_BF16, c.stream);
+    if (rows > 0)
+        OM(c, om_sum_ggemm_output_row_weights_grad, ptr(dx_rows), ix.cum_ep, ix.out, ptr(base), ptr(dx), T, H, OM_BF16, fp(row_dot),
+           parts, rows, ix.sel, ptr(drw), K, dtype_code(drw), c.stream);
+    else
+        OM(c, om_sum_ggemm_output, ptr(dx_rows), ix.cum_ep, ix.out, ptr(base), ptr(dx), T, H, OM_BF16, c.stream);
     return {dx, drw};
 }
 

@@ -37,22 +37,63 @@ template <> __device__ __forceinline__ float round_as<uint16_t>(float x) {
     return bf16_bits_to_f32(f32_to_bf16_bits(x));
 }
 
+// The gradient of a token's routing weights beside the sum of its rows: dw[t,k] = sum over the `parts` column ranges of
+// row_dot[part][pos], added in order, pos the row of pair (t,k); zero where the pair has none here.  A launch of its own for this
+// (and one that zeroed dw under an expert window) is mostly a launch; here its loads go out beside those of the rows.  us, sum +
+// launch of its own -> together: 2048 tokens of 256, top-2, 4.1 + 4.0 -> 4.5; 512 of 2048, top-8, 5.8 + 4.8 -> 7.3; 3001 of 1000, top-3, 6.8 + 4.6
+// -> 8.5; 16384 of 2048, top-8, 107.5 + 13.8 -> 107.5; 8192 of 7168, a window of an eighth, 87.0 + 6.8 + 4.8 -> 93.2.
+struct RowGrads {
+    const float *row_dot = nullptr;
+    const int32_t *selected_experts_indices = nullptr;
+    void *dw = nullptr;
+    int64_t row_pitch = 0;   // entries of a part
+    int parts = 0, K = 0, bf16 = 0;
+    __device__ __forceinline__ void put(int64_t at, float v) const {
+        if (bf16) static_cast<uint16_t *>(dw)[at] = f32_to_bf16_bits(v);
+        else static_cast<float *>(dw)[at] = v;
+    }
+    // token t, whose pairs are entries i0 .. i1 - 1; one wavefront
+    __device__ __forceinline__ void token(const int32_t *output_indices, int64_t t, int32_t i0, int32_t i1, int lane) const {
+        for (int32_t ib = i0; ib < i1; ib += 64) {
+            if (ib + lane >= i1) continue;
+            const int32_t pos = output_indices[ib + lane];
+            const int k = selected_experts_indices[ib + lane];
+            float s = 0.0f;
+            for (int p0 = 0; p0 < parts; p0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = (p0 + u < parts) ? row_dot[(p0 + u) * row_pitch + pos] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < 8; u++) s += v[u];
+            }
+            put(t * K + k, s);
+        }
+        if (i1 - i0 == K) return;
+        for (int k = lane; k < K; k += 64) {
+            bool here = false;
+            for (int32_t i = i0; i < i1; i++) here |= selected_experts_indices[i] == k;
+            if (!here) put(t * K + k, 0.0f);
+        }
+    }
+};
+
 // hidden_grad[t,:] = sum_i ggemm_input_grad[output_indices[i],:],  i in [cum_ep[t], cum_ep[t+1])
 // SCALE: final[t,:] = sum_i w[t, sel_idx[i]] * y[output_indices[i],:]
 // residual != null: final[t,:] = residual[t,:] + T(that sum), the sum rounded to T first
 // CH: 64-vector column chunks that a lane owns per pass; RU: rows in flight per chunk; the chunks are dealt
 // over blockIdx.y (see few_tokens).
-template <typename T, typename TW, bool SCALE, int CH, int RU>
+template <typename T, typename TW, bool SCALE, int CH, int RU, bool GRADS = false>
 __global__ __launch_bounds__(256) void token_reduce_kernel(
     const T *__restrict__ rows, const TW *__restrict__ routing_weights,
     const int32_t *__restrict__ cum_expert_counts_ep,
     const int32_t *__restrict__ selected_experts_indices,
     const int32_t *__restrict__ output_indices, T *__restrict__ out, int64_t T_tokens, int K,
-    int64_t E, bool vec_ok, const T *__restrict__ residual = nullptr) {
+    int64_t E, bool vec_ok, const T *__restrict__ residual, const RowGrads grads) {
     const int lane = threadIdx.x & 63;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * ROWS_PER_BLOCK + (threadIdx.x >> 6);
     if (t >= T_tokens) return;
     const int32_t i0 = cum_expert_counts_ep[t], i1 = cum_expert_counts_ep[t + 1];
+    if (GRADS && blockIdx.y == 0) grads.token(output_indices, t, i0, i1, lane);
     T *dst = out + t * E;
     const T *res = residual ? residual + t * E : nullptr;
     constexpr int V = Elem<T>::VEC;
@@ -275,17 +316,18 @@ template <typename T> bool row_vec_ok(const void *a, const void *b, const void *
 // 6.8 -> 3.8, 512 9.9 -> 4.8, 1024 10.7 -> 7.6, 2048 13.2 -> 14.7; hidden 7168, 8 rows: 64 tokens 27 -> 4, 512
 // 32 -> 11; 1 row: 512 9.2 -> 6.7, 1024 10.2 -> 11.9; hence the line.
 inline bool few_tokens(int64_t tokens, int64_t vectors) { return tokens <= 512 || tokens * vectors <= (1 << 18); }
-template <typename T, typename TW, bool SCALE>
+template <typename T, typename TW, bool SCALE, bool GRADS = false>
 void token_reduce_launch(const T *rows, const TW *weights, const int32_t *cum_ep, const int32_t *sel, const int32_t *out_idx,
-                         T *out, int64_t T_tokens, int K, int64_t E, bool vec_ok, const T *residual, hipStream_t st) {
+                         T *out, int64_t T_tokens, int K, int64_t E, bool vec_ok, const T *residual, hipStream_t st,
+                         const RowGrads &grads = RowGrads()) {
     const int64_t vectors = E / Elem<T>::VEC, chunks = (vectors + 63) / 64;
     const bool few = few_tokens(T_tokens, vectors);
     const dim3 grid(static_cast<unsigned>((T_tokens + ROWS_PER_BLOCK - 1) / ROWS_PER_BLOCK),
                     few ? static_cast<unsigned>(chunks < 1 ? 1 : chunks > 65535 ? 65535 : chunks) : 1u);
     if (few)
-        token_reduce_kernel<T, TW, SCALE, 1, 8><<<grid, 256, 0, st>>>(rows, weights, cum_ep, sel, out_idx, out, T_tokens, K, E, vec_ok, residual);
+        token_reduce_kernel<T, TW, SCALE, 1, 8, GRADS><<<grid, 256, 0, st>>>(rows, weights, cum_ep, sel, out_idx, out, T_tokens, K, E, vec_ok, residual, grads);
     else
-        token_reduce_kernel<T, TW, SCALE, 4, 1><<<grid, 256, 0, st>>>(rows, weights, cum_ep, sel, out_idx, out, T_tokens, K, E, vec_ok, residual);
+        token_reduce_kernel<T, TW, SCALE, 4, 1, GRADS><<<grid, 256, 0, st>>>(rows, weights, cum_ep, sel, out_idx, out, T_tokens, K, E, vec_ok, residual, grads);
 }
 
 inline unsigned row_blocks(int64_t rows) {
@@ -416,6 +458,40 @@ extern "C" int om_sum_ggemm_output(const void *ggemm_output, const int32_t *cum_
                                    void *stream) {
     return reduce_ggemm_output_launch(ggemm_output, nullptr, cum_expert_counts_ep, nullptr, output_indices,
                                       final_hidden_states, T, 0, E, dtype, OM_F32, 1, residual, stream);
+}
+
+extern "C" int om_sum_ggemm_output_row_weights_grad(const void *ggemm_output, const int32_t *cum_expert_counts_ep,
+                                                    const int32_t *output_indices, const void *residual,
+                                                    void *final_hidden_states, int64_t T, int64_t E, int dtype,
+                                                    const float *row_dot, int parts, int64_t rows,
+                                                    const int32_t *selected_experts_indices, void *routing_weights_grad,
+                                                    int K, int weights_dtype, void *stream) {
+    if (dtype != OM_F32 && dtype != OM_BF16) return OM_ERR_DTYPE;
+    if (weights_dtype != OM_F32 && weights_dtype != OM_BF16) return OM_ERR_DTYPE;
+    if (T < 0 || E < 0 || T > 0x7fffffffLL || rows < 0 || K < 1 || parts < 1) return OM_ERR_SHAPE;
+    if (T == 0) return OM_OK;
+    if (!cum_expert_counts_ep || !routing_weights_grad || (E > 0 && !final_hidden_states)) return OM_ERR_NULL;
+    if (rows > 0 && (!row_dot || !selected_experts_indices || !output_indices)) return OM_ERR_NULL;
+    RowGrads grads;
+    grads.row_dot = row_dot;
+    grads.selected_experts_indices = selected_experts_indices;
+    grads.dw = routing_weights_grad;
+    grads.row_pitch = rows;
+    grads.parts = parts;
+    grads.K = K;
+    grads.bf16 = weights_dtype == OM_BF16;
+    hipStream_t st = om_stream(stream);
+    if (dtype == OM_F32)
+        token_reduce_launch<float, float, false, true>(static_cast<const float *>(ggemm_output), nullptr, cum_expert_counts_ep, nullptr,
+                                                       output_indices, static_cast<float *>(final_hidden_states), T, 0, E,
+                                                       row_vec_ok<float>(ggemm_output, final_hidden_states, residual, E),
+                                                       static_cast<const float *>(residual), st, grads);
+    else
+        token_reduce_launch<uint16_t, float, false, true>(static_cast<const uint16_t *>(ggemm_output), nullptr, cum_expert_counts_ep, nullptr,
+                                                          output_indices, static_cast<uint16_t *>(final_hidden_states), T, 0, E,
+                                                          row_vec_ok<uint16_t>(ggemm_output, final_hidden_states, residual, E),
+                                                          static_cast<const uint16_t *>(residual), st, grads);
+    return om_launch_status();
 }
 
 extern "C" int om_moe_row_weights(const void *routing_weights, const int32_t *selected_experts_indices,

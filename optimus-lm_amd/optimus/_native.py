@@ -149,6 +149,8 @@ SIGNATURES = {
                                                   c_int, c_int, c_int, c_i64, c_void_p]),
     "om_moe_row_weights_grad": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_i64,
                                         c_int, c_int, c_void_p]),
+    "om_sum_ggemm_output_row_weights_grad": (c_int, [c_void_p] * 5 + [c_i64, c_i64, c_int, c_void_p, c_int, c_i64, c_void_p,
+                                             c_void_p, c_int, c_int, c_void_p]),
     "om_merged_mlp_down_dgrad": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                          c_void_p, c_i64, c_int, c_int, c_int, c_i64, c_void_p]),
     "om_merged_mlp_gate_up_dgrad": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

@@ -211,6 +211,15 @@ def test_routing_weight_folded_into_the_expert_mlp(lib):
     assert lib.om_moe_row_weights_grad(None, 16, P, P, P, P, 131072, 8, F32, None) == NULL
     assert lib.om_moe_row_weights_grad(P, 16, P, P, P, P, 131072, 8, 9, None) == DTYPE
     assert lib.om_moe_row_weights_grad(None, 16, None, None, None, None, 0, 8, F32, None) == OK
+    sums = lib.om_sum_ggemm_output_row_weights_grad
+    assert sums(P, None, P, None, P, 16384, 2048, BF16, P, 16, 131072, P, P, 8, BF16, None) == NULL
+    assert sums(P, P, P, None, P, 16384, 2048, BF16, None, 16, 131072, P, P, 8, BF16, None) == NULL
+    assert sums(P, P, P, None, P, 16384, 2048, BF16, P, 16, 131072, P, None, 8, BF16, None) == NULL
+    assert sums(P, P, P, None, P, 16384, 2048, BF16, P, 0, 131072, P, P, 8, BF16, None) == SHAPE
+    assert sums(P, P, P, None, P, 16384, 2048, BF16, P, 16, 131072, P, P, 0, BF16, None) == SHAPE
+    assert sums(P, P, P, None, P, 16384, 2048, 7, P, 16, 131072, P, P, 8, BF16, None) == DTYPE
+    assert sums(P, P, P, None, P, 16384, 2048, BF16, P, 16, 131072, P, P, 8, 7, None) == DTYPE
+    assert sums(None, None, None, None, None, 0, 2048, BF16, None, 16, 0, None, None, 8, BF16, None) == OK
 
 
 def test_products_over_a_bound_of_the_rows(lib):

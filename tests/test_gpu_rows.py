@@ -134,3 +134,35 @@ def test_token_sums_on_both_sides_of_the_few_tokens_line(cuda, oracle_lib, dtype
         hg = torch.empty(T, E, dtype=dtype, device=cuda)
         ops.shuffle_sub_matrix_reduce(y.to(cuda), ce, oi, hg)
         assert np.array_equal(bits(hg), oracle_lib.shuffle_sub_matrix_reduce(bits(y), idx["cum_expert_counts_ep"], idx["output_indices"], T))
+
+
+@pytest.mark.parametrize("T,N,K,E,I,start,end,dtype,wdt", [
+    (8, 4, 2, 8, 8, 0, 4, torch.bfloat16, torch.bfloat16), (80, 8, 3, 264, 200, 0, 8, torch.bfloat16, torch.bfloat16),
+    (704, 16, 8, 1000, 1048, 4, 6, torch.bfloat16, torch.float32), (600, 130, 70, 2048, 64, 0, 130, torch.bfloat16, torch.float32),
+    (40, 12, 3, 12, 520, 6, 12, torch.float32, torch.float32), (24, 8, 2, 64, 72, 0, 1, torch.bfloat16, torch.bfloat16)])
+def test_row_sum_with_the_routing_weights_gradient(cuda, oracle_lib, T, N, K, E, I, start, end, dtype, wdt):
+    """One launch against om_sum_ggemm_output and the column ranges added in order; `rows` is a bound under a window."""
+    from optimus import _native as n
+    se, idx, _, y, _ = _setup(T, N, K, E, start, end, dtype, oracle_lib, seed=T)
+    TR = idx["num_routed_tokens"]
+    rows = T * K if end - start < N else TR
+    parts = n.lib().om_merged_mlp_row_dot_parts(I)
+    dot = torch.randn(parts, rows, generator=torch.Generator().manual_seed(4))
+    d = lambda a: torch.from_numpy(a).to(cuda)
+    oi, si, ce = d(idx["output_indices"]), d(idx["selected_experts_indices"]), d(idx["cum_expert_counts_ep"])
+    yg, dotg, residual = y.to(cuda), dot.to(cuda), torch.randn(T, E, generator=torch.Generator().manual_seed(5)).to(dtype).to(cuda)
+    for res in (None, residual):
+        want, got = torch.empty(T, E, dtype=dtype, device=cuda), torch.empty(T, E, dtype=dtype, device=cuda)
+        dw = torch.full((T, K), 7.0, dtype=wdt, device=cuda)
+        n.check(n.lib().om_sum_ggemm_output(n.ptr(yg), n.ptr(ce), n.ptr(oi), n.ptr(res), n.ptr(want), T, E, n.dtype_code(yg), n.stream()), "sum")
+        n.check(n.lib().om_sum_ggemm_output_row_weights_grad(n.ptr(yg), n.ptr(ce), n.ptr(oi), n.ptr(res), n.ptr(got), T, E,
+                                                             n.dtype_code(yg), n.ptr(dotg), parts, rows, n.ptr(si), n.ptr(dw), K,
+                                                             n.dtype_code(dw), n.stream()), "sum and gradient")
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+        sums = torch.zeros(rows)
+        for part in dot:
+            sums += part
+        token = np.repeat(np.arange(T), np.diff(idx["cum_expert_counts_ep"]))
+        ref = torch.zeros(T, K)
+        ref[torch.from_numpy(token), torch.from_numpy(idx["selected_experts_indices"]).long()] = sums[torch.from_numpy(idx["output_indices"]).long()]
+        assert torch.equal(dw.cpu(), ref.to(wdt))
