@@ -213,6 +213,16 @@ int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t T, int H, 
                          void *dweight, int dweight_dtype, void *workspace,
                          int64_t workspace_bytes, void *stream);
 
+/* om_router_softmax_bwd: the whole backward of a softmax router of up to 64 experts in one call, with the bits of the
+ * separate calls: om_route_softmax_topk_bwd, the sum with another gradient `dlogits` of the logits (null, or [T,N] in
+ * their type; rounded to it), om_router_gate_dgrad (dx [T,H] bf16 = base + dlogits @ gate_weight, base may be null) and
+ * om_router_gate_wgrad (dweight [N,H]).  T >= 1; workspace: om_router_softmax_bwd_workspace_bytes, 16-byte aligned.  */
+int64_t om_router_softmax_bwd_workspace_bytes(int64_t T, int H, int N);
+int om_router_softmax_bwd(const void *x, const void *gate_weight, const void *logits, int logits_dtype, const int64_t *experts,
+                          const void *dweights, int dweights_dtype, const void *dlogits, const void *base, void *dx,
+                          void *dweight, int dweight_dtype, int64_t T, int H, int N, int K, int norm_topk_prob, void *workspace,
+                          int64_t workspace_bytes, void *stream);
+
 /* The gate projection of a float32 module and its backward, replacing the nn.Linear behind
  * `router_logits = self.gate(hidden_states)` (optimus/models/common/moe.py:456) where the block is
  * kept in float32 (the reference's small CPU-runnable configuration): plain float32 products,

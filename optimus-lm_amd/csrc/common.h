@@ -154,3 +154,8 @@ int om_ggemm_stream_fwd(const void *x, const void *w, void *out, const int32_t *
 int om_gate_route_splits(int64_t T, int H, int N);
 void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int N, int splits, float *partial,
                              hipStream_t stream);
+// The softmax router's backward (route.hip) as the gate's gradients' producer: dlogits in float32 (rounded to the logits' type on the
+// way, as the separate entry point stores them; `more`: another gradient of the logits, in their type, is added with that type's rounding), and `n_zero` words zeroed.
+void om_launch_softmax_bwd(const void *logits, int logits_dtype, const int64_t *experts, const void *dweights, int dweights_dtype,
+                           const void *more, int64_t T, int N, int K, int renorm, float *dlogits, unsigned *zero, int n_zero,
+                           hipStream_t stream);

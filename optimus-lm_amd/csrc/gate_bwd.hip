@@ -58,21 +58,19 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 // grid (H / 128, splits); 256 threads.  NB accumulators per wavefront cover N = 32 NB rows of dW, of
 // which the first n_real exist (the rest are zero columns of the dlogits tile); wavefront w owns
 // the 32 columns [h0 + 32 w, h0 + 32 w + 32) of the block's slice and all rows of dW.
-template <int NB>
-__global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restrict__ x,
-                                                         const float *__restrict__ dlogits,
-                                                         int64_t T, int H, int n_real,
-                                                         int64_t tokens_per_split,
-                                                         float *__restrict__ partial) {
+// SHARED: the partials are stored at device scope, for the block of the launch that adds them up.
+template <int NB> constexpr int WGRAD_LDS = TC * HT * 2 + TC * (NB * 32 < 128 ? 128 : NB * 32) * 2;
+template <int NB, bool SHARED>
+__device__ __forceinline__ void gate_wgrad_block(const uint16_t *__restrict__ x, const float *__restrict__ dlogits, int64_t T, int H,
+                                                 int n_real, int64_t tokens_per_split, float *partial, int slice, int split, char *lds) {
     constexpr int N = NB * 32;
     constexpr int RD = N < 128 ? 128 : N;       // LDS row length of the dlogits tile (elements)
     constexpr int XL = TC * HT / 8 / 256;       // 16-byte x chunks per thread per stage
     constexpr int DL = TC * N / 4 / 256;        // float4 dlogits loads per thread per stage
-    __shared__ __attribute__((aligned(16))) char xs[TC * HT * 2];
-    __shared__ __attribute__((aligned(16))) char ds[TC * RD * 2];
+    char *const xs = lds, *const ds = lds + TC * HT * 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h0 = blockIdx.x * HT;
-    const int64_t t_begin = static_cast<int64_t>(blockIdx.y) * tokens_per_split;
+    const int h0 = slice * HT;
+    const int64_t t_begin = static_cast<int64_t>(split) * tokens_per_split;
     int64_t t_end = t_begin + tokens_per_split;
     if (t_end > T) t_end = T;
 
@@ -146,14 +144,22 @@ __global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restr
         }
     }
     const int h = h0 + wave * 32 + (lane & 31);
-    float *out = partial + (static_cast<int64_t>(blockIdx.y) * n_real) * H + h;
+    float *out = partial + (static_cast<int64_t>(split) * n_real) * H + h;
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int n = b * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-            if (n < n_real && h < H) out[static_cast<int64_t>(n) * H] = acc[b][r];
+            if (n >= n_real || h >= H) continue;
+            if (SHARED) __hip_atomic_store(out + static_cast<int64_t>(n) * H, acc[b][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else out[static_cast<int64_t>(n) * H] = acc[b][r];
         }
+}
+template <int NB>
+__global__ __launch_bounds__(256) void gate_wgrad_kernel(const uint16_t *__restrict__ x, const float *__restrict__ dlogits, int64_t T, int H,
+                                                         int n_real, int64_t tokens_per_split, float *__restrict__ partial) {
+    __shared__ __attribute__((aligned(16))) char lds[WGRAD_LDS<NB>];
+    gate_wgrad_block<NB, false>(x, dlogits, T, H, n_real, tokens_per_split, partial, blockIdx.x, blockIdx.y, lds);
 }
 
 // The same for more than 128 experts, a multiple of 4 of them: 256 rows and 256 columns of dW per block of eight wavefronts (64 x
@@ -305,6 +311,12 @@ __global__ __launch_bounds__(256) void gate_wgrad_reduce_kernel(const float *__r
     }
 }
 
+void gate_wgrad_reduce_launch(const float *ws, int splits, int64_t nh, void *dweight, int dweight_dtype, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>((nh / 4 + 255) / 256));
+    if (dweight_dtype == OM_F32) gate_wgrad_reduce_kernel<float><<<grid, dim3(256), 0, st>>>(ws, splits, nh, static_cast<float *>(dweight));
+    else gate_wgrad_reduce_kernel<uint16_t><<<grid, dim3(256), 0, st>>>(ws, splits, nh, static_cast<uint16_t *>(dweight));
+}
+
 inline bool gate_wgrad_wide(int N) { return N > 128 && N % 4 == 0; }
 
 // Token ranges: the blocks that the chip holds at once (two per CU, one of the wide kernel's), at least two stages of tokens each.
@@ -344,14 +356,12 @@ inline size_t gate_dgrad_lds(int N) {
 // experts 146 -> 113 us, 16384 x 2048, 64 experts 41 -> 36, 3001 x 1000, 12 experts 10.8 -> 6.4.
 // BATCHES * 4 slices of 16 experts; ALIGNED: rows of dlogits are whole 16-byte vectors (N % 4 == 0)
 template <int BATCHES, bool ALIGNED>
-__global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restrict__ dlogits,
-                                                            const uint16_t *__restrict__ weight,
-                                                            const uint16_t *base, uint16_t *out, int64_t T,
-                                                            int H, int N) {
-    extern __shared__ __attribute__((aligned(16))) char lds[];
+__device__ __forceinline__ void gate_dgrad_block(const float *__restrict__ dlogits, const uint16_t *__restrict__ weight,
+                                                 const uint16_t *base, uint16_t *out, int64_t T, int H, int N, int slice,
+                                                 int64_t token_block, char *lds) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h0 = blockIdx.x * DG_HT;
-    const int64_t t0 = static_cast<int64_t>(blockIdx.y) * DG_TOK + wave * 32;
+    const int h0 = slice * DG_HT;
+    const int64_t t0 = token_block * DG_TOK + wave * 32;
     const int n_pad = (N + 15) & ~15;
     for (int q = tid; q < n_pad * (DG_HT / 8); q += 256) {
         const int n = q / (DG_HT / 8), ch = q % (DG_HT / 8);
@@ -460,6 +470,68 @@ __global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restr
             }
             __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(out + o));
         }
+    }
+}
+
+template <int BATCHES, bool ALIGNED>
+__global__ __launch_bounds__(256, 2) void gate_dgrad_kernel(const float *__restrict__ dlogits, const uint16_t *__restrict__ weight,
+                                                            const uint16_t *base, uint16_t *out, int64_t T, int H, int N) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    gate_dgrad_block<BATCHES, ALIGNED>(dlogits, weight, base, out, T, H, N, blockIdx.x, blockIdx.y, lds);
+}
+
+// Both gradients of the gate in one launch, up to 64 experts: either alone leaves most of the chip idle at small sizes and waits for one miss
+// after the other.  us, two launches -> one: 2048 tokens, hidden 256, 8 experts 5.8 + 4.8 (and 2.9 for the sum of the ranges) -> 7.4 with that
+// sum; 3001 of 1000, 12 experts 6.4 + 5.6 -> 7.6; 512 of 2048, 64 experts 7.2 + 5.9 -> 7.7; 16384 of 2048 34.8 + 22.6 -> 51.6.  Blocks 0 .. slices * splits - 1 are those of the weight gradient, the
+// others those of the input gradient.  TOGETHER: the block that finishes a slice's last token range adds the ranges up (`done`: a count
+// per slice, zero before the launch); else a launch behind this one does.
+template <int NB, bool ALIGNED, bool TOGETHER, typename TD>
+__global__ __launch_bounds__(256, 2) void gate_bwd_kernel(const uint16_t *__restrict__ x, const float *__restrict__ dlogits,
+                                                          const uint16_t *__restrict__ weight, const uint16_t *base, uint16_t *dx,
+                                                          int64_t T, int H, int N, int64_t tokens_per_split, int splits, float *partial,
+                                                          unsigned *done, TD *dweight) {
+    __shared__ __attribute__((aligned(16))) char lds[WGRAD_LDS<NB> > DG_STRIPS ? WGRAD_LDS<NB> : DG_STRIPS];
+    static_assert(NB * 32 * DG_HT * 2 <= DG_STRIPS && HT == DG_HT, "the weight tile lies in the strips' place");
+    const int slices = (H + HT - 1) / HT, b = blockIdx.x, slice = b % slices;
+    if (b >= slices * splits) {
+        gate_dgrad_block<1, ALIGNED>(dlogits, weight, base, dx, T, H, N, slice, b / slices - splits, lds);
+        return;
+    }
+    gate_wgrad_block<NB, TOGETHER>(x, dlogits, T, H, N, tokens_per_split, partial, slice, b / slices, lds);
+    if (!TOGETHER) return;
+    // This block's partials are stored, and the others' read, at device scope, and the stores have completed before the block is
+    // counted, so the last one sees them all (without writing back an L2: see grad_sumsq_kernel in gradnorm.hip).
+    __shared__ bool last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(done + slice, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned>(splits) - 1;
+    __syncthreads();
+    if (!last) return;
+    const int h = slice * HT + threadIdx.x % HT;
+    if (h >= H) return;
+    const int64_t nh = static_cast<int64_t>(N) * H;
+    constexpr int ROWS = 4, STEP = 256 / HT;     // rows of dW in flight per thread, and how far they are apart
+    for (int n0 = threadIdx.x / HT; n0 < N; n0 += ROWS * STEP) {
+        const float *from[ROWS];
+        float s[ROWS] = {};
+#pragma unroll
+        for (int i = 0; i < ROWS; i++) from[i] = partial + static_cast<int64_t>(min(n0 + i * STEP, N - 1)) * H + h;
+        for (int k0 = 0; k0 < splits; k0 += 8) {   // as gate_wgrad_reduce_kernel adds them
+            float v[8][ROWS];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int i = 0; i < ROWS; i++)
+                    v[u][i] = __hip_atomic_load(from[i] + min(k0 + u, splits - 1) * nh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int i = 0; i < ROWS; i++) s[i] += k0 + u < splits ? v[u][i] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < ROWS; i++)
+            if (n0 + i * STEP < N) Elem<TD>::store(dweight + static_cast<int64_t>(n0 + i * STEP) * H + h, s[i]);
     }
 }
 
@@ -598,6 +670,11 @@ __global__ __launch_bounds__(512) void gate_dgrad_wide_kernel(const float *__res
     }
 }
 
+// Whether the last block of a slice adds its token ranges: where it has at most two rounds of loads to wait for.  It stores and loads
+// past the L2s: 8 experts, 16 ranges 2 us for the launch of 3; with a round per eight rows and eight ranges 12 experts, 23 ranges
+// took 10 us for 4, 64 experts, 4 ranges 17 for 5.
+inline bool gate_bwd_together(int splits, int N) { return (N + 7) / 8 * ((splits + 7) / 8) <= 2; }
+
 }  // namespace
 
 extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weight, const void *base,
@@ -656,6 +733,57 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
     return om_launch_status();
 }
 
+namespace {
+bool gate_bwd_shape_ok(int64_t T, int H, int N) {
+    return T >= 1 && H >= 8 && H % 8 == 0 && N >= 1 && N <= 64 && (T + DG_TOK - 1) / DG_TOK * ((H + DG_HT - 1) / DG_HT) <= (1 << 24);
+}
+int64_t gate_bwd_counts(int H) { return ((H + HT - 1) / HT + 3) / 4 * 4; }   // (16-byte aligned behind them)
+}  // namespace
+
+// workspace of om_router_softmax_bwd: counts, dlogits, partials
+extern "C" int64_t om_router_softmax_bwd_workspace_bytes(int64_t T, int H, int N) {
+    if (!gate_bwd_shape_ok(T, H, N)) return OM_ERR_SHAPE;
+    return (gate_bwd_counts(H) + (T * N + 3) / 4 * 4 + static_cast<int64_t>(gate_wgrad_splits(T, H, N)) * N * H) * 4;
+}
+
+extern "C" int om_router_softmax_bwd(const void *x, const void *gate_weight, const void *logits, int logits_dtype, const int64_t *experts,
+                                     const void *dweights, int dweights_dtype, const void *dlogits, const void *base, void *dx,
+                                     void *dweight, int dweight_dtype, int64_t T, int H, int N, int K, int norm_topk_prob,
+                                     void *workspace, int64_t workspace_bytes, void *stream) {
+    for (int dtype : {logits_dtype, dweights_dtype, dweight_dtype})
+        if (dtype != OM_BF16 && dtype != OM_F32) return OM_ERR_DTYPE;
+    if (!gate_bwd_shape_ok(T, H, N) || K < 1 || K > N) return OM_ERR_SHAPE;
+    if (!x || !gate_weight || !logits || !experts || !dweights || !dx || !dweight || !workspace) return OM_ERR_NULL;
+    for (const void *p : {x, gate_weight, base, static_cast<const void *>(dx), static_cast<const void *>(dweight), static_cast<const void *>(workspace)})
+        if (!om_aligned16(p)) return OM_ERR_ALIGN;
+    if (workspace_bytes < om_router_softmax_bwd_workspace_bytes(T, H, N)) return OM_ERR_WORKSPACE;
+    const int splits = gate_wgrad_splits(T, H, N), slices = (H + HT - 1) / HT;
+    const int64_t nh = static_cast<int64_t>(N) * H;
+    unsigned *done = static_cast<unsigned *>(workspace);
+    float *dl = static_cast<float *>(workspace) + gate_bwd_counts(H), *ws = dl + (T * N + 3) / 4 * 4;
+    hipStream_t st = om_stream(stream);
+    om_launch_softmax_bwd(logits, logits_dtype, experts, dweights, dweights_dtype, dlogits, T, N, K, norm_topk_prob, dl, done, slices, st);
+    const int64_t stages = (T + TC - 1) / TC, tokens_per_split = (stages + splits - 1) / splits * TC;
+    const dim3 grid(slices * splits + static_cast<unsigned>((T + DG_TOK - 1) / DG_TOK) * slices);
+    const bool together = gate_bwd_together(splits, N);
+#define OM_BWD(NB, ALIGNED, TOGETHER, TD)                                                                                                         gate_bwd_kernel<NB, ALIGNED, TOGETHER, TD><<<grid, dim3(256), 0, st>>>(static_cast<const uint16_t *>(x), dl, static_cast<const uint16_t *>(gate_weight),                                                                  static_cast<const uint16_t *>(base), static_cast<uint16_t *>(dx), T, H, N,                                                                      tokens_per_split, splits, ws, done, static_cast<TD *>(dweight))
+#define OM_BWD_N(TD)                                       \
+    do {                                                   \
+        if (together && N % 4 == 0) OM_BWD(1, true, true, TD);  \
+        else if (together) OM_BWD(1, false, true, TD);     \
+        else if (N <= 32 && N % 4 == 0) OM_BWD(1, true, false, TD); \
+        else if (N <= 32) OM_BWD(1, false, false, TD);     \
+        else if (N % 4 == 0) OM_BWD(2, true, false, TD);   \
+        else OM_BWD(2, false, false, TD);                  \
+    } while (0)
+    if (dweight_dtype == OM_F32) OM_BWD_N(float);
+    else OM_BWD_N(uint16_t);
+#undef OM_BWD_N
+#undef OM_BWD
+    if (!together) gate_wgrad_reduce_launch(ws, splits, nh, dweight, dweight_dtype, st);
+    return om_launch_status();
+}
+
 extern "C" int64_t om_router_gate_wgrad_workspace_bytes(int64_t T, int H, int N) {
     if (!gate_wgrad_shape_ok(T, H, N)) return OM_ERR_SHAPE;
     return static_cast<int64_t>(gate_wgrad_splits(T, H, N)) * N * H * 4;
@@ -689,10 +817,6 @@ extern "C" int om_router_gate_wgrad(const void *x, const float *dlogits, int64_t
         gate_wgrad_kernel<4><<<grid, dim3(256), 0, st>>>(xp, dlogits, T, H, N, tokens_per_split, ws);
     else
         gate_wgrad_kernel<8><<<grid, dim3(256), 0, st>>>(xp, dlogits, T, H, N, tokens_per_split, ws);
-    const unsigned rblocks = static_cast<unsigned>((nh / 4 + 255) / 256);
-    if (dweight_dtype == OM_F32)
-        gate_wgrad_reduce_kernel<float><<<dim3(rblocks), dim3(256), 0, st>>>(ws, splits, nh, static_cast<float *>(dweight));
-    else
-        gate_wgrad_reduce_kernel<uint16_t><<<dim3(rblocks), dim3(256), 0, st>>>(ws, splits, nh, static_cast<uint16_t *>(dweight));
+    gate_wgrad_reduce_launch(ws, splits, nh, dweight, dweight_dtype, st);
     return om_launch_status();
 }

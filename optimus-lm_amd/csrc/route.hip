@@ -206,12 +206,15 @@ __global__ __launch_bounds__(256) void partial_softmax_topk_kernel(const float *
 
 // dlogits_i = p_i * (dp_i - sum_j dp_j p_j), dp = scatter of dw over the selected experts, and
 // with renormalisation dw_k = (dw'_k - sum_j dw'_j w_j / S) / S, S = sum_k w_k, w_k = p[e_k].
-template <int PER, typename T, typename TW>
+// TO: T, or float for the gate's gradients (om_launch_softmax_bwd, which says what the last three arguments are).
+template <int PER, typename T, typename TW, typename TO>
 __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(const T *__restrict__ logits,
                                                                const int64_t *__restrict__ experts,
                                                                const TW *__restrict__ dweights,
                                                                int64_t Tn, int N, int K, int renorm,
-                                                               T *__restrict__ dlogits) {
+                                                               TO *__restrict__ dlogits, const T *__restrict__ more, unsigned *zero, int n_zero) {
+    if (n_zero > 0 && blockIdx.x == 0)
+        for (int i = threadIdx.x; i < n_zero; i += 256) zero[i] = 0;
     const int lane = threadIdx.x & 63;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * TOKENS_PER_BLOCK + (threadIdx.x >> 6);
     if (t >= Tn) return;
@@ -241,7 +244,14 @@ __global__ __launch_bounds__(256) void softmax_topk_bwd_kernel(const T *__restri
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int i = lane + 64 * j;
-        if (i < N) Elem<T>::store(dlogits + t * N + i, p[j] * (dp[j] - inner));
+        if (i >= N) continue;
+        float d = p[j] * (dp[j] - inner);
+        if (sizeof(T) == 2) d = bf16_bits_to_f32(f32_to_bf16_bits(d));
+        if (more) {
+            d += load_logit<T>(more + t * N + i);
+            if (sizeof(T) == 2) d = bf16_bits_to_f32(f32_to_bf16_bits(d));
+        }
+        Elem<TO>::store(dlogits + t * N + i, d);
     }
 }
 
@@ -822,16 +832,31 @@ extern "C" int om_route_softmax_topk_bwd(const void *logits, int logits_dtype, c
     hipStream_t st = om_stream(stream);
     const unsigned nb = token_blocks(T);
 #define OM_RB(TL, TW)                                                                          \
-    OM_DISPATCH_PER(N, (softmax_topk_bwd_kernel<PER, TL, TW><<<nb, 256, 0, st>>>(              \
+    OM_DISPATCH_PER(N, (softmax_topk_bwd_kernel<PER, TL, TW, TL><<<nb, 256, 0, st>>>(          \
                            static_cast<const TL *>(logits), experts,                           \
                            static_cast<const TW *>(dweights), T, N, K, norm_topk_prob,         \
-                           static_cast<TL *>(dlogits))))
+                           static_cast<TL *>(dlogits), nullptr, nullptr, 0)))
     if (logits_dtype == OM_F32 && weights_dtype == OM_F32) { OM_RB(float, float); }
     else if (logits_dtype == OM_F32) { OM_RB(float, uint16_t); }
     else if (weights_dtype == OM_F32) { OM_RB(uint16_t, float); }
     else { OM_RB(uint16_t, uint16_t); }
 #undef OM_RB
     return om_launch_status();
+}
+
+// (up to 64 experts)
+void om_launch_softmax_bwd(const void *logits, int logits_dtype, const int64_t *experts, const void *dweights, int dweights_dtype,
+                           const void *more, int64_t T, int N, int K, int renorm, float *dlogits, unsigned *zero, int n_zero,
+                           hipStream_t stream) {
+#define OM_RB(TL, TW)                                                                                                               \
+    softmax_topk_bwd_kernel<1, TL, TW, float><<<token_blocks(T), 256, 0, stream>>>(static_cast<const TL *>(logits), experts,            \
+                                                                                  static_cast<const TW *>(dweights), T, N, K, renorm, \
+                                                                                  dlogits, static_cast<const TL *>(more), zero, n_zero)
+    if (logits_dtype == OM_F32 && dweights_dtype == OM_F32) OM_RB(float, float);
+    else if (logits_dtype == OM_F32) OM_RB(float, uint16_t);
+    else if (dweights_dtype == OM_F32) OM_RB(uint16_t, float);
+    else OM_RB(uint16_t, uint16_t);
+#undef OM_RB
 }
 
 extern "C" int om_route_sigmoid_group_topk(const float *logits, const float *bias, int64_t T, int N,

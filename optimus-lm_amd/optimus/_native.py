@@ -134,6 +134,9 @@ SIGNATURES = {
     "om_grouped_gemm_wgrad_gathered_out_accumulate": (c_int, [c_void_p, c_void_p, c_i64, c_void_p, c_void_p,
                                                               c_void_p, c_i64, c_int, c_int, c_int, c_i64,
                                                               c_void_p]),
+    "om_router_softmax_bwd_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
+    "om_router_softmax_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int] + [c_void_p] * 4 +
+                              [c_int, c_i64, c_int, c_int, c_int, c_int, c_void_p, c_i64, c_void_p]),
     "om_moe_row_weights": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int,
                                    c_void_p]),
     "om_merged_mlp_gate_up_fwd_weighted": (c_int, [c_void_p, c_void_p, c_i64, c_void_p, c_void_p, c_void_p,
@@ -204,7 +207,7 @@ _UNTIMED = {"om_version", "om_arch", "om_strerror", "om_moe_sort_workspace_bytes
             "om_moe_sort_static_capacity_bytes",
             "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes",
             "om_router_gate_wgrad_workspace_bytes", "om_router_gate_route_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
-            "om_merged_mlp_row_dot_parts", "om_grad_norm_fits"}
+            "om_merged_mlp_row_dot_parts", "om_router_softmax_bwd_workspace_bytes", "om_grad_norm_fits"}
 
 
 class NativeLibraryError(RuntimeError):

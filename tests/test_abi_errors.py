@@ -179,6 +179,20 @@ def test_grouped_gemms(lib):
     assert lib.om_grouped_gemm_wgrad_gathered(P, P, P, 16384, ODD, P, *g) == ALIGN
 
 
+def test_router_backward_in_one_call(lib):
+    need = lib.om_router_softmax_bwd_workspace_bytes(2048, 256, 8)
+    assert need > 0
+    for T, H, N in ((0, 256, 8), (64, 12, 8), (64, 256, 65)):
+        assert lib.om_router_softmax_bwd_workspace_bytes(T, H, N) == SHAPE
+    f = lib.om_router_softmax_bwd
+    tail = (2048, 256, 8, 2, 1)
+    assert f(P, P, P, F32, P, P, BF16, None, None, P, P, BF16, 2048, 256, 8, 9, 1, P, 1 << 30, None) == SHAPE
+    assert f(P, P, P, 7, P, P, BF16, None, None, P, P, BF16, *tail, P, 1 << 30, None) == DTYPE
+    assert f(P, P, P, F32, None, P, BF16, None, None, P, P, BF16, *tail, P, 1 << 30, None) == NULL
+    assert f(P, P, P, F32, P, P, BF16, None, ODD, P, P, BF16, *tail, P, 1 << 30, None) == ALIGN
+    assert f(P, P, P, F32, P, P, BF16, None, None, P, P, BF16, *tail, P, need - 1, None) == WORKSPACE
+
+
 def test_routing_weight_folded_into_the_expert_mlp(lib):
     g = (131072, 64, 1024, 2048, 0, None)
     assert lib.om_moe_row_weights(P, P, P, P, P, 131072, 8, 7, None) == DTYPE

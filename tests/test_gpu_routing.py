@@ -569,3 +569,52 @@ def test_gate_of_many_experts(cuda, T, H, N, base):
     bound = (T / 16 + 300) * 2.0 ** -24 * (d16.abs().t() @ x.double().abs()) + 1e-30
     assert bool(((dw[:N].double() - d16.t() @ x.double()).abs() <= bound).all())
     assert bool((dw[N] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,H,N,K,renorm,ldt,wdt", [
+    (1, 8, 1, 1, False, torch.float32, torch.bfloat16), (127, 136, 8, 2, True, torch.float32, torch.bfloat16),
+    (2048, 256, 8, 2, True, torch.float32, torch.bfloat16), (512, 2048, 64, 8, False, torch.float32, torch.bfloat16),
+    (129, 264, 12, 12, True, torch.float32, torch.float32), (65, 1000, 33, 9, False, torch.float32, torch.bfloat16),
+    (300, 512, 64, 20, True, torch.bfloat16, torch.bfloat16), (9000, 2048, 64, 8, False, torch.float32, torch.bfloat16), (3001, 1000, 13, 3, False, torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("extra", [False, True])
+def test_softmax_router_backward_in_one_call(cuda, T, H, N, K, renorm, ldt, wdt, extra):
+    """The bits of the separate calls, whether the token ranges are added in the launch or behind it; a workspace of any content."""
+    from optimus import _native as n
+    lib = n.lib()
+    g = torch.Generator().manual_seed(T + H + N)
+    x, w = _gate_inputs(T, H, N, seed=T)
+    logits = (x.float() @ w.float().t()).to(ldt)
+    experts = torch.topk(torch.softmax(logits.float(), 1), K, dim=1).indices
+    d = lambda t: None if t is None else t.to(cuda).contiguous()
+    xg, wg, lg, eg, dg = map(d, (x, w, logits, experts, torch.randn(T, K, generator=g).to(wdt)))
+    more = d((torch.randn(T, N, generator=g) * 0.1).to(ldt)) if extra else None
+    base = d(torch.randn(T, H, generator=g).to(torch.bfloat16)) if extra else None
+    st = n.stream()
+    dl = torch.empty_like(lg)
+    n.check(lib.om_route_softmax_topk_bwd(n.ptr(lg), n.dtype_code(lg), n.ptr(eg), n.ptr(dg), n.dtype_code(dg), T, N, K, int(renorm), n.ptr(dl), st), "softmax")
+    dl = (dl if more is None else dl + more).float()
+    for dw_dtype in (torch.bfloat16, torch.float32):
+        want_dx, want_dw, dx, dw = torch.empty_like(xg), torch.empty_like(wg, dtype=dw_dtype), torch.empty_like(xg), torch.empty_like(wg, dtype=dw_dtype)
+        ws = torch.empty(max(lib.om_router_gate_wgrad_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+        n.check(lib.om_router_gate_dgrad(n.ptr(dl), n.ptr(wg), n.ptr(base), n.ptr(want_dx), T, H, N, st), "dgrad")
+        n.check(lib.om_router_gate_wgrad(n.ptr(xg), n.ptr(dl), T, H, N, n.ptr(want_dw), n.dtype_code(want_dw), n.ptr(ws), ws.numel(), st), "wgrad")
+        ws = torch.full((lib.om_router_softmax_bwd_workspace_bytes(T, H, N),), 255, dtype=torch.uint8, device=cuda)
+        for _ in range(2):
+            n.check(lib.om_router_softmax_bwd(n.ptr(xg), n.ptr(wg), n.ptr(lg), n.dtype_code(lg), n.ptr(eg), n.ptr(dg), n.dtype_code(dg), n.ptr(more),
+                                              n.ptr(base), n.ptr(dx), n.ptr(dw), n.dtype_code(dw), T, H, N, K, int(renorm), n.ptr(ws), ws.numel(), st),
+                    "om_router_softmax_bwd")
+        assert torch.equal(dx, want_dx) and torch.equal(dw, want_dw)
+
+
+def test_softmax_router_backward_keeps_what_is_not_finite(cuda):
+    """A token whose logits hold NaN or +inf has NaN gradients, as in the separate kernels, and the others are untouched."""
+    from optimus.models.common.moe import GateSoftmaxTopkFunction
+    T, H, N, K = 130, 512, 64, 4
+    x, w = _gate_inputs(T, H, N, seed=8)
+    x[3, 5] = float("nan")
+    x[77, 1] = float("inf")
+    xg, wg = x.to(cuda).requires_grad_(True), w.to(cuda).requires_grad_(True)
+    weights, _, _, _ = GateSoftmaxTopkFunction.apply(xg, wg, K, False, torch.float32)
+    weights.sum().backward()
+    bad = torch.isnan(xg.grad).all(1).cpu()
+    assert bad[3] and bad[77] and int(torch.isnan(xg.grad).any(1).sum()) == 2 and torch.isnan(wg.grad).any()
