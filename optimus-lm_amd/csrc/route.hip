@@ -5,6 +5,9 @@
 // depend on lane scheduling.  Scores live in registers, expert i = lane + 64*j.
 #include "common.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace {
 
 #pragma clang fp contract(off)
@@ -626,6 +629,136 @@ __global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint1
     }
 }
 
+// Projection and routing of up to 64 experts in one launch, 16 tokens at a time, for gates of a small weight: what bounds those is a chain of
+// waits and launches.  So a block has eight wavefronts for every 32 experts, each with a slice of H or two, and a wavefront asks for
+// 128 columns at a time before it waits: straight into the fragments of v_mfma_f32_16x16x32_bf16, a weight is used by one wavefront only.
+// Slices of 64 columns (WHOLE): the weight stays in registers for the block's further tokens, whose x is on its way while the last
+// ones are routed (hidden 256: 64 experts, 2048 tokens 9.4 -> 7.6 us, 16384 20.2 -> 16.8).  The slices are added in their order: the sums, and so
+// the logits, are those of the split projection, bit for bit.
+constexpr int ROWS_TOKENS = 16;
+
+// CH: pieces of 32 columns that are loaded at once; SL: slices at most; WHOLE: a wavefront has at most one slice, of CH pieces.
+template <int NH, int CH, int SL, bool WHOLE, typename TL, typename TW>
+__global__ __launch_bounds__(NH * 512) void gate_route_rows_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ wg, int64_t Tn, int H,
+                                                                   int N, int K, int renorm, int slices, int slice_len,
+                                                                   TL *__restrict__ logits_out, TW *__restrict__ weights_out,
+                                                                   int64_t *__restrict__ experts_out) {
+    constexpr int NP = NH * 32, LD = NP + 4, Q = NP / 16, BUFS = SL > 8 ? 1 : 2;
+    __shared__ __attribute__((aligned(16))) float part[BUFS][SL][ROWS_TOKENS][LD];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int half = wave % NH, first_slice = wave / NH;
+    const int l16 = lane & 15, g = lane >> 4;
+    uint32_t w_row[2];                                      // bytes; rows past the last expert: it again, results unused
+#pragma unroll
+    for (int m = 0; m < 2; m++) w_row[m] = static_cast<uint32_t>(min(half * 32 + m * 16 + l16, N - 1)) * static_cast<uint32_t>(H) * 2;
+    u32x4 wf[CH][2], xf[CH];
+    auto at = [](const uint16_t *base, uint32_t bytes) { return *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(base) + bytes); };
+    // byte of the lane's chunk in piece i of CH that `columns` are left of: past them the last chunk again, of tokens zeros
+    auto chunk = [&](int i, int columns) { return static_cast<uint32_t>(WHOLE ? i * 32 + g * 8 : min(i * 32 + g * 8, columns - 8)) * 2; };
+    auto load_w = [&](int begin, int columns) {
+#pragma unroll
+        for (int i = 0; i < CH; i++)
+#pragma unroll
+            for (int m = 0; m < 2; m++) wf[i][m] = at(wg + begin, w_row[m] + chunk(i, columns));
+    };
+    auto load_x = [&](int64_t tile, int begin, int columns) {
+        const uint32_t row = static_cast<uint32_t>(min(static_cast<int64_t>(l16), Tn - 1 - tile * ROWS_TOKENS)) * static_cast<uint32_t>(H) * 2;
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            xf[i] = at(x + tile * ROWS_TOKENS * H + begin, row + chunk(i, columns));
+            if (!WHOLE && i * 32 + g * 8 >= columns) xf[i] = u32x4{0, 0, 0, 0};
+        }
+    };
+    const int64_t tiles = (Tn + ROWS_TOKENS - 1) / ROWS_TOKENS;
+    const bool mine = first_slice < slices;
+    if (WHOLE && mine) {
+        load_w(first_slice * slice_len, 0);
+        load_x(blockIdx.x, first_slice * slice_len, 0);
+    }
+    int buf = 0;
+    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        for (int s = first_slice; s < slices; s += 8) {
+            f32x4 acc[2] = {};
+            const int begin = s * slice_len, len = min(H - begin, slice_len);
+            for (int c = 0; c < (WHOLE ? 1 : len); c += CH * 32) {
+                if (!WHOLE) {
+                    load_w(begin + c, len - c);
+                    load_x(tile, begin + c, len - c);
+                }
+#pragma unroll
+                for (int i = 0; i < CH; i++)
+#pragma unroll
+                    for (int m = 0; m < 2; m++)
+                        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i][m]), __builtin_bit_cast(bf16x8, xf[i]), acc[m], 0, 0, 0);
+            }
+            // element r of lane l: expert 4 * (l / 16) + r of token l % 16
+#pragma unroll
+            for (int m = 0; m < 2; m++) *reinterpret_cast<f32x4 *>(&part[buf][s][l16][half * 32 + m * 16 + g * 4]) = acc[m];
+            if (WHOLE) break;
+        }
+        // (with two buffers the wavefronts that route a tile are at the next tile's barrier before theirs is written again)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (wave < ROWS_TOKENS / 4) {                       // a row of 16 lanes per token
+            const int tk = wave * 4 + g;
+            const int64_t t = tile * ROWS_TOKENS + tk;
+            float p[Q];
+#pragma unroll
+            for (int j = 0; j < Q; j++) p[j] = part[buf][0][tk][l16 + 16 * j];
+#pragma unroll 2
+            for (int s = 1; s < slices; s++)
+#pragma unroll
+                for (int j = 0; j < Q; j++) p[j] += part[buf][s][tk][l16 + 16 * j];
+            const bool there = t < Tn;
+#pragma unroll
+            for (int j = 0; j < Q; j++) {
+                const int n = l16 + 16 * j;
+                if (logits_out && there && n < N) Elem<TL>::store(logits_out + t * N + n, p[j]);
+                if (sizeof(TL) == 2) p[j] = bf16_bits_to_f32(f32_to_bf16_bits(p[j]));
+                if (n >= N) p[j] = -INFINITY;
+            }
+            float w; int e;
+            row_softmax_topk<Q>(p, N, K, l16, w, e);
+            if (renorm) w = w / row_sum(l16 < K ? w : 0.0f);
+            if (there && l16 < K) {
+                Elem<TW>::store(weights_out + t * K + l16, w);
+                experts_out[t * K + l16] = e;
+            }
+        }
+        // (the wavefronts that route ask later than the others: beside the weight they have no registers for both)
+        if (WHOLE && mine && tile + gridDim.x < tiles) load_x(tile + gridDim.x, first_slice * slice_len, 0);
+        if (BUFS == 2) buf ^= 1;
+        else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+}
+
+// Hidden sizes that gate_route_slices_kernel does not take, up to 64 K weights: a block takes in all of them, from memory behind a layer's
+// expert products.  Two launches -> one, us, the router alone: 8 experts, hidden 256, 2048 tokens 9.6 -> 6.2, 16384 16.2 -> 9.6; 12 of 1000, 3001
+// 10.9 -> 7.1, 16000 21.2 -> 18.0; 64 of 256, 2048 13.9 -> 7.6; 40 of 776, 512 12.1 -> 10.7, 4096 15.5 -> 9.2; 61 of 1000, 512 13.2 -> 13.0, 4096
+// 20.8 -> 10.9, 16384 32.4 -> 31.4; but 12 of 4040, 9000 27.2 -> 29.6, 60 of 3000, 9000 34.4 -> 46.5, 64 of 6000, 9000 48.8 -> 84.9.  Hidden sizes that are multiples of
+// 512 as fast here as by slices, or up to 15 % slower; with 64 experts of 2048 in a layer, 512 tokens 15.6 against 13.9 in two launches.
+inline bool gate_rows_fit(int64_t T, int H, int N, int K) {
+    return N <= 64 && K <= 16 && H % 512 != 0 && N * H <= (64 << 10) && om_gate_route_splits(T, H, N) <= 16;
+}
+
+template <typename TL, typename TW>
+int launch_gate_rows(const void *x, const void *wg, int64_t T, int H, int N, int K, int renorm, void *logits_out, void *weights_out,
+                     int64_t *experts_out, hipStream_t st) {
+    const int slices = om_gate_route_splits(T, H, N), slice_len = ((H + 63) / 64 + slices - 1) / slices * 64;
+    const dim3 grid(static_cast<unsigned>(std::min<int64_t>((T + ROWS_TOKENS - 1) / ROWS_TOKENS, 256)));
+    const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(wg);
+    TL *lo = static_cast<TL *>(logits_out);
+    TW *wo = static_cast<TW *>(weights_out);
+#define OM_ROWS(NH, CH, SL, WHOLE)                                                                                                        \
+    gate_route_rows_kernel<NH, CH, SL, WHOLE, TL, TW><<<grid, NH * 512, 0, st>>>(xp, wp, T, H, N, K, renorm, slices, slice_len, lo, wo, experts_out)
+    const bool whole = slices <= 8 && slice_len == 64 && slices * 64 == H;
+    if (N <= 32 && whole) OM_ROWS(1, 2, 8, true);
+    else if (N <= 32) OM_ROWS(1, 4, 16, false);
+    else if (whole) OM_ROWS(2, 2, 8, true);
+    else OM_ROWS(2, 4, 16, false);
+#undef OM_ROWS
+    return om_launch_status();
+}
+
 // shapes of gate_route_slices_kernel
 inline bool gate_slices_fit(int H, int N) { return N <= 64 && H % 512 == 0; }
 
@@ -953,6 +1086,12 @@ extern "C" int om_router_gate_split_softmax_topk(const void *x, const void *gate
     // selections, hidden 2048: 600 24.8 -> 13.0, 8192 28.0 -> 27.4, 12000 53.2 -> 38.9; hidden 512, 40 of 62: 4 tokens 10.1 -> 12.4, 20 of
     // 40: 52 tokens 15.4 -> 9.5.
     const bool one_launch = K <= 16 ? T > 512 || H < 1024 : H < 1024 && T <= 16 ? true : N > 32 && (T - 1) % 8192 >= 6144;
+    if (gate_rows_fit(T, H, N, K)) {
+#define OM_GR(TL, TW) launch_gate_rows<TL, TW>(x, gate_weight, T, H, N, K, norm_topk_prob, logits_out, weights_out, experts_out, st)
+        if (logits_dtype == OM_F32) return weights_dtype == OM_F32 ? OM_GR(float, float) : OM_GR(float, uint16_t);
+        return weights_dtype == OM_F32 ? OM_GR(uint16_t, float) : OM_GR(uint16_t, uint16_t);
+#undef OM_GR
+    }
     if (gate_slices_fit(H, N) && one_launch) {
 #define OM_GS(TL, TW) \
     launch_gate_slices<TL, TW, true>(x, gate_weight, T, H, N, K, norm_topk_prob, logits_out, weights_out, experts_out, st)

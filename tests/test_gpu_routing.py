@@ -618,3 +618,26 @@ def test_softmax_router_backward_keeps_what_is_not_finite(cuda):
     weights.sum().backward()
     bad = torch.isnan(xg.grad).all(1).cpu()
     assert bad[3] and bad[77] and int(torch.isnan(xg.grad).any(1).sum()) == 2 and torch.isnan(wg.grad).any()
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 8, 1, 1), (15, 64, 64, 16), (17, 72, 33, 8), (16, 256, 32, 16), (2049, 256, 8, 2), (4113, 256, 64, 8),
+                                     (33, 264, 31, 5), (300, 1000, 12, 3), (4097, 1000, 61, 16), (2000, 1096, 59, 4), (64, 2040, 32, 8), (5000, 5000, 13, 6)])
+@pytest.mark.parametrize("bf16_logits", [False, True])
+def test_small_gate_router_in_one_launch(cuda, T, H, N, K, bf16_logits):
+    """Bit for bit the split projection and the routing of its logits: partial groups of tokens and experts, slices and pieces that end early."""
+    from optimus import _native as n
+    lib, st = n.lib(), n.stream()
+    x, w = (t.to(cuda) for t in _gate_inputs(T, H, N, seed=T + H))
+    ldt = torch.bfloat16 if bf16_logits else torch.float32
+    ref = torch.empty(T, N, device=cuda)
+    ws = torch.empty(max(lib.om_router_gate_logits_split_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+    n.check(lib.om_router_gate_logits_split(n.ptr(x), n.ptr(w), T, H, N, n.ptr(ref), n.ptr(ws), ws.numel(), st), "logits")
+    ref = ref.to(ldt)
+    for renorm in (0, 1):
+        want_w, want_e = torch.empty(T, K, dtype=torch.bfloat16, device=cuda), torch.empty(T, K, dtype=torch.int64, device=cuda)
+        n.check(lib.om_route_softmax_topk(n.ptr(ref), n.dtype_code(ref), T, N, K, renorm, n.ptr(want_w), n.dtype_code(want_w), n.ptr(want_e), st), "route")
+        logits, got_w, got_e = torch.empty_like(ref), torch.empty_like(want_w), torch.empty_like(want_e)
+        ws = torch.empty(max(lib.om_router_gate_route_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+        n.check(lib.om_router_gate_split_softmax_topk(n.ptr(x), n.ptr(w), T, H, N, K, renorm, n.ptr(logits), n.dtype_code(logits), n.ptr(got_w),
+                                                      n.dtype_code(got_w), n.ptr(got_e), n.ptr(ws), ws.numel(), st), "one launch")
+        assert torch.equal(logits, ref) and torch.equal(got_e, want_e) and torch.equal(got_w, want_w)
