@@ -197,6 +197,12 @@ int om_router_gate_split_sigmoid_group_topk(const void *x, const void *gate_weig
                                             int N, int n_group, int topk_group, int K, int norm_topk_prob,
                                             double routed_scaling_factor, float *logits_out, int64_t *experts_out,
                                             float *weights_out, void *workspace, int64_t workspace_bytes, void *stream);
+/* The same with the bias in bias_dtype (OM_F32 / OM_BF16; a module cast to bf16 casts its buffers too). */
+int om_router_gate_split_sigmoid_group_topk_bias(const void *x, const void *gate_weight, const void *bias, int bias_dtype,
+                                                 int64_t T, int H, int N, int n_group, int topk_group, int K,
+                                                 int norm_topk_prob, double routed_scaling_factor, float *logits_out,
+                                                 int64_t *experts_out, float *weights_out, void *workspace,
+                                                 int64_t workspace_bytes, void *stream);
 
 /* om_router_gate_wgrad: gradient of the gate's weight,
  *   dweight[n,h] = sum_t dlogits[t,n] * x[t,h]

@@ -1058,7 +1058,8 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
     refuse_transforms({x, weight, bias});
     require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0);
-    TORCH_CHECK_TYPE(bias.scalar_type() == at::kFloat, "router bias must be float32 (got ", bias.scalar_type(), ")");
+    TORCH_CHECK_TYPE(bias.scalar_type() == at::kFloat || bias.scalar_type() == at::kBFloat16,
+                     "router bias must be float32 or bfloat16 (got ", bias.scalar_type(), ")");
     if (bias.numel() != N) throw NativeError("router bias: expected one value per expert");
     Tensor logits, weights, experts;
     {
@@ -1071,13 +1072,14 @@ std::tuple<Tensor, Tensor, Tensor> route_sigmoid(const Tensor &x, const Tensor &
         experts = make({T, top_k}, x, at::kLong);
         if (x.scalar_type() == at::kFloat) {
             logits = gate_logits_forward(c, x, weight);
-            OM(c, om_route_sigmoid_group_topk, fp(logits), fp(bias), T, N, n_group, topk_group, top_k, renorm, scale,
+            const Tensor bias_f32 = bias.to(at::kFloat);
+            OM(c, om_route_sigmoid_group_topk, fp(logits), fp(bias_f32), T, N, n_group, topk_group, top_k, renorm, scale,
                experts.data_ptr<int64_t>(), fpm(weights), c.stream);
         } else {
             require_gate_shape(weight, "gate projection");
             logits = make({T, N}, x, at::kFloat);
             const Tensor ws = route_workspace(x, T, x.size(1), N);
-            OM(c, om_router_gate_split_sigmoid_group_topk, ptr(x), ptr(weight), fp(bias), T, x.size(1), N, n_group, topk_group,
+            OM(c, om_router_gate_split_sigmoid_group_topk_bias, ptr(x), ptr(weight), ptr(bias), dtype_code(bias), T, x.size(1), N, n_group, topk_group,
                top_k, renorm, scale, fpm(logits), experts.data_ptr<int64_t>(), fpm(weights), ptr(ws), ws.numel(), c.stream);
         }
     }

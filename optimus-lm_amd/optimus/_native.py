@@ -54,6 +54,8 @@ SIGNATURES = {
     "om_router_gate_route_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
     "om_router_gate_split_softmax_topk": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                                   c_void_p, c_int, c_void_p, c_void_p, c_i64, c_void_p]),
+    "om_router_gate_split_sigmoid_group_topk_bias": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_i64] + [c_int] * 6 +
+                                                     [c_double] + [c_void_p] * 4 + [c_i64, c_void_p]),
     "om_router_gate_split_sigmoid_group_topk": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int,
                                                         c_int, c_int, c_double, c_void_p, c_void_p, c_void_p, c_void_p,
                                                         c_i64, c_void_p]),

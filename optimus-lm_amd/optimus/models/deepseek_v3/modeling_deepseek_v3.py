@@ -114,8 +114,11 @@ class DeepseekV3ParallelTopkRouter(nn.Module):
         if hidden_states.dtype != self.weight.dtype or hidden_states.dtype not in (torch.bfloat16, torch.float32):
             raise TypeError(f"router gate: activations and weight must both be bfloat16 or both float32 "
                             f"(got {hidden_states.dtype}, {self.weight.dtype})")
+        bias = self.e_score_correction_bias
+        if bias.dtype != torch.bfloat16:     # (the kernels widen bfloat16 themselves)
+            bias = bias.float()
         return _n.host().route_sigmoid(
-            hidden_states.contiguous(), self.weight.contiguous(), self.e_score_correction_bias.float().contiguous(),
+            hidden_states.contiguous(), self.weight.contiguous(), bias.contiguous(),
             self.n_group, self.topk_group, self.top_k, bool(self.norm_topk_prob), float(self.routed_scaling_factor))
 
 

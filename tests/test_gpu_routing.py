@@ -641,3 +641,29 @@ def test_small_gate_router_in_one_launch(cuda, T, H, N, K, bf16_logits):
         n.check(lib.om_router_gate_split_softmax_topk(n.ptr(x), n.ptr(w), T, H, N, K, renorm, n.ptr(logits), n.dtype_code(logits), n.ptr(got_w),
                                                       n.dtype_code(got_w), n.ptr(got_e), n.ptr(ws), ws.numel(), st), "one launch")
         assert torch.equal(logits, ref) and torch.equal(got_e, want_e) and torch.equal(got_w, want_w)
+
+
+@pytest.mark.parametrize("T,H,N,n_group,topk_group,K", [(1, 7168, 256, 8, 4, 8), (64, 7168, 256, 8, 4, 8), (1025, 512, 256, 1, 1, 12), (300, 264, 16, 4, 2, 2),
+                                                        (77, 512, 64, 8, 3, 6), (500, 72, 24, 3, 1, 8), (40, 512, 96, 8, 3, 5), (2000, 1000, 128, 32, 9, 16)])
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("ties", [False, True])
+def test_group_router_behind_the_split_projection(cuda, T, H, N, n_group, topk_group, K, bias_dtype, ties):
+    """Bit for bit the router on the logits that it writes, also where experts and groups tie."""
+    from optimus import _native as n
+    lib, st = n.lib(), n.stream()
+    x, w = _gate_inputs(T, H, N, seed=T + N)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2)).mul(0.1).to(bias_dtype)
+    if ties:
+        w, bias = w[: max(N // n_group // 2, 1)].repeat(2 * n_group, 1)[:N], torch.zeros(N, dtype=bias_dtype)
+    xg, wg, bg = x.to(cuda), w.to(cuda).contiguous(), bias.to(cuda)
+    logits = torch.empty(T, N, device=cuda)
+    got_e, got_w = torch.empty(T, K, dtype=torch.int64, device=cuda), torch.empty(T, K, device=cuda)
+    ws = torch.empty(max(lib.om_router_gate_route_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+    for renorm in (0, 1):
+        n.check(lib.om_router_gate_split_sigmoid_group_topk_bias(n.ptr(xg), n.ptr(wg), n.ptr(bg), n.dtype_code(bg), T, H, N, n_group, topk_group, K,
+                                                                 renorm, 2.5, n.ptr(logits), n.ptr(got_e), n.ptr(got_w), n.ptr(ws), ws.numel(), st), "fused")
+        bf, want_e, want_w = bg.float(), torch.empty_like(got_e), torch.empty_like(got_w)
+        n.check(lib.om_route_sigmoid_group_topk(n.ptr(logits), n.ptr(bf), T, N, n_group, topk_group, K, renorm, 2.5, n.ptr(want_e), n.ptr(want_w), st), "router")
+        assert torch.equal(got_e, want_e) and torch.equal(got_w, want_w)
+    ref = x.double() @ w.double().t()
+    assert bool(((logits.cpu().double() - ref).abs() <= 8 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30).all())
