@@ -246,6 +246,12 @@ int om_router_gate_dgrad_f32_add(const float *dlogits, const float *gate_weight,
                                  int H, int N, float *dx, void *stream);
 int om_router_gate_wgrad_f32(const float *x, const float *dlogits, int64_t T, int H, int N,
                              float *dweight, void *stream);
+/* The two gradients in one launch, T >= 1 (base [T,H] may be null); and the projection with the softmax router behind it
+ * (om_route_softmax_topk on its logits, same bits) in one launch, N <= 64. */
+int om_router_gate_bwd_f32(const float *x, const float *dlogits, const float *gate_weight, const float *base, int64_t T, int H,
+                           int N, float *dx, float *dweight, void *stream);
+int om_router_gate_softmax_topk_f32(const float *x, const float *gate_weight, int64_t T, int H, int N, int K, int norm_topk_prob,
+                                    float *logits_out, void *weights_out, int weights_dtype, int64_t *experts_out, void *stream);
 
 /* om_router_gate_dgrad: gradient of the gate's input,
  *   dx[t,h] = (base[t,h] +) sum_n bf16(dlogits[t,n]) * gate_weight[n,h]

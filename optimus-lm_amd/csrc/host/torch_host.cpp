@@ -857,9 +857,15 @@ std::pair<Tensor, Tensor> gate_backward(const Call &c, const Tensor &x, const Te
     Tensor dx, dw;
     if (x.scalar_type() == at::kFloat) {
         const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
+        const Tensor base = other_grad.defined() ? other_grad.contiguous() : Tensor();
+        if (need_x && need_w && T > 0) {
+            dx = make(x.sizes(), x);
+            dw = make(weight.sizes(), weight);
+            OM(c, om_router_gate_bwd_f32, fp(x), fp(dlogits), fp(weight), fp(base), T, H, N, fpm(dx), fpm(dw), c.stream);
+            return {dx, dw};
+        }
         if (need_x) {
             dx = make(x.sizes(), x);
-            const Tensor base = other_grad.defined() ? other_grad.contiguous() : Tensor();
             OM(c, om_router_gate_dgrad_f32_add, fp(dlogits), fp(weight), fp(base), T, H, N, fpm(dx), c.stream);
         }
         if (need_w) {
@@ -1024,7 +1030,11 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
         require_device(weight);
         weights = make({T, top_k}, x, out_dtype);
         experts = make({T, top_k}, x, at::kLong);
-        if (x.scalar_type() == at::kFloat) {
+        if (x.scalar_type() == at::kFloat && N <= 64) {
+            logits = make({T, N}, x, at::kFloat);
+            OM(c, om_router_gate_softmax_topk_f32, fp(x), fp(weight), T, H, N, top_k, renorm, fpm(logits), ptr(weights),
+               dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);
+        } else if (x.scalar_type() == at::kFloat) {
             logits = gate_logits_forward(c, x, weight);
             OM(c, om_route_softmax_topk, ptr(logits), dtype_code(logits), T, N, top_k, renorm, ptr(weights),
                dtype_code(weights), experts.data_ptr<int64_t>(), c.stream);

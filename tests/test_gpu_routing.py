@@ -667,3 +667,29 @@ def test_group_router_behind_the_split_projection(cuda, T, H, N, n_group, topk_g
         assert torch.equal(got_e, want_e) and torch.equal(got_w, want_w)
     ref = x.double() @ w.double().t()
     assert bool(((logits.cpu().double() - ref).abs() <= 8 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 1e-30).all())
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 7, 1, 1), (5, 64, 8, 2), (2048, 256, 8, 2), (777, 100, 13, 13), (513, 520, 64, 9), (3, 1000, 33, 4)])
+def test_float32_router_launches_equal_their_steps(cuda, T, H, N, K):
+    """Projection with routing, and both gradients of the gate, in one launch: the bits of the separate calls."""
+    from optimus import _native as n
+    lib, st = n.lib(), n.stream()
+    g = torch.Generator().manual_seed(T + H + N)
+    x, w, dl, base = (torch.randn(*s, generator=g).to(cuda) for s in ((T, H), (N, H), (T, N), (T, H)))
+    new = lambda *s: torch.empty(*s, device=cuda)
+    logits, got_logits = new(T, N), new(T, N)
+    n.check(lib.om_router_gate_logits_f32(n.ptr(x), n.ptr(w), T, H, N, n.ptr(logits), st), "logits")
+    for wdt in (torch.float32, torch.bfloat16):
+        want_w, got_w = new(T, K).to(wdt), new(T, K).to(wdt)
+        want_e, got_e = (torch.empty(T, K, dtype=torch.int64, device=cuda) for _ in range(2))
+        for renorm in (0, 1):
+            n.check(lib.om_route_softmax_topk(n.ptr(logits), n.OM_F32, T, N, K, renorm, n.ptr(want_w), n.dtype_code(want_w), n.ptr(want_e), st), "route")
+            n.check(lib.om_router_gate_softmax_topk_f32(n.ptr(x), n.ptr(w), T, H, N, K, renorm, n.ptr(got_logits), n.ptr(got_w),
+                                                        n.dtype_code(got_w), n.ptr(got_e), st), "one launch")
+            assert torch.equal(got_logits, logits) and torch.equal(got_e, want_e) and torch.equal(got_w, want_w)
+    for b in (None, base):
+        want_dx, want_dw, dx, dw = new(T, H), new(N, H), new(T, H), new(N, H)
+        n.check(lib.om_router_gate_dgrad_f32_add(n.ptr(dl), n.ptr(w), n.ptr(b), T, H, N, n.ptr(want_dx), st), "dx")
+        n.check(lib.om_router_gate_wgrad_f32(n.ptr(x), n.ptr(dl), T, H, N, n.ptr(want_dw), st), "dw")
+        n.check(lib.om_router_gate_bwd_f32(n.ptr(x), n.ptr(dl), n.ptr(w), n.ptr(b), T, H, N, n.ptr(dx), n.ptr(dw), st), "both")
+        assert torch.equal(dx, want_dx) and torch.equal(dw, want_dw)
