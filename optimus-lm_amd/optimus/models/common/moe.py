@@ -32,12 +32,13 @@ _announced_switches = set()
 def note_unfused_path(what, why, instead="running the unfused sequence of kernels (same mathematics, bf16 "
                                             "roundings in other places)"):
     """Called where a block leaves a fused kernel path for the unfused sequence."""
+    if (what, why) in _announced_switches and not strict_fused_paths:
+        return
     message = f"{what}: {why}; {instead}"
     if strict_fused_paths:
         raise _n.NativeLibraryError(message + " [strict_fused_paths is set]")
-    if (what, why) not in _announced_switches:
-        _announced_switches.add((what, why))
-        warnings.warn(message, stacklevel=3)
+    _announced_switches.add((what, why))
+    warnings.warn(message, stacklevel=3)
 
 
 def get_tensor_list(tensor, cum_token_counts):
@@ -900,20 +901,17 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
                 router_logits, flat = gate_logits_with_passthrough(flat, self.gate)
             routing_weights, selected_experts = SoftmaxTopkRouterFunction.apply(
                 router_logits.contiguous(), self.num_experts_per_tok, self.norm_topk_prob, flat.dtype)
-        hidden_states = flat.view(batch_size, sequence_length, hidden_dim)
 
-        def expert_computation_block(hidden_states, selected_experts, routing_weights, residual=None):
-            b, s, h = hidden_states.shape
+        def expert_computation_block(flat, selected_experts, routing_weights, residual=None):
             gathered = self._gathered_experts_fn if self.fuse_input_gather else None
             fused = self._fused_experts_fn if (self.fuse_input_gather and self.fuse_routing_weights) else None
-            out = expert_computation(hidden_states.reshape(-1, h), routing_weights, selected_experts,
-                                     self.expert_start_idx, self.expert_end_idx, self._experts_fn,
-                                     self.num_experts, gathered_experts_fn=gathered,
-                                     residual=None if residual is None else residual.reshape(-1, h),
-                                     fused_experts_fn=fused)
-            return out.reshape(b, s, h)
+            return expert_computation(flat, routing_weights, selected_experts,
+                                      self.expert_start_idx, self.expert_end_idx, self._experts_fn,
+                                      self.num_experts, gathered_experts_fn=gathered,
+                                      residual=None if residual is None else residual.reshape(-1, hidden_dim),
+                                      fused_experts_fn=fused)
 
-        args = [hidden_states, selected_experts, routing_weights]
+        args = [flat, selected_experts, routing_weights]
         if residual is not None:
             args.append(residual)
         if self.use_activation_checkpointing_for_moe:
@@ -921,6 +919,7 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
                                                               use_reentrant=False)
         else:
             final_hidden_states = expert_computation_block(*args)
+        final_hidden_states = final_hidden_states.reshape(batch_size, sequence_length, hidden_dim)
 
         if self.output_router_logits:
             return final_hidden_states, router_logits

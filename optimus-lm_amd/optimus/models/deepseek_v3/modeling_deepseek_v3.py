@@ -202,24 +202,21 @@ class DeepseekV3ParallelMoE(nn.Module):
         # the experts are fed from the gate projection's pass-through of the hidden states, so that
         # their input gradient and the gate's are added inside one kernel
         topk_indices, topk_weights, flat = self.gate.forward_with_passthrough(hidden_states)
-        hidden_states = flat.view(hidden_states.shape)
+        orig_shape = hidden_states.shape
 
-        def expert_computation_block(hidden_states, topk_indices, topk_weights):
-            residuals = hidden_states
-            orig_shape = hidden_states.shape
-            flat = hidden_states.reshape(-1, hidden_states.shape[-1])
+        def expert_computation_block(flat, topk_indices, topk_weights):
             # routed + shared (reference :265): the shared experts' output goes into the combine
             # kernel as its residual, which rounds the routed sum first and then adds: the same two
             # roundings as `moe(...) + shared_experts(...)`
             if self._fuses_routing_weights() and self._routed_kernels_fit(flat, topk_weights):
-                return self.moe(flat, topk_indices, topk_weights, with_shared=True).view(*orig_shape)
-            shared = self.shared_experts(residuals).reshape(flat.shape)
-            return self.moe(flat, topk_indices, topk_weights, residual=shared).view(*orig_shape)
+                return self.moe(flat, topk_indices, topk_weights, with_shared=True)
+            shared = self.shared_experts(flat.view(orig_shape)).reshape(flat.shape)
+            return self.moe(flat, topk_indices, topk_weights, residual=shared)
 
-        args = [hidden_states, topk_indices, topk_weights]
+        args = [flat, topk_indices, topk_weights]
         if self.use_activation_checkpointing_for_moe:
-            return torch_activation_checkpoint(expert_computation_block, *args, use_reentrant=False)
-        return expert_computation_block(*args)
+            return torch_activation_checkpoint(expert_computation_block, *args, use_reentrant=False).view(orig_shape)
+        return expert_computation_block(*args).view(orig_shape)
 
     def set_parameters_from_full_module(self, module):
         self.gate.load_state_dict(module.gate.state_dict())

@@ -6,30 +6,47 @@ The reference marks events with a SYCL profiling tag on the XPU queue
 (pytorch_xpu_extensions/pcl.xpu.profiler/csrc/profiler/profile.dp.cpp:36-42); here an event is a
 HIP event recorded on PyTorch's current stream, so nothing synchronises until `summary()`.
 """
-from contextlib import contextmanager
+from contextlib import ContextDecorator
 
 import torch
 
 import optimus.globals
 
 
-@contextmanager
-def record_pcl_function(full_name, tag=None, exclude_from_trace=False, key="", ignore=False):
-    profiler = optimus.globals.profiler
-    if ignore or profiler is None:
-        yield
-        return
-    tokens = full_name.split("--")
-    names = ["--".join(tokens[0:i + 1]) for i in range(len(tokens))]
-    try:
-        for name in names:
-            if name not in profiler.timers:
-                profiler.register_timer(name, tag=tag, exclude_from_trace=exclude_from_trace)
-            profiler.start(name, key=key)
-        yield
-    finally:
-        for name in names:
-            profiler.stop(name)
+class record_pcl_function(ContextDecorator):
+    """record_pcl_function(full_name, tag, exclude_from_trace, key, ignore): the nested timers run inside the scope."""
+    __slots__ = ("args", "names")
+
+    def __init__(self, full_name, tag=None, exclude_from_trace=False, key="", ignore=False):
+        self.args = (full_name, tag, exclude_from_trace, key, ignore)
+        self.names = None
+
+    def _recreate_cm(self):
+        return type(self)(*self.args)      # (as a decorator: a scope of its own for every call)
+
+    def __enter__(self):
+        profiler = optimus.globals.profiler
+        if profiler is None or self.args[4]:
+            return
+        full_name, tag, exclude_from_trace, key, _ = self.args
+        tokens = full_name.split("--")
+        names = ["--".join(tokens[0:i + 1]) for i in range(len(tokens))]
+        self.names = (profiler, names)
+        try:
+            for name in names:
+                if name not in profiler.timers:
+                    profiler.register_timer(name, tag=tag, exclude_from_trace=exclude_from_trace)
+                profiler.start(name, key=key)
+        except BaseException:
+            self.__exit__(None, None, None)
+            raise
+
+    def __exit__(self, *exception):
+        if self.names is not None:
+            (profiler, names), self.names = self.names, None
+            for name in names:
+                profiler.stop(name)
+        return False
 
 
 class PclProfiler:
