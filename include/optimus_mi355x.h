@@ -197,7 +197,17 @@ int om_router_gate_split_sigmoid_group_topk(const void *x, const void *gate_weig
                                             int N, int n_group, int topk_group, int K, int norm_topk_prob,
                                             double routed_scaling_factor, float *logits_out, int64_t *experts_out,
                                             float *weights_out, void *workspace, int64_t workspace_bytes, void *stream);
-/* The same with the bias in bias_dtype (OM_F32 / OM_BF16; a module cast to bf16 casts its buffers too). */
+/* om_router_gate_softmax_topk_sort: om_router_gate_split_softmax_topk and om_moe_sort_weighted (row_weights may be null) on
+ * its selections, the routing and the sort in one launch; same bits.  For a few tokens: om_router_gate_softmax_topk_sort_fits
+ * returns 1 for the sizes that it takes (others: OM_ERR_SHAPE).  0 <= expert_start_idx < expert_end_idx <= N. */
+int om_router_gate_softmax_topk_sort_fits(int64_t T, int H, int N, int K);
+int om_router_gate_softmax_topk_sort(const void *x, const void *gate_weight, int64_t T, int H, int N, int K, int norm_topk_prob,
+                                     void *logits_out, int logits_dtype, void *weights_out, int weights_dtype,
+                                     int64_t *experts_out, int expert_start_idx, int expert_end_idx,
+                                     int32_t *cum_token_counts, int32_t *cum_expert_counts_ep, int32_t *input_indices,
+                                     int32_t *output_indices, int32_t *selected_experts_indices, float *row_weights,
+                                     void *workspace, int64_t workspace_bytes, void *stream);
+/* om_router_gate_split_sigmoid_group_topk with the bias in bias_dtype (OM_F32 / OM_BF16; a module cast to bf16 casts its buffers too). */
 int om_router_gate_split_sigmoid_group_topk_bias(const void *x, const void *gate_weight, const void *bias, int bias_dtype,
                                                  int64_t T, int H, int N, int n_group, int topk_group, int K,
                                                  int norm_topk_prob, double routed_scaling_factor, float *logits_out,

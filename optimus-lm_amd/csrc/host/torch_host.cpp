@@ -345,20 +345,28 @@ std::vector<Tensor> sort_tensors(const Call &c, const Tensor &experts, int64_t s
     return r;
 }
 
+// The one-buffer form for T tokens of K selections, its arrays in `buffer` or, where that is undefined, in a new one with
+// `more` words behind them.
+int64_t index_words(int64_t T, int64_t K, int64_t NR) { return NR + 1 + T + 1 + 4 * T * K; }
+Index one_buffer_index(int64_t T, int64_t K, int64_t NR, Tensor buffer, const Tensor &like = Tensor(), int64_t more = 0) {
+    Index ix;
+    ix.T = T;
+    ix.NR = NR;
+    ix.TK = ix.rows = T * K;
+    if (!buffer.defined()) buffer = at::empty({index_words(T, K, NR) + more}, like.options().dtype(at::kInt));
+    ix.owners = {std::move(buffer)};
+    ix.resolve();
+    return ix;
+}
+template <typename T> T *rwp(const T *p) { return const_cast<T *>(p); }
+
 Index sort_index(const Call &c, const Tensor &experts, int64_t start, int64_t end, const Tensor &rw) {
     require_device(experts);
     require_device(rw);
-    Index ix;
-    const int64_t K = experts.size(1);
-    ix.T = experts.size(0);
-    ix.NR = end - start;
-    ix.TK = ix.rows = ix.T * K;
-    const int64_t ws_bytes = om_moe_sort_workspace_bytes(ix.T, K, ix.NR);
-    const int64_t ws_at = ix.NR + 1 + ix.T + 1 + 4 * ix.TK;
-    ix.owners = {at::empty({ws_at + std::max<int64_t>(ws_bytes / 4, 1)}, experts.options().dtype(at::kInt))};
-    ix.resolve();
+    const int64_t K = experts.size(1), T = experts.size(0), NR = end - start;
+    const int64_t ws_bytes = om_moe_sort_workspace_bytes(T, K, NR), ws_at = index_words(T, K, NR);
+    Index ix = one_buffer_index(T, K, NR, Tensor(), experts, std::max<int64_t>(ws_bytes / 4, 1));
     int32_t *p = ix.owners[0].data_ptr<int32_t>();
-    auto rwp = [](const auto *q) { return const_cast<std::remove_const_t<std::remove_pointer_t<decltype(q)>> *>(q); };
     OM(c, om_moe_sort_weighted, ptr(experts), index_code(experts), ix.T, K, start, end, rwp(ix.cum), rwp(ix.cum_ep),
        rwp(ix.in), rwp(ix.out), rwp(ix.sel), ptr(rw), dtype_code(rw), rwp(ix.row_weights), p + ws_at, ws_bytes, c.stream);
     return ix;
@@ -1030,15 +1038,18 @@ Tensor route_workspace(const Tensor &x, int64_t T, int64_t H, int64_t N) {
 // softmax top-K router -> (routing_weights, selected_experts int64, logits, x).  `one_pass`: one launch for
 // projection and routing (shapes of om_router_gate_softmax_topk).  `bf16_logits`: the logits are rounded
 // to bf16 before the softmax, as a bf16 linear layer returns them.
-std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
-                                                         at::ScalarType out_dtype, bool one_pass, bool bf16_logits) {
+// start, end (end > start): the experts that the selections are to be sorted by, where the router's launch can do that too; the
+// fifth result is then moe_experts' `index`, else undefined.
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const Tensor &weight, int64_t top_k, bool renorm,
+                                                                 at::ScalarType out_dtype, bool one_pass, bool bf16_logits,
+                                                                 int64_t start, int64_t end) {
     refuse_transforms({x, weight});
     require_gate_operands(x, weight);
     const int64_t T = x.size(0), N = weight.size(0), H = weight.size(1);
     // Few tokens: one CU would take in all of the gate weight, the projection split over the chip and a launch behind it
     // are sooner; with many selections it depends (om_router_gate_split_softmax_topk, which has the figures and decides).
     if (one_pass && N <= 64 && H % 512 == 0 && (top_k > 16 || (T <= 512 && H >= 1024))) one_pass = false;
-    Tensor logits, weights, experts;
+    Tensor logits, weights, experts, index;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Call c = begin_call();
@@ -1062,7 +1073,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
             require_gate_shape(weight, "gate projection");
             logits = make({T, N}, x, bf16_logits ? at::kBFloat16 : at::kFloat);
             const Tensor ws = route_workspace(x, T, H, N);
-            OM(c, om_router_gate_split_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, ptr(logits),
+            if (end > start && om_router_gate_softmax_topk_sort_fits(T, static_cast<int>(H), static_cast<int>(N), static_cast<int>(top_k))) {
+                const Index ix = one_buffer_index(T, top_k, end - start, Tensor(), x);
+                index = ix.owners[0];
+                OM(c, om_router_gate_softmax_topk_sort, ptr(x), ptr(weight), T, H, N, top_k, renorm, ptr(logits), dtype_code(logits),
+                   ptr(weights), dtype_code(weights), experts.data_ptr<int64_t>(), start, end, rwp(ix.cum), rwp(ix.cum_ep), rwp(ix.in),
+                   rwp(ix.out), rwp(ix.sel), rwp(ix.row_weights), ptr(ws), ws.numel(), c.stream);
+            } else
+                OM(c, om_router_gate_split_softmax_topk, ptr(x), ptr(weight), T, H, N, top_k, renorm, ptr(logits),
                dtype_code(logits), ptr(weights), dtype_code(weights), experts.data_ptr<int64_t>(), ptr(ws), ws.numel(), c.stream);
         }
     }
@@ -1075,7 +1093,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> route_softmax(const Tensor &x, const 
         node->renorm = renorm;
         set_outputs(node, &logits, &weights, x_out);
     }
-    return {weights, experts, logits, x_out};
+    return {weights, experts, logits, x_out, index};
 }
 
 // sigmoid / group-limited router -> (selected_experts int64, routing_weights float32, x)
@@ -1313,10 +1331,11 @@ bool waits_ahead_of_shared(int64_t expected, int64_t G, int64_t I, int64_t H, in
 }
 
 // Sort (with the routing weights laid out per sorted row) and experts in one call: hidden_states [T,H], the experts [start, end) of n_total.
-// sync_free: never read the routed-row count of an expert window back (else up to a limit: sized_by_bound).
+// sync_free: never read the routed-row count of an expert window back (else up to a limit: sized_by_bound).  `sorted`: the index that
+// route_softmax made of these selections and weights.
 Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t start, int64_t end, int64_t n_total,
                    bool sync_free, const std::optional<Tensor> &residual, bool merged, const std::vector<Tensor> &leaves,
-                   bool has_shared, const std::optional<Tensor> &one) {
+                   bool has_shared, const std::optional<Tensor> &one, const std::optional<Tensor> &sorted) {
     refuse_transforms({x, rw, residual.value_or(Tensor())});
     refuse_transforms(leaves);
     if (experts.dim() != 2 || x.dim() != 2 || experts.size(0) != x.size(0) || rw.sizes() != experts.sizes())
@@ -1327,7 +1346,14 @@ Tensor moe_experts(const Tensor &x, Tensor rw, const Tensor &experts, int64_t st
     {
         at::AutoDispatchBelowADInplaceOrView below;
         ProfiledScope scope(c, "1moeblock--3index_calculation");
-        ix = sort_index(c, experts, start, end, rw);
+        if (sorted) {
+            if (sorted->scalar_type() != at::kInt || sorted->numel() != index_words(x.size(0), experts.size(1), end - start))
+                throw NativeError("expert MLP: the sorted index is of other sizes");
+            require_device(*sorted);
+            ix = one_buffer_index(x.size(0), experts.size(1), end - start, *sorted);
+        } else {
+            ix = sort_index(c, experts, start, end, rw);
+        }
     }
     const bool windowed = !(start == 0 && end == n_total);
     if (windowed) {
@@ -1688,12 +1714,23 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                               bool bf16_logits) {
         const at::ScalarType dt = torch::python::detail::py_object_to_dtype(dtype);
         py::gil_scoped_release nogil;
-        return route_softmax(x, w, top_k, renorm, dt, fused, bf16_logits);
+        auto r = route_softmax(x, w, top_k, renorm, dt, fused, bf16_logits, 0, 0);
+        return std::make_tuple(std::get<0>(r), std::get<1>(r), std::get<2>(r), std::get<3>(r));
+    });
+    // with the index for moe_experts of the experts [start, end), or None
+    m.def("route_softmax_sorted", [](const Tensor &x, const Tensor &w, int64_t top_k, bool renorm, py::object dtype, bool fused,
+                                     bool bf16_logits, int64_t start, int64_t end) {
+        const at::ScalarType dt = torch::python::detail::py_object_to_dtype(dtype);
+        py::gil_scoped_release nogil;
+        auto r = route_softmax(x, w, top_k, renorm, dt, fused, bf16_logits, start, end);
+        return std::make_tuple(std::get<0>(r), std::get<1>(r), std::get<2>(r), std::get<3>(r),
+                               std::get<4>(r).defined() ? std::optional<Tensor>(std::get<4>(r)) : std::nullopt);
     });
     m.def("route_sigmoid", &route_sigmoid, no_gil);
     m.def("routed_mlp_forward", &routed_mlp_forward, no_gil);
     m.def("routed_mlp_backward", &routed_mlp_backward, no_gil);
-    m.def("moe_experts", &moe_experts, no_gil);
+    m.def("moe_experts", &moe_experts, no_gil, py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(), py::arg(),
+          py::arg(), py::arg(), py::arg(), py::arg("sorted") = std::optional<Tensor>());
     m.def("merged_mlp", &merged_mlp, no_gil);
     m.def("merged_mlp_forward", &merged_mlp_forward, no_gil);
     m.def("merged_mlp_backward", &merged_mlp_backward, no_gil);

@@ -3,7 +3,7 @@
 //  * sigmoid -> bias-corrected group-limited top-K of the DeepSeek-V3 block, forward and backward.
 // Selection order is total: (score descending, expert index ascending), so the result does not
 // depend on lane scheduling.  Scores live in registers, expert i = lane + 64*j.
-#include "common.h"
+#include "sort_block.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -761,6 +761,62 @@ __global__ __launch_bounds__(NB * 512) void gate_route_slices_kernel(const uint1
     }
 }
 
+// partial_softmax_topk_kernel and the sort of its selections (om_moe_sort_weighted) by one block, for up to 64 tokens: a row of 16 lanes per
+// token, then a thread per pair.  Either alone is a launch and one chain of waits: one token of 64 experts, top-8, 3.2 + 3.4 -> 5.2 us, 37
+// tokens 4.9 + 4.8 -> 8.2 (traced; whole passes 1.7 and 1.4 less).
+constexpr int ROUTE_SORT_TOKENS = 64;
+struct SortOut {
+    int start, end, nbits;
+    int32_t *cum_token_counts, *cum_expert_counts_ep, *input_indices, *output_indices, *selected_experts_indices;
+    float *row_weights;
+};
+template <int Q, typename TL, typename TW>
+__global__ __launch_bounds__(1024) void partial_softmax_topk_sort_kernel(const float *__restrict__ partial, int splits, int Tn, int N, int K,
+                                                                         int renorm, TL *__restrict__ logits_out, TW *__restrict__ weights_out,
+                                                                         int64_t *__restrict__ experts_out, const SortOut out) {
+    __shared__ int pair_expert[ROUTE_SORT_TOKENS * 16];
+    __shared__ float pair_weight[ROUTE_SORT_TOKENS * 16];
+    const int l16 = threadIdx.x & 15, t = threadIdx.x >> 4;
+    const bool there = t < Tn;
+    if ((t & ~3) < Tn) {                                    // (the whole wavefront)
+        const float *row = partial + min(t, Tn - 1) * N;
+        float p[Q] = {};
+        for (int k0 = 0; k0 < splits; k0 += 8) {            // as partial_logits adds them
+            float v[8][Q];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int j = 0; j < Q; j++) v[u][j] = row[static_cast<int64_t>(min(k0 + u, splits - 1)) * Tn * N + min(l16 + 16 * j, N - 1)];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int j = 0; j < Q; j++) p[j] += k0 + u < splits ? v[u][j] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < Q; j++) {
+            const int n = l16 + 16 * j;
+            if (there && n < N) Elem<TL>::store(logits_out + t * N + n, p[j]);
+            if (sizeof(TL) == 2) p[j] = bf16_bits_to_f32(f32_to_bf16_bits(p[j]));
+            if (n >= N) p[j] = -INFINITY;
+        }
+        float w; int e;
+        row_softmax_topk<Q>(p, N, K, l16, w, e);
+        if (renorm) w = w / row_sum(l16 < K ? w : 0.0f);
+        if (there && l16 < K) {
+            Elem<TW>::store(weights_out + t * K + l16, w);
+            experts_out[t * K + l16] = e;
+            pair_expert[t * K + l16] = e;
+            pair_weight[t * K + l16] = sizeof(TW) == 2 ? bf16_bits_to_f32(f32_to_bf16_bits(w)) : w;   // (as stored)
+        }
+    }
+    __syncthreads();
+    const int n_pairs = Tn * K, pair = min(static_cast<int>(threadIdx.x), n_pairs - 1);
+    const int e[1] = {pair_expert[pair]};
+    const float w[1] = {pair_weight[pair]};
+    sort_block<16, 1>(e, w, n_pairs, K, out.start, out.end, out.end - out.start, out.nbits, out.cum_token_counts, out.cum_expert_counts_ep,
+                      out.input_indices, out.output_indices, out.selected_experts_indices, out.row_weights);
+}
+
 // Projection and routing of up to 64 experts in one launch, 16 tokens at a time, for gates of a small weight: what bounds those is a chain of
 // waits and launches.  So a block has eight wavefronts for every 32 experts, each with a slice of H or two, and a wavefront asks for
 // 128 columns at a time before it waits: straight into the fragments of v_mfma_f32_16x16x32_bf16, a weight is used by one wavefront only.
@@ -1217,6 +1273,49 @@ int gate_partials(const void *x, const void *gate_weight, int64_t T, int H, int 
     return splits;
 }
 }  // namespace
+
+// Whether the router of these sizes is the split projection and a routing launch that can sort as well.
+extern "C" int om_router_gate_softmax_topk_sort_fits(int64_t T, int H, int N, int K) {
+    if (T < 1 || T > ROUTE_SORT_TOKENS || H < 8 || H % 8 != 0 || N < 1 || N > 64 || K < 1 || K > N || K > 16) return 0;
+    return gate_rows_fit(T, H, N, K) || (gate_slices_fit(H, N) && H < 1024) ? 0 : 1;
+}
+
+extern "C" int om_router_gate_softmax_topk_sort(const void *x, const void *gate_weight, int64_t T, int H, int N, int K, int norm_topk_prob,
+                                                void *logits_out, int logits_dtype, void *weights_out, int weights_dtype,
+                                                int64_t *experts_out, int expert_start_idx, int expert_end_idx,
+                                                int32_t *cum_token_counts, int32_t *cum_expert_counts_ep, int32_t *input_indices,
+                                                int32_t *output_indices, int32_t *selected_experts_indices, float *row_weights,
+                                                void *workspace, int64_t workspace_bytes, void *stream) {
+    if ((weights_dtype != OM_F32 && weights_dtype != OM_BF16) || (logits_dtype != OM_F32 && logits_dtype != OM_BF16))
+        return OM_ERR_DTYPE;
+    if (!om_router_gate_softmax_topk_sort_fits(T, H, N, K) || expert_start_idx < 0 || expert_end_idx <= expert_start_idx || expert_end_idx > N)
+        return OM_ERR_SHAPE;
+    for (const void *p : {static_cast<const void *>(logits_out), static_cast<const void *>(weights_out), static_cast<const void *>(experts_out),
+                          static_cast<const void *>(cum_token_counts), static_cast<const void *>(cum_expert_counts_ep),
+                          static_cast<const void *>(input_indices), static_cast<const void *>(output_indices),
+                          static_cast<const void *>(selected_experts_indices)})
+        if (!p) return OM_ERR_NULL;
+    const int rc = gate_operands(x, gate_weight, T, H, N, workspace, workspace_bytes);
+    if (rc != OM_OK) return rc;
+    const int splits = gate_partials(x, gate_weight, T, H, N, workspace, stream);
+    const SortOut out = {expert_start_idx, expert_end_idx, key_bits(expert_end_idx - expert_start_idx), cum_token_counts, cum_expert_counts_ep,
+                         input_indices, output_indices, selected_experts_indices, row_weights};
+#define OM_PS(Q, TL, TW)                                                                                                            \
+    partial_softmax_topk_sort_kernel<Q, TL, TW><<<1, 1024, 0, om_stream(stream)>>>(static_cast<const float *>(workspace), splits,      \
+        static_cast<int>(T), N, K, norm_topk_prob, static_cast<TL *>(logits_out), static_cast<TW *>(weights_out), experts_out, out)
+#define OM_PS_Q(TL, TW)                       \
+    do {                                      \
+        if (N <= 32) OM_PS(2, TL, TW);        \
+        else OM_PS(4, TL, TW);                \
+    } while (0)
+    if (logits_dtype == OM_F32 && weights_dtype == OM_F32) OM_PS_Q(float, float);
+    else if (logits_dtype == OM_F32) OM_PS_Q(float, uint16_t);
+    else if (weights_dtype == OM_F32) OM_PS_Q(uint16_t, float);
+    else OM_PS_Q(uint16_t, uint16_t);
+#undef OM_PS_Q
+#undef OM_PS
+    return om_launch_status();
+}
 
 extern "C" int om_router_gate_split_softmax_topk(const void *x, const void *gate_weight, int64_t T, int H, int N, int K,
                                                  int norm_topk_prob, void *logits_out, int logits_dtype,

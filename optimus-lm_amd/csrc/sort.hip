@@ -14,7 +14,7 @@
 // 5.3 + 6.3 + 11.6, 9003 pairs of 12 7.0 + 3.1 + 16.3 -> 4.0 + 3.0 + 8.4.
 // Also: the reference's two index operators with their own [expert][column] table layout, one
 // wavefront per column.
-#include "common.h"
+#include "sort_block.h"
 #include <mutex>
 
 namespace {
@@ -49,18 +49,6 @@ __device__ __forceinline__ int local_key(const TI *selected_experts, int64_t j, 
     const long long e = static_cast<long long>(selected_experts[j]);
     return (e >= start && e < end) ? static_cast<int>(e - start) : NR;
 }
-
-// Mask of the lanes of this wavefront that hold the same key (keys < 2^nbits).
-__device__ __forceinline__ unsigned long long match_key(int key, int nbits) {
-    unsigned long long m = ~0ull;
-    for (int b = 0; b < nbits; b++) {
-        const unsigned long long vote = __ballot((key >> b) & 1);
-        m &= ((key >> b) & 1) ? vote : ~vote;
-    }
-    return m;
-}
-
-__device__ __forceinline__ unsigned long long lanemask_lt(int lane) { return (1ull << lane) - 1ull; }
 
 // The keys of a wavefront's SORT_ITERS*64 pairs, all loads in flight at once.
 template <typename TI>
@@ -109,15 +97,6 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_count_kernel(const TI *__re
         for (int w = 0; w < SORT_WAVES; w++) s += lds[w * NR + e];
         block_hist[static_cast<int64_t>(blockIdx.x) * NR + e] = s;
     }
-}
-
-// Inclusive prefix sum over the 64 lanes of a wavefront.
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, 64);
-        if (lane >= o) v += u;
-    }
-    return v;
 }
 
 // One block.  block_hist [NB][NR] -> in place: exclusive offset of (expert e, block b) in the
@@ -249,27 +228,16 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
     }
 }
 
-// Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (up to 8 x 64)
-// pairs' keys, weights and ranks in registers between the passes.  A decode batch or a small training batch spends
-// nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced), one of 6 when the
-// caches are warm.  So no step waits for another's loads (ITERS, the 64-pair steps of a wavefront, is known to the compiler, and
-// pairs past the end are read as the last one), the rank of a pair within its expert comes from the counting pass, and
-// only that pass is a chain through LDS: 4096 pairs with cold caches, in a training step of 512 tokens of 64 experts, 15.2 ->
-// 9.8 us.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront) reaches what the three
-// launches take.
+// Few pairs: count, scan and scatter by one block, in one launch (sort_block.h).
 constexpr int SMALL_WAVES = 16, SMALL_MAX_ITERS = 8;
 constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SMALL_MAX_ITERS;
-constexpr int SMALL_MAX_NR = 256;
 template <typename TI, int ITERS>
 __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
     const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
     int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
     int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
     int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
-    __shared__ int off[SMALL_WAVES][SMALL_MAX_NR];   // counts, then the first position of a wavefront's rows of an expert
-    __shared__ __attribute__((aligned(16))) int wave_hits[SMALL_WAVES], chunk_total[SMALL_MAX_NR / 64];
-    __shared__ int kept_total;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int base = wv * ITERS * 64 + lane;
     TI e[ITERS];
 #pragma unroll
@@ -285,86 +253,8 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
 #pragma unroll
         for (int it = 0; it < ITERS; it++) weight[it] = static_cast<const float *>(rw.routing_weights)[min(base + it * 64, n_pairs - 1)];
     }
-    volatile int *mine = off[wv];
-    for (int i = lane; i < NR; i += 64) mine[i] = 0;
-    __builtin_amdgcn_wave_barrier();
-    int key[ITERS], rank[ITERS], before_in_step[ITERS], hits = 0;   // before_in_step: kept pairs of this wavefront before this one
-#pragma unroll
-    for (int it = 0; it < ITERS; it++) {
-        const long long v = static_cast<long long>(e[it]);
-        const bool kept = base + it * 64 < n_pairs && v >= start && v < end;
-        key[it] = kept ? static_cast<int>(v - start) : NR;
-        const unsigned long long m = match_key(key[it], nbits), all = __ballot(kept);
-        const int seen = mine[kept ? key[it] : 0];
-        __builtin_amdgcn_wave_barrier();
-        rank[it] = seen + __popcll(m & lanemask_lt(lane));
-        if (kept && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] = seen + __popcll(m);
-        before_in_step[it] = hits + __popcll(all & lanemask_lt(lane));
-        hits += __popcll(all);
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (lane == 0) wave_hits[wv] = hits;
-    __syncthreads();
-    // thread e: expert e's total over the wavefronts, exclusive positions of the wavefronts within it
-    int total = 0, at[SMALL_WAVES];
-    if (tid < NR) {
-#pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) at[w] = off[w][tid];
-#pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) {
-            const int c = at[w];
-            at[w] = total;
-            total += c;
-        }
-    }
-    const int incl = wave_incl_scan(total, lane);
-    if (tid < SMALL_MAX_NR && lane == 63) chunk_total[wv] = incl;
-    __syncthreads();
-    int before = incl - total;   // rows of the experts before this one
-#pragma unroll
-    for (int w = 0; w < SMALL_MAX_NR / 64; w++) before += w < wv ? chunk_total[w] : 0;
-    if (tid < NR) {
-#pragma unroll
-        for (int w = 0; w < SMALL_WAVES; w++) off[w][tid] = before + at[w];
-        cum_token_counts[tid] = before;
-        if (tid == NR - 1) {
-            cum_token_counts[NR] = before + total;
-            cum_expert_counts_ep[n_pairs / K] = before + total;
-            kept_total = before + total;
-        }
-    }
-    __syncthreads();
-    int oi_base = 0;
-#pragma unroll
-    for (int w = 0; w < SMALL_WAVES; w++) oi_base += w < wv ? wave_hits[w] : 0;
-    const int kept_all = kept_total;
-#pragma unroll
-    for (int it = 0; it < ITERS; it++) {
-        const int j = base + it * 64;
-        if (j >= n_pairs) continue;
-        if (j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
-            output_indices[j] = -1;
-            input_indices[j] = 0;
-            selected_experts_indices[j] = 0;
-        }
-        const int oi = oi_base + before_in_step[it];
-        const uint32_t t = static_cast<uint32_t>(j) / static_cast<uint32_t>(K);
-        const int k = j - static_cast<int>(t) * K;
-        if (k == 0) cum_expert_counts_ep[t] = oi;
-        if (key[it] < NR) {
-            const int pos = off[wv][key[it]] + rank[it];
-            input_indices[pos] = static_cast<int32_t>(t);
-            output_indices[oi] = pos;
-            selected_experts_indices[oi] = k;
-            rw.put(pos, weight[it]);
-        }
-    }
-}
-
-inline int key_bits(int NR) {  // keys 0..NR (NR = "not local")
-    int b = 1;
-    while ((1 << b) <= NR) b++;
-    return b;
+    sort_block<SMALL_WAVES, ITERS>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
+                                   output_indices, selected_experts_indices, rw.row_weights);
 }
 
 // ---- the reference's table layout [expert][column] ---------------------------------------------
@@ -488,7 +378,7 @@ int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, in
                     const RowWeights &rw = RowWeights()) {
     const int NR = expert_end_idx - expert_start_idx;
     const int64_t n_pairs = T * K;
-    if (n_pairs > 0 && n_pairs <= SMALL_PAIRS && NR <= SMALL_MAX_NR) {
+    if (n_pairs > 0 && n_pairs <= SMALL_PAIRS && NR <= SORT_BLOCK_MAX_NR) {
 #define OM_SMALL(TI, ITERS)                                                                                                     \
     sort_small_kernel<TI, ITERS><<<1, SMALL_WAVES * 64, 0, st>>>(                                                               \
         static_cast<const TI *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR,          \

@@ -54,6 +54,9 @@ SIGNATURES = {
     "om_router_gate_route_workspace_bytes": (c_i64, [c_i64, c_int, c_int]),
     "om_router_gate_split_softmax_topk": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int, c_void_p, c_int,
                                                   c_void_p, c_int, c_void_p, c_void_p, c_i64, c_void_p]),
+    "om_router_gate_softmax_topk_sort_fits": (c_int, [c_i64, c_int, c_int, c_int]),
+    "om_router_gate_softmax_topk_sort": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
+                                                 c_void_p, c_int, c_int] + [c_void_p] * 7 + [c_i64, c_void_p]),
     "om_router_gate_split_sigmoid_group_topk_bias": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_i64] + [c_int] * 6 +
                                                      [c_double] + [c_void_p] * 4 + [c_i64, c_void_p]),
     "om_router_gate_split_sigmoid_group_topk": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int,
@@ -212,7 +215,8 @@ _UNTIMED = {"om_version", "om_arch", "om_strerror", "om_moe_sort_workspace_bytes
             "om_moe_sort_static_capacity_bytes",
             "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes",
             "om_router_gate_wgrad_workspace_bytes", "om_router_gate_route_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
-            "om_merged_mlp_row_dot_parts", "om_router_softmax_bwd_workspace_bytes", "om_grad_norm_fits"}
+            "om_merged_mlp_row_dot_parts", "om_router_softmax_bwd_workspace_bytes", "om_router_gate_softmax_topk_sort_fits",
+            "om_grad_norm_fits"}
 
 
 class NativeLibraryError(RuntimeError):

@@ -10,6 +10,7 @@ Pipeline of FastOlmoeParallelSparseMoeBlock.forward (reference moe.py:454-621):
 and the mirrored backward.  There is one code path: the reference's `use_triton_path_*` and
 `use_ref_path_*` switches are accepted where its signatures have them and ignored.
 """
+import functools
 import warnings
 
 import torch
@@ -855,8 +856,9 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         return group_mlp(hidden_states, cum_token_counts, self.experts, input_indices, cum_expert_counts_ep,
                          output_indices)
 
-    def _fused_experts_fn(self, hidden_states, routing_weights, selected_experts, residual):
-        """Permutation and RoutedMLPFunction in one call; None when the kernels do not take the operands."""
+    def _fused_experts_fn(self, hidden_states, routing_weights, selected_experts, residual, sorted_index=None):
+        """Permutation and RoutedMLPFunction in one call; None when the kernels do not take the operands.
+        `sorted_index`: the permutation, where the router's launch has made it."""
         merged = isinstance(self.experts, MergedMLP)
         if merged:
             # (as attributes: a weight may be parametrized, or a plain tensor that a wrapper has put there)
@@ -870,7 +872,7 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
             return None
         return _n.host().moe_experts(hidden_states, routing_weights, selected_experts, self.expert_start_idx,
                                      self.expert_end_idx, self.num_experts, self.sync_free_expert_window,
-                                     residual, merged, weights, False, None)
+                                     residual, merged, weights, False, None, sorted_index)
 
     def forward_with_residual(self, hidden_states, residual):
         """(residual + forward(hidden_states)[0], router_logits): the decoder layer's
@@ -888,12 +890,16 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         # (the experts are fed from the router's pass-through of the hidden states, so that their input
         # gradient and the gate's are added in one kernel)
         weight = self.gate.weight.contiguous()
+        sorted_index = None
         if flat.is_cuda and flat.dtype == weight.dtype and flat.dtype in (torch.bfloat16, torch.float32) \
                 and self.gate.bias is None:
             bf16 = flat.dtype == torch.bfloat16
-            routing_weights, selected_experts, router_logits, flat = _n.host().route_softmax(
+            # (the router sorts its selections where one launch can, for the experts called right behind it)
+            sorts = bf16 and self.fuse_input_gather and self.fuse_routing_weights and not self.use_activation_checkpointing_for_moe
+            routing_weights, selected_experts, router_logits, flat, sorted_index = _n.host().route_softmax_sorted(
                 flat.contiguous(), weight, self.num_experts_per_tok, bool(self.norm_topk_prob), flat.dtype,
-                self.router_logits_fp32 and gate_unfit is None, bf16 and not self.router_logits_fp32)
+                self.router_logits_fp32 and gate_unfit is None, bf16 and not self.router_logits_fp32,
+                self.expert_start_idx if sorts else 0, self.expert_end_idx if sorts else 0)
         else:
             if self.router_logits_fp32:
                 router_logits, flat = fp32_logits_with_passthrough(flat, weight)
@@ -905,6 +911,8 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         def expert_computation_block(flat, selected_experts, routing_weights, residual=None):
             gathered = self._gathered_experts_fn if self.fuse_input_gather else None
             fused = self._fused_experts_fn if (self.fuse_input_gather and self.fuse_routing_weights) else None
+            if sorted_index is not None:
+                fused = functools.partial(fused, sorted_index=sorted_index)
             return expert_computation(flat, routing_weights, selected_experts,
                                       self.expert_start_idx, self.expert_end_idx, self._experts_fn,
                                       self.num_experts, gathered_experts_fn=gathered,

@@ -179,6 +179,22 @@ def test_grouped_gemms(lib):
     assert lib.om_grouped_gemm_wgrad_gathered(P, P, P, 16384, ODD, P, *g) == ALIGN
 
 
+def test_router_that_sorts(lib):
+    fits = lib.om_router_gate_softmax_topk_sort_fits
+    assert fits(1, 2048, 64, 8) == 1 and fits(64, 2048, 64, 16) == 1
+    for T, H, N, K in ((65, 2048, 64, 8), (0, 2048, 64, 8), (1, 2044, 64, 8), (1, 2048, 65, 8), (1, 2048, 64, 17), (1, 256, 8, 2), (1, 512, 64, 8)):
+        assert fits(T, H, N, K) == 0
+    f = lib.om_router_gate_softmax_topk_sort
+    head, index = (P, P, 1, 2048, 64, 8, 0, P, BF16, P, BF16, P), (P,) * 6
+    assert f(*head, 0, 65, *index, P, 1 << 20, None) == SHAPE
+    assert f(*head, 8, 8, *index, P, 1 << 20, None) == SHAPE
+    assert f(P, P, 65, *head[3:], 0, 64, *index, P, 1 << 20, None) == SHAPE
+    assert f(*head[:8], 7, *head[9:], 0, 64, *index, P, 1 << 20, None) == DTYPE
+    assert f(*head, 0, 64, P, P, None, P, P, P, P, 1 << 20, None) == NULL
+    assert f(ODD, *head[1:], 0, 64, *index, P, 1 << 20, None) == ALIGN
+    assert f(*head, 0, 64, *index, P, 16, None) == WORKSPACE
+
+
 def test_router_backward_in_one_call(lib):
     need = lib.om_router_softmax_bwd_workspace_bytes(2048, 256, 8)
     assert need > 0

@@ -693,3 +693,34 @@ def test_float32_router_launches_equal_their_steps(cuda, T, H, N, K):
         n.check(lib.om_router_gate_wgrad_f32(n.ptr(x), n.ptr(dl), T, H, N, n.ptr(want_dw), st), "dw")
         n.check(lib.om_router_gate_bwd_f32(n.ptr(x), n.ptr(dl), n.ptr(w), n.ptr(b), T, H, N, n.ptr(dx), n.ptr(dw), st), "both")
         assert torch.equal(dx, want_dx) and torch.equal(dw, want_dw)
+
+
+@pytest.mark.parametrize("T,H,N,K,start,end", [(1, 2048, 64, 8, 0, 64), (3, 1024, 33, 16, 0, 33), (4, 4096, 17, 1, 5, 9), (5, 7168, 8, 8, 0, 1), (37, 2048, 64, 8, 0, 64),
+                                               (64, 1536, 32, 16, 8, 24), (63, 3000, 64, 3, 60, 64)])
+@pytest.mark.parametrize("bf16_logits", [False, True])
+def test_router_that_sorts_its_selections(cuda, T, H, N, K, start, end, bf16_logits):
+    """Bit for bit the router and the sort of what it selects."""
+    from optimus import _native as n
+    lib, st = n.lib(), n.stream()
+    assert lib.om_router_gate_softmax_topk_sort_fits(T, H, N, K) == 1
+    x, w = (t.to(cuda) for t in _gate_inputs(T, H, N, seed=T + H))
+    ldt = torch.bfloat16 if bf16_logits else torch.float32
+    ws = torch.empty(max(lib.om_router_gate_route_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+    i32 = lambda k: torch.full((k,), -7, dtype=torch.int32, device=cuda)
+    NR = end - start
+    for renorm, wdt in ((0, torch.bfloat16), (1, torch.float32)):
+        def buffers():
+            return ([torch.empty(T, N, dtype=ldt, device=cuda), torch.empty(T, K, dtype=wdt, device=cuda), torch.empty(T, K, dtype=torch.int64, device=cuda)],
+                    [i32(NR + 1), i32(T + 1), i32(T * K), i32(T * K), i32(T * K), torch.full((T * K,), -7.0, device=cuda)])
+        (logits, weights, experts), index = buffers()
+        n.check(lib.om_router_gate_split_softmax_topk(n.ptr(x), n.ptr(w), T, H, N, K, renorm, n.ptr(logits), n.dtype_code(logits), n.ptr(weights),
+                                                      n.dtype_code(weights), n.ptr(experts), n.ptr(ws), ws.numel(), st), "router")
+        sort_ws = i32(max(lib.om_moe_sort_workspace_bytes(T, K, NR) // 4, 1))
+        n.check(lib.om_moe_sort_weighted(n.ptr(experts), n.OM_I64, T, K, start, end, *(n.ptr(t) for t in index[:5]), n.ptr(weights), n.dtype_code(weights),
+                                         n.ptr(index[5]), n.ptr(sort_ws), sort_ws.numel() * 4, st), "sort")
+        (g_logits, g_weights, g_experts), g_index = buffers()
+        n.check(lib.om_router_gate_softmax_topk_sort(n.ptr(x), n.ptr(w), T, H, N, K, renorm, n.ptr(g_logits), n.dtype_code(g_logits), n.ptr(g_weights),
+                                                     n.dtype_code(g_weights), n.ptr(g_experts), start, end, *(n.ptr(t) for t in g_index), n.ptr(ws),
+                                                     ws.numel(), st), "router and sort")
+        for got, want in zip([g_logits, g_weights, g_experts] + g_index, [logits, weights, experts] + index):
+            assert torch.equal(got, want)
