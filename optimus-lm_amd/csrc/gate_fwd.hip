@@ -130,6 +130,45 @@ __global__ __launch_bounds__(256) void gate_logits_split_kernel(const uint16_t *
     }
 }
 
+// The same for few tokens: a wavefront per 16 tokens, 16 experts and slice, all of a slice's 256 columns under way at once, straight into
+// the fragments of v_mfma_f32_16x16x32_bf16 (the same sums).  What bounds it is one miss after another, above four of them at hidden
+// 2048 (two stages of 64 columns), here one.  us, with the
+// routing, weights out of the caches: hidden 2048, 64 experts, 1 token 12.5 -> 10.1, 64 13.7 -> 10.3, 512 15.8 -> 10.9; hidden 7168, 64 experts,
+// 512 tokens 25.0 -> 16.3, 8 experts 20.5 -> 10.6.  Every 16 tokens read the weight again: hidden 3000, 60 experts, 1000 tokens 17.4 -> 19.8, 4000 21.3 ->
+// 33.7, hidden 4040, 20 experts, 2000 tokens 14.8 -> 15.5.  Hence the line.
+constexpr int64_t GATE_FEW_TOKENS = 512;
+template <int CH>
+__global__ __launch_bounds__(64) void gate_logits_few_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int64_t T, int H, int N,
+                                                             int h_per_split, float *__restrict__ partial) {
+    const int lane = threadIdx.x, l16 = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16, split = blockIdx.y;
+    const int64_t t = static_cast<int64_t>(blockIdx.z) * 16 + l16;
+    const int begin = split * h_per_split, len = min(H - begin, h_per_split);
+    // rows past the end (tokens, experts): the last one, results unused; columns past the end: the last chunk again, of tokens zeros
+    const uint16_t *xr = x + min(t, T - 1) * H + begin, *wr = w + static_cast<int64_t>(min(n0 + l16, N - 1)) * H + begin;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int c = 0; c < len; c += CH * 32) {
+        u32x4 wf[CH], xf[CH];
+#pragma unroll
+        for (int i = 0; i < CH; i++) {
+            const int k = c + i * 32 + g * 8, at = min(k, len - 8);
+            wf[i] = *reinterpret_cast<const u32x4 *>(wr + at);
+            xf[i] = *reinterpret_cast<const u32x4 *>(xr + at);
+            if (k >= len) xf[i] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int i = 0; i < CH; i++)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wf[i]), __builtin_bit_cast(bf16x8, xf[i]), acc, 0, 0, 0);
+    }
+    // element r of lane l: expert 4 * (l / 16) + r of token l % 16
+    if (t < T) {
+        float *out = partial + (static_cast<int64_t>(split) * T + t) * N + n0 + g * 4;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (n0 + g * 4 + r < N) out[r] = acc[r];
+    }
+}
+
 // The same for more than 64 experts, where a step's weights (32 KB for 256) are most of what a CU takes in: 128 tokens and all
 // experts per block of eight wavefronts (64 x 64 of the logits each, NB = 4: 32 x 64), tokens and weights both by direct loads of
 // whole 128-byte rows, two steps ahead, through a ring of three.  Rows, chunks and the last step as above, but that the
@@ -282,7 +321,9 @@ void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, 
     const dim3 grid(static_cast<unsigned>((T + GT - 1) / GT), splits);
     const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(gate_weight);
     const int hps = ((H + GK - 1) / GK + splits - 1) / splits * GK;
-    if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    if (N <= 64 && T <= GATE_FEW_TOKENS) {
+        gate_logits_few_kernel<8><<<dim3((N + 15) / 16, splits, static_cast<unsigned>((T + 15) / 16)), dim3(64), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    } else if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
     else if (N <= 128) gate_logits_wide_kernel<4><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);
     else gate_logits_wide_kernel<8><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);
 }

@@ -724,3 +724,14 @@ def test_router_that_sorts_its_selections(cuda, T, H, N, K, start, end, bf16_log
                                                      ws.numel(), st), "router and sort")
         for got, want in zip([g_logits, g_weights, g_experts] + g_index, [logits, weights, experts] + index):
             assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("H,N", [(1024, 64), (2048, 61), (4608, 50), (7168, 17), (1536, 1)])
+def test_few_tokens_have_the_logits_of_many(cuda, H, N):
+    """Up to 512 tokens a wavefront takes 16 tokens and experts of a slice, above them a block goes through it: the same eight sums in order."""
+    from optimus import _native as n
+    x, w = (t.to(cuda) for t in _gate_inputs(513, H, N, seed=H + N))
+    _, _, many, _ = n.host().route_softmax(x, w, 1, False, torch.bfloat16, False, False)
+    for T in (1, 16, 17, 512):
+        _, _, few, _ = n.host().route_softmax(x[:T], w, 1, False, torch.bfloat16, False, False)
+        assert torch.equal(few, many[:T])
