@@ -127,7 +127,7 @@ int om_shard_clip_multiplier(const float *value, int mode, int grad_dtype, doubl
  * i.e. the in-place multiply of clip_grads_with_norm_ (optimizers.py:145/150/154) without its
  * read-modify-write pass over the gradients.  *grad_scale is a device fp32 scalar (the clip_coef
  * above).  store_scaled_grad != 0 also writes g back into `grad`, which leaves the gradient
- * buffer as the reference leaves it (+2 B/element of traffic in bf16 mode); 0 leaves `grad`
+ * buffer as the reference leaves it (+2 B/element of traffic in bf16 mode where the bits change); 0 leaves `grad`
  * untouched.                                                                              */
 int om_adamw_step_clipped(void *param, void *grad, float *master, float *exp_avg,
                           float *exp_avg_sq, int64_t n, double lr, double beta1, double beta2,

@@ -118,6 +118,32 @@ def test_clipped_step_fp32_bit_exact(cuda, oracle_lib, store):
     assert np.array_equal(g.cpu().numpy(), go if store else g0.numpy())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [257, 4096 + 3, (9 << 20) + 5])     # one launch with its tail; past the caches and a launch for the tail
+@pytest.mark.parametrize("coef", [1.0, 1.0 - 2.0 ** -8, 0.5])
+def test_clipped_step_gradients_that_keep_their_bits(cuda, oracle_lib, dtype, n, coef):
+    """Gradients that the coefficient leaves as they are (all of them, wavefronts of zeros, single values that round back) are what
+    scaling and storing every one of them gives."""
+    from optimus.optimizers import adamw_step_
+    g0 = _grad(n, dtype, 11, 1e-3)
+    g0[256:1024] = 0.0                                    # whole wavefronts, of 256 elements, that keep their bits
+    g0[1024:2048:3] = -0.0
+    if coef == 1.0:
+        g0[5], g0[200] = float("inf"), float("nan")
+    st = _state(n)
+    w = st["master"].clone().to(cuda); m = st["exp_avg"].clone().to(cuda); v = st["exp_avg_sq"].clone().to(cuda)
+    p = w if dtype == torch.float32 else st["param"].clone().to(cuda)
+    g = g0.clone().to(cuda)
+    adamw_step_(p, g, w, m, v, 100, HP["lr"], HP["beta1"], HP["beta2"], HP["eps"], HP["weight_decay"],
+                grad_scale=torch.tensor([coef], dtype=torch.float32, device=cuda), store_scaled_grad=True)
+    torch.cuda.synchronize()
+    go = bits(g0).copy() if dtype == torch.bfloat16 else g0.numpy().copy()
+    with np.errstate(invalid="ignore"):
+        oracle_lib.scale_grads(go, coef)
+    got = bits(g) if dtype == torch.bfloat16 else g.cpu().numpy()
+    assert np.array_equal(got, go) if dtype == torch.bfloat16 else np.array_equal(got, go, equal_nan=True)
+
+
 class _Net(torch.nn.Module):
     def __init__(self):
         super().__init__()
