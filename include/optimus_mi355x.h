@@ -452,13 +452,20 @@ int om_reduce_ggemm_output_backward(const void *final_hidden_states_grad, const 
  *   out, h_out share `dtype`; E a multiple of 8 (bf16) / 4 (fp32); rows of any length.
  * om_rmsnorm_bwd: dx [rows,E] = r * (g*w - xn * mean(g*w*xn)), xn = float(h)*r, g = dy, and
  *   dweight [E] = sum_rows dy * cast(xn) (fp32 accumulation, deterministic order), from h (the
- *   tensor that was normalised) and rstd.  workspace: om_rmsnorm_bwd_workspace_bytes.        */
+ *   tensor that was normalised) and rstd.  workspace: om_rmsnorm_bwd_workspace_bytes at least; with
+ *   om_rmsnorm_bwd_workspace_spread_bytes few rows are spread over more of the chip.
+ * om_rmsnorm_bwd_residual: the same with h_grad [rows,E] (NULL: none) added to dx, rounded to the dtype before and
+ *   after the addition: the gradient that h receives as the next residual.                           */
 int om_rmsnorm_fwd(const void *x, const void *residual, const void *weight, double eps, void *out,
                    void *h_out, float *rstd_out, int64_t rows, int64_t E, int dtype, void *stream);
 int64_t om_rmsnorm_bwd_workspace_bytes(int64_t rows, int64_t E);
+int64_t om_rmsnorm_bwd_workspace_spread_bytes(int64_t rows, int64_t E);
 int om_rmsnorm_bwd(const void *dy, const void *h, const void *weight, const float *rstd, void *dx,
                    void *dweight, void *workspace, int64_t workspace_bytes, int64_t rows, int64_t E,
                    int dtype, void *stream);
+int om_rmsnorm_bwd_residual(const void *dy, const void *h, const void *weight, const float *rstd, const void *h_grad,
+                            void *dx, void *dweight, void *workspace, int64_t workspace_bytes, int64_t rows, int64_t E,
+                            int dtype, void *stream);
 
 /* ------------------------------------------------------------------------------------
  * Grouped expert GEMMs (bf16 operands, fp32 MFMA accumulation, bf16 results)

@@ -83,8 +83,10 @@ SIGNATURES = {
     "om_rmsnorm_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_double, c_void_p, c_void_p, c_void_p,
                                c_i64, c_i64, c_int, c_void_p]),
     "om_rmsnorm_bwd_workspace_bytes": (c_i64, [c_i64, c_i64]),
+    "om_rmsnorm_bwd_workspace_spread_bytes": (c_i64, [c_i64, c_i64]),
     "om_rmsnorm_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                c_i64, c_i64, c_i64, c_int, c_void_p]),
+    "om_rmsnorm_bwd_residual": (c_int, [c_void_p] * 8 + [c_i64, c_i64, c_i64, c_int, c_void_p]),
     "om_route_sigmoid_group_topk": (c_int, [c_void_p, c_void_p, c_i64, c_int, c_int, c_int, c_int,
                                             c_int, c_double, c_void_p, c_void_p, c_void_p]),
     "om_route_sigmoid_topk_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int, c_int,
@@ -213,7 +215,7 @@ launch_log = None
 launch_filter = None   # optional set of entry-point names: only these are timed while launch_log is set
 _UNTIMED = {"om_version", "om_arch", "om_strerror", "om_moe_sort_workspace_bytes",
             "om_moe_sort_static_capacity_bytes",
-            "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes",
+            "om_router_balance_workspace_bytes", "om_rmsnorm_bwd_workspace_bytes", "om_rmsnorm_bwd_workspace_spread_bytes",
             "om_router_gate_wgrad_workspace_bytes", "om_router_gate_route_workspace_bytes", "om_router_gate_logits_split_workspace_bytes",
             "om_merged_mlp_row_dot_parts", "om_router_softmax_bwd_workspace_bytes", "om_router_gate_softmax_topk_sort_fits",
             "om_grad_norm_fits"}

@@ -69,3 +69,41 @@ def test_backward(cuda, rows, E, dtype):
     assert rel(xg.grad, xr.grad) <= tol and rel(rg.grad, rr.grad) <= tol
     assert rel(m.weight.grad, wr.grad) <= (1e-5 if dtype == torch.float32 else 6e-3)
     assert torch.equal(xg.grad, rg.grad)
+
+
+# one to four vectors a lane, one lane short and over, the first row length that a wavefront does not hold; less than a wavefront's
+# rows, a partial chunk (four rows up to 2048, then eight), both ways of loading (more than 8 M elements)
+@pytest.mark.parametrize("rows,vecs", [(1, 1), (3, 64), (5, 65), (2047, 129), (2049, 192), (2051, 193), (4100, 256), (70, 257), (4099, 250),
+                                       (16387, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_that_a_wavefront_holds(cuda, rows, vecs, dtype):
+    from optimus.models.olmoe.modeling_olmoe import OlmoeParallelRMSNorm
+    E = vecs * (8 if dtype == torch.bfloat16 else 4)
+    x, res, w = _inputs(rows, E, dtype, seed=rows + vecs)
+    dy = torch.randn(rows, E, generator=torch.Generator().manual_seed(4)).to(dtype)
+    m = OlmoeParallelRMSNorm(E, eps=1e-5).to(dtype).to(cuda)
+    with torch.no_grad():
+        m.weight.copy_(w)
+    xg = x.to(cuda).requires_grad_(True)
+    y, h = m.forward_with_residual(xg, res.to(cuda))
+    gh = torch.randn(rows, E, generator=torch.Generator().manual_seed(5)).to(dtype)
+    dx_alone, dw_alone = torch.autograd.grad(y, (xg, m.weight), dy.to(cuda), retain_graph=True)
+    torch.autograd.backward([y, h], [dy.to(cuda), gh.to(cuda)])
+    assert torch.equal(xg.grad, dx_alone + gh.to(cuda)) and torch.equal(m.weight.grad, dw_alone)
+    y_ref, h_ref = rmsnorm(x, w, 1e-5, residual=res)
+    assert torch.equal(h.detach().cpu(), h_ref)
+    if dtype == torch.float32:
+        torch.testing.assert_close(y.detach().cpu(), y_ref, rtol=2e-6, atol=1e-7)
+    else:
+        _close_bf16(y.detach().cpu(), y_ref)
+    # the gradients in float64, from the sum as the dtype holds it and (the weight's) the normalised value as it rounds it
+    hd, gd, wd = h_ref.double(), dy.double(), w.double()
+    r = (hd.pow(2).mean(1, keepdim=True) + 1e-5).rsqrt()
+    xn, dxn = hd * r, gd * wd
+    dx = r * (dxn - xn * (dxn * xn).mean(1, keepdim=True))
+    # one rounding of the result (2^-9 / 2^-24 of it) and the float32 sums before it: at most E + rows terms' relative 2^-24 each
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -21
+    assert float((dx_alone.cpu().double() - dx).norm() / dx.norm()) <= eps
+    terms = gd * xn.to(dtype).double()
+    bound = eps * terms.sum(0).abs() + terms.abs().sum(0) * (2.0 ** -24 * (rows / 4 + 8) + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22))
+    assert bool(((m.weight.grad.cpu().double() - terms.sum(0)).abs() <= bound).all())
