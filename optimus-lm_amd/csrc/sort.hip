@@ -1,6 +1,7 @@
 // Token permutation for the fast MoE block: a stable counting sort of the (token, k) pairs by
 // local expert, producing exactly the arrays the reference builds with its two index kernels and
-// two cumsums.  Up to 8192 pairs are one launch of one block (sort_small_kernel); more are three:
+// two cumsums.  Up to 65536 pairs are one launch: of one block up to 1024 (sort_small_kernel), of a block for every 1024 beyond
+// (sort_spread_kernel); more pairs, or more than 256 local experts, are three:
 //   count   — every block histograms its chunk of pairs per expert (wave ballots -> LDS);
 //   scan    — one block (16 wavefront-wide scans at a time) turns the [block][expert] table into exclusive offsets in
 //             (expert-major, block-minor) order = the stable order, and writes cum_token_counts;
@@ -16,6 +17,7 @@
 // wavefront per column.
 #include "sort_block.h"
 #include <mutex>
+#include <type_traits>
 
 namespace {
 
@@ -229,32 +231,64 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
 }
 
 // Few pairs: count, scan and scatter by one block, in one launch (sort_block.h).
-constexpr int SMALL_WAVES = 16, SMALL_MAX_ITERS = 8;
-constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64 * SMALL_MAX_ITERS;
-template <typename TI, int ITERS>
+constexpr int SMALL_WAVES = 16;
+constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64;
+template <typename TI>
 __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
     const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
     int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
     int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
     int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int base = wv * ITERS * 64 + lane;
-    TI e[ITERS];
+    const TI e[1] = {selected_experts[min(static_cast<int>(threadIdx.x), n_pairs - 1)]};
+    const float weight[1] = {rw.get(threadIdx.x, n_pairs)};
+    sort_block<SMALL_WAVES, 1>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
+                               output_indices, selected_experts_indices, rw.row_weights);
+}
+
+// More pairs in one launch: a block sorts 1024 of them, as above, and counts all the others by itself, with LDS atomics on eight
+// copies of the counts, so that the lanes of a wavefront that meet at one expert are few.  That is more work in all than count, scan
+// and scatter, but not for a compute unit: 64 pairs a thread at the line, against two more launches and the waits in each.  us, as
+// before (up to 8192 pairs one block of eight steps a wavefront, then three launches) -> so, operands in the caches / caches full of written data: 4096
+// pairs of 64 experts 8.7 -> 6.5 / 11.8 -> 9.1, 8000 14.7 -> 6.8 / 18.2 -> 9.6, 16384 17 -> 7.6 / 20.4 -> 10.4, 32768 17 -> 9.5 / 20.7 -> 12.5 (uneven
+// the same), 65536 17.9 -> 13.8 / 21.5 -> 17.1, 131072 21.3 -> 22.5 / 25.1 -> 26; 9003 of 12 13.2 -> 6.6 / 17 -> 9.2.
+constexpr int64_t SPREAD_PAIRS = 1 << 16;
+// VEC: selections in a load, 16 bytes of them where they are aligned
+template <typename TI, int VEC>
+__global__ __launch_bounds__(SMALL_WAVES * 64) void sort_spread_kernel(
+    const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
+    int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
+    int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
+    int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
+    constexpr int THREADS = SMALL_WAVES * 64, AHEAD = 8, CELLS = SORT_BLOCK_MAX_NR * SPREAD_COPIES;
+    typedef TI vec __attribute__((ext_vector_type(VEC)));
+    __shared__ int counts[2 * CELLS];   // of the pairs before this block's and of those after them
+    const int tid = threadIdx.x, first = blockIdx.x * THREADS, last = min(first + THREADS, n_pairs);
+    const TI e[1] = {selected_experts[min(first + tid, n_pairs - 1)]};
+    const float weight[1] = {rw.get(first + tid, n_pairs)};
+    for (int i = tid; i < 2 * CELLS; i += THREADS) counts[i] = 0;
+    __syncthreads();
+    const int n_vec = n_pairs / VEC, copy = tid % SPREAD_COPIES;
+    auto count = [&](TI value, int at) {
+        const long long v = static_cast<long long>(value);
+        if (v >= start && v < end && (at < first || at >= last))
+            atomicAdd(&counts[(at < first ? 0 : CELLS) + static_cast<int>(v - start) * SPREAD_COPIES + copy], 1);
+    };
+    for (int v0 = 0; v0 < n_vec; v0 += AHEAD * THREADS) {
+        vec q[AHEAD];
 #pragma unroll
-    for (int it = 0; it < ITERS; it++) e[it] = selected_experts[min(base + it * 64, n_pairs - 1)];
-    float weight[ITERS] = {};
-    if (rw.row_weights && rw.bf16) {
-        uint16_t bits[ITERS];
+        for (int u = 0; u < AHEAD; u++) q[u] = reinterpret_cast<const vec *>(selected_experts)[min(v0 + u * THREADS + tid, n_vec - 1)];
 #pragma unroll
-        for (int it = 0; it < ITERS; it++) bits[it] = static_cast<const uint16_t *>(rw.routing_weights)[min(base + it * 64, n_pairs - 1)];
+        for (int u = 0; u < AHEAD; u++) {
+            const int at = v0 + u * THREADS + tid;
+            if (at < n_vec)
 #pragma unroll
-        for (int it = 0; it < ITERS; it++) weight[it] = bf16_bits_to_f32(bits[it]);
-    } else if (rw.row_weights) {
-#pragma unroll
-        for (int it = 0; it < ITERS; it++) weight[it] = static_cast<const float *>(rw.routing_weights)[min(base + it * 64, n_pairs - 1)];
+                for (int x = 0; x < VEC; x++) count(q[u][x], at * VEC + x);
+        }
     }
-    sort_block<SMALL_WAVES, ITERS>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
-                                   output_indices, selected_experts_indices, rw.row_weights);
+    if (tid < n_pairs - n_vec * VEC) count(selected_experts[n_vec * VEC + tid], n_vec * VEC + tid);
+    // (sort_block's first barrier comes before it reads the counts)
+    sort_block<SMALL_WAVES, 1, true>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
+                                     output_indices, selected_experts_indices, rw.row_weights, {first, counts, counts + CELLS});
 }
 
 // ---- the reference's table layout [expert][column] ---------------------------------------------
@@ -378,22 +412,21 @@ int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, in
                     const RowWeights &rw = RowWeights()) {
     const int NR = expert_end_idx - expert_start_idx;
     const int64_t n_pairs = T * K;
-    if (n_pairs > 0 && n_pairs <= SMALL_PAIRS && NR <= SORT_BLOCK_MAX_NR) {
-#define OM_SMALL(TI, ITERS)                                                                                                     \
-    sort_small_kernel<TI, ITERS><<<1, SMALL_WAVES * 64, 0, st>>>(                                                               \
-        static_cast<const TI *>(selected_experts), static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR,          \
-        key_bits(NR), cum_token_counts, cum_expert_counts_ep, input_indices, output_indices, selected_experts_indices, rw)
-#define OM_SMALL_ITERS(TI)                                              \
-    do {                                                                \
-        if (n_pairs <= SMALL_WAVES * 64) OM_SMALL(TI, 1);               \
-        else if (n_pairs <= 2 * SMALL_WAVES * 64) OM_SMALL(TI, 2);      \
-        else if (n_pairs <= 4 * SMALL_WAVES * 64) OM_SMALL(TI, 4);      \
-        else OM_SMALL(TI, SMALL_MAX_ITERS);                             \
-    } while (0)
-        if (index_dtype == OM_I64) OM_SMALL_ITERS(int64_t);
-        else OM_SMALL_ITERS(int32_t);
-#undef OM_SMALL_ITERS
-#undef OM_SMALL
+    if (n_pairs > 0 && n_pairs <= SPREAD_PAIRS && NR <= SORT_BLOCK_MAX_NR) {
+        const unsigned blocks = static_cast<unsigned>((n_pairs + SMALL_PAIRS - 1) / SMALL_PAIRS);
+        auto sort = [&](const auto *experts) {
+            using TI = std::remove_const_t<std::remove_pointer_t<decltype(experts)>>;
+            auto launch = [&](auto kernel) {
+                kernel<<<blocks, SMALL_WAVES * 64, 0, st>>>(experts, static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR, key_bits(NR),
+                                                            cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
+                                                            selected_experts_indices, rw);
+            };
+            if (blocks == 1) launch(sort_small_kernel<TI>);
+            else if (om_aligned16(experts)) launch(sort_spread_kernel<TI, 16 / sizeof(TI)>);
+            else launch(sort_spread_kernel<TI, 1>);
+        };
+        if (index_dtype == OM_I64) sort(static_cast<const int64_t *>(selected_experts));
+        else sort(static_cast<const int32_t *>(selected_experts));
         return om_launch_status();
     }
     const int64_t NB = (n_pairs + SORT_CHUNK - 1) / SORT_CHUNK;

@@ -1,4 +1,4 @@
-// A stable counting sort of a few (token, k) pairs by local expert, by one block: what sort.hip's one-launch form and the router that
+// A stable counting sort of a few (token, k) pairs by local expert, by one block: what sort.hip's one-launch forms and the router that
 // sorts its own selections (route.hip) have in common.
 #pragma once
 #include "common.h"
@@ -32,26 +32,31 @@ inline int key_bits(int NR) {  // keys 0..NR (NR = "not local")
     return b;
 }
 
-// Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (up to 8 x 64)
-// pairs' keys, weights and ranks in registers between the passes.  A decode batch or a small training batch spends
-// nothing on bandwidth here, only on latencies: three launches of 4-17 us for 512 tokens x 8 (traced), one of 6 when the
-// caches are warm.  So no step waits for another's loads (ITERS, the 64-pair steps of a wavefront, is known to the compiler, and
-// pairs past the end are read as the last one), the rank of a pair within its expert comes from the counting pass, and
-// only that pass is a chain through LDS: 4096 pairs with cold caches, in a training step of 512 tokens of 64 experts, 15.2 ->
-// 9.8 us.  The line at 8192 pairs is where the single block's serial work (8 steps per wavefront) reaches what the three
-// launches take.
+// Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (ITERS x 64) pairs' keys, weights and ranks in
+// registers between the passes.  A decode batch or a small training batch spends nothing on bandwidth here, only on latencies.
+// So no step waits for another's loads (ITERS, the 64-pair steps of a wavefront, is known to the compiler, and pairs past the end are
+// read as the last one), the rank of a pair within its expert comes from the counting pass, and only that pass is a chain through LDS.
 constexpr int SORT_BLOCK_MAX_NR = 256;
+// Of a block that sorts some of the pairs: the first of them, and how many pairs of an expert come before the first and after the last, as
+// SPREAD_COPIES counts each that are added up here.
+constexpr int SPREAD_COPIES = 8;
+struct SpreadPart {
+    int first;
+    const int *before, *after;   // LDS, [expert][SPREAD_COPIES]
+};
 // Thread t of a wavefront's ITERS * 64 pairs (wavefront-major, step by step): e and weight; pairs past the end hold anything.
-template <int WAVES, int ITERS, typename TI>
+// SPREAD: the block sorts the pairs from part.first on, otherwise all of them.
+template <int WAVES, int ITERS, bool SPREAD = false, typename TI>
 __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&weight)[ITERS], int n_pairs, int K, int start, int end, int NR,
                                            int nbits, int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
                                            int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
-                                           int32_t *__restrict__ selected_experts_indices, float *__restrict__ row_weights) {
+                                           int32_t *__restrict__ selected_experts_indices, float *__restrict__ row_weights,
+                                           const SpreadPart part = {}) {
     __shared__ int off[WAVES][SORT_BLOCK_MAX_NR];   // counts, then the first position of a wavefront's rows of an expert
     __shared__ __attribute__((aligned(16))) int wave_hits[WAVES], chunk_total[SORT_BLOCK_MAX_NR / 64];
-    __shared__ int kept_total;
+    __shared__ int kept_total, kept_before[SORT_BLOCK_MAX_NR / 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int base = wv * ITERS * 64 + lane;
+    const int base = (SPREAD ? part.first : 0) + wv * ITERS * 64 + lane;
     volatile int *mine = off[wv];
     for (int i = lane; i < NR; i += 64) mine[i] = 0;
     __builtin_amdgcn_wave_barrier();
@@ -73,7 +78,7 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
     if (lane == 0) wave_hits[wv] = hits;
     __syncthreads();
     // thread e: expert e's total over the wavefronts, exclusive positions of the wavefronts within it
-    int total = 0, at[WAVES];
+    int total = 0, ahead = 0, at[WAVES];   // ahead: SPREAD, the expert's pairs before this block's
     if (tid < NR) {
 #pragma unroll
         for (int w = 0; w < WAVES; w++) at[w] = off[w][tid];
@@ -83,6 +88,18 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
             at[w] = total;
             total += c;
         }
+        if (SPREAD) {
+#pragma unroll
+            for (int x = 0; x < SPREAD_COPIES; x++) {
+                ahead += part.before[tid * SPREAD_COPIES + x];
+                total += part.after[tid * SPREAD_COPIES + x];
+            }
+            total += ahead;
+        }
+    }
+    if (SPREAD && tid < SORT_BLOCK_MAX_NR) {
+        const int kept = wave_sum_i(ahead);
+        if (lane == 0) kept_before[wv] = kept;
     }
     const int incl = wave_incl_scan(total, lane);
     if (tid < SORT_BLOCK_MAX_NR && lane == 63) chunk_total[wv] = incl;
@@ -92,11 +109,14 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
     for (int w = 0; w < SORT_BLOCK_MAX_NR / 64; w++) before += w < wv ? chunk_total[w] : 0;
     if (tid < NR) {
 #pragma unroll
-        for (int w = 0; w < WAVES; w++) off[w][tid] = before + at[w];
-        cum_token_counts[tid] = before;
+        for (int w = 0; w < WAVES; w++) off[w][tid] = before + ahead + at[w];
+        const bool first = !SPREAD || part.first == 0;
+        if (first) cum_token_counts[tid] = before;
         if (tid == NR - 1) {
-            cum_token_counts[NR] = before + total;
-            cum_expert_counts_ep[n_pairs / K] = before + total;
+            if (first) {
+                cum_token_counts[NR] = before + total;
+                cum_expert_counts_ep[n_pairs / K] = before + total;
+            }
             kept_total = before + total;
         }
     }
@@ -104,6 +124,10 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
     int oi_base = 0;
 #pragma unroll
     for (int w = 0; w < WAVES; w++) oi_base += w < wv ? wave_hits[w] : 0;
+    if (SPREAD) {
+#pragma unroll
+        for (int w = 0; w < SORT_BLOCK_MAX_NR / 64; w++) oi_base += kept_before[w];
+    }
     const int kept_all = kept_total;
 #pragma unroll
     for (int it = 0; it < ITERS; it++) {

@@ -174,3 +174,22 @@ def test_one_block_sort_at_its_edges(cuda, oracle_lib, T, N, K, start, end):
     """Up to 8192 pairs, around 1, 2, 4 and 8 steps a wavefront, experts around whole wavefronts."""
     for dt in (torch.float32, torch.bfloat16):
         test_weighted_sort_on_both_sides_of_the_one_block_line(cuda, oracle_lib, T, N, K, start, end, dt)
+
+
+@pytest.mark.parametrize("T,N,K,start,end", [
+    (1025, 64, 1, 0, 64), (9003, 12, 1, 0, 12), (8192, 64, 8, 0, 64), (65535, 9, 1, 2, 7), (65537, 9, 1, 2, 7), (4099, 256, 3, 0, 256),
+    (20000, 300, 2, 299, 300), (2049, 40, 5, 30, 40)])
+def test_sort_by_several_blocks_at_its_edges(cuda, oracle_lib, T, N, K, start, end):
+    """1025 to 65536 pairs, and the first count beyond; blocks without a local pair; no whole number of blocks or vectors; selections
+    that begin between 16-byte boundaries, in both index types: the arrays of the aligned ones."""
+    test_weighted_sort_on_both_sides_of_the_one_block_line(cuda, oracle_lib, T, N, K, start, end, torch.float32)
+    se = routed_experts(T, N, K, seed=T + N, skew=0.7)
+    ref = oracle_lib.index_construction(se.numpy(), end - start, start, end, tokens_per_thread=1)
+    TR = ref["num_routed_tokens"]
+    for dt in (torch.int64, torch.int32):
+        shifted = torch.empty(T * K + 1, dtype=dt, device=cuda)[1:].view(T, K)
+        shifted.copy_(se)
+        cum, cum_ep, ii, oi, si = _gpu_sort(shifted, start, end, cuda)
+        assert np.array_equal(cum, ref["cum_token_counts"]) and np.array_equal(cum_ep, ref["cum_expert_counts_ep"])
+        assert np.array_equal(ii[:TR], ref["input_indices"]) and np.array_equal(oi[:TR], ref["output_indices"])
+        assert np.array_equal(si[:TR], ref["selected_experts_indices"])
