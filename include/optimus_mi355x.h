@@ -666,6 +666,13 @@ int om_merged_mlp_gate_up_fwd_weighted_dense(const void *x, const int32_t *x_row
                                              void *g, void *u, void *h, const int32_t *cum_token_counts,
                                              int64_t rows, int64_t expected_rows, int G, int I, int H,
                                              int64_t w_stride, const om_dense_expert *dense, void *stream);
+/* om_merged_mlp_hidden_fwd: only the h of the gate+up products, the same bits, where no backward follows that needs g and u:
+ * gathered with x_rows, weighted with row_weights (which needs x_rows), beside a dense expert (which needs both; its c[0]
+ * and c[1] are not used); each of the three may be NULL.  rows and expected_rows as in the _bound forms.       */
+int om_merged_mlp_hidden_fwd(const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate, const void *w_up,
+                             const float *row_weights, void *h, const int32_t *cum_token_counts, int64_t rows,
+                             int64_t expected_rows, int G, int I, int H, int64_t w_stride, const om_dense_expert *dense,
+                             void *stream);
 int om_grouped_gemm_fwd_dense(const void *input, const void *weight, void *output,
                               const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int N,
                               int K, int64_t w_stride, const om_dense_expert *dense, void *stream);

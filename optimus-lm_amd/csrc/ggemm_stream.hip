@@ -30,7 +30,7 @@ __device__ __attribute__((aligned(16))) const uint16_t zero_chunk[8] = {};
 struct StreamParams {
     const uint16_t *x;
     const uint16_t *w[2];      // SWIGLU: gate and up; else w[0] twice
-    uint16_t *out[3];          // SWIGLU: g, u, h; else out[0]
+    uint16_t *out[3];          // SWIGLU: g, u (or neither), h; else out[0]
     const int32_t *cum;
     const int32_t *row_index;  // != null: sorted row r is row row_index[r] of x
     const float *row_scale;    // != null: h is scaled by it
@@ -149,8 +149,10 @@ __device__ __forceinline__ void stream_tile(const StreamParams &p, int expert, i
                 const int64_t o = static_cast<int64_t>(row) * p.n_cols + n0 + col;
                 float h = (g * fast_sigmoid(g)) * u;
                 if (p.row_scale) h *= p.row_scale[row];
-                p.out[0][o] = f32_to_bf16_bits(g);
-                p.out[1][o] = f32_to_bf16_bits(u);
+                if (p.out[0]) {
+                    p.out[0][o] = f32_to_bf16_bits(g);
+                    p.out[1][o] = f32_to_bf16_bits(u);
+                }
                 p.out[2][o] = f32_to_bf16_bits(h);
             }
         } else {

@@ -412,16 +412,20 @@ void gemm_dtype(const Tensor &a, const Tensor &b, const Tensor &c) {
 const float *fp(const Tensor &t) { return static_cast<const float *>(ptr(t)); }
 float *fpm(const Tensor &t) { return static_cast<float *>(ptr(t)); }
 
-// y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment; with x_rows the MLP input is x[x_rows]
+// y = (silu(x Wg^T) * (x Wu^T)) Wd^T per expert segment; with x_rows the MLP input is x[x_rows].  `keep`: whether a backward may
+// follow, which needs g and u.
 Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const int32_t *cum, const int32_t *x_rows,
-                      int64_t rows, MlpState &s) {
+                      int64_t rows, MlpState &s, bool keep = true) {
     require_mlp_operands(x, w);
     require_device(x);
     gemm_dtype(x, w.gate, w.up);
     gemm_dtype(x, w.gate, w.down);
     const int64_t G = w.G(), I = w.I(), H = w.H();
-    s.g = make({rows, I}, x);
-    s.u = make({rows, I}, x);
+    keep = keep || x.scalar_type() == at::kFloat;
+    if (keep) {
+        s.g = make({rows, I}, x);
+        s.u = make({rows, I}, x);
+    }
     s.h = make({rows, I}, x);
     Tensor y = make({rows, H}, x);
     ProfiledScope scope(c, "1moeblock--7gmlp_fwd");
@@ -432,7 +436,10 @@ Tensor merged_forward(const Call &c, const Tensor &x, const MlpWeights &w, const
         return y;
     }
     const int64_t pitch = shared_pitch(w);
-    if (x_rows && rows > 0)
+    if (!keep)
+        OM(c, om_merged_mlp_hidden_fwd, ptr(x), rows ? x_rows : nullptr, x.size(0), ptr(w.gate), ptr(w.up), nullptr, ptr(s.h), cum, rows,
+           rows, G, I, H, pitch, nullptr, c.stream);
+    else if (x_rows && rows > 0)
         OM(c, om_merged_mlp_gate_up_fwd_gathered, ptr(x), x_rows, x.size(0), ptr(w.gate), ptr(w.up), ptr(s.g), ptr(s.u),
            ptr(s.h), cum, rows, G, I, H, pitch, c.stream);
     else
@@ -562,7 +569,7 @@ om_dense_expert dense_expert(std::array<const Tensor *, 2> a, std::array<const T
 // The routed half of a bf16 block: gather, weighted SwiGLU MLP, unweighted sum of a token's rows.  `along`: and the shared
 // expert, whose output is the residual.
 Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const Index &ix, const MlpWeights &w,
-                      Tensor residual, MlpState &s, Tensor &row_weights, Alongside *along = nullptr) {
+                      Tensor residual, MlpState &s, Tensor &row_weights, Alongside *along = nullptr, bool keep = true) {
     require_mlp_operands(x, w);
     if (rw.dim() != 2 || rw.size(0) != x.size(0)) throw NativeError("routing weights: expected [tokens, top_k]");
     if (residual.defined()) {
@@ -578,8 +585,10 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
     require_bf16(w.down);
     const int64_t T = x.size(0), H = x.size(1), K = rw.size(1), rows = ix.rows, G = w.G(), I = w.I();
     const int64_t pitch = shared_pitch(w);
-    s.g = make({rows, I}, x);
-    s.u = make({rows, I}, x);
+    if (keep) {
+        s.g = make({rows, I}, x);
+        s.u = make({rows, I}, x);
+    }
     s.h = make({rows, I}, x);
     Tensor y = make({rows, H}, x), final = make({T, H}, x);
     {
@@ -592,16 +601,26 @@ Tensor routed_forward(const Call &c, const Tensor &x, const Tensor &rw, const In
         }
         if (along) {
             MlpState &d = along->s;
-            for (Tensor *t : {&d.g, &d.u, &d.h}) *t = make({T, I}, x);
+            if (keep) {
+                d.g = make({T, I}, x);
+                d.u = make({T, I}, x);
+            }
+            d.h = make({T, I}, x);
             residual = along->y = make({T, H}, x);
             const om_dense_expert up = dense_expert({&x, nullptr}, {&along->w.gate, &along->w.up}, {&d.g, &d.u, &d.h}, d, T);
-            OM(c, om_merged_mlp_gate_up_fwd_weighted_dense, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g), ptr(s.u),
+            if (!keep)
+                OM(c, om_merged_mlp_hidden_fwd, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.h), ix.cum, rows,
+                   ix.to_choose_by(), G, I, H, pitch, &up, c.stream);
+            else OM(c, om_merged_mlp_gate_up_fwd_weighted_dense, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g), ptr(s.u),
                ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, &up, c.stream);
             const om_dense_expert down = dense_expert({&d.h, nullptr}, {&along->w.down, nullptr}, {&along->y, nullptr, nullptr}, d, T);
             OM(c, om_grouped_gemm_fwd_dense, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
                expert_stride(w.down), &down, c.stream);
         } else {
-            OM_BOUND(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
+            if (!keep)
+                OM(c, om_merged_mlp_hidden_fwd, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.h), ix.cum, rows,
+                   ix.to_choose_by(), G, I, H, pitch, nullptr, c.stream);
+            else OM_BOUND(c, om_merged_mlp_gate_up_fwd_weighted, ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), weights, ptr(s.g),
                      ptr(s.u), ptr(s.h), ix.cum, rows, ix.to_choose_by(), G, I, H, pitch, c.stream);
             OM_BOUND(c, om_grouped_gemm_fwd, ptr(s.h), ptr(w.down), ptr(y), ix.cum, rows, ix.to_choose_by(), G, H, I,
                      expert_stride(w.down), c.stream);
@@ -1197,6 +1216,7 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
     MlpWeights w, ws;
     MlpState s, ss;
     Tensor row_weights, final, xc, rwc;
+    const bool keep = any_requires_grad(inputs);
     {
         at::AutoDispatchBelowADInplaceOrView below;
         w = weights_of(routed, merged, G);
@@ -1210,12 +1230,12 @@ Tensor routed_experts(const Call &c, Tensor x, Tensor rw, Index ix, const Tensor
             // (the host waits for the rows behind the shared expert's kernels, where it has to)
             together = !after_shared && Alongside::rides(ws, w, ix.to_choose_by(), xc.size(0), OM_DENSE_GATE_UP | OM_DENSE_DOWN);
             if (together) require_shared_operands(xc, ws, one, ss);
-            else residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss);
+            else residual = merged_forward(c, xc, ws, iptr(one), nullptr, xc.size(0), ss, keep);
         }
         if (after_shared) after_shared(ix);
-        final = routed_forward(c, xc, rwc, ix, w, residual, s, row_weights, together ? &along : nullptr);
+        final = routed_forward(c, xc, rwc, ix, w, residual, s, row_weights, together ? &along : nullptr, keep);
     }
-    if (any_requires_grad(inputs)) {
+    if (keep) {
         auto node = make_node<RoutedNode>(inputs);
         node->vars.reserve(21);
         node->save(xc.is_same(x) ? x : xc);

@@ -177,6 +177,8 @@ SIGNATURES = {
     "om_merged_mlp_dense_rides": (c_int, [c_i64, c_int, c_int, c_int, c_i64]),
     "om_merged_mlp_dense_products": (c_int, [c_i64, c_int, c_int, c_int, c_i64]),
     "om_grouped_gemm_fwd_dense": (c_int, [c_void_p] * 4 + [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_void_p, c_void_p]),
+    "om_merged_mlp_hidden_fwd": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 5 + [c_i64, c_i64, c_int, c_int, c_int, c_i64,
+                                                                                        c_void_p, c_void_p]),
     "om_merged_mlp_gate_up_fwd_weighted_dense": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 7 +
                                                  [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_void_p, c_void_p]),
     "om_merged_mlp_down_dgrad_weighted_dense": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 8 +

@@ -883,3 +883,52 @@ def test_products_over_a_bound_of_the_rows(cuda, expected, N, K):
             assert ((got.float() - ref).abs() <= ref.abs() * rel + 1e-6 * k ** 0.5 * factor).all(), (name, e)
         terms = dh * gb * sig * ub
         assert ((dot[:, s].sum(0) - terms.sum(1)).abs() <= (2 ** -8 + 1e-5) * terms.abs().sum(1) + 1e-6).all(), e
+
+
+# rows an expert: streamed, 128x128 tiles with remainders and extents that no tile divides, 256x256 tiles with partial ones
+@pytest.mark.parametrize("rows_e,I,H", [((1, 0, 3), 64, 128), ((1, 0, 3), 72, 200), ((140, 0, 129, 64), 712, 200),
+                                        ((300, 97, 256, 0, 513, 400, 330, 290), 2048, 512)])
+@pytest.mark.parametrize("form", ["plain", "gathered", "weighted"])
+def test_hidden_alone_is_the_h_of_the_full_product(cuda, rows_e, I, H, form):
+    """om_merged_mlp_hidden_fwd: the bits of h, for each kernel that can take the product, and no g and u."""
+    from optimus import _native as n
+    L, P, G, rows, T = n.lib(), n.ptr, len(rows_e), sum(rows_e), 77
+    gen = torch.Generator().manual_seed(rows)
+    bf = lambda *s: torch.randn(*s, generator=gen).mul(0.2).bfloat16().to(cuda)
+    x = bf(rows if form == "plain" else T, H)
+    wg, wu = bf(G, I, H), bf(G, I, H)
+    cum = torch.tensor([0] + list(torch.tensor(rows_e).cumsum(0)), dtype=torch.int32, device=cuda)
+    index = torch.randint(0, T, (rows,), generator=gen, dtype=torch.int32).to(cuda)
+    scale = torch.rand(rows, generator=gen).to(cuda)
+    out = [torch.full((rows, I), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(4)]
+    g, u, h, alone = out
+    args = (rows, G, I, H, 0, n.stream())
+    if form == "plain":
+        n.check(L.om_merged_mlp_gate_up_fwd(P(x), P(wg), P(wu), P(g), P(u), P(h), P(cum), *args), "full")
+    elif form == "gathered":
+        n.check(L.om_merged_mlp_gate_up_fwd_gathered(P(x), P(index), T, P(wg), P(wu), P(g), P(u), P(h), P(cum), *args), "full")
+    else:
+        n.check(L.om_merged_mlp_gate_up_fwd_weighted(P(x), P(index), T, P(wg), P(wu), P(scale), P(g), P(u), P(h), P(cum), *args), "full")
+    n.check(L.om_merged_mlp_hidden_fwd(P(x), None if form == "plain" else P(index), T, P(wg), P(wu), P(scale) if form == "weighted" else None,
+                                       P(alone), P(cum), rows, rows, G, I, H, 0, None, n.stream()), "alone")
+    torch.cuda.synchronize()
+    assert torch.equal(alone, h) and not torch.equal(g, h)
+    assert L.om_merged_mlp_hidden_fwd(P(x), None, T, P(wg), P(wu), P(scale), P(alone), P(cum), rows, rows, G, I, H, 0, None,
+                                      n.stream()) == L.om_merged_mlp_gate_up_fwd(P(x), P(wg), P(wu), None, P(u), P(h), P(cum), *args) != 0
+
+
+@pytest.mark.parametrize("tokens", [1, 37, 200, 4000])
+@pytest.mark.parametrize("parallel", [1, 4])
+def test_layer_without_gradients_gives_the_same_bits(cuda, tokens, parallel):
+    """A layer with a shared expert, alone or in the routed experts' launch, and a window of the experts: with and without autograd."""
+    from optimus.models.deepseek_v3.modeling_deepseek_v3 import DeepseekV3ParallelMoE
+    from optimus.models.deepseek_v3.configuration_deepseek_v3 import DeepseekV3ParallelConfig
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    cfg = DeepseekV3ParallelConfig(hidden_size=256, moe_intermediate_size=264, n_routed_experts=16, n_group=4, topk_group=2,
+                                   num_experts_per_tok=4, expert_parallelism=parallel)
+    torch.manual_seed(tokens)
+    block = DeepseekV3ParallelMoE(cfg, ParallelDpPpEpTpMapper(expert_parallelism=parallel, rank=0)).to(torch.bfloat16).to(cuda)
+    x = torch.randn(tokens, 1, 256, device=cuda, dtype=torch.bfloat16)
+    with torch.no_grad():
+        alone = block(x)
+    assert torch.equal(alone, block(x).detach())
