@@ -304,6 +304,13 @@ int om_router_balance_stats(const void *logits, int logits_dtype, int64_t T, int
                             int64_t workspace_bytes, void *stream);
 int om_router_balance_bwd(const void *logits, int logits_dtype, const float *prob_grad, int64_t T,
                           int N, void *dlogits, void *stream);
+/* One layer's loss in the statistics' launches: loss [1] = scale * sum_e (count[e]/T) * (prob_sum[e]/T), with scale the
+ * number of experts (optimus/models/common/ral_functions.py:6-15); count [N] is what om_router_balance_loss_bwd needs, whose
+ * loss_grad [1] is the loss's gradient on the device.  workspace: om_router_balance_workspace_bytes.  T >= 1.  */
+int om_router_balance_loss(const void *logits, int logits_dtype, int64_t T, int N, int K, double scale, float *count,
+                           float *loss, void *workspace, int64_t workspace_bytes, void *stream);
+int om_router_balance_loss_bwd(const void *logits, int logits_dtype, const float *count, const float *loss_grad,
+                               double scale, int64_t T, int N, void *dlogits, void *stream);
 
 /* om_route_sigmoid_group_topk replaces DeepseekV3ParallelTopkRouter.get_topk_indices and
  *   the weight computation of its forward,

@@ -992,7 +992,7 @@ int launch_gate(const void *x, const void *wg, int64_t T, int H, int N, int K, i
 // What bounds both is a chain of latencies, not the 4 MB of logits: with four wavefronts a block took 16
 // softmax and top-K selections one after another (46 us at 16384 tokens, 64 experts), and one thread per
 // expert then added 256 rows with one load in flight (66 us).  Sixteen wavefronts per block and 16 loads in
-// flight: 17.5 + 8.6 us.
+// flight: 17.5 us and balance_sums'.
 constexpr int BAL_TOKENS = 64, BAL_WAVES = 16;
 template <int PER, typename T>
 __global__ __launch_bounds__(BAL_WAVES * 64) void balance_stats_kernel(const T *__restrict__ logits,
@@ -1043,46 +1043,87 @@ __global__ __launch_bounds__(BAL_WAVES * 64) void balance_stats_kernel(const T *
     }
 }
 
-__global__ __launch_bounds__(64) void balance_reduce_kernel(const float *__restrict__ part_prob,
-                                                            const float *__restrict__ part_count,
-                                                            int n_blocks, int N,
-                                                            float *__restrict__ prob_sum,
-                                                            float *__restrict__ count) {
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    if (i >= N) return;
+// The partial rows of 64 experts: a sixteenth of them to each wavefront, 16 loads in flight, then the wavefronts' sums in a fixed
+// order; lane i of wavefront 0 has expert i's.  (One wavefront for all: 256 rows 8.6 us -> 4.3.)
+__device__ __forceinline__ void balance_sums(const float *part_prob, const float *part_count, int n_blocks, int N, int i, float &prob, float &count) {
+    __shared__ float lds_p[BAL_WAVES][64];
+    __shared__ double lds_c[BAL_WAVES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float ps = 0.0f;
     // a block's partial is a sum of at most BAL_TOKENS token weights (whole numbers for 0/1 weights
     // and without weights); adding the partials in double keeps whole-number counts exact at any
     // token count (a hot expert can exceed 2^24 tokens), one rounding to float at the end
     double c = 0.0;
-    int b = 0;
-    for (; b + 16 <= n_blocks; b += 16) {
-        float p[16], q[16];
+    if (i < N) {
+        int b = static_cast<int>(static_cast<int64_t>(n_blocks) * wave / BAL_WAVES);
+        const int end = static_cast<int>(static_cast<int64_t>(n_blocks) * (wave + 1) / BAL_WAVES);
+        for (; b + 16 <= end; b += 16) {
+            float p[16], q[16];
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            p[u] = part_prob[static_cast<int64_t>(b + u) * N + i];
-            q[u] = part_count[static_cast<int64_t>(b + u) * N + i];
+            for (int u = 0; u < 16; u++) {
+                p[u] = part_prob[static_cast<int64_t>(b + u) * N + i];
+                q[u] = part_count[static_cast<int64_t>(b + u) * N + i];
+            }
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                ps += p[u];
+                c += static_cast<double>(q[u]);
+            }
         }
-#pragma unroll
-        for (int u = 0; u < 16; u++) {
-            ps += p[u];
-            c += static_cast<double>(q[u]);
+        for (; b < end; b++) {
+            ps += part_prob[static_cast<int64_t>(b) * N + i];
+            c += static_cast<double>(part_count[static_cast<int64_t>(b) * N + i]);
         }
     }
-    for (; b < n_blocks; b++) {
-        ps += part_prob[static_cast<int64_t>(b) * N + i];
-        c += static_cast<double>(part_count[static_cast<int64_t>(b) * N + i]);
+    __syncthreads();   // (a group of experts before this one has been read)
+    lds_p[wave][lane] = ps;
+    lds_c[wave][lane] = c;
+    __syncthreads();
+    if (wave == 0) {
+        for (int w = 1; w < BAL_WAVES; w++) {
+            ps += lds_p[w][lane];
+            c += lds_c[w][lane];
+        }
     }
-    prob_sum[i] = ps;
-    count[i] = static_cast<float>(c);
+    prob = ps;
+    count = static_cast<float>(c);
+}
+__global__ __launch_bounds__(BAL_WAVES * 64) void balance_reduce_kernel(const float *__restrict__ part_prob, const float *__restrict__ part_count,
+                                                                        int n_blocks, int N, float *__restrict__ prob_sum,
+                                                                        float *__restrict__ count) {
+    const int i = blockIdx.x * 64 + (threadIdx.x & 63);
+    float p, c;
+    balance_sums(part_prob, part_count, n_blocks, N, i, p, c);
+    if (threadIdx.x < 64 && i < N) {
+        prob_sum[i] = p;
+        count[i] = c;
+    }
+}
+// The same, and loss = scale * sum over the experts of (count / T) * (prob_sum / T): one block.
+__global__ __launch_bounds__(BAL_WAVES * 64) void balance_loss_kernel(const float *__restrict__ part_prob, const float *__restrict__ part_count,
+                                                                      int n_blocks, int64_t Tn, int N, float scale, float *__restrict__ count,
+                                                                      float *__restrict__ loss) {
+    const float t = static_cast<float>(Tn);
+    float sum = 0.0f;
+    for (int e0 = 0; e0 < N; e0 += 64) {
+        const int i = e0 + (threadIdx.x & 63);
+        float p, c;
+        balance_sums(part_prob, part_count, n_blocks, N, i, p, c);
+        if (i < N) sum += (c / t) * (p / t);
+        if (threadIdx.x < 64 && i < N) count[i] = c;
+    }
+    sum = wave_sum(sum);
+    if (threadIdx.x == 0) *loss = sum * scale;
 }
 
 // dlogits[t,i] = p_i * (g_i - sum_j p_j g_j): the softmax backward of sum_i g_i * p[t,i].
-template <int PER, typename T>
+// LOSS: g holds the counts, and the gradient of the probabilities' sums is that of the loss: grad * scale * (count / T) / T.
+template <int PER, typename T, bool LOSS = false>
 __global__ __launch_bounds__(256) void balance_bwd_kernel(const T *__restrict__ logits,
                                                           const float *__restrict__ g,
                                                           const float *__restrict__ token_weight,
-                                                          int64_t Tn, int N, T *__restrict__ dlogits) {
+                                                          int64_t Tn, int N, T *__restrict__ dlogits,
+                                                          const float *__restrict__ grad = nullptr, float scale = 0.0f) {
     const int lane = threadIdx.x & 63;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * TOKENS_PER_BLOCK + (threadIdx.x >> 6);
     if (t >= Tn) return;
@@ -1093,6 +1134,7 @@ __global__ __launch_bounds__(256) void balance_bwd_kernel(const T *__restrict__ 
     for (int j = 0; j < PER; j++) {
         const int i = lane + 64 * j;
         gv[j] = (i < N) ? g[i] : 0.0f;
+        if (LOSS) gv[j] = ((*grad * scale) * (gv[j] / static_cast<float>(Tn))) / static_cast<float>(Tn);
         dot += p[j] * gv[j];
     }
     dot = wave_sum(dot);
@@ -1433,15 +1475,10 @@ extern "C" int64_t om_router_balance_workspace_bytes(int64_t T, int N) {
     return blocks * N * 8;   // one float and one int per (block, expert)
 }
 
-extern "C" int om_router_balance_stats_masked(const void *logits, int logits_dtype,
-                                              const float *token_weight, int64_t T, int N, int K,
-                                              float *prob_sum, float *count, void *workspace,
-                                              int64_t workspace_bytes, void *stream) {
-    if (logits_dtype != OM_F32 && logits_dtype != OM_BF16) return OM_ERR_DTYPE;
-    if (T < 1 || N < 1 || N > 512 || K < 1 || K > N || K > 64 || T > 0x7fffffffLL) return OM_ERR_SHAPE;
-    if (!logits || !prob_sum || !count || !workspace) return OM_ERR_NULL;
-    if (workspace_bytes < om_router_balance_workspace_bytes(T, N)) return OM_ERR_WORKSPACE;
-    hipStream_t st = om_stream(stream);
+namespace {
+struct BalancePartials { const float *prob, *count; int blocks; };
+BalancePartials balance_partials(const void *logits, int logits_dtype, const float *token_weight, int64_t T, int N, int K, void *workspace,
+                                 hipStream_t st) {
     const int nb = static_cast<int>((T + BAL_TOKENS - 1) / BAL_TOKENS);
     float *pp = static_cast<float *>(workspace);
     float *pc = pp + static_cast<int64_t>(nb) * N;
@@ -1452,7 +1489,21 @@ extern "C" int om_router_balance_stats_masked(const void *logits, int logits_dty
         OM_DISPATCH_PER(N, (balance_stats_kernel<PER, uint16_t><<<nb, BAL_WAVES * 64, 0, st>>>(
                                static_cast<const uint16_t *>(logits), token_weight, T, N, K, pp, pc)));
     }
-    balance_reduce_kernel<<<(N + 63) / 64, 64, 0, st>>>(pp, pc, nb, N, prob_sum, count);
+    return {pp, pc, nb};
+}
+}  // namespace
+
+extern "C" int om_router_balance_stats_masked(const void *logits, int logits_dtype,
+                                              const float *token_weight, int64_t T, int N, int K,
+                                              float *prob_sum, float *count, void *workspace,
+                                              int64_t workspace_bytes, void *stream) {
+    if (logits_dtype != OM_F32 && logits_dtype != OM_BF16) return OM_ERR_DTYPE;
+    if (T < 1 || N < 1 || N > 512 || K < 1 || K > N || K > 64 || T > 0x7fffffffLL) return OM_ERR_SHAPE;
+    if (!logits || !prob_sum || !count || !workspace) return OM_ERR_NULL;
+    if (workspace_bytes < om_router_balance_workspace_bytes(T, N)) return OM_ERR_WORKSPACE;
+    hipStream_t st = om_stream(stream);
+    const BalancePartials p = balance_partials(logits, logits_dtype, token_weight, T, N, K, workspace, st);
+    balance_reduce_kernel<<<(N + 63) / 64, BAL_WAVES * 64, 0, st>>>(p.prob, p.count, p.blocks, N, prob_sum, count);
     return om_launch_status();
 }
 
@@ -1480,6 +1531,35 @@ extern "C" int om_router_balance_bwd_masked(const void *logits, int logits_dtype
         OM_DISPATCH_PER(N, (balance_bwd_kernel<PER, uint16_t><<<nb, 256, 0, st>>>(
                                static_cast<const uint16_t *>(logits), prob_grad, token_weight, T, N,
                                static_cast<uint16_t *>(dlogits))));
+    }
+    return om_launch_status();
+}
+
+extern "C" int om_router_balance_loss(const void *logits, int logits_dtype, int64_t T, int N, int K, double scale, float *count, float *loss,
+                                      void *workspace, int64_t workspace_bytes, void *stream) {
+    if (logits_dtype != OM_F32 && logits_dtype != OM_BF16) return OM_ERR_DTYPE;
+    if (T < 1 || N < 1 || N > 512 || K < 1 || K > N || K > 64 || T > 0x7fffffffLL) return OM_ERR_SHAPE;
+    if (!logits || !count || !loss || !workspace) return OM_ERR_NULL;
+    if (workspace_bytes < om_router_balance_workspace_bytes(T, N)) return OM_ERR_WORKSPACE;
+    hipStream_t st = om_stream(stream);
+    const BalancePartials p = balance_partials(logits, logits_dtype, nullptr, T, N, K, workspace, st);
+    balance_loss_kernel<<<1, BAL_WAVES * 64, 0, st>>>(p.prob, p.count, p.blocks, T, N, static_cast<float>(scale), count, loss);
+    return om_launch_status();
+}
+
+extern "C" int om_router_balance_loss_bwd(const void *logits, int logits_dtype, const float *count, const float *loss_grad, double scale,
+                                          int64_t T, int N, void *dlogits, void *stream) {
+    if (logits_dtype != OM_F32 && logits_dtype != OM_BF16) return OM_ERR_DTYPE;
+    if (T < 1 || N < 1 || N > 512 || T > 0x7fffffffLL) return OM_ERR_SHAPE;
+    if (!logits || !count || !loss_grad || !dlogits) return OM_ERR_NULL;
+    hipStream_t st = om_stream(stream);
+    const float s = static_cast<float>(scale);
+    if (logits_dtype == OM_F32) {
+        OM_DISPATCH_PER(N, (balance_bwd_kernel<PER, float, true><<<token_blocks(T), 256, 0, st>>>(
+                               static_cast<const float *>(logits), count, nullptr, T, N, static_cast<float *>(dlogits), loss_grad, s)));
+    } else {
+        OM_DISPATCH_PER(N, (balance_bwd_kernel<PER, uint16_t, true><<<token_blocks(T), 256, 0, st>>>(
+                               static_cast<const uint16_t *>(logits), count, nullptr, T, N, static_cast<uint16_t *>(dlogits), loss_grad, s)));
     }
     return om_launch_status();
 }

@@ -48,6 +48,37 @@ class RouterBalanceStatsFunction(torch.autograd.Function):
         return dlogits, None, None
 
 
+class RouterBalanceLossFunction(torch.autograd.Function):
+    """num_experts * sum_e (count[e]/T) * (prob_sum[e]/T) of one layer's logits [T,N], T >= 1, with the mean and the product in the
+    launches of the statistics: as tensor operations they were eleven more launches, forward and backward."""
+
+    @staticmethod
+    def forward(ctx, logits, top_k, num_experts):
+        _n.require_cuda_contiguous(logits)
+        T, N = logits.shape
+        count = torch.empty(N, dtype=torch.float32, device=logits.device)
+        loss = torch.empty((), dtype=torch.float32, device=logits.device)     # (a tensor of its own: a caller may scale it in place)
+        ws_bytes = _n.lib().om_router_balance_workspace_bytes(T, N)
+        ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=logits.device)
+        _n.check(_n.lib().om_router_balance_loss(_n.ptr(logits), _n.dtype_code(logits), T, N, int(top_k), float(num_experts),
+                                                 _n.ptr(count), _n.ptr(loss), _n.ptr(ws), ws_bytes, _n.stream()),
+                 "om_router_balance_loss")
+        ctx.save_for_backward(logits, count)
+        ctx.num_experts = float(num_experts)
+        return loss
+
+    @staticmethod
+    def backward(ctx, g_loss):
+        logits, count = ctx.saved_tensors
+        T, N = logits.shape
+        g = g_loss.float().contiguous()
+        dlogits = torch.empty_like(logits)
+        _n.check(_n.lib().om_router_balance_loss_bwd(_n.ptr(logits), _n.dtype_code(logits), _n.ptr(count), _n.ptr(g),
+                                                     ctx.num_experts, T, N, _n.ptr(dlogits), _n.stream()),
+                 "om_router_balance_loss_bwd")
+        return dlogits, None, None
+
+
 def _layer_sums(gate_logits, top_k, token_weight=None):
     """Per layer: (prob_sum, count, weight of the layer's tokens)."""
     out = []
@@ -64,6 +95,8 @@ def _layer_sums(gate_logits, top_k, token_weight=None):
 def single_input_load_balancing_loss_func(gate_logits, num_experts, top_k):
     """Reference ral_functions.py:6-15 (one layer's logits [T,N])."""
     T = gate_logits.shape[0]
+    if T > 0 and isinstance(num_experts, (int, float)):
+        return RouterBalanceLossFunction.apply(gate_logits.contiguous(), top_k, num_experts)
     prob_sum, count = RouterBalanceStatsFunction.apply(gate_logits.contiguous(), top_k, None)
     return torch.sum((count / T) * (prob_sum / T)) * num_experts
 

@@ -735,3 +735,28 @@ def test_few_tokens_have_the_logits_of_many(cuda, H, N):
     for T in (1, 16, 17, 512):
         _, _, few, _ = n.host().route_softmax(x[:T], w, 1, False, torch.bfloat16, False, False)
         assert torch.equal(few, many[:T])
+
+
+# one token, a partial block of 64, more partial rows than a round of loads a wavefront, several groups of 64 experts
+@pytest.mark.parametrize("T,N,K", [(1, 8, 2), (63, 64, 8), (1025, 100, 5), (4097, 512, 8), (16384 + 64 * 17, 64, 8), (300, 2, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_balance_loss_in_one_function_is_the_composed_one(cuda, T, N, K, dtype):
+    """single_input_load_balancing_loss_func against the same expression of RouterBalanceStatsFunction's sums, loss and gradient."""
+    from optimus.models.common.ral_functions import RouterBalanceStatsFunction, single_input_load_balancing_loss_func
+    base = _valid_logits(T, N, K, seed=T + N).to(dtype).to(cuda)
+    a, b = base.clone().requires_grad_(True), base.clone().requires_grad_(True)
+    loss = single_input_load_balancing_loss_func(a, N, K)
+    prob_sum, count = RouterBalanceStatsFunction.apply(b, K, None)
+    want = torch.sum((count / T) * (prob_sum / T)) * N
+    # N products' sum in another order, and one rounding of each of them
+    assert loss.shape == () and loss.dtype == torch.float32
+    assert abs(float(loss.detach().double() - want.detach().double())) <= (N + 4) * 2.0 ** -24 * float(want.detach())
+    (want * 0.01).backward()
+    loss *= 0.01                                   # in place, as a caller may
+    loss.backward()
+    # dlogits = p (g - sum p g), where g = 0.01 N (count / T) / T: the tensor expression multiplies by 1 / T, so each of g and the sum is
+    # off by at most 2 + 2 roundings of g's size, which the difference may cancel down to; in bf16 one rounding of the result
+    p = torch.softmax(base.float(), 1).max()
+    g = 0.01 * N * float(count.max()) / T / T
+    bound = float(p) * g * 2 * 4 * 2.0 ** -24 + (2.0 ** -8 * float(b.grad.abs().max()) if dtype == torch.bfloat16 else 0.0)
+    assert float((a.grad.float() - b.grad.float()).abs().max()) <= bound
