@@ -67,6 +67,8 @@ GEMM_ENTRY_PRODUCTS = {     # C-ABI entry -> number of [rows x N x K] products p
     "om_grouped_gemm_wgrad_accumulate": 1, "om_grouped_gemm_wgrad_gathered_accumulate": 1,
     "om_grouped_gemm_wgrad_gathered_out_accumulate": 1,
     "om_grouped_gemm_wgrad_merged": 3, "om_grouped_gemm_wgrad_merged_accumulate": 3,
+    "om_grouped_gemm_wgrad_merged_dgrad": 5, "om_grouped_gemm_wgrad_merged_dgrad_accumulate": 5,
+    "om_merged_mlp_hidden_fwd": 2,
     # with a shared expert's rows as well
     "om_merged_mlp_gate_up_fwd_weighted_dense": 2, "om_grouped_gemm_fwd_dense": 1,
     "om_merged_mlp_down_dgrad_weighted_dense": 1, "om_merged_mlp_gate_up_dgrad_dense": 2,

@@ -689,6 +689,18 @@ int om_merged_mlp_down_dgrad_weighted_dense(const void *dy, const int32_t *dy_ro
                                             const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
                                             int G, int I, int H, int64_t w_stride, const om_dense_expert *dense,
                                             void *stream);
+/* om_grouped_gemm_wgrad_merged_dgrad(_accumulate): om_grouped_gemm_wgrad_merged(_accumulate)_bound and
+ * om_merged_mlp_gate_up_dgrad_bound, the same bits, in one launch where om_merged_mlp_backward_joins (by the sizes) gives 1 and no
+ * two gradients share memory.  rows >= 1; w_stride is that of w_gate and w_up.                                 */
+int om_merged_mlp_backward_joins(int64_t expected_rows, int G, int I, int H);
+int om_grouped_gemm_wgrad_merged_dgrad(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
+    const void *du, const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate, const void *w_up, void *dx,
+    void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
+    int I, int H, int64_t w_stride, int64_t down_stride, int64_t gate_stride, int64_t up_stride, void *stream);
+int om_grouped_gemm_wgrad_merged_dgrad_accumulate(const void *dout, const int32_t *dout_rows, const void *h, const void *dg,
+    const void *du, const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate, const void *w_up, void *dx,
+    void *dw_down, void *dw_gate, void *dw_up, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G,
+    int I, int H, int64_t w_stride, int64_t down_stride, int64_t gate_stride, int64_t up_stride, void *stream);
 int om_merged_mlp_gate_up_dgrad_dense(const void *dg, const void *du, const void *w_gate, const void *w_up,
                                       void *dx, const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows,
                                       int G, int I, int H, int64_t w_stride, const om_dense_expert *dense,

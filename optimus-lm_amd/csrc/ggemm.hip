@@ -416,9 +416,23 @@ template <int V> using IntC = std::integral_constant<int, V>;
 // launched on whole tiles and steps only and carry none of that.
 // (second launch bound: two wavefronts per SIMD, i.e. at most 256 registers, for the 128x128 tile, whose two blocks per
 // CU depend on it; the 256x256 tile's 8 wavefronts imply it already)
-template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool ACCUM = false,
-          bool EDGE = false, bool ONCE = false, bool DENSE = false>
-__global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
+// What a block of a kernel keeps in LDS beside its two stages: how many of each.
+template <int BM, int EPI, int GATHER, bool EDGE> struct Tables {
+    static constexpr bool WGRAD = EPI == EPI_WGRAD, GATHER_W = WGRAD && GATHER != GATHER_NONE;
+    static constexpr bool SHARES = !WGRAD || !EDGE;                                  // whether the launch may be one with p.share != 0
+    static constexpr int LDS = 4 * (BM / 64) * 8192;                                 // A of even and odd steps, then B
+    static constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
+    static constexpr int PARTS = SHARES ? SHARE_MAX_EXPERTS : 1;
+    static constexpr int ENDS = !WGRAD ? MAX_EXPERTS : PARTS;                        // see build_tile_table, build_part_table
+    static constexpr int SEGS = WGRAD ? 1 : MAX_EXPERTS + 1;                         // see build_tile_table; p.share: build_first_tiles
+};
+
+// A block's tiles, counted from the other end of its XCD's blocks with FROM_END.  (The tables one by one: as members of one object the compiler keeps their accesses in order
+// with those of the stages, which in the weight gradients cost registers.)
+template <int BM, int AKIND, int BKIND, int EPI, int GATHER, bool ROWW, bool ACCUM, bool EDGE, bool ONCE, bool DENSE, bool FROM_END = false,
+          typename D = Tables<BM, EPI, GATHER, EDGE>>
+__device__ __forceinline__ void ggemm_tiles(const GemmParams p, char (&lds)[D::LDS], int (&idx_cache)[D::IDX_CACHE], int (&order)[D::PARTS],
+                                            Part (&part)[D::PARTS], int (&tile_end)[D::ENDS], int (&seg)[D::SEGS]) {
     constexpr int BN = BM, WAVES_N = BN / 64, NW = 2 * WAVES_N;
     constexpr int TM = BM / 64, TN = 2;     // row units of a tile, accumulators of a wavefront in each
     static_assert(GATHER == GATHER_NONE || (GATHER == GATHER_A && AKIND == CONTIG && EPI != EPI_WGRAD) ||
@@ -434,15 +448,10 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     constexpr int L = 8 / NW;              // direct loads per wavefront per unit
     constexpr int A_STAGE = UA * UNIT, B_STAGE = UB * UNIT;
     constexpr int B0 = 2 * A_STAGE;        // A of even and odd steps, then B of even and odd steps
-    __shared__ __attribute__((aligned(1024))) char lds[2 * A_STAGE + 2 * B_STAGE];
-    constexpr int IDX_CACHE = GATHER_W ? (BM == 256 ? 4096 : 2048) : 1;
-    __shared__ int idx_cache[IDX_CACHE];
+    static_assert(D::LDS == 2 * A_STAGE + 2 * B_STAGE, "two stages");
+    constexpr int IDX_CACHE = D::IDX_CACHE;
     int cached_expert = -1;            // (MERGED: and product)
-    constexpr bool SHARES = !WGRAD || !EDGE;            // whether the launch may be one with p.share != 0
-    __shared__ int order[SHARES ? SHARE_MAX_EXPERTS : 1];
-    __shared__ __attribute__((aligned(16))) Part part[SHARES ? SHARE_MAX_EXPERTS : 1];
-    __shared__ int tile_end[!WGRAD ? MAX_EXPERTS : SHARES ? SHARE_MAX_EXPERTS : 1];   // see build_tile_table, build_part_table
-    __shared__ int seg[WGRAD ? 1 : MAX_EXPERTS + 1];   // see build_tile_table; p.share: build_first_tiles
+    constexpr bool SHARES = D::SHARES;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -797,7 +806,7 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     };
     constexpr int RA = AKIND == CONTIG ? 4 : 8, RB = BKIND == CONTIG ? 8 : 16;   // LDS reads of a unit of A, of a step of B
 
-    const int nbx = gridDim.x / NUM_XCD, slot_x = blockIdx.x / NUM_XCD;
+    const int nbx = gridDim.x / NUM_XCD, slot_x = FROM_END ? nbx - 1 - static_cast<int>(blockIdx.x / NUM_XCD) : static_cast<int>(blockIdx.x / NUM_XCD);
     int total_tiles = p.total_tiles, per = 0, rem = 0, run_lo = 0;
     if (SHARES && p.share) {
         expert_order(p.cum, p.n_experts, tid, lane, order);
@@ -1247,6 +1256,41 @@ __global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggem
     }  // tile loop
 }
 
+template <int BM, int AKIND, int BKIND, int EPI, int GATHER = GATHER_NONE, bool ROWW = false, bool ACCUM = false,
+          bool EDGE = false, bool ONCE = false, bool DENSE = false>
+__global__ __launch_bounds__(BM == 256 ? 512 : 256, BM == 128 ? 2 : 1) void ggemm_kernel(const GemmParams p) {
+    using D = Tables<BM, EPI, GATHER, EDGE>;
+    __shared__ __attribute__((aligned(1024))) char lds[D::LDS];
+    __shared__ int idx_cache[D::IDX_CACHE];
+    __shared__ int order[D::PARTS];
+    __shared__ __attribute__((aligned(16))) Part part[D::PARTS];
+    __shared__ int tile_end[D::ENDS];
+    __shared__ int seg[D::SEGS];
+    ggemm_tiles<BM, AKIND, BKIND, EPI, GATHER, ROWW, ACCUM, EDGE, ONCE, DENSE>(p, lds, idx_cache, order, part, tile_end, seg);
+}
+
+
+// The input gradient of gate and up and the three weight gradients of experts whose tiles are 128x128: independent of each other, so that
+// the tiles of both share the rounds.  A block works through its row tiles and then, counted from the other end of its XCD's blocks,
+// through its tiles of the weight gradients.
+template <bool ACCUM> __global__ __launch_bounds__(256, 2) void ggemm_backward_kernel(const GemmParams rows, const GemmParams w) {
+    using R = Tables<128, EPI_STORE, GATHER_NONE, true>;
+    using W = Tables<128, EPI_WGRAD, MERGED, true>;
+    static_assert(R::LDS == W::LDS, "the stages of one are the other's");
+    __shared__ __attribute__((aligned(1024))) char lds[R::LDS];
+    // the tables of one where the other's were
+    struct RowTables { Part part[R::PARTS]; int order[R::PARTS], tile_end[R::ENDS], seg[R::SEGS]; };
+    static_assert(sizeof(int[W::IDX_CACHE]) <= sizeof(RowTables), "as many blocks on a CU as of either kernel alone");
+    __shared__ __attribute__((aligned(16))) char tables[sizeof(RowTables)];
+    __shared__ Part no_part[1];
+    __shared__ int none[1];
+    RowTables &t = *reinterpret_cast<RowTables *>(tables);
+    ggemm_tiles<128, CONTIG, STRIDED, EPI_STORE, GATHER_NONE, false, false, true, false, false>(rows, lds, none, t.order, t.part, t.tile_end, t.seg);
+    __syncthreads();
+    ggemm_tiles<128, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, ACCUM, true, false, false, true>(
+        w, lds, *reinterpret_cast<int (*)[W::IDX_CACHE]>(tables), none, no_part, none, none);
+}
+
 // ---- host side ---------------------------------------------------------------------------------
 
 // Two tile shapes: 256x256 (8 wavefronts of 128x64) for the training shapes, 128x128 (4 wavefronts
@@ -1622,10 +1666,12 @@ extern "C" int om_grouped_gemm_wgrad_gathered_out_accumulate(const void *output_
 namespace {
 // dW_down (+)= dout^T h, dW_gate (+)= dg^T x, dW_up (+)= du^T x, in one launch where that saves rounds of tiles: those of an
 // expert's three gradients come one after the other.
+// `beside`: the gate/up input gradient, whose tiles join the launch where it is one of 128x128 tiles; *joined says whether they did.
 int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du, const void *x,
                         const int32_t *x_rows, int64_t src_rows, void *dw_down, void *dw_gate, void *dw_up,
                         const int32_t *cum_token_counts, int64_t rows, int64_t expected, int G, int I, int H, int64_t down_stride,
-                        int64_t gate_stride, int64_t up_stride, bool accumulate, void *stream) {
+                        int64_t gate_stride, int64_t up_stride, bool accumulate, void *stream, const GemmParams *beside = nullptr,
+                        bool *joined = nullptr) {
     if (rows < 0 || expected < 0 || expected > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
     if (!dw_down || !dw_gate || !dw_up || !cum_token_counts || (rows > 0 && (!dout || !h || !dg || !du || !x))) return OM_ERR_NULL;
     if ((dout_rows || x_rows) && src_rows < 1) return OM_ERR_SHAPE;
@@ -1696,8 +1742,16 @@ int wgrad_merged_launch(const void *dout, const int32_t *dout_rows, const void *
     p.stream = true;
     for (const WgradSet &s : p.set) p.stream &= s.n <= STREAM_MAX_PITCH && om_weights_pass_caches(s.C, 3 * packed * G, s.n, s.strideC);
     p.total_tiles = static_cast<int>(tiles);
-    const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     hipStream_t st = om_stream(stream);
+    if (beside && !big) {
+        const int64_t row_tiles = ((rows + 127) / 128 + G) * ((H + 127) / 128);
+        const dim3 both(persistent_blocks<128>(tiles + row_tiles));
+        *joined = true;
+        if (accumulate) ggemm_backward_kernel<true><<<both, dim3(THREADS<128>), 0, st>>>(*beside, p);
+        else ggemm_backward_kernel<false><<<both, dim3(THREADS<128>), 0, st>>>(*beside, p);
+        return om_launch_status();
+    }
+    const dim3 grid(big ? persistent_blocks<256>(tiles) : persistent_blocks<128>(tiles)), block(big ? THREADS<256> : THREADS<128>);
     if (big && accumulate) ggemm_kernel<256, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, true><<<grid, block, 0, st>>>(p);
     else if (big) ggemm_kernel<256, STRIDED, STRIDED, EPI_WGRAD, MERGED><<<grid, block, 0, st>>>(p);
     else if (accumulate) ggemm_kernel<128, STRIDED, STRIDED, EPI_WGRAD, MERGED, false, true, true><<<grid, block, 0, st>>>(p);
@@ -1999,22 +2053,13 @@ extern "C" int om_merged_mlp_gate_up_dgrad(const void *dg, const void *du, const
 }
 
 namespace {
-int gate_up_dgrad_launch(const void *dg, const void *du, const void *w_gate, const void *w_up, void *dx,
-                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I, int H,
-                         int64_t w_stride, const om_dense_expert *dense, void *stream) {
-    if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
-    if (dense && (dense->rows < 1 || !fits_gather(dense->rows))) return OM_ERR_SHAPE;
-    if (dense && (!dense->a[0] || !dense->a[1] || !dense->w[0] || !dense->w[1] || !dense->c[0] || !dense->cum)) return OM_ERR_NULL;
-    auto dense_alone = [&]() {
-        return gate_up_dgrad_launch(dense->a[0], dense->a[1], dense->w[0], dense->w[1], dense->c[0], dense->cum, dense->rows,
-                                    dense->rows, 1, I, H, 0, nullptr, stream);
-    };
-    if (rows == 0) return dense ? dense_alone() : OM_OK;
+// The product's operands, checked; rows > 0.
+int gate_up_dgrad_params(const void *dg, const void *du, const void *w_gate, const void *w_up, void *dx, const int32_t *cum_token_counts,
+                         int64_t rows, int G, int I, int H, int64_t w_stride, GemmParams &p) {
     if (!dg || !du || !w_gate || !w_up || !dx || !cum_token_counts) return OM_ERR_NULL;
     if (!om_aligned16(dg) || !om_aligned16(du) || !om_aligned16(w_gate) || !om_aligned16(w_up) ||
         !om_aligned16(dx))
         return OM_ERR_ALIGN;
-    GemmParams p = {};
     p.A[0] = static_cast<const uint16_t *>(dg);
     p.A[1] = static_cast<const uint16_t *>(du);
     p.B[0] = static_cast<const uint16_t *>(w_gate);  // [G, I, H]: c = i, operand row = h
@@ -2026,6 +2071,22 @@ int gate_up_dgrad_launch(const void *dg, const void *du, const void *w_gate, con
     if (!pitch_ok(p.strideB)) return OM_ERR_ALIGN;
     if (!fits_span(rows * H) || !fits_span(rows * I) || !fits_span(p.strideB * G)) return OM_ERR_SHAPE;
     p.rows = rows; p.n_experts = G; p.n_cols = H; p.kc = I; p.phases = 2;
+    return OM_OK;
+}
+int gate_up_dgrad_launch(const void *dg, const void *du, const void *w_gate, const void *w_up, void *dx,
+                         const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I, int H,
+                         int64_t w_stride, const om_dense_expert *dense, void *stream) {
+    if (rows < 0 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    if (dense && (dense->rows < 1 || !fits_gather(dense->rows))) return OM_ERR_SHAPE;
+    if (dense && (!dense->a[0] || !dense->a[1] || !dense->w[0] || !dense->w[1] || !dense->c[0] || !dense->cum)) return OM_ERR_NULL;
+    auto dense_alone = [&]() {
+        return gate_up_dgrad_launch(dense->a[0], dense->a[1], dense->w[0], dense->w[1], dense->c[0], dense->cum, dense->rows,
+                                    dense->rows, 1, I, H, 0, nullptr, stream);
+    };
+    if (rows == 0) return dense ? dense_alone() : OM_OK;
+    GemmParams p = {};
+    const int params = gate_up_dgrad_params(dg, du, w_gate, w_up, dx, cum_token_counts, rows, G, I, H, w_stride, p);
+    if (params != OM_OK) return params;
     if (dense) {
         if (dense_rides<EPI_STORE>(p, expected_rows, dense->rows)) {
             if (!dense_operands(p, dense)) return OM_ERR_ALIGN;
@@ -2043,6 +2104,58 @@ extern "C" int om_merged_mlp_gate_up_dgrad_bound(const void *dg, const void *du,
                                                  int64_t rows, int64_t expected_rows, int G, int I, int H,
                                                  int64_t w_stride, void *stream) {
     return gate_up_dgrad_launch(dg, du, w_gate, w_up, dx, cum_token_counts, rows, expected_rows, G, I, H, w_stride, nullptr, stream);
+}
+
+// Where the tiles of both are 128x128 and no more than 8 rounds of two blocks a CU: the last round of either launch is then a good part of it, and
+// with few tiles either leaves most of the chip idle.  Two launches -> one, us, caches full of written data, gradients written / added: 8
+// experts of 256/512, 4096 rows (0.5 rounds in all) 34.4 -> 26.2 / 36.2 -> 27.5; 16 of 512/256, 1200 rows 24.2 -> 17.4 / 28.2 -> 19.4; 12 of 1000/712,
+// 9003 rows (4.6) 130 -> 122 / 140 -> 133, uneven 157 -> 142 / 164 -> 151, 900 rows 56.5 -> 53.3 / 66.9 -> 60.4; 16 of 1304/600, 4096 rows (6.0) 97 ->
+// 92 / 114 -> 110; 8 of 2000/1000, 8000 rows (8.1) 259 -> 259 / 282 -> 283; 32 of 1000/1000, 32000 rows (16) 533 -> 534 / 557 -> 555.
+extern "C" int om_merged_mlp_backward_joins(int64_t expected_rows, int G, int I, int H) {
+    if (expected_rows < 0 || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    GemmParams p = {};
+    p.n_experts = G; p.n_cols = H; p.kc = I;
+    if (expected_rows < 1 || G > MAX_EXPERTS || rows_share(p, expected_rows) || uses_big_tile<EPI_STORE>(H, I, G, expected_rows) ||
+        2 * static_cast<int64_t>(G) * I * H >= CACHED_WEIGHTS || wgrad_big_tile(H, I, 3 * static_cast<int64_t>(G)))
+        return 0;
+    const int64_t across = (H + 127) / 128, weight_tiles = 3 * across * ((I + 127) / 128) * G, row_tiles = (expected_rows / 128 + (G + 1) / 2) * across;
+    return weight_tiles + row_tiles <= 8 * 2 * static_cast<int64_t>(device_cu_count()) ? 1 : 0;
+}
+
+namespace {
+int backward_launch(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du,
+                    const void *x, const int32_t *x_rows, int64_t src_rows, const void *w_gate,
+                    const void *w_up, void *dx, void *dw_down, void *dw_gate, void *dw_up,
+                    const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I,
+                    int H, int64_t w_stride, int64_t down_stride, int64_t gate_stride, int64_t up_stride,
+                    bool accumulate, void *stream) {
+    if (rows < 1 || expected_rows < 0 || expected_rows > rows || G < 1 || !mult(I, 8) || !mult(H, 8)) return OM_ERR_SHAPE;
+    GemmParams p = {};
+    int code = gate_up_dgrad_params(dg, du, w_gate, w_up, dx, cum_token_counts, rows, G, I, H, w_stride, p);
+    if (code != OM_OK) return code;
+    bool joined = false;
+    const bool may = om_merged_mlp_backward_joins(expected_rows, G, I, H) == 1;
+    code = wgrad_merged_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, dw_down, dw_gate, dw_up, cum_token_counts, rows,
+                               expected_rows, G, I, H, down_stride, gate_stride, up_stride, accumulate, stream, may ? &p : nullptr, &joined);
+    if (code != OM_OK || joined) return code;
+    return launch_rows_auto<CONTIG, STRIDED, EPI_STORE>(p, rows, expected_rows, om_stream(stream));
+}
+}  // namespace
+
+extern "C" int om_grouped_gemm_wgrad_merged_dgrad(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du, const void *x, const int32_t *x_rows,
+    int64_t src_rows, const void *w_gate, const void *w_up, void *dx, void *dw_down, void *dw_gate, void *dw_up,
+    const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t w_stride, int64_t down_stride,
+    int64_t gate_stride, int64_t up_stride, void *stream) {
+    return backward_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, w_gate, w_up, dx, dw_down, dw_gate, dw_up, cum_token_counts, rows,
+                           expected_rows, G, I, H, w_stride, down_stride, gate_stride, up_stride, false, stream);
+}
+
+extern "C" int om_grouped_gemm_wgrad_merged_dgrad_accumulate(const void *dout, const int32_t *dout_rows, const void *h, const void *dg, const void *du, const void *x, const int32_t *x_rows,
+    int64_t src_rows, const void *w_gate, const void *w_up, void *dx, void *dw_down, void *dw_gate, void *dw_up,
+    const int32_t *cum_token_counts, int64_t rows, int64_t expected_rows, int G, int I, int H, int64_t w_stride, int64_t down_stride,
+    int64_t gate_stride, int64_t up_stride, void *stream) {
+    return backward_launch(dout, dout_rows, h, dg, du, x, x_rows, src_rows, w_gate, w_up, dx, dw_down, dw_gate, dw_up, cum_token_counts, rows,
+                           expected_rows, G, I, H, w_stride, down_stride, gate_stride, up_stride, true, stream);
 }
 
 extern "C" int om_merged_mlp_gate_up_dgrad_dense(const void *dg, const void *du, const void *w_gate,

@@ -663,12 +663,21 @@ std::pair<Tensor, Tensor> routed_backward(const Call &c, const Tensor &dfinal, c
                 OM_BOUND(c, om_merged_mlp_down_dgrad_weighted, ptr(dfinal), ix.in, T, ptr(w.down), ptr(s.g), ptr(s.u), row_w, ptr(dg),
                          ptr(du), fpm(row_dot), ix.cum, rows, ix.to_choose_by(), G, I, H, expert_stride(w.down), c.stream);
             }
-            wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, ix.to_choose_by(), G, I, H);
+            const bool joined = !along && k.gate.accumulate == k.up.accumulate && k.gate.accumulate == k.down.accumulate &&
+                                om_merged_mlp_backward_joins(ix.to_choose_by(), G, I, H) == 1;
+#define OM_JOINED(fn)                                                                                                                 \
+    OM(c, fn, ptr(dfinal), ix.in, ptr(s.h), ptr(dg), ptr(du), ptr(x), ix.in, T, ptr(w.gate), ptr(w.up), ptr(dx_rows), ptr(k.down.grad), \
+       ptr(k.gate.grad), ptr(k.up.grad), ix.cum, rows, ix.to_choose_by(), G, I, H, expert_stride(w.gate), k.down.pitch, k.gate.pitch,   \
+       k.up.pitch, c.stream)
+            if (joined && k.gate.accumulate) OM_JOINED(om_grouped_gemm_wgrad_merged_dgrad_accumulate);
+            else if (joined) OM_JOINED(om_grouped_gemm_wgrad_merged_dgrad);
+#undef OM_JOINED
+            else wgrads(c, dfinal, ix.in, s.h, dg, du, x, ix.in, k, ix.cum, rows, ix.to_choose_by(), G, I, H);
             if (along) {
                 const om_dense_expert d = dense_expert({&dense_dg, &dense_du}, {&along->w.gate, &along->w.up}, {&base, nullptr, nullptr}, along->s, T);
                 OM(c, om_merged_mlp_gate_up_dgrad_dense, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
                    ix.to_choose_by(), G, I, H, expert_stride(w.gate), &d, c.stream);
-            } else {
+            } else if (!joined) {
                 OM_BOUND(c, om_merged_mlp_gate_up_dgrad, ptr(dg), ptr(du), ptr(w.gate), ptr(w.up), ptr(dx_rows), ix.cum, rows,
                          ix.to_choose_by(), G, I, H, expert_stride(w.gate), c.stream);
             }

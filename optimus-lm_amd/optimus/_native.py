@@ -187,6 +187,11 @@ SIGNATURES = {
     "om_merged_mlp_down_dgrad_weighted_dense": (c_int, [c_void_p, c_void_p, c_i64] + [c_void_p] * 8 +
                                                 [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_void_p, c_void_p]),
     "om_merged_mlp_gate_up_dgrad_dense": (c_int, [c_void_p] * 6 + [c_i64, c_i64, c_int, c_int, c_int, c_i64, c_void_p, c_void_p]),
+    "om_merged_mlp_backward_joins": (c_int, [c_i64, c_int, c_int, c_int]),
+    "om_grouped_gemm_wgrad_merged_dgrad": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 7 + [c_i64, c_i64, c_int, c_int, c_int] +
+                                           [c_i64] * 4 + [c_void_p]),
+    "om_grouped_gemm_wgrad_merged_dgrad_accumulate": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 7 +
+                                                      [c_i64, c_i64, c_int, c_int, c_int] + [c_i64] * 4 + [c_void_p]),
     "om_grouped_gemm_wgrad_merged": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 4 +
                                      [c_i64, c_int, c_int, c_int, c_i64, c_i64, c_i64, c_void_p]),
     "om_grouped_gemm_wgrad_merged_accumulate": (c_int, [c_void_p] * 7 + [c_i64] + [c_void_p] * 4 +

@@ -932,3 +932,39 @@ def test_layer_without_gradients_gives_the_same_bits(cuda, tokens, parallel):
     with torch.no_grad():
         alone = block(x)
     assert torch.equal(alone, block(x).detach())
+
+
+# experts without rows, partial tiles of both extents, one tile in all, more row tiles than blocks, sizes that do not join
+@pytest.mark.parametrize("rows_e,I,H", [((0, 3, 0), 8, 16), ((130, 0, 1, 257), 200, 136), ((64,) * 8, 512, 256), ((700, 0, 129, 500, 3000), 712, 1000),
+                                        ((20000, 5000), 264, 520), ((300, 500), 1024, 2048)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+@pytest.mark.parametrize("shared_memory", [False, True])
+def test_input_and_weight_gradients_in_one_call_are_those_of_two(cuda, rows_e, I, H, accumulate, shared_memory):
+    """om_grouped_gemm_wgrad_merged_dgrad: the bits of the two entry points, in one launch or in several (the gradients of gate and up
+    one buffer), and what those refuse is refused."""
+    from optimus import _native as n
+    L, P, G, rows, T = n.lib(), n.ptr, len(rows_e), sum(rows_e), 501
+    gen = torch.Generator(device=cuda).manual_seed(rows + I)
+    bf = lambda *s: (torch.randn(*s, generator=gen, device=cuda) * 0.1).bfloat16()
+    x, dy, h, dg, du = bf(T, H), bf(T, H), bf(rows, I), bf(rows, I), bf(rows, I)
+    wg, wu = bf(G, I, H), bf(G, I, H)
+    cum = torch.tensor([0] + list(torch.tensor(rows_e).cumsum(0)), dtype=torch.int32, device=cuda)
+    index = torch.randint(0, T, (rows,), generator=gen, device=cuda, dtype=torch.int32)
+    start = [bf(G, H, I), bf(G, I, H), bf(G, I, H)]
+    got, want = [t.clone() for t in start], [t.clone() for t in start]
+    if shared_memory:
+        got[2], want[2] = got[1], want[1]
+    dx, dx_want = torch.full((2, rows, H), 7.0, dtype=torch.bfloat16, device=cuda)
+    wgrad = L.om_grouped_gemm_wgrad_merged_accumulate_bound if accumulate else L.om_grouped_gemm_wgrad_merged_bound
+    n.check(wgrad(P(dy), P(index), P(h), P(dg), P(du), P(x), P(index), T, *(P(t) for t in want), P(cum), rows, rows, G, I, H, 0, 0, 0,
+                  n.stream()), "weights")
+    n.check(L.om_merged_mlp_gate_up_dgrad_bound(P(dg), P(du), P(wg), P(wu), P(dx_want), P(cum), rows, rows, G, I, H, 0, n.stream()), "input")
+    both = L.om_grouped_gemm_wgrad_merged_dgrad_accumulate if accumulate else L.om_grouped_gemm_wgrad_merged_dgrad
+    call = lambda r, i: both(P(dy), P(index), P(h), P(dg), P(du), P(x), P(index), T, P(wg), P(wu), P(dx), *(P(t) for t in got),
+                             P(cum), r, min(r, rows), G, i, H, 0, 0, 0, 0, n.stream())
+    n.check(call(rows, I), "both")
+    torch.cuda.synchronize()
+    assert torch.equal(dx, dx_want) and all(torch.equal(a, b) for a, b in zip(got, want))
+    assert call(0, I) == call(rows, I + 4) == L.om_merged_mlp_gate_up_dgrad(P(dg), P(du), P(wg), P(wu), P(dx), P(cum), rows, G, I + 4, H, 0,
+                                                                          n.stream())
+    assert L.om_merged_mlp_backward_joins(rows, G, I, H) == (0 if (I, H) == (1024, 2048) else 1)
