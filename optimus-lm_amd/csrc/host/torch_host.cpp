@@ -2,7 +2,7 @@
 // autograd nodes around them, as the Python module `optimus_torch_host`.
 //
 // What bounded the small calls was the interpreter: a training step of the tiny layer was 22 launches
-// (15 now) of 2-14 us each, and enqueueing them through ctypes and Python autograd functions took 510 us.  Here a
+// (10 now) of 2-14 us each, and enqueueing them through ctypes and Python autograd functions took 510 us.  Here a
 // layer is two autograd nodes (router, experts) whose forward and backward run without the interpreter:
 // each reads the three run-time switches of the Python modules once (launch log, profiler, in-place
 // weight gradients) and then only allocates and launches.
@@ -1569,7 +1569,7 @@ Tensor combine(const Tensor &y, const Tensor &rw_in, const Tensor &cum_ep, const
 
 // ---- optimizer ----------------------------------------------------------------------------------------
 // A step of a small optimizer is two launches of 7 to 10 us; through ctypes, with the operands looked over in Python, they
-// took the host 29 us (22 now, 21 a step among others).
+// took the host 29 us (19 now).
 
 bool flat_buffer(const Tensor &t, int64_t n) { return t.is_cuda() && t.is_contiguous() && t.numel() == n; }
 
