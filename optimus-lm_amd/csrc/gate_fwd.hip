@@ -136,7 +136,12 @@ __global__ __launch_bounds__(256) void gate_logits_split_kernel(const uint16_t *
 // routing, weights out of the caches: hidden 2048, 64 experts, 1 token 12.5 -> 10.1, 64 13.7 -> 10.3, 512 15.8 -> 10.9; hidden 7168, 64 experts,
 // 512 tokens 25.0 -> 16.3, 8 experts 20.5 -> 10.6.  Every 16 tokens read the weight again: hidden 3000, 60 experts, 1000 tokens 17.4 -> 19.8, 4000 21.3 ->
 // 33.7, hidden 4040, 20 experts, 2000 tokens 14.8 -> 15.5.  Hence the line.
-constexpr int64_t GATE_FEW_TOKENS = 512;
+// More than 64 experts have more to read again, and it stays the sooner one up to about 100 tokens; the projection with the launch that adds the
+// slices, weights out of the caches: 256 experts of 7168, 1 token 13.7 -> 9.6, 64 14.8 -> 12.4, 96 15.7 -> 15.2, 128 16.2 -> 16.3, 200 17.0 ->
+// 21.5; of 2048, 64 tokens 11.8 -> 10.4, 96 12.5 -> 11.8; 160 of 1624, 64 tokens 11.7 -> 10.0.
+// CH: chunks of 32 columns under way, no more than a slice has (64 columns asked for as 256: 64 tokens of 2048, 256 experts 12.8, 512 tokens of
+// 1024, 64 experts 11.8 for 9.4, 300 of 2048 13.8 for 10.7).
+constexpr int64_t GATE_FEW_TOKENS = 512, GATE_FEW_TOKENS_WIDE = 64;
 template <int CH>
 __global__ __launch_bounds__(64) void gate_logits_few_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, int64_t T, int H, int N,
                                                              int h_per_split, float *__restrict__ partial) {
@@ -321,8 +326,11 @@ void om_launch_gate_partials(const void *x, const void *gate_weight, int64_t T, 
     const dim3 grid(static_cast<unsigned>((T + GT - 1) / GT), splits);
     const uint16_t *xp = static_cast<const uint16_t *>(x), *wp = static_cast<const uint16_t *>(gate_weight);
     const int hps = ((H + GK - 1) / GK + splits - 1) / splits * GK;
-    if (N <= 64 && T <= GATE_FEW_TOKENS) {
-        gate_logits_few_kernel<8><<<dim3((N + 15) / 16, splits, static_cast<unsigned>((T + 15) / 16)), dim3(64), 0, st>>>(xp, wp, T, H, N, hps, ws);
+    if (T <= (N <= 64 ? GATE_FEW_TOKENS : GATE_FEW_TOKENS_WIDE)) {
+        const dim3 tiles((N + 15) / 16, splits, static_cast<unsigned>((T + 15) / 16));
+        if (hps > 128) gate_logits_few_kernel<8><<<tiles, dim3(64), 0, st>>>(xp, wp, T, H, N, hps, ws);
+        else if (hps > 64) gate_logits_few_kernel<4><<<tiles, dim3(64), 0, st>>>(xp, wp, T, H, N, hps, ws);
+        else gate_logits_few_kernel<2><<<tiles, dim3(64), 0, st>>>(xp, wp, T, H, N, hps, ws);
     } else if (N <= 64) gate_logits_split_kernel<2><<<grid, dim3(256), 0, st>>>(xp, wp, T, H, N, hps, ws);
     else if (N <= 128) gate_logits_wide_kernel<4><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);
     else gate_logits_wide_kernel<8><<<grid, dim3(512), 0, st>>>(xp, wp, T, H, N, hps, ws);

@@ -760,3 +760,26 @@ def test_balance_loss_in_one_function_is_the_composed_one(cuda, T, N, K, dtype):
     g = 0.01 * N * float(count.max()) / T / T
     bound = float(p) * g * 2 * 4 * 2.0 ** -24 + (2.0 ** -8 * float(b.grad.abs().max()) if dtype == torch.bfloat16 else 0.0)
     assert float((a.grad.float() - b.grad.float()).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("H,N", [(7168, 256), (2048, 256), (1624, 160), (1000, 65), (264, 200), (8, 100)])
+def test_few_tokens_of_many_experts_have_the_logits_of_many(cuda, H, N):
+    """Up to 64 tokens of more than 64 experts, around the tiles of 16, slices of one to several chunks: the bits that the same tokens
+    have among 128 (as many slices)."""
+    from optimus import _native as n
+    L = n.lib()
+    x = torch.randn(128, H, device=cuda).bfloat16()
+    w = (torch.randn(N, H, device=cuda) * 0.1).bfloat16()
+
+    def logits(T):
+        out = torch.full((T, N), 7.0, device=cuda)
+        ws = torch.empty(L.om_router_gate_logits_split_workspace_bytes(T, H, N), dtype=torch.uint8, device=cuda)
+        n.check(L.om_router_gate_logits_split(n.ptr(x), n.ptr(w), T, H, N, n.ptr(out), n.ptr(ws), ws.numel(), n.stream()), "logits")
+        return out
+
+    many = logits(128)
+    exact = x.double() @ w.double().T
+    # float32 sums of H exact products: at most H roundings of the largest partial sum
+    assert bool(((many.double() - exact).abs() <= H * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all())
+    for T in (1, 15, 16, 17, 63, 64, 65):
+        assert torch.equal(logits(T), many[:T]), T
