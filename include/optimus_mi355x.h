@@ -321,7 +321,8 @@ int om_router_balance_loss_bwd(const void *logits, int logits_dtype, const float
  *   experts, divided by (sum + 1e-20) when norm_topk_prob, times routed_scaling_factor.
  *   logits [T,N] fp32, bias [N] fp32 -> experts_out [T,K] int64 (descending choice value,
  *   lower index first among equals), weights_out [T,K] fp32.  N <= 512, N % n_group == 0.
- * om_route_sigmoid_topk_bwd: dlogits [T,N] fp32 (dense, zero off the selected experts).   */
+ * om_route_sigmoid_topk_bwd: dlogits [T,N] fp32 (dense, zero off the selected experts); a number in `experts`
+ *   outside 0 .. N-1 has no weight and no gradient.                                          */
 int om_route_sigmoid_group_topk(const float *logits, const float *bias, int64_t T, int N,
                                 int n_group, int topk_group, int K, int norm_topk_prob,
                                 double routed_scaling_factor, int64_t *experts_out,

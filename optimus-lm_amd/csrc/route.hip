@@ -473,9 +473,10 @@ __global__ __launch_bounds__(256) void sigmoid_topk_bwd_kernel(const float *__re
     const int lane = threadIdx.x & 63;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * TOKENS_PER_BLOCK + (threadIdx.x >> 6);
     if (t >= Tn) return;
-    const int e = (lane < K) ? static_cast<int>(experts[t * K + lane]) : -1;
+    const int64_t selected = (lane < K) ? experts[t * K + lane] : -1;
+    const int e = selected >= 0 && selected < N ? static_cast<int>(selected) : -1;   // (a number that is no expert's: no weight, no gradient)
     float sk = 0.0f;
-    if (lane < K) sk = 1.0f / (1.0f + expf(-logits[t * N + e]));
+    if (e >= 0) sk = 1.0f / (1.0f + expf(-logits[t * N + e]));
     float d = (lane < K) ? dweights[t * K + lane] * scale : 0.0f;  // through "* scale"
     if (renorm) {
         const float S = wave_sum(sk) + 1e-20f;

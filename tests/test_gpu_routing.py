@@ -783,3 +783,25 @@ def test_few_tokens_of_many_experts_have_the_logits_of_many(cuda, H, N):
     assert bool(((many.double() - exact).abs() <= H * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all())
     for T in (1, 15, 16, 17, 63, 64, 65):
         assert torch.equal(logits(T), many[:T]), T
+
+
+@pytest.mark.parametrize("renorm", [0, 1])
+def test_sigmoid_router_backward_of_numbers_that_are_no_experts(cuda, renorm):
+    """A selection outside the experts has no weight and no gradient: the others' gradients are those of the token without it."""
+    from optimus import _native as n
+    lib, st, T, N, K = n.lib(), n.stream(), 5, 72, 3
+    g = torch.Generator().manual_seed(3)
+    logits, dw = torch.randn(T, N, generator=g), torch.randn(T, K, generator=g)
+    experts = torch.tensor([[1, 70, 9], [0x7fffffff, 71, 0], [5, -1, N], [0x7fffffff] * 3, [2 ** 32 + 1, 2, 71]])
+    lg, eg, dg = logits.to(cuda), experts.to(cuda), dw.to(cuda)
+    got = torch.full((T, N), 7.0, device=cuda)
+    n.check(lib.om_route_sigmoid_topk_bwd(n.ptr(lg), n.ptr(eg), n.ptr(dg), T, N, K, renorm, 2.5, n.ptr(got), st), "backward")
+    x = logits.double().requires_grad_(True)
+    loss = 0.0
+    for t in range(T):
+        kept = [k for k in range(K) if 0 <= experts[t, k] < N]
+        s = torch.sigmoid(x[t, experts[t, kept]])
+        loss = loss + (dw[t, kept].double() * 2.5 * (s / (s.sum() + 1e-20) if renorm else s)).sum()
+    loss.backward()
+    # a dozen float32 operations of terms no larger than 2.5 |dw| each
+    assert float((got.cpu().double() - x.grad).abs().max()) <= 16 * 2.0 ** -24 * 2.5 * float(dw.abs().max()) * K
