@@ -129,9 +129,18 @@ __device__ __forceinline__ void row_softmax(const T *row, int N, int lane, float
     softmax_in_place<PER>(N, lane, p);
 }
 
+// The lowest expert that is not among the first r selections, of which lane q holds the q-th: what a group-limited router selects where no
+// score is left that compares (NaN, or biases of -inf).
+__device__ __forceinline__ int lowest_free(int e, int r, int lane) {
+    int i = 0;
+    while (__ballot(lane < r && e == i) != 0) i++;
+    return i;
+}
+
 // K rounds of wave arg-max over s[PER] (entries with index >= N must be < every real score).
-// Lane r keeps the r-th winner in (my_v, my_i).
-template <int PER>
+// Lane r keeps the r-th winner in (my_v, my_i).  Scores that are NaN or -inf never win; where no other is left the index is
+// 0x7fffffff, or with FREE the lowest that was not selected.
+template <int PER, bool FREE = false>
 __device__ __forceinline__ void select_topk(float (&s)[PER], int N, int K, int lane, float &my_v,
                                             int &my_i) {
     my_v = 0.0f;
@@ -145,6 +154,7 @@ __device__ __forceinline__ void select_topk(float (&s)[PER], int N, int K, int l
             if (i < N && (s[j] > bv)) { bv = s[j]; bi = i; }  // ascending i: first max wins
         }
         wave_argmax(bv, bi);
+        if (FREE && bi == 0x7fffffff) bi = lowest_free(my_i, r, lane);
         if (lane == r) { my_v = bv; my_i = bi; }
 #pragma unroll
         for (int j = 0; j < PER; j++)
@@ -340,6 +350,7 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
             if (v > a) { b = a; a = v; } else if (v > b) { b = v; }
         }
         gscore = (gs >= 2) ? (a + b) : a;
+        if (gscore != gscore) gscore = -INFINITY;   // (+inf and nothing beside it)
     }
     // keep the topk_group best groups (score desc, group index asc)
     unsigned long long keep = 0ull;
@@ -356,7 +367,7 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
         if (i < N && !((keep >> (i / gs)) & 1ull)) choice[j] = 0.0f;
     }
     float cv; int e;
-    select_topk<PER>(choice, N, K, lane, cv, e);
+    select_topk<PER, true>(choice, N, K, lane, cv, e);
     // weight = sigmoid score (no bias) at the selected expert
     float w = fetch_expert_value<PER>(score, e);
     if (lane >= K) w = 0.0f;
@@ -408,29 +419,33 @@ __global__ __launch_bounds__(256) void sigmoid_group_quads_kernel(const float *_
         score[j] = inside ? 1.0f / (1.0f + expf(-x[j])) : 0.0f;
         choice[j] = inside ? score[j] + b[j] : -INFINITY;
     }
-    // the two largest of the lane's, then of its group's lanes
+    // the two largest of the lane's, then of its group's lanes; NaN is none of them, as in the scan
     const int lanes = N / n_group / QUADS;
-    float best = fmaxf(choice[0], choice[1]), next = fminf(choice[0], choice[1]);
+    float best = -INFINITY, next = -INFINITY;
 #pragma unroll
-    for (int j = 2; j < QUADS; j++) {
-        next = fmaxf(next, fminf(best, choice[j]));
-        best = fmaxf(best, choice[j]);
+    for (int j = 0; j < QUADS; j++) {
+        const float v = choice[j] == choice[j] ? choice[j] : -INFINITY;
+        next = fmaxf(next, fminf(best, v));
+        best = fmaxf(best, v);
     }
     for (int o = 1; o < lanes; o <<= 1) {
         const float other = __shfl_xor(best, o, 64), other_next = __shfl_xor(next, o, 64);
         next = fmaxf(fmaxf(next, other_next), fminf(best, other));
         best = fmaxf(best, other);
     }
-    // kept: the groups that fewer than topk_group others precede (score descending, group ascending)
-    const float mine = best + next;
+    // kept: the groups that fewer than topk_group others precede (score descending, group ascending).  A group with less than two
+    // scores that compare has -inf and is not kept, but where such groups are reached at all the first group is.
+    const float sum = best + next, mine = sum == sum ? sum : -INFINITY;
     const int group = i0 / (lanes * QUADS);
-    int before = 0;
+    int before = 0, above = 0;
     for (int q = 0; q < n_group; q++) {
         const float other = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), q * lanes));
         before += other > mine || (other == mine && q < group) ? 1 : 0;
+        above += other > -INFINITY ? 1 : 0;
     }
+    const bool kept = mine > -INFINITY ? before < topk_group : group == 0 && above < topk_group;
     // masked_fill(~mask, 0.0): dropped groups compete with the value 0.0
-    if (inside && before >= topk_group) {
+    if (inside && !kept) {
 #pragma unroll
         for (int j = 0; j < QUADS; j++) choice[j] = 0.0f;
     }
@@ -443,6 +458,7 @@ __global__ __launch_bounds__(256) void sigmoid_group_quads_kernel(const float *_
         for (int j = 0; j < QUADS; j++)
             if (inside && choice[j] > bv) { bv = choice[j]; bi = i0 + j; }   // ascending experts: the first maximum wins
         wave_argmax(bv, bi);
+        if (bi == 0x7fffffff) bi = lowest_free(e, r, lane);
         if (lane == r) e = bi;
 #pragma unroll
         for (int j = 0; j < QUADS; j++)

@@ -805,3 +805,57 @@ def test_sigmoid_router_backward_of_numbers_that_are_no_experts(cuda, renorm):
     loss.backward()
     # a dozen float32 operations of terms no larger than 2.5 |dw| each
     assert float((got.cpu().double() - x.grad).abs().max()) <= 16 * 2.0 ** -24 * 2.5 * float(dw.abs().max()) * K
+
+
+# (groups of one lane, of several, all kept, a single group, more selections than the groups that are left have experts)
+@pytest.mark.parametrize("T,H,N,n_group,topk_group,K", [(9, 512, 256, 8, 4, 8), (1030, 264, 64, 8, 3, 6), (40, 512, 96, 3, 3, 5), (33, 72, 24, 1, 1, 8),
+                                                        (12, 512, 16, 4, 2, 16), (10, 512, 12, 4, 2, 5)])
+@pytest.mark.parametrize("bad", ["token", "expert", "group", "expert bias", "-inf biases", "-inf bias of all", "+inf alone"])
+def test_group_router_of_what_is_not_finite(cuda, T, H, N, n_group, topk_group, K, bad):
+    """Scores that do not compare: K different experts of the model for every token, those that om_route_sigmoid_group_topk selects; tokens
+    with finite scores as without the others; and NaN gradients where the weights are NaN."""
+    from optimus import _native as n
+    lib, st, gs, nan = n.lib(), n.stream(), N // n_group, float("nan")
+    x, w = _gate_inputs(T, H, N, seed=T + N)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2)).mul(0.1)
+
+    def route(x, w, bias):
+        xg, wg, bg = x.to(cuda), w.to(cuda).contiguous(), bias.to(cuda)
+        logits, e, wt = torch.empty(T, N, device=cuda), torch.empty(T, K, dtype=torch.int64, device=cuda), torch.empty(T, K, device=cuda)
+        ws = torch.empty(max(lib.om_router_gate_route_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+        n.check(lib.om_router_gate_split_sigmoid_group_topk(n.ptr(xg), n.ptr(wg), n.ptr(bg), T, H, N, n_group, topk_group, K, 1, 2.5, n.ptr(logits),
+                                                            n.ptr(e), n.ptr(wt), n.ptr(ws), ws.numel(), st), "fused")
+        want_e, want_w = torch.empty_like(e), torch.empty_like(wt)
+        n.check(lib.om_route_sigmoid_group_topk(n.ptr(logits), n.ptr(bg), T, N, n_group, topk_group, K, 1, 2.5, n.ptr(want_e), n.ptr(want_w), st), "router")
+        assert torch.equal(e, want_e) and torch.equal(torch.isnan(wt), torch.isnan(want_w)) and torch.equal(wt.nan_to_num(7.0), want_w.nan_to_num(7.0))
+        assert bool(((e >= 0) & (e < N)).all()) and bool((e.sort(1).values.diff(dim=1) > 0).all())
+        return logits, e, wt
+    good_logits, good_e, good_w = route(x, w, bias)
+    if bad == "token":
+        x[T // 2, 3] = nan
+    elif bad == "expert":
+        w[N // 2] = nan
+    elif bad == "group":
+        w[N - gs:] = nan
+    elif bad == "expert bias":
+        bias[1] = nan
+    elif bad == "-inf biases":
+        bias[torch.randperm(N, generator=torch.Generator().manual_seed(4))[:N - 3]] = float("-inf")
+    elif bad == "-inf bias of all":
+        bias[:] = float("-inf")
+    else:
+        bias[:gs] = float("-inf")
+        bias[0] = float("inf")
+    logits, e, wt = route(x, w, bias)
+    if bad != "token":
+        return
+    # the NaN token: no group compares, so the first is kept, and the zeros of the others come first
+    order = list(range(gs, N)) + list(range(gs))
+    if n_group == 1:
+        order = list(range(N))
+    assert e[T // 2].tolist() == order[:K] and bool(torch.isnan(wt[T // 2]).all())
+    others = torch.arange(T, device=cuda) != T // 2
+    assert torch.equal(logits[others], good_logits[others]) and torch.equal(e[others], good_e[others]) and torch.equal(wt[others], good_w[others])
+    dw, dl = torch.ones(T, K, device=cuda), torch.full((T, N), 7.0, device=cuda)
+    n.check(lib.om_route_sigmoid_topk_bwd(n.ptr(logits), n.ptr(e), n.ptr(dw), T, N, K, 1, 2.5, n.ptr(dl), st), "backward")
+    assert bool(torch.isnan(dl[T // 2][e[T // 2]]).all()) and bool(torch.isfinite(dl[others]).all())
