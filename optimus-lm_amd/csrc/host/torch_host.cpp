@@ -976,9 +976,11 @@ struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits 
         if (weights_grad.defined()) {
             const Tensor &logits = kept[2], &experts = kept[3];
             const int64_t T = logits.size(0), N = logits.size(1), K = experts.size(1);
-            if (!sigmoid && xs.scalar_type() == at::kBFloat16 && task_should_compute_output(0) && task_should_compute_output(1) &&
-                N <= 64 && (!logits_grad.defined() || logits_grad.scalar_type() == logits.scalar_type()))
-                return softmax_backward(c, xs, ws, logits, experts, weights_grad, logits_grad, x_grad);
+            const bool both = !sigmoid && xs.scalar_type() == at::kBFloat16 && task_should_compute_output(0) && task_should_compute_output(1) &&
+                              (!logits_grad.defined() || logits_grad.scalar_type() == logits.scalar_type());
+            // (negative for sizes that it does not take: more than 64 experts, no tokens)
+            const int64_t ws_bytes = both ? om_router_softmax_bwd_workspace_bytes(T, xs.size(1), N) : -1;
+            if (ws_bytes > 0) return softmax_backward(c, xs, ws, logits, experts, weights_grad, logits_grad, x_grad, ws_bytes);
             dlogits = make(logits.sizes(), logits);
             if (sigmoid) {
                 weights_grad = weights_grad.contiguous().to(at::kFloat);
@@ -996,7 +998,7 @@ struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits 
     }
     // Both gradients of the gate behind a softmax router in one call.
     variable_list softmax_backward(const Call &c, const Tensor &x, const Tensor &weight, const Tensor &logits, const Tensor &experts,
-                                   Tensor weights_grad, Tensor logits_grad, Tensor x_grad) const {
+                                   Tensor weights_grad, Tensor logits_grad, Tensor x_grad, int64_t ws_bytes) const {
         const int64_t T = x.size(0), H = x.size(1), N = weight.size(0), K = experts.size(1);
         weights_grad = weights_grad.contiguous();
         if (logits_grad.defined()) logits_grad = logits_grad.contiguous();
@@ -1004,9 +1006,6 @@ struct RouterNode : HostNode {       // saves x, weight, and (selecting) logits 
             x_grad = x_grad.contiguous();
             require_bf16(x_grad);
         }
-        require_gate_shape(weight, "router backward");
-        const int64_t ws_bytes = om_router_softmax_bwd_workspace_bytes(T, H, N);
-        if (ws_bytes < 0) check(static_cast<int>(ws_bytes), "om_router_softmax_bwd_workspace_bytes");
         Tensor ws = make({ws_bytes}, x, at::kByte), dx = make(x.sizes(), x), dw = make(weight.sizes(), weight);
         OM(c, om_router_softmax_bwd, ptr(x), ptr(weight), ptr(logits), dtype_code(logits), experts.data_ptr<int64_t>(),
            ptr(weights_grad), dtype_code(weights_grad), ptr(logits_grad), ptr(x_grad), ptr(dx), ptr(dw), dtype_code(dw), T, H, N, K,

@@ -469,3 +469,22 @@ def test_unfused_paths_are_announced_or_refused(cuda):
             blk(x)
     finally:
         moe.strict_fused_paths = False
+
+
+@pytest.mark.parametrize("H,N,dtype,fp32_logits", [(256, 8, torch.bfloat16, True), (2048, 64, torch.bfloat16, False), (512, 100, torch.bfloat16, True),
+                                                   (256, 8, torch.float32, True)])
+def test_training_step_without_tokens(cuda, H, N, dtype, fp32_logits):
+    """No tokens (a rank whose batch is empty): the step runs and every weight's gradient is zeros."""
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    from optimus.models.common.moe import FastOlmoeParallelSparseMoeBlock
+    from optimus.models.olmoe.configuration_olmoe import OlmoeParallelConfig
+    cfg = OlmoeParallelConfig(hidden_size=H, intermediate_size=64, num_experts=N, num_experts_per_tok=2, norm_topk_prob=True,
+                              use_fast_moe=True, use_merged_mlp_in_fast_moe=True)
+    cfg.router_logits_fp32 = fp32_logits
+    block = FastOlmoeParallelSparseMoeBlock(cfg, ParallelDpPpEpTpMapper()).to(cuda).to(dtype)
+    x = torch.empty(1, 0, H, device=cuda, dtype=dtype, requires_grad=True)
+    out, _ = block(x)
+    out.backward(torch.empty_like(out))
+    assert out.shape == x.shape == x.grad.shape
+    for name, p in block.named_parameters():
+        assert p.grad is not None and p.grad.shape == p.shape and not bool(p.grad.any()), name
