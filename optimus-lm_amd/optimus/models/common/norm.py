@@ -42,13 +42,17 @@ class RMSNormFunction(torch.autograd.Function):
         dw = torch.empty_like(weight)
         ws_bytes = _n.lib().om_rmsnorm_bwd_workspace_spread_bytes(rows, E)
         ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=h.device)
-        # h also feeds the next residual connection: its gradient is added in the kernel, or by autograd where that records the sum
-        recorded = gh is not None and torch.is_grad_enabled() and gh.requires_grad
-        added = gh.contiguous() if gh is not None and not recorded else None
+        # h also feeds the next residual connection: its gradient is added in the kernel, or behind it where the kernel cannot read it
+        # (a batch of gradients, which has no memory of its own; an address between 16-byte boundaries) or autograd records the sum
+        added = None
+        if gh is not None and not (torch.is_grad_enabled() and gh.requires_grad) and torch._C._has_storage(gh):
+            added = gh.contiguous()
+            if added.data_ptr() % 16:
+                added = None
         _n.check(_n.lib().om_rmsnorm_bwd_residual(_n.ptr(gy), _n.ptr(h), _n.ptr(weight), _n.ptr(rstd),
                                                   _n.ptr(added), _n.ptr(dx), _n.ptr(dw), _n.ptr(ws), ws_bytes,
                                                   rows, E, _n.dtype_code(h), _n.stream()), "om_rmsnorm_bwd_residual")
-        if recorded:
+        if gh is not None and added is None:
             dx = dx + gh
         return dx, (dx if ctx.has_residual else None), dw, None
 

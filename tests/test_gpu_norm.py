@@ -107,3 +107,30 @@ def test_rows_that_a_wavefront_holds(cuda, rows, vecs, dtype):
     terms = gd * xn.to(dtype).double()
     bound = eps * terms.sum(0).abs() + terms.abs().sum(0) * (2.0 ** -24 * (rows / 4 + 8) + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -22))
     assert bool(((m.weight.grad.cpu().double() - terms.sum(0)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("E", [256, 2056])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_residual_gradients_that_the_kernel_does_not_read(cuda, E, dtype):
+    """A gradient of h between 16-byte boundaries (a part of a larger tensor's) and a batch of them: dx + gh, as with one that it reads."""
+    from optimus.models.olmoe.modeling_olmoe import OlmoeParallelRMSNorm
+    rows = 7
+    x, res, w = (t.to(cuda) for t in _inputs(rows, E, dtype, seed=E))
+    m = OlmoeParallelRMSNorm(E, eps=1e-5).to(dtype).to(cuda)
+    with torch.no_grad():
+        m.weight.copy_(w)
+    x.requires_grad_(True)
+    y, h = m.forward_with_residual(x, res)
+    gen = torch.Generator(device=cuda).manual_seed(1)
+    gy, gh = (torch.randn(rows, E, generator=gen, device=cuda).to(dtype) for _ in range(2))
+    want = torch.autograd.grad([y, h], [x, m.weight], [gy, gh], retain_graph=True)
+    shifted = torch.empty(rows * E + 1, dtype=dtype, device=cuda)[1:].view(rows, E).copy_(gh)
+    assert shifted.data_ptr() % 16 and shifted.is_contiguous()
+    got = torch.autograd.grad([y, h], [x, m.weight], [gy, shifted], retain_graph=True)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    joined = torch.cat([torch.ones(1, device=cuda, dtype=dtype), h.flatten()])    # its gradient's part is such a tensor
+    got = torch.autograd.grad([y, joined], [x], [gy, torch.cat([gh[0, :1], gh.flatten()])], retain_graph=True)
+    assert torch.equal(got[0], want[0])
+    batch = torch.stack([gh, 2 * gh, gh - 1])
+    got, = torch.autograd.grad(h, x, batch, is_grads_batched=True)
+    assert torch.equal(got, batch)                                                # (nothing comes through y)
