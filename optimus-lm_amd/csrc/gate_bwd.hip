@@ -734,8 +734,9 @@ extern "C" int om_router_gate_dgrad(const float *dlogits, const void *gate_weigh
 }
 
 namespace {
+// (with the weight gradient's blocks less than 2^32 threads)
 bool gate_bwd_shape_ok(int64_t T, int H, int N) {
-    return T >= 1 && H >= 8 && H % 8 == 0 && N >= 1 && N <= 64 && (T + DG_TOK - 1) / DG_TOK * ((H + DG_HT - 1) / DG_HT) <= (1 << 24);
+    return T >= 1 && H >= 8 && H % 8 == 0 && N >= 1 && N <= 64 && (T + DG_TOK - 1) / DG_TOK * ((H + DG_HT - 1) / DG_HT) <= (1 << 22);
 }
 int64_t gate_bwd_counts(int H) { return ((H + HT - 1) / HT + 3) / 4 * 4; }   // (16-byte aligned behind them)
 }  // namespace

@@ -132,7 +132,7 @@ extern "C" int om_router_gate_bwd_f32(const float *x, const float *dlogits, cons
     if (!x || !dlogits || !gate_weight || !dx || !dweight) return OM_ERR_NULL;
     const int64_t wgrad_blocks = static_cast<int64_t>((H + GW_H - 1) / GW_H) * ((N + GW_N - 1) / GW_N);
     const int64_t blocks = wgrad_blocks + (H + 255) / 256 * ((T + 3) / 4);
-    if (blocks > 0x7fffffffLL) {
+    if (blocks * (GW_WAVES * 64) > 0xffffffffLL) {   // (a launch of more threads runs a part of them, without an error)
         const int code = om_router_gate_wgrad_f32(x, dlogits, T, H, N, dweight, stream);
         return code == OM_OK ? om_router_gate_dgrad_f32_add(dlogits, gate_weight, base, T, H, N, dx, stream) : code;
     }

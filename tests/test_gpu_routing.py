@@ -859,3 +859,21 @@ def test_group_router_of_what_is_not_finite(cuda, T, H, N, n_group, topk_group, 
     dw, dl = torch.ones(T, K, device=cuda), torch.full((T, N), 7.0, device=cuda)
     n.check(lib.om_route_sigmoid_topk_bwd(n.ptr(logits), n.ptr(e), n.ptr(dw), T, N, K, 1, 2.5, n.ptr(dl), st), "backward")
     assert bool(torch.isnan(dl[T // 2][e[T // 2]]).all()) and bool(torch.isfinite(dl[others]).all())
+
+
+def test_float32_gate_gradients_of_more_tokens_than_one_grid_holds(cuda):
+    """A launch holds less than 2^32 threads: from there on the two gradients are launches of their own, with the same results."""
+    from optimus import _native as n
+    lib, st, T, H, N = n.lib(), n.stream(), (1 << 24) + 3, 8, 2
+    g = torch.Generator(device=cuda).manual_seed(1)
+    x, dl = (torch.randn(T, k, generator=g, device=cuda) for k in (H, N))
+    w = torch.randn(N, H, generator=g, device=cuda)
+    dx, dw = torch.full((T, H), 7.0, device=cuda), torch.full((N, H), 7.0, device=cuda)
+    n.check(lib.om_router_gate_bwd_f32(n.ptr(x), n.ptr(dl), n.ptr(w), None, T, H, N, n.ptr(dx), n.ptr(dw), st), "both")
+    want_dx, want_dw = torch.empty_like(dx), torch.empty_like(dw)
+    n.check(lib.om_router_gate_dgrad_f32(n.ptr(dl), n.ptr(w), T, H, N, n.ptr(want_dx), st), "dx")
+    n.check(lib.om_router_gate_wgrad_f32(n.ptr(x), n.ptr(dl), T, H, N, n.ptr(want_dw), st), "dw")
+    assert torch.equal(dx, want_dx) and torch.equal(dw, want_dw)
+    # two products and their sum, a rounding each
+    ref = dl[-5:].double() @ w.double()
+    assert bool(((dx[-5:].double() - ref).abs() <= 3 * 2.0 ** -24 * (dl[-5:].double().abs() @ w.double().abs())).all())
