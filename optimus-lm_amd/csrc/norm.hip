@@ -267,8 +267,9 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rows_kernel(const T *__restri
 }
 inline int64_t bwd_chunk(int64_t rows) { return (rows + 2047) / 2048 * 4; }
 
-// dx of longer rows (and with little workspace), one wavefront per row, read twice.
-template <typename T>
+// dx of longer rows, and with little workspace, one wavefront per row.  Rows that fit the registers are read once (16384 rows of 2048 bf16,
+// the whole backward, operands in the caches: 77 us read twice, 62 so; 4096 rows 39 and 36); longer ones twice.
+template <typename T, bool FITS, bool ADD>
 __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ dy,
                                                          const T *__restrict__ h,
                                                          const T *__restrict__ weight,
@@ -284,6 +285,7 @@ __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ d
     const u32x4 *dyr = reinterpret_cast<const u32x4 *>(dy + row * E);
     const u32x4 *hr = reinterpret_cast<const u32x4 *>(h + row * E);
     u32x4 *dxr = reinterpret_cast<u32x4 *>(dx + row * E);
+    float dxn[ROW_VECS][V], xn[ROW_VECS][V];   // FITS: of the whole row
     float dot = 0.0f;
     for (int64_t c0 = 0; c0 < nv; c0 += 64 * ROW_VECS) {
 #pragma unroll
@@ -295,7 +297,11 @@ __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ d
                 Elem<T>::unpack(hr[c], f);
                 Elem<T>::unpack(wr[c], w);
 #pragma unroll
-                for (int j = 0; j < V; j++) dot += (g[j] * w[j]) * (f[j] * r);
+                for (int j = 0; j < V; j++) {
+                    xn[u][j] = f[j] * r;
+                    dxn[u][j] = g[j] * w[j];
+                    dot += dxn[u][j] * xn[u][j];
+                }
             }
         }
     }
@@ -305,13 +311,18 @@ __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ d
         for (int u = 0; u < ROW_VECS; u++) {
             const int64_t c = c0 + u * 64 + lane;
             if (c < nv) {
-                float g[V], f[V], w[V], o[V];
-                Elem<T>::unpack(dyr[c], g);
-                Elem<T>::unpack(hr[c], f);
-                Elem<T>::unpack(wr[c], w);
+                if (!FITS) {
+                    float g[V], f[V], w[V];
+                    Elem<T>::unpack(dyr[c], g);
+                    Elem<T>::unpack(hr[c], f);
+                    Elem<T>::unpack(wr[c], w);
 #pragma unroll
-                for (int j = 0; j < V; j++) o[j] = r * (g[j] * w[j] - (f[j] * r) * dot);
-                if (h_grad) add_rounded<T>(reinterpret_cast<const u32x4 *>(h_grad + row * E)[c], o);
+                    for (int j = 0; j < V; j++) { xn[u][j] = f[j] * r; dxn[u][j] = g[j] * w[j]; }
+                }
+                float o[V];
+#pragma unroll
+                for (int j = 0; j < V; j++) o[j] = r * (dxn[u][j] - xn[u][j] * dot);
+                if (ADD) add_rounded<T>(reinterpret_cast<const u32x4 *>(h_grad + row * E)[c], o);
                 dxr[c] = Elem<T>::pack(o);
             }
         }
@@ -370,14 +381,13 @@ __global__ __launch_bounds__(4 * DW_REDUCE) void rmsnorm_dw_reduce_kernel(const 
     int b = n_blocks * wave / 4;
     float s = 0.0f;
     if (e < E) {
-        for (; b + 16 <= end; b += 16) {
+        for (; b < end; b += 16) {         // (past the last of them: it again, not added)
             float v[16];
 #pragma unroll
-            for (int u = 0; u < 16; u++) v[u] = dw_part[static_cast<int64_t>(b + u) * E + e];
+            for (int u = 0; u < 16; u++) v[u] = dw_part[static_cast<int64_t>(min(b + u, end - 1)) * E + e];
 #pragma unroll
-            for (int u = 0; u < 16; u++) s += v[u];
+            for (int u = 0; u < 16; u++) s += b + u < end ? v[u] : 0.0f;
         }
-        for (; b < end; b++) s += dw_part[static_cast<int64_t>(b) * E + e];
     }
     quarter[wave][lane] = s;
     __syncthreads();
@@ -475,7 +485,12 @@ extern "C" int om_rmsnorm_bwd_residual(const void *dy, const void *h, const void
         });
         if (!fits) {
             chunks = static_cast<int>((rows + DW_ROWS - 1) / DW_ROWS);
-            rmsnorm_dx_kernel<T><<<static_cast<unsigned>((rows + NORM_ROWS - 1) / NORM_ROWS), 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            const dim3 grid(static_cast<unsigned>((rows + NORM_ROWS - 1) / NORM_ROWS));
+            const bool row_fits = E / V <= 64 * ROW_VECS;
+            if (row_fits && hg) rmsnorm_dx_kernel<T, true, true><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            else if (row_fits) rmsnorm_dx_kernel<T, true, false><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            else if (hg) rmsnorm_dx_kernel<T, false, true><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            else rmsnorm_dx_kernel<T, false, false><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
             rmsnorm_dw_kernel<T><<<dim3(static_cast<unsigned>((E / V + 63) / 64), static_cast<unsigned>(chunks)), 256, 0, st>>>(g, hh, rstd, part, rows, E);
         }
         rmsnorm_dw_reduce_kernel<T><<<static_cast<unsigned>((E + DW_REDUCE - 1) / DW_REDUCE), 4 * DW_REDUCE, 0, st>>>(part, chunks, E, static_cast<T *>(dweight));

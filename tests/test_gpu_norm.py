@@ -134,3 +134,32 @@ def test_residual_gradients_that_the_kernel_does_not_read(cuda, E, dtype):
     batch = torch.stack([gh, 2 * gh, gh - 1])
     got, = torch.autograd.grad(h, x, batch, is_grads_batched=True)
     assert torch.equal(got, batch)                                                # (nothing comes through y)
+
+
+@pytest.mark.parametrize("rows,vecs", [(1, 1), (131, 64), (700, 250), (2100, 256), (300, 257), (17 * 128, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("add", [False, True])
+def test_backward_with_the_least_workspace(cuda, rows, vecs, dtype, add):
+    """om_rmsnorm_bwd_workspace_bytes, where the other size spreads the rows over more chunks: the same bits of dx, the weight gradient's
+    sums in another order."""
+    from optimus import _native as n
+    L, st, E = n.lib(), n.stream(), vecs * (8 if dtype == torch.bfloat16 else 4)
+    gen = torch.Generator(device=cuda).manual_seed(rows + vecs)
+    dy, h, gh = (torch.randn(rows, E, generator=gen, device=cuda).to(dtype) for _ in range(3))
+    w, rstd = torch.randn(E, generator=gen, device=cuda).to(dtype), torch.rand(rows, generator=gen, device=cuda) + 0.5
+    got = []
+    for size in (L.om_rmsnorm_bwd_workspace_bytes(rows, E), L.om_rmsnorm_bwd_workspace_spread_bytes(rows, E)):
+        dx, dw = torch.full_like(h, 7.0), torch.full_like(w, 7.0)
+        ws = torch.empty(size, dtype=torch.uint8, device=cuda)
+        n.check(L.om_rmsnorm_bwd_residual(n.ptr(dy), n.ptr(h), n.ptr(w), n.ptr(rstd), n.ptr(gh) if add else None, n.ptr(dx), n.ptr(dw), n.ptr(ws),
+                                          size, rows, E, n.dtype_code(h), st), "backward")
+        got.append((dx, dw))
+    assert torch.equal(got[0][0], got[1][0])
+    # either is within one rounding of the result and a float32 rounding a term of the sum of dy * cast(h * rstd)
+    terms = dy.double() * (h.float() * rstd[:, None]).to(dtype).double()
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23
+    for _, dw in got:
+        assert bool(((dw.double() - terms.sum(0)).abs() <= eps * terms.sum(0).abs() + rows * 2.0 ** -24 * terms.abs().sum(0)).all())
+    with_ws = lambda size: L.om_rmsnorm_bwd(n.ptr(dy), n.ptr(h), n.ptr(w), n.ptr(rstd), n.ptr(got[0][0]), n.ptr(got[0][1]), n.ptr(ws), size, rows, E,
+                                            n.dtype_code(h), st)
+    assert with_ws(L.om_rmsnorm_bwd_workspace_bytes(rows, E) - 1) != 0
