@@ -114,7 +114,8 @@ def _grouped_gemm(kind, a, b, out, cum, rows, G, N, K, w_stride, accumulate=Fals
 # ----------------------------------------------------------------------------------------------
 def gate_kernel_unfit_reason(x, weight):
     """None when the fused gate + routing kernel (om_router_gate_softmax_topk) takes these operands,
-    else why not."""
+    else why not.  (om_router_gate_split_softmax_topk takes the others; for small gates, up to 64 experts
+    and 65536 weights, that is one launch too, but not this kernel.)"""
     if not (x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16):
         return f"operands are not bfloat16 device tensors ({x.dtype}, {weight.dtype})"
     N, H = weight.shape
@@ -886,7 +887,8 @@ class FastOlmoeParallelSparseMoeBlock(nn.Module):
         gate_unfit = gate_kernel_unfit_reason(flat, self.gate.weight) if self.router_logits_fp32 else None
         if self.router_logits_fp32 and gate_unfit is not None and flat.dtype == torch.bfloat16:
             note_unfused_path("gate projection fused with the routing", gate_unfit,
-                              instead="running the projection and the routing as separate kernels (same fp32 logits)")
+                              instead="running the kernels of other hidden sizes (same fp32 logits): one launch for a small gate, "
+                                      "else the projection and the routing as separate kernels")
         # (the experts are fed from the router's pass-through of the hidden states, so that their input
         # gradient and the gate's are added in one kernel)
         weight = self.gate.weight.contiguous()
