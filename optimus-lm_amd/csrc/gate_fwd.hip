@@ -149,7 +149,8 @@ __global__ __launch_bounds__(64) void gate_logits_few_kernel(const uint16_t *__r
     const int n0 = blockIdx.x * 16, split = blockIdx.y;
     const int64_t t = static_cast<int64_t>(blockIdx.z) * 16 + l16;
     const int begin = split * h_per_split, len = min(H - begin, h_per_split);
-    // rows past the end (tokens, experts): the last one, results unused; columns past the end: the last chunk again, of tokens zeros
+    // rows past the end (tokens, experts): the last one, results unused; columns past the end: the last chunk again, as zeros (of both: zero
+    // times an infinite weight is NaN)
     const uint16_t *xr = x + min(t, T - 1) * H + begin, *wr = w + static_cast<int64_t>(min(n0 + l16, N - 1)) * H + begin;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int c = 0; c < len; c += CH * 32) {
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64) void gate_logits_few_kernel(const uint16_t *__r
             const int k = c + i * 32 + g * 8, at = min(k, len - 8);
             wf[i] = *reinterpret_cast<const u32x4 *>(wr + at);
             xf[i] = *reinterpret_cast<const u32x4 *>(xr + at);
-            if (k >= len) xf[i] = u32x4{0, 0, 0, 0};
+            if (k >= len) wf[i] = xf[i] = u32x4{0, 0, 0, 0};
         }
 #pragma unroll
         for (int i = 0; i < CH; i++)

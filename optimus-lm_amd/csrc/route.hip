@@ -858,13 +858,17 @@ __global__ __launch_bounds__(NH * 512) void gate_route_rows_kernel(const uint16_
     for (int m = 0; m < 2; m++) w_row[m] = static_cast<uint32_t>(min(half * 32 + m * 16 + l16, N - 1)) * static_cast<uint32_t>(H) * 2;
     u32x4 wf[CH][2], xf[CH];
     auto at = [](const uint16_t *base, uint32_t bytes) { return *reinterpret_cast<const u32x4 *>(reinterpret_cast<const char *>(base) + bytes); };
-    // byte of the lane's chunk in piece i of CH that `columns` are left of: past them the last chunk again, of tokens zeros
+    // byte of the lane's chunk in piece i of CH that `columns` are left of: past them the last chunk again, as zeros (of both: zero times an
+    // infinite weight is NaN)
     auto chunk = [&](int i, int columns) { return static_cast<uint32_t>(WHOLE ? i * 32 + g * 8 : min(i * 32 + g * 8, columns - 8)) * 2; };
     auto load_w = [&](int begin, int columns) {
 #pragma unroll
         for (int i = 0; i < CH; i++)
 #pragma unroll
-            for (int m = 0; m < 2; m++) wf[i][m] = at(wg + begin, w_row[m] + chunk(i, columns));
+            for (int m = 0; m < 2; m++) {
+                wf[i][m] = at(wg + begin, w_row[m] + chunk(i, columns));
+                if (!WHOLE && i * 32 + g * 8 >= columns) wf[i][m] = u32x4{0, 0, 0, 0};
+            }
     };
     auto load_x = [&](int64_t tile, int begin, int columns) {
         const uint32_t row = static_cast<uint32_t>(min(static_cast<int64_t>(l16), Tn - 1 - tile * ROWS_TOKENS)) * static_cast<uint32_t>(H) * 2;

@@ -877,3 +877,34 @@ def test_float32_gate_gradients_of_more_tokens_than_one_grid_holds(cuda):
     # two products and their sum, a rounding each
     ref = dl[-5:].double() @ w.double()
     assert bool(((dx[-5:].double() - ref).abs() <= 3 * 2.0 ** -24 * (dl[-5:].double().abs() @ w.double().abs())).all())
+
+
+# slices of 64, 128, 192 and 256 columns, whole ones and shorter last ones, taken in pieces of 64, 128 and 256 columns; both kinds of kernel
+@pytest.mark.parametrize("T,H,N,K", [(1, 1536, 64, 8), (37, 1536, 17, 3), (64, 2880, 128, 4), (5, 1088, 96, 2), (3, 2048, 64, 8), (33, 1096, 65, 2),
+                                     (40, 776, 40, 8), (300, 1000, 12, 3), (2049, 1088, 20, 4), (50, 256, 8, 2)])
+def test_infinite_gate_weights_meet_their_own_tokens_only(cuda, T, H, N, K):
+    """An expert whose weights are all infinite, behind positive tokens: its logits are infinite (not NaN, as by a column past a slice's end, whose
+    token counts as zero), the others' are those of any weight there."""
+    from optimus import _native as n
+    lib, st = n.lib(), n.stream()
+    x, w = (t.to(cuda) for t in _gate_inputs(T, H, N, seed=T + H))
+    x = x.abs() + 0.125
+    bad = w.clone()
+    bad[N // 2] = float("inf")
+    others = [i for i in range(N) if i != N // 2]
+    got = []
+    for weight in (w, bad):
+        logits, ws = torch.empty(T, N, device=cuda), torch.empty(lib.om_router_gate_logits_split_workspace_bytes(T, H, N), dtype=torch.uint8, device=cuda)
+        if N > 64 or T <= 512:
+            n.check(lib.om_router_gate_logits_split(n.ptr(x), n.ptr(weight), T, H, N, n.ptr(logits), n.ptr(ws), ws.numel(), st), "logits")
+            got.append(logits)
+        if N <= 64:
+            logits, experts = torch.empty(T, N, device=cuda), torch.empty(T, K, dtype=torch.int64, device=cuda)
+            weights = torch.empty(T, K, device=cuda)
+            ws = torch.empty(max(lib.om_router_gate_route_workspace_bytes(T, H, N), 16), dtype=torch.uint8, device=cuda)
+            n.check(lib.om_router_gate_split_softmax_topk(n.ptr(x), n.ptr(weight), T, H, N, K, 0, n.ptr(logits), n.OM_F32, n.ptr(weights), n.OM_F32,
+                                                          n.ptr(experts), n.ptr(ws), ws.numel(), st), "router")
+            got.append(logits)
+    half = len(got) // 2
+    for fine, infinite in zip(got[:half], got[half:]):
+        assert bool(torch.isposinf(infinite[:, N // 2]).all()) and torch.equal(infinite[:, others], fine[:, others])
