@@ -968,3 +968,35 @@ def test_input_and_weight_gradients_in_one_call_are_those_of_two(cuda, rows_e, I
     assert call(0, I) == call(rows, I + 4) == L.om_merged_mlp_gate_up_dgrad(P(dg), P(du), P(wg), P(wu), P(dx), P(cum), rows, G, I + 4, H, 0,
                                                                           n.stream())
     assert L.om_merged_mlp_backward_joins(rows, G, I, H) == (0 if (I, H) == (1024, 2048) else 1)
+
+
+@pytest.mark.parametrize("rows_e,I,H", [((0, 3, 0), 8, 16), ((130, 0, 1, 257), 200, 136), ((700, 0, 129, 500, 1000), 712, 1000), ((300, 500), 1024, 2048)])
+@pytest.mark.parametrize("accumulate", [0, 1])
+def test_input_and_weight_gradients_in_one_call_over_a_bound_of_the_rows(cuda, rows_e, I, H, accumulate):
+    """As under an expert window: the buffers and `rows` are those of all pairs, `expected` lies between, below or above what the device counts.
+    The bits of the two entry points over the same bound, rows past the routed ones neither read (they hold NaN) nor written."""
+    from optimus import _native as n
+    L, P, G, routed, T = n.lib(), n.ptr, len(rows_e), sum(rows_e), 501
+    rows = 4 * routed + 61
+    gen = torch.Generator(device=cuda).manual_seed(routed + I)
+    bf = lambda *s: (torch.randn(*s, generator=gen, device=cuda) * 0.1).bfloat16()
+    x, dy, h, dg, du = bf(T, H), bf(T, H), bf(rows, I), bf(rows, I), bf(rows, I)
+    for t in (h, dg, du):
+        t[routed:] = float("nan")
+    wg, wu = bf(G, I, H), bf(G, I, H)
+    cum = torch.tensor([0] + list(torch.tensor(rows_e).cumsum(0)), dtype=torch.int32, device=cuda)
+    index = torch.randint(0, T, (rows,), generator=gen, device=cuda, dtype=torch.int32)
+    index[routed:] = 0
+    start = [bf(G, H, I), bf(G, I, H), bf(G, I, H)]
+    wgrad = L.om_grouped_gemm_wgrad_merged_accumulate_bound if accumulate else L.om_grouped_gemm_wgrad_merged_bound
+    both = L.om_grouped_gemm_wgrad_merged_dgrad_accumulate if accumulate else L.om_grouped_gemm_wgrad_merged_dgrad
+    for expected in (routed // 2, (routed + rows) // 2, rows):
+        got, want = [t.clone() for t in start], [t.clone() for t in start]
+        dx, dx_want = torch.full((2, rows, H), 7.0, dtype=torch.bfloat16, device=cuda)
+        n.check(wgrad(P(dy), P(index), P(h), P(dg), P(du), P(x), P(index), T, *(P(t) for t in want), P(cum), rows, expected, G, I, H, 0, 0, 0,
+                      n.stream()), "weights")
+        n.check(L.om_merged_mlp_gate_up_dgrad_bound(P(dg), P(du), P(wg), P(wu), P(dx_want), P(cum), rows, expected, G, I, H, 0, n.stream()), "input")
+        n.check(both(P(dy), P(index), P(h), P(dg), P(du), P(x), P(index), T, P(wg), P(wu), P(dx), *(P(t) for t in got), P(cum), rows, expected,
+                     G, I, H, 0, 0, 0, 0, n.stream()), "both")
+        assert torch.equal(dx, dx_want) and all(torch.equal(a, b) for a, b in zip(got, want)), expected
+        assert bool((dx[routed:] == 7.0).all()) and bool(torch.isfinite(dx).all()) and all(bool(torch.isfinite(t).all()) for t in got)

@@ -488,3 +488,54 @@ def test_training_step_without_tokens(cuda, H, N, dtype, fp32_logits):
     assert out.shape == x.shape == x.grad.shape
     for name, p in block.named_parameters():
         assert p.grad is not None and p.grad.shape == p.shape and not bool(p.grad.any()), name
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 2048, 64, 8), (37, 2048, 64, 8), (64, 1536, 32, 3), (5, 3000, 64, 16)])
+@pytest.mark.parametrize("parallel,sync_free", [(1, False), (4, False), (4, True)])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_router_that_sorts_gives_the_layer_of_one_that_does_not(cuda, monkeypatch, T, H, N, K, parallel, sync_free, with_residual):
+    """Few tokens: the permutation that the router's launch made against the one that the experts' call makes, alone and under an expert window;
+    output and every gradient bit for bit."""
+    from optimus import _native as n
+    from optimus.mapper import ParallelDpPpEpTpMapper
+    from optimus.models.common.moe import FastOlmoeParallelSparseMoeBlock
+    from optimus.models.olmoe.configuration_olmoe import OlmoeParallelConfig
+    assert n.lib().om_router_gate_softmax_topk_sort_fits(T, H, N, K) == 1
+    cfg = OlmoeParallelConfig(hidden_size=H, intermediate_size=72, num_experts=N, num_experts_per_tok=K, norm_topk_prob=True,
+                              use_fast_moe=True, use_merged_mlp_in_fast_moe=True, expert_parallelism=parallel)
+    cfg.sync_free_expert_window = sync_free
+    torch.manual_seed(T)
+    block = FastOlmoeParallelSparseMoeBlock(cfg, ParallelDpPpEpTpMapper(expert_parallelism=parallel, rank=parallel // 2))
+    for p in block.parameters():
+        torch.nn.init.normal_(p, std=0.03)
+    block = block.to(cuda).to(torch.bfloat16)
+    assert block.sync_free_expert_window == sync_free and block.expert_end_idx - block.expert_start_idx == N // parallel
+    g = torch.Generator().manual_seed(T + H)
+    x, dout, residual = (torch.randn(T, 1, H, generator=g).bfloat16().to(cuda) for _ in range(3))
+    host, made = n.host(), []
+
+    class Host:
+        sorts = True
+
+        def __getattr__(self, name):
+            return getattr(host, name)
+
+        def route_softmax_sorted(self, *args):
+            r = host.route_softmax_sorted(*(args if self.sorts else args[:-2] + (0, 0)))
+            made.append(r[4] is not None)
+            return r
+    proxy = Host()
+    monkeypatch.setattr(n, "host", lambda: proxy)
+    results = []
+    for proxy.sorts in (True, False):
+        xi, ri = x.clone().requires_grad_(True), residual.clone().requires_grad_(True)
+        with torch.no_grad():
+            alone = block(xi, residual=ri if with_residual else None)[0]
+        block.zero_grad(set_to_none=True)
+        out = block(xi, residual=ri if with_residual else None)[0]
+        out.backward(dout)
+        assert torch.equal(out, alone)
+        results.append([out.detach(), xi.grad] + ([ri.grad] if with_residual else []) + [p.grad for p in block.parameters()])
+    assert made == [True, True, False, False]
+    for a, b in zip(*results):
+        assert a is b is None or torch.equal(a, b)     # (None: a window that no token reached)

@@ -166,3 +166,23 @@ def test_row_sum_with_the_routing_weights_gradient(cuda, oracle_lib, T, N, K, E,
         ref = torch.zeros(T, K)
         ref[torch.from_numpy(token), torch.from_numpy(idx["selected_experts_indices"]).long()] = sums[torch.from_numpy(idx["output_indices"]).long()]
         assert torch.equal(dw.cpu(), ref.to(wdt))
+
+
+@pytest.mark.parametrize("T,N,K,I,start,end,wdt", [(8, 4, 2, 8, 0, 4, torch.bfloat16), (80, 8, 3, 200, 0, 8, torch.float32), (704, 16, 8, 1048, 4, 6, torch.float32),
+                                                   (600, 130, 70, 64, 0, 130, torch.bfloat16)])
+def test_routing_weights_gradient_alone(cuda, oracle_lib, T, N, K, I, start, end, wdt):
+    """om_moe_row_weights_grad: the column ranges added in order; entries of pairs outside the window keep what they held."""
+    from optimus import _native as n
+    _, idx, _, _, _ = _setup(T, N, K, 8, start, end, torch.bfloat16, oracle_lib, seed=T)
+    TR, parts = idx["num_routed_tokens"], n.lib().om_merged_mlp_row_dot_parts(I)
+    dot = torch.randn(parts, TR, generator=torch.Generator().manual_seed(4))
+    ii, oi, si = (torch.from_numpy(idx[k]).to(cuda) for k in ("input_indices", "output_indices", "selected_experts_indices"))
+    dotg, dw = dot.to(cuda), torch.full((T, K), 7.0, dtype=wdt, device=cuda)
+    n.check(n.lib().om_moe_row_weights_grad(n.ptr(dotg), parts, n.ptr(si), n.ptr(ii), n.ptr(oi), n.ptr(dw), TR, K, n.dtype_code(dw), n.stream()), "gradient")
+    sums = torch.zeros(TR)
+    for part in dot:
+        sums += part
+    pos = torch.from_numpy(idx["output_indices"]).long()
+    ref = torch.full((T, K), 7.0)
+    ref[torch.from_numpy(idx["input_indices"]).long()[pos], torch.from_numpy(idx["selected_experts_indices"]).long()] = sums[pos]
+    assert torch.equal(dw.cpu(), ref.to(wdt))
