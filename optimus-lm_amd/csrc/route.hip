@@ -828,10 +828,8 @@ __global__ __launch_bounds__(1024) void partial_softmax_topk_sort_kernel(const f
     }
     __syncthreads();
     const int n_pairs = Tn * K, pair = min(static_cast<int>(threadIdx.x), n_pairs - 1);
-    const int e[1] = {pair_expert[pair]};
-    const float w[1] = {pair_weight[pair]};
-    sort_block<16, 1>(e, w, n_pairs, K, out.start, out.end, out.end - out.start, out.nbits, out.cum_token_counts, out.cum_expert_counts_ep,
-                      out.input_indices, out.output_indices, out.selected_experts_indices, out.row_weights);
+    sort_block(pair_expert[pair], pair_weight[pair], n_pairs, K, out.start, out.end, out.end - out.start, out.nbits, out.cum_token_counts,
+               out.cum_expert_counts_ep, out.input_indices, out.output_indices, out.selected_experts_indices, out.row_weights);
 }
 
 // Projection and routing of up to 64 experts in one launch, 16 tokens at a time, for gates of a small weight: what bounds those is a chain of

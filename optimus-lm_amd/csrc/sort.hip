@@ -7,12 +7,13 @@
 //             (expert-major, block-minor) order = the stable order, and writes cum_token_counts;
 //   scatter — every block re-reads its chunk and places each pair at offset + stable rank.
 // Ranks come from wavefront ballots (lanes holding the same expert form a mask; rank = popcount of
-// the mask below the lane), per-wave running offsets live in LDS: no atomics, so the result is
-// deterministic.
+// the mask below the lane), per-wave running offsets live in LDS.  Atomics only count (sort_spread_kernel,
+// whole numbers in LDS, a sum that no order changes), so the result is deterministic.
 // The three launches move a few bytes per pair and wait all the time: a wavefront's steps are a serial chain.
 // Hence eight wavefronts of four steps per block (it was four of eight), and a wavefront's keys and weights
 // fetched at once, not step by step: us, count + scan + scatter, 32768 pairs of 64 experts 9.2 + 6.7 + 21.4 ->
-// 5.3 + 6.3 + 11.6, 9003 pairs of 12 7.0 + 3.1 + 16.3 -> 4.0 + 3.0 + 8.4.
+// 5.3 + 6.3 + 11.6, 9003 pairs of 12 7.0 + 3.1 + 16.3 -> 4.0 + 3.0 + 8.4 (sizes that took three launches then; 131072 pairs, which do
+// now, 21.3 in all).
 // Also: the reference's two index operators with their own [expert][column] table layout, one
 // wavefront per column.
 #include "sort_block.h"
@@ -231,18 +232,14 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_scatter_kernel(
 }
 
 // Few pairs: count, scan and scatter by one block, in one launch (sort_block.h).
-constexpr int SMALL_WAVES = 16;
-constexpr int64_t SMALL_PAIRS = SMALL_WAVES * 64;
 template <typename TI>
-__global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
+__global__ __launch_bounds__(SORT_BLOCK_PAIRS) void sort_small_kernel(
     const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
     int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
     int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
     int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
-    const TI e[1] = {selected_experts[min(static_cast<int>(threadIdx.x), n_pairs - 1)]};
-    const float weight[1] = {rw.get(threadIdx.x, n_pairs)};
-    sort_block<SMALL_WAVES, 1>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
-                               output_indices, selected_experts_indices, rw.row_weights);
+    sort_block(selected_experts[min(static_cast<int>(threadIdx.x), n_pairs - 1)], rw.get(threadIdx.x, n_pairs), n_pairs, K, start, end, NR, nbits,
+               cum_token_counts, cum_expert_counts_ep, input_indices, output_indices, selected_experts_indices, rw.row_weights);
 }
 
 // More pairs in one launch: a block sorts 1024 of them, as above, and counts all the others by itself, with LDS atomics on eight
@@ -254,17 +251,17 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_small_kernel(
 constexpr int64_t SPREAD_PAIRS = 1 << 16;
 // VEC: selections in a load, 16 bytes of them where they are aligned
 template <typename TI, int VEC>
-__global__ __launch_bounds__(SMALL_WAVES * 64) void sort_spread_kernel(
+__global__ __launch_bounds__(SORT_BLOCK_PAIRS) void sort_spread_kernel(
     const TI *__restrict__ selected_experts, int n_pairs, int K, int start, int end, int NR, int nbits,
     int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
     int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
     int32_t *__restrict__ selected_experts_indices, const RowWeights rw) {
-    constexpr int THREADS = SMALL_WAVES * 64, AHEAD = 8, CELLS = SORT_BLOCK_MAX_NR * SPREAD_COPIES;
+    constexpr int THREADS = SORT_BLOCK_PAIRS, AHEAD = 8, CELLS = SORT_BLOCK_MAX_NR * SPREAD_COPIES;
     typedef TI vec __attribute__((ext_vector_type(VEC)));
     __shared__ int counts[2 * CELLS];   // of the pairs before this block's and of those after them
     const int tid = threadIdx.x, first = blockIdx.x * THREADS, last = min(first + THREADS, n_pairs);
-    const TI e[1] = {selected_experts[min(first + tid, n_pairs - 1)]};
-    const float weight[1] = {rw.get(first + tid, n_pairs)};
+    const TI e = selected_experts[min(first + tid, n_pairs - 1)];
+    const float weight = rw.get(first + tid, n_pairs);
     for (int i = tid; i < 2 * CELLS; i += THREADS) counts[i] = 0;
     __syncthreads();
     const int n_vec = n_pairs / VEC, copy = tid % SPREAD_COPIES;
@@ -287,8 +284,8 @@ __global__ __launch_bounds__(SMALL_WAVES * 64) void sort_spread_kernel(
     }
     if (tid < n_pairs - n_vec * VEC) count(selected_experts[n_vec * VEC + tid], n_vec * VEC + tid);
     // (sort_block's first barrier comes before it reads the counts)
-    sort_block<SMALL_WAVES, 1, true>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices,
-                                     output_indices, selected_experts_indices, rw.row_weights, {first, counts, counts + CELLS});
+    sort_block<true>(e, weight, n_pairs, K, start, end, NR, nbits, cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
+                     selected_experts_indices, rw.row_weights, {first, counts, counts + CELLS});
 }
 
 // ---- the reference's table layout [expert][column] ---------------------------------------------
@@ -413,11 +410,11 @@ int moe_sort_launch(const void *selected_experts, int index_dtype, int64_t T, in
     const int NR = expert_end_idx - expert_start_idx;
     const int64_t n_pairs = T * K;
     if (n_pairs > 0 && n_pairs <= SPREAD_PAIRS && NR <= SORT_BLOCK_MAX_NR) {
-        const unsigned blocks = static_cast<unsigned>((n_pairs + SMALL_PAIRS - 1) / SMALL_PAIRS);
+        const unsigned blocks = static_cast<unsigned>((n_pairs + SORT_BLOCK_PAIRS - 1) / SORT_BLOCK_PAIRS);
         auto sort = [&](const auto *experts) {
             using TI = std::remove_const_t<std::remove_pointer_t<decltype(experts)>>;
             auto launch = [&](auto kernel) {
-                kernel<<<blocks, SMALL_WAVES * 64, 0, st>>>(experts, static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR, key_bits(NR),
+                kernel<<<blocks, SORT_BLOCK_PAIRS, 0, st>>>(experts, static_cast<int>(n_pairs), K, expert_start_idx, expert_end_idx, NR, key_bits(NR),
                                                             cum_token_counts, cum_expert_counts_ep, input_indices, output_indices,
                                                             selected_experts_indices, rw);
             };

@@ -32,10 +32,9 @@ inline int key_bits(int NR) {  // keys 0..NR (NR = "not local")
     return b;
 }
 
-// Few pairs: count, scan and scatter by one block, in one launch.  A wavefront keeps its (ITERS x 64) pairs' keys, weights and ranks in
-// registers between the passes.  A decode batch or a small training batch spends nothing on bandwidth here, only on latencies.
-// So no step waits for another's loads (ITERS, the 64-pair steps of a wavefront, is known to the compiler, and pairs past the end are
-// read as the last one), the rank of a pair within its expert comes from the counting pass, and only that pass is a chain through LDS.
+// Few pairs: count, scan and scatter by one block, in one launch.  A thread keeps its pair's key, weight and rank in registers between the
+// passes.  A decode batch or a small training batch spends nothing on bandwidth here, only on latencies.  So pairs past the end are read
+// as the last one, not behind a condition, and the rank of a pair within its expert comes from the counting pass.
 constexpr int SORT_BLOCK_MAX_NR = 256;
 // Of a block that sorts some of the pairs: the first of them, and how many pairs of an expert come before the first and after the last, as
 // SPREAD_COPIES counts each that are added up here.
@@ -44,38 +43,31 @@ struct SpreadPart {
     int first;
     const int *before, *after;   // LDS, [expert][SPREAD_COPIES]
 };
-// Thread t of a wavefront's ITERS * 64 pairs (wavefront-major, step by step): e and weight; pairs past the end hold anything.
-// SPREAD: the block sorts the pairs from part.first on, otherwise all of them.
-template <int WAVES, int ITERS, bool SPREAD = false, typename TI>
-__device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&weight)[ITERS], int n_pairs, int K, int start, int end, int NR,
-                                           int nbits, int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
+// e and weight: of this thread's pair; past the last pair anything.  SPREAD: the block sorts the pairs from part.first on, otherwise all of
+// them.
+constexpr int SORT_BLOCK_WAVES = 16, SORT_BLOCK_PAIRS = SORT_BLOCK_WAVES * 64;
+template <bool SPREAD = false, typename TI>
+__device__ __forceinline__ void sort_block(const TI e, const float weight, int n_pairs, int K, int start, int end, int NR, int nbits,
+                                           int32_t *__restrict__ cum_token_counts, int32_t *__restrict__ cum_expert_counts_ep,
                                            int32_t *__restrict__ input_indices, int32_t *__restrict__ output_indices,
                                            int32_t *__restrict__ selected_experts_indices, float *__restrict__ row_weights,
                                            const SpreadPart part = {}) {
+    constexpr int WAVES = SORT_BLOCK_WAVES;
     __shared__ int off[WAVES][SORT_BLOCK_MAX_NR];   // counts, then the first position of a wavefront's rows of an expert
     __shared__ __attribute__((aligned(16))) int wave_hits[WAVES], chunk_total[SORT_BLOCK_MAX_NR / 64];
     __shared__ int kept_total, kept_before[SORT_BLOCK_MAX_NR / 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int base = (SPREAD ? part.first : 0) + wv * ITERS * 64 + lane;
+    const int j = (SPREAD ? part.first : 0) + tid;
     volatile int *mine = off[wv];
     for (int i = lane; i < NR; i += 64) mine[i] = 0;
     __builtin_amdgcn_wave_barrier();
-    int key[ITERS], rank[ITERS], before_in_step[ITERS], hits = 0;   // before_in_step: kept pairs of this wavefront before this one
-#pragma unroll
-    for (int it = 0; it < ITERS; it++) {
-        const long long v = static_cast<long long>(e[it]);
-        const bool kept = base + it * 64 < n_pairs && v >= start && v < end;
-        key[it] = kept ? static_cast<int>(v - start) : NR;
-        const unsigned long long m = match_key(key[it], nbits), all = __ballot(kept);
-        const int seen = mine[kept ? key[it] : 0];
-        __builtin_amdgcn_wave_barrier();
-        rank[it] = seen + __popcll(m & lanemask_lt(lane));
-        if (kept && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key[it]] = seen + __popcll(m);
-        before_in_step[it] = hits + __popcll(all & lanemask_lt(lane));
-        hits += __popcll(all);
-        __builtin_amdgcn_wave_barrier();
-    }
-    if (lane == 0) wave_hits[wv] = hits;
+    const long long v = static_cast<long long>(e);
+    const bool kept = j < n_pairs && v >= start && v < end;
+    const int key = kept ? static_cast<int>(v - start) : NR;
+    const unsigned long long m = match_key(key, nbits), all = __ballot(kept);
+    const int rank = __popcll(m & lanemask_lt(lane));
+    if (kept && (__ffsll(static_cast<long long>(m)) - 1) == lane) mine[key] = __popcll(m);
+    if (lane == 0) wave_hits[wv] = __popcll(all);
     __syncthreads();
     // thread e: expert e's total over the wavefronts, exclusive positions of the wavefronts within it
     int total = 0, ahead = 0, at[WAVES];   // ahead: SPREAD, the expert's pairs before this block's
@@ -98,8 +90,8 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
         }
     }
     if (SPREAD && tid < SORT_BLOCK_MAX_NR) {
-        const int kept = wave_sum_i(ahead);
-        if (lane == 0) kept_before[wv] = kept;
+        const int kept_ahead = wave_sum_i(ahead);
+        if (lane == 0) kept_before[wv] = kept_ahead;
     }
     const int incl = wave_incl_scan(total, lane);
     if (tid < SORT_BLOCK_MAX_NR && lane == 63) chunk_total[wv] = incl;
@@ -121,34 +113,28 @@ __device__ __forceinline__ void sort_block(const TI (&e)[ITERS], const float (&w
         }
     }
     __syncthreads();
-    int oi_base = 0;
+    int oi = __popcll(all & lanemask_lt(lane));   // kept pairs before this one: of its wavefront, the block and the blocks before
 #pragma unroll
-    for (int w = 0; w < WAVES; w++) oi_base += w < wv ? wave_hits[w] : 0;
+    for (int w = 0; w < WAVES; w++) oi += w < wv ? wave_hits[w] : 0;
     if (SPREAD) {
 #pragma unroll
-        for (int w = 0; w < SORT_BLOCK_MAX_NR / 64; w++) oi_base += kept_before[w];
+        for (int w = 0; w < SORT_BLOCK_MAX_NR / 64; w++) oi += kept_before[w];
     }
-    const int kept_all = kept_total;
-#pragma unroll
-    for (int it = 0; it < ITERS; it++) {
-        const int j = base + it * 64;
-        if (j >= n_pairs) continue;
-        if (j >= kept_all) {   // past the kept pairs: see sort_scatter_kernel
-            output_indices[j] = -1;
-            input_indices[j] = 0;
-            selected_experts_indices[j] = 0;
-        }
-        const int oi = oi_base + before_in_step[it];
-        const uint32_t t = static_cast<uint32_t>(j) / static_cast<uint32_t>(K);
-        const int k = j - static_cast<int>(t) * K;
-        if (k == 0) cum_expert_counts_ep[t] = oi;
-        if (key[it] < NR) {
-            const int pos = off[wv][key[it]] + rank[it];
-            input_indices[pos] = static_cast<int32_t>(t);
-            output_indices[oi] = pos;
-            selected_experts_indices[oi] = k;
-            if (row_weights) row_weights[pos] = weight[it];
-        }
+    if (j >= n_pairs) return;
+    if (j >= kept_total) {   // past the kept pairs: see sort_scatter_kernel
+        output_indices[j] = -1;
+        input_indices[j] = 0;
+        selected_experts_indices[j] = 0;
+    }
+    const uint32_t t = static_cast<uint32_t>(j) / static_cast<uint32_t>(K);
+    const int k = j - static_cast<int>(t) * K;
+    if (k == 0) cum_expert_counts_ep[t] = oi;
+    if (kept) {
+        const int pos = off[wv][key] + rank;
+        input_indices[pos] = static_cast<int32_t>(t);
+        output_indices[oi] = pos;
+        selected_experts_indices[oi] = k;
+        if (row_weights) row_weights[pos] = weight;
     }
 }
 
