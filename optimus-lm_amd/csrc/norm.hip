@@ -267,15 +267,16 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_rows_kernel(const T *__restri
 }
 inline int64_t bwd_chunk(int64_t rows) { return (rows + 2047) / 2048 * 4; }
 
-// dx of longer rows, and with little workspace, one wavefront per row.  Rows that fit the registers are read once (16384 rows of 2048 bf16,
-// the whole backward, operands in the caches: 77 us read twice, 62 so; 4096 rows 39 and 36); longer ones twice.
-template <typename T, bool FITS, bool ADD>
+// dx of longer rows, and with little workspace, one wavefront per row.  Rows that fit the registers are read once, VECS vectors a lane: the whole
+// backward with little workspace, operands in the caches, us, read twice -> so: 16384 rows of 2048 bf16 71 -> 55, 4096 33.0 -> 30.4, 16384 of 512
+// 30.4 -> 29.1 (32.6 with registers for the longest row), 4096 of 1024 float32 29.0 -> 25.5.  Longer rows twice (VECS = 0).
+template <typename T, int VECS, bool ADD>
 __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ dy,
                                                          const T *__restrict__ h,
                                                          const T *__restrict__ weight,
                                                          const float *__restrict__ rstd, const T *__restrict__ h_grad,
                                                          T *__restrict__ dx, int64_t rows, int64_t E) {
-    constexpr int V = Elem<T>::VEC;
+    constexpr int V = Elem<T>::VEC, U = VECS ? VECS : ROW_VECS;
     const int lane = threadIdx.x & 63;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * NORM_ROWS + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -285,11 +286,11 @@ __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ d
     const u32x4 *dyr = reinterpret_cast<const u32x4 *>(dy + row * E);
     const u32x4 *hr = reinterpret_cast<const u32x4 *>(h + row * E);
     u32x4 *dxr = reinterpret_cast<u32x4 *>(dx + row * E);
-    float dxn[ROW_VECS][V], xn[ROW_VECS][V];   // FITS: of the whole row
+    float dxn[U][V], xn[U][V];   // VECS: of the whole row
     float dot = 0.0f;
-    for (int64_t c0 = 0; c0 < nv; c0 += 64 * ROW_VECS) {
+    for (int64_t c0 = 0; c0 < nv; c0 += 64 * U) {
 #pragma unroll
-        for (int u = 0; u < ROW_VECS; u++) {
+        for (int u = 0; u < U; u++) {
             const int64_t c = c0 + u * 64 + lane;
             if (c < nv) {
                 float g[V], f[V], w[V];
@@ -306,12 +307,12 @@ __global__ __launch_bounds__(256) void rmsnorm_dx_kernel(const T *__restrict__ d
         }
     }
     dot = wave_sum(dot) / static_cast<float>(E);
-    for (int64_t c0 = 0; c0 < nv; c0 += 64 * ROW_VECS) {
+    for (int64_t c0 = 0; c0 < nv; c0 += 64 * U) {
 #pragma unroll
-        for (int u = 0; u < ROW_VECS; u++) {
+        for (int u = 0; u < U; u++) {
             const int64_t c = c0 + u * 64 + lane;
             if (c < nv) {
-                if (!FITS) {
+                if (!VECS) {
                     float g[V], f[V], w[V];
                     Elem<T>::unpack(dyr[c], g);
                     Elem<T>::unpack(hr[c], f);
@@ -381,7 +382,16 @@ __global__ __launch_bounds__(4 * DW_REDUCE) void rmsnorm_dw_reduce_kernel(const 
     int b = n_blocks * wave / 4;
     float s = 0.0f;
     if (e < E) {
-        for (; b < end; b += 16) {         // (past the last of them: it again, not added)
+        for (; b + 16 <= end; b += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = dw_part[static_cast<int64_t>(b + u) * E + e];
+#pragma unroll
+            for (int u = 0; u < 16; u++) s += v[u];
+        }
+        // the rest together too (past the last of them: it again, not added): 3001 rows of 1000 bf16, whole backward, 13.6 -> 10.7 us; in every
+        // round it cost 16384 rows of 2048 1.6 us
+        if (b < end) {
             float v[16];
 #pragma unroll
             for (int u = 0; u < 16; u++) v[u] = dw_part[static_cast<int64_t>(min(b + u, end - 1)) * E + e];
@@ -486,11 +496,12 @@ extern "C" int om_rmsnorm_bwd_residual(const void *dy, const void *h, const void
         if (!fits) {
             chunks = static_cast<int>((rows + DW_ROWS - 1) / DW_ROWS);
             const dim3 grid(static_cast<unsigned>((rows + NORM_ROWS - 1) / NORM_ROWS));
-            const bool row_fits = E / V <= 64 * ROW_VECS;
-            if (row_fits && hg) rmsnorm_dx_kernel<T, true, true><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
-            else if (row_fits) rmsnorm_dx_kernel<T, true, false><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
-            else if (hg) rmsnorm_dx_kernel<T, false, true><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
-            else rmsnorm_dx_kernel<T, false, false><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            auto rows_dx = [&](auto vecs) {
+                constexpr int N = decltype(vecs)::value;
+                if (hg) rmsnorm_dx_kernel<T, N, true><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+                else rmsnorm_dx_kernel<T, N, false><<<grid, 256, 0, st>>>(g, hh, wt, rstd, hg, to, rows, E);
+            };
+            if (!with_vecs(E / V, rows_dx)) rows_dx(std::integral_constant<int, 0>());
             rmsnorm_dw_kernel<T><<<dim3(static_cast<unsigned>((E / V + 63) / 64), static_cast<unsigned>(chunks)), 256, 0, st>>>(g, hh, rstd, part, rows, E);
         }
         rmsnorm_dw_reduce_kernel<T><<<static_cast<unsigned>((E + DW_REDUCE - 1) / DW_REDUCE), 4 * DW_REDUCE, 0, st>>>(part, chunks, E, static_cast<T *>(dweight));

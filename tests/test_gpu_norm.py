@@ -163,3 +163,11 @@ def test_backward_with_the_least_workspace(cuda, rows, vecs, dtype, add):
     with_ws = lambda size: L.om_rmsnorm_bwd(n.ptr(dy), n.ptr(h), n.ptr(w), n.ptr(rstd), n.ptr(got[0][0]), n.ptr(got[0][1]), n.ptr(ws), size, rows, E,
                                             n.dtype_code(h), st)
     assert with_ws(L.om_rmsnorm_bwd_workspace_bytes(rows, E) - 1) != 0
+
+
+@pytest.mark.parametrize("rows,vecs", [(130, 65), (515, 128), (1000, 129), (257, 192), (900, 193)])
+def test_backward_with_the_least_workspace_for_every_length_that_fits(cuda, rows, vecs):
+    """Two, three and four vectors a lane, whole and partial."""
+    for dtype in (torch.bfloat16, torch.float32):
+        for add in (False, True):
+            test_backward_with_the_least_workspace(cuda, rows, vecs, dtype, add)
