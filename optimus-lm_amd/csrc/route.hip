@@ -386,7 +386,8 @@ __global__ __launch_bounds__(256) void sigmoid_group_topk_kernel(
 // experts, so a slice's partial sums are one load a lane, of sixteen slices under way at once, and a group's two best meet by exchanges
 // between its lanes (above, one lane scans a group's scores in LDS).  A token waits for its loads and for chains of a few
 // instructions; with few tokens a wavefront per block.  Same sums, same order of selection.  us, 256 experts, 64 tokens of 28
-// slices 13.6 -> 8.0, 8192 of 4 slices 22.4 -> 17.2 (and 5 less for a bias in bf16, which was widened by a launch of its own).
+// slices 13.6 -> 8.0, 8192 of 4 slices 22.4 -> 17.2 (and 5 less for a bias in bf16, which was widened by a launch of its own); 0.2 of it
+// for scores that are not finite.
 constexpr int QUADS = 4;
 template <typename TB>
 __global__ __launch_bounds__(256) void sigmoid_group_quads_kernel(const float *__restrict__ partial, int splits, float *__restrict__ logits_out,
