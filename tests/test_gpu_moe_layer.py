@@ -450,8 +450,8 @@ def test_dsv3_block_one_rank_share(cuda, ep_ind):
 
 
 def test_unfused_paths_are_announced_or_refused(cuda):
-    """A shape the fused gate+routing kernel does not take makes the block run the kernels of other hidden sizes: announced once
-    as a UserWarning, refused when strict_fused_paths is set."""
+    """A shape the fused gate+routing kernel does not take makes the block run the projection and the
+    routing separately: announced once as a UserWarning, refused when strict_fused_paths is set."""
     import warnings
     from optimus._native import NativeLibraryError
     from optimus.models.common import moe
